@@ -30,10 +30,12 @@ Engine::Engine(const cavs_session_config &cfg, void *external_stream, std::share
   if (cfg.loss < 0 || cfg.loss > 2) fail(CAVS_EINVAL, "unknown loss " + std::to_string(cfg.loss));
   if (cfg.pairing < 0 || cfg.pairing > 1) fail(CAVS_EINVAL, "unknown pairing");
   if (cfg.H <= 0) fail(CAVS_EINVAL, "hidden size must be positive");
-  const size_t H = cfg.H;
+  own_stream_ = external_stream == nullptr;
   E_ = cfg.model == CAVS_MODEL_LSTM ? cfg.H : cfg.E;  // the chain LSTM requires E == H
+  pad_sizes();
+  const size_t H = cfg_.H, h = uH_, e = uE_;
   ld_e_ = cfg.model == CAVS_MODEL_TREELSTM ? E_ + 4 : E_;
-  mw_ = cfg.model == CAVS_MODEL_TREEFC ? cfg.H : 2 * cfg.H;
+  mw_ = cfg.model == CAVS_MODEL_TREEFC ? H : 2 * H;
   nch_ = cfg.model == CAVS_MODEL_LSTM ? 1 : 2;
   if (cell_) {
     if (cell_->H != cfg.H || cell_->K < 1 || cell_->K > 2 || (int)cell_->params.size() > CA_MAX_PARAMS)
@@ -50,24 +52,37 @@ Engine::Engine(const cavs_session_config &cfg, void *external_stream, std::share
     fail(CAVS_EINVAL, "vocabulary and embedding sizes must be positive");
   if (cfg.loss == CAVS_LOSS_SOFTMAX && cfg.C <= 0) fail(CAVS_EINVAL, "class count must be positive");
   check(cavs_init(cfg.device));
-  if (external_stream) {
+  if (external_stream)
     stream_ = external_stream;
-    own_stream_ = false;
-  } else {
+  else
     check(cavs_stream_create(&stream_));
-  }
   for (auto &e : ev_) check(cavs_event_create(&e));
+  // where the blocks of the declared parameters lie in the stored ones (none: they are the same)
+  auto gates = [&](bool pad, size_t user, size_t eng, int n, size_t rows) {  // [rows, n h] -> [., n H]: a block per gate
+    std::vector<PadBlock> b;
+    for (int k = 0; pad && k < n; k++) b.push_back({user + k * h, n * h, eng + k * H, n * H, (int)rows, (int)h});
+    return b;
+  };
+  auto both = [](std::vector<PadBlock> a, const std::vector<PadBlock> &b) {
+    a.insert(a.end(), b.begin(), b.end());
+    return a;
+  };
+  auto rows = [&](size_t n, size_t width, size_t stored) {
+    return width != stored ? std::vector<PadBlock>{{0, width, 0, stored, (int)n, (int)width}} : std::vector<PadBlock>{};
+  };
+  const size_t E = E_;
   switch (cfg.model) {
     case CAVS_MODEL_TREELSTM:
-      add_param("Emb", (size_t)cfg.V * E_);
-      add_param("W", (size_t)E_ * 4 * H, 4 * 4 * H);  // four more rows (one used): the bias gradient comes out of the same product
-      add_param("U", 4 * H * H);
-      add_param("Bv", 4 * H);
+      add_param("Emb", cfg.V * E, 0, rows(cfg.V, e, E));
+      // four more rows (one used): the bias gradient comes out of the same product
+      add_param("W", E * 4 * H, 4 * 4 * H, gates(h != H || e != E, 0, 0, 4, e));
+      add_param("U", 4 * H * H, 0, both(gates(h != H, 0, 0, 3, h), gates(h != H, 3 * h * h, 3 * H * H, 1, h)));
+      add_param("Bv", 4 * H, 0, rows(4, h, H));
       break;
     case CAVS_MODEL_LSTM:
-      add_param("Emb", (size_t)cfg.V * H);
-      add_param("W", 8 * H * H);
-      add_param("Bv", 4 * H);
+      add_param("Emb", cfg.V * E, 0, rows(cfg.V, e, E));
+      add_param("W", 4 * H * (E + H), 0, both(gates(h != H, 0, 0, 4, e), gates(h != H, 4 * h * e, 4 * H * E, 4, h)));
+      add_param("Bv", 4 * H, 0, rows(4, h, H));
       break;
     case CAVS_MODEL_CELL:
       for (const CellParam &p : cell_->params) add_param(p.name, (size_t)p.size);
@@ -78,14 +93,40 @@ Engine::Engine(const cavs_session_config &cfg, void *external_stream, std::share
       }
       break;
     default:
-      add_param("W", 2 * H * H);
-      if (cfg.use_bias) add_param("Bv", H);
+      add_param("W", 2 * H * H, 0, both(gates(h != H, 0, 0, 1, h), gates(h != H, h * h, H * H, 1, h)));
+      if (cfg.use_bias) add_param("Bv", H, 0, rows(1, h, H));
   }
   if (cfg.loss == CAVS_LOSS_SOFTMAX) {
-    add_param("Wfc", (size_t)cfg.C * H);
+    add_param("Wfc", (size_t)cfg.C * H, 0, rows(cfg.C, h, H));
     add_param("bfc", cfg.C);
   }
   tail_setup();
+}
+
+// Sizes the kernels run at.  The fused rounds take hidden sizes in whole tiles of 32 columns, the
+// products of x read sixteen bytes at a time: other sizes are stored with zero columns up to the next
+// multiple (cfg_.H, E_; the declared ones stay in uH_, uE_).  A padding column stays zero: its weights
+// and biases are zero, so u = tanh(0) = 0, c = i u + f c' = 0 and h = o tanh(c) = 0, and with d h = 0
+// from the head and from the rounds above every gate gradient and every weight gradient of the
+// column is a product with a zero.  Without it such a size runs a round as six to ten separate launches
+// (Tree-LSTM, H = 150, 25 trees: 0.78 ms per step, 0.24 padded).
+// Not for a caller's own tensors (their layout is the caller's), not where no fused round runs.
+void Engine::pad_sizes() {
+  uH_ = cfg_.H;
+  uE_ = E_;
+  if (!own_stream_ || cell_ || !(cfg_.opt & CAVS_OPT_BATCHING) || cfg_.fused_round_rows < 0) return;
+  cfg_.H = (uH_ + 31) / 32 * 32;
+  // the lookup's row offset is id * E in single precision (EmbeddingLookup): where that is not
+  // exact for every id, the rows stay where they are
+  if (E_ > 0 && (double)cfg_.V * E_ <= (double)(1 << 24)) E_ = (E_ + 3) / 4 * 4;
+}
+
+const float *Engine::user_rows(const float *src, size_t n, int blocks) {
+  const int h = uH_, H = cfg_.H;
+  if (h == H) return src;
+  ensure(pad_stage_, n * blocks * h);
+  check(cavs_copy_rows(pad_stage_.get(), h, src, H, (int)(n * blocks), h, stream_));
+  return pad_stage_.get();
 }
 
 // ------------------------------------------------------------------ the rounds near the roots in one launch
@@ -173,9 +214,14 @@ Engine::~Engine() {
   if (own_stream_) cavs_stream_destroy(stream_);
 }
 
-void Engine::add_param(const std::string &name, size_t n, size_t extra_grad) {
+void Engine::add_param(const std::string &name, size_t n, size_t extra_grad, std::vector<PadBlock> blocks) {
   auto p = std::make_unique<Param>();
-  p->n = n;
+  p->n = p->user_n = n;
+  if (!blocks.empty()) {
+    p->user_n = 0;
+    for (const PadBlock &b : blocks) p->user_n += (size_t)b.rows * b.cols;
+    p->blocks = std::move(blocks);
+  }
   p->own_w.reserve(n);
   p->own_g.reserve(n + extra_grad);
   p->w = p->own_w.get();
@@ -219,7 +265,7 @@ bool Engine::update_jobs(float *w, float *g, float lr, std::vector<cavs_task> *o
     out->push_back({CAVS_TASK_SGD_PACK, lr, H, 3 * H, 0, Upk_.get(), w, g, nullptr});
     out->push_back({CAVS_TASK_SGD_PACK, lr, H, H, 0, Upk_.at((size_t)3 * H * H), w + 3 * H * H, g + 3 * H * H, nullptr});
   } else if (cfg_.model == CAVS_MODEL_LSTM && w == param("W").w) {  // [U' | W'], W' with its packed copy
-    const long long half = 4 * H * H;
+    const long long half = 4 * H * E_;
     out->push_back({CAVS_TASK_SGD, lr, half, 0, 0, w, g, nullptr, nullptr});
     out->push_back({CAVS_TASK_SGD_PACK, lr, H, 4 * H, 0, Upk_.get(), w + half, g + half, nullptr});
   } else {
@@ -231,9 +277,12 @@ bool Engine::update_jobs(float *w, float *g, float lr, std::vector<cavs_task> *o
 
 void Engine::set_param(const std::string &name, const float *host, size_t n) {
   Param &p = param(name);
-  if (n != p.n || !host)
-    fail(CAVS_EINVAL, "parameter '" + name + "' has " + std::to_string(p.n) + " elements, got " + std::to_string(n));
-  check(cavs_memcpy_h2d(p.w, host, n * 4, stream_));
+  if (n != p.user_n || !host)
+    fail(CAVS_EINVAL, "parameter '" + name + "' has " + std::to_string(p.user_n) + " elements, got " + std::to_string(n));
+  if (!p.blocks.empty()) ensure(pad_stage_, n);
+  check(cavs_memcpy_h2d(p.blocks.empty() ? p.w : pad_stage_.get(), host, n * 4, stream_));
+  for (const PadBlock &b : p.blocks)
+    check(cavs_copy_rows(p.w + b.eng, (int)b.ld_eng, pad_stage_.at(b.user), (int)b.ld_user, b.rows, b.cols, stream_));
   check(cavs_stream_sync(stream_));
   upk_valid_ = wfct_valid_ = false;
   state_epoch_++;
@@ -241,10 +290,17 @@ void Engine::set_param(const std::string &name, const float *host, size_t n) {
 
 void Engine::get_param(const std::string &name, float *host, size_t n, bool grad) {
   Param &p = param(name);
-  if (n != p.n || !host)
-    fail(CAVS_EINVAL, "parameter '" + name + "' has " + std::to_string(p.n) + " elements, got " + std::to_string(n));
+  if (n != p.user_n || !host)
+    fail(CAVS_EINVAL, "parameter '" + name + "' has " + std::to_string(p.user_n) + " elements, got " + std::to_string(n));
   aux_join();
-  check(cavs_memcpy_d2h(host, grad ? p.g : p.w, n * 4, stream_));
+  const float *src = grad ? p.g : p.w;
+  if (!p.blocks.empty()) {
+    ensure(pad_stage_, n);
+    for (const PadBlock &b : p.blocks)
+      check(cavs_copy_rows(pad_stage_.at(b.user), (int)b.ld_user, src + b.eng, (int)b.ld_eng, b.rows, b.cols, stream_));
+    src = pad_stage_.get();
+  }
+  check(cavs_memcpy_d2h(host, src, n * 4, stream_));
   check(cavs_stream_sync(stream_));
 }
 
@@ -359,10 +415,11 @@ void Engine::scatter(float *dst, int ld_dst, const int *ids, const float *inp, i
 }
 
 // Growing a buffer frees the old storage, which enqueued kernels may still read.
-void Engine::ensure(DeviceArray<float> &a, size_t n) {
-  if (n <= a.capacity()) return;
+bool Engine::ensure(DeviceArray<float> &a, size_t n) {
+  if (n <= a.capacity()) return false;
   check(cavs_stream_sync(stream_));
   a.reserve(n);
+  return true;
 }
 
 // the identity list 0, 1, 2, ... of at least n entries
@@ -451,7 +508,8 @@ void Engine::reserve_edges() {
     R(gates_, cap * 6 * H);
     R(dc_, cap * H);
   } else {
-    if (cfg_.use_x) R(xs_, cap * H);
+    // (the gathered rows have the declared width: what is beyond stays zero)
+    if (cfg_.use_x && ensure(xs_, cap * H) && uH_ != cfg_.H) check(cavs_zero(xs_.get(), cap * H * 4, stream_));
     R(dxW_, cap * H);
     R(r_z_, rc * H);
   }
@@ -943,9 +1001,9 @@ void Engine::step(const int *graph, int B, int maxlen, const void *x, const void
     ~StepTimer() { e->host_step_ms_ = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count(); }
   } step_timer{this, step_t0};
   begin_step(graph, B, maxlen);
-  const int N = N_, H = cfg_.H;
+  const int N = N_;
   const bool needs_x = cfg_.model != CAVS_MODEL_TREEFC || cfg_.use_x;
-  const size_t xw = cfg_.model == CAVS_MODEL_TREEFC ? H : 1;
+  const size_t xw = cfg_.model == CAVS_MODEL_TREEFC ? uH_ : 1;
   if (needs_x && !x) fail(CAVS_EINVAL, "vertex input feed is null");
   if (cfg_.loss == CAVS_LOSS_SOFTMAX && !labels) fail(CAVS_EINVAL, "label feed is null");
   if (on_device) {
@@ -1494,14 +1552,14 @@ void Engine::gemm_group_embedding_backward(const std::vector<cavs_gemm_desc> &pr
 // ------------------------------------------------------------------ chain LSTM
 // apps/paper/seq-lstm-cavs.cc:62-86
 void Engine::lstm_forward() {
-  const int N = N_, H = cfg_.H;
-  const float *Wx = param("W").w, *Wh = Wx + (size_t)4 * H * H, *Bv = param("Bv").w;
+  const int N = N_, H = cfg_.H, E = E_;
+  const float *Wx = param("W").w, *Wh = Wx + (size_t)4 * H * E, *Bv = param("Bv").w;
   {  // Pull of the token id, the lookup and x * W_x: one launch
     ProfScope ps(this, K_GEMM);
-    check(cavs_embed_pull_sgemm(xW_.get(), 4 * H, e_.get(), H, xs_.get(), d_x_, d_t2j_, param("Emb").w, N, H, Wx, 4 * H, 4 * H, 0, 0,
+    check(cavs_embed_pull_sgemm(xW_.get(), 4 * H, e_.get(), E, xs_.get(), d_x_, d_t2j_, param("Emb").w, N, E, Wx, 4 * H, 4 * H, 0, 0,
                                 stream_));
   }
-  c_gemm_flops_ += 2.0 * N * 4 * H * H;
+  c_gemm_flops_ += 2.0 * N * 4 * H * E;
   c_launches_ += 1;
   if (!sched_->batching) check(cavs_zero(G_.get(), (size_t)N * 2 * H * 4, stream_));
   const int fused = fused_rows();
@@ -1547,8 +1605,8 @@ void Engine::lstm_forward() {
 }
 
 void Engine::lstm_backward() {
-  const int N = N_, H = cfg_.H;
-  const float *Wx = param("W").w, *Wh = Wx + (size_t)4 * H * H;
+  const int N = N_, H = cfg_.H, E = E_;
+  const float *Wx = param("W").w, *Wh = Wx + (size_t)4 * H * E;
   const int fused = fused_rows();
   const bool dret_folded = fused > 0 && sched_->max_round <= fused;
   if (!dret_folded && !forest_) gather(dret_.get(), H, d_dgo_, H, d_t2j_, N, H);
@@ -1632,11 +1690,11 @@ void Engine::lstm_backward() {
   const int lp = sched_->leaf_prefix;
   float *dW = param("W").g;
   gemm_group_embedding_backward({
-      {0, 1, N, H, 4 * H, 1.f, 0.f, dxW_.get(), 4 * H, Wx, 4 * H, de_.get(), H},
-      {1, 0, H, 4 * H, N, 1.f, 0.f, e_.get(), H, dxW_.get(), 4 * H, dW, 4 * H},
+      {0, 1, N, E, 4 * H, 1.f, 0.f, dxW_.get(), 4 * H, Wx, 4 * H, de_.get(), E},
+      {1, 0, E, 4 * H, N, 1.f, 0.f, e_.get(), E, dxW_.get(), 4 * H, dW, 4 * H},
       {1, 0, H, 4 * H, N - lp, 1.f, 0.f, G_.at((size_t)lp * 2 * H), 2 * H, dxW_.at((size_t)lp * 4 * H), 4 * H,
-       dW + (size_t)4 * H * H, 4 * H},
-  }, H);
+       dW + (size_t)4 * H * E, 4 * H},
+  }, E);
   bias_gradient("Bv", dxW_.get(), N, 4 * H, bias_parts_);
 }
 
@@ -1646,7 +1704,7 @@ void Engine::treefc_forward() {
   const int N = N_, H = cfg_.H;
   const float *W = param("W").w;
   const float *Bv = cfg_.use_bias ? param("Bv").w : nullptr;
-  if (cfg_.use_x) gather(xs_.get(), H, d_x_, H, d_t2j_, N, H);
+  if (cfg_.use_x) gather(xs_.get(), H, d_x_, uH_, d_t2j_, N, uH_);
   if (!sched_->batching) check(cavs_zero(G_.get(), (size_t)N * 2 * H * 4, stream_));
   const int fused = fused_rows();
   out_folded_ = fused > 0 && sched_->max_round <= fused && fwd_out_ != nullptr;
@@ -2123,7 +2181,18 @@ void Engine::head_forward_backward(bool backward) {
     colsum_fixed(loss_.get(), colacc, H, 1);
     c_launches_ += 1;
     if (backward) {
-      check(cavs_fill(dGO_.get(), 1.f, (size_t)N * H, stream_));
+      if (uH_ == H) {
+        check(cavs_fill(dGO_.get(), 1.f, (size_t)N * H, stream_));
+      } else {  // ones in the declared columns
+        if (pad_mask_.reserve(H)) {
+          std::vector<float> mask(H, 0.f);
+          std::fill(mask.begin(), mask.begin() + uH_, 1.f);
+          check(cavs_memcpy_h2d(pad_mask_.get(), mask.data(), (size_t)H * 4, stream_));
+          check(cavs_stream_sync(stream_));
+        }
+        check(cavs_zero(dGO_.get(), (size_t)N * H * 4, stream_));
+        check(cavs_bias_add_rows(dGO_.get(), dGO_.get(), pad_mask_.get(), N, H, stream_));
+      }
       c_launches_ += 1;
     }
   }
@@ -2254,26 +2323,31 @@ void Engine::sync() {
 }
 
 void Engine::fetch(const std::string &what, float *host, size_t n) {
-  const size_t N = N_, H = cfg_.H;
+  const size_t N = N_, h = uH_;
   const float *src = nullptr;
   size_t want = 0;
+  int blocks = 0;  // rows of so many blocks of the hidden size
   if (what == "loss") {
     src = loss_.get();
     want = cfg_.loss == CAVS_LOSS_SOFTMAX ? N : 1;
   } else if (what == "graph_out") {
     src = GO_.get();
-    want = N * H;
+    want = N * h;
+    blocks = 1;
   } else if (what == "dgraph_out") {
     src = dGO_.get();
-    want = N * H;
+    want = N * h;
+    blocks = 1;
   } else if (what == "msg_pool") {
     src = pool_.get();
-    want = N * mw_;
+    blocks = mw_ / cfg_.H;
+    want = N * h * blocks;
   } else {
     fail(CAVS_EINVAL, "unknown result '" + what + "'");
   }
   if (N == 0) fail(CAVS_EINVAL, "no step has run yet");
   if (n != want || !host) fail(CAVS_EINVAL, "'" + what + "' holds " + std::to_string(want) + " floats, got " + std::to_string(n));
+  if (blocks > 0) src = user_rows(src, N, blocks);
   check(cavs_memcpy_d2h(host, src, want * 4, stream_));
   check(cavs_stream_sync(stream_));
   tail_check();

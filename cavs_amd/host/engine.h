@@ -21,10 +21,19 @@
 
 namespace cavs {
 
+// One block of a parameter the engine stores wider than its owner declares it (Engine::pad_sizes):
+// `rows` rows of `cols` elements at `user` (row stride ld_user) of the declared layout are those at
+// `eng` (row stride ld_eng) of the engine's.
+struct PadBlock {
+  size_t user, ld_user, eng, ld_eng;
+  int rows, cols;
+};
+
 struct Param {
   float *w = nullptr, *g = nullptr;  // owned storage below, or bound to a caller's tensors
   DeviceArray<float> own_w, own_g;
-  size_t n = 0;
+  size_t n = 0, user_n = 0;          // elements stored, elements declared
+  std::vector<PadBlock> blocks;      // empty: stored as declared
 };
 
 class Engine {
@@ -89,9 +98,13 @@ class Engine {
 
  private:
   Param &param(const std::string &name);
-  void add_param(const std::string &name, size_t n, size_t extra_grad = 0);
+  void add_param(const std::string &name, size_t n, size_t extra_grad = 0, std::vector<PadBlock> blocks = {});
+  void pad_sizes();
+  // device rows [n, uH per block] of `src`, whose rows are blocks of the stored width H: where the
+  // declared width differs, packed to it in the staging buffer
+  const float *user_rows(const float *src, size_t n, int blocks);
   void reserve_edges();
-  void ensure(DeviceArray<float> &a, size_t n);  // grow after draining the stream
+  bool ensure(DeviceArray<float> &a, size_t n);  // grow after draining the stream; true when it did
   void upload_index_arena();
   // one model each: forward rounds, backward rounds + deferred weight gradients
   void treelstm_forward();
@@ -139,7 +152,10 @@ class Engine {
   std::vector<void *> prof_events_;
   size_t prof_used_ = 0;
 
-  cavs_session_config cfg_;
+  cavs_session_config cfg_;       // (cfg_.H: the hidden size the kernels run at)
+  int uH_ = 0, uE_ = 0;           // hidden and embedding size as declared
+  DeviceArray<float> pad_stage_;  // parameters and results on their way between the two layouts
+  DeviceArray<float> pad_mask_;   // [H] 1 where a column is declared, 0 where it is padding
   void *stream_ = nullptr;
   bool own_stream_ = true;
   void *ev_[4] = {nullptr, nullptr, nullptr, nullptr};  // fwd begin/end, bwd begin/end

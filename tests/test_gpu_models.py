@@ -676,3 +676,32 @@ def test_recorded_graph_of_a_cached_plan_gives_the_steps_of_the_host_loop(model,
     np.testing.assert_allclose(out[1], out[0], rtol=2e-6, atol=1e-7)
     for s in sessions:
         s.close()
+
+
+@pytest.mark.parametrize("H,E", [(1, 3), (31, 13), (33, 32), (100, 101)])
+@pytest.mark.parametrize("model,loss,kw", [("treelstm", "softmax", {}), ("lstm", "softmax", {}),
+                                           ("treefc", "root_sq", dict(act=1, use_bias=True, use_x=True)),
+                                           ("treefc", "sum_abs", dict(act=1, use_bias=True, use_x=True))])
+def test_sizes_that_are_no_multiple_of_a_tile(oracle, model, loss, kw, H, E):
+    """The session stores such sizes with zero columns up to the next multiple: one pass against the
+    oracle, then two SGD steps whose gradients and parameters must be those of w - lr * g."""
+    if model == "lstm":
+        E = H
+    w = small_workload(model, 811, B=7, H=H, E=E)
+    got, want = run_both(oracle, w, loss=loss, **kw)
+    compare(got, want, loss)
+    s = session.Session(model, H=H, E=w["E"], V=w["V"], C_=w["C"], loss=loss, **kw)
+    p = {k: np.array(v, np.float32) for k, v in w["params"].items() if loss == "softmax" or not k.endswith("fc")}
+    s.set_params(p)
+    lr = np.float32(0.05)
+    for step in range(2):
+        s.step(w["graph"], w["x"], w["labels"], backward=True, lr=float(lr))
+        want = oracle.model_step(model, w["graph"], w["x"], w["labels"], dict(w["params"], **p), H=H, E=w["E"], V=w["V"], Cc=w["C"],
+                                 loss=loss, precise=True, **kw)
+        close(s.fetch("loss"), want["loss"], f"loss of step {step}")
+        for k, v in want["grads"].items():
+            if k[1:] not in p:
+                continue
+            p[k[1:]] = (p[k[1:]].ravel() - lr * np.asarray(v, np.float32).ravel()).reshape(p[k[1:]].shape)
+            close(s.param(k[1:], p[k[1:]].shape), p[k[1:]], k[1:])
+    s.close()
