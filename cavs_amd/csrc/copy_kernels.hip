@@ -158,11 +158,60 @@ static int launch_gather(float *out, int ld_out, const float *src, int ld_src, c
   return CAVS_OK;
 }
 
+// Copies of column blocks, several to a launch (cavs_copy_blocks): the blocks of a step's parameters are
+// tens of kilobytes each, and a launch per block cost more than its bytes (nine blocks of a Tree-LSTM at
+// H = 150: 9 x 3 us, 4.5 us in one).  A workgroup takes 2048 consecutive elements of one block,
+// thread by thread along its rows.
+constexpr int kBlockCopies = 32, kBlockElems = 2048;
+struct BlockCopies {
+  cavs_block_copy b[kBlockCopies];
+  int first[kBlockCopies + 1];
+  int count;
+};
+__global__ __launch_bounds__(256) void copy_blocks_kernel(BlockCopies a) {
+  int p = 0;
+  while (p + 1 < a.count && (int)blockIdx.x >= a.first[p + 1]) p++;
+  const cavs_block_copy &c = a.b[p];
+  const long total = (long)c.rows * c.cols, i0 = (long)(blockIdx.x - a.first[p]) * kBlockElems + threadIdx.x;
+  float v[kBlockElems / 256];
+#pragma unroll
+  for (int k = 0; k < kBlockElems / 256; k++) {
+    const long i = i0 + 256 * k;
+    if (i < total) v[k] = c.src[i / c.cols * c.ld_src + i % c.cols];
+  }
+#pragma unroll
+  for (int k = 0; k < kBlockElems / 256; k++) {
+    const long i = i0 + 256 * k;
+    if (i < total) c.dst[i / c.cols * c.ld_dst + i % c.cols] = v[k];
+  }
+}
+
 }  // namespace cavs
 
 using namespace cavs;
 
 extern "C" {
+
+int cavs_copy_blocks(int count, const cavs_block_copy *blocks, void *stream) {
+  CAVS_REQUIRE(count >= 0 && count <= kBlockCopies && (count == 0 || blocks), "cavs_copy_blocks: %d blocks, at most %d", count, kBlockCopies);
+  BlockCopies a{};
+  for (int i = 0; i < count; i++) {
+    const cavs_block_copy &b = blocks[i];
+    CAVS_REQUIRE(b.rows >= 0 && b.cols >= 0 && b.ld_dst >= b.cols && b.ld_src >= b.cols, "cavs_copy_blocks: bad shape of block %d: %d x %d", i,
+                 b.rows, b.cols);
+    if (b.rows == 0 || b.cols == 0) continue;
+    CAVS_REQUIRE(b.dst && b.src, "cavs_copy_blocks: null pointer");
+    const long wgs = ((long)b.rows * b.cols + kBlockElems - 1) / kBlockElems;
+    CAVS_REQUIRE(a.first[a.count] + wgs < (1L << 30), "cavs_copy_blocks: too many elements");
+    a.b[a.count] = b;
+    a.first[a.count + 1] = a.first[a.count] + (int)wgs;
+    a.count++;
+  }
+  if (a.count == 0) return CAVS_OK;
+  launch(copy_blocks_kernel, (unsigned)a.first[a.count], 256, 0, as_stream(stream), a);
+  CAVS_LAUNCH_CHECK();
+  return CAVS_OK;
+}
 
 int cavs_gather_rows(float *out, int ld_out, const float *src, int ld_src, const int *ids, int n,
                      int w, void *stream) {

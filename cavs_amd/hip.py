@@ -42,6 +42,11 @@ class GemmDesc(C.Structure):
                 ("zero_kind", _I), ("zero_rows", _I), ("zero_col", _I)]
 
 
+class BlockCopy(C.Structure):
+    """cavs_block_copy: one block of cavs_copy_blocks"""
+    _fields_ = [("dst", _P), ("src", _P), ("ld_dst", C.c_longlong), ("ld_src", C.c_longlong), ("rows", _I), ("cols", _I)]
+
+
 GEMM_C_UNUSED, GEMM_A_ZERO, GEMM_B_ZERO = 1, 2, 3
 
 
@@ -75,6 +80,7 @@ _SIGS = {
     "cavs_scatter_rows": [_P, _I, _P, _P, _I, _I, _I, _P],
     "cavs_zero_rows": [_P, _I, _I, _I, _P],
     "cavs_copy_rows": [_P, _I, _P, _I, _I, _I, _P],
+    "cavs_copy_blocks": [_I, C.POINTER(BlockCopy), _P],
     "cavs_add_rows": [_P, _I, _P, _I, _I, _I, _P],
     "cavs_gather_children": [_P, _P, _P, _P, _I, _I, _I, _P],
     "cavs_sgemm": [_I, _I, _I, _I, _I, _F, _P, _I, _P, _I, _F, _P, _I, _P],

@@ -18,6 +18,14 @@
 
 namespace cavs {
 
+// One block of a parameter that is stored wider than it is declared (hidden sizes that are no multiple
+// of a tile): `rows` rows of `cols` elements at `user` (row stride ld_user) of the declared layout
+// are those at `eng` (row stride ld_eng) of the stored one, whose other elements are zero.
+struct PadBlock {
+  size_t user, ld_user, eng, ld_eng;
+  int rows, cols;
+};
+
 struct CellParamRef {
   int param = -1;    // index into CellSpec::params
   long offset = 0;   // first element of the view inside that parameter
@@ -50,10 +58,13 @@ struct CellBias {
 
 struct CellParam {
   std::string name;  // engine parameter ("Emb" for the embedding table, else "P<i>")
-  long size = 0;
+  long size = 0;     // elements as the kernels read it
+  long declared = 0; // elements as declared
+  std::vector<PadBlock> blocks;  // how the two correspond (empty: they are the same)
 };
 
 struct CellSpec {
+  int uH = 0;                   // hidden size as declared; H is the next multiple of 32
   int H = 0, K = 0, S = 0;      // block width, children per vertex, state blocks of the message it writes
   int SI = 0;                   // state blocks of the rows it gathers (the children's messages; = S for a function of one stage)
   int E = 0, V = 0, NX = 0;     // embedding width, vocabulary, blocks of x * W (0: F looks no vertex input up)

@@ -33,12 +33,13 @@ Engine::Engine(const cavs_session_config &cfg, void *external_stream, std::share
   own_stream_ = external_stream == nullptr;
   E_ = cfg.model == CAVS_MODEL_LSTM ? cfg.H : cfg.E;  // the chain LSTM requires E == H
   pad_sizes();
+  if (cell_) cfg_.H = cell_->H;
   const size_t H = cfg_.H, h = uH_, e = uE_;
   ld_e_ = cfg.model == CAVS_MODEL_TREELSTM ? E_ + 4 : E_;
   mw_ = cfg.model == CAVS_MODEL_TREEFC ? H : 2 * H;
   nch_ = cfg.model == CAVS_MODEL_LSTM ? 1 : 2;
   if (cell_) {
-    if (cell_->H != cfg.H || cell_->K < 1 || cell_->K > 2 || (int)cell_->params.size() > CA_MAX_PARAMS)
+    if (cell_->uH != cfg.H || cell_->K < 1 || cell_->K > 2 || (int)cell_->params.size() > CA_MAX_PARAMS)
       fail(CAVS_EINVAL, "the description of the lowered vertex function does not fit the session");
     E_ = ld_e_ = cell_->E;
     const CellSpec *tail = cell_.get();
@@ -85,7 +86,7 @@ Engine::Engine(const cavs_session_config &cfg, void *external_stream, std::share
       add_param("Bv", 4 * H, 0, rows(4, h, H));
       break;
     case CAVS_MODEL_CELL:
-      for (const CellParam &p : cell_->params) add_param(p.name, (size_t)p.size);
+      for (const CellParam &p : cell_->params) add_param(p.name, (size_t)p.size, 0, p.blocks, (size_t)p.declared);
       for (std::shared_ptr<const CellSpec> c = cell_; c; c = c->next) {
         cells_.emplace_back();
         cells_.back().spec = c;
@@ -110,12 +111,15 @@ Engine::Engine(const cavs_session_config &cfg, void *external_stream, std::share
 // from the head and from the rounds above every gate gradient and every weight gradient of the
 // column is a product with a zero.  Without it such a size runs a round as six to ten separate launches
 // (Tree-LSTM, H = 150, 25 trees: 0.78 ms per step, 0.24 padded).
-// Not for a caller's own tensors (their layout is the caller's), not where no fused round runs.
+// A caller's own tensors (bind_param) keep their layout: they are copied block by block into the stored
+// one when a forward pass begins, and the gradients back when a backward pass ends; the embedding
+// table, of which a pass reads a few rows, is not worth copying and stays as it is.
 void Engine::pad_sizes() {
   uH_ = cfg_.H;
   uE_ = E_;
-  if (!own_stream_ || cell_ || !(cfg_.opt & CAVS_OPT_BATCHING) || cfg_.fused_round_rows < 0) return;
+  if (cell_ || !(cfg_.opt & CAVS_OPT_BATCHING) || cfg_.fused_round_rows < 0) return;
   cfg_.H = (uH_ + 31) / 32 * 32;
+  if (!own_stream_) return;
   // the lookup's row offset is id * E in single precision (EmbeddingLookup): where that is not
   // exact for every id, the rows stay where they are
   if (E_ > 0 && (double)cfg_.V * E_ <= (double)(1 << 24)) E_ = (E_ + 3) / 4 * 4;
@@ -214,12 +218,28 @@ Engine::~Engine() {
   if (own_stream_) cavs_stream_destroy(stream_);
 }
 
-void Engine::add_param(const std::string &name, size_t n, size_t extra_grad, std::vector<PadBlock> blocks) {
+void Engine::block_jobs(const Param &p, float *user, float *stored, bool to_user, std::vector<cavs_block_copy> *jobs) {
+  for (const PadBlock &b : p.blocks) {
+    float *u = user + b.user, *e = stored + b.eng;
+    if (to_user) jobs->push_back({u, e, (long long)b.ld_user, (long long)b.ld_eng, b.rows, b.cols});
+    else jobs->push_back({e, u, (long long)b.ld_eng, (long long)b.ld_user, b.rows, b.cols});
+  }
+}
+
+void Engine::copy_blocks(const std::vector<cavs_block_copy> &jobs) {
+  for (size_t at = 0; at < jobs.size(); at += 32) {
+    check(cavs_copy_blocks((int)std::min<size_t>(32, jobs.size() - at), jobs.data() + at, stream_));
+    c_launches_ += 1;
+  }
+}
+
+void Engine::add_param(const std::string &name, size_t n, size_t extra_grad, std::vector<PadBlock> blocks, size_t declared) {
   auto p = std::make_unique<Param>();
   p->n = p->user_n = n;
   if (!blocks.empty()) {
-    p->user_n = 0;
-    for (const PadBlock &b : blocks) p->user_n += (size_t)b.rows * b.cols;
+    p->user_n = declared;
+    for (const PadBlock &b : blocks)
+      if (declared == 0) p->user_n += (size_t)b.rows * b.cols;
     p->blocks = std::move(blocks);
   }
   p->own_w.reserve(n);
@@ -240,8 +260,17 @@ Param &Engine::param(const std::string &name) {
 void Engine::bind_param(const std::string &name, float *w, float *g) {
   Param &p = param(name);
   if (!w) fail(CAVS_EINVAL, "bind_param('" + name + "'): null weight pointer");
-  if (p.w != w) upk_valid_ = wfct_valid_ = false;
   state_epoch_++;
+  if (!p.blocks.empty()) {
+    p.uw = w;
+    if (!g && p.own_ug.capacity() == 0) {
+      p.own_ug.reserve(p.user_n);
+      check(cavs_zero(p.own_ug.get(), p.user_n * 4, stream_));
+    }
+    p.ug = g ? g : p.own_ug.get();
+    return;
+  }
+  if (p.w != w) upk_valid_ = wfct_valid_ = false;
   p.w = w;
   p.g = g ? g : p.own_g.get();
 }
@@ -281,8 +310,9 @@ void Engine::set_param(const std::string &name, const float *host, size_t n) {
     fail(CAVS_EINVAL, "parameter '" + name + "' has " + std::to_string(p.user_n) + " elements, got " + std::to_string(n));
   if (!p.blocks.empty()) ensure(pad_stage_, n);
   check(cavs_memcpy_h2d(p.blocks.empty() ? p.w : pad_stage_.get(), host, n * 4, stream_));
-  for (const PadBlock &b : p.blocks)
-    check(cavs_copy_rows(p.w + b.eng, (int)b.ld_eng, pad_stage_.at(b.user), (int)b.ld_user, b.rows, b.cols, stream_));
+  std::vector<cavs_block_copy> jobs;
+  block_jobs(p, pad_stage_.get(), p.w, false, &jobs);
+  copy_blocks(jobs);
   check(cavs_stream_sync(stream_));
   upk_valid_ = wfct_valid_ = false;
   state_epoch_++;
@@ -293,11 +323,12 @@ void Engine::get_param(const std::string &name, float *host, size_t n, bool grad
   if (n != p.user_n || !host)
     fail(CAVS_EINVAL, "parameter '" + name + "' has " + std::to_string(p.user_n) + " elements, got " + std::to_string(n));
   aux_join();
-  const float *src = grad ? p.g : p.w;
+  float *src = grad ? p.g : p.w;
   if (!p.blocks.empty()) {
     ensure(pad_stage_, n);
-    for (const PadBlock &b : p.blocks)
-      check(cavs_copy_rows(pad_stage_.at(b.user), (int)b.ld_user, src + b.eng, (int)b.ld_eng, b.rows, b.cols, stream_));
+    std::vector<cavs_block_copy> jobs;
+    block_jobs(p, pad_stage_.get(), src, true, &jobs);
+    copy_blocks(jobs);
     src = pad_stage_.get();
   }
   check(cavs_memcpy_d2h(host, src, n * 4, stream_));
@@ -451,7 +482,7 @@ void Engine::reserve_edges() {
   R(pool_, cap * mw);
   R(dpool_, cap * mw);
   R(GO_, cap * H);
-  R(dGO_, cap * H);
+  if (ensure(dGO_, cap * H) && uH_ != cfg_.H) check(cavs_zero(dGO_.get(), cap * H * 4, stream_));
   R(dret_, cap * H);
   R(G_, cap * nch_ * mw);
   R(r_dmsg_, rc * mw);
@@ -875,11 +906,23 @@ void Engine::forward_only(const int *graph, int B, int maxlen, const float *x_de
   if (reads_x && !x_dev) fail(CAVS_EINVAL, "vertex input feed is null");
   d_x_ = x_dev;
   check(cavs_event_record(ev_[0], stream_));
-  fwd_out_ = graph_out ? graph_out : GO_.get();
+  fwd_out_ = graph_out && uH_ == cfg_.H ? graph_out : GO_.get();
   out_folded_ = false;
   head_chunked_ = false;
+  if (uH_ != cfg_.H) {  // the caller may have written its tensors since the last pass
+    std::vector<cavs_block_copy> jobs;
+    for (auto &kv : params_)
+      if (kv.second->uw) block_jobs(*kv.second, kv.second->uw, kv.second->w, false, &jobs);
+    copy_blocks(jobs);
+    upk_valid_ = false;
+  }
   model_forward();
   pop_ret(fwd_out_);
+  if (uH_ != cfg_.H) {
+    ensure(go_user_, grow((size_t)N_ * uH_, go_user_.capacity()));
+    check(cavs_copy_rows(graph_out ? graph_out : go_user_.get(), uH_, fwd_out_, cfg_.H, N_, uH_, stream_));
+    c_launches_ += 1;
+  }
   check(cavs_event_record(ev_[1], stream_));
   ev_valid_ = true;
   ev_bwd_valid_ = false;
@@ -896,8 +939,26 @@ void Engine::backward_only(const float *dgraph_out, bool settle_biases) {
   d_dgo_ = dgraph_out;
   head_chunked_ = false;
   check(cavs_event_record(ev_[2], stream_));
+  if (uH_ != cfg_.H) {  // (the columns beyond stay zero)
+    check(cavs_copy_rows(dGO_.get(), cfg_.H, dgraph_out, uH_, N_, uH_, stream_));
+    c_launches_ += 1;
+    d_dgo_ = dGO_.get();
+  }
   model_backward();
-  if (settle_biases) settle_bias_jobs(0.f, nullptr);  // no update follows in here: the bias gradients are delivered now
+  // no update follows in here, or not in the stored layout: the bias gradients are delivered now
+  if (settle_biases || uH_ != cfg_.H) settle_bias_jobs(0.f, nullptr);
+  if (uH_ != cfg_.H) {
+    std::vector<cavs_block_copy> jobs;
+    for (auto &kv : params_) {
+      Param &p = *kv.second;
+      if (!p.uw) continue;
+      size_t covered = 0;
+      for (const PadBlock &b : p.blocks) covered += (size_t)b.rows * b.cols;
+      if (covered < p.user_n) check(cavs_zero(p.ug, p.user_n * 4, stream_));  // (what F does not read has no gradient)
+      block_jobs(p, p.ug, p.g, true, &jobs);
+    }
+    copy_blocks(jobs);
+  }
   check(cavs_event_record(ev_[3], stream_));
   ev_bwd_valid_ = true;
 }

@@ -21,19 +21,15 @@
 
 namespace cavs {
 
-// One block of a parameter the engine stores wider than its owner declares it (Engine::pad_sizes):
-// `rows` rows of `cols` elements at `user` (row stride ld_user) of the declared layout are those at
-// `eng` (row stride ld_eng) of the engine's.
-struct PadBlock {
-  size_t user, ld_user, eng, ld_eng;
-  int rows, cols;
-};
-
 struct Param {
   float *w = nullptr, *g = nullptr;  // owned storage below, or bound to a caller's tensors
   DeviceArray<float> own_w, own_g;
   size_t n = 0, user_n = 0;          // elements stored, elements declared
   std::vector<PadBlock> blocks;      // empty: stored as declared
+  // a caller's tensors in the declared layout when the parameter is stored in another: w is filled from
+  // uw when a forward pass begins, ug from g when a backward pass ends
+  float *uw = nullptr, *ug = nullptr;
+  DeviceArray<float> own_ug;
 };
 
 class Engine {
@@ -47,20 +43,29 @@ class Engine {
   // end's Variable tensors) instead of the engine's own copies.  g may be null: then the
   // engine keeps the gradient in its own buffer (read it with grad_ptr()).
   void bind_param(const std::string &name, float *w, float *g);
+  // somebody else has written bound weights: no copy of them is current
+  void weights_written() {
+    upk_valid_ = wfct_valid_ = false;
+    state_epoch_++;
+  }
   // where the next backward pass leaves the gradient of `name` (null: the engine's own buffer)
   void bind_param_grad(const std::string &name, float *g) {
     state_epoch_++;
     Param &p = param(name);
-    p.g = g ? g : p.own_g.get();
+    if (!p.blocks.empty()) p.ug = g ? g : p.own_ug.get();
+    else p.g = g ? g : p.own_g.get();
   }
-  const float *grad_ptr(const std::string &name) { return param(name).g; }
+  const float *grad_ptr(const std::string &name) {
+    const Param &p = param(name);
+    return p.blocks.empty() ? p.g : p.ug;
+  }
   // For a caller that applies w -= lr * g to bound parameters itself (the front end's optimizer):
   // when w is the recurrent weights whose tile-major copy the forward rounds read, appends the
   // jobs of a cavs_run_tasks launch that update them and the copy together and returns true --
   // the copy then counts as current until the parameter is bound elsewhere; otherwise false, and
   // the caller's plain update will do.  Such a caller must route every write of w through here.
   bool update_jobs(float *w, float *g, float lr, std::vector<cavs_task> *out);
-  float *graph_out_ptr() const { return GO_.get(); }
+  float *graph_out_ptr() const { return uH_ == cfg_.H ? GO_.get() : go_user_.get(); }
   // The two halves of step() for a caller that runs the loss head itself: forward F into
   // graph_out [N,H] (vertex order), then backward F from d graph_out.
   void forward_only(const int *graph, int B, int maxlen, const float *x_dev, float *graph_out);
@@ -98,8 +103,10 @@ class Engine {
 
  private:
   Param &param(const std::string &name);
-  void add_param(const std::string &name, size_t n, size_t extra_grad = 0, std::vector<PadBlock> blocks = {});
+  void add_param(const std::string &name, size_t n, size_t extra_grad = 0, std::vector<PadBlock> blocks = {}, size_t declared = 0);
   void pad_sizes();
+  void copy_blocks(const std::vector<cavs_block_copy> &jobs);
+  static void block_jobs(const Param &p, float *user, float *stored, bool to_user, std::vector<cavs_block_copy> *jobs);
   // device rows [n, uH per block] of `src`, whose rows are blocks of the stored width H: where the
   // declared width differs, packed to it in the staging buffer
   const float *user_rows(const float *src, size_t n, int blocks);
@@ -155,6 +162,7 @@ class Engine {
   cavs_session_config cfg_;       // (cfg_.H: the hidden size the kernels run at)
   int uH_ = 0, uE_ = 0;           // hidden and embedding size as declared
   DeviceArray<float> pad_stage_;  // parameters and results on their way between the two layouts
+  DeviceArray<float> go_user_;    // [N, uH] what forward_only returns, in the declared width
   DeviceArray<float> pad_mask_;   // [H] 1 where a column is declared, 0 where it is padding
   void *stream_ = nullptr;
   bool own_stream_ = true;

@@ -107,7 +107,7 @@ struct Reader : Body {
     if (!ve) no("no Variable edge " + r.var);
     CellParam p;
     p.name = embedding ? "Emb" : "P" + std::to_string(spec.params.size());
-    p.size = ve->width();
+    p.size = p.declared = ve->width();
     spec.params.push_back(p);
     if ((int)spec.params.size() > CA_MAX_PARAMS) no("more than " + std::to_string(CA_MAX_PARAMS) + " Variables");
     return param_of[r.var] = (int)spec.params.size() - 1;
@@ -197,8 +197,8 @@ struct Reader : Body {
       scatters += n->def.name() == "Scatter";
     }
     if (pushes != 1 || scatters != 1) no("F must end in one Scatter and one Push");
-    if (s.H <= 0 || s.H % 32) no("the pushed value's width is not a multiple of 32");
-    const int H = s.H;
+    if (s.H <= 0) no("the pushed value has no width");
+    const int H = s.uH = s.H;
     for (auto &np : func->nodes) {
       const Node *n = np.get();
       const OpDef &d = n->def;
@@ -528,7 +528,8 @@ struct Writer {
 
   void kernels() {
     const int H = s.H, NT = s.terms(), NP = (int)s.products.size(), NA = (int)s.asrc.size();
-    o << "#define CELL_H " << H << "\n#define CELL_K " << s.K << "\n#define CELL_S " << s.S << "\n#define CELL_MW " << s.S * H
+    if (s.uH != H) o << "// hidden size " << s.uH << ", stored as " << H << " columns (the next multiple of 32)\n";
+    o << "#define CELL_UH " << s.uH << "\n#define CELL_H " << H << "\n#define CELL_K " << s.K << "\n#define CELL_S " << s.S << "\n#define CELL_MW " << s.S * H
       << "\n#define CELL_SI " << s.SI << "\n#define CELL_MWI " << s.SI * H << "\n#define CELL_HAS_RET " << (s.has_ret ? 1 : 0)
       << "\n#define CELL_NX " << s.NX << "\n#define CELL_XD " << s.XD << "\n#define CELL_NP " << NP << "\n#define CELL_NA " << NA << "\n#define CELL_NT " << NT
       << "\n#define CELL_ND " << s.ND << "\n#define CELL_NSV " << s.NSV << "\n#define CELL_KS " << s.waves << "\n#define CELL_DS_MASK "
@@ -730,6 +731,7 @@ struct Chain {
       CellSpec &cs = c.spec;
       const CellSpec &rs = reader.spec;
       cs.H = rs.H;
+      cs.uH = rs.uH;
       cs.E = rs.E;
       cs.V = rs.V;
       cs.NX = rs.NX;
@@ -818,6 +820,75 @@ struct Chain {
       nfwd.push_back((int)c.dag.n.size());
       derived.push_back(derive(c));
     }
+    pad();
+  }
+
+  // A hidden size that is no multiple of 32 runs at the next one.  Every view of a parameter that F
+  // reads -- the right operand of a MatMul, a block of biases -- gets a place of its own in the stored
+  // parameter, its H-wide blocks spread to whole tiles; the views the cells refer to are
+  // renamed accordingly.  (Two views that overlap without being the same would each need their
+  // gradient added into the other's: not of this shape.)
+  void pad() {
+    CellSpec &rs = reader.spec;
+    const long h = rs.H, H = (h + 31) / 32 * 32;
+    if (h == H) return;
+    struct View {
+      int param;
+      long at, ld, rows;  // as declared: `rows` rows of ld elements
+      long eng;
+    };
+    std::vector<View> views;
+    auto note = [&](int param, long at, long ld, long rows) {
+      for (View &v : views)
+        if (v.param == param && v.at == at && v.ld == ld) {
+          v.rows = std::max(v.rows, rows);
+          return;
+        }
+      views.push_back({param, at, ld, rows, 0});
+    };
+    if (rs.NX > 0) note(rs.W.param, rs.W.offset, rs.NX * h, rs.E);
+    for (const Body &c : cells) {
+      for (const CellProduct &p : c.spec.products)
+        for (const CellTerm &t : p.terms) note(p.B.param, p.B.offset, p.ldb, t.brow + h);
+      for (const CellBias &b : c.spec.biases) note(b.ref.param, b.ref.offset, h, 1);
+    }
+    std::vector<CellParam> params = rs.params;
+    for (size_t i = 0; i < views.size(); i++) {
+      View &v = views[i];
+      CellParam &p = params[v.param];
+      if (p.name == "Emb") no("the embedding table is used as a weight");
+      for (size_t k = 0; k < i; k++)
+        if (views[k].param == v.param && views[k].at < v.at + v.rows * v.ld && v.at < views[k].at + views[k].rows * views[k].ld)
+          no("overlapping views of one Variable at a hidden size that is not a multiple of 32");
+      if (p.blocks.empty()) p.size = 0;
+      v.eng = p.size;
+      // (the rows of x * W's right operand are the embedding's, the others come h at a time)
+      const bool xw = rs.NX > 0 && v.param == rs.W.param && v.at == rs.W.offset && v.ld == rs.NX * h;
+      const long br = xw || v.rows == 1 ? v.rows : h, ld = v.ld / h * H;
+      for (long r = 0; r < v.rows; r += br)
+        for (long c = 0; c < v.ld; c += h)
+          p.blocks.push_back({(size_t)(v.at + r * v.ld + c), (size_t)v.ld, (size_t)(v.eng + r / br * (br == h ? H : 0) * ld + c / h * H), (size_t)ld,
+                              (int)br, (int)h});
+      p.size += (br == h ? v.rows / h * H : v.rows) * ld;
+    }
+    auto place = [&](const CellParamRef &ref, long ld) {
+      for (const View &v : views)
+        if (v.param == ref.param && v.at == ref.offset && v.ld == ld) return v.eng;
+      no("internal: a view without a place");
+    };
+    auto rename = [&](CellSpec &s) {
+      if (s.NX > 0) s.W.offset = place(s.W, s.NX * h);
+      for (CellProduct &p : s.products) {
+        p.B.offset = place(p.B, p.ldb);
+        p.ldb = (int)(p.ldb / h * H);
+        p.col = p.col / h * H;
+        for (CellTerm &t : p.terms) t.brow = t.brow / h * H;
+      }
+      for (CellBias &b : s.biases) b.ref.offset = place(b.ref, h);
+      s.params = params;
+      s.H = (int)H;
+    };
+    for (Body &c : cells) rename(c.spec);
   }
 };
 

@@ -90,6 +90,7 @@ void Executor::set_variable(const std::string &name, const float *data, size_t n
   if (t) {
     check(cavs_memcpy_h2d(t->base, data, n * 4, stream_));
     check(cavs_stream_sync(stream_));
+    if (engine_) engine_->weights_written();
   }
 }
 

@@ -243,7 +243,7 @@ std::unique_ptr<Lowering> match_vertex_function(const Graph &g, int mode) {
   if (!m) return nullptr;
   auto lw = std::make_unique<Lowering>();
   lw->model = CAVS_MODEL_CELL;
-  lw->H = m->spec->H;
+  lw->H = m->spec->uH;
   lw->E = m->spec->E;
   lw->V = m->spec->V;
   lw->use_x = m->spec->NX > 0 || m->spec->XD > 0;

@@ -106,6 +106,15 @@ int cavs_zero_rows(float *out, int ld_out, int n, int w, void *stream);
 /* out[b, 0:w] = inp[b, 0:w]  (Push, Slice, Concat: column blocks via ld) */
 int cavs_copy_rows(float *out, int ld_out, const float *inp, int ld_inp, int n, int w,
                    void *stream);
+/* Up to 32 such copies in one launch, to and from disjoint places (a parameter's blocks between the
+ * layout it is declared in and one with rows and columns added up to whole tiles). */
+typedef struct {
+  float *dst;
+  const float *src;
+  long long ld_dst, ld_src;
+  int rows, cols;
+} cavs_block_copy;
+int cavs_copy_blocks(int count, const cavs_block_copy *blocks, void *stream);
 /* out[b, 0:w] += inp[b, 0:w]: PartialAccumulate, the gradient of Slice
  * (BinaryStridedKernel, cavs/backend/op_impl_elementwise.cuh:141-150;
  * cavs/backend/op_impl_elementwise_common.h:97-122) */

@@ -229,3 +229,39 @@ def test_training_steps_of_a_chain_of_cells_over_changing_batches(model):
     for k in NAMES[model]:
         close(a.grad(k, p[k].shape, grad=False), p[k], f"{k} after 3 steps")
     a.close()
+
+
+@pytest.mark.parametrize("H", [31, 40])
+@pytest.mark.parametrize("model", ["treelstm", "lstm", "treefc_x", "treelstm2", "treegate", "treegru", "treedeep", "cell39", "cell65539"])
+def test_hidden_sizes_that_are_no_multiple_of_a_tile(model, H):
+    """Lowered, such a function runs at the next multiple of 32 on copies of its parameters: two SGD
+    steps against the same program run operator by operator, and a parameter set in between."""
+    base = {"treefc_x": "treefc"}.get(model, "lstm" if model == "lstm" else "treelstm")
+    E, V, C_ = (H if model == "lstm" else 13), 29, 5
+    w = small_workload(base, 331, B=6, H=H, E=E, V=V, C=C_)
+    B, maxlen = w["graph"].shape
+    rng = synth.SplitMix64(9)
+    p, res = {}, {}
+    for mode in (1, 2, 0):
+        a = apps.App(model, B=B, maxlen=maxlen, H=H, E=E, V=V, C_=C_, opt=session.OPT_BATCHING, lr=0.05, pairing="rowid", allow_fused=mode)
+        if not p:
+            p = {k: rng.bulk_uniform(a.var_size(k), -0.2, 0.2) for k in (("W", "Bv") if base == "treefc" else ("Emb", "W", "U", "Bv"))
+                 if not (k == "U" and model == "lstm")}
+            if base != "treefc":
+                p["Wfc"], p["bfc"] = w["params"]["Wfc"], w["params"]["bfc"]
+        a.set_params(p)
+        kw = dict(root_mask=np.ones((w["N"], H), np.float32)) if base == "treefc" else {}
+        print(f"[case] {model} H={H} N={w['N']} lowering mode={mode}", flush=True)
+        got = []
+        for step in range(2):
+            loss, go = a.step(w["graph"], w["x"], w["labels"], train=True, **kw)
+            got.append((loss, go, {"d" + k: a.grad(k, (np.size(v),)) for k, v in p.items()}))
+        assert bool(a.fused_kind) == bool(mode)
+        a.set_params({"W": 0.5 * p["W"]})
+        loss, go = a.step(w["graph"], w["x"], w["labels"], train=True, **kw)
+        got.append((loss, go, {"W": a.grad("W", (np.size(p["W"]),), grad=False)}))
+        res[mode] = got
+        a.close()
+    for mode in (1, 2):
+        for got, want in zip(res[mode], res[0]):
+            compare((*got, 2), dict(loss=want[0], graph_out=want[1], grads=want[2]))
