@@ -117,7 +117,7 @@ class App:
 
     def grad(self, name, shape, grad=True):
         a, _ = libs()
-        out = np.zeros(shape, np.float32)
+        out = np.empty(shape, np.float32)
         n = a.cavs_app_read_param(name.encode(), int(grad), out.ctypes.data, out.size)
         if n != out.size:
             raise hip.CavsError(f"read_param({name}) -> {n}, expected {out.size}")

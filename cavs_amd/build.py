@@ -22,7 +22,7 @@ HIP_FLAGS = ["-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17", "-I", os.pat
              # packed fp32 math is disabled on this target by policy
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 CXX = os.environ.get("CXX", "g++")
-CXX_FLAGS = ["-O2", "-fPIC", "-std=c++17", "-Wall", "-Wextra", "-Wno-unused-parameter", "-Wno-missing-field-initializers", "-I",
+CXX_FLAGS = ["-O2", "-fPIC", "-pthread", "-std=c++17", "-Wall", "-Wextra", "-Wno-unused-parameter", "-Wno-missing-field-initializers", "-I",
              os.path.join(ROOT, "include"), "-I", HOST]
 
 
@@ -56,7 +56,7 @@ def build_host():
     objs = [os.path.join(OBJ, "host_" + os.path.relpath(s, HOST).replace(os.sep, "_")[:-3] + ".o") for s in srcs]
     with ThreadPoolExecutor(max_workers=8) as ex:
         list(ex.map(lambda so: _run([CXX] + CXX_FLAGS + ["-c", so[0], "-o", so[1]]), zip(srcs, objs)))
-    _run([CXX, "-shared", "-o", HOST_SO] + objs + ["-L", LIB, "-lcavs_hip", "-Wl,-rpath,$ORIGIN"])
+    _run([CXX, "-shared", "-pthread", "-o", HOST_SO] + objs + ["-L", LIB, "-lcavs_hip", "-Wl,-rpath,$ORIGIN"])
     # the benchmark applications written against the front end (a user-side program)
     apps = sorted(glob.glob(os.path.join(HOST, "apps", "*.cc")))
     if apps:

@@ -555,10 +555,10 @@ long cavs_app_read_param(const char *name, int grad, float *out, size_t cap) {
   for (auto &v : g_app->vars)
     if (v.first == name) {
       try {
-        vector<float> t = g_app->sess->Read(v.second.output(0) + (grad ? "_grad" : ""));
-        if (t.size() > cap) return -(long)t.size();
-        std::memcpy(out, t.data(), t.size() * 4);
-        return (long)t.size();
+        const std::string edge = v.second.output(0) + (grad ? "_grad" : "");
+        const long n = C_ReadTensor(g_app->sess->handle(), edge.c_str(), out, cap);
+        if (n == 0) throw std::runtime_error("no tensor named " + edge);
+        return n;
       } catch (const std::exception &e) {
         std::fprintf(stderr, "cavs_app_read_param: %s\n", e.what());
         return -2;

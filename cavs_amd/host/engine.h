@@ -17,6 +17,7 @@
 #include "cavs_session.h"
 #include "cell.h"
 #include "device.h"
+#include "readback.h"
 #include "scheduler.h"
 
 namespace cavs {
@@ -159,6 +160,7 @@ class Engine {
   std::vector<void *> prof_events_;
   size_t prof_used_ = 0;
 
+  Readback readback_;
   cavs_session_config cfg_;       // (cfg_.H: the hidden size the kernels run at)
   int uH_ = 0, uE_ = 0;           // hidden and embedding size as declared
   DeviceArray<float> pad_stage_;  // parameters and results on their way between the two layouts

@@ -921,8 +921,7 @@ long Executor::read_tensor(const std::string &name, float *out, size_t cap) {
   if (e && e->src && e->src->def.name() == "Placeholder" && e->src->def.device() == CPU) return 0;
   size_t n = t->count();
   if (!out || cap < n) return -(long)n;
-  check(cavs_memcpy_d2h(out, t->base, n * 4, stream_));
-  check(cavs_stream_sync(stream_));
+  readback_.read(out, t->base, n * 4, stream_);
   if (engine_) engine_->tail_check();
   return (long)n;
 }

@@ -114,6 +114,7 @@ class Executor {
   int nch_ = 0;          // Gather children used by F
   long pool_w_ = 0, ret_w_ = 0, arg_w_ = 0;
   DeviceArray<float> pool_, dpool_, ret_, ws_;
+  Readback readback_;
   PinnedArray<int> idx_host_;
   DeviceArray<int> idx_dev_;
   const int *d_t2j_ = nullptr, *d_pair_ = nullptr, *d_child_[2] = {nullptr, nullptr};

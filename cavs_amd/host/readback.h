@@ -1,0 +1,70 @@
+// Device memory to ordinary host memory, for whoever reads parameters, gradients or results back.
+// A plain copy to pageable memory goes through the runtime's own bounce buffer on the calling thread,
+// which also takes the page faults of a freshly allocated destination: 12 GB/s on one MI355X host, where
+// the link does 55.  Here the link fills a small ring of pinned slots and a few threads carry them on,
+// so that copying and first touch of the destination run beside the transfer and beside each other.
+// One ring and one set of threads per process, made by the first large read and gone with the last
+// object that holds them.
+#ifndef CAVS_HOST_READBACK_H_
+#define CAVS_HOST_READBACK_H_
+
+#include <atomic>
+#include <condition_variable>
+#include <cstddef>
+#include <memory>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "device.h"
+
+namespace cavs {
+
+class ReadbackPool {
+ public:
+  static std::shared_ptr<ReadbackPool> shared();
+  ~ReadbackPool();
+  // `events`: one per slot, of the device the stream belongs to
+  void read(char *host, const char *dev, size_t bytes, void *stream, const std::vector<void *> &events);
+  // a megabyte per slot: long enough for the link (19 us), short enough that the last chunk's copy is short
+  static constexpr size_t kSlot = size_t(1) << 20;
+  static constexpr int kSlots = 16;
+
+ private:
+  ReadbackPool();
+  struct Job {
+    char *host = nullptr;
+    size_t bytes = 0;
+    long chunks = 0;
+    const std::vector<void *> *events = nullptr;
+    std::atomic<long> queued{0}, next{0}, done{0};
+    std::atomic<long> slot_done[kSlots];  // chunks of this slot carried on so far
+    std::atomic<bool> failed{false};
+  };
+  void work(Job &j, bool caller);
+  void thread_main();
+
+  std::mutex one_read_;  // the ring serves one read at a time
+  std::mutex m_;
+  std::condition_variable wake_, idle_;
+  Job *job_ = nullptr;   // guarded by m_
+  int inside_ = 0;       // threads that hold job_
+  bool stop_ = false;
+  PinnedArray<char> ring_;
+  std::vector<std::thread> threads_;
+};
+
+// What one engine or executor reads through.
+class Readback {
+ public:
+  ~Readback();
+  // `bytes` of `dev` are at `host` when this returns; waits for what `stream` holds before it.
+  void read(void *host, const void *dev, size_t bytes, void *stream);
+
+ private:
+  std::shared_ptr<ReadbackPool> pool_;
+  std::vector<void *> events_;
+};
+
+}  // namespace cavs
+#endif

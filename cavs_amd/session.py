@@ -202,12 +202,12 @@ class Session:
             _check(lib().cavs_session_set_param(self._h, k.encode(), a.ctypes.data, a.size), f"set_param({k})")
 
     def param(self, name, shape):
-        a = np.zeros(shape, np.float32)
+        a = np.empty(shape, np.float32)
         _check(lib().cavs_session_get_param(self._h, name.encode(), a.ctypes.data, a.size), f"get_param({name})")
         return a
 
     def grad(self, name, shape):
-        a = np.zeros(shape, np.float32)
+        a = np.empty(shape, np.float32)
         _check(lib().cavs_session_get_grad(self._h, name.encode(), a.ctypes.data, a.size), f"get_grad({name})")
         return a
 
@@ -242,7 +242,7 @@ class Session:
         N, H = self.N, self.H
         shape = {"loss": (N if self.loss == "softmax" else 1,), "graph_out": (N, H), "dgraph_out": (N, H),
                  "msg_pool": (N, self.mw)}[what]
-        a = np.zeros(shape, np.float32)
+        a = np.empty(shape, np.float32)
         _check(lib().cavs_session_fetch(self._h, what.encode(), a.ctypes.data, a.size), f"fetch({what})")
         return a
 
