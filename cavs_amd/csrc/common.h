@@ -34,6 +34,26 @@ struct LaunchProbe {
 };
 LaunchProbe &launch_probe();
 
+// Launches whose workgroups wait for each other must not share the device with another such launch: each
+// could hold the CUs the other's missing workgroups need, and both waits would run into their bound.  Two
+// sessions on two streams get there by themselves, so such launches of a process are ordered per
+// device: an object of this kind, alive around the launch, makes `stream` wait for the last one of
+// another stream.  (Inside a graph capture there is nothing to wait for: the graph's launch is ordered.)
+class ResidentOrder {
+ public:
+  explicit ResidentOrder(hipStream_t stream);
+  ~ResidentOrder();
+  int rc() const { return rc_; }
+  static void stream_created(hipStream_t s);
+  static void stream_gone(hipStream_t s);     // about to be destroyed
+  static void capture_begins(hipStream_t s);
+
+ private:
+  hipStream_t stream_;
+  int dev_ = 0, rc_ = 0;
+  bool captured_ = false;
+};
+
 // Every kernel of this library is launched through here.
 template <typename... KArgs, typename... Args>
 inline void launch(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t lds, hipStream_t st, Args &&...args) {

@@ -154,6 +154,45 @@ __device__ inline void treelstm_gates_rows_at(const BwdGatesRowsArgs &a, long id
 }
 
 
+// The gates of one hidden unit of one chain vertex (apps/paper/seq-lstm-cavs.cc:62-86): xw = the unit's four
+// columns of x * W ([i|f|u|o]), v = those of h * W', c_prev = the predecessor's c.
+struct LstmCell {
+  float i, f, u, o, tc, h, c;
+};
+__device__ inline LstmCell lstm_cell(const float (&xw)[4], const float (&v)[4], const float (&bias)[4], float c_prev) {
+  LstmCell q;
+  q.i = sigm_r((xw[0] + v[0]) + bias[0]);
+  q.f = sigm_r((xw[1] + v[1]) + bias[1]);
+  q.u = tanh_r((xw[2] + v[2]) + bias[2]);
+  q.o = sigm_r((xw[3] + v[3]) + bias[3]);
+  q.c = q.i * q.u + q.f * c_prev;
+  q.tc = tanh_r(q.c);
+  q.h = q.o * q.tc;
+  return q;
+}
+
+// Gate gradients of one hidden unit of one chain vertex.  mh, mc: gradient of its message
+// ([h|c] halves); dr: gradient of its pushed return value; cprev: the predecessor's c (zero at
+// the first step).
+struct LstmGateGrad {
+  float di, df, du, d_o, dc;
+};
+__device__ inline LstmGateGrad lstm_gate_grad(float i, float f, float u, float o, float tc, float mh, float mc, float dr,
+                                              float cprev) {
+  LstmGateGrad g;
+  const float dh = mh + dr;
+  const float d_o = dh * tc;
+  const float dc = mc + (dh * o) * (1.f - tc * tc);
+  g.di = (dc * u) * (i * (1.f - i));
+  g.df = (dc * cprev) * (f * (1.f - f));
+  g.du = (dc * i) * (1.f - u * u);
+  g.d_o = d_o * (o * (1.f - o));
+  g.dc = dc;
+  return g;
+}
+__device__ inline float treefc_dz(float dh, float y, int act) { return act ? dh * (1.f - y * y) : (y > 0.f ? dh : 0.f); }
+
+
 // Parks the per-wavefront partial tiles of NP products in LDS as
 // [region][row tile][product][accumulator element][lane].  There are NREG regions: the
 // wavefronts with k-split index below NREG write theirs, the others add onto region

@@ -273,19 +273,13 @@ __global__ __launch_bounds__(WAVES * 64) void lstm_round_fwd_kernel(LstmFwdArgs 
     sum_regions<NP, NR, NREG>(v, red, el.lds[q], RSZ);
     const int b = el.b[q], j = el.j[q];
     // same association as the separate path: (x*W + h*W') + bias
-    const float i = sigm_r((exw[q][0] + v[0]) + ebias[q][0]);
-    const float f = sigm_r((exw[q][1] + v[1]) + ebias[q][1]);
-    const float u = tanh_r((exw[q][2] + v[2]) + ebias[q][2]);
-    const float o = sigm_r((exw[q][3] + v[3]) + ebias[q][3]);
-    const float c = i * u + f * ecprev[q];
-    const float tc = tanh_r(c);
-    const float h = o * tc;
+    const LstmCell k = lstm_cell(exw[q], v, ebias[q], ecprev[q]);
     float *g = a.gates + (long)b * 5 * H + j;
-    g[0] = i; g[H] = f; g[2 * H] = u; g[3 * H] = o; g[4 * H] = tc;
+    g[0] = k.i; g[H] = k.f; g[2 * H] = k.u; g[3 * H] = k.o; g[4 * H] = k.tc;
     float *m = a.msg + b * H2 + j;
-    m[0] = h; m[H] = c;
-    if (edst[q] >= 0) { a.pool_out[edst[q] * H2 + j] = h; a.pool_out[edst[q] * H2 + H + j] = c; }
-    if (eout[q] >= 0) a.go[(long)eout[q] * H + j] = h;
+    m[0] = k.h; m[H] = k.c;
+    if (edst[q] >= 0) { a.pool_out[edst[q] * H2 + j] = k.h; a.pool_out[edst[q] * H2 + H + j] = k.c; }
+    if (eout[q] >= 0) a.go[(long)eout[q] * H + j] = k.h;
     float *gp = a.G + b * H2 + j;
     gp[0] = ehp[q]; gp[H] = ecprev[q];
   }
@@ -330,27 +324,6 @@ __global__ void lstm_round_leaves_fwd_kernel(LstmLeavesArgs a) {
   if (dst >= 0) { stw<W>(a.pool + dst * H2 + j, mh); stw<W>(a.pool + dst * H2 + H + j, mc); }
   if (out >= 0) stw<W>(a.go + (long)out * H + j, mh);
 }
-
-// Gate gradients of one hidden unit of one chain vertex.  mh, mc: gradient of its message
-// ([h|c] halves); dr: gradient of its pushed return value; cprev: the predecessor's c (zero at
-// the first step).
-struct LstmGateGrad {
-  float di, df, du, d_o, dc;
-};
-__device__ inline LstmGateGrad lstm_gate_grad(float i, float f, float u, float o, float tc, float mh, float mc, float dr,
-                                              float cprev) {
-  LstmGateGrad g;
-  const float dh = mh + dr;
-  const float d_o = dh * tc;
-  const float dc = mc + (dh * o) * (1.f - tc * tc);
-  g.di = (dc * u) * (i * (1.f - i));
-  g.df = (dc * cprev) * (f * (1.f - f));
-  g.du = (dc * i) * (1.f - u * u);
-  g.d_o = d_o * (o * (1.f - o));
-  g.dc = dc;
-  return g;
-}
-__device__ inline float treefc_dz(float dh, float y, int act) { return act ? dh * (1.f - y * y) : (y > 0.f ? dh : 0.f); }
 
 struct LstmBwdGatesArgs {
   const float *dpool;

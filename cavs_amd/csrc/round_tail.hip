@@ -26,7 +26,7 @@
 // / treelstm_round_bwd_children_kernel with ROWS4): the same MFMAs on the same operands in the
 // same order, the same order of sums, the same gate function -- and a row's result does not
 // depend on which rows share its tile -- so the results equal the per-round launches' bit for bit.
-#include "round_common.h"
+#include "round_sync.h"
 
 namespace cavs {
 
@@ -48,227 +48,6 @@ struct TailPlan {
   int start[kTailGroups][kTailMaxRounds];
   short count[kTailGroups][kTailMaxRounds], flags[kTailGroups][kTailMaxRounds];
 };
-
-// The sync block: word 1 = status (all groups); group g owns the 32 words from 32 (g + 1): arrivals,
-// then the XCDs its workgroups saw (bit mask).  A cache line per group: they live in different L2s.
-enum { TAIL_STATUS = 1, TAIL_GROUP_WORDS = 32, TAIL_ARRIVALS = 0, TAIL_XCC = 1 };
-
-__device__ inline int xcc_id() { return __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11)) & 15; }  // HW_REG_XCC_ID[3:0]
-
-// This workgroup's results of a round are written: tell the others of the group.  The last
-// arrival of the launch leaves the group's words as the next launch expects them.
-__device__ inline void tail_arrive(unsigned *gsync, unsigned total) {
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stores are acknowledged by the L2
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const unsigned old = __hip_atomic_fetch_add(gsync + TAIL_ARRIVALS, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (old + 1 == total) {
-      __hip_atomic_store(gsync + TAIL_XCC, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(gsync + TAIL_ARRIVALS, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
-}
-
-// Waits until `target` arrivals of the group are in.  False when the wait gave up (spin_max polls,
-// or another workgroup already did, or the group's workgroups turned out to sit on more than one
-// XCD): the status word says why and the caller returns.  Ends with a workgroup barrier either way.
-__device__ inline bool tail_wait(unsigned *status, unsigned *gsync, unsigned target, int spin_max, bool check_xcc, int *s_bail) {
-  if (threadIdx.x == 0) {
-    int bail = 0, tries = 0;
-    while (__hip_atomic_load(gsync + TAIL_ARRIVALS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-      if (++tries > spin_max) {
-        __hip_atomic_store(status, (unsigned)CAVS_TAIL_TIMEOUT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        bail = 1;
-        break;
-      }
-      if ((tries & 15) == 0 && __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-        bail = 1;
-        break;
-      }
-    }
-    if (!bail && check_xcc) {
-      const unsigned seen = __hip_atomic_load(gsync + TAIL_XCC, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (seen & (seen - 1)) {  // more than one XCD: the L2 is not shared, nothing read here can be trusted
-        __hip_atomic_store(status, (unsigned)CAVS_TAIL_SPREAD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        bail = 1;
-      }
-    }
-    *s_bail = bail;
-  }
-  __syncthreads();
-  asm volatile("buffer_inv sc0" ::: "memory");  // nothing this CU cached before the barrier is used after it
-  return *s_bail == 0;
-}
-
-// A row another workgroup of the group wrote in an earlier round.  No line of such a row can be in
-// this CU's L1 when the load is issued: the L1 starts a kernel empty, rows are whole cache lines,
-// and a row is first read after the barrier that follows its round (tail_wait also invalidates
-// the L1, for good measure).  So an ordinary load is served by the L2 the writers share.  (Loads
-// that bypass the L1 by scope -- agent-scope atomic loads -- were measured at about sixty cycles per
-// wavefront and access here, one request per lane: three times the MFMA time of a tile.)
-__device__ inline float ld_row(const float *p) { return *p; }
-
-// The four k slots of an element added up across the wavefront, for the four rows of NP products
-// at once: afterwards the lanes of k slot s hold, in r[p][0], the sum of row s of product p --
-// (v[x] + v[x+16]) + (v[x+32] + v[x+48]) with v = that row's accumulator, the order in which the
-// per-round kernels add the slots up.  v_permlane16_swap exchanges the odd 16-lane rows of its first
-// operand with the even rows of its second, v_permlane32_swap the upper half of the first with the
-// lower half of the second; swapping two rows' accumulators and adding puts both partial sums into
-// one register, a butterfly of three swaps and three adds per product on the vector ALU (a shuffle
-// through the LDS crossbar costs eight cycles of a unit all eight wavefronts share).  Spelled out
-// as instructions because the compiler's builtins for the two swaps return the first result twice.
-// The compiler does not look inside such a statement, so the waits an instruction needs after the
-// one that produced its operand are the caller's: all() carries its own (twelve cycles cover the
-// six a two-pass MFMA asks for before a vector-ALU read, two between an add and the swap that reads
-// it); the stages are for callers that put at least that many instructions between them.
-template <int NP>
-struct SlotSums;
-template <>
-struct SlotSums<5> {
-  float r[5][4];
-  __device__ inline void take(const floatx4 (&acc)[5]) {
-#pragma unroll
-    for (int p = 0; p < 5; p++)
-#pragma unroll
-      for (int k = 0; k < 4; k++) r[p][k] = acc[p][k];
-  }
-  // the stages one at a time, for a caller that puts other work (MFMAs of the next tile) between them
-  __device__ inline void stage_a() {
-    asm volatile(
-        "v_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\t"
-        "v_permlane16_swap_b32 %4, %5\n\tv_permlane16_swap_b32 %6, %7\n\t"
-        "v_permlane16_swap_b32 %8, %9\n\tv_permlane16_swap_b32 %10, %11\n\t"
-        "v_permlane16_swap_b32 %12, %13\n\tv_permlane16_swap_b32 %14, %15\n\t"
-        "v_permlane16_swap_b32 %16, %17\n\tv_permlane16_swap_b32 %18, %19"
-        : "+v"(r[0][0]), "+v"(r[0][1]), "+v"(r[0][2]), "+v"(r[0][3]), "+v"(r[1][0]), "+v"(r[1][1]), "+v"(r[1][2]), "+v"(r[1][3]), "+v"(r[2][0]), "+v"(r[2][1]), "+v"(r[2][2]), "+v"(r[2][3]), "+v"(r[3][0]), "+v"(r[3][1]), "+v"(r[3][2]), "+v"(r[3][3]), "+v"(r[4][0]), "+v"(r[4][1]), "+v"(r[4][2]), "+v"(r[4][3]));
-  }
-  __device__ inline void stage_b() {
-    asm volatile(
-        "v_add_f32 %0, %0, %1\n\tv_add_f32 %2, %2, %3\n\t"
-        "v_add_f32 %4, %4, %5\n\tv_add_f32 %6, %6, %7\n\t"
-        "v_add_f32 %8, %8, %9\n\tv_add_f32 %10, %10, %11\n\t"
-        "v_add_f32 %12, %12, %13\n\tv_add_f32 %14, %14, %15\n\t"
-        "v_add_f32 %16, %16, %17\n\tv_add_f32 %18, %18, %19"
-        : "+v"(r[0][0]), "+v"(r[0][1]), "+v"(r[0][2]), "+v"(r[0][3]), "+v"(r[1][0]), "+v"(r[1][1]), "+v"(r[1][2]), "+v"(r[1][3]), "+v"(r[2][0]), "+v"(r[2][1]), "+v"(r[2][2]), "+v"(r[2][3]), "+v"(r[3][0]), "+v"(r[3][1]), "+v"(r[3][2]), "+v"(r[3][3]), "+v"(r[4][0]), "+v"(r[4][1]), "+v"(r[4][2]), "+v"(r[4][3]));
-  }
-  __device__ inline void stage_c() {
-    asm volatile(
-        "v_permlane32_swap_b32 %0, %2\n\t"
-        "v_permlane32_swap_b32 %4, %6\n\t"
-        "v_permlane32_swap_b32 %8, %10\n\t"
-        "v_permlane32_swap_b32 %12, %14\n\t"
-        "v_permlane32_swap_b32 %16, %18"
-        : "+v"(r[0][0]), "+v"(r[0][1]), "+v"(r[0][2]), "+v"(r[0][3]), "+v"(r[1][0]), "+v"(r[1][1]), "+v"(r[1][2]), "+v"(r[1][3]), "+v"(r[2][0]), "+v"(r[2][1]), "+v"(r[2][2]), "+v"(r[2][3]), "+v"(r[3][0]), "+v"(r[3][1]), "+v"(r[3][2]), "+v"(r[3][3]), "+v"(r[4][0]), "+v"(r[4][1]), "+v"(r[4][2]), "+v"(r[4][3]));
-  }
-  __device__ inline void stage_d() {
-    asm volatile(
-        "v_add_f32 %0, %0, %2\n\t"
-        "v_add_f32 %4, %4, %6\n\t"
-        "v_add_f32 %8, %8, %10\n\t"
-        "v_add_f32 %12, %12, %14\n\t"
-        "v_add_f32 %16, %16, %18"
-        : "+v"(r[0][0]), "+v"(r[0][1]), "+v"(r[0][2]), "+v"(r[0][3]), "+v"(r[1][0]), "+v"(r[1][1]), "+v"(r[1][2]), "+v"(r[1][3]), "+v"(r[2][0]), "+v"(r[2][1]), "+v"(r[2][2]), "+v"(r[2][3]), "+v"(r[3][0]), "+v"(r[3][1]), "+v"(r[3][2]), "+v"(r[3][3]), "+v"(r[4][0]), "+v"(r[4][1]), "+v"(r[4][2]), "+v"(r[4][3]));
-  }
-  // all of it at once, right after the MFMAs that produced the accumulators
-  __device__ inline void all() {
-    asm volatile(
-      "s_nop 7\n\ts_nop 3\n\t"
-      "v_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\t"
-      "v_permlane16_swap_b32 %4, %5\n\tv_permlane16_swap_b32 %6, %7\n\t"
-      "v_permlane16_swap_b32 %8, %9\n\tv_permlane16_swap_b32 %10, %11\n\t"
-      "v_permlane16_swap_b32 %12, %13\n\tv_permlane16_swap_b32 %14, %15\n\t"
-      "v_permlane16_swap_b32 %16, %17\n\tv_permlane16_swap_b32 %18, %19\n\t"
-      "s_nop 1\n\t"
-      "v_add_f32 %0, %0, %1\n\tv_add_f32 %2, %2, %3\n\t"
-      "v_add_f32 %4, %4, %5\n\tv_add_f32 %6, %6, %7\n\t"
-      "v_add_f32 %8, %8, %9\n\tv_add_f32 %10, %10, %11\n\t"
-      "v_add_f32 %12, %12, %13\n\tv_add_f32 %14, %14, %15\n\t"
-      "v_add_f32 %16, %16, %17\n\tv_add_f32 %18, %18, %19\n\t"
-      "s_nop 1\n\t"
-      "v_permlane32_swap_b32 %0, %2\n\t"
-      "v_permlane32_swap_b32 %4, %6\n\t"
-      "v_permlane32_swap_b32 %8, %10\n\t"
-      "v_permlane32_swap_b32 %12, %14\n\t"
-      "v_permlane32_swap_b32 %16, %18\n\t"
-      "s_nop 1\n\t"
-      "v_add_f32 %0, %0, %2\n\t"
-      "v_add_f32 %4, %4, %6\n\t"
-      "v_add_f32 %8, %8, %10\n\t"
-      "v_add_f32 %12, %12, %14\n\t"
-      "v_add_f32 %16, %16, %18"
-        : "+v"(r[0][0]), "+v"(r[0][1]), "+v"(r[0][2]), "+v"(r[0][3]), "+v"(r[1][0]), "+v"(r[1][1]), "+v"(r[1][2]), "+v"(r[1][3]), "+v"(r[2][0]), "+v"(r[2][1]), "+v"(r[2][2]), "+v"(r[2][3]), "+v"(r[3][0]), "+v"(r[3][1]), "+v"(r[3][2]), "+v"(r[3][3]), "+v"(r[4][0]), "+v"(r[4][1]), "+v"(r[4][2]), "+v"(r[4][3]));
-  }
-};
-template <>
-struct SlotSums<3> {
-  float r[3][4];
-  __device__ inline void take(const floatx4 (&acc)[3]) {
-#pragma unroll
-    for (int p = 0; p < 3; p++)
-#pragma unroll
-      for (int k = 0; k < 4; k++) r[p][k] = acc[p][k];
-  }
-  // the stages one at a time, for a caller that puts other work (MFMAs of the next tile) between them
-  __device__ inline void stage_a() {
-    asm volatile(
-        "v_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\t"
-        "v_permlane16_swap_b32 %4, %5\n\tv_permlane16_swap_b32 %6, %7\n\t"
-        "v_permlane16_swap_b32 %8, %9\n\tv_permlane16_swap_b32 %10, %11"
-        : "+v"(r[0][0]), "+v"(r[0][1]), "+v"(r[0][2]), "+v"(r[0][3]), "+v"(r[1][0]), "+v"(r[1][1]), "+v"(r[1][2]), "+v"(r[1][3]), "+v"(r[2][0]), "+v"(r[2][1]), "+v"(r[2][2]), "+v"(r[2][3]));
-  }
-  __device__ inline void stage_b() {
-    asm volatile(
-        "v_add_f32 %0, %0, %1\n\tv_add_f32 %2, %2, %3\n\t"
-        "v_add_f32 %4, %4, %5\n\tv_add_f32 %6, %6, %7\n\t"
-        "v_add_f32 %8, %8, %9\n\tv_add_f32 %10, %10, %11"
-        : "+v"(r[0][0]), "+v"(r[0][1]), "+v"(r[0][2]), "+v"(r[0][3]), "+v"(r[1][0]), "+v"(r[1][1]), "+v"(r[1][2]), "+v"(r[1][3]), "+v"(r[2][0]), "+v"(r[2][1]), "+v"(r[2][2]), "+v"(r[2][3]));
-  }
-  __device__ inline void stage_c() {
-    asm volatile(
-        "v_permlane32_swap_b32 %0, %2\n\t"
-        "v_permlane32_swap_b32 %4, %6\n\t"
-        "v_permlane32_swap_b32 %8, %10"
-        : "+v"(r[0][0]), "+v"(r[0][1]), "+v"(r[0][2]), "+v"(r[0][3]), "+v"(r[1][0]), "+v"(r[1][1]), "+v"(r[1][2]), "+v"(r[1][3]), "+v"(r[2][0]), "+v"(r[2][1]), "+v"(r[2][2]), "+v"(r[2][3]));
-  }
-  __device__ inline void stage_d() {
-    asm volatile(
-        "v_add_f32 %0, %0, %2\n\t"
-        "v_add_f32 %4, %4, %6\n\t"
-        "v_add_f32 %8, %8, %10"
-        : "+v"(r[0][0]), "+v"(r[0][1]), "+v"(r[0][2]), "+v"(r[0][3]), "+v"(r[1][0]), "+v"(r[1][1]), "+v"(r[1][2]), "+v"(r[1][3]), "+v"(r[2][0]), "+v"(r[2][1]), "+v"(r[2][2]), "+v"(r[2][3]));
-  }
-  // all of it at once, right after the MFMAs that produced the accumulators
-  __device__ inline void all() {
-    asm volatile(
-      "s_nop 7\n\ts_nop 3\n\t"
-      "v_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\t"
-      "v_permlane16_swap_b32 %4, %5\n\tv_permlane16_swap_b32 %6, %7\n\t"
-      "v_permlane16_swap_b32 %8, %9\n\tv_permlane16_swap_b32 %10, %11\n\t"
-      "s_nop 1\n\t"
-      "v_add_f32 %0, %0, %1\n\tv_add_f32 %2, %2, %3\n\t"
-      "v_add_f32 %4, %4, %5\n\tv_add_f32 %6, %6, %7\n\t"
-      "v_add_f32 %8, %8, %9\n\tv_add_f32 %10, %10, %11\n\t"
-      "s_nop 1\n\t"
-      "v_permlane32_swap_b32 %0, %2\n\t"
-      "v_permlane32_swap_b32 %4, %6\n\t"
-      "v_permlane32_swap_b32 %8, %10\n\t"
-      "s_nop 1\n\t"
-      "v_add_f32 %0, %0, %2\n\t"
-      "v_add_f32 %4, %4, %6\n\t"
-      "v_add_f32 %8, %8, %10"
-        : "+v"(r[0][0]), "+v"(r[0][1]), "+v"(r[0][2]), "+v"(r[0][3]), "+v"(r[1][0]), "+v"(r[1][1]), "+v"(r[1][2]), "+v"(r[1][3]), "+v"(r[2][0]), "+v"(r[2][1]), "+v"(r[2][2]), "+v"(r[2][3]));
-  }
-};
-
-// One k-group of four-row tiles is four MFMAs of sixteen 4 x 4 x 1 blocks each; block l / 4 of
-// lane l is (column group (l / 4) % 4, k slot l / 16).  An MFMA can take its A operand, for the four
-// blocks of a k slot, from one of them (A broadcast inside groups of four blocks: CBSZ = 2, ABID =
-// which).  So lane l = 16 slot + 4 j + r fetches ONE float4 per operand row and tile: tile row r at
-// k = 16 j + 4 slot .. + 3 of the wavefront's 64 k -- the wavefront's 64 float4 are the whole
-// 4 x 64 piece of the operand, nothing is fetched twice and nothing crosses lanes -- and the MFMA
-// of k-group g, step c reads component c with ABID = g: the operands the per-round kernels feed the
-// same MFMAs after moving them across lanes.
-#define CAVS_MMA4(acc, a, b, abid) acc = __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, acc, 2, abid, 0)
 
 // ------------------------------------------------------------------ forward
 struct TailFwdArgs {
@@ -804,13 +583,15 @@ extern "C" {
 int cavs_tail_rounds_ok(int n, int H) { return (H == kTailH && n >= 1 && n <= kTailRows) ? 1 : 0; }
 int cavs_tail_max_rounds(void) { return kTailMaxRounds; }
 int cavs_tail_max_groups(void) { return kTailGroups; }
-size_t cavs_tail_sync_bytes(void) { return (size_t)TAIL_GROUP_WORDS * (kTailGroups + 1) * sizeof(unsigned); }
+size_t cavs_tail_sync_bytes(void) { return (size_t)TAIL_GROUP_WORDS * (kSyncGroups + 1) * sizeof(unsigned); }
 
 int cavs_tail_probe(unsigned *sync, int H, int spin_max, void *stream) {
   CAVS_REQUIRE(sync && H == kTailH && spin_max >= 0, "cavs_tail_probe: bad arguments (H = %d only)", kTailH);
   constexpr size_t lds = kTailFwdRed * sizeof(float) + kTailTabBytes;
   static int attr = tail_lds_attr(reinterpret_cast<const void *>(tail_probe_kernel), lds);
   if (attr != CAVS_OK) return attr;
+  ResidentOrder order(as_stream(stream));
+  if (order.rc()) return order.rc();
   launch(tail_probe_kernel, dim3(8 * (H / 16)), 512, lds, as_stream(stream), sync, spin_max, H / 16);
   CAVS_LAUNCH_CHECK();
   return CAVS_OK;
@@ -834,6 +615,8 @@ int cavs_treelstm_tail_fwd(float *pool, const int *child, const int *pair, const
   constexpr size_t lds = kTailFwdRed * sizeof(float) + kTailTabBytes;
   static int attr = tail_lds_attr(reinterpret_cast<const void *>(treelstm_tail_fwd_kernel), lds);
   if (attr != CAVS_OK) return attr;
+  ResidentOrder order(as_stream(stream));
+  if (order.rc()) return order.rc();
   launch(treelstm_tail_fwd_kernel, dim3(8 * (H / 16)), 512, lds, as_stream(stream), a);
   CAVS_LAUNCH_CHECK();
   return CAVS_OK;
@@ -857,6 +640,8 @@ int cavs_treelstm_tail_bwd(float *dxW, int ld_dxw, float *dF, float *dc, const f
   constexpr size_t lds = kTailBwdRed * sizeof(float) + kTailTabBytes;
   static int attr = tail_lds_attr(reinterpret_cast<const void *>(treelstm_tail_bwd_kernel), lds);
   if (attr != CAVS_OK) return attr;
+  ResidentOrder order(as_stream(stream));
+  if (order.rc()) return order.rc();
   launch(treelstm_tail_bwd_kernel, dim3(8 * (H / 16)), 512, lds, as_stream(stream), a);
   CAVS_LAUNCH_CHECK();
   return CAVS_OK;

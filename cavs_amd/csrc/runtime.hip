@@ -2,6 +2,8 @@
 #include "common.h"
 
 #include <cstring>
+#include <mutex>
+#include <set>
 
 namespace cavs {
 
@@ -30,6 +32,79 @@ int num_cus() {
     if (g_cus <= 0) g_cus = 256;
   }
   return g_cus;
+}
+
+namespace {
+constexpr int kOrderDevices = 64;
+struct ResidentState {
+  std::mutex m;                     // held around every ordered launch
+  std::set<hipStream_t> own;        // streams of cavs_stream_create: known to live until stream_gone
+  struct PerDevice {
+    hipStream_t last = nullptr;     // stream of the last ordered launch (null: none, or it is over)
+    hipEvent_t ev = nullptr;
+    bool recorded = false;          // ev stands behind that launch
+  } dev[kOrderDevices];
+};
+ResidentState &resident_state() {
+  static ResidentState *s = new ResidentState;  // (outlives every static destructor)
+  return *s;
+}
+bool mark(ResidentState::PerDevice &d) {
+  if (!d.ev && hipEventCreateWithFlags(&d.ev, hipEventDisableTiming) != hipSuccess) return false;
+  if (hipEventRecord(d.ev, d.last) != hipSuccess) return false;
+  return d.recorded = true;
+}
+}  // namespace
+
+ResidentOrder::ResidentOrder(hipStream_t stream) : stream_(stream) {
+  ResidentState &s = resident_state();
+  s.m.lock();
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipGetDevice(&dev_) != hipSuccess || dev_ < 0 || dev_ >= kOrderDevices) {
+    rc_ = set_error(CAVS_EHIP, "ordering a resident launch: no usable device");
+    return;
+  }
+  captured_ = stream && hipStreamIsCapturing(stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+  if (captured_) return;
+  ResidentState::PerDevice &d = s.dev[dev_];
+  if (!d.last || d.last == stream) return;
+  if ((!d.recorded && !mark(d)) || hipStreamWaitEvent(stream, d.ev, 0) != hipSuccess)
+    rc_ = set_error(CAVS_EHIP, "ordering a resident launch behind another stream's: %s", hipGetErrorString(hipGetLastError()));
+}
+
+ResidentOrder::~ResidentOrder() {
+  ResidentState &s = resident_state();
+  if (rc_ == 0 && !captured_) {
+    ResidentState::PerDevice &d = s.dev[dev_];
+    d.last = stream_;
+    d.recorded = false;
+    if (!s.own.count(stream_)) (void)mark(d);  // a caller's stream may be gone before the next launch asks
+  }
+  s.m.unlock();
+}
+
+void ResidentOrder::stream_created(hipStream_t st) {
+  ResidentState &s = resident_state();
+  std::lock_guard<std::mutex> lock(s.m);
+  s.own.insert(st);
+}
+
+void ResidentOrder::stream_gone(hipStream_t st) {
+  ResidentState &s = resident_state();
+  std::lock_guard<std::mutex> lock(s.m);
+  s.own.erase(st);
+  for (auto &d : s.dev)
+    if (d.last == st) {
+      if (!d.recorded) (void)hipStreamSynchronize(st);
+      d.last = nullptr;
+    }
+}
+
+void ResidentOrder::capture_begins(hipStream_t st) {
+  ResidentState &s = resident_state();
+  std::lock_guard<std::mutex> lock(s.m);
+  for (auto &d : s.dev)
+    if (d.last == st && !d.recorded) (void)mark(d);
 }
 
 __global__ void fill_kernel(float *p, float v, size_t n) {
@@ -162,11 +237,15 @@ int cavs_stream_create(void **stream) {
   hipStream_t s;
   CAVS_HIP_TRY(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
   *stream = s;
+  ResidentOrder::stream_created(s);
   return CAVS_OK;
 }
 
 int cavs_stream_destroy(void *stream) {
-  if (stream) CAVS_HIP_TRY(hipStreamDestroy(as_stream(stream)));
+  if (stream) {
+    ResidentOrder::stream_gone(as_stream(stream));
+    CAVS_HIP_TRY(hipStreamDestroy(as_stream(stream)));
+  }
   return CAVS_OK;
 }
 
@@ -215,6 +294,7 @@ int cavs_event_elapsed_ms(float *ms, void *start, void *stop) {
 
 int cavs_graph_capture_begin(void *stream) {
   CAVS_REQUIRE(stream, "cavs_graph_capture_begin: the default stream cannot be captured");
+  ResidentOrder::capture_begins(as_stream(stream));
   // relaxed: other threads of the process (an allocator, another session) may go on calling the runtime
   CAVS_HIP_TRY(hipStreamBeginCapture(as_stream(stream), hipStreamCaptureModeRelaxed));
   return CAVS_OK;
@@ -255,6 +335,8 @@ int cavs_graph_capture_end(void *stream, void **graph_exec) {
 
 int cavs_graph_launch(void *graph_exec, void *stream) {
   CAVS_REQUIRE(graph_exec, "cavs_graph_launch: null graph");
+  ResidentOrder order(as_stream(stream));  // (it may hold such launches)
+  if (order.rc()) return order.rc();
   CAVS_HIP_TRY(hipGraphLaunch(static_cast<hipGraphExec_t>(graph_exec), as_stream(stream)));
   return CAVS_OK;
 }

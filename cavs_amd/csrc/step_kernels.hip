@@ -326,8 +326,9 @@ __global__ __launch_bounds__(256) void tasks_kernel(TaskList L) {
       // sixty-four float4 are one contiguous kilobyte.  A workgroup moves 16 columns x 64 k.
       const float *__restrict__ in = static_cast<const float *>(t.p1);
       float4 *__restrict__ out = static_cast<float4 *>(t.p0);
-      const int N = (int)t.n0, K = (int)t.n1, kc = K / 64;
+      const int N = (int)t.n0, K = (int)t.n1, kc = (K + 63) / 64;
       const int tcol = b / kc, k0 = (b % kc) * 64, r = tid >> 4, q = tid & 15;
+      if (k0 + 4 * q >= K) break;  // (K is a multiple of 16)
       const float4 v = *reinterpret_cast<const float4 *>(in + (long)(16 * tcol + r) * K + k0 + 4 * q);
       const long g = k0 / 16 + q / 4;
       out[((g * (N / 16) + tcol) * 4 + (q & 3)) * 16 + r] = v;
@@ -339,11 +340,12 @@ __global__ __launch_bounds__(256) void tasks_kernel(TaskList L) {
       float *__restrict__ w = static_cast<float *>(t.p1);
       const float *__restrict__ g = static_cast<const float *>(t.p2);
       float4 *__restrict__ out = static_cast<float4 *>(t.p0);
-      const int N = (int)t.n1, nc = N / 64;
+      const int N = (int)t.n1, nc = (N + 63) / 64;
       const int kg = b / nc, cb = b % nc, kk = tid >> 4, q = tid & 15;
       const long at = (long)(16 * kg + kk) * N + 64 * cb + 4 * q;
-      float4 v = *reinterpret_cast<const float4 *>(w + at);
-      if (g) {
+      const bool in = 64 * cb + 4 * q < N;  // (N is a multiple of 16)
+      float4 v = in ? *reinterpret_cast<const float4 *>(w + at) : zero4();
+      if (g && in) {
         const float4 d = *reinterpret_cast<const float4 *>(g + at);
         v.x -= t.f0 * d.x; v.y -= t.f0 * d.y; v.z -= t.f0 * d.z; v.w -= t.f0 * d.w;
         *reinterpret_cast<float4 *>(w + at) = v;
@@ -351,6 +353,7 @@ __global__ __launch_bounds__(256) void tasks_kernel(TaskList L) {
       lds.pk[kk][4 * q] = v.x; lds.pk[kk][4 * q + 1] = v.y; lds.pk[kk][4 * q + 2] = v.z; lds.pk[kk][4 * q + 3] = v.w;
       __syncthreads();
       const int tt = tid >> 6, slot = (tid >> 4) & 3, x = tid & 15, col = 16 * tt + x;
+      if (16 * (4 * cb + tt) >= N) break;
       out[(((long)kg * (N / 16) + 4 * cb + tt) * 4 + slot) * 16 + x] =
           make_float4(lds.pk[4 * slot][col], lds.pk[4 * slot + 1][col], lds.pk[4 * slot + 2][col], lds.pk[4 * slot + 3][col]);
       break;
@@ -527,20 +530,20 @@ int cavs_run_tasks(int count, const cavs_task *tasks, void *stream) {
         blocks = ((t.n0 + 31) / 32) * ((t.n1 + 31) / 32);
         break;
       case CAVS_TASK_PACK_T:
-        CAVS_REQUIRE(t.n0 >= 0 && t.n1 >= 0 && t.n0 < (1 << 24) && t.n1 < (1 << 24) && t.n0 % 16 == 0 && t.n1 % 64 == 0,
-                     "cavs_run_tasks: job %d: bad shape to pack (rows a multiple of 16, columns of 64)", i);
+        CAVS_REQUIRE(t.n0 >= 0 && t.n1 >= 0 && t.n0 < (1 << 24) && t.n1 < (1 << 24) && t.n0 % 16 == 0 && t.n1 % 16 == 0,
+                     "cavs_run_tasks: job %d: bad shape to pack (rows and columns multiples of 16)", i);
         if (t.n0 == 0 || t.n1 == 0) continue;
         CAVS_REQUIRE(t.p0 && t.p1 && t.p0 != t.p1, "cavs_run_tasks: job %d: null or aliased pointer", i);
         CAVS_REQUIRE(aligned16(t.p0) && aligned16(t.p1), "cavs_run_tasks: job %d: pack needs 16-byte aligned pointers", i);
-        blocks = (t.n0 / 16) * (t.n1 / 64);
+        blocks = (t.n0 / 16) * ((t.n1 + 63) / 64);
         break;
       case CAVS_TASK_SGD_PACK:
-        CAVS_REQUIRE(t.n0 >= 0 && t.n1 >= 0 && t.n0 < (1 << 24) && t.n1 < (1 << 24) && t.n0 % 16 == 0 && t.n1 % 64 == 0,
-                     "cavs_run_tasks: job %d: bad shape to pack (rows a multiple of 16, columns of 64)", i);
+        CAVS_REQUIRE(t.n0 >= 0 && t.n1 >= 0 && t.n0 < (1 << 24) && t.n1 < (1 << 24) && t.n0 % 16 == 0 && t.n1 % 16 == 0,
+                     "cavs_run_tasks: job %d: bad shape to pack (rows and columns multiples of 16)", i);
         if (t.n0 == 0 || t.n1 == 0) continue;
         CAVS_REQUIRE(t.p0 && t.p1 && t.p0 != t.p1 && t.p0 != t.p2, "cavs_run_tasks: job %d: null or aliased pointer", i);
         CAVS_REQUIRE(aligned16(t.p0) && aligned16(t.p1) && aligned16(t.p2), "cavs_run_tasks: job %d: pack needs 16-byte aligned pointers", i);
-        blocks = (t.n0 / 16) * (t.n1 / 64);
+        blocks = (t.n0 / 16) * ((t.n1 + 63) / 64);
         break;
       case CAVS_TASK_ZERO_ROWS:
         CAVS_REQUIRE(t.n0 >= 0 && t.n1 > 0 && t.n1 < (1 << 30), "cavs_run_tasks: job %d: bad shape", i);

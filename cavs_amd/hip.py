@@ -50,6 +50,11 @@ class BlockCopy(C.Structure):
 GEMM_C_UNUSED, GEMM_A_ZERO, GEMM_B_ZERO = 1, 2, 3
 
 
+class GroupPlan(C.Structure):
+    """cavs_group_plan"""
+    _fields_ = [("groups", _P), ("lists", _P), ("recs", _P), ("ngroups", _I), ("sync", _P), ("spin_max", _I), ("extra_arrivals", _I)]
+
+
 # name -> argtypes (every function returns int unless listed in _RESTYPE)
 _SIGS = {
     "cavs_init": [_I],
@@ -120,6 +125,12 @@ _SIGS = {
     "cavs_tail_probe": [_P, _I, _I, _P],
     "cavs_treelstm_tail_fwd": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _P, _I, _I, _P],
     "cavs_treelstm_tail_bwd": [_P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _I, _P, _P, _P, _P, _I, _I, _P, _I, _I, _P],
+    "cavs_treelstm_group_fwd": [_P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, C.POINTER(GroupPlan), _P],
+    "cavs_treelstm_group_bwd": [_P, _I, _P, _P, _P, _P, _P, _P, _I, _I, C.POINTER(GroupPlan), _P],
+    "cavs_lstm_group_fwd": [_P, _P, _I, _P, _P, _P, _P, _P, _P, _I, C.POINTER(GroupPlan), _P],
+    "cavs_lstm_group_bwd": [_P, _I, _P, _P, _P, _P, _P, _I, _I, C.POINTER(GroupPlan), _P],
+    "cavs_treefc_group_fwd": [_P, _P, _P, _P, _P, _P, _P, _I, _I, C.POINTER(GroupPlan), _P],
+    "cavs_treefc_group_bwd": [_P, _P, _P, _P, _I, _I, C.POINTER(GroupPlan), _P],
     "cavs_transpose": [_P, _P, _I, _I, _P],
     "cavs_lstm_round_fwd": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P],
     "cavs_lstm_round_fwd_packed": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P],
@@ -158,7 +169,7 @@ _RESTYPE = {"cavs_last_error": C.c_char_p, "cavs_abi_version": _I, "cavs_sgemm_s
             "cavs_fc_softmax_xent_workspace": _Z, "cavs_colsum_blocks_workspace": _Z,
             "cavs_clip_grads_workspace": _Z, "cavs_sgemm_group_workspace": _Z, "cavs_fc_softmax_xent_parts": _I,
             "cavs_colsum_parts": _I, "cavs_round_packed_ok": _I, "cavs_lstm_round_packed_ok": _I,
-            "cavs_tail_rounds_ok": _I, "cavs_tail_max_rounds": _I, "cavs_tail_max_groups": _I, "cavs_tail_sync_bytes": _Z,
+            "cavs_group_rounds_ok": _I, "cavs_group_max_groups": _I, "cavs_group_rows": _I, "cavs_tail_rounds_ok": _I, "cavs_tail_max_rounds": _I, "cavs_tail_max_groups": _I, "cavs_tail_sync_bytes": _Z,
             "cavs_sgemm_splitk_static_max_bytes": _Z,
             "cavs_schedule_arena_scratch": _Z}
 _NOCHECK = {"cavs_last_error": [], "cavs_abi_version": [], "cavs_sgemm_splitk_workspace": [_I, _I, _I],
@@ -166,7 +177,7 @@ _NOCHECK = {"cavs_last_error": [], "cavs_abi_version": [], "cavs_sgemm_splitk_wo
             "cavs_clip_grads_workspace": [_I], "cavs_sgemm_group_workspace": [_I, C.POINTER(GemmDesc)],
             "cavs_fc_softmax_xent_parts": [_I], "cavs_colsum_parts": [_I], "cavs_round_packed_ok": [_I, _I],
             "cavs_lstm_round_packed_ok": [_I, _I], "cavs_sgemm_splitk_static_max_bytes": [],
-            "cavs_tail_rounds_ok": [_I, _I], "cavs_tail_max_rounds": [], "cavs_tail_max_groups": [], "cavs_tail_sync_bytes": [],
+            "cavs_group_rounds_ok": [_I], "cavs_group_max_groups": [_I], "cavs_group_rows": [], "cavs_tail_rounds_ok": [_I, _I], "cavs_tail_max_rounds": [], "cavs_tail_max_groups": [], "cavs_tail_sync_bytes": [],
             "cavs_schedule_arena_scratch": [_I, _I]}
 
 EW_BINARY = dict(add=0, sub=1, mul=2, div=3, sigmoid_grad=4, tanh_grad=5, relu_grad=6, equal=7)

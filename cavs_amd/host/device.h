@@ -89,6 +89,7 @@ class PinnedArray {
     cap_ = n;
   }
   T *get() const { return p_; }
+  size_t capacity() const { return cap_; }
 
  private:
   T *p_ = nullptr;

@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cstring>
+#include <mutex>
 
 // runs one backend call inside a profiling bracket of the given kernel class
 #define CAVS_TIMED(cls, call)   \
@@ -134,30 +135,77 @@ const float *Engine::user_rows(const float *src, size_t n, int blocks) {
 }
 
 // ------------------------------------------------------------------ the rounds near the roots in one launch
-// Whether this device runs the workgroups of such a launch all at once on one XCD is asked once,
-// with the barrier alone (cavs_tail_probe); a device that does not keeps to one launch per round.
+// Whether this device runs the workgroups of such a launch all at once on one XCD is asked once per
+// process, with the barrier alone (cavs_tail_probe: 32 workgroups on each XCD, one to a CU, the most any
+// launch asks for); a device that does not keeps to one launch per round.
 void Engine::tail_setup() {
+  static std::mutex m;
+  static std::map<int, bool> known;
   tail_ready_ = false;
-  if (cfg_.model != CAVS_MODEL_TREELSTM || !(cfg_.opt & CAVS_OPT_BATCHING) || cfg_.tail_rows < 0) return;
-  if (!cavs_tail_rounds_ok(1, cfg_.H)) return;
+  if (cell_ || !(cfg_.opt & CAVS_OPT_BATCHING) || cfg_.tail_rows < 0 || !cavs_group_rounds_ok(cfg_.H)) return;
   const size_t words = cavs_tail_sync_bytes() / sizeof(int);
   tail_sync_.reserve(words);
   check(cavs_zero(tail_sync_.get(), words * sizeof(int), stream_));
-  check(cavs_tail_probe(reinterpret_cast<unsigned *>(tail_sync_.get()), cfg_.H, kTailSpins, stream_));
-  int head[4] = {0, 0, 0, 0};
-  check(cavs_memcpy_d2h(head, tail_sync_.get(), sizeof(head), stream_));
-  check(cavs_stream_sync(stream_));
-  tail_ready_ = head[1] == 0;
-  if (!tail_ready_) check(cavs_zero(tail_sync_.get(), words * sizeof(int), stream_));
+  std::lock_guard<std::mutex> lock(m);
+  auto it = known.find(cfg_.device);
+  if (it == known.end()) {
+    check(cavs_tail_probe(reinterpret_cast<unsigned *>(tail_sync_.get()), 512, kTailSpins, stream_));
+    int head[4] = {0, 0, 0, 0};
+    check(cavs_memcpy_d2h(head, tail_sync_.get(), sizeof(head), stream_));
+    check(cavs_stream_sync(stream_));
+    it = known.emplace(cfg_.device, head[1] == 0).first;
+    if (!it->second) check(cavs_zero(tail_sync_.get(), words * sizeof(int), stream_));
+  }
+  tail_ready_ = it->second;
 }
 
 int Engine::tail_limit() const {
-  if (!tail_ready_ || fused_rows() <= 0) return 0;
+  if (!tail_ready_ || fused_rows() <= 0 || cfg_.model != CAVS_MODEL_TREELSTM || !cavs_tail_rounds_ok(1, cfg_.H)) return 0;
   // a round whose rows are dealt so that some group gets more than this stays a launch of its own
   // (the launches take a group's share of a round in slices of at most 32 rows).  64 takes in every
   // round above the leaves of a batch of 64 parse trees: measured 0.363 ms per step against 0.366
   // with 32, where the first one or two rounds stay launches of their own; 96 and 128: the same.
   return cfg_.tail_rows > 0 ? cfg_.tail_rows : 64;
+}
+
+// A group takes a round of up to this many rows (in slices of 32); larger rounds are launches of their own.
+int Engine::group_limit() const {
+  if (!tail_ready_ || fused_rows() <= 0 || cell_ || !cavs_group_rounds_ok(cfg_.H)) return 0;
+  if (cfg_.model == CAVS_MODEL_TREELSTM && cavs_tail_rounds_ok(1, cfg_.H)) return 0;  // (the tail launches are tuned for that size)
+  return cfg_.tail_rows > 0 ? cfg_.tail_rows : 64;
+}
+
+cavs_group_plan Engine::group_plan(const GroupLists::Launch &l) const {
+  return {d_group_ + l.groups, d_group_ + l.lists, d_group_ + l.recs, group_.ngroups, reinterpret_cast<unsigned *>(tail_sync_.get()), kTailSpins, 0};
+}
+
+void Engine::group_launched() {
+  const double rows = (double)group_.rows, per = cfg_.model == CAVS_MODEL_TREELSTM ? 5.0 : cfg_.model == CAVS_MODEL_LSTM ? 4.0 : 2.0;
+  c_round_flops_ += 2.0 * rows * cfg_.H * per * cfg_.H;
+  c_gather_rows_ += nch_ * rows;
+  c_scatter_rows_ += rows;
+  c_launches_ += 1;
+  c_tail_launches_ += 1;
+  c_tail_rounds_ += (double)(sched_->rounds.size() - group_.first);
+  tail_pending_ = true;
+}
+
+void Engine::ensure_packed() {
+  if (upk_valid_) return;
+  const long long H = cfg_.H;
+  std::vector<cavs_task> pack;
+  Param &p = param(cfg_.model == CAVS_MODEL_TREELSTM ? "U" : "W");
+  if (cfg_.model == CAVS_MODEL_TREELSTM) {
+    pack.push_back({CAVS_TASK_SGD_PACK, 0.f, H, 3 * H, 0, Upk_.get(), p.w, nullptr, nullptr});
+    pack.push_back({CAVS_TASK_SGD_PACK, 0.f, H, H, 0, Upk_.at((size_t)3 * H * H), p.w + (size_t)3 * H * H, nullptr, nullptr});
+  } else if (cfg_.model == CAVS_MODEL_LSTM) {
+    pack.push_back({CAVS_TASK_SGD_PACK, 0.f, H, 4 * H, 0, Upk_.get(), p.w + (size_t)4 * H * E_, nullptr, nullptr});
+  } else {
+    pack.push_back({CAVS_TASK_SGD_PACK, 0.f, 2 * H, H, 0, Upk_.get(), p.w, nullptr, nullptr});
+  }
+  check(cavs_run_tasks((int)pack.size(), pack.data(), stream_));
+  c_launches_ += 1;
+  upk_valid_ = p.w == p.own_w.get();
 }
 
 // The rounds inside the tail launches and who runs which row (build_tail_lists): the groups' row
@@ -197,6 +245,10 @@ Engine::~Engine() {
   for (CellStage &st : cells_) cavs_cell_release(st.module);
   for (auto &e : ev_) cavs_event_destroy(e);
   for (auto &h : hlists_) {
+    if (h.free_ev) cavs_event_destroy(h.free_ev);
+    if (h.up_ev) cavs_event_destroy(h.up_ev);
+  }
+  for (auto &h : hfeeds_) {
     if (h.free_ev) cavs_event_destroy(h.free_ev);
     if (h.up_ev) cavs_event_destroy(h.up_ev);
   }
@@ -297,6 +349,8 @@ bool Engine::update_jobs(float *w, float *g, float lr, std::vector<cavs_task> *o
     const long long half = 4 * H * E_;
     out->push_back({CAVS_TASK_SGD, lr, half, 0, 0, w, g, nullptr, nullptr});
     out->push_back({CAVS_TASK_SGD_PACK, lr, H, 4 * H, 0, Upk_.get(), w + half, g + half, nullptr});
+  } else if (cfg_.model == CAVS_MODEL_TREEFC && w == param("W").w) {
+    out->push_back({CAVS_TASK_SGD_PACK, lr, 2 * H, H, 0, Upk_.get(), w, g, nullptr});
   } else {
     return false;
   }
@@ -547,6 +601,10 @@ void Engine::reserve_edges() {
   if (fused_rows() > 0 && ((cfg_.model == CAVS_MODEL_TREELSTM && (cavs_round_packed_ok(1, H) || cavs_round_packed_ok(65, H))) ||
                            (cfg_.model == CAVS_MODEL_LSTM && (cavs_lstm_round_packed_ok(1, H) || cavs_lstm_round_packed_ok(65, H)))))
     R(Upk_, (size_t)4 * H * H);
+  if (group_.first >= 0) {
+    R(Upk_, (size_t)(cfg_.model == CAVS_MODEL_TREEFC ? 2 : 4) * H * H);
+    R(UTp_, (size_t)(cfg_.model == CAVS_MODEL_TREEFC ? 2 : 4) * H * H);
+  }
   if (cfg_.model == CAVS_MODEL_TREELSTM) {
     R(hlr_, cap * H);
     R(dF_, cap * 2 * H);
@@ -579,6 +637,9 @@ void Engine::upload_index_arena() {
   const bool want_forest = !cfg_.split_backward_rounds && fused_rows() > 0;
   const bool want_tail = want_forest && tail_limit() > 0;
   const size_t total = (size_t)N * (2 + nch_) + s.B + (want_forest ? (size_t)N * (nch_ + 1) : 0) + (want_tail ? (size_t)N : 0);
+  const int group_lim = want_forest ? group_limit() : 0, ngroups = group_lim > 0 ? cavs_group_max_groups(cfg_.H) : 0;
+  const size_t group_at = (total + 3) / 4 * 4;  // (16-byte aligned on the device)
+  const size_t room = group_lim > 0 ? group_at + group_lists_bound(N, ngroups) : total;
   // Two sets of buffers (pinned staging + device lists) alternate, and the copy runs on a stream
   // of its own: the lists of step k + 1 are built and uploaded while the kernels of step k run,
   // instead of the copy sitting in the compute stream between two steps.  A set is rewritten only
@@ -594,8 +655,8 @@ void Engine::upload_index_arena() {
     wait_ms_ = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - w0).count();
     h.busy = false;
   }
-  h.host.reserve(total);
-  h.dev.reserve(grow(total, h.dev.capacity()));
+  h.host.reserve(grow(room, h.host.capacity()));
+  h.dev.reserve(grow(room, h.dev.capacity()));
   int *t2j = h.host.get(), *pair = t2j + N, *child = pair + N, *roots = child + (size_t)nch_ * N;
   std::string err = build_index_lists(s, nch_, cfg_.pairing, t2j, pair, child, roots);
   if (!err.empty()) fail(CAVS_EUNSUPPORTED, err);
@@ -604,7 +665,11 @@ void Engine::upload_index_arena() {
   tail_ = TailPlan();
   int *tail_rows = roots + s.B + (size_t)N * (nch_ + 1);
   if (want_tail && forest_) build_tail_plan(roots + s.B, tail_rows);
-  check(cavs_memcpy_h2d(h.dev.get(), h.host.get(), total * sizeof(int), sched_stream_));
+  group_ = GroupLists();
+  if (group_lim > 0 && forest_)
+    build_group_lists(s, nch_, t2j, pair, child, roots + s.B, group_lim, ngroups, cavs_group_rows(), &group_, h.host.get() + group_at);
+  d_group_ = h.dev.get() + group_at;
+  check(cavs_memcpy_h2d(h.dev.get(), h.host.get(), (group_.first >= 0 ? group_at + group_.ints : total) * sizeof(int), sched_stream_));
   check(cavs_event_record(h.up_ev, sched_stream_));
   check(cavs_event_sync(h.up_ev));  // a few microseconds; the compute stream is still busy with the previous step
   last_free_ev_ = h.free_ev;
@@ -670,6 +735,12 @@ void Engine::remember_plan(const int *graph, int B, int maxlen, uint64_t hash) {
   p->forest = forest_;
   p->last_used = ++plan_clock_;
   p->tail = tail_;
+  p->group = group_;
+  if (group_.first >= 0) {
+    p->group_dev.reserve(group_.ints);
+    check(cavs_memcpy_d2d(p->group_dev.get(), d_group_, group_.ints * sizeof(int), stream_));
+    d_group_ = p->group_dev.get();
+  }
   p->head_chunks = head_chunks_;
   p->lists.reserve(2 * N + 2 * nk + B + N + N);
   int *base = p->lists.get();
@@ -806,6 +877,23 @@ void Engine::schedule_on_device(const int *graph, int B, int maxlen) {
       d_tail_rows_ = d.tail_dev.get();
     }
   }
+  // The group launches' block is host work on all of the lists: they come back, the block goes up.
+  if (forest_ && group_limit() > 0 && N > 0) {
+    const size_t all = BM * (2 + 2 * (size_t)nch_);
+    const int ngroups = cavs_group_max_groups(cfg_.H);
+    d.kid_host.reserve(all);
+    d.tail_host.reserve(group_lists_bound(N, ngroups));
+    check(cavs_memcpy_d2h(d.kid_host.get(), t2j, all * sizeof(int), sched_stream_));
+    check(cavs_stream_sync(sched_stream_));
+    const int *h = d.kid_host.get();
+    build_group_lists(s, nch_, h, h + BM, h + 2 * BM, h + (2 + nch_) * BM, group_limit(), ngroups, cavs_group_rows(), &group_, d.tail_host.get());
+    if (group_.first >= 0) {
+      d.tail_dev.reserve(grow(group_.ints, d.tail_dev.capacity()));
+      check(cavs_memcpy_h2d(d.tail_dev.get(), d.tail_host.get(), group_.ints * sizeof(int), sched_stream_));
+      check(cavs_stream_sync(sched_stream_));
+      d_group_ = d.tail_dev.get();
+    }
+  }
   last_free_ev_ = d.free_ev;
   last_busy_ = &d.busy;
   sched_ms_ = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -843,6 +931,11 @@ void Engine::begin_step(const int *graph, int B, int maxlen) {
     *last_busy_ = true;
     last_free_ev_ = nullptr;
   }
+  if (hfeeds_used_) {
+    check(cavs_event_record(hfeeds_used_->free_ev, stream_));
+    hfeeds_used_->busy = true;
+    hfeeds_used_ = nullptr;
+  }
   c_gather_rows_ = c_scatter_rows_ = c_gemm_flops_ = c_gemm_flops_hinted_ = c_launches_ = c_gather_bytes_ = c_scatter_bytes_ = 0;
   c_round_flops_ = 0;
   c_tail_rounds_ = c_tail_launches_ = 0;
@@ -878,10 +971,13 @@ void Engine::begin_step(const int *graph, int B, int maxlen) {
     d_orphans_ = base + 2 * N + 2 * nk + B;
     d_tail_rows_ = base + 3 * N + 2 * nk + B;
     tail_ = (forest_ && tail_limit() > 0) ? hit->tail : TailPlan();
+    group_ = (forest_ && group_limit() > 0) ? hit->group : GroupLists();
+    d_group_ = hit->group_dev.get();
     if (forest_ && !cfg_.graph_replay) head_chunks_ = hit->head_chunks;
     sched_ms_ = 0.f;
   } else {
-    tail_ = TailPlan();  // (the host-built lists bring a new one)
+    tail_ = TailPlan();  // (the host-built lists bring new ones)
+    group_ = GroupLists();
     const bool on_device = cfg_.schedule_mode == 1 && (cfg_.opt & CAVS_OPT_BATCHING);
     // (one wavefront per sample with its parent row in LDS: a limit of the kernels, and the caller's to know)
     if (on_device && maxlen > 2048)
@@ -1052,6 +1148,40 @@ void Engine::restore_step_state(const StepState &st) {
   ev_valid_ = ev_bwd_valid_ = false;
 }
 
+// Feeds from the caller's memory, which is free again when this returns.  They used to go up on the
+// session's own stream with a wait for all of it, i.e. for the step before (Tree-LSTM, H = 150, 25
+// trees: 0.261 ms per step, 0.245 this way).
+void Engine::upload_feeds(const void *x, size_t nx, const void *labels, size_t nl) {
+  const size_t lab0 = (nx + 3) / 4 * 4, total = lab0 + nl;
+  if (total == 0) return;
+  HostFeeds &h = hfeeds_[hfeeds_slot_];
+  hfeeds_slot_ ^= 1;
+  if (!sched_stream_) check(cavs_stream_create(&sched_stream_));
+  if (!h.free_ev) check(cavs_event_create(&h.free_ev));
+  if (!h.up_ev) check(cavs_event_create(&h.up_ev));
+  if (h.busy) {  // the step before last read these
+    check(cavs_event_sync(h.free_ev));
+    h.busy = false;
+  }
+  h.dev.reserve(grow(total, h.dev.capacity()));
+  // (rows of megabytes: the runtime's own path for pageable memory copies them no slower than this thread would)
+  const bool stage = total * 4 <= (size_t(1) << 20);
+  if (stage) {
+    h.host.reserve(total);
+    if (nx) std::memcpy(h.host.get(), x, nx * 4);
+    if (nl) std::memcpy(h.host.get() + lab0, labels, nl * 4);
+    check(cavs_memcpy_h2d(h.dev.get(), h.host.get(), total * 4, sched_stream_));
+  } else {
+    if (nx) check(cavs_memcpy_h2d(h.dev.get(), x, nx * 4, sched_stream_));
+    if (nl) check(cavs_memcpy_h2d(h.dev.at(lab0), labels, nl * 4, sched_stream_));
+  }
+  check(cavs_event_record(h.up_ev, sched_stream_));
+  check(cavs_event_sync(h.up_ev));
+  hfeeds_used_ = &h;
+  if (nx) d_x_ = h.dev.get();
+  if (nl) d_labels_ = h.dev.at(lab0);
+}
+
 void Engine::step(const int *graph, int B, int maxlen, const void *x, const void *labels,
                   bool on_device, bool backward, float lr) {
   auto step_t0 = std::chrono::steady_clock::now();
@@ -1070,18 +1200,7 @@ void Engine::step(const int *graph, int B, int maxlen, const void *x, const void
     d_x_ = static_cast<const float *>(x);
     d_labels_ = static_cast<const float *>(labels);
   } else {
-    if (needs_x) {
-      ensure(x_in_, grow((size_t)N * xw, x_in_.capacity()));
-      check(cavs_memcpy_h2d(x_in_.get(), x, (size_t)N * xw * 4, stream_));
-      d_x_ = x_in_.get();
-    }
-    if (cfg_.loss == CAVS_LOSS_SOFTMAX) {
-      ensure(labels_in_, grow(N, labels_in_.capacity()));
-      check(cavs_memcpy_h2d(labels_in_.get(), labels, (size_t)N * 4, stream_));
-      d_labels_ = labels_in_.get();
-    }
-    // pageable sources: make sure the copies are done before the caller reuses them
-    check(cavs_stream_sync(stream_));
+    upload_feeds(x, needs_x ? (size_t)N * xw : 0, labels, cfg_.loss == CAVS_LOSS_SOFTMAX ? (size_t)N : 0);
   }
 
   // A batch structure seen before, on the same feed buffers, with the session in the state it was
@@ -1226,14 +1345,7 @@ void Engine::treelstm_forward() {
   bool any_packed = false;
   if (Upk_.capacity() > 0)
     for (const Round &r : sched_->rounds) any_packed |= !leaf_round(r) && r.n <= fused && cavs_round_packed_ok(r.n, H);
-  if (any_packed && !upk_valid_) {  // U was written by somebody else since the last update here
-    cavs_task pack[2] = {{CAVS_TASK_SGD_PACK, 0.f, H, 3 * H, 0, Upk_.get(), const_cast<float *>(U), nullptr, nullptr},
-                         {CAVS_TASK_SGD_PACK, 0.f, H, H, 0, Upk_.at((size_t)3 * H * H), const_cast<float *>(U) + (size_t)3 * H * H, nullptr,
-                          nullptr}};
-    check(cavs_run_tasks(2, pack, stream_));
-    c_launches_ += 1;
-    upk_valid_ = U == param("U").own_w.get();
-  }
+  if (any_packed || group_.first >= 0) ensure_packed();
   // Pull of the word id, the lookup and x * W: one launch
   {
     ProfScope ps(this, K_GEMM);
@@ -1269,6 +1381,13 @@ void Engine::treelstm_forward() {
       c_tail_launches_ += 1;
       c_tail_rounds_ += (double)(sched_->rounds.size() - tail_from);
       tail_pending_ = true;
+      break;
+    }
+    if (group_.first >= 0 && (int)rk == group_.first) {
+      const cavs_group_plan plan = group_plan(group_.fwd);
+      CAVS_TIMED(K_ROUND, cavs_treelstm_group_fwd(pool_.get(), xW_.get(), 4 * H, Upk_.get(), Bv, G_.get(), hlr_.get(), gates_.get(),
+                                                  out_folded_ ? nullptr : msg_.get(), go, H, &plan, stream_));
+      group_launched();
       break;
     }
     const size_t off = r.offset;
@@ -1336,8 +1455,11 @@ void Engine::treelstm_backward() {
   // one launch per round when the message flow is a forest (below); then, if every such launch has
   // a packed variant, the transposed weights are written tile-major instead of plain
   bool packed = forest_;
-  for (const Round &r : sched_->rounds)
+  for (size_t k = 0; k < sched_->rounds.size(); k++) {
+    const Round &r = sched_->rounds[k];
+    if (group_backward((int)k)) break;  // (the group launches read the packed copy)
     if (!leaf_round(r) && !cavs_round_packed_ok(r.n, H)) packed = false;
+  }
   // one launch per round when the message flow is a forest: the roots' gate gradients first, then
   // every round hands d h, d c on to its children and does their gate gradients in its epilogue
   const bool folded = forest_;
@@ -1348,6 +1470,10 @@ void Engine::treelstm_backward() {
     const int kind = packed ? CAVS_TASK_PACK_T : CAVS_TASK_TRANSPOSE;
     opening.push_back({kind, 0.f, H, 3 * H, 0, UT_.get(), const_cast<float *>(U), nullptr, nullptr});
     opening.push_back({kind, 0.f, H, H, 0, UT_.at((size_t)3 * H * H), const_cast<float *>(U) + (size_t)3 * H * H, nullptr, nullptr});
+    if (group_.first >= 0 && !packed) {
+      opening.push_back({CAVS_TASK_PACK_T, 0.f, H, 3 * H, 0, UTp_.get(), const_cast<float *>(U), nullptr, nullptr});
+      opening.push_back({CAVS_TASK_PACK_T, 0.f, H, H, 0, UTp_.at((size_t)3 * H * H), const_cast<float *>(U) + (size_t)3 * H * H, nullptr, nullptr});
+    }
   }
   if (roots_ride)
     opening.push_back({CAVS_TASK_TREELSTM_GATES_ROWS, 0.f, n_orphans_, H, (long long)sched_->leaf_prefix | ((long long)(4 * H) << 32),
@@ -1379,10 +1505,17 @@ void Engine::treelstm_backward() {
     c_tail_rounds_ += (double)tail_n;
     tail_pending_ = true;
   }
+  if (group_.first >= 0) {
+    const cavs_group_plan plan = group_plan(group_.bwd);
+    CAVS_TIMED(K_ROUND, cavs_treelstm_group_bwd(dxW_.get(), 4 * H, dF_.get(), dc_.get(), packed ? UT_.get() : UTp_.get(), gates_.get(), G_.get(),
+                                                d_dgo_, sched_->leaf_prefix, H, &plan, stream_));
+    group_launched();
+  }
   for (size_t bi = tail_n; bi < sched_->bwd_rounds.size(); bi++) {
     const int k = sched_->bwd_rounds[bi];
     const Round &r = sched_->rounds[k];
     const size_t off = r.offset;
+    if (group_backward(k)) continue;
     if (folded) {
       c_gather_rows_ += r.n;
       if (leaf_round(r)) continue;
@@ -1626,15 +1759,17 @@ void Engine::lstm_forward() {
   bool any_packed = false;
   if (Upk_.capacity() > 0)
     for (const Round &r : sched_->rounds) any_packed |= !leaf_round(r) && r.n <= fused && cavs_lstm_round_packed_ok(r.n, H);
-  if (any_packed && !upk_valid_) {  // W' was written by somebody else since the last update here
-    cavs_task pack{CAVS_TASK_SGD_PACK, 0.f, H, 4 * H, 0, Upk_.get(), const_cast<float *>(Wh), nullptr, nullptr};
-    check(cavs_run_tasks(1, &pack, stream_));
-    c_launches_ += 1;
-    upk_valid_ = Wx == param("W").own_w.get();
-  }
+  if (any_packed || group_.first >= 0) ensure_packed();
   out_folded_ = fused > 0 && sched_->max_round <= fused && fwd_out_ != nullptr;
   float *go = out_folded_ ? fwd_out_ : nullptr;
-  for (const Round &r : sched_->rounds) {
+  for (size_t rk = 0; rk < sched_->rounds.size(); rk++) {
+    const Round &r = sched_->rounds[rk];
+    if (group_.first >= 0 && (int)rk == group_.first) {
+      const cavs_group_plan plan = group_plan(group_.fwd);
+      CAVS_TIMED(K_ROUND, cavs_lstm_group_fwd(pool_.get(), xW_.get(), 4 * H, Upk_.get(), Bv, G_.get(), gates_.get(), msg_.get(), go, H, &plan, stream_));
+      group_launched();
+      break;
+    }
     const size_t off = r.offset;
     float *a = xW_.at(off * 4 * H), *msg = msg_.at(off * 2 * H), *G = nullptr;
     if (r.n <= fused) {  // one launch: Gather, h*W', gates, Scatter, Push/PopRet
@@ -1671,12 +1806,16 @@ void Engine::lstm_backward() {
   const bool dret_folded = fused > 0 && sched_->max_round <= fused;
   if (!dret_folded && !forest_) gather(dret_.get(), H, d_dgo_, H, d_t2j_, N, H);
   bool packed = forest_;  // as in treelstm_backward
-  for (const Round &r : sched_->rounds)
+  for (size_t k = 0; k < sched_->rounds.size(); k++) {
+    const Round &r = sched_->rounds[k];
+    if (group_backward((int)k)) break;
     if (!leaf_round(r) && !cavs_lstm_round_packed_ok(r.n, H)) packed = false;
+  }
   if (fused > 0) {  // W'^T: the B operand of d h_prev = da * W'^T, k-major
-    backward_prologue({{packed ? CAVS_TASK_PACK_T : CAVS_TASK_TRANSPOSE, 0.f, H, 4 * H, 0, UT_.get(), const_cast<float *>(Wh), nullptr,
-                        nullptr}},
-                      true);
+    std::vector<cavs_task> opening{{packed ? CAVS_TASK_PACK_T : CAVS_TASK_TRANSPOSE, 0.f, H, 4 * H, 0, UT_.get(), const_cast<float *>(Wh), nullptr,
+                                    nullptr}};
+    if (group_.first >= 0 && !head_chunked_ && !packed) opening.push_back({CAVS_TASK_PACK_T, 0.f, H, 4 * H, 0, UTp_.get(), const_cast<float *>(Wh), nullptr, nullptr});
+    backward_prologue(opening, true);
   } else {
     backward_prologue({}, true);
   }
@@ -1689,6 +1828,14 @@ void Engine::lstm_backward() {
     CAVS_TIMED(K_GATES, cavs_lstm_bwd_gates_rows(d_orphans_, n_orphans_, d_dgo_, d_t2j_, gates_.get(), G_.get(), dxW_.get(), 4 * H,
                                                  dc_.get(), sched_->leaf_prefix, H, stream_));
     c_launches_ += 1;
+  }
+  // (Not under a wide head in chunks: beside its products a launch that stays on every CU and the products
+  // slow each other down more than a launch per round does -- C4 3.89 ms per step against 3.60.)
+  if (group_.first >= 0 && !head_chunked_) {
+    const cavs_group_plan plan = group_plan(group_.bwd);
+    CAVS_TIMED(K_ROUND, cavs_lstm_group_bwd(dxW_.get(), 4 * H, dc_.get(), packed ? UT_.get() : UTp_.get(), gates_.get(), G_.get(), d_dgo_,
+                                            sched_->leaf_prefix, H, &plan, stream_));
+    group_launched();
   }
   for (int k : sched_->bwd_rounds) {
     const Round &r = sched_->rounds[k];
@@ -1707,6 +1854,7 @@ void Engine::lstm_backward() {
         c_launches_ += 1;
       }
     }
+    if (group_backward(k)) continue;
     if (folded) {
       c_gather_rows_ += r.n;
       if (leaf_round(r)) continue;
@@ -1769,7 +1917,16 @@ void Engine::treefc_forward() {
   const int fused = fused_rows();
   out_folded_ = fused > 0 && sched_->max_round <= fused && fwd_out_ != nullptr;
   float *go = out_folded_ ? fwd_out_ : nullptr;
-  for (const Round &r : sched_->rounds) {
+  if (group_.first >= 0) ensure_packed();
+  for (size_t rk = 0; rk < sched_->rounds.size(); rk++) {
+    const Round &r = sched_->rounds[rk];
+    if (group_.first >= 0 && (int)rk == group_.first) {
+      const cavs_group_plan plan = group_plan(group_.fwd);
+      CAVS_TIMED(K_ROUND, cavs_treefc_group_fwd(pool_.get(), cfg_.use_x ? xs_.get() : nullptr, Upk_.get(), Bv, G_.get(), msg_.get(), go, H, cfg_.act, &plan,
+                                                stream_));
+      group_launched();
+      break;
+    }
     const size_t off = r.offset;
     const float *xin = cfg_.use_x ? xs_.at(off * H) : nullptr;
     float *msg = msg_.at(off * H);
@@ -1813,7 +1970,12 @@ void Engine::treefc_backward() {
   const bool dret_folded = fused > 0 && sched_->max_round <= fused;
   if (!dret_folded && !forest_) gather(dret_.get(), H, d_dgo_, H, d_t2j_, N, H);
   if (fused > 0) {  // W^T [H, 2H]: the B operand of d[h_l;h_r] = dz * W^T, k-major
-    backward_prologue({{CAVS_TASK_TRANSPOSE, 0.f, 2 * H, H, 0, UT_.get(), const_cast<float *>(W), nullptr, nullptr}}, false);
+    std::vector<cavs_task> opening;
+    bool rest = group_.first < 0;  // rounds that are launches of their own
+    for (int k = 0; k < group_.first; k++) rest |= !leaf_round(sched_->rounds[k]);
+    if (rest) opening.push_back({CAVS_TASK_TRANSPOSE, 0.f, 2 * H, H, 0, UT_.get(), const_cast<float *>(W), nullptr, nullptr});
+    if (group_.first >= 0) opening.push_back({CAVS_TASK_PACK_T, 0.f, 2 * H, H, 0, UTp_.get(), const_cast<float *>(W), nullptr, nullptr});
+    backward_prologue(opening, false);
   } else {
     backward_prologue({}, false);
   }
@@ -1822,8 +1984,14 @@ void Engine::treefc_backward() {
     CAVS_TIMED(K_GATES, cavs_treefc_bwd_rows(d_orphans_, n_orphans_, d_dgo_, d_t2j_, msg_.get(), dxW_.get(), H, cfg_.act, stream_));
     c_launches_ += 1;
   }
+  if (group_.first >= 0) {
+    const cavs_group_plan plan = group_plan(group_.bwd);
+    CAVS_TIMED(K_ROUND, cavs_treefc_group_bwd(dxW_.get(), UTp_.get(), msg_.get(), d_dgo_, H, cfg_.act, &plan, stream_));
+    group_launched();
+  }
   for (int k : sched_->bwd_rounds) {
     const Round &r = sched_->rounds[k];
+    if (group_backward(k)) continue;
     const size_t off = r.offset;
     float *dz = dxW_.at(off * H);
     if (folded) {

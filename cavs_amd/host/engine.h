@@ -202,7 +202,7 @@ class Engine {
   // builds every list there, and only the round offsets come back.  Two sets of buffers alternate,
   // so that the lists of step k + 1 are built while the kernels of step k still read theirs.
   struct DeviceSched {
-    PinnedArray<int> graph_host, meta_host, kid_host, tail_host;
+    PinnedArray<int> graph_host, meta_host, kid_host, tail_host;  // (tail_host: the group launches' block as well)
     DeviceArray<int> graph_dev, lists, meta_dev, tail_dev;
     long cap = 0;          // rows per list
     void *free_ev = nullptr;  // recorded once everything that read `lists` has been enqueued
@@ -221,6 +221,18 @@ class Engine {
   struct TailPlan : TailLists {
     double flops = 0, vertices = 0;
   };
+
+  // ---- rounds in one launch per direction at any hidden size of whole tiles up to 512 (cavs_*_group_*)
+  GroupLists group_;                     // of this step's schedule; first < 0: one launch per round
+  const int *d_group_ = nullptr;         // its block on the device
+  DeviceArray<float> UTp_;               // transposed weights tile-major, beside UT_ where other rounds want that plain
+  int group_limit() const;               // rows of a round a group may get (0: no such launches)
+  // whether round k of the backward pass is inside such a launch
+  bool group_backward(int k) const { return group_.first >= 0 && k >= group_.first && !head_chunked_; }
+  cavs_group_plan group_plan(const GroupLists::Launch &l) const;
+  void group_launched();
+  // packs the weights the forward launches read tile-major, where somebody else wrote them since
+  void ensure_packed();
 
   // ---- plan cache (cfg.plan_cache entries): the schedule and the device lists of a graph feed,
   // keyed by the feed's bytes, so that a batch structure seen before costs neither the scheduler
@@ -301,6 +313,8 @@ class Engine {
     int n_orphans = 0;
     bool forest = false;
     TailPlan tail;
+    GroupLists group;
+    DeviceArray<int> group_dev;
     std::vector<HeadChunk> head_chunks;
     uint64_t last_used = 0;
   };
@@ -312,8 +326,17 @@ class Engine {
   Plan *find_plan(const int *graph, int B, int maxlen, uint64_t hash);
   void remember_plan(const int *graph, int B, int maxlen, uint64_t hash);
 
-  // feeds
-  DeviceArray<float> x_in_, labels_in_;
+  // feeds from host memory: [x | labels], pinned staging and its device copy, two sets that alternate
+  // so that a step's feeds go up while the step before still runs
+  struct HostFeeds {
+    PinnedArray<float> host;
+    DeviceArray<float> dev;
+    void *free_ev = nullptr, *up_ev = nullptr;
+    bool busy = false;
+  } hfeeds_[2];
+  int hfeeds_slot_ = 0;
+  HostFeeds *hfeeds_used_ = nullptr;  // what the current step reads
+  void upload_feeds(const void *x, size_t nx, const void *labels, size_t nl);
   const float *d_x_ = nullptr, *d_labels_ = nullptr, *d_dgo_ = nullptr;
 
   // edges (rows = tensor ids unless marked round-local)

@@ -354,6 +354,109 @@ void build_tail_lists(const Schedule &s, const int *kid_rows, int lim, int group
   }
 }
 
+size_t group_lists_bound(size_t N, int groups) {
+  // two sets of records, forward and backward lists of at least a row each, two tables of groups
+  return N * (16 + 8) + 2 * (size_t)groups * 4;
+}
+
+void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pair, const int *child, const int *kid_rows, int lim, int groups,
+                       int slice, GroupLists *out, int *block) {
+  *out = GroupLists();
+  const int R = (int)s.rounds.size(), N = s.N;
+  auto leaf_round = [](const Round &r) { return r.gather_begin[0] == r.gather_end[0] && r.gather_begin[1] == r.gather_end[1]; };
+  if (lim <= 0 || groups < 1 || slice < 1 || !s.batching || R < 3) return;
+  int k0 = R;  // the rounds with children that no larger one follows
+  while (k0 > 1 && !leaf_round(s.rounds[k0 - 1]) && s.rounds[k0 - 1].n <= (long)groups * lim) k0--;
+  std::vector<int> comp, weight, order, group, per;
+  for (; R - k0 >= 2; k0++) {
+    const int lo = s.rounds[k0].offset, nr = R - k0;
+    comp.assign(N - lo, -1);
+    weight.clear();
+    for (int v = N - 1; v >= lo; v--) {  // a row's consumer sits in a later round: parents come first
+      if (comp[v - lo] < 0) {
+        comp[v - lo] = (int)weight.size();
+        weight.push_back(0);
+      }
+      weight[comp[v - lo]]++;
+      for (int i = 0; i < nch; i++) {
+        const int c = kid_rows[(size_t)nch * v + i];
+        if (c >= lo) comp[c - lo] = comp[v - lo];
+      }
+    }
+    // heaviest tree first to the group with the least so far
+    const int G = std::min<int>(groups, (int)weight.size());
+    order.resize(weight.size());
+    for (size_t i = 0; i < order.size(); i++) order[i] = (int)i;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return weight[a] > weight[b]; });
+    group.assign(weight.size(), 0);
+    std::vector<int> load(G, 0);
+    for (int c : order) {
+      const int best = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+      group[c] = best;
+      load[best] += weight[c];
+    }
+    per.assign((size_t)G * nr, 0);
+    bool ok = true;
+    for (int k = k0; k < R; k++)
+      for (int b = s.rounds[k].offset; b < s.rounds[k].offset + s.rounds[k].n; b++)
+        ok &= ++per[(size_t)group[comp[b - lo]] * nr + (k - k0)] <= lim;
+    if (!ok) continue;
+
+    GroupLists &t = *out;
+    t.first = k0;
+    t.ngroups = G;
+    t.rows = (size_t)(N - lo);
+    // the records, group by group, round by round
+    std::vector<int> at((size_t)G * nr), cur;
+    int fill = 0;
+    for (size_t i = 0; i < at.size(); i++) {
+      at[i] = fill;
+      fill += per[i];
+    }
+    t.fwd.recs = 0;
+    t.bwd.recs = t.rows * 8;
+    cur = at;
+    for (int k = k0; k < R; k++)
+      for (int b = s.rounds[k].offset; b < s.rounds[k].offset + s.rounds[k].n; b++) {
+        const int i = cur[(size_t)group[comp[b - lo]] * nr + (k - k0)]++;
+        int *f = block + t.fwd.recs + 8 * (size_t)i, *w = block + t.bwd.recs + 8 * (size_t)i;
+        const int *c = child + (size_t)nch * b, *q = kid_rows + (size_t)nch * b;
+        const int c1 = nch == 2 ? c[1] : -1, q1 = nch == 2 ? q[1] : -1;
+        const int fr[8] = {b, c[0], c1, pair[b], t2j[b], 0, 0, 0};
+        const int br[8] = {b, q[0], q1, q[0] >= 0 ? t2j[q[0]] : -1, q1 >= 0 ? t2j[q1] : -1, 0, 0, 0};
+        std::copy(fr, fr + 8, f);
+        std::copy(br, br + 8, w);
+      }
+    size_t end = 2 * t.rows * 8;
+    // A direction: a group's share of a round as lists of at most `slice` rows; the first waits for the
+    // rounds the group has done so far, the last is an arrival.
+    for (int back = 0; back < 2; back++) {
+      GroupLists::Launch &l = back ? t.bwd : t.fwd;
+      l.groups = end;
+      l.lists = end + (size_t)G * 4;
+      int *lists = block + l.lists, nl = 0;
+      for (int g = 0; g < G; g++) {
+        int *gd = block + l.groups + 4 * (size_t)g, done = 0;
+        gd[0] = nl;
+        for (int i = 0; i < nr; i++) {
+          const int k = back ? nr - 1 - i : i, c = per[(size_t)g * nr + k];
+          for (int c0 = 0; c0 < c; c0 += slice, nl++) {
+            const int row[4] = {at[(size_t)g * nr + k] + c0, std::min(slice, c - c0), c0 == 0 ? done : 0, c0 + slice >= c};
+            std::copy(row, row + 4, lists + 4 * (size_t)nl);
+          }
+          done += c > 0;
+        }
+        gd[1] = nl - gd[0];
+        gd[2] = done;
+        gd[3] = 0;
+      }
+      end = l.lists + 4 * (size_t)nl;
+    }
+    t.ints = end;
+    return;
+  }
+}
+
 void schedule_from_lists(int B, int maxlen, int N, int nch, const int *round2offset, int R, const int *t2j,
                          const int *pair, const int *child, const int *roots, Schedule *out) {
   *out = Schedule();

@@ -87,6 +87,23 @@ struct TailLists {
   size_t rows = 0;                                // length of the list of slab rows
   int lists_max = 0, tiles_max = 0;               // the longest group: its lists, its tiles of four rows
 };
+// What the launches over rounds of any hidden size run (cavs_*_group_fwd / _bwd), as one block of ints
+// for the device (layouts: cavs_group_plan): the rounds from `first` on, their rows dealt to at most
+// `groups` groups by whole trees of the message flow.
+struct GroupLists {
+  struct Launch {
+    size_t groups = 0, lists = 0, recs = 0;  // where its arrays start in the block
+  };
+  int first = -1, ngroups = 0;
+  Launch fwd, bwd;
+  size_t ints = 0, rows = 0;
+};
+// ints the block may take for N vertices
+size_t group_lists_bound(size_t N, int groups);
+// lists as build_index_lists / build_forest_lists leave them; lim: most rows of a round a group may
+// get; slice: most rows per list.  out->first stays -1 when no two rounds qualify.
+void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pair, const int *child, const int *kid_rows, int lim, int groups,
+                       int slice, GroupLists *out, int *block);
 // kid_rows as build_forest_lists leaves them (binary trees); rows_out: room for N ints.
 void build_tail_lists(const Schedule &s, const int *kid_rows, int lim, int groups, int max_lists, int slice, TailLists *out,
                       int *rows_out);

@@ -443,6 +443,40 @@ size_t cavs_tail_sync_bytes(void);
  * the status word, after the stream has drained) whether this device runs every group's
  * workgroups all at once on one XCD. */
 int cavs_tail_probe(unsigned *sync, int H, int spin_max, void *stream);
+
+/* The rounds of a batch in one launch per direction, for every hidden size of whole tiles up to 512
+ * (cavs_group_rounds_ok) and all three vertex functions (the loops of cavs/midend/statement.cc:69-76,
+ * 106-111 without the round trips to the host): as the tail launches above, with
+ *   groups  [ngroups][4]  first list, number of lists, arrivals of the launch, 0
+ *   lists   [*][4]        first record, rows (at most cavs_group_rows()), arrivals that must be in, arrives (0 / 1)
+ *   recs    [*][8]        forward:  slab row, pool rows of its children (-1: none), pool row its message goes
+ *                                   to (-1: none), row of graph_out, 0, 0, 0
+ *                         backward: slab row, slab rows of its children, row of dret of child 0, of child 1, 0, 0, 0
+ * in device memory, 16-byte aligned; group g runs on XCD g % 8, at most cavs_group_max_groups(H) of them.
+ * Weights tile-major: forward as CAVS_TASK_SGD_PACK writes them (Tree-LSTM: pack(U_iou), then pack(U_f);
+ * chain LSTM: pack(W'); Tree-FC: pack(W)), backward as CAVS_TASK_PACK_T does.  sync, spin_max and
+ * extra_arrivals as for the tail launches (the same sync block serves both, one launch at a time). */
+typedef struct {
+  const int *groups, *lists, *recs;
+  int ngroups;
+  unsigned *sync;
+  int spin_max, extra_arrivals;
+} cavs_group_plan;
+int cavs_group_rounds_ok(int H);
+int cavs_group_max_groups(int H);
+int cavs_group_rows(void);
+int cavs_treelstm_group_fwd(float *pool, const float *xW, int ld_xw, const float *Upk, const float *bias, float *G, float *hlr,
+                            float *gates, float *msg, float *graph_out, int H, const cavs_group_plan *plan, void *stream);
+int cavs_treelstm_group_bwd(float *dxW, int ld_dxw, float *dF, float *dc, const float *UTp, const float *gates, const float *G,
+                            const float *dret, int leaf_rows, int H, const cavs_group_plan *plan, void *stream);
+int cavs_lstm_group_fwd(float *pool, const float *xW, int ld_xw, const float *Whp, const float *bias, float *G, float *gates,
+                        float *msg, float *graph_out, int H, const cavs_group_plan *plan, void *stream);
+int cavs_lstm_group_bwd(float *da, int ld_da, float *dc, const float *WhTp, const float *gates, const float *G, const float *dret,
+                        int leaf_rows, int H, const cavs_group_plan *plan, void *stream);
+int cavs_treefc_group_fwd(float *pool, const float *x, const float *Wp, const float *bias, float *G, float *msg, float *graph_out,
+                          int H, int act, const cavs_group_plan *plan, void *stream);
+int cavs_treefc_group_bwd(float *dz, const float *WTp, const float *h, const float *dret, int H, int act, const cavs_group_plan *plan,
+                          void *stream);
 int cavs_treelstm_tail_fwd(float *pool, const int *child, const int *pair, const float *xW, int ld_xw,
                            const float *Upk, const float *bias, float *G, float *hlr, float *gates,
                            float *msg, float *graph_out, const int *out_rows, const int *rows,
@@ -572,12 +606,12 @@ int cavs_transpose(float *out, const float *in, int rows, int cols, void *stream
  *                        parameter's (the gate bias, apps/paper/tree-lstm-cavs.cc:120-123 vs :143-148).
  *                        With P = n2 >> 32 above 1, p1 holds P such rows and the job adds them up first,
  *                        in index order (the chunk sums cavs_colsum_blocks leaves behind).
- *   CAVS_TASK_PACK_T     p0 = B = p1^T (p1 [n0, n1] row-major, so B is [K = n1, N = n0]; n0 a multiple of 16,
- *                        n1 of 64) in the tile-major layout of the packed round entry points: for k-group
+ *   CAVS_TASK_PACK_T     p0 = B = p1^T (p1 [n0, n1] row-major, so B is [K = n1, N = n0]; both multiples
+ *                        of 16) in the tile-major layout of the packed round entry points: for k-group
  *                        g (16 k) and column tile t (16 columns), floats [((g * N/16 + t) * 256, +256) hold
  *                        B[16g + 4s + c][16t + x] at [s][x][c], s < 4, x < 16, c < 4.
  *   CAVS_TASK_SGD_PACK   p1[i] -= f0 * p2[i] (skipped when p2 is null), then p0 = B = p1 ([K = n0, N = n1]
- *                        row-major; n0 a multiple of 16, n1 of 64) in the same tile-major layout: the
+ *                        row-major; both multiples of 16) in the same tile-major layout: the
  *                        parameter update (cavs/backend/op_impl_sgd.cu) and the packed copy the next
  *                        forward pass reads, in one pass over the weights.
  *   CAVS_TASK_SGD_TRANSPOSE  p1[i] -= f0 * p2[i] (skipped when p2 is null), then p0[c][r] = p1[r][c], n0 rows,
