@@ -437,6 +437,20 @@ __global__ __launch_bounds__(kThreads) void sgemm_group_kernel(GemmGroup G) {
   }
 }
 
+// p[0] + p[stride] + ... in that order, four loads in flight at a time (one at a time, a reduction over
+// four splits was four trips to memory in a row)
+__device__ inline float sum_splits(const float *__restrict__ p, int splits, long stride) {
+  float acc = 0.f;
+  for (int z = 0; z < splits; z += 4) {
+    float v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = z + k < splits ? p[(long)(z + k) * stride] : 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; k++) acc += v[k];
+  }
+  return acc;
+}
+
 // the split products of a group, reduced in one launch (same fixed order as splitk_reduce_kernel)
 __global__ void splitk_reduce_group_kernel(GemmGroup R) {
   // first[] counts 256-thread workgroups per product here
@@ -447,8 +461,7 @@ __global__ void splitk_reduce_group_kernel(GemmGroup R) {
   long idx = (long)(blockIdx.x - R.first[p]) * blockDim.x + threadIdx.x;
   long total = (long)g.M * g.N;
   if (idx >= total) return;
-  float acc = 0.f;
-  for (int z = 0; z < splits; z++) acc += g.ws[(long)z * total + idx];
+  const float acc = sum_splits(g.ws + idx, splits, total);
   int r = (int)(idx / g.N), c = (int)(idx % g.N);
   float v = g.alpha * acc;
   if (g.beta != 0.f) v += g.beta * g.C[r * g.ldc + c];
@@ -505,8 +518,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_group_embed_kernel(GemmGrou
   long idx = (long)(blockIdx.x - R.first[p]) * blockDim.x + threadIdx.x;
   long total = (long)g.M * g.N;
   if (idx >= total) return;
-  float acc = 0.f;
-  for (int z = 0; z < splits; z++) acc += g.ws[(long)z * total + idx];
+  const float acc = sum_splits(g.ws + idx, splits, total);
   int r = (int)(idx / g.N), c = (int)(idx % g.N);
   float v = g.alpha * acc;
   if (g.beta != 0.f) v += g.beta * g.C[r * g.ldc + c];
@@ -519,8 +531,7 @@ __global__ void splitk_reduce_kernel(GemmArgs g, int splits) {
   long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   long total = (long)g.M * g.N;
   if (idx >= total) return;
-  float acc = 0.f;
-  for (int z = 0; z < splits; z++) acc += g.ws[(long)z * total + idx];
+  const float acc = sum_splits(g.ws + idx, splits, total);
   int r = (int)(idx / g.N), c = (int)(idx % g.N);
   float v = g.alpha * acc;
   if (g.beta != 0.f) v += g.beta * g.C[r * g.ldc + c];
@@ -546,6 +557,21 @@ __global__ __launch_bounds__(W * 64) void sgemm_skinny_kernel(GemmArgs g) {
   const int kper = ((g.K + W - 1) / W + 7) / 8 * 8;
   const int kb = wave * kper, ke = min(g.K, kb + kper);
   const bool col_ok = n0 + j < g.N;
+  // where row m0 + 32 t + j of A is, in floats from g.A (-1: a zero row); looked-up rows (GemmArgs::pull_*)
+  // go on into pull_copy, a wavefront's k range per column tile
+  long arow[TM];
+  const bool pulls = g.pull_rows != nullptr;
+  const bool copies = pulls && (int)(wave % gridDim.x) == (int)blockIdx.x;
+#pragma unroll
+  for (int t = 0; t < TM; t++) {
+    const int row = m0 + 32 * t + j;
+    arow[t] = row < g.M ? (long)row * g.lda : -1;
+    if (pulls && row < g.M) {
+      const float id = g.pull_x[g.pull_rows[row]];
+      arow[t] = (long)(int)(id * (float)g.K);
+      if (blockIdx.x == 0 && wave == 0 && h == 0) g.pull_ids[row] = id;
+    }
+  }
 
   floatx16 acc[TM];
 #pragma unroll
@@ -562,9 +588,11 @@ __global__ __launch_bounds__(W * 64) void sgemm_skinny_kernel(GemmArgs g) {
       const bool kin = kk < ke;
 #pragma unroll
       for (int t = 0; t < TM; t++) {
-        const int row = m0 + 32 * t + j;
-        a[u][t] = (kin && row < g.M) ? *reinterpret_cast<const float4 *>(g.A + (long)row * g.lda + kk)
-                                     : make_float4(0.f, 0.f, 0.f, 0.f);
+        a[u][t] = (kin && arow[t] >= 0) ? *reinterpret_cast<const float4 *>(g.A + arow[t] + kk) : make_float4(0.f, 0.f, 0.f, 0.f);
+        if (copies && kin) {
+          const int row = m0 + 32 * t + j;
+          if (row < g.M) *reinterpret_cast<float4 *>(g.pull_copy + (long)row * g.ld_copy + kk) = a[u][t];
+        }
       }
       if constexpr (TB) {
         float4 q = (kin && col_ok) ? *reinterpret_cast<const float4 *>(g.B + (long)(n0 + j) * g.ldb + kk)
@@ -801,7 +829,9 @@ static int run_gemm(const char *who, int tA, int tB, int M, int N, int K, float 
                     const BlockHint *hint = nullptr) {
   int rc = check_gemm(who, tA, tB, M, N, K, A, lda, B, ldb, C, ldc);
   if (rc || M == 0 || N == 0) return rc;
-  GemmPlan p = plan_gemm(tA, tB, M, N, K, !pull && skinny_ok(tA, tB, K, A, lda, B, ldb), ws != nullptr);
+  // Looked-up rows: up to 128 of them the skinny kernel, beyond it the 64 x 64 tiles (M x 2048 x 300..512: 21
+  // rows 12.4 -> 7.9 us, 120 rows 19.7 -> 15.1, 300 rows 20.5 and 26.2).
+  GemmPlan p = plan_gemm(tA, tB, M, N, K, (!pull || M <= 128) && skinny_ok(tA, tB, K, A, lda, B, ldb), ws != nullptr);
   hipStream_t st = as_stream(stream);
   GemmArgs g{M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, D, ldd, dshift, p.kchunk, nullptr};
   if (hint) hint->set(&g, tA, tB, beta == 0.f && !D);

@@ -386,6 +386,7 @@ void Engine::get_param(const std::string &name, float *host, size_t n, bool grad
     src = pad_stage_.get();
   }
   readback_.read(host, src, n * 4, stream_);
+  idle_ = true;
 }
 
 // ------------------------------------------------------------------ profiling
@@ -669,9 +670,12 @@ void Engine::upload_index_arena() {
   if (group_lim > 0 && forest_)
     build_group_lists(s, nch_, t2j, pair, child, roots + s.B, group_lim, ngroups, cavs_group_rows(), &group_, h.host.get() + group_at);
   d_group_ = h.dev.get() + group_at;
-  check(cavs_memcpy_h2d(h.dev.get(), h.host.get(), (group_.first >= 0 ? group_at + group_.ints : total) * sizeof(int), sched_stream_));
-  check(cavs_event_record(h.up_ev, sched_stream_));
-  check(cavs_event_sync(h.up_ev));  // a few microseconds; the compute stream is still busy with the previous step
+  check(cavs_memcpy_h2d(h.dev.get(), h.host.get(), (group_.first >= 0 ? group_at + group_.ints : total) * sizeof(int),
+                        direct_ ? stream_ : sched_stream_));
+  if (!direct_) {
+    check(cavs_event_record(h.up_ev, sched_stream_));
+    check(cavs_event_sync(h.up_ev));  // a few microseconds; the compute stream is still busy with the previous step
+  }
   last_free_ev_ = h.free_ev;
   last_busy_ = &h.busy;
   d_t2j_ = h.dev.get();
@@ -926,6 +930,8 @@ const Schedule &Engine::schedule() {
 void Engine::begin_step(const int *graph, int B, int maxlen) {
   auto t0 = std::chrono::steady_clock::now();
   if (!graph || B <= 0 || maxlen <= 0) fail(CAVS_EINVAL, "graph feed rejected: empty graph feed");
+  direct_ = idle_;
+  idle_ = false;
   if (last_free_ev_) {  // everything that reads the previous step's lists is enqueued by now
     check(cavs_event_record(last_free_ev_, stream_));
     *last_busy_ = true;
@@ -1170,13 +1176,15 @@ void Engine::upload_feeds(const void *x, size_t nx, const void *labels, size_t n
     h.host.reserve(total);
     if (nx) std::memcpy(h.host.get(), x, nx * 4);
     if (nl) std::memcpy(h.host.get() + lab0, labels, nl * 4);
-    check(cavs_memcpy_h2d(h.dev.get(), h.host.get(), total * 4, sched_stream_));
+    check(cavs_memcpy_h2d(h.dev.get(), h.host.get(), total * 4, direct_ ? stream_ : sched_stream_));
   } else {
     if (nx) check(cavs_memcpy_h2d(h.dev.get(), x, nx * 4, sched_stream_));
     if (nl) check(cavs_memcpy_h2d(h.dev.at(lab0), labels, nl * 4, sched_stream_));
   }
-  check(cavs_event_record(h.up_ev, sched_stream_));
-  check(cavs_event_sync(h.up_ev));
+  if (!stage || !direct_) {
+    check(cavs_event_record(h.up_ev, sched_stream_));
+    check(cavs_event_sync(h.up_ev));
+  }
   hfeeds_used_ = &h;
   if (nx) d_x_ = h.dev.get();
   if (nl) d_labels_ = h.dev.at(lab0);
@@ -2547,6 +2555,7 @@ void Engine::aux_join() {
 void Engine::sync() {
   aux_join();
   check(cavs_stream_sync(stream_));
+  idle_ = true;
   tail_check();
 }
 
@@ -2577,6 +2586,7 @@ void Engine::fetch(const std::string &what, float *host, size_t n) {
   if (n != want || !host) fail(CAVS_EINVAL, "'" + what + "' holds " + std::to_string(want) + " floats, got " + std::to_string(n));
   if (blocks > 0) src = user_rows(src, N, blocks);
   readback_.read(host, src, want * 4, stream_);
+  idle_ = true;
   tail_check();
 }
 

@@ -168,6 +168,10 @@ class Engine {
   DeviceArray<float> pad_mask_;   // [H] 1 where a column is declared, 0 where it is padding
   void *stream_ = nullptr;
   bool own_stream_ = true;
+  // Nothing has been enqueued since the stream was last waited for.  A step that begins that way (one
+  // request at a time) sends its lists and feeds up on the stream itself: its kernels wait for them
+  // there, and the host neither records nor waits for an event.
+  bool idle_ = false, direct_ = false;
   void *ev_[4] = {nullptr, nullptr, nullptr, nullptr};  // fwd begin/end, bwd begin/end
   bool ev_valid_ = false, ev_bwd_valid_ = false;
   float parse_ms_ = 0.f, sched_ms_ = 0.f, wait_ms_ = 0.f, host_step_ms_ = 0.f;

@@ -64,6 +64,7 @@ class Readback {
  private:
   std::shared_ptr<ReadbackPool> pool_;
   std::vector<void *> events_;
+  PinnedArray<char> small_;
 };
 
 }  // namespace cavs
