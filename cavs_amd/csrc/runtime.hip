@@ -262,6 +262,14 @@ int cavs_event_create(void **event) {
   return CAVS_OK;
 }
 
+int cavs_event_create_device(void **event) {
+  CAVS_REQUIRE(event, "cavs_event_create_device: null out pointer");
+  hipEvent_t e;
+  CAVS_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
+  *event = e;
+  return CAVS_OK;
+}
+
 int cavs_event_destroy(void *event) {
   if (event) CAVS_HIP_TRY(hipEventDestroy(static_cast<hipEvent_t>(event)));
   return CAVS_OK;
@@ -351,6 +359,16 @@ int cavs_profile_arm(void *start_event, void *stop_event) {
   LaunchProbe &p = launch_probe();
   p.start = static_cast<hipEvent_t>(start_event);
   p.stop = static_cast<hipEvent_t>(stop_event);
+  p.armed = true;
+  p.started = false;
+  return CAVS_OK;
+}
+
+int cavs_stop_event_arm(void *event) {
+  CAVS_REQUIRE(event, "cavs_stop_event_arm: null event");
+  LaunchProbe &p = launch_probe();
+  p.start = nullptr;
+  p.stop = static_cast<hipEvent_t>(event);
   p.armed = true;
   p.started = false;
   return CAVS_OK;

@@ -146,6 +146,8 @@ _SIGS = {
     "cavs_treefc_round_bwd_children_act": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
     "cavs_treefc_bwd_rows": [_P, _I, _P, _P, _P, _P, _I, _I, _P],
     "cavs_profile_arm": [_P, _P],
+    "cavs_stop_event_arm": [_P],
+    "cavs_event_create_device": [C.POINTER(_P)],
     "cavs_profile_disarm": [_P],
     "cavs_fc_softmax_xent": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _P],
     "cavs_run_tasks": [_I, C.POINTER(Task), _P],

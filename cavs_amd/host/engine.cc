@@ -58,7 +58,8 @@ Engine::Engine(const cavs_session_config &cfg, void *external_stream, std::share
     stream_ = external_stream;
   else
     check(cavs_stream_create(&stream_));
-  for (auto &e : ev_) check(cavs_event_create(&e));
+  for (auto &e : ev_) check(cavs_event_create_device(&e));
+  for (auto &m : marks_) check(cavs_event_create_device(&m.ev));
   // where the blocks of the declared parameters lie in the stored ones (none: they are the same)
   auto gates = [&](bool pad, size_t user, size_t eng, int n, size_t rows) {  // [rows, n h] -> [., n H]: a block per gate
     std::vector<PadBlock> b;
@@ -245,11 +246,9 @@ Engine::~Engine() {
   for (CellStage &st : cells_) cavs_cell_release(st.module);
   for (auto &e : ev_) cavs_event_destroy(e);
   for (auto &h : hlists_) {
-    if (h.free_ev) cavs_event_destroy(h.free_ev);
     if (h.up_ev) cavs_event_destroy(h.up_ev);
   }
   for (auto &h : hfeeds_) {
-    if (h.free_ev) cavs_event_destroy(h.free_ev);
     if (h.up_ev) cavs_event_destroy(h.up_ev);
   }
   for (auto &e : prof_events_) cavs_event_destroy(e);
@@ -265,8 +264,8 @@ Engine::~Engine() {
   }
   for (void *e : chunk_done_ev_)
     if (e) cavs_event_destroy(e);
-  for (auto &d : dsched_)
-    if (d.free_ev) cavs_event_destroy(d.free_ev);
+  for (auto &m : marks_)
+    if (m.ev) cavs_event_destroy(m.ev);
   if (own_stream_) cavs_stream_destroy(stream_);
 }
 
@@ -386,7 +385,7 @@ void Engine::get_param(const std::string &name, float *host, size_t n, bool grad
     src = pad_stage_.get();
   }
   readback_.read(host, src, n * 4, stream_);
-  idle_ = true;
+  stream_idle();
 }
 
 // ------------------------------------------------------------------ profiling
@@ -648,14 +647,14 @@ void Engine::upload_index_arena() {
   HostLists &h = hlists_[hlists_slot_];
   hlists_slot_ ^= 1;
   if (!sched_stream_) check(cavs_stream_create(&sched_stream_));
-  if (!h.free_ev) check(cavs_event_create(&h.free_ev));
   if (!h.up_ev) check(cavs_event_create(&h.up_ev));
-  if (h.busy) {
+  {
     auto w0 = std::chrono::steady_clock::now();
-    check(cavs_event_sync(h.free_ev));
+    wait_step(h.used);
     wait_ms_ = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - w0).count();
-    h.busy = false;
   }
+  h.used = steps_;
+  buffers_used_ = true;
   h.host.reserve(grow(room, h.host.capacity()));
   h.dev.reserve(grow(room, h.dev.capacity()));
   int *t2j = h.host.get(), *pair = t2j + N, *child = pair + N, *roots = child + (size_t)nch_ * N;
@@ -676,8 +675,6 @@ void Engine::upload_index_arena() {
     check(cavs_event_record(h.up_ev, sched_stream_));
     check(cavs_event_sync(h.up_ev));  // a few microseconds; the compute stream is still busy with the previous step
   }
-  last_free_ev_ = h.free_ev;
-  last_busy_ = &h.busy;
   d_t2j_ = h.dev.get();
   d_pair_ = d_t2j_ + N;
   d_child_ = d_pair_ + N;
@@ -792,13 +789,13 @@ void Engine::schedule_on_device(const int *graph, int B, int maxlen) {
   DeviceSched &d = dsched_[dsched_slot_];
   dsched_slot_ ^= 1;
   if (!sched_stream_) check(cavs_stream_create(&sched_stream_));
-  if (!d.free_ev) check(cavs_event_create(&d.free_ev));
-  if (d.busy) {  // the step before last read these lists
+  {  // the step before last read these lists
     auto w0 = std::chrono::steady_clock::now();
-    check(cavs_event_sync(d.free_ev));
+    wait_step(d.used);
     wait_ms_ = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - w0).count();
-    d.busy = false;
   }
+  d.used = steps_;
+  buffers_used_ = true;
   const size_t BM = (size_t)B * maxlen, nmeta = (size_t)maxlen + 9;
   const size_t need = BM * (2 + 2 * (size_t)nch_) + 2 * (size_t)B;
   d.graph_host.reserve(BM);
@@ -898,8 +895,6 @@ void Engine::schedule_on_device(const int *graph, int B, int maxlen) {
       d_group_ = d.tail_dev.get();
     }
   }
-  last_free_ev_ = d.free_ev;
-  last_busy_ = &d.busy;
   sched_ms_ = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
 
@@ -926,22 +921,36 @@ const Schedule &Engine::schedule() {
   return *sched_;
 }
 
+void Engine::wait_step(uint64_t step) {
+  if (step <= done_step_) return;
+  const StepMark *best = nullptr;  // the earliest mark at or behind that step
+  for (const StepMark &m : marks_)
+    if (m.step >= step && (!best || m.step < best->step)) best = &m;
+  if (best) {
+    check(cavs_event_sync(best->ev));
+    done_step_ = best->step;
+  } else {
+    check(cavs_stream_sync(stream_));
+    done_step_ = steps_ - 1;  // (the current step may have enqueued nothing yet)
+  }
+}
+
 // ------------------------------------------------------------------ step
 void Engine::begin_step(const int *graph, int B, int maxlen) {
   auto t0 = std::chrono::steady_clock::now();
   if (!graph || B <= 0 || maxlen <= 0) fail(CAVS_EINVAL, "graph feed rejected: empty graph feed");
   direct_ = idle_;
   idle_ = false;
-  if (last_free_ev_) {  // everything that reads the previous step's lists is enqueued by now
-    check(cavs_event_record(last_free_ev_, stream_));
-    *last_busy_ = true;
-    last_free_ev_ = nullptr;
+  if (!direct_ && buffers_used_ && !end_stamped_) {  // everything of the previous step is enqueued by now
+    StepMark &m = marks_[steps_ & 3];
+    check(cavs_event_record(m.ev, stream_));
+    m.step = steps_;
   }
-  if (hfeeds_used_) {
-    check(cavs_event_record(hfeeds_used_->free_ev, stream_));
-    hfeeds_used_->busy = true;
-    hfeeds_used_ = nullptr;
-  }
+  // (the forward pass's time counts from the end of the step before while steps follow each other)
+  begin_ev_ = !direct_ && end_stamped_ ? marks_[steps_ & 3].ev : nullptr;
+  steps_++;
+  end_stamped_ = buffers_used_ = false;
+  std::fill(stamped_, stamped_ + 4, false);
   c_gather_rows_ = c_scatter_rows_ = c_gemm_flops_ = c_gemm_flops_hinted_ = c_launches_ = c_gather_bytes_ = c_scatter_bytes_ = 0;
   c_round_flops_ = 0;
   c_tail_rounds_ = c_tail_launches_ = 0;
@@ -1006,7 +1015,8 @@ void Engine::forward_only(const int *graph, int B, int maxlen, const float *x_de
   const bool reads_x = cell_ ? cell_->NX > 0 || cell_->XD > 0 : (cfg_.model != CAVS_MODEL_TREEFC || cfg_.use_x);
   if (reads_x && !x_dev) fail(CAVS_EINVAL, "vertex input feed is null");
   d_x_ = x_dev;
-  check(cavs_event_record(ev_[0], stream_));
+  begin_ev_ = nullptr;
+  mark_point(0);
   fwd_out_ = graph_out && uH_ == cfg_.H ? graph_out : GO_.get();
   out_folded_ = false;
   head_chunked_ = false;
@@ -1024,7 +1034,7 @@ void Engine::forward_only(const int *graph, int B, int maxlen, const float *x_de
     check(cavs_copy_rows(graph_out ? graph_out : go_user_.get(), uH_, fwd_out_, cfg_.H, N_, uH_, stream_));
     c_launches_ += 1;
   }
-  check(cavs_event_record(ev_[1], stream_));
+  mark_point(1);
   ev_valid_ = true;
   ev_bwd_valid_ = false;
 }
@@ -1039,7 +1049,7 @@ void Engine::backward_only(const float *dgraph_out, bool settle_biases) {
   state_epoch_++;
   d_dgo_ = dgraph_out;
   head_chunked_ = false;
-  check(cavs_event_record(ev_[2], stream_));
+  mark_point(2);
   if (uH_ != cfg_.H) {  // (the columns beyond stay zero)
     check(cavs_copy_rows(dGO_.get(), cfg_.H, dgraph_out, uH_, N_, uH_, stream_));
     c_launches_ += 1;
@@ -1060,29 +1070,29 @@ void Engine::backward_only(const float *dgraph_out, bool settle_biases) {
     }
     copy_blocks(jobs);
   }
-  check(cavs_event_record(ev_[3], stream_));
+  mark_point(3);
   ev_bwd_valid_ = true;
 }
 
 // The forward rounds, the loss head and the backward rounds of a step (everything between the
 // feeds and the parameter update).  While a graph is being recorded the timing events stay out of it.
 void Engine::run_passes(bool backward) {
-  if (!capturing_) check(cavs_event_record(ev_[0], stream_));
+  if (!capturing_ && !begin_ev_) mark_point(0);
   fwd_out_ = GO_.get();
   out_folded_ = false;
   head_chunked_ = backward && !head_chunks_.empty() && !profile_ && !capturing_ && cfg_.loss == CAVS_LOSS_SOFTMAX;
   model_forward();
   pop_ret(GO_.get());
-  if (!capturing_) check(cavs_event_record(ev_[1], stream_));
+  if (!capturing_) mark_point(1);
   ev_valid_ = !capturing_;
   head_forward_backward(backward);
   d_dgo_ = dGO_.get();
   did_backward_ = backward;
   ev_bwd_valid_ = false;
   if (backward) {
-    if (!capturing_) check(cavs_event_record(ev_[2], stream_));
+    if (!capturing_) mark_point(2);
     model_backward();
-    if (!capturing_) check(cavs_event_record(ev_[3], stream_));
+    if (!capturing_) mark_point(3);
     ev_bwd_valid_ = !capturing_;
   }
 }
@@ -1163,12 +1173,10 @@ void Engine::upload_feeds(const void *x, size_t nx, const void *labels, size_t n
   HostFeeds &h = hfeeds_[hfeeds_slot_];
   hfeeds_slot_ ^= 1;
   if (!sched_stream_) check(cavs_stream_create(&sched_stream_));
-  if (!h.free_ev) check(cavs_event_create(&h.free_ev));
   if (!h.up_ev) check(cavs_event_create(&h.up_ev));
-  if (h.busy) {  // the step before last read these
-    check(cavs_event_sync(h.free_ev));
-    h.busy = false;
-  }
+  wait_step(h.used);  // (the step before last)
+  h.used = steps_;
+  buffers_used_ = true;
   h.dev.reserve(grow(total, h.dev.capacity()));
   // (rows of megabytes: the runtime's own path for pageable memory copies them no slower than this thread would)
   const bool stage = total * 4 <= (size_t(1) << 20);
@@ -1185,7 +1193,6 @@ void Engine::upload_feeds(const void *x, size_t nx, const void *labels, size_t n
     check(cavs_event_record(h.up_ev, sched_stream_));
     check(cavs_event_sync(h.up_ev));
   }
-  hfeeds_used_ = &h;
   if (nx) d_x_ = h.dev.get();
   if (nl) d_labels_ = h.dev.at(lab0);
 }
@@ -1298,7 +1305,9 @@ void Engine::step(const int *graph, int B, int maxlen, const void *x, const void
         }
         tasks.push_back({CAVS_TASK_SGD, lr, (long long)p.n, 0, 0, p.w, p.g, nullptr, nullptr});
       }
-      check(cavs_run_tasks((int)tasks.size(), tasks.data(), stream_));
+      StepMark &m = marks_[steps_ & 3];
+      stamping(m.ev, &end_stamped_, [&] { check(cavs_run_tasks((int)tasks.size(), tasks.data(), stream_)); });
+      if (end_stamped_) m.step = steps_;
       c_launches_ += 1;
     } else {
       settle_bias_jobs(0.f, nullptr);
@@ -1328,7 +1337,7 @@ void Engine::model_backward() {
 
 void Engine::pop_ret(float *graph_out) {
   if (out_folded_) return;  // already written by the rounds
-  scatter(graph_out, cfg_.H, d_t2j_, msg_.get(), mw_, N_, cfg_.H);
+  last_launch(1, true, [&] { scatter(graph_out, cfg_.H, d_t2j_, msg_.get(), mw_, N_, cfg_.H); });
 }
 
 // ------------------------------------------------------------------ Tree-LSTM
@@ -1377,11 +1386,13 @@ void Engine::treelstm_forward() {
   for (size_t rk = 0; rk < sched_->rounds.size(); rk++) {
     const Round &r = sched_->rounds[rk];
     if (rk == tail_from) {
-      CAVS_TIMED(K_ROUND, cavs_treelstm_tail_fwd(pool_.get(), d_child_, d_pair_, xW_.get(), 4 * H, Upk_.get(), Bv, G_.get(), hlr_.get(),
-                                                 gates_.get(), out_folded_ ? nullptr : msg_.get(), go, d_t2j_, d_tail_rows_,
-                                                 (int)tail_.nrounds.size(), tail_.nrounds.data(), tail_.start.data(), tail_.count.data(),
-                                                 tail_.flags.data(), tail_.max_rounds, H, reinterpret_cast<unsigned *>(tail_sync_.get()), kTailSpins, 0,
-                                                 stream_));
+      last_launch(1, out_folded_, [&] {
+        CAVS_TIMED(K_ROUND, cavs_treelstm_tail_fwd(pool_.get(), d_child_, d_pair_, xW_.get(), 4 * H, Upk_.get(), Bv, G_.get(), hlr_.get(),
+                                                   gates_.get(), out_folded_ ? nullptr : msg_.get(), go, d_t2j_, d_tail_rows_,
+                                                   (int)tail_.nrounds.size(), tail_.nrounds.data(), tail_.start.data(), tail_.count.data(),
+                                                   tail_.flags.data(), tail_.max_rounds, H, reinterpret_cast<unsigned *>(tail_sync_.get()), kTailSpins,
+                                                   0, stream_));
+      });
       c_round_flops_ += tail_.flops;
       c_gather_rows_ += 2.0 * tail_.vertices;
       c_scatter_rows_ += tail_.vertices;
@@ -1393,8 +1404,10 @@ void Engine::treelstm_forward() {
     }
     if (group_.first >= 0 && (int)rk == group_.first) {
       const cavs_group_plan plan = group_plan(group_.fwd);
-      CAVS_TIMED(K_ROUND, cavs_treelstm_group_fwd(pool_.get(), xW_.get(), 4 * H, Upk_.get(), Bv, G_.get(), hlr_.get(), gates_.get(),
-                                                  out_folded_ ? nullptr : msg_.get(), go, H, &plan, stream_));
+      last_launch(1, out_folded_, [&] {
+        CAVS_TIMED(K_ROUND, cavs_treelstm_group_fwd(pool_.get(), xW_.get(), 4 * H, Upk_.get(), Bv, G_.get(), hlr_.get(), gates_.get(),
+                                                    out_folded_ ? nullptr : msg_.get(), go, H, &plan, stream_));
+      });
       group_launched();
       break;
     }
@@ -1609,7 +1622,7 @@ void Engine::treelstm_backward() {
   const int lp = sched_->leaf_prefix;
   float *dU = param("U").g;
   const bool bias_row = bias_row_ok();  // the ones column of e_ turns row E of dW into the column sums of dxW
-  gemm_group_embedding_backward({
+  const std::vector<cavs_gemm_desc> products = {
       {0, 1, N, E, 4 * H, 1.f, 0.f, dxW_.get(), 4 * H, W, 4 * H, de_.get(), E, CAVS_GEMM_A_ZERO, lp, 3 * H},
       // (all four padding columns of e_ take part, so that the product keeps 16-byte operand loads)
       {1, 0, bias_row ? ld_e_ : E, 4 * H, N, 1.f, 0.f, e_.get(), ld_e_, dxW_.get(), 4 * H, param("W").g, 4 * H, CAVS_GEMM_B_ZERO, lp,
@@ -1617,7 +1630,8 @@ void Engine::treelstm_backward() {
       {1, 0, H, 3 * H, N - lp, 1.f, 0.f, hlr_.at((size_t)lp * H), H, dxW_.at((size_t)lp * 4 * H), 4 * H, dU, 3 * H},
       {1, 0, H, H, 2 * (N - lp), 1.f, 0.f, G_.at((size_t)2 * lp * 2 * H), 2 * H, dF_.at((size_t)2 * lp * H), H,
        dU + (size_t)3 * H * H, H},
-  }, E);
+  };
+  last_launch(3, bias_row, [&] { gemm_group_embedding_backward(products, E); });
   // bias blocks [i|f|u|o] from dxW columns [i|o|u|f]
   if (bias_row) {
     // settled by the launch that ends the step (or right after this pass); block k of the row
@@ -1774,7 +1788,9 @@ void Engine::lstm_forward() {
     const Round &r = sched_->rounds[rk];
     if (group_.first >= 0 && (int)rk == group_.first) {
       const cavs_group_plan plan = group_plan(group_.fwd);
-      CAVS_TIMED(K_ROUND, cavs_lstm_group_fwd(pool_.get(), xW_.get(), 4 * H, Upk_.get(), Bv, G_.get(), gates_.get(), msg_.get(), go, H, &plan, stream_));
+      last_launch(1, out_folded_, [&] {
+        CAVS_TIMED(K_ROUND, cavs_lstm_group_fwd(pool_.get(), xW_.get(), 4 * H, Upk_.get(), Bv, G_.get(), gates_.get(), msg_.get(), go, H, &plan, stream_));
+      });
       group_launched();
       break;
     }
@@ -1911,7 +1927,7 @@ void Engine::lstm_backward() {
       {1, 0, H, 4 * H, N - lp, 1.f, 0.f, G_.at((size_t)lp * 2 * H), 2 * H, dxW_.at((size_t)lp * 4 * H), 4 * H,
        dW + (size_t)4 * H * E, 4 * H},
   }, E);
-  bias_gradient("Bv", dxW_.get(), N, 4 * H, bias_parts_);
+  last_launch(3, true, [&] { bias_gradient("Bv", dxW_.get(), N, 4 * H, bias_parts_); });
 }
 
 // ------------------------------------------------------------------ Tree-FC
@@ -1930,8 +1946,10 @@ void Engine::treefc_forward() {
     const Round &r = sched_->rounds[rk];
     if (group_.first >= 0 && (int)rk == group_.first) {
       const cavs_group_plan plan = group_plan(group_.fwd);
-      CAVS_TIMED(K_ROUND, cavs_treefc_group_fwd(pool_.get(), cfg_.use_x ? xs_.get() : nullptr, Upk_.get(), Bv, G_.get(), msg_.get(), go, H, cfg_.act, &plan,
-                                                stream_));
+      last_launch(1, out_folded_, [&] {
+        CAVS_TIMED(K_ROUND, cavs_treefc_group_fwd(pool_.get(), cfg_.use_x ? xs_.get() : nullptr, Upk_.get(), Bv, G_.get(), msg_.get(), go, H, cfg_.act,
+                                                  &plan, stream_));
+      });
       group_launched();
       break;
     }
@@ -2036,7 +2054,7 @@ void Engine::treefc_backward() {
   gemm_splitk(1, 0, 2 * H, H, N - lp, G_.at((size_t)2 * lp * H), 2 * H, dxW_.at((size_t)lp * H), H,
               param("W").g, H);
   if (cfg_.use_bias) {
-    bias_gradient("Bv", dxW_.get(), N, H, bias_parts_);
+    last_launch(3, true, [&] { bias_gradient("Bv", dxW_.get(), N, H, bias_parts_); });
   }
 }
 
@@ -2339,8 +2357,10 @@ void Engine::head_forward_backward(bool backward) {
         check(cavs_stream_sync(stream_));  // the last step's jobs may still read the old buffer
         head_parts_.reserve(head_bytes / 4 + 1);
       }
-      check(cavs_fc_softmax_xent(GO_.get(), Wfc.w, bfc.w, d_labels_, loss_.get(), logits_.get(), backward ? dGO_.get() : nullptr,
-                                 nullptr, nullptr, head_parts_.get(), head_bytes, N, H, C, stream_));
+      last_launch(2, backward, [&] {
+        check(cavs_fc_softmax_xent(GO_.get(), Wfc.w, bfc.w, d_labels_, loss_.get(), logits_.get(), backward ? dGO_.get() : nullptr,
+                                   nullptr, nullptr, head_parts_.get(), head_bytes, N, H, C, stream_));
+      });
       if (backward)
         pending_tasks_.push_back({CAVS_TASK_SUM_PARTS, 0.f, cavs_fc_softmax_xent_parts(N), (long long)C * H + C, (long long)C * H,
                                   head_parts_.get(), Wfc.g, bfc.g, nullptr});
@@ -2390,7 +2410,7 @@ void Engine::head_forward_backward(bool backward) {
       } else {
         // both read d logits and write different outputs: one launch when they are small
         gemm_group({dWd, dGd});
-        bias_gradient("bfc", dlogits_.get(), N, C, head_bias_parts_);
+        last_launch(2, true, [&] { bias_gradient("bfc", dlogits_.get(), N, C, head_bias_parts_); });
       }
     }
     return;
@@ -2555,7 +2575,7 @@ void Engine::aux_join() {
 void Engine::sync() {
   aux_join();
   check(cavs_stream_sync(stream_));
-  idle_ = true;
+  stream_idle();
   tail_check();
 }
 
@@ -2586,7 +2606,7 @@ void Engine::fetch(const std::string &what, float *host, size_t n) {
   if (n != want || !host) fail(CAVS_EINVAL, "'" + what + "' holds " + std::to_string(want) + " floats, got " + std::to_string(n));
   if (blocks > 0) src = user_rows(src, N, blocks);
   readback_.read(host, src, want * 4, stream_);
-  idle_ = true;
+  stream_idle();
   tail_check();
 }
 
@@ -2599,7 +2619,7 @@ float Engine::timing(const std::string &name) {
   if (name == "HostWait") return wait_ms_;
   if (name == "HostStep") return host_step_ms_;
   if (name == "RNNForward" && ev_valid_) {
-    check(cavs_event_elapsed_ms(&ms, ev_[0], ev_[1]));
+    check(cavs_event_elapsed_ms(&ms, begin_ev_ ? begin_ev_ : ev_[0], ev_[1]));
     return ms;
   }
   if (name == "RNNBackward" && ev_bwd_valid_) {

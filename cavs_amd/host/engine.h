@@ -174,6 +174,48 @@ class Engine {
   bool idle_ = false, direct_ = false;
   void *ev_[4] = {nullptr, nullptr, nullptr, nullptr};  // fwd begin/end, bwd begin/end
   bool ev_valid_ = false, ev_bwd_valid_ = false;
+  // An event recorded between two kernels holds the second one back by four microseconds, and a step has
+  // five such points (the ends of its passes, and the end of the step, behind which the buffers the
+  // host filled for it are free).  So the last kernel before a point stamps the event itself where
+  // the engine knows which one that is; the event is recorded only where it does not.
+  bool stamped_[4] = {false, false, false, false};
+  template <class F>
+  void stamping(void *ev, bool *stamped, F &&call) {
+    if (profile_ || capturing_) return call();
+    check(cavs_stop_event_arm(ev));
+    int launched = 0;
+    try {
+      call();
+    } catch (...) {
+      cavs_profile_disarm(nullptr);
+      throw;
+    }
+    check(cavs_profile_disarm(&launched));
+    *stamped = launched != 0;
+  }
+  // the last launch of a pass (point: 1 end of the forward rounds, 2 before the backward pass, 3 its end)
+  template <class F>
+  void last_launch(int point, bool last, F &&call) {
+    if (last) stamping(ev_[point], &stamped_[point], call);
+    else call();
+  }
+  void mark_point(int point) {
+    if (!stamped_[point]) check(cavs_event_record(ev_[point], stream_));
+    stamped_[point] = false;
+  }
+  // When the steps ended: the events of the last few, and up to which one they are known to be over.
+  struct StepMark {
+    void *ev = nullptr;
+    uint64_t step = 0;
+  } marks_[4];
+  uint64_t steps_ = 0, done_step_ = 0;
+  bool end_stamped_ = false, buffers_used_ = false;  // of the current step
+  void *begin_ev_ = nullptr;                          // where the forward pass's time counts from
+  void wait_step(uint64_t step);                      // returns when that step's kernels are over
+  void stream_idle() {
+    idle_ = true;
+    done_step_ = steps_;
+  }
   float parse_ms_ = 0.f, sched_ms_ = 0.f, wait_ms_ = 0.f, host_step_ms_ = 0.f;
   std::map<std::string, std::unique_ptr<Param>> params_;
 
@@ -185,16 +227,13 @@ class Engine {
   int N_ = 0, cap_ = 0, rcap_ = 0, E_ = 0, mw_ = 0, nch_ = 1;
 
   // per-step device index arena: [t2j | pair | child | roots | kid_rows | orphans]
-  struct HostLists {  // host-built lists: pinned staging, their device copy, and who still reads it
+  struct HostLists {  // host-built lists: pinned staging, their device copy, and who reads it
     PinnedArray<int> host;
     DeviceArray<int> dev;
-    void *free_ev = nullptr, *up_ev = nullptr;
-    bool busy = false;
+    void *up_ev = nullptr;
+    uint64_t used = 0;  // the step that reads them (0: none)
   } hlists_[2];
   int hlists_slot_ = 0;
-  // the event to record, and the flag to raise, once the current step's kernels are all enqueued
-  void *last_free_ev_ = nullptr;
-  bool *last_busy_ = nullptr;
   const int *d_t2j_ = nullptr, *d_pair_ = nullptr, *d_child_ = nullptr, *d_roots_ = nullptr;
   // Tree-LSTM, message flow of the batch is a forest: children by slab row, and the slab rows
   // nobody sends a message to
@@ -209,8 +248,7 @@ class Engine {
     PinnedArray<int> graph_host, meta_host, kid_host, tail_host;  // (tail_host: the group launches' block as well)
     DeviceArray<int> graph_dev, lists, meta_dev, tail_dev;
     long cap = 0;          // rows per list
-    void *free_ev = nullptr;  // recorded once everything that read `lists` has been enqueued
-    bool busy = false;
+    uint64_t used = 0;     // the step that reads `lists`
   } dsched_[2];
   DeviceArray<int> dsched_scratch_;
   void *sched_stream_ = nullptr;
@@ -335,11 +373,10 @@ class Engine {
   struct HostFeeds {
     PinnedArray<float> host;
     DeviceArray<float> dev;
-    void *free_ev = nullptr, *up_ev = nullptr;
-    bool busy = false;
+    void *up_ev = nullptr;
+    uint64_t used = 0;
   } hfeeds_[2];
   int hfeeds_slot_ = 0;
-  HostFeeds *hfeeds_used_ = nullptr;  // what the current step reads
   void upload_feeds(const void *x, size_t nx, const void *labels, size_t nl);
   const float *d_x_ = nullptr, *d_labels_ = nullptr, *d_dgo_ = nullptr;
 

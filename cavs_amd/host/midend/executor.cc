@@ -748,8 +748,8 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
       if (!copy_stream_) {
         check(cavs_stream_create(&copy_stream_));
         check(cavs_event_create(&feeds_up_ev_));
-        check(cavs_event_create(&run_done_ev_[0]));
-        check(cavs_event_create(&run_done_ev_[1]));
+        check(cavs_event_create_device(&run_done_ev_[0]));
+        check(cavs_event_create_device(&run_done_ev_[1]));
       }
       FeedStage &st = feed_stages_[f.first];
       const size_t bytes = (size_t)t.width * 4;
@@ -776,9 +776,10 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
   struct MarkRunDone {  // once everything this Run enqueues is in the stream, whichever way it leaves
     Executor *e;
     int parity;
-    bool on;
+    bool on, stamped = false;  // (stamped: the last kernel of the Run recorded the event itself)
     ~MarkRunDone() {
-      if (on && cavs_event_record(e->run_done_ev_[parity], e->stream_) == CAVS_OK) e->run_busy_[parity] = true;
+      if (on && stamped) e->run_busy_[parity] = true;
+      else if (on && cavs_event_record(e->run_done_ev_[parity], e->stream_) == CAVS_OK) e->run_busy_[parity] = true;
     }
   } mark_done{this, parity, copy_stream_ != nullptr};  // every Run, so that a later one can tell when this one's reads are over
   bool train = false;
@@ -885,7 +886,13 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
       if (engine_ && engine_->update_jobs(w.base, gr.base, g.opt.lr, &updates)) continue;
       updates.push_back({CAVS_TASK_SGD, g.opt.lr, (long long)w.count(), 0, 0, w.base, gr.base, nullptr, nullptr});
     }
-    check(cavs_run_tasks((int)updates.size(), updates.data(), stream_));
+    const bool stamp = mark_done.on && pass + 1 == passes;
+    if (stamp) check(cavs_stop_event_arm(run_done_ev_[parity]));
+    const int rc = cavs_run_tasks((int)updates.size(), updates.data(), stream_);
+    int launched = 0;
+    if (stamp) check(cavs_profile_disarm(&launched));
+    check(rc);
+    mark_done.stamped = launched != 0;
   }
   }  // passes
   results->assign(outputs.size(), nullptr);

@@ -60,6 +60,10 @@ int cavs_stream_create(void **stream);
 int cavs_stream_destroy(void *stream);
 int cavs_stream_sync(void *stream);
 int cavs_event_create(void **event);
+/* For events that are recorded between kernels of one device and waited for by the host or by another
+ * stream of it: recording one does not flush the caches to the host (2.6 us between dependent
+ * kernels, 4.1 otherwise).  Not for a host that goes on to read memory the kernels wrote. */
+int cavs_event_create_device(void **event);
 int cavs_event_destroy(void *event);
 int cavs_event_record(void *event, void *stream);
 int cavs_event_sync(void *event); /* host waits until the event has happened */
@@ -74,6 +78,10 @@ int cavs_event_elapsed_ms(float *ms, void *start, void *stop);
  * reference (it times whole statements on the host, cavs/midend/statement.cc:53-84). */
 int cavs_profile_arm(void *start_event, void *stop_event);
 int cavs_profile_disarm(int *launched); /* waits for `stop` */
+/* The stop half alone: until cavs_profile_disarm every kernel this thread launches through the library
+ * stamps `event` when it ends.  What follows such a kernel need not wait for a packet of the event's own
+ * in the stream (measured between dependent kernels: 1.5 us against 4.1 for cavs_event_record). */
+int cavs_stop_event_arm(void *event);
 
 /* A stretch of a stream's work recorded once and enqueued again as one call: everything enqueued on
  * `stream` between cavs_graph_capture_begin and cavs_graph_capture_end is recorded instead of run

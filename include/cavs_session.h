@@ -158,7 +158,8 @@ int cavs_schedule_trace_from_lists(int B, int maxlen, int N, int nchild, const i
                                    int with_backward, int *out, int cap);
 
 /* Timers of the last step in ms, by the reference's names (cavs/midend/statement.cc:
- * 53,65,68,84,102,122): "GraphParsing" (host), "RNNForward", "RNNBackward" (device); and the
+ * 53,65,68,84,102,122): "GraphParsing" (host), "RNNForward", "RNNBackward" (device; the forward time of a
+ * step that directly follows another counts from the end of that one); and the
  * host-side split "HostSchedule" (scheduler), "HostWait" (waiting for the device to release
  * an index staging buffer), "HostStep" (the whole enqueueing call). */
 int cavs_session_timing(cavs_session *s, const char *name, float *ms);
