@@ -1,0 +1,124 @@
+// What the matrix product kernels share: their arguments, how workgroups map to tiles, which part of
+// K a tile runs over and how its accumulators are stored.
+#pragma once
+#include "common.h"
+
+namespace cavs {
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+constexpr int kThreads = 256;
+
+struct GemmArgs {
+  int M, N, K;
+  const float *A;
+  long lda;
+  const float *B;
+  long ldb;
+  float *C;
+  long ldc;
+  float alpha, beta;
+  const float *D;  // optional addend rows D[r >> dshift, :]
+  long ldd;
+  int dshift;
+  int kchunk;      // K range per blockIdx.y (multiple of BK); == K when not split
+  float *ws;       // split-K workspace (counters + partial tiles) or nullptr
+  // cavs_embed_pull_sgemm (NN form only): row r of A is row int(pull_x[pull_rows[r]] * K) / K of the
+  // table A points at (a negative id: a zero row); the workgroups of a row tile also leave the
+  // rows they read in pull_copy (row stride ld_copy; each takes every tilesN-th k-tile) and those
+  // of the first column tile the ids in pull_ids
+  const int *pull_rows = nullptr;
+  const float *pull_x = nullptr;
+  float *pull_copy = nullptr;
+  long ld_copy = 0;
+  float *pull_ids = nullptr;
+  // A block the caller knows about (cavs_gemm_desc::zero_kind and friends): the tiles it covers
+  // run a shorter k range, or none
+  int zkind = 0, zrows = 0, zcol = 0;
+  // > 0: the launch is two launches back to back, the first zseg tiles (the row tiles inside the
+  // block, whose workgroups do less) and the rest, each padded to a multiple of 8 workgroups and
+  // dealt to the XCDs by itself: with one deal over all tiles the XCDs that hold the first
+  // tiles would finish early and the others set the time as before
+  int zseg = 0;
+};
+
+// Remap the linear workgroup id so that ids that are consecutive after the remap
+// were dispatched to the same XCD (hardware deals workgroups round-robin over 8 XCDs).
+__device__ inline int xcd_remap(int l, int total) {
+  constexpr int X = 8;
+  int per = total / X, rem = total % X;
+  int xcd = l % X, local = l / X;
+  return xcd * per + (xcd < rem ? xcd : rem) + local;
+}
+
+// The part of K the tile at (m0, n0) of split `z` runs over.
+template <int BM, int BN, bool TA, bool TB>
+__device__ inline void tile_k_range(const GemmArgs &g, int m0, int n0, int z, int *beg, int *end) {
+  int kbeg = z * g.kchunk;
+  int kend = min(g.K, kbeg + g.kchunk);
+  if (g.zkind == CAVS_GEMM_C_UNUSED) {  // rows below zrows of C are not wanted from column zcol on: left zero
+    if (m0 + BM <= g.zrows && n0 >= g.zcol) kend = kbeg;
+  } else if (g.zkind == CAVS_GEMM_A_ZERO) {  // rows below zrows of A (row-major M x K) are zero from k = zcol on
+    if (!TA && m0 + BM <= g.zrows) kend = max(kbeg, min(kend, g.zcol));
+  } else if (g.zkind == CAVS_GEMM_B_ZERO) {  // rows k < zrows of B (row-major K x N) are zero from column zcol on
+    if (!TB && n0 >= g.zcol) kbeg = min(kend, max(kbeg, g.zrows / 32 * 32));
+  }
+  *beg = kbeg;
+  *end = kend;
+}
+
+// Stores the TM x TN accumulators of a wavefront whose first row and column are m0 and n0; `more`: adds them
+// to what the same wavefront has stored before.
+template <int TM, int TN>
+__device__ inline void store_tile(const GemmArgs &g, const floatx16 (&acc)[TM][TN], int m0, int n0, int z, int lane, bool more) {
+  const int khalf = lane >> 5;
+  // C layout of the 32x32 accumulator: element r of lane l is row 8*(r/4) + 4*(l/32) + r%4,
+  // column l%32.
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      const int col = n0 + 32 * j + (lane & 31);
+      if (col >= g.N) continue;
+      const int rbase = m0 + 32 * i + 4 * khalf;
+      if (more) {
+        float *c = g.ws ? g.ws + (long)z * g.M * g.N + col : g.C + col;
+        const long ld = g.ws ? g.N : g.ldc;
+        const float alpha = g.ws ? 1.f : g.alpha;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int row = rbase + 8 * (r / 4) + (r % 4);
+          if (row < g.M) c[row * ld] += alpha * acc[i][j][r];
+        }
+        continue;
+      }
+      // the three forms of the store are chosen once per tile (the conditions are the same
+      // for every lane), not once per element
+      if (g.ws) {  // split K: park the partial sum, the reduce kernel finishes the job
+        float *w = g.ws + (long)z * g.M * g.N + col;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int row = rbase + 8 * (r / 4) + (r % 4);
+          if (row < g.M) w[(long)row * g.N] = acc[i][j][r];
+        }
+      } else if (g.beta == 0.f && !g.D) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int row = rbase + 8 * (r / 4) + (r % 4);
+          if (row < g.M) g.C[row * g.ldc + col] = g.alpha * acc[i][j][r];
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int row = rbase + 8 * (r / 4) + (r % 4);
+          if (row >= g.M) continue;
+          float v = g.alpha * acc[i][j][r];
+          if (g.beta != 0.f) v += g.beta * g.C[row * g.ldc + col];
+          if (g.D) v += g.D[(long)(row >> g.dshift) * g.ldd + col];
+          g.C[row * g.ldc + col] = v;
+        }
+      }
+    }
+}
+
+}  // namespace cavs

@@ -1,13 +1,7 @@
-// FP32 GEMM on the CDNA4 matrix cores (v_mfma_f32_32x32x2_f32), row-major, for the
-// gate products of the vertex functions: NN (X*W), NT (dY*W^T) and TN (X^T*dY).
-//
-// Workgroup = 4 wavefronts (2x2) over a BM x BN tile of C, BK deep (128x128x16 for
-// problems that fill the chip, 64x64x32 otherwise).  A and B
-// tiles are staged through LDS as [k][m] / [k][n] panels (double buffered, one
-// barrier per k-tile), so each MFMA operand read is a conflict-free ds_read_b32 of
-// 32 consecutive floats per half-wave.  Global loads are 16-byte per lane; the
-// k-contiguous operand (A of NN/NT, B of NT) is transposed on its way into LDS.
-// Workgroup ids are remapped so that consecutive tiles (which share an A row panel)
+// fp32 products for the gate products of the vertex functions, row-major: NN (X*W), NT (dY*W^T) and
+// TN (X^T*dY), on the bf16 matrix pipe at full fp32 precision (gemm_split.h): tiles of 128 x 128 for
+// problems that fill the chip, 64 x 64 otherwise.
+// Workgroup ids are remapped so that consecutive tiles (which share operand panels)
 // run on the same XCD and hit the same L2.  Products with too few tiles to fill the
 // chip take one of two other routes: skinny ones (the tail rounds of a batch) a
 // kernel whose wavefronts split K inside the workgroup, tall-K ones (the deferred
@@ -21,383 +15,10 @@
 #include "bench_probes.h"
 #include "common.h"
 #include "embed_common.h"
+#include "gemm_common.h"
+#include "gemm_split.h"
 
 namespace cavs {
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-
-constexpr int PAD = 4;
-constexpr int kThreads = 256;
-
-struct GemmArgs {
-  int M, N, K;
-  const float *A;
-  long lda;
-  const float *B;
-  long ldb;
-  float *C;
-  long ldc;
-  float alpha, beta;
-  const float *D;  // optional addend rows D[r >> dshift, :]
-  long ldd;
-  int dshift;
-  int kchunk;      // K range per blockIdx.y (multiple of BK); == K when not split
-  float *ws;       // split-K workspace (counters + partial tiles) or nullptr
-  // cavs_embed_pull_sgemm (NN form only): row r of A is row int(pull_x[pull_rows[r]] * K) / K of the
-  // table A points at (a negative id: a zero row); the workgroups of a row tile also leave the
-  // rows they read in pull_copy (row stride ld_copy; each takes every tilesN-th k-tile) and those
-  // of the first column tile the ids in pull_ids
-  const int *pull_rows = nullptr;
-  const float *pull_x = nullptr;
-  float *pull_copy = nullptr;
-  long ld_copy = 0;
-  float *pull_ids = nullptr;
-  // A block the caller knows about (cavs_gemm_desc::zero_kind and friends): the tiles it covers
-  // run a shorter k range, or none
-  int zkind = 0, zrows = 0, zcol = 0;
-  // > 0: the launch is two launches back to back, the first zseg tiles (the row tiles inside the
-  // block, whose workgroups do less) and the rest, each padded to a multiple of 8 workgroups and
-  // dealt to the XCDs by itself: with one deal over all tiles the XCDs that hold the first
-  // tiles would finish early and the others set the time as before
-  int zseg = 0;
-};
-
-// Loader of one BX x BK operand tile.  KC: the operand's k index is the contiguous
-// one in memory (element (x,k) at P[x*ld + k]); otherwise element at P[k*ld + x].
-template <int BX, int BK, bool KC, bool VEC, bool FASTK = false>
-struct TileLoader {
-  static constexpr int NV = BX * BK / 4 / kThreads;  // float4 per thread
-  static constexpr int KQ = BK / 4;                  // float4 per row of a k-contiguous tile
-  static constexpr int PER = BX / 4;                 // float4 per k row otherwise
-  float4 reg[NV];
-  // Fixed per thread before the k loop (prepare): where float4 i of this thread sits in the
-  // operand at k = 0, which of its x are inside, and its k relative to the tile's first.  In
-  // the loop only the tile's k advances -- a pointer bump, or a wave-uniform k * ld -- instead
-  // of a 64-bit row * stride product on the vector ALU per load and k-tile.
-  long base[NV];
-  int krel[NV];
-  bool xin[NV][4];
-  // Fast path (VEC): when every x of the tile is inside the operand and the offsets fit 32 bits,
-  // a k-tile that lies wholly inside the k range is fetched with unconditional loads at a
-  // wave-uniform pointer plus this byte offset -- no predicate, no 64-bit address arithmetic on
-  // the vector ALU (8192^3: 126.6 -> 133.9 TFLOP/s).  The k loop runs in two parts, the k-tiles
-  // that take it and the rest, so that neither carries the other's code.
-  unsigned boff[NV];
-  bool fast = false;
-  // gathered rows (prepare_pull): where the float4 goes as well, or nullptr; the workgroup copies
-  // the k-tiles whose number is copy_rem modulo copy_mod (the column tiles of a row tile share the
-  // copying of the panel they all read)
-  float *copy[NV];
-  int copy_mod = 1, copy_rem = 0;
-
-  __device__ inline void prepare(long ld, int x0, int X, int tid) {
-#pragma unroll
-    for (int i = 0; i < NV; i++) {
-      copy[i] = nullptr;
-      if constexpr (KC) {
-        const int gx = x0 + tid / KQ + (kThreads / KQ) * i;
-        krel[i] = 4 * (tid % KQ);
-        base[i] = (long)gx * ld + krel[i];
-#pragma unroll
-        for (int c = 0; c < 4; c++) xin[i][c] = gx < X;
-      } else {
-        const int gx = x0 + 4 * (tid % PER);
-        krel[i] = tid / PER + (kThreads / PER) * i;
-        base[i] = (long)krel[i] * ld + gx;
-#pragma unroll
-        for (int c = 0; c < 4; c++) xin[i][c] = gx + c < X;
-      }
-      if constexpr (FASTK) boff[i] = (unsigned)(base[i] * 4);
-    }
-    if constexpr (FASTK) fast = VEC && x0 + BX <= X && (KC ? (long)X * ld : (long)BK * ld) < (1L << 30);
-  }
-
-  // k-contiguous operand whose rows are looked up: row x0 + r of the operand is the table row that
-  // starts at float int(ids(x0 + r) * K) of P (EmbeddingLookup's offset), ids(b) = px[rows[b]]
-  __device__ inline void prepare_pull(const int *__restrict__ rows, const float *__restrict__ px, int K, int x0, int X, int tid,
-                                      float *__restrict__ copy_to, long ld_copy, float *__restrict__ ids_out, int mod, int rem) {
-    static_assert(KC, "looked-up rows are k-contiguous");
-    copy_mod = mod;
-    copy_rem = rem;
-    fast = false;
-#pragma unroll
-    for (int i = 0; i < NV; i++) {
-      const int gx = x0 + tid / KQ + (kThreads / KQ) * i;
-      krel[i] = 4 * (tid % KQ);
-      long off = -1;
-      if (gx < X) {
-        const float id = px[rows[gx]];
-        off = (long)(int)(id * (float)K);
-        if (ids_out && krel[i] == 0) ids_out[gx] = id;
-      }
-      base[i] = (off >= 0 ? off : 0) + krel[i];
-#pragma unroll
-      for (int c = 0; c < 4; c++) xin[i][c] = off >= 0;
-      copy[i] = (copy_to && gx < X) ? copy_to + (long)gx * ld_copy + krel[i] : nullptr;
-    }
-  }
-
-  // the tile whose first k is k0, wholly inside the k range, of an operand with `fast` set
-  __device__ inline void load_fast(const float *__restrict__ P, long ld, int k0) {
-    const char *Pk = reinterpret_cast<const char *>(KC ? P + k0 : P + (long)k0 * ld);
-#pragma unroll
-    for (int i = 0; i < NV; i++) reg[i] = *reinterpret_cast<const float4 *>(Pk + boff[i]);
-  }
-
-  // the tile whose first k is k0 (wave-uniform)
-  __device__ inline void load(const float *__restrict__ P, long ld, int k0, int Kend) {
-    const float *Pk = KC ? P + k0 : P + (long)k0 * ld;
-#pragma unroll
-    for (int i = 0; i < NV; i++) {
-      bool kin[4];
-#pragma unroll
-      for (int c = 0; c < 4; c++) kin[c] = KC ? (k0 + krel[i] + c < Kend) : (k0 + krel[i] < Kend);
-      const float *q = Pk + base[i];
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      if constexpr (VEC) {
-        // whole float4 in or out (X, K multiples of 4 along the contiguous index)
-        if (xin[i][0] && kin[0]) v = *reinterpret_cast<const float4 *>(q);
-      } else {
-        if (xin[i][0] && kin[0]) v.x = q[0];
-        if (xin[i][1] && kin[1]) v.y = q[1];
-        if (xin[i][2] && kin[2]) v.z = q[2];
-        if (xin[i][3] && kin[3]) v.w = q[3];
-      }
-      reg[i] = v;
-      if constexpr (KC) {
-        if (copy[i] && (k0 / BK) % copy_mod == copy_rem) {  // (a row without an id leaves zeros)
-          if constexpr (VEC) {
-            if (kin[0]) *reinterpret_cast<float4 *>(copy[i] + k0) = v;
-          } else {
-            if (kin[0]) copy[i][k0] = v.x;
-            if (kin[1]) copy[i][k0 + 1] = v.y;
-            if (kin[2]) copy[i][k0 + 2] = v.z;
-            if (kin[3]) copy[i][k0 + 3] = v.w;
-          }
-        }
-      }
-    }
-  }
-
-  __device__ inline void store(float *__restrict__ S, int tid) const {
-    constexpr int LD = BX + PAD;
-#pragma unroll
-    for (int i = 0; i < NV; i++) {
-      if constexpr (KC) {
-        int x = tid / KQ + (kThreads / KQ) * i, k = 4 * (tid % KQ);
-        S[(k + 0) * LD + x] = reg[i].x;
-        S[(k + 1) * LD + x] = reg[i].y;
-        S[(k + 2) * LD + x] = reg[i].z;
-        S[(k + 3) * LD + x] = reg[i].w;
-      } else {
-        int k = tid / PER + (kThreads / PER) * i, x = 4 * (tid % PER);
-        *reinterpret_cast<float4 *>(S + k * LD + x) = reg[i];
-      }
-    }
-  }
-};
-
-// Remap the linear workgroup id so that ids that are consecutive after the remap
-// were dispatched to the same XCD (hardware deals workgroups round-robin over 8 XCDs).
-__device__ inline int xcd_remap(int l, int total) {
-  constexpr int X = 8;
-  int per = total / X, rem = total % X;
-  int xcd = l % X, local = l / X;
-  return xcd * per + (xcd < rem ? xcd : rem) + local;
-}
-
-// One BM x BN tile of C (or of split `z` of its K range) by the calling workgroup.  `t` is the
-// tile's index, row-major over the tiles of C; As / Bs are the workgroup's two LDS panels of
-// 2 * BK * (BM + PAD) and 2 * BK * (BN + PAD) floats.
-// FASTK: the k loop has a first part for k-tiles that take the loaders' fast path.
-template <int BM, int BN, int BK, bool TA, bool TB, bool VEC, bool FASTK = true>
-__device__ __forceinline__ void gemm_tile(const GemmArgs &g, int t, int z, float *__restrict__ As_, float *__restrict__ Bs_) {
-  constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
-  constexpr int LDA = BM + PAD, LDB = BN + PAD;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int tilesN = (g.N + BN - 1) / BN;
-  const int m0 = (t / tilesN) * BM, n0 = (t % tilesN) * BN;
-  int kbeg = z * g.kchunk;
-  int kend = min(g.K, kbeg + g.kchunk);
-  if (g.zkind == CAVS_GEMM_C_UNUSED) {  // rows below zrows of C are not wanted from column zcol on: left zero
-    if (m0 + BM <= g.zrows && n0 >= g.zcol) kend = kbeg;
-  } else if (g.zkind == CAVS_GEMM_A_ZERO) {  // rows below zrows of A (row-major M x K) are zero from k = zcol on
-    if (!TA && m0 + BM <= g.zrows) kend = max(kbeg, min(kend, g.zcol));
-  } else if (g.zkind == CAVS_GEMM_B_ZERO) {  // rows k < zrows of B (row-major K x N) are zero from column zcol on
-    if (!TB && n0 >= g.zcol) kbeg = min(kend, max(kbeg, g.zrows / 32 * 32));
-  }
-
-  TileLoader<BM, BK, !TA, VEC, FASTK> la;
-  TileLoader<BN, BK, TB, VEC, FASTK> lb;
-  if constexpr (!TA) {
-    if (g.pull_rows) {
-      // the column tiles of this row tile that do run share the copying
-      const int active = (g.zkind == CAVS_GEMM_C_UNUSED && m0 + BM <= g.zrows) ? min(tilesN, (g.zcol + BN - 1) / BN) : tilesN;
-      la.prepare_pull(g.pull_rows, g.pull_x, g.K, m0, g.M, tid, g.pull_copy, g.ld_copy, n0 == 0 ? g.pull_ids : nullptr, active,
-                      t % tilesN);
-    }
-    else la.prepare(g.lda, m0, g.M, tid);
-  } else {
-    la.prepare(g.lda, m0, g.M, tid);
-  }
-  lb.prepare(g.ldb, n0, g.N, tid);
-
-  floatx16 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; i++)
-#pragma unroll
-    for (int j = 0; j < TN; j++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
-
-  const int nk = (kend - kbeg + BK - 1) / BK;
-  // k-tiles 0 .. nfast - 1 lie wholly inside the k range of operands that take the fast loads
-  const int nfast = (FASTK && la.fast && lb.fast) ? (kend - kbeg) / BK : 0;
-  if (nk > 0) {
-    if (FASTK && nfast > 0) {
-      la.load_fast(g.A, g.lda, kbeg);
-      lb.load_fast(g.B, g.ldb, kbeg);
-    } else {
-      la.load(g.A, g.lda, kbeg, kend);
-      lb.load(g.B, g.ldb, kbeg, kend);
-    }
-    la.store(As_, tid);
-    lb.store(Bs_, tid);
-  }
-  __syncthreads();
-  const int arow = wm * WM + (lane & 31), brow = wn * WN + (lane & 31), khalf = lane >> 5;
-  // The MFMAs of the k-tile in LDS buffer `cur` (spelled out in each loop through a macro: as a
-  // lambda the compiler scheduled the 64 x 64 kernels 2 % slower).  Operand fragments: the reads of
-  // AHEAD steps are in flight while a step's MFMAs issue, so a wavefront does not stall on LDS
-  // latency between them; the scheduler barriers keep that order (the compiler's scheduler would
-  // sink each read to its use).
-  constexpr int STEPS = BK / 2, AHEAD = (TM * TN == 1) ? 4 : 2;
-#define CAVS_TILE_PRODUCTS(cur)                                                                            \
-  do {                                                                                                     \
-    const float *as = As_ + (cur) * (BK * LDA), *bs = Bs_ + (cur) * (BK * LDB);                            \
-    float a[STEPS][TM], b[STEPS][TN];                                                                      \
-    auto read = [&](int st) {                                                                              \
-      _Pragma("unroll") for (int i = 0; i < TM; i++) a[st][i] = as[(2 * st + khalf) * LDA + arow + 32 * i]; \
-      _Pragma("unroll") for (int j = 0; j < TN; j++) b[st][j] = bs[(2 * st + khalf) * LDB + brow + 32 * j]; \
-    };                                                                                                     \
-    _Pragma("unroll") for (int st = 0; st < AHEAD && st < STEPS; st++) read(st);                           \
-    __builtin_amdgcn_sched_barrier(0);                                                                     \
-    _Pragma("unroll") for (int st = 0; st < STEPS; st++) {                                                 \
-      if (st + AHEAD < STEPS) read(st + AHEAD);                                                            \
-      __builtin_amdgcn_sched_barrier(0);                                                                   \
-      _Pragma("unroll") for (int i = 0; i < TM; i++)                                                       \
-        _Pragma("unroll") for (int j = 0; j < TN; j++)                                                     \
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[st][i], b[st][j], acc[i][j], 0, 0, 0);        \
-      __builtin_amdgcn_sched_barrier(0);                                                                   \
-    }                                                                                                      \
-  } while (0)
-  // iteration kt fetches tile kt + 1 while it multiplies tile kt
-  if constexpr (FASTK) {
-    // first the iterations whose next tile takes the fast loads, then the rest
-    const int split = nfast > 1 ? nfast - 1 : 0;
-    for (int kt = 0; kt < split; kt++) {
-      const int cur = kt & 1;
-      la.load_fast(g.A, g.lda, kbeg + (kt + 1) * BK);
-      lb.load_fast(g.B, g.ldb, kbeg + (kt + 1) * BK);
-      CAVS_TILE_PRODUCTS(cur);
-      la.store(As_ + (cur ^ 1) * (BK * LDA), tid);
-      lb.store(Bs_ + (cur ^ 1) * (BK * LDB), tid);
-      __syncthreads();
-    }
-    for (int kt = split; kt < nk; kt++) {
-      const int cur = kt & 1;
-      if (kt + 1 < nk) {
-        la.load(g.A, g.lda, kbeg + (kt + 1) * BK, kend);
-        lb.load(g.B, g.ldb, kbeg + (kt + 1) * BK, kend);
-      }
-      CAVS_TILE_PRODUCTS(cur);
-      if (kt + 1 < nk) {
-        la.store(As_ + (cur ^ 1) * (BK * LDA), tid);
-        lb.store(Bs_ + (cur ^ 1) * (BK * LDB), tid);
-      }
-      __syncthreads();
-    }
-  } else {
-    for (int kt = 0; kt < nk; kt++) {
-      const int cur = kt & 1;
-      if (kt + 1 < nk) {
-        la.load(g.A, g.lda, kbeg + (kt + 1) * BK, kend);
-        lb.load(g.B, g.ldb, kbeg + (kt + 1) * BK, kend);
-      }
-      CAVS_TILE_PRODUCTS(cur);
-      if (kt + 1 < nk) {
-        la.store(As_ + (cur ^ 1) * (BK * LDA), tid);
-        lb.store(Bs_ + (cur ^ 1) * (BK * LDB), tid);
-      }
-      __syncthreads();
-    }
-  }
-
-#undef CAVS_TILE_PRODUCTS
-  // C layout of the 32x32 accumulator: element r of lane l is row 8*(r/4) + 4*(l/32) + r%4,
-  // column l%32.
-#pragma unroll
-  for (int i = 0; i < TM; i++)
-#pragma unroll
-    for (int j = 0; j < TN; j++) {
-      const int col = n0 + wn * WN + 32 * j + (lane & 31);
-      if (col >= g.N) continue;
-      const int rbase = m0 + wm * WM + 32 * i + 4 * khalf;
-      // the three forms of the store are chosen once per tile (the conditions are the same
-      // for every lane), not once per element
-      if (g.ws) {  // split K: park the partial sum, the reduce kernel finishes the job
-        float *w = g.ws + (long)z * g.M * g.N + col;
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int row = rbase + 8 * (r / 4) + (r % 4);
-          if (row < g.M) w[(long)row * g.N] = acc[i][j][r];
-        }
-      } else if (g.beta == 0.f && !g.D) {
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int row = rbase + 8 * (r / 4) + (r % 4);
-          if (row < g.M) g.C[row * g.ldc + col] = g.alpha * acc[i][j][r];
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int row = rbase + 8 * (r / 4) + (r % 4);
-          if (row >= g.M) continue;
-          float v = g.alpha * acc[i][j][r];
-          if (g.beta != 0.f) v += g.beta * g.C[row * g.ldc + col];
-          if (g.D) v += g.D[(long)(row >> g.dshift) * g.ldd + col];
-          g.C[row * g.ldc + col] = v;
-        }
-      }
-    }
-}
-
-template <int BM, int BN, int BK, bool TA, bool TB, bool VEC>
-__global__ __launch_bounds__(kThreads) void sgemm_mfma_kernel(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) float As[2 * BK * (BM + PAD)];
-  __shared__ __attribute__((aligned(16))) float Bs[2 * BK * (BN + PAD)];
-  const int tiles = ((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
-  int t;
-  if (g.zseg > 0) {
-    const int first = (g.zseg + 7) & ~7, b = blockIdx.x;
-    if (b < first) {
-      t = xcd_remap(b, first);
-      if (t >= g.zseg) return;
-    } else {
-      const int rest = tiles - g.zseg;
-      t = xcd_remap(b - first, (rest + 7) & ~7);
-      if (t >= rest) return;
-      t += g.zseg;
-    }
-  } else {
-    t = xcd_remap(blockIdx.x, tiles);
-  }
-  // (the fast part of the k loop pays on the large tile; the 64 x 64 launches are products with
-  // short K or ragged edges, which it only made larger)
-  gemm_tile<BM, BN, BK, TA, TB, VEC, BM == 128>(g, t, blockIdx.y, As, Bs);
-}
 
 // Several independent products in one launch (the deferred weight gradients of a step and the
 // embedding gradient's product): alone, each of them is a single round of workgroups that all
@@ -416,10 +37,9 @@ struct GemmGroup {
 };
 
 template <bool VEC>
-__global__ __launch_bounds__(kThreads) void sgemm_group_kernel(GemmGroup G) {
-  constexpr int BM = 64, BN = 64, BK = 32;
-  __shared__ __attribute__((aligned(16))) float As[2 * BK * (BM + PAD)];
-  __shared__ __attribute__((aligned(16))) float Bs[2 * BK * (BN + PAD)];
+__global__ __launch_bounds__(kThreads, 4) void sgemm_group_kernel(GemmGroup G) {
+  constexpr int BM = 64, BN = 64, BK = 16;
+  __shared__ __attribute__((aligned(16))) char S[split_lds_bytes(BM, BN, BK)];
   int p = 0;
   while (p + 1 < G.count && (int)blockIdx.x >= G.first[p + 1]) p++;
   const int local = blockIdx.x - G.first[p];
@@ -429,11 +49,12 @@ __global__ __launch_bounds__(kThreads) void sgemm_group_kernel(GemmGroup G) {
   if (w >= share) return;
   const int t = w % G.tiles[p], z = w / G.tiles[p];
   const GemmArgs &g = G.g[p];
+  const int tilesN = (g.N + BN - 1) / BN, m0 = t / tilesN * BM, n0 = t % tilesN * BN;
   switch (G.form[p]) {
-    case 0: gemm_tile<BM, BN, BK, false, false, VEC, true>(g, t, z, As, Bs); break;
-    case 1: gemm_tile<BM, BN, BK, false, true, VEC, true>(g, t, z, As, Bs); break;
-    case 2: gemm_tile<BM, BN, BK, true, false, VEC, true>(g, t, z, As, Bs); break;
-    default: gemm_tile<BM, BN, BK, true, true, VEC, true>(g, t, z, As, Bs); break;
+    case 0: split_tile<BM, BN, BK, false, false, VEC>(g, m0, n0, z, S); break;
+    case 1: split_tile<BM, BN, BK, false, true, VEC>(g, m0, n0, z, S); break;
+    case 2: split_tile<BM, BN, BK, true, false, VEC>(g, m0, n0, z, S); break;
+    default: split_tile<BM, BN, BK, true, true, VEC>(g, m0, n0, z, S); break;
   }
 }
 
@@ -668,70 +289,58 @@ static bool skinny_ok(int tA, int tB, int K, const float *A, int lda, const floa
   return true;
 }
 
-static GemmPlan plan_gemm(int tA, int tB, int M, int N, int K, bool skinny_allowed, bool allow_split) {
+// Rows of a k-contiguous operand further apart than the large tile's 32-bit offsets reach.
+static bool far_rows(int tA, int tB, int lda, int ldb) { return (!tA && lda >= 1 << 23) || (tB && ldb >= 1 << 23); }
+
+static GemmPlan plan_gemm(int tA, int tB, int M, int N, int K, bool skinny_allowed, bool allow_split, bool large_ok = true) {
   GemmPlan p;
   const long cus = num_cus();
   const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
   const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
-  p.splits = 1;
-  p.kchunk = K > 0 ? K : 1;
-  // the large tile needs at least two rounds of workgroups to hide its ragged last round
-  if (t128 >= 2 * cus) {
-    p.kind = GemmPlan::TILE128;
-    p.tiles = t128;
+  auto split = [&](GemmPlan::Kind kind, long tiles, long s) {
+    p.kind = kind;
+    p.tiles = tiles;
+    p.kchunk = K;
+    p.splits = 1;
+    if (s > 1) {
+      p.kchunk = (int)(((K + s - 1) / s + 31) / 32 * 32);
+      p.splits = (K + p.kchunk - 1) / p.kchunk;
+    }
     return p;
-  }
-  // Tall-K products whose large tiles give each CU one workgroup or less (the deferred weight
-  // gradients of big batches: 8x32 tiles, K = all rows): one workgroup per CU cannot hide the
-  // latency of its own global loads, so K is split until about three share a CU.
-  if (allow_split && 4 * t128 >= cus && K >= 4096) {
+  };
+  // A CU holds three workgroups of the large tile; from two per CU on it is the faster one (4700 x 2048 x
+  // 300, 592 tiles: 44.6 us against 49.8; 2368 rows, 304 tiles: 31.1 against 27.3).
+  if (large_ok && t128 >= 2 * cus) return split(GemmPlan::TILE128, t128, 1);
+  // Fewer large tiles: K is split until about three share a CU, if that leaves each split at least 512 of K
+  // (4000 x 1024 x 3072: 150 us against 170 on the small tile).
+  if (large_ok && allow_split && 4 * t128 >= cus && K >= 2048) {
     long s = (3 * cus + t128 - 1) / t128;
-    // one or two more splits when they even out the workgroups per CU (316 tiles: three splits are
-    // 3.7 per CU, a fourth round at 70 %; four splits are 4.94: 90.8 -> 95.5 TFLOP/s at 512 x 10000
-    // x 7331); ties keep the fewer splits (less partial traffic)
+    // one or two more splits when they even out the workgroups per CU; ties keep the fewer splits
+    // (less partial traffic)
     auto fill = [&](long sp) {
       const long w = t128 * sp, rounds = (w + cus - 1) / cus;
       return (double)w / (double)(rounds * cus);
     };
     for (long c = s + 1; c <= s + 2; c++)
       if (fill(c) > fill(s) + 0.02) s = c;
-    if (s > K / 1024) s = K / 1024;
-    if (s > 1) {
-      int kchunk = (int)(((K + s - 1) / s + 31) / 32 * 32);
-      int splits = (K + kchunk - 1) / kchunk;
-      if (splits > 1) {
-        p.kind = GemmPlan::TILE128;
-        p.tiles = t128;
-        p.splits = splits;
-        p.kchunk = kchunk;
-        return p;
-      }
-    }
+    s = std::min<long>(s, K / 512);
+    if (t128 * s >= 2 * cus) return split(GemmPlan::TILE128, t128, s);
   }
-  p.kind = GemmPlan::TILE64;
-  p.tiles = t64;
-  if (t64 >= 2 * cus || K < 64) return p;
+  if (t64 >= 2 * cus || K < 64) return split(GemmPlan::TILE64, t64, 1);
   // the skinny kernel reads a k-contiguous B (NT) sixteen bytes per lane and row, which only
   // pays for a handful of rows; with B row-major (NN) it holds up to about a thousand
   if (skinny_allowed && M <= (tB ? 128 : 1024)) {
     p.kind = GemmPlan::SKINNY;
+    p.splits = 1;
+    p.kchunk = K;
+    p.tiles = t64;
     return p;
   }
+  long s = 1;
   if (allow_split && K >= 256) {
-    long want = (3 * cus + t64 - 1) / t64;
-    long maxs = K / 128;  // at least four k-tiles per split
-    long s = want < maxs ? want : maxs;
-    if (s > 32) s = 32;
-    if (s > 1) {
-      int kchunk = (int)(((K + s - 1) / s + 31) / 32 * 32);
-      int splits = (K + kchunk - 1) / kchunk;
-      if (splits > 1) {
-        p.splits = splits;
-        p.kchunk = kchunk;
-      }
-    }
+    s = std::min({(3 * cus + t64 - 1) / t64, (long)(K / 128), 32L});  // at least 128 of K per split
   }
-  return p;
+  return split(GemmPlan::TILE64, t64, s);
 }
 
 static size_t plan_workspace(const GemmPlan &p, int M, int N) {
@@ -750,22 +359,28 @@ static bool vec_path_ok(const GemmArgs &g, int tA, int tB) {
 // workgroups then take more of a CU than they use, and fewer of them share one
 static thread_local unsigned t_lds_pad = 0;
 
-template <int BM, int BN, int BK>
-static void launch_tile(const GemmArgs &args, int tA, int tB, bool vec, const GemmPlan &p, hipStream_t st) {
-  GemmArgs g = args;
-  dim3 grid((unsigned)p.tiles, p.splits), block(kThreads);
-  if (g.zkind == CAVS_GEMM_A_ZERO || g.zkind == CAVS_GEMM_C_UNUSED) {
-    const long inside = (long)(std::min(g.zrows, g.M) / BM) * ((g.N + BN - 1) / BN);
+// The grid of a launch of BM x BN tiles: a known block of whole row tiles becomes a launch of its own (GemmArgs::zseg).
+static dim3 tile_grid(GemmArgs *g, int BM, int BN, const GemmPlan &p) {
+  dim3 grid((unsigned)p.tiles, p.splits);
+  if (g->zkind == CAVS_GEMM_A_ZERO || g->zkind == CAVS_GEMM_C_UNUSED) {
+    const long inside = (long)(std::min(g->zrows, g->M) / BM) * ((g->N + BN - 1) / BN);
     if (inside > 0 && inside < p.tiles) {
-      g.zseg = (int)inside;
+      g->zseg = (int)inside;
       grid.x = (unsigned)((inside + 7) / 8 * 8 + (p.tiles - inside + 7) / 8 * 8);
     }
   }
-#define CAVS_GEMM_CASE(TA, TB)                                                  \
-  if (vec)                                                                      \
-    launch(sgemm_mfma_kernel<BM, BN, BK, TA, TB, true>, grid, block, t_lds_pad, st, g);      \
-  else                                                                          \
-    launch(sgemm_mfma_kernel<BM, BN, BK, TA, TB, false>, grid, block, t_lds_pad, st, g)
+  return grid;
+}
+
+template <int BM, int BN, int BK>
+static void launch_split(const GemmArgs &args, int tA, int tB, bool vec, const GemmPlan &p, hipStream_t st) {
+  GemmArgs g = args;
+  const dim3 grid = tile_grid(&g, BM, BN, p), block(kThreads);
+#define CAVS_GEMM_CASE(TA, TB)                                                                                \
+  if (vec)                                                                                                    \
+    launch(sgemm_split_kernel<BM, BN, BK, TA, TB, true>, grid, block, t_lds_pad, st, g);                      \
+  else                                                                                                        \
+    launch(sgemm_split_kernel<BM, BN, BK, TA, TB, false>, grid, block, t_lds_pad, st, g)
   if (!tA && !tB) { CAVS_GEMM_CASE(false, false); }
   else if (!tA && tB) { CAVS_GEMM_CASE(false, true); }
   else if (tA && !tB) { CAVS_GEMM_CASE(true, false); }
@@ -831,7 +446,8 @@ static int run_gemm(const char *who, int tA, int tB, int M, int N, int K, float 
   if (rc || M == 0 || N == 0) return rc;
   // Looked-up rows: up to 128 of them the skinny kernel, beyond it the 64 x 64 tiles (M x 2048 x 300..512: 21
   // rows 12.4 -> 7.9 us, 120 rows 19.7 -> 15.1, 300 rows 20.5 and 26.2).
-  GemmPlan p = plan_gemm(tA, tB, M, N, K, (!pull || M <= 128) && skinny_ok(tA, tB, K, A, lda, B, ldb), ws != nullptr);
+  GemmPlan p = plan_gemm(tA, tB, M, N, K, (!pull || M <= 128) && skinny_ok(tA, tB, K, A, lda, B, ldb), ws != nullptr,
+                         !pull && !far_rows(tA, tB, lda, ldb));
   hipStream_t st = as_stream(stream);
   GemmArgs g{M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, D, ldd, dshift, p.kchunk, nullptr};
   if (hint) hint->set(&g, tA, tB, beta == 0.f && !D);
@@ -853,18 +469,15 @@ static int run_gemm(const char *who, int tA, int tB, int M, int N, int K, float 
     g.ws = static_cast<float *>(ws);
   }
   bool vec = vec_path_ok(g, tA, tB);
-  // The chip holds four 64x64 workgroups per CU with K panels of 32 (their LDS) and eight with
-  // panels of 16.  A launch of a few more than four per CU runs them as a second round behind
-  // the first (2048 x 2048 x 300: 29.0 us; 2112 rows: 36.7), so launches between one and two
-  // rounds take the narrow panels and stay resident at once (2482 rows: 40.2 -> 33.1 us);
-  // everywhere else the wide panels are faster.
-  const long wgs = p.tiles * p.splits, slots = 4L * num_cus();
-  if (p.kind == GemmPlan::TILE128)
-    launch_tile<128, 128, 16>(g, tA, tB, vec, p, st);
-  else if (wgs > slots && wgs <= 2 * slots)
-    launch_tile<64, 64, 16>(g, tA, tB, vec, p, st);
-  else
-    launch_tile<64, 64, 32>(g, tA, tB, vec, p, st);
+  if (pull) {
+    const dim3 grid = tile_grid(&g, 64, 64, p), block(kThreads);
+    if (vec) launch(sgemm_split_kernel<64, 64, 16, false, false, true, true>, grid, block, 0, st, g);
+    else launch(sgemm_split_kernel<64, 64, 16, false, false, false, true>, grid, block, 0, st, g);
+  } else if (p.kind == GemmPlan::TILE128) {
+    launch_split<128, 128, 16>(g, tA, tB, vec, p, st);
+  } else {
+    launch_split<64, 64, 16>(g, tA, tB, vec, p, st);
+  }
   CAVS_LAUNCH_CHECK();
   if (p.splits > 1) {
     long total = (long)M * N;
@@ -908,7 +521,7 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
                  "cavs_sgemm_group: bad block hint in product %d (kind %d, rows %d, col %d)", p, q.zero_kind, q.zero_rows, q.zero_col);
     tiles[p] = (long)((q.M + 63) / 64) * ((q.N + 63) / 64);
     // a product that fills the chip with large tiles by itself is better off on them, alone
-    alone[p] = q.M > 0 && q.N > 0 && plan_gemm(q.transA, q.transB, q.M, q.N, q.K, false, true).kind == GemmPlan::TILE128;
+    alone[p] = q.M > 0 && q.N > 0 && plan_gemm(q.transA, q.transB, q.M, q.N, q.K, false, true, !far_rows(q.transA, q.transB, q.lda, q.ldb)).kind == GemmPlan::TILE128;
     if (!alone[p] && q.M > 0 && q.N > 0) grouped++;
   }
   for (int p = 0; p < count; p++) {
@@ -919,7 +532,7 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
       continue;
     }
     alone[p] = true;
-    most = std::max(most, plan_workspace(plan_gemm(q.transA, q.transB, q.M, q.N, q.K, false, true), q.M, q.N));
+    most = std::max(most, plan_workspace(plan_gemm(q.transA, q.transB, q.M, q.N, q.K, false, true, !far_rows(q.transA, q.transB, q.lda, q.ldb)), q.M, q.N));
   }
   const long slots = 4 * num_cus();
   long kc = (long)(work / (double)slots);
@@ -1094,7 +707,7 @@ int cavs_sgemm_group(int count, const cavs_gemm_desc *products, void *workspace,
 
 int cavs_sgemm_group_beside(int count, const cavs_gemm_desc *products, void *workspace, size_t workspace_bytes,
                             void *stream) {
-  t_lds_pad = 22u << 10;  // with the 33 KB of a tile's panels: two workgroups per CU
+  t_lds_pad = 10u << 10;  // with the 48 KB of a large tile's panels: two workgroups per CU
   const int rc = run_group(count, products, workspace, workspace_bytes, nullptr, stream);
   t_lds_pad = 0;
   return rc;
@@ -1147,7 +760,7 @@ int cavs_sgemm_addrows(int transA, int transB, int M, int N, int K, const float 
 size_t cavs_sgemm_splitk_workspace(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   // sized for the split plan whether or not a given call ends up taking the skinny path
-  return plan_workspace(plan_gemm(0, 0, M, N, K, false, true), M, N);
+  return std::max(plan_workspace(plan_gemm(0, 0, M, N, K, false, true), M, N), plan_workspace(plan_gemm(0, 0, M, N, K, false, true, false), M, N));
 }
 
 int cavs_sgemm_splitk(int transA, int transB, int M, int N, int K, float alpha, const float *A,

@@ -1772,3 +1772,23 @@ def test_kernel_stamped_timing_probe(g):
     hip.call("cavs_event_destroy", e1)
     with pytest.raises(hip.CavsError, match="null event"):
         hip.call("cavs_profile_arm", None, None)
+
+
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K,ld", [(70, 68, 17, 1), (2945, 2949, 33, 3), (129, 65, 20000, 4)])
+def test_sgemm_keeps_every_bit_of_its_operands(g, tA, tB, M, N, K, ld):
+    """The three-part products: operands whose low bits carry the result (a large part that cancels), ragged
+    tiles and k tails in every form, rows at odd strides, and a K long enough to be added up in pieces."""
+    r = rng(M + 5 * N + 7 * K + 2 * tA + tB)
+    half = K // 2
+    A, B = r.bulk_uniform(M * K, -1, 1).reshape(M, K), r.bulk_uniform(N * K, -1, 1).reshape(N, K)
+    A[:, half:2 * half] = -A[:, :half] * (1 + r.bulk_uniform(M * half, -1, 1).reshape(M, half) * 2.0 ** -18)
+    B[:, half:2 * half] = B[:, :half]
+    A, B = A.astype(np.float32), B.astype(np.float32)
+    pad = lambda X: np.pad(X, ((0, 0), (0, ld)), constant_values=np.nan)  # noqa: E731
+    Ad, Bd = pad(A.T if tA else A), pad(B if tB else B.T)
+    Cd = g.zeros(M, N, fill=float("nan"))
+    g.call("cavs_sgemm", tA, tB, M, N, K, 1.0, g.P(g.devf(Ad)), Ad.shape[1], g.P(g.devf(Bd)), Bd.shape[1], 0.0, g.P(Cd), N, g.stream())
+    exact = A.astype(np.float64) @ B.astype(np.float64).T
+    # (rounding of sums of K terms of order a third)
+    assert np.abs(g.host(Cd) - exact).max() <= 2.0 ** -24 * 8 * np.sqrt(K)
