@@ -661,7 +661,6 @@ void Engine::upload_index_arena() {
   std::string err = build_index_lists(s, nch_, cfg_.pairing, t2j, pair, child, roots);
   if (!err.empty()) fail(CAVS_EUNSUPPORTED, err);
   forest_ = want_forest && build_forest_lists(s, nch_, fused_rows(), pair, child, roots + s.B, roots + s.B + (size_t)nch_ * N, &n_orphans_);
-  plan_head_chunks(roots + s.B + (size_t)nch_ * N);
   tail_ = TailPlan();
   int *tail_rows = roots + s.B + (size_t)N * (nch_ + 1);
   if (want_tail && forest_) build_tail_plan(roots + s.B, tail_rows);
@@ -669,6 +668,7 @@ void Engine::upload_index_arena() {
   if (group_lim > 0 && forest_)
     build_group_lists(s, nch_, t2j, pair, child, roots + s.B, group_lim, ngroups, cavs_group_rows(), &group_, h.host.get() + group_at);
   d_group_ = h.dev.get() + group_at;
+  plan_head_chunks(roots + s.B + (size_t)nch_ * N);
   check(cavs_memcpy_h2d(h.dev.get(), h.host.get(), (group_.first >= 0 ? group_at + group_.ints : total) * sizeof(int),
                         direct_ ? stream_ : sched_stream_));
   if (!direct_) {
@@ -2495,6 +2495,9 @@ void Engine::plan_head_chunks(const int *orphans_host) {
   if (cfg_.head_chunks < 0 || cfg_.model != CAVS_MODEL_LSTM || !wide_head() || !s.batching || !forest_ || cfg_.graph_replay || R < 8 ||
       N < 256)
     return;
+  // Where the rounds are one launch per direction, a head whose products fill the chip by themselves runs in
+  // one piece: beside them the rounds take three times as long (C4: 3.32 ms per step, in one piece 3.26).
+  if (cfg_.head_chunks == 0 && group_.first >= 0 && (double)N * cfg_.C >= 512.0 * 128 * 128) return;
   const int K = cfg_.head_chunks > 0 ? std::min(cfg_.head_chunks, (int)kHeadChunks) : 2;
   int k = 0;
   for (int c = 0; c < K; c++) {

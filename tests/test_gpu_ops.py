@@ -1790,5 +1790,5 @@ def test_sgemm_keeps_every_bit_of_its_operands(g, tA, tB, M, N, K, ld):
     Cd = g.zeros(M, N, fill=float("nan"))
     g.call("cavs_sgemm", tA, tB, M, N, K, 1.0, g.P(g.devf(Ad)), Ad.shape[1], g.P(g.devf(Bd)), Bd.shape[1], 0.0, g.P(Cd), N, g.stream())
     exact = A.astype(np.float64) @ B.astype(np.float64).T
-    # (rounding of sums of K terms of order a third)
-    assert np.abs(g.host(Cd) - exact).max() <= 2.0 ** -24 * 8 * np.sqrt(K)
+    # (up to K roundings of partial sums of up to sqrt(K) terms of order a third)
+    assert np.abs(g.host(Cd) - exact).max() <= 2.0 ** -24 * (K + 16)
