@@ -40,7 +40,21 @@ struct GemmArgs {
   // dealt to the XCDs by itself: with one deal over all tiles the XCDs that hold the first
   // tiles would finish early and the others set the time as before
   int zseg = 0;
+  const int *live = nullptr;  // cavs_gemm_desc::live
 };
+
+// The sizes a launch with `live` runs at: rows of C (TA = false) or K (TA = true), the known block's rows.
+__device__ inline void apply_live(GemmArgs &g, bool TA, int splits) {
+  if (!g.live) return;
+  const int n = g.live[0];
+  if (g.zkind) g.zrows = g.live[1];
+  if (TA) {
+    g.K = min(g.K, n);
+    g.kchunk = max(32, ((g.K + splits - 1) / splits + 31) / 32 * 32);
+  } else {
+    g.M = min(g.M, n);
+  }
+}
 
 // Remap the linear workgroup id so that ids that are consecutive after the remap
 // were dispatched to the same XCD (hardware deals workgroups round-robin over 8 XCDs).

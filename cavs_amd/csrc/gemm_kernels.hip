@@ -43,12 +43,14 @@ __global__ __launch_bounds__(kThreads, 4) void sgemm_group_kernel(GemmGroup G) {
   int p = 0;
   while (p + 1 < G.count && (int)blockIdx.x >= G.first[p + 1]) p++;
   const int local = blockIdx.x - G.first[p];
-  const int share = G.tiles[p] * G.splits[p];
-  const int padded = G.first[p + 1] - G.first[p];
+  GemmArgs g = G.g[p];
+  apply_live(g, G.form[p] >= 2, G.splits[p]);
+  const int tiles = g.live ? (g.M + BM - 1) / BM * ((g.N + BN - 1) / BN) : G.tiles[p];
+  const int share = tiles * G.splits[p], padded = (share + 7) & ~7;
+  if (local >= padded) return;
   const int w = xcd_remap(local, padded);
   if (w >= share) return;
-  const int t = w % G.tiles[p], z = w / G.tiles[p];
-  const GemmArgs &g = G.g[p];
+  const int t = w % tiles, z = w / tiles;
   const int tilesN = (g.N + BN - 1) / BN, m0 = t / tilesN * BM, n0 = t % tilesN * BN;
   switch (G.form[p]) {
     case 0: split_tile<BM, BN, BK, false, false, VEC>(g, m0, n0, z, S); break;
@@ -77,7 +79,8 @@ __global__ void splitk_reduce_group_kernel(GemmGroup R) {
   // first[] counts 256-thread workgroups per product here
   int p = 0;
   while (p + 1 < R.count && (int)blockIdx.x >= R.first[p + 1]) p++;
-  const GemmArgs &g = R.g[p];
+  GemmArgs g = R.g[p];
+  apply_live(g, R.form[p] >= 2, R.splits[p]);
   const int splits = R.splits[p];
   long idx = (long)(blockIdx.x - R.first[p]) * blockDim.x + threadIdx.x;
   long total = (long)g.M * g.N;
@@ -123,18 +126,25 @@ struct EmbedTail {
   float *copy;       // where the summed result goes as well (the product's C) when parts > 1
   long ld_copy;
   int n, E, gx;      // gx row chunks of 64
+  const int *live;   // cavs_gemm_desc::live of the product
 };
 
 __global__ __launch_bounds__(256) void splitk_reduce_group_embed_kernel(GemmGroup R, EmbedTail e) {
   const int nred = R.first[R.count];
   if ((int)blockIdx.x >= nred) {
     const int vb = blockIdx.x - nred;
+    if (e.live) {
+      e.n = min(e.n, e.live[0]);
+      if (e.parts > 1) e.part_stride = (long)e.n * e.ld_dy;
+      if (vb % e.gx * kEmbedRows >= e.n) return;
+    }
     embed_bwd_block(e.dtable, e.ids, e.dy, e.ld_dy, e.parts, e.part_stride, e.copy, e.ld_copy, e.n, e.E, vb % e.gx, vb / e.gx);
     return;
   }
   int p = 0;
   while (p + 1 < R.count && (int)blockIdx.x >= R.first[p + 1]) p++;
-  const GemmArgs &g = R.g[p];
+  GemmArgs g = R.g[p];
+  apply_live(g, R.form[p] >= 2, R.splits[p]);
   const int splits = R.splits[p];
   long idx = (long)(blockIdx.x - R.first[p]) * blockDim.x + threadIdx.x;
   long total = (long)g.M * g.N;
@@ -148,7 +158,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_group_embed_kernel(GemmGrou
 
 // C = alpha * sum_z ws[z] + beta * C (+ D rows), z ascending: a fixed order, so the
 // result does not depend on how the workgroups were scheduled.
-__global__ void splitk_reduce_kernel(GemmArgs g, int splits) {
+__global__ void splitk_reduce_kernel(GemmArgs g, int splits, bool tA) {
+  apply_live(g, tA, splits);
   long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   long total = (long)g.M * g.N;
   if (idx >= total) return;
@@ -343,6 +354,21 @@ static GemmPlan plan_gemm(int tA, int tB, int M, int N, int K, bool skinny_allow
   return split(GemmPlan::TILE64, t64, s);
 }
 
+// The plan of a product of which `expect` rows of C (or of K) are thought to take part: tiles for all of them.
+static GemmPlan plan_live(int tA, int tB, int M, int N, int K, int lda, int ldb, bool allow_split, int expect) {
+  const int m = tA ? M : std::min(M, std::max(expect, 1)), k = tA ? std::min(K, std::max(expect, 1)) : K;
+  GemmPlan p = plan_gemm(tA, tB, m, N, k, false, allow_split, !far_rows(tA, tB, lda, ldb));
+  const int tile = p.kind == GemmPlan::TILE128 ? 128 : 64;
+  p.tiles = (long)((M + tile - 1) / tile) * ((N + tile - 1) / tile);
+  if (tA) p.kchunk = K;  // (set by the kernel)
+  return p;
+}
+
+static GemmPlan plan_product(const cavs_gemm_desc &q) {
+  return q.live ? plan_live(q.transA, q.transB, q.M, q.N, q.K, q.lda, q.ldb, true, q.live_expect)
+                : plan_gemm(q.transA, q.transB, q.M, q.N, q.K, false, true, !far_rows(q.transA, q.transB, q.lda, q.ldb));
+}
+
 static size_t plan_workspace(const GemmPlan &p, int M, int N) {
   return p.splits > 1 ? sizeof(float) * (size_t)p.splits * M * N : 0;
 }
@@ -362,6 +388,10 @@ static thread_local unsigned t_lds_pad = 0;
 // The grid of a launch of BM x BN tiles: a known block of whole row tiles becomes a launch of its own (GemmArgs::zseg).
 static dim3 tile_grid(GemmArgs *g, int BM, int BN, const GemmPlan &p) {
   dim3 grid((unsigned)p.tiles, p.splits);
+  if (g->live) {  // (the kernel counts its tiles; room for two padded launches)
+    grid.x = (unsigned)((p.tiles + 7) / 8 * 8 + 8);
+    return grid;
+  }
   if (g->zkind == CAVS_GEMM_A_ZERO || g->zkind == CAVS_GEMM_C_UNUSED) {
     const long inside = (long)(std::min(g->zrows, g->M) / BM) * ((g->N + BN - 1) / BN);
     if (inside > 0 && inside < p.tiles) {
@@ -441,15 +471,17 @@ struct BlockHint {
 static int run_gemm(const char *who, int tA, int tB, int M, int N, int K, float alpha, const float *A,
                     int lda, const float *B, int ldb, float beta, float *C, int ldc, const float *D,
                     int ldd, int dshift, void *ws, size_t ws_bytes, void *stream, const PullRows *pull = nullptr,
-                    const BlockHint *hint = nullptr) {
+                    const BlockHint *hint = nullptr, const int *live = nullptr, int live_expect = 0) {
   int rc = check_gemm(who, tA, tB, M, N, K, A, lda, B, ldb, C, ldc);
   if (rc || M == 0 || N == 0) return rc;
   // Looked-up rows: up to 128 of them the skinny kernel, beyond it the 64 x 64 tiles (M x 2048 x 300..512: 21
   // rows 12.4 -> 7.9 us, 120 rows 19.7 -> 15.1, 300 rows 20.5 and 26.2).
-  GemmPlan p = plan_gemm(tA, tB, M, N, K, (!pull || M <= 128) && skinny_ok(tA, tB, K, A, lda, B, ldb), ws != nullptr,
-                         !pull && !far_rows(tA, tB, lda, ldb));
+  GemmPlan p = live ? plan_live(tA, tB, M, N, K, lda, ldb, ws != nullptr, live_expect)
+                    : plan_gemm(tA, tB, M, N, K, (!pull || M <= 128) && skinny_ok(tA, tB, K, A, lda, B, ldb), ws != nullptr,
+                                !pull && !far_rows(tA, tB, lda, ldb));
   hipStream_t st = as_stream(stream);
   GemmArgs g{M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, D, ldd, dshift, p.kchunk, nullptr};
+  g.live = live;
   if (hint) hint->set(&g, tA, tB, beta == 0.f && !D);
   if (pull) {
     g.pull_rows = pull->rows;
@@ -481,7 +513,7 @@ static int run_gemm(const char *who, int tA, int tB, int M, int N, int K, float 
   CAVS_LAUNCH_CHECK();
   if (p.splits > 1) {
     long total = (long)M * N;
-    launch(splitk_reduce_kernel, (unsigned)((total + 255) / 256), 256, 0, st, g, p.splits);
+    launch(splitk_reduce_kernel, (unsigned)((total + 255) / 256), 256, 0, st, g, p.splits, tA != 0);
     CAVS_LAUNCH_CHECK();
   }
   return CAVS_OK;
@@ -502,9 +534,16 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
     CAVS_REQUIRE(q.alpha == 1.f && q.beta == 0.f, "cavs_sgemm_group_embed_bwd: the product that feeds the table takes alpha = 1, beta = 0");
     CAVS_REQUIRE((q.M == 0 || q.N == 0) || (dtable && ids), "cavs_sgemm_group_embed_bwd: null pointer");
     // unsplit (or run alone): the scatter-add reads C
-    tail = EmbedTail{dtable, ids, q.C, q.ldc, 0, 1, nullptr, 0, q.M, q.N, (q.M + kEmbedRows - 1) / kEmbedRows};
+    tail = EmbedTail{dtable, ids, q.C, q.ldc, 0, 1, nullptr, 0, q.M, q.N, (q.M + kEmbedRows - 1) / kEmbedRows,
+                     q.live};
   }
   GemmGroup G{}, R{};
+  // K as the plan sees it, and the number of tiles it expects (cavs_gemm_desc::live)
+  auto plan_K = [](const cavs_gemm_desc &q) { return q.live && q.transA ? std::min(q.K, std::max(q.live_expect, 1)) : q.K; };
+  auto plan_tiles = [](const cavs_gemm_desc &q) {
+    const int m = q.live && !q.transA ? std::min(q.M, std::max(q.live_expect, 1)) : q.M;
+    return (long)((m + 63) / 64) * ((q.N + 63) / 64);
+  };
   double work = 0;
   long tiles[kGroupMax];
   bool alone[kGroupMax];
@@ -521,18 +560,18 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
                  "cavs_sgemm_group: bad block hint in product %d (kind %d, rows %d, col %d)", p, q.zero_kind, q.zero_rows, q.zero_col);
     tiles[p] = (long)((q.M + 63) / 64) * ((q.N + 63) / 64);
     // a product that fills the chip with large tiles by itself is better off on them, alone
-    alone[p] = q.M > 0 && q.N > 0 && plan_gemm(q.transA, q.transB, q.M, q.N, q.K, false, true, !far_rows(q.transA, q.transB, q.lda, q.ldb)).kind == GemmPlan::TILE128;
+    alone[p] = q.M > 0 && q.N > 0 && plan_product(q).kind == GemmPlan::TILE128;
     if (!alone[p] && q.M > 0 && q.N > 0) grouped++;
   }
   for (int p = 0; p < count; p++) {
     const cavs_gemm_desc &q = d[p];
     if (q.M == 0 || q.N == 0) continue;
     if (!alone[p] && grouped >= 2) {
-      work += (double)tiles[p] * q.K;
+      work += (double)plan_tiles(q) * plan_K(q);
       continue;
     }
     alone[p] = true;
-    most = std::max(most, plan_workspace(plan_gemm(q.transA, q.transB, q.M, q.N, q.K, false, true, !far_rows(q.transA, q.transB, q.lda, q.ldb)), q.M, q.N));
+    most = std::max(most, plan_workspace(plan_product(q), q.M, q.N));
   }
   const long slots = 4 * num_cus();
   long kc = (long)(work / (double)slots);
@@ -547,11 +586,12 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
     for (int p = 0; p < count; p++) {
       const cavs_gemm_desc &q = d[p];
       if (q.M == 0 || q.N == 0 || alone[p]) continue;
-      long s = q.K > 0 ? (q.K + chunk / 2) / chunk : 1;
+      const long K = plan_K(q);
+      long s = K > 0 ? (K + chunk / 2) / chunk : 1;
       if (s < 1) s = 1;
-      const long kchunk = q.K > 0 ? ((q.K + s - 1) / s + 31) / 32 * 32 : 1;
-      const long splits = q.K > 0 ? (q.K + kchunk - 1) / kchunk : 1;
-      total += (tiles[p] * splits + 7) / 8 * 8;
+      const long kchunk = K > 0 ? ((K + s - 1) / s + 31) / 32 * 32 : 1;
+      const long splits = K > 0 ? (K + kchunk - 1) / kchunk : 1;
+      total += (plan_tiles(q) * splits + 7) / 8 * 8;
     }
     return total;
   };
@@ -563,12 +603,14 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
   for (int p = 0; p < count; p++) {
     const cavs_gemm_desc &q = d[p];
     if (q.M == 0 || q.N == 0 || alone[p]) continue;
-    long s = q.K > 0 ? (q.K + kc / 2) / kc : 1;
+    const int K = plan_K(q);
+    long s = K > 0 ? (K + kc / 2) / kc : 1;
     if (s < 1) s = 1;
-    int kchunk = q.K > 0 ? (int)(((q.K + s - 1) / s + 31) / 32 * 32) : 1;
-    int splits = q.K > 0 ? (q.K + kchunk - 1) / kchunk : 1;
+    int kchunk = K > 0 ? (int)(((K + s - 1) / s + 31) / 32 * 32) : 1;
+    int splits = K > 0 ? (K + kchunk - 1) / kchunk : 1;
     GemmArgs g{q.M, q.N, q.K, q.A, q.lda, q.B, q.ldb, q.C, q.ldc, q.alpha, q.beta, nullptr, 0, 0, kchunk, nullptr};
-    BlockHint{q.zero_kind, q.zero_rows, q.zero_col}.set(&g, q.transA, q.transB, q.beta == 0.f);
+    g.live = q.live;
+    BlockHint{q.zero_kind, q.live ? 1 : q.zero_rows, q.zero_col}.set(&g, q.transA, q.transB, q.beta == 0.f);
     if (splits > 1) {
       if (ws) g.ws = reinterpret_cast<float *>(static_cast<char *>(ws) + need);
       need += ((size_t)splits * q.M * q.N * sizeof(float) + 255) / 256 * 256;
@@ -591,6 +633,7 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
     } else if (splits > 1) {
       R.g[nr] = g;
       R.splits[nr] = splits;
+      R.form[nr] = q.transA ? 2 : 0;
       R.first[nr + 1] = R.first[nr] + (int)(((long)q.M * q.N + 255) / 256);
       nr++;
     }
@@ -607,9 +650,9 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
   for (int p = 0; p < count; p++) {
     const cavs_gemm_desc &q = d[p];
     if (q.M == 0 || q.N == 0 || !alone[p]) continue;
-    const BlockHint hint{q.zero_kind, q.zero_rows, q.zero_col};
+    const BlockHint hint{q.zero_kind, q.live ? 1 : q.zero_rows, q.zero_col};
     int rc = run_gemm("cavs_sgemm_group", q.transA, q.transB, q.M, q.N, q.K, q.alpha, q.A, q.lda, q.B, q.ldb, q.beta,
-                      q.C, q.ldc, nullptr, 0, 0, ws, ws_bytes, stream, nullptr, &hint);
+                      q.C, q.ldc, nullptr, 0, 0, ws, ws_bytes, stream, nullptr, &hint, q.live, q.live_expect);
     if (rc) return rc;
   }
   hipStream_t st = as_stream(stream);

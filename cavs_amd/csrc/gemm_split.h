@@ -319,19 +319,30 @@ __device__ inline void split_tile_at(int t, int row0, int rows, int tilesN, int 
 template <int BM, int BN, int BK, bool TA, bool TB, bool VEC, bool PULL = false>
 __global__ __launch_bounds__(kThreads, 3) void sgemm_split_kernel(GemmArgs g) {
   __shared__ __attribute__((aligned(16))) char S[split_lds_bytes(BM, BN, BK)];
+  apply_live(g, TA, gridDim.y);
   const int tilesN = (g.N + BN - 1) / BN, tilesM = (g.M + BM - 1) / BM;
+  if (g.live && (g.zkind == CAVS_GEMM_A_ZERO || g.zkind == CAVS_GEMM_C_UNUSED)) {
+    const int inside = min(g.zrows, g.M) / BM * tilesN;
+    g.zseg = inside < tilesM * tilesN ? inside : 0;
+  }
   int t, row0 = 0, rows = tilesM;
   if (g.zseg > 0) {
-    const int first = (g.zseg + 7) & ~7, b = blockIdx.x;
+    const int first = (g.zseg + 7) & ~7, rest = (tilesM * tilesN - g.zseg + 7) & ~7, b = blockIdx.x;
+    if (b >= first + rest) return;
     if (b < first) {
       t = xcd_remap(b, first);
       rows = g.zseg / tilesN;
     } else {
-      t = xcd_remap(b - first, (tilesM * tilesN - g.zseg + 7) & ~7);
+      t = xcd_remap(b - first, rest);
       row0 = g.zseg / tilesN;
       rows = tilesM - row0;
     }
     if (t >= rows * tilesN) return;
+  } else if (g.live) {
+    const int all = (tilesM * tilesN + 7) & ~7;
+    if ((int)blockIdx.x >= all) return;
+    t = xcd_remap(blockIdx.x, all);
+    if (t >= tilesM * tilesN) return;
   } else {
     t = xcd_remap(blockIdx.x, tilesM * tilesN);
   }

@@ -39,7 +39,7 @@ class GemmDesc(C.Structure):
     """cavs_gemm_desc: one product of cavs_sgemm_group"""
     _fields_ = [("transA", _I), ("transB", _I), ("M", _I), ("N", _I), ("K", _I), ("alpha", _F), ("beta", _F),
                 ("A", _P), ("lda", _I), ("B", _P), ("ldb", _I), ("C", _P), ("ldc", _I),
-                ("zero_kind", _I), ("zero_rows", _I), ("zero_col", _I)]
+                ("zero_kind", _I), ("zero_rows", _I), ("zero_col", _I), ("live", _P), ("live_expect", _I)]
 
 
 class BlockCopy(C.Structure):
@@ -99,6 +99,11 @@ _SIGS = {
     "cavs_embed_fwd": [_P, _I, _P, _P, _I, _I, _P],
     "cavs_embed_pull_fwd": [_P, _I, _P, _P, _P, _P, _I, _I, _P],
     "cavs_embed_pull_sgemm": [_P, _I, _P, _I, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _I, _P],
+    "cavs_embed_index": [_P, _P, _P, _P, _I, _I, _I, _P, _Z, _P],
+    "cavs_embed_words": [_P, _I, _P, _P, _I, _I, _P],
+    "cavs_embed_words_bwd": [_P, _P, _P, _I, _I, _I, _P],
+    "cavs_spread_rows": [_P, _I, _P, _I, _P, _I, _I, _I, _I, _P, _P, _P],
+    "cavs_gather_sums": [_P, _I, _P, _I, _P, _I, _I, _P, _Z, _P],
     "cavs_embed_bwd": [_P, _P, _P, _I, _I, _I, _P],
     "cavs_bias_add_rows": [_P, _P, _P, _I, _I, _P],
     "cavs_softmax_xent": [_P, _P, _P, _P, _I, _I, _P],
@@ -173,6 +178,7 @@ _RESTYPE = {"cavs_last_error": C.c_char_p, "cavs_abi_version": _I, "cavs_sgemm_s
             "cavs_colsum_parts": _I, "cavs_round_packed_ok": _I, "cavs_lstm_round_packed_ok": _I,
             "cavs_group_rounds_ok": _I, "cavs_group_max_groups": _I, "cavs_group_rows": _I, "cavs_tail_rounds_ok": _I, "cavs_tail_max_rounds": _I, "cavs_tail_max_groups": _I, "cavs_tail_sync_bytes": _Z,
             "cavs_sgemm_splitk_static_max_bytes": _Z,
+            "cavs_embed_index_ints": _Z, "cavs_embed_index_workspace": _Z, "cavs_gather_sums_workspace": _Z,
             "cavs_schedule_arena_scratch": _Z}
 _NOCHECK = {"cavs_last_error": [], "cavs_abi_version": [], "cavs_sgemm_splitk_workspace": [_I, _I, _I],
             "cavs_fc_softmax_xent_workspace": [_I, _I, _I], "cavs_colsum_blocks_workspace": [_I, _I, _I],
@@ -180,6 +186,7 @@ _NOCHECK = {"cavs_last_error": [], "cavs_abi_version": [], "cavs_sgemm_splitk_wo
             "cavs_fc_softmax_xent_parts": [_I], "cavs_colsum_parts": [_I], "cavs_round_packed_ok": [_I, _I],
             "cavs_lstm_round_packed_ok": [_I, _I], "cavs_sgemm_splitk_static_max_bytes": [],
             "cavs_group_rounds_ok": [_I], "cavs_group_max_groups": [_I], "cavs_group_rows": [], "cavs_tail_rounds_ok": [_I, _I], "cavs_tail_max_rounds": [], "cavs_tail_max_groups": [], "cavs_tail_sync_bytes": [],
+            "cavs_embed_index_ints": [_I], "cavs_embed_index_workspace": [_I], "cavs_gather_sums_workspace": [_I, _I],
             "cavs_schedule_arena_scratch": [_I, _I]}
 
 EW_BINARY = dict(add=0, sub=1, mul=2, div=3, sigmoid_grad=4, tanh_grad=5, relu_grad=6, equal=7)

@@ -2,6 +2,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 
@@ -266,6 +267,7 @@ Engine::~Engine() {
     if (e) cavs_event_destroy(e);
   for (auto &m : marks_)
     if (m.ev) cavs_event_destroy(m.ev);
+  if (word_ev_) cavs_event_destroy(word_ev_);
   if (own_stream_) cavs_stream_destroy(stream_);
 }
 
@@ -454,7 +456,13 @@ void Engine::gemm(int tA, int tB, int M, int N, int K, const float *A, int lda, 
 
 // flops of a product that its block hint declares to be zero or unwanted (the kernels skip them
 // tile by tile)
+static double desc_flops(const cavs_gemm_desc &q) {
+  const double m = q.live && !q.transA ? std::min(q.M, q.live_expect) : q.M, k = q.live && q.transA ? std::min(q.K, q.live_expect) : q.K;
+  return 2.0 * m * q.N * k;
+}
+
 static double hinted_flops(const cavs_gemm_desc &q) {
+  if (q.live) return 0;
   double mnk = 0;
   if (q.zero_kind == CAVS_GEMM_A_ZERO && !q.transA)
     mnk = (double)std::min(q.zero_rows, q.M) * std::max(0, q.K - q.zero_col) * q.N;
@@ -469,7 +477,7 @@ void Engine::gemm_group(const std::vector<cavs_gemm_desc> &products) {
   ProfScope ps(this, K_GEMM);
   check(cavs_sgemm_group(count, products.data(), ws, ws_.capacity() * 4, stream_));
   for (const cavs_gemm_desc &q : products) {
-    c_gemm_flops_ += 2.0 * q.M * q.N * q.K;
+    c_gemm_flops_ += desc_flops(q);
     c_gemm_flops_hinted_ += hinted_flops(q);
   }
   c_launches_ += 1;
@@ -597,6 +605,30 @@ void Engine::reserve_edges() {
     R(dxW_, cap * H);
     R(r_z_, rc * H);
   }
+  // (beside: on the scheduler's stream, while the kernels of the last step run)
+  // (not while the lists of a cached plan are still being copied)
+  words_beside_ = own_stream_ && !direct_ && !cfg_.graph_replay && (cfg_.plan_cache == 0 || (hit_plan_ && hit_plan_->made <= done_step_));
+  words_ = words_wanted(words_beside_);
+  if (words_) {
+    const size_t w = cell_ ? (size_t)cell_->NX * H : 4 * H;
+    size_t most = cell_ ? 0 : w;
+    for (CellStage &st : cells_) {
+      const size_t sw = (size_t)std::max(0, st.spec->xw_hi - st.spec->xw_lo) * H;
+      R(st.word_d, cap * sw);
+      most = std::max(most, sw);
+    }
+    R(xW_words_, cap * w);
+    if (!cell_) R(d_words_, cap * w);
+    R(word_parts_, cavs_gather_sums_workspace((int)cap, (int)most) / 4);
+    for (WordIndex &wi : word_index_) {
+      const size_t ints = cavs_embed_index_ints((int)cap);
+      if (wi.index.capacity() >= ints) continue;
+      check(cavs_stream_sync(stream_));
+      wi.index.reserve(ints);
+      wi.ids.reserve(cap);
+      wi.scratch.reserve(cavs_embed_index_workspace((int)cap) / 4);
+    }
+  }
   if (fused_rows() > 0 && !cell_) R(UT_, (size_t)(cfg_.model == CAVS_MODEL_TREEFC ? 2 : 4) * H * H);
   if (fused_rows() > 0 && ((cfg_.model == CAVS_MODEL_TREELSTM && (cavs_round_packed_ok(1, H) || cavs_round_packed_ok(65, H))) ||
                            (cfg_.model == CAVS_MODEL_LSTM && (cavs_lstm_round_packed_ok(1, H) || cavs_lstm_round_packed_ok(65, H)))))
@@ -621,6 +653,68 @@ void Engine::reserve_edges() {
     R(logits_, (size_t)sched_->B * H + 1);   // root rows / |h| scratch
     R(dlogits_, std::max<size_t>((size_t)sched_->B * H, cap * H));
   }
+}
+
+// Whether x * W and its gradients go by words: every different id of the batch once (cavs_embed_index).
+// Saved: the products' rows of the ids met before (a parse tree's inner vertices all look up one word), at
+// 140 TFLOP/s.  Paid: the index where the step has to wait for it (2368 vertices 15 us, 16000 65, 73000
+// 360), spreading the rows (5 / 24 / 256 us at 2048, 2048, 4096 columns), in the backward pass adding up
+// their gradients (10 / 36 / 345 us).
+bool Engine::words_wanted(bool beside) const {
+  if (N_ < 2048 || cfg_.V <= 0 || cfg_.V >= 1 << 24) return false;
+  if (cell_ ? cell_->NX == 0 || cfg_.H % 4 : cfg_.model != CAVS_MODEL_TREELSTM && cfg_.model != CAVS_MODEL_LSTM) return false;
+  const double n = N_, w = (double)(cell_ ? cell_->NX : 4) * cfg_.H;
+  const double saved = 2.0 * (n - words_expected()) * w * E_ * (trains_ ? 3 : 1) / 140e6;
+  const double paid = (beside ? 0.0 : 8.0 + 0.004 * n) + 6.0 + n * w / 1e6 + (trains_ ? 6.0 + n * w / 0.8e6 : 0.0);
+  return saved > 1.5 * paid;  // (2368 vertices, 2048 columns: 31 against 23 us on paper, no difference measured)
+}
+
+// How many different ids to expect (plans and flop counts only): the leaves' of a tree, half of a text's.
+int Engine::words_expected() const {
+  const double n = nch_ == 2 ? sched_->leaf_prefix + 1.0 : 0.5 * N_, V = cfg_.V;
+  return std::max(1, (int)(V * (1.0 - std::exp(-n / V))));
+}
+
+void Engine::words_index(int leaf_rows) {
+  WordIndex &wi = word_index_[word_slot_];
+  word_slot_ ^= 1;
+  d_words_index_ = wi.index.get();
+  if (words_beside_) {
+    wait_step(wi.used);  // (the step before last)
+    if (!sched_stream_) check(cavs_stream_create(&sched_stream_));
+    if (!word_ev_) check(cavs_event_create(&word_ev_));
+  }
+  wi.used = steps_;
+  buffers_used_ = true;
+  check(cavs_embed_index(wi.index.get(), wi.ids.get(), d_x_, d_t2j_, N_, cfg_.V, leaf_rows, wi.scratch.get(), wi.scratch.capacity() * 4,
+                         words_beside_ ? sched_stream_ : stream_));
+  if (words_beside_) {
+    check(cavs_event_record(word_ev_, sched_stream_));
+    check(cavs_event_sync(word_ev_));
+  }
+}
+
+// xW_ [N, w] = looked-up rows times W; rows of leaves are only wanted below column leaf_w
+void Engine::words_forward(const float *W, int w, int leaf_w) {
+  const int N = N_, lp = leaf_w < w ? sched_->leaf_prefix : 0;
+  const float *ids = word_index_[word_slot_].ids.get();
+  words_index(lp);
+  {
+    ProfScope ps(this, K_GATHER);
+    check(cavs_embed_words(e_.get(), ld_e_, d_words_index_, param("Emb").w, N, E_, stream_));
+  }
+  gemm_group({{0, 0, N, w, E_, 1.f, 0.f, e_.get(), ld_e_, W, w, xW_words_.get(), w, lp > 0 ? CAVS_GEMM_C_UNUSED : 0, lp, leaf_w, d_words_index_,
+               words_expected()}});
+  ProfScope ps(this, K_GATHER);
+  check(cavs_spread_rows(xW_.get(), w, xW_words_.get(), w, d_words_index_, N, w, lp, leaf_w, ids, xs_.get(), stream_));
+  c_launches_ += 3;
+}
+
+// dst [L, w] = the rows of src [N, w] added up by word
+void Engine::words_sum(float *dst, const float *src, int ld_src, int w) {
+  ProfScope ps(this, K_SCATTER);
+  check(cavs_gather_sums(dst, w, src, ld_src, d_words_index_, N_, w, word_parts_.get(), word_parts_.capacity() * 4, stream_));
+  c_launches_ += 2;
 }
 
 // One upload per step (the reference copies a list from pageable memory before every
@@ -726,6 +820,7 @@ void Engine::remember_plan(const int *graph, int B, int maxlen, uint64_t hash) {
   }
   const size_t N = N_, nk = (size_t)nch_ * N;
   p->hash = hash;
+  p->made = steps_;
   p->B = B;
   p->maxlen = maxlen;
   p->pairing = cfg_.pairing;
@@ -1011,6 +1106,7 @@ void Engine::begin_step(const int *graph, int B, int maxlen) {
 
 void Engine::forward_only(const int *graph, int B, int maxlen, const float *x_dev, float *graph_out) {
   state_epoch_++;
+  trains_ = true;
   begin_step(graph, B, maxlen);
   const bool reads_x = cell_ ? cell_->NX > 0 || cell_->XD > 0 : (cfg_.model != CAVS_MODEL_TREEFC || cfg_.use_x);
   if (reads_x && !x_dev) fail(CAVS_EINVAL, "vertex input feed is null");
@@ -1205,6 +1301,7 @@ void Engine::step(const int *graph, int B, int maxlen, const void *x, const void
     std::chrono::steady_clock::time_point t0;
     ~StepTimer() { e->host_step_ms_ = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count(); }
   } step_timer{this, step_t0};
+  trains_ = backward;
   begin_step(graph, B, maxlen);
   const int N = N_;
   const bool needs_x = cfg_.model != CAVS_MODEL_TREEFC || cfg_.use_x;
@@ -1363,16 +1460,17 @@ void Engine::treelstm_forward() {
   if (Upk_.capacity() > 0)
     for (const Round &r : sched_->rounds) any_packed |= !leaf_round(r) && r.n <= fused && cavs_round_packed_ok(r.n, H);
   if (any_packed || group_.first >= 0) ensure_packed();
-  // Pull of the word id, the lookup and x * W: one launch
-  {
+  if (words_) {
+    words_forward(W, 4 * H, 3 * H);
+  } else {  // Pull of the word id, the lookup and x * W: one launch
     ProfScope ps(this, K_GEMM);
     // (a leaf gathers zero rows, so its forget gates multiply zero: their columns of x * W are not wanted)
     check(cavs_embed_pull_sgemm(xW_.get(), 4 * H, e_.get(), ld_e_, xs_.get(), d_x_, d_t2j_, param("Emb").w, N, E, W, 4 * H, 4 * H,
                                 sched_->leaf_prefix, 3 * H, stream_));
+    c_gemm_flops_ += 2.0 * N * 4 * H * E;
+    c_gemm_flops_hinted_ += 2.0 * sched_->leaf_prefix * H * E;
+    c_launches_ += 1;
   }
-  c_gemm_flops_ += 2.0 * N * 4 * H * E;
-  c_gemm_flops_hinted_ += 2.0 * sched_->leaf_prefix * H * E;
-  c_launches_ += 1;
   if (!sched_->batching) {  // leaves are interleaved with internal vertices: their child rows must read as zero
     check(cavs_zero(G_.get(), (size_t)N * 2 * 2 * H * 4, stream_));
     check(cavs_zero(hlr_.get(), (size_t)N * H * 4, stream_));
@@ -1622,11 +1720,18 @@ void Engine::treelstm_backward() {
   const int lp = sched_->leaf_prefix;
   float *dU = param("U").g;
   const bool bias_row = bias_row_ok();  // the ones column of e_ turns row E of dW into the column sums of dxW
+  const float *dx = dxW_.get();  // the gradients of x * W, by vertex or by word
+  const int *live = nullptr;
+  if (words_) {
+    words_sum(d_words_.get(), dxW_.get(), 4 * H, 4 * H);
+    dx = d_words_.get();
+    live = d_words_index_;
+  }
   const std::vector<cavs_gemm_desc> products = {
-      {0, 1, N, E, 4 * H, 1.f, 0.f, dxW_.get(), 4 * H, W, 4 * H, de_.get(), E, CAVS_GEMM_A_ZERO, lp, 3 * H},
+      {0, 1, N, E, 4 * H, 1.f, 0.f, dx, 4 * H, W, 4 * H, de_.get(), E, CAVS_GEMM_A_ZERO, lp, 3 * H, live, words_expected()},
       // (all four padding columns of e_ take part, so that the product keeps 16-byte operand loads)
-      {1, 0, bias_row ? ld_e_ : E, 4 * H, N, 1.f, 0.f, e_.get(), ld_e_, dxW_.get(), 4 * H, param("W").g, 4 * H, CAVS_GEMM_B_ZERO, lp,
-       3 * H},
+      {1, 0, bias_row ? ld_e_ : E, 4 * H, N, 1.f, 0.f, e_.get(), ld_e_, dx, 4 * H, param("W").g, 4 * H, CAVS_GEMM_B_ZERO, lp,
+       3 * H, live, words_expected()},
       {1, 0, H, 3 * H, N - lp, 1.f, 0.f, hlr_.at((size_t)lp * H), H, dxW_.at((size_t)lp * 4 * H), 4 * H, dU, 3 * H},
       {1, 0, H, H, 2 * (N - lp), 1.f, 0.f, G_.at((size_t)2 * lp * 2 * H), 2 * H, dF_.at((size_t)2 * lp * H), H,
        dU + (size_t)3 * H * H, H},
@@ -1752,10 +1857,11 @@ void Engine::gemm_group_embedding_backward(const std::vector<cavs_gemm_desc> &pr
   float *ws = workspace(cavs_sgemm_group_workspace(count, products.data()));
   {
     ProfScope ps(this, K_GEMM);
-    check(cavs_sgemm_group_embed_bwd(count, products.data(), 0, emb.g, xs_.get(), ws, ws_.capacity() * 4, stream_));
+    const float *ids = words_ ? reinterpret_cast<const float *>(d_words_index_ + 4 + 3 * (size_t)N_) : xs_.get();
+    check(cavs_sgemm_group_embed_bwd(count, products.data(), 0, emb.g, ids, ws, ws_.capacity() * 4, stream_));
   }
   for (const cavs_gemm_desc &q : products) {
-    c_gemm_flops_ += 2.0 * q.M * q.N * q.K;
+    c_gemm_flops_ += desc_flops(q);
     c_gemm_flops_hinted_ += hinted_flops(q);
   }
   c_launches_ += 2;
@@ -1769,13 +1875,15 @@ void Engine::gemm_group_embedding_backward(const std::vector<cavs_gemm_desc> &pr
 void Engine::lstm_forward() {
   const int N = N_, H = cfg_.H, E = E_;
   const float *Wx = param("W").w, *Wh = Wx + (size_t)4 * H * E, *Bv = param("Bv").w;
-  {  // Pull of the token id, the lookup and x * W_x: one launch
+  if (words_) {
+    words_forward(Wx, 4 * H, 4 * H);
+  } else {  // Pull of the token id, the lookup and x * W_x: one launch
     ProfScope ps(this, K_GEMM);
     check(cavs_embed_pull_sgemm(xW_.get(), 4 * H, e_.get(), E, xs_.get(), d_x_, d_t2j_, param("Emb").w, N, E, Wx, 4 * H, 4 * H, 0, 0,
                                 stream_));
+    c_gemm_flops_ += 2.0 * N * 4 * H * E;
+    c_launches_ += 1;
   }
-  c_gemm_flops_ += 2.0 * N * 4 * H * E;
-  c_launches_ += 1;
   if (!sched_->batching) check(cavs_zero(G_.get(), (size_t)N * 2 * H * 4, stream_));
   const int fused = fused_rows();
   bool any_packed = false;
@@ -1921,9 +2029,16 @@ void Engine::lstm_backward() {
   }
   const int lp = sched_->leaf_prefix;
   float *dW = param("W").g;
+  const float *dx = dxW_.get();  // the gradients of x * W, by vertex or by word
+  const int *live = nullptr;
+  if (words_) {
+    words_sum(d_words_.get(), dxW_.get(), 4 * H, 4 * H);
+    dx = d_words_.get();
+    live = d_words_index_;
+  }
   gemm_group_embedding_backward({
-      {0, 1, N, E, 4 * H, 1.f, 0.f, dxW_.get(), 4 * H, Wx, 4 * H, de_.get(), E},
-      {1, 0, E, 4 * H, N, 1.f, 0.f, e_.get(), E, dxW_.get(), 4 * H, dW, 4 * H},
+      {0, 1, N, E, 4 * H, 1.f, 0.f, dx, 4 * H, Wx, 4 * H, de_.get(), E, 0, 0, 0, live, words_expected()},
+      {1, 0, E, 4 * H, N, 1.f, 0.f, e_.get(), E, dx, 4 * H, dW, 4 * H, 0, 0, 0, live, words_expected()},
       {1, 0, H, 4 * H, N - lp, 1.f, 0.f, G_.at((size_t)lp * 2 * H), 2 * H, dxW_.at((size_t)lp * 4 * H), 4 * H,
        dW + (size_t)4 * H * E, 4 * H},
   }, E);
@@ -2120,7 +2235,9 @@ void Engine::cell_forward() {
   const CellSpec &c0 = *cells_[0].spec;
   const int N = N_, H = cfg_.H;
   if (!sched_->batching) fail(CAVS_EUNSUPPORTED, "the lowered vertex function needs the batch scheduler (OPT_BATCHING)");
-  if (c0.NX > 0) {
+  if (words_) {
+    words_forward(param(c0.params[c0.W.param].name).w + c0.W.offset, c0.NX * H, c0.NX * H);
+  } else if (c0.NX > 0) {
     ProfScope ps(this, K_GEMM);
     check(cavs_embed_pull_sgemm(xW_.get(), c0.NX * H, e_.get(), ld_e_, xs_.get(), d_x_, d_t2j_, param("Emb").w, N, E_,
                                 param(c0.params[c0.W.param].name).w + c0.W.offset, c0.NX * H, c0.NX * H, 0, 0, stream_));
@@ -2248,18 +2365,22 @@ void Engine::cell_backward() {
   };
   if (c0.NX > 0) {
     float *W = param(c0.params[c0.W.param].name).w + c0.W.offset, *dW = param(c0.params[c0.W.param].name).g + c0.W.offset;
+    const int *live = words_ ? d_words_index_ : nullptr;
     // d e first: the launch that reduces the first group of a function of one stage also scatters it into the table's gradient
-    for (const CellStage &st : cells_) {
+    for (CellStage &st : cells_) {
       const CellSpec &c = *st.spec;
       if (c.xw_hi <= c.xw_lo) continue;
       const int w = (c.xw_hi - c.xw_lo) * H;
-      add({0, 1, N, E_, w, 1.f, 0.f, st.d.at((size_t)c.xw_lo * H), c.ND * H, W + (size_t)c.xw_lo * H, c.NX * H, de_.get(), E_});
+      if (words_) words_sum(st.word_d.get(), st.d.at((size_t)c.xw_lo * H), c.ND * H, w);
+      add({0, 1, N, E_, w, 1.f, 0.f, words_ ? st.word_d.get() : st.d.at((size_t)c.xw_lo * H), words_ ? w : c.ND * H, W + (size_t)c.xw_lo * H, c.NX * H,
+           de_.get(), E_, 0, 0, 0, live, words_expected()});
     }
     for (const CellStage &st : cells_) {
       const CellSpec &c = *st.spec;
       if (c.xw_hi <= c.xw_lo) continue;
       const int w = (c.xw_hi - c.xw_lo) * H;
-      add({1, 0, E_, w, N, 1.f, 0.f, e_.get(), ld_e_, st.d.at((size_t)c.xw_lo * H), c.ND * H, dW + (size_t)c.xw_lo * H, c.NX * H});
+      add({1, 0, E_, w, N, 1.f, 0.f, e_.get(), ld_e_, words_ ? st.word_d.get() : st.d.at((size_t)c.xw_lo * H), words_ ? w : c.ND * H,
+           dW + (size_t)c.xw_lo * H, c.NX * H, 0, 0, 0, live, words_expected()});
     }
   }
   for (size_t ci = 0; ci < cells_.size(); ci++) {
@@ -2332,7 +2453,10 @@ void Engine::embedding_backward_rows() {
     check(cavs_zero(emb.g, emb.n * 4, stream_));
     c_launches_ += 1;
   }
-  check(cavs_embed_bwd(emb.g, xs_.get(), de_.get(), E_, N_, E_, stream_));
+  if (words_)
+    check(cavs_embed_words_bwd(emb.g, d_words_index_, de_.get(), E_, N_, E_, stream_));
+  else
+    check(cavs_embed_bwd(emb.g, xs_.get(), de_.get(), E_, N_, E_, stream_));
   c_launches_ += 1;
   xs_.swap(xs_prev_);
   emb_dirty_n_ = N_;

@@ -347,6 +347,7 @@ class Engine {
     bool graph_off = false;  // recording failed once: ordinary steps from then on
     int recordings = 0;
     uint64_t hash = 0;
+    uint64_t made = 0;  // the step whose stream work fills the lists
     int B = 0, maxlen = 0, pairing = 0;
     std::vector<int32_t> graph;
     std::shared_ptr<Schedule> sched;
@@ -396,6 +397,24 @@ class Engine {
   // Tree-LSTM: e_ carries a column of ones after its E columns, so that the deferred product
   // e^T * dxW yields the bias gradient (column sums of dxW) as row E of dW for free
   int ld_e_ = 0;
+  // x * W and its gradients by words (words_wanted): the index, the products' rows, the gradients' sums
+  struct WordIndex {
+    DeviceArray<int> index;
+    DeviceArray<float> ids, scratch;
+    uint64_t used = 0;  // the last step that reads it
+  };
+  WordIndex word_index_[2];  // of this step and the last: the index is made beside the last step's kernels
+  int word_slot_ = 0;
+  void *word_ev_ = nullptr;
+  bool words_ = false, words_beside_ = false;
+  bool trains_ = true;  // a backward pass follows
+  const int *d_words_index_ = nullptr;
+  DeviceArray<float> xW_words_, d_words_, word_parts_;
+  bool words_wanted(bool beside) const;
+  int words_expected() const;
+  void words_index(int leaf_rows);
+  void words_forward(const float *W, int w, int leaf_w);
+  void words_sum(float *dst, const float *src, int ld_src, int w);
   size_t e_ones_rows_ = 0;       // rows of e_ whose ones column is initialised
   DeviceArray<float> ones_col_;  // [ld_e_]: 1 at column E
   bool bias_row_ok() const;
@@ -483,7 +502,7 @@ class Engine {
   struct CellStage {
     std::shared_ptr<const CellSpec> spec;
     void *module = nullptr;
-    DeviceArray<float> sv, asrc, d, ds, bt, colsum, rows, drows;
+    DeviceArray<float> sv, asrc, d, ds, bt, colsum, rows, drows, word_d;
   };
   std::shared_ptr<const CellSpec> cell_;  // the head of the chain
   std::deque<CellStage> cells_;  // (the arrays do not move)

@@ -196,6 +196,12 @@ typedef struct cavs_gemm_desc {
    * With the zeros where the caller says, results are those without the hint bit for bit (the
    * skipped terms are +-0); a hint is a licence, never an obligation.  0: none. */
   int zero_kind, zero_rows, zero_col;
+  /* Optional: a product over the words of cavs_embed_index, whose number is only known on the device.
+   * live[0] = how many of the M rows of A and C (transA = 0) or of K (transA = 1) take part, at most as
+   * many as the description says; live[1] takes the place of zero_rows if zero_kind is set.
+   * live_expect: the caller's guess of live[0], which only the plan reads.  Null: all of them. */
+  const int *live;
+  int live_expect;
 } cavs_gemm_desc;
 enum { CAVS_GEMM_C_UNUSED = 1, CAVS_GEMM_A_ZERO = 2, CAVS_GEMM_B_ZERO = 3 };
 size_t cavs_sgemm_group_workspace(int count, const cavs_gemm_desc *products);
@@ -250,6 +256,30 @@ int cavs_embed_pull_fwd(float *out, int ld_out, float *ids_out, const float *x, 
 int cavs_embed_pull_sgemm(float *C, int ldc, float *e_out, int ld_e, float *ids_out, const float *x,
                           const int *rows, const float *table, int n, int E, const float *B, int ldb,
                           int N, int unused_rows, int unused_col, void *stream);
+/* The words of a batch, each once, so that what depends on the word alone is done once per word
+ * (cavs/backend/op_impl_embedding_lookup.cu:37-148 looks a row up, and adds a gradient row, per vertex).
+ * cavs_embed_index: ids_out[b] = x[rows[b]] for b < n, and in `index` (cavs_embed_index_ints(n) ints)
+ *   [0]: the number L of different ids; [1]: how many of them occur only in rows below leaf_rows (these
+ *   words come first); then n ints each: the word of row b; the rows ordered by id; the word at each
+ *   place of that order; then n floats, the ids of the words.  Ids that are no whole number
+ *   in [0, V), V < 2^24, are a word per row.
+ * cavs_embed_words: out[s, 0:E] = the table row of word s, s < L.
+ * cavs_embed_words_bwd: the table row of word s += dy[s, 0:E], s < L.
+ * cavs_spread_rows: dst[b, 0:w] = src[word of b, 0:w]; rows below head_rows only columns below head_w; and
+ *   ids_out[b] = ids[b] unless they are null.
+ * cavs_gather_sums: dst[s, 0:w] = the sum of src[b, 0:w] over the rows b of word s, in a fixed order.
+ * Widths and strides are multiples of 4, pointers 16-byte aligned. */
+size_t cavs_embed_index_ints(int n);
+size_t cavs_embed_index_workspace(int n);
+int cavs_embed_index(int *index, float *ids_out, const float *x, const int *rows, int n, int V, int leaf_rows, void *workspace,
+                     size_t workspace_bytes, void *stream);
+int cavs_embed_words(float *out, int ld_out, const int *index, const float *table, int n, int E, void *stream);
+int cavs_embed_words_bwd(float *dtable, const int *index, const float *dy, int ld_dy, int n, int E, void *stream);
+int cavs_spread_rows(float *dst, int ld_dst, const float *src, int ld_src, const int *index, int n, int w, int head_rows, int head_w,
+                     const float *ids, float *ids_out, void *stream);
+size_t cavs_gather_sums_workspace(int n, int w);
+int cavs_gather_sums(float *dst, int ld_dst, const float *src, int ld_src, const int *index, int n, int w, void *workspace,
+                     size_t workspace_bytes, void *stream);
 /* out[r, :] = inp[r, :] + bias[:]  (BinaryBroadcastingKernel,
  * cavs/backend/op_impl_elementwise.cuh:128-139; also the ones-vector bias GEMM of
  * cavs/backend/op_impl_fullyconnected_cublas.cc:74-76) */

@@ -1792,3 +1792,109 @@ def test_sgemm_keeps_every_bit_of_its_operands(g, tA, tB, M, N, K, ld):
     exact = A.astype(np.float64) @ B.astype(np.float64).T
     # (up to K roundings of partial sums of up to sqrt(K) terms of order a third)
     assert np.abs(g.host(Cd) - exact).max() <= 2.0 ** -24 * (K + 16)
+
+
+@pytest.mark.parametrize("n,V,E,w,leaf_rows", [(1, 5, 8, 4, 1), (63, 4, 12, 260, 40), (64, 255, 4, 256, 0), (65, 256, 20, 8, 65), (2368, 21701, 300, 512, 1216),
+                                               (4096, 70000, 8, 12, 100), (4097, 65535, 8, 300, 4000), (9000, 300, 16, 64, 5000), (16384, 1000, 8, 16, 9000),
+                                               (16385, 1000, 8, 16, 9000)])
+def test_words_of_a_batch(g, n, V, E, w, leaf_rows):
+    """cavs_embed_index and what runs over its words, against numpy: one id shared by most rows (segments over many
+    pieces), ids that are no table row, sizes at the edges of a wavefront, of the digits and of the sort in LDS."""
+    import torch
+
+    r = rng(n + V)
+    x = np.floor(r.bulk_uniform(n) * V).astype(np.float32)
+    x[leaf_rows:] = 0.0
+    x[:: max(2, n // 7)] = V - 1
+    if n > 70:
+        x[[3, 17]], x[[40, 41]] = -1.0, [0.5, 0.5]
+    rows = np.argsort(r.bulk_uniform(n)).astype(np.int32)
+    feed = np.empty(n, np.float32)
+    feed[rows] = x
+    L = hip.lib()
+    index, ids = g.devi(np.full(L.cavs_embed_index_ints(n), -9, np.int32)), g.zeros(n)
+    nbytes = max(L.cavs_embed_index_workspace(n), L.cavs_gather_sums_workspace(n, w), 16)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    g.call("cavs_embed_index", g.P(index), g.P(ids), g.P(g.devf(feed)), g.P(g.devi(rows)), n, V, leaf_rows, g.P(ws), nbytes, g.stream())
+    got = g.host(index)
+    np.testing.assert_array_equal(g.host(ids), x)
+    words, leaf_words = got[:2]
+    slot, order, at, word = got[4:4 + n], got[4 + n:4 + 2 * n], got[4 + 2 * n:4 + 3 * n], got[4 + 3 * n:].view(np.float32)
+    odd = (x < 0) | (x != np.floor(x))
+    assert words == len(np.unique(x[~odd])) + odd.sum()
+    inner = np.zeros(words, bool)
+    inner[slot[leaf_rows:]] = True
+    assert leaf_words == (~inner).sum() and not inner[:leaf_words].any()
+    np.testing.assert_array_equal(word[slot], x)
+    np.testing.assert_array_equal(at, slot[order])
+    np.testing.assert_array_equal(np.sort(order), np.arange(n))
+    same = at[1:] == at[:-1]
+    assert (order[1:] > order[:-1])[same].all()
+    # the rows of the words, and what every vertex gets back
+    table = r.bulk_uniform((V + 1) * E, -1, 1).reshape(V + 1, E)
+    out = g.zeros(n, E + 4, fill=7.0)
+    g.call("cavs_embed_words", g.P(out), E + 4, g.P(index), g.P(g.devf(table)), n, E, g.stream())
+    off = (word[:words] * np.float32(E)).astype(np.int64)
+    flat = table.reshape(-1)
+    want = np.stack([flat[o:o + E] if o >= 0 else np.zeros(E, np.float32) for o in off])
+    np.testing.assert_array_equal(g.host(out)[:words, :E], want)
+    np.testing.assert_array_equal(g.host(out)[words:], 7.0)
+    dt = g.zeros(V + 1, E)
+    dy = r.bulk_uniform(n * E, -1, 1).reshape(n, E)
+    g.call("cavs_embed_words_bwd", g.P(dt), g.P(index), g.P(g.devf(dy)), E, n, E, g.stream())
+    dwant = np.zeros((V + 1) * E)
+    for s, o in enumerate(off):
+        if o >= 0:
+            dwant[o:o + E] += dy[s]
+    close(g.host(dt).reshape(-1), dwant)
+    src = r.bulk_uniform(n * w, -1, 1).reshape(n, w)
+    head = w // 8 * 4
+    dst, ids_copy = g.zeros(n, w + 4, fill=7.0), g.zeros(n)
+    g.call("cavs_spread_rows", g.P(dst), w + 4, g.P(g.devf(src)), w, g.P(index), n, w, leaf_rows, head, g.P(ids), g.P(ids_copy), g.stream())
+    np.testing.assert_array_equal(g.host(ids_copy), x)
+    spread = np.full((n, w + 4), 7.0, np.float32)
+    spread[:, :w] = src[slot]
+    spread[:leaf_rows, head:w] = 7.0
+    np.testing.assert_array_equal(g.host(dst), spread)
+    outs = []
+    for _ in range(2):
+        dst = g.zeros(n, w + 4, fill=7.0)
+        g.call("cavs_gather_sums", g.P(dst), w + 4, g.P(g.devf(src)), w, g.P(index), n, w, g.P(ws), nbytes, g.stream())
+        outs.append(g.host(dst))
+    np.testing.assert_array_equal(outs[0], outs[1])
+    sums = np.zeros((words, w))
+    np.add.at(sums, slot, src.astype(np.float64))
+    close(outs[0][:words, :w], sums)
+    np.testing.assert_array_equal(outs[0][words:], 7.0)
+
+
+@pytest.mark.parametrize("M,N,K,L,Z", [(200, 68, 516, 0, 0), (200, 68, 516, 130, 70), (8000, 1024, 300, 4100, 2000), (3000, 300, 2048, 1290, 1200)])
+def test_products_over_the_words_alone(g, M, N, K, L, Z):
+    """cavs_gemm_desc.live: only the first L of the M rows, or of K rows, take part, the known block ends at row Z;
+    alone and grouped, with the guess right, low and high."""
+    import torch
+
+    r = rng(M + N + L)
+    A, B = r.bulk_uniform(M * K, -1, 1).reshape(M, K), r.bulk_uniform(N * K, -1, 1).reshape(N, K)
+    zc = K // 2 // 4 * 4
+    A[:Z, zc:] = 0
+    Y = r.bulk_uniform(M * N, -1, 1).reshape(M, N)
+    A[L:], Y[L:] = np.nan, np.nan
+    live = g.devi(np.array([L, Z], np.int32))
+    dA, dB, dY = g.devf(A), g.devf(B), g.devf(Y)
+    wantC = A[:L].astype(np.float64) @ B.astype(np.float64).T
+    wantG = Y[:L].astype(np.float64).T @ A[:L].astype(np.float64)
+    for expect in (max(L, 1), 1, M):
+        for count in (1, 2):
+            Cd, Gd = g.zeros(M, N, fill=5.0), g.zeros(N, K, fill=float("nan"))
+            descs = (hip.GemmDesc * 2)(hip.GemmDesc(0, 1, M, N, K, 1.0, 0.0, g.P(dA), K, g.P(dB), K, g.P(Cd), N, 2, 0, zc, g.P(live), expect),
+                                       hip.GemmDesc(1, 0, N, K, M, 1.0, 0.0, g.P(dY), N, g.P(dA), K, g.P(Gd), K, 3, 0, zc, g.P(live), expect))
+            for first in ((0, 1) if count == 1 else (0,)):
+                part = (hip.GemmDesc * count)(*descs[first:first + count])
+                nbytes = hip.lib().cavs_sgemm_group_workspace(count, part)
+                ws = torch.empty(max(nbytes // 4, 1), dtype=torch.float32, device="cuda")
+                g.call("cavs_sgemm_group", count, part, g.P(ws), nbytes, g.stream())
+            got = g.host(Cd)
+            close(got[:L], wantC, "rows of the words")
+            np.testing.assert_array_equal(got[L:], 5.0)
+            close(g.host(Gd), wantG, "sum over the words")
