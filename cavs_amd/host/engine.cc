@@ -861,9 +861,18 @@ void Engine::remember_plan(const int *graph, int B, int maxlen, uint64_t hash) {
   plans_.push_back(std::move(p));
 }
 
+// A schedule nobody holds any more (no cached plan), or a new one: a step's vectors keep their memory.
+std::shared_ptr<Schedule> Engine::spare_schedule() {
+  for (auto &s : spare_)
+    if (s.use_count() == 1) return s;
+  auto fresh = std::make_shared<Schedule>();
+  spare_[spare_at_++ % 3] = fresh;
+  return fresh;
+}
+
 void Engine::schedule_on_host(const int *graph, int B, int maxlen) {
   auto t0 = std::chrono::steady_clock::now();
-  auto fresh = std::make_shared<Schedule>();
+  std::shared_ptr<Schedule> fresh = spare_schedule();
   std::string err = build_schedule(graph, B, maxlen, (cfg_.opt & CAVS_OPT_BATCHING) != 0, fresh.get());
   sched_ms_ = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count();
   if (!err.empty()) fail(CAVS_EINVAL, "graph feed rejected: " + err);

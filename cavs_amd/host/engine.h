@@ -220,6 +220,9 @@ class Engine {
   std::map<std::string, std::unique_ptr<Param>> params_;
 
   std::shared_ptr<Schedule> sched_ = std::make_shared<Schedule>();
+  std::shared_ptr<Schedule> spare_[3];
+  unsigned spare_at_ = 0;
+  std::shared_ptr<Schedule> spare_schedule();
   bool sched_lists_on_host_ = true;  // false: the device scheduler built the lists, sched_ holds the rounds only
   bool did_backward_ = false;
   float *fwd_out_ = nullptr;   // where the forward pass returns h by vertex id

@@ -1,94 +1,130 @@
 #include "scheduler.h"
 
 #include <algorithm>
+#include <cstring>
 
 namespace cavs {
 
-// LoadGraph, cavs/midend/graph_scheduler.cc:12-71.
+void Schedule::clear() {
+  B = maxlen = N = executed = max_round = leaf_prefix = 0;
+  batching = true;
+  for (auto *v : {&sample_offset, &parent, &kids, &tids_to_jobids, &jobids_to_tids, &round2offset, &gather_ids[0], &gather_ids[1], &scatter_ids,
+                  &root_tids, &bwd_rounds})
+    v->clear();
+  rounds.clear();
+}
+
+// LoadGraph, cavs/midend/graph_scheduler.cc:12-71.  Children in ascending vertex id (:52-58 appends in
+// vertex order), two slots a vertex.
 static std::string load_graph(const int32_t *g, int B, int maxlen, Schedule *s) {
   s->B = B;
   s->maxlen = maxlen;
-  s->sample_offset.assign(B, 0);
-  s->parent.clear();
-  int off = 0;
+  s->sample_offset.resize(B);
+  int N = 0;
   for (int i = 0; i < B; i++) {
     const int32_t *row = g + (size_t)i * maxlen;
     int k = 0;
     while (k < maxlen && row[k] != -1) k++;
     if (k == maxlen) return "sample " + std::to_string(i) + " has no -1 terminator within maxlen";
-    int len = k + 1;
-    s->sample_offset[i] = off;
+    s->sample_offset[i] = N;
+    N += k + 1;
+  }
+  s->N = N;
+  s->parent.resize(N);
+  s->kids.assign(2 * (size_t)N, -1);
+  // (which of two slots a child takes, and below which child completes its parent, is as good as random:
+  // both without a branch, 21 -> 8 ns per vertex for the schedule of 256 parse trees)
+  std::vector<unsigned char> count(N, 0);
+  int *parent = s->parent.data(), *kids = s->kids.data();
+  unsigned crowded = 0;
+  for (int i = 0; i < B; i++) {
+    const int32_t *row = g + (size_t)i * maxlen;
+    const int off = s->sample_offset[i], len = (i + 1 < B ? s->sample_offset[i + 1] : N) - off;
     for (int j = 0; j < len - 1; j++) {
       if (row[j] < 0 || row[j] >= len)
         return "sample " + std::to_string(i) + ": parent id out of range at vertex " + std::to_string(j);
-      s->parent.push_back(off + row[j]);
+      const int p = off + row[j];
+      parent[off + j] = p;
+      const unsigned n = count[p];
+      count[p] = (unsigned char)(n < 2 ? n + 1 : 2);
+      kids[2 * (size_t)p + (n != 0)] = off + j;
+      crowded |= n & 2;
     }
-    s->parent.push_back(-1);
-    off += len;
+    parent[off + len - 1] = -1;
   }
-  const int N = s->N = off;
-  // children in ascending vertex id (graph_scheduler.cc:52-58 appends in vertex order)
-  s->child_begin.assign(N + 1, 0);
-  for (int v = 0; v < N; v++)
-    if (s->parent[v] >= 0) s->child_begin[s->parent[v] + 1]++;
-  for (int v = 0; v < N; v++) s->child_begin[v + 1] += s->child_begin[v];
-  s->child.assign(s->child_begin[N], 0);
-  std::vector<int> fill(s->child_begin.begin(), s->child_begin.end() - 1);
-  for (int v = 0; v < N; v++)
-    if (s->parent[v] >= 0) s->child[fill[s->parent[v]]++] = v;
+  for (int v = 0; crowded && v < N; v++) {
+    const long n = count[v] < 2 ? 0 : std::count(s->parent.begin(), s->parent.end(), v);
+    if (n > 2)
+      return "vertex " + std::to_string(v) + " has " + std::to_string(n) + " children; the scheduler's gather lists hold two (graph_scheduler.h:16-18)";
+  }
   return "";
 }
 
-static inline int nchild(const Schedule &s, int v) { return s.child_begin[v + 1] - s.child_begin[v]; }
+static inline int nchild(const Schedule &s, int v) { return (s.kids[2 * (size_t)v] >= 0) + (s.kids[2 * (size_t)v + 1] >= 0); }
 
 // BatchGraphScheduler::Initialize / ActivateNext, forward branch
-// (cavs/midend/graph_scheduler.cc:169-193, 202-245).
+// (cavs/midend/graph_scheduler.cc:169-193, 202-245).  One pass over the vertices in tensor-id order: a vertex
+// joins the next round when the last of its children has its id.
 static void batch_rounds(Schedule *s) {
   const int N = s->N;
-  s->tids_to_jobids.assign(N, 0);
+  s->tids_to_jobids.assign(N + 1, 0);  // (one more: a candidate behind the last vertex)
   s->jobids_to_tids.assign(N, 0);
+  s->scatter_ids.resize(N);
+  for (auto &g : s->gather_ids) g.resize(N);
   s->round2offset.assign(1, 0);
-  std::vector<int> activated(N, 0);
+  std::vector<int> waiting(N);  // children that have not run
+  const int *parent = s->parent.data(), *kids = s->kids.data();
+  int *job = s->tids_to_jobids.data(), *tid = s->jobids_to_tids.data(), *scatter = s->scatter_ids.data();
+  int *gather[2] = {s->gather_ids[0].data(), s->gather_ids[1].data()}, gathers[2] = {0, 0}, scatters = 0;
   int begin = 0, end = 0;  // current round = tids [begin, end)
-  for (int v = 0; v < N; v++)
-    if (nchild(*s, v) == 0 && s->parent[v] >= 0) {
-      s->tids_to_jobids[end] = v;
-      s->jobids_to_tids[v] = end;
-      end++;
+  for (int v = 0; v < N; v++) {
+    const int n = (kids[2 * (size_t)v] >= 0) + (kids[2 * (size_t)v + 1] >= 0);
+    waiting[v] = n;
+    if (n == 0 && parent[v] >= 0) {
+      job[end] = v;
+      tid[v] = end++;
     }
+  }
   s->leaf_prefix = end;
   while (end > begin) {
+    // lists this round exposes: gather lists were appended while the round was being
+    // formed (below); the scatter list holds the non-root jobs in job order
     Round r;
     r.offset = begin;
     r.n = end - begin;
-    // lists this round exposes: gather lists were appended while the round was being
-    // formed (below); the scatter list holds the non-root jobs in job order
-    for (int c = 0; c < 2; c++) r.gather_end[c] = (int)s->gather_ids[c].size();
-    r.scatter_begin = (int)s->scatter_ids.size();
-    for (int t = begin; t < end; t++)
-      if (s->parent[s->tids_to_jobids[t]] >= 0) s->scatter_ids.push_back(t);
-    r.scatter_end = (int)s->scatter_ids.size();
-    for (int c = 0; c < 2; c++)
+    for (int c = 0; c < 2; c++) {
+      r.gather_end[c] = gathers[c];
       r.gather_begin[c] = s->rounds.empty() ? r.gather_end[c] : s->rounds.back().gather_end[c];
+    }
+    r.scatter_begin = scatters;
+    int next = end;
+    for (int t = begin; t < end; t++) {
+      const int p = parent[job[t]];
+      if (p < 0) continue;
+      scatter[scatters++] = t;
+      job[next] = p;  // (stays if this was the last child; the next candidate overwrites it otherwise)
+      tid[p] = next;
+      next += --waiting[p] == 0;
+    }
+    for (int t = end; t < next; t++) {
+      const int p = job[t];
+      for (int i = 0; i < 2; i++) {
+        const int c = kids[2 * (size_t)p + i];
+        if (c >= 0) gather[i][gathers[i]++] = tid[c];
+      }
+      if (parent[p] < 0) s->root_tids.push_back(t);
+    }
+    r.scatter_end = scatters;
     s->rounds.push_back(r);
     s->max_round = std::max(s->max_round, r.n);
     s->round2offset.push_back(end);
-    int next = end;
-    for (int t = begin; t < end; t++) {
-      int p = s->parent[s->tids_to_jobids[t]];
-      if (p < 0) continue;
-      if (++activated[p] == nchild(*s, p)) {
-        s->tids_to_jobids[next] = p;
-        s->jobids_to_tids[p] = next;
-        for (int i = 0; i < nchild(*s, p) && i < 2; i++)
-          s->gather_ids[i].push_back(s->jobids_to_tids[s->child[s->child_begin[p] + i]]);
-        if (s->parent[p] < 0) s->root_tids.push_back(next);
-        next++;
-      }
-    }
     begin = end;
     end = next;
   }
+  if (end < N) job[end] = 0;  // (a candidate that never became ready)
+  s->tids_to_jobids.resize(N);
+  s->scatter_ids.resize(scatters);
+  for (int c = 0; c < 2; c++) s->gather_ids[c].resize(gathers[c]);
   s->executed = end;
   for (int k = (int)s->rounds.size() - 1; k >= 0; k--) s->bwd_rounds.push_back(k);
 }
@@ -118,7 +154,7 @@ static void serial_rounds(Schedule *s) {
     r.n = 1;
     for (int c = 0; c < 2; c++) {
       r.gather_begin[c] = (int)s->gather_ids[c].size();
-      if (nchild(*s, v) > c) s->gather_ids[c].push_back(s->child[s->child_begin[v] + c]);
+      if (nchild(*s, v) > c) s->gather_ids[c].push_back(s->kids[2 * (size_t)v + c]);
       r.gather_end[c] = (int)s->gather_ids[c].size();
     }
     r.scatter_begin = (int)s->scatter_ids.size();
@@ -147,7 +183,7 @@ static void serial_rounds(Schedule *s) {
   for (size_t head = 0; head < bf.size(); head++) {
     int v = bf[head];
     if (nchild(*s, v) > 0) {
-      for (int k = s->child_begin[v]; k < s->child_begin[v + 1]; k++) bf.push_back(s->child[k]);
+      for (int k = 0; k < nchild(*s, v); k++) bf.push_back(s->kids[2 * (size_t)v + k]);
     } else if (++sample_id < s->B) {
       init_sample(sample_id);
     }
@@ -156,15 +192,11 @@ static void serial_rounds(Schedule *s) {
 }
 
 std::string build_schedule(const int32_t *graph, int B, int maxlen, bool batching, Schedule *out) {
-  *out = Schedule();
+  out->clear();
   out->batching = batching;
   if (!graph || B <= 0 || maxlen <= 0) return "empty graph feed";
   std::string err = load_graph(graph, B, maxlen, out);
   if (!err.empty()) return err;
-  for (int v = 0; v < out->N; v++)
-    if (nchild(*out, v) > 2)
-      return "vertex " + std::to_string(v) + " has " + std::to_string(nchild(*out, v)) +
-             " children; the scheduler's gather lists hold two (graph_scheduler.h:16-18)";
   if (batching) batch_rounds(out); else serial_rounds(out);
   if (out->executed != out->N) {
     // A sample of a single vertex is never executed (graph_scheduler.cc:180); the schedule of the
@@ -185,28 +217,42 @@ std::string build_schedule(const int32_t *graph, int B, int maxlen, bool batchin
 std::string build_index_lists(const Schedule &s, int nch, int pairing, int *t2j, int *pair, int *child, int *roots) {
   const int N = s.N;
   std::copy(s.tids_to_jobids.begin(), s.tids_to_jobids.end(), t2j);
-  std::fill(pair, pair + N, -1);
-  std::fill(child, child + (size_t)nch * N, -1);
+  if (s.executed != N) {  // (rows no round covers)
+    std::fill(pair, pair + N, -1);
+    std::fill(child, child + (size_t)nch * N, -1);
+  }
   for (const Round &r : s.rounds) {
     const int m = r.scatter_end - r.scatter_begin;
+    const int *sc = s.scatter_ids.data() + r.scatter_begin;
     if (pairing == 0) {
-      for (int b = 0; b < m; b++) pair[r.offset + b] = s.scatter_ids[r.scatter_begin + b];
+      std::copy(sc, sc + m, pair + r.offset);
+      std::fill(pair + r.offset + m, pair + r.offset + r.n, -1);
     } else {
-      for (int b = 0; b < m; b++) pair[s.scatter_ids[r.scatter_begin + b]] = s.scatter_ids[r.scatter_begin + b];
+      std::fill(pair + r.offset, pair + r.offset + r.n, -1);
+      for (int b = 0; b < m; b++) pair[sc[b]] = sc[b];
     }
-    if (r.gather_begin[0] == r.gather_end[0] && r.gather_begin[1] == r.gather_end[1]) continue;  // a round of leaves
-    for (int c = 0; c < nch; c++) {
-      const int len = r.gather_end[c] - r.gather_begin[c];
-      if (len != r.n)
+    int *ch = child + (size_t)nch * r.offset;
+    if (r.gather_begin[0] == r.gather_end[0] && r.gather_begin[1] == r.gather_end[1]) {  // a round of leaves
+      std::fill(ch, ch + (size_t)nch * r.n, -1);
+      continue;
+    }
+    for (int c = 0; c < nch; c++)
+      if (r.gather_end[c] - r.gather_begin[c] != r.n)
         return "round at tensor id " + std::to_string(r.offset) + " mixes vertices with and without child " + std::to_string(c) +
                " (the reference's gather lists misalign there too)";
-      for (int b = 0; b < len; b++) child[(size_t)nch * (r.offset + b) + c] = s.gather_ids[c][r.gather_begin[c] + b];
+    const int *g0 = s.gather_ids[0].data() + r.gather_begin[0], *g1 = s.gather_ids[1].data() + r.gather_begin[1];
+    if (nch == 1) {
+      std::copy(g0, g0 + r.n, ch);
+      if (r.gather_end[1] != r.gather_begin[1]) return "a chain vertex function got a vertex with two children";
+    } else {
+      for (int b = 0; b < r.n; b++) {
+        ch[2 * (size_t)b] = g0[b];
+        ch[2 * (size_t)b + 1] = g1[b];
+      }
     }
-    if (nch == 1 && r.gather_end[1] != r.gather_begin[1]) return "a chain vertex function got a vertex with two children";
   }
-  int nr = 0;
-  for (int v = 0; v < N; v++)
-    if (s.parent[v] < 0) roots[nr++] = v;
+  // (a sample ends with its root, load_graph)
+  for (int i = 0; i < s.B; i++) roots[i] = (i + 1 < s.B ? s.sample_offset[i + 1] : N) - 1;
   return "";
 }
 
@@ -216,35 +262,50 @@ bool build_forest_lists(const Schedule &s, int nch, int fused_limit, const int *
   *n_orphans = 0;
   auto leaf_round = [](const Round &r) { return r.gather_begin[0] == r.gather_end[0] && r.gather_begin[1] == r.gather_end[1]; };
   if (!s.batching || s.rounds.empty() || !leaf_round(s.rounds[0]) || s.rounds[0].n != s.leaf_prefix) return false;
-  std::vector<int> inv_pair(N, -1), round_of_row(N);
-  for (size_t k = 0; k < s.rounds.size(); k++) {
-    const Round &r = s.rounds[k];
-    if (k > 0 && (leaf_round(r) || r.n > fused_limit)) return false;  // every round with children runs as a fused launch
-    for (int b = 0; b < r.n; b++) round_of_row[r.offset + b] = (int)k;
-  }
+  for (size_t k = 1; k < s.rounds.size(); k++)
+    if (leaf_round(s.rounds[k]) || s.rounds[k].n > fused_limit) return false;  // every round with children runs as a fused launch
+  std::vector<int> writer(N, -1);  // of a pool row; -2: read
   for (int v = 0; v < N; v++) {
     const int p = pair[v];
-    if (p < 0) continue;
-    if (p >= N || inv_pair[p] >= 0) return false;  // two writers of one pool row
-    inv_pair[p] = v;
+    if (p < 0) {
+      orphans[(*n_orphans)++] = v;
+      continue;
+    }
+    if (p >= N || writer[p] >= 0) return false;  // two writers of one pool row
+    writer[p] = v;
   }
-  std::vector<char> read(N, 0);
-  for (size_t i = 0; i < (size_t)nch * N; i++) {
-    kid_rows[i] = -1;
-    const int p = child[i];
-    if (p < 0) continue;
-    const int b = (int)(i / nch);
-    if (p >= N || inv_pair[p] < 0 || read[p]) return false;  // reads a row nobody wrote, or a second reader
-    const int v = inv_pair[p];
-    if (round_of_row[v] >= round_of_row[b]) return false;
-    read[p] = 1;
-    kid_rows[i] = v;
+  int unread = N - *n_orphans;
+  for (const Round &r : s.rounds)
+    for (size_t i = (size_t)nch * r.offset; i < (size_t)nch * (r.offset + r.n); i++) {
+      kid_rows[i] = -1;
+      const int p = child[i];
+      if (p < 0) continue;
+      // reads a row nobody wrote, or a second reader, or a reader in a round not after its writer's
+      if (p >= N || writer[p] < 0 || writer[p] >= r.offset) return false;
+      kid_rows[i] = writer[p];
+      writer[p] = -2;
+      unread--;
+    }
+  return unread == 0;  // (a message nobody reads: its gradient is whatever the pool holds)
+}
+
+// The trees of the message flow among the rows from `lo` on: comp[v] the tree of row v (v >= lo), weight its rows.
+static void label_trees(const int *kid_rows, int nch, int N, int lo, std::vector<int> *comp_out, std::vector<int> *weight) {
+  comp_out->assign((size_t)N + 1, -1);
+  weight->clear();
+  int *comp = comp_out->data();
+  for (int v = N - 1; v >= lo; v--) {  // a row's consumer sits in a later round: parents come first
+    if (comp[v] < 0) {
+      comp[v] = (int)weight->size();
+      weight->push_back(0);
+    }
+    (*weight)[comp[v]]++;
+    // (rows before `lo` and missing children too: without a branch that is as good as random)
+    for (int i = 0; i < nch; i++) {
+      const int c = kid_rows[(size_t)nch * v + i];
+      comp[c < 0 ? N : c] = comp[v];
+    }
   }
-  for (int v = 0; v < N; v++) {
-    if (pair[v] >= 0 && !read[pair[v]]) return false;  // a message nobody reads: its gradient is whatever the pool holds
-    if (pair[v] < 0) orphans[(*n_orphans)++] = v;
-  }
-  return true;
 }
 
 // Which rounds run inside the tail launches, and who runs which row.  The rounds are a suffix of the
@@ -267,19 +328,7 @@ void build_tail_lists(const Schedule &s, const int *kid_rows, int lim, int group
     for (int k = k0; k < R && ok; k++) ok = !leaf_round(s.rounds[k]);
     if (!ok) continue;
     const int lo = s.rounds[k0].offset;
-    comp.assign(N - lo, -1);
-    weight.clear();
-    for (int v = N - 1; v >= lo; v--) {  // a row's consumer sits in a later round: parents come first
-      if (comp[v - lo] < 0) {
-        comp[v - lo] = (int)weight.size();
-        weight.push_back(0);
-      }
-      weight[comp[v - lo]]++;
-      for (int i = 0; i < 2; i++) {
-        const int c = kid_rows[2 * (size_t)v + i];
-        if (c >= lo) comp[c - lo] = comp[v - lo];
-      }
-    }
+    label_trees(kid_rows, 2, N, lo, &comp, &weight);
     order.resize(weight.size());
     for (size_t i = 0; i < order.size(); i++) order[i] = (int)i;
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return weight[a] > weight[b]; });
@@ -296,7 +345,7 @@ void build_tail_lists(const Schedule &s, const int *kid_rows, int lim, int group
     const int nr = R - k0;
     per.assign((size_t)G * nr, 0);
     for (int k = k0; k < R; k++)
-      for (int b = s.rounds[k].offset; b < s.rounds[k].offset + s.rounds[k].n; b++) per[(size_t)group[comp[b - lo]] * nr + (k - k0)]++;
+      for (int b = s.rounds[k].offset; b < s.rounds[k].offset + s.rounds[k].n; b++) per[(size_t)group[comp[b]] * nr + (k - k0)]++;
     int lists = 0;
     for (int g = 0; g < G && ok; g++) {
       int mine = 0;
@@ -325,7 +374,7 @@ void build_tail_lists(const Schedule &s, const int *kid_rows, int lim, int group
     {
       std::vector<int> cur(at);
       for (int k = k0; k < R; k++)
-        for (int b = s.rounds[k].offset; b < s.rounds[k].offset + s.rounds[k].n; b++) rows_out[cur[(size_t)group[comp[b - lo]] * nr + (k - k0)]++] = b;
+        for (int b = s.rounds[k].offset; b < s.rounds[k].offset + s.rounds[k].n; b++) rows_out[cur[(size_t)group[comp[b]] * nr + (k - k0)]++] = b;
     }
     // A group's share of a round as lists of at most `slice` rows: the first waits for the rounds the
     // group has done so far, the last is an arrival.  Forward: rounds in order; backward: reversed.
@@ -367,22 +416,10 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
   if (lim <= 0 || groups < 1 || slice < 1 || !s.batching || R < 3) return;
   int k0 = R;  // the rounds with children that no larger one follows
   while (k0 > 1 && !leaf_round(s.rounds[k0 - 1]) && s.rounds[k0 - 1].n <= (long)groups * lim) k0--;
-  std::vector<int> comp, weight, order, group, per;
+  std::vector<int> comp, weight, order, group, per, cell;
   for (; R - k0 >= 2; k0++) {
     const int lo = s.rounds[k0].offset, nr = R - k0;
-    comp.assign(N - lo, -1);
-    weight.clear();
-    for (int v = N - 1; v >= lo; v--) {  // a row's consumer sits in a later round: parents come first
-      if (comp[v - lo] < 0) {
-        comp[v - lo] = (int)weight.size();
-        weight.push_back(0);
-      }
-      weight[comp[v - lo]]++;
-      for (int i = 0; i < nch; i++) {
-        const int c = kid_rows[(size_t)nch * v + i];
-        if (c >= lo) comp[c - lo] = comp[v - lo];
-      }
-    }
+    label_trees(kid_rows, nch, N, lo, &comp, &weight);
     // heaviest tree first to the group with the least so far
     const int G = std::min<int>(groups, (int)weight.size());
     order.resize(weight.size());
@@ -397,9 +434,13 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
     }
     per.assign((size_t)G * nr, 0);
     bool ok = true;
+    cell.resize(N - lo);  // which group's share of which round a row belongs to
     for (int k = k0; k < R; k++)
-      for (int b = s.rounds[k].offset; b < s.rounds[k].offset + s.rounds[k].n; b++)
-        ok &= ++per[(size_t)group[comp[b - lo]] * nr + (k - k0)] <= lim;
+      for (int b = s.rounds[k].offset; b < s.rounds[k].offset + s.rounds[k].n; b++) {
+        const int i = group[comp[b]] * nr + (k - k0);
+        cell[b - lo] = i;
+        ok &= ++per[i] <= lim;
+      }
     if (!ok) continue;
 
     GroupLists &t = *out;
@@ -416,17 +457,16 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
     t.fwd.recs = 0;
     t.bwd.recs = t.rows * 8;
     cur = at;
-    for (int k = k0; k < R; k++)
-      for (int b = s.rounds[k].offset; b < s.rounds[k].offset + s.rounds[k].n; b++) {
-        const int i = cur[(size_t)group[comp[b - lo]] * nr + (k - k0)]++;
-        int *f = block + t.fwd.recs + 8 * (size_t)i, *w = block + t.bwd.recs + 8 * (size_t)i;
-        const int *c = child + (size_t)nch * b, *q = kid_rows + (size_t)nch * b;
-        const int c1 = nch == 2 ? c[1] : -1, q1 = nch == 2 ? q[1] : -1;
-        const int fr[8] = {b, c[0], c1, pair[b], t2j[b], 0, 0, 0};
-        const int br[8] = {b, q[0], q1, q[0] >= 0 ? t2j[q[0]] : -1, q1 >= 0 ? t2j[q1] : -1, 0, 0, 0};
-        std::copy(fr, fr + 8, f);
-        std::copy(br, br + 8, w);
-      }
+    for (int b = lo; b < N; b++) {
+      const int i = cur[cell[b - lo]]++;
+      int *f = block + t.fwd.recs + 8 * (size_t)i, *w = block + t.bwd.recs + 8 * (size_t)i;
+      const int *c = child + (size_t)nch * b, *q = kid_rows + (size_t)nch * b;
+      const int c1 = nch == 2 ? c[1] : -1, q1 = nch == 2 ? q[1] : -1;
+      const int fr[8] = {b, c[0], c1, pair[b], t2j[b], 0, 0, 0};
+      const int br[8] = {b, q[0], q1, q[0] >= 0 ? t2j[q[0]] : -1, q1 >= 0 ? t2j[q1] : -1, 0, 0, 0};
+      std::memcpy(f, fr, sizeof fr);
+      std::memcpy(w, br, sizeof br);
+    }
     size_t end = 2 * t.rows * 8;
     // A direction: a group's share of a round as lists of at most `slice` rows; the first waits for the
     // rounds the group has done so far, the last is an arrival.
@@ -459,7 +499,7 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
 
 void schedule_from_lists(int B, int maxlen, int N, int nch, const int *round2offset, int R, const int *t2j,
                          const int *pair, const int *child, const int *roots, Schedule *out) {
-  *out = Schedule();
+  out->clear();
   Schedule &s = *out;
   s.B = B;
   s.maxlen = maxlen;
@@ -501,15 +541,12 @@ void schedule_from_lists(int B, int maxlen, int N, int nch, const int *round2off
   s.executed = N;
   s.leaf_prefix = R > 0 ? round2offset[1] : 0;
   for (int k = R - 1; k >= 0; k--) s.bwd_rounds.push_back(k);
-  // children in ascending vertex id, as LoadGraph builds them
-  s.child_begin.assign(N + 1, 0);
+  s.kids.assign(2 * (size_t)N, -1);  // as load_graph builds them
   for (int v = 0; v < N; v++)
-    if (s.parent[v] >= 0) s.child_begin[s.parent[v] + 1]++;
-  for (int v = 0; v < N; v++) s.child_begin[v + 1] += s.child_begin[v];
-  s.child.assign(s.child_begin[N], 0);
-  std::vector<int> fill(s.child_begin.begin(), s.child_begin.end() - 1);
-  for (int v = 0; v < N; v++)
-    if (s.parent[v] >= 0) s.child[fill[s.parent[v]]++] = v;
+    if (s.parent[v] >= 0) {
+      int *k = &s.kids[2 * (size_t)s.parent[v]];
+      k[k[0] >= 0] = v;
+    }
 }
 
 // trace_format: [N, R_fwd, R_bwd, then per round: offset, n_exec, exec..., n_g0, g0...,

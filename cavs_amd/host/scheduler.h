@@ -28,8 +28,7 @@ struct Schedule {
   bool batching = true;
   std::vector<int> sample_offset;  // [B]
   std::vector<int> parent;         // [N] global parent id or -1
-  std::vector<int> child_begin;    // [N+1] CSR over children, ascending vertex id
-  std::vector<int> child;          // [N - roots]
+  std::vector<int> kids;           // [2N] children of a vertex, ascending vertex id; -1: none
   std::vector<Round> rounds;       // forward order; backward replays them reversed
   std::vector<int> tids_to_jobids; // [N] (= concatenated job lists of the rounds)
   std::vector<int> jobids_to_tids; // [N]
@@ -41,6 +40,8 @@ struct Schedule {
   int executed = 0;                // vertices that ran (N minus single-vertex samples)
   int max_round = 0;               // largest round size
   int leaf_prefix = 0;             // leading tensor ids that are all leaves (batch: round 0)
+
+  void clear();  // as after construction, but the vectors keep their memory
 
   // Serialises the rounds exactly as the reference's ops would see them, forward
   // then (optionally) backward: see `trace_format` in scheduler.cc.
