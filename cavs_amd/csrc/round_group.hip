@@ -13,6 +13,7 @@
 //     stands between two rounds;
 //   * the plan is read from memory, so a launch runs any number of rounds (chains of hundreds).
 // A wavefront owns ceil(H / 128) k-groups of 16 of its workgroup's columns; those beyond H multiply by zero weights.
+#include <algorithm>
 #include <type_traits>
 
 #include "round_sync.h"
@@ -51,10 +52,10 @@ struct GroupWalk {
   const int4 *lists, *recs;
   unsigned *status, *gsync;
   int nlists, ct;
-  unsigned total;
+  unsigned arrived;
   int4 cur, nxt, ahead, rec;
   bool first_wait;
-  __device__ inline bool start(const GroupPlan &p, int4 (*s_rec)[2 * kGroupRows]) {
+  __device__ inline bool start(const GroupPlan &p, int4 (*s_rec)[2 * kGroupRows], int *s_bail) {
     const int idx = blockIdx.x >> 3, grp = (blockIdx.x & 7) + 8 * (idx / p.wgs);  // workgroup b sits on XCD b % 8
     ct = idx % p.wgs;
     if (grp >= p.ngroups) return false;
@@ -67,8 +68,9 @@ struct GroupWalk {
     if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return false;
     lists = p.lists + g.x;
     recs = p.recs;
-    total = (unsigned)g.z * p.expect;
+    arrived = 0;
     first_wait = true;
+    if (threadIdx.x == 0) *s_bail = 0;
     cur = lists[0];
     nxt = lists[nlists > 1 ? 1 : 0];
     if (threadIdx.x < 2 * kGroupRows) s_rec[0][threadIdx.x] = record(cur);
@@ -83,22 +85,19 @@ struct GroupWalk {
     ahead = lists[r + 2 < nlists ? r + 2 : nlists - 1];
     if (threadIdx.x < 2 * kGroupRows) rec = record(nxt);
   }
-  // false: give up
-  __device__ inline bool wait(const GroupPlan &p, int *s_bail) {
-    if (cur.z > 0) {
-      if (!tail_wait(status, gsync, (unsigned)cur.z * p.expect, p.spin_max, first_wait, s_bail)) return false;
-      first_wait = false;
-    } else {
-      __syncthreads();
-    }
-    return true;
+  // (where there is nothing to wait for, the barrier at the end of the list before is enough; a wait that gives up
+  // sets *s_bail, looked at behind the barrier that completes the partial sums)
+  __device__ inline void wait(const GroupPlan &p, int *s_bail) {
+    if (cur.z <= 0) return;
+    tail_wait(status, gsync, (unsigned)cur.z, p.expect, p.spin_max, first_wait, s_bail);
+    first_wait = false;
   }
   // before the barrier that completes the list's partial sums
   __device__ inline void keep_next(int r, int4 (*s_rec)[2 * kGroupRows]) const {
     if (threadIdx.x < 2 * kGroupRows) s_rec[(r + 1) & 1][threadIdx.x] = rec;
   }
   __device__ inline void done() {
-    if (cur.w) tail_arrive(gsync, total);
+    if (cur.w) tail_arrive(gsync, ct, ++arrived);
     else __syncthreads();
   }
   __device__ inline void advance() {
@@ -148,7 +147,7 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
   __shared__ int4 s_rec[2][2 * kGroupRows];
   __shared__ int s_bail;
   GroupWalk w;
-  if (!w.start(a.plan, s_rec)) return;
+  if (!w.start(a.plan, s_rec, &s_bail)) return;
   const int H = a.H, KG = H / 16, tid = threadIdx.x, lane = tid & 63, ks = tid >> 6;
   const int x = lane & 15, slot = lane >> 4, j0 = w.ct * 16, ej = j0 + x;
   const long MW = MODEL == GROUP_TREEFC ? H : 2L * H;
@@ -203,7 +202,7 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
         for (int k = 0; k < (MODEL == GROUP_TREEFC ? 1 : 4); k++) xw[k] = p[k * H];
       }
     }
-    if (!w.wait(a.plan, &s_bail)) return;
+    w.wait(a.plan, &s_bail);
 
     // Operand rows, one float4 per child and tile, unconditionally (a missing child reads row 0 and is
     // masked); the next tile's are on their way while a tile is multiplied.
@@ -267,6 +266,7 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
     }
     w.keep_next(r, s_rec);
     __syncthreads();
+    if (s_bail) return;
 
     float st[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, h = 0.f, cc = 0.f;  // what the backward pass wants, and the state
     if (eon) {
@@ -316,6 +316,7 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
     }
     w.advance();
   }
+  tail_leave(w.gsync, a.plan.wgs);
 }
 
 // ------------------------------------------------------------------ backward
@@ -340,7 +341,7 @@ __global__ __launch_bounds__(512, 1) void group_bwd_kernel(GroupBwdArgs a) {
   __shared__ int4 s_rec[2][2 * kGroupRows];
   __shared__ int s_bail;
   GroupWalk w;
-  if (!w.start(a.plan, s_rec)) return;
+  if (!w.start(a.plan, s_rec, &s_bail)) return;
   const int H = a.H, KG = H / 16, tid = threadIdx.x, lane = tid & 63, ks = tid >> 6;
   const int x = lane & 15, slot = lane >> 4, ej = w.ct * 16 + x;
   const int LG = MODEL == GROUP_TREELSTM ? 3 * KG : MODEL == GROUP_LSTM ? 4 * KG : KG;  // k-groups of dA's product
@@ -426,7 +427,7 @@ __global__ __launch_bounds__(512, 1) void group_bwd_kernel(GroupBwdArgs a) {
         }
       }
     }
-    if (!w.wait(a.plan, &s_bail)) return;
+    w.wait(a.plan, &s_bail);
     float pdc = 0.f;
     if (MODEL != GROUP_TREEFC && eon) pdc = ld_row(a.dc + (long)rec.x * H + ej);
 
@@ -489,6 +490,7 @@ __global__ __launch_bounds__(512, 1) void group_bwd_kernel(GroupBwdArgs a) {
     }
     w.keep_next(r, s_rec);
     __syncthreads();
+    if (s_bail) return;
 
     if (eon) {
       float v[NP];
@@ -520,6 +522,7 @@ __global__ __launch_bounds__(512, 1) void group_bwd_kernel(GroupBwdArgs a) {
     w.done();
     w.advance();
   }
+  tail_leave(w.gsync, a.plan.wgs);
 }
 
 static int group_lds(const void *kernel) {
@@ -534,7 +537,7 @@ static int group_plan(const char *who, const cavs_group_plan *p, int H, GroupPla
   CAVS_REQUIRE(p->ngroups >= 1 && p->ngroups <= cavs_group_max_groups(H) && p->spin_max >= 0 && p->extra_arrivals >= 0,
                "%s: bad plan (1..%d groups)", who, cavs_group_max_groups(H));
   *out = GroupPlan{reinterpret_cast<const int4 *>(p->groups), reinterpret_cast<const int4 *>(p->lists), reinterpret_cast<const int4 *>(p->recs),
-                   p->sync, p->ngroups, H / 16, p->spin_max, H / 16 + p->extra_arrivals};
+                   p->sync, p->ngroups, H / 16, p->spin_max, std::min(H / 16 + p->extra_arrivals, 64)};
   return CAVS_OK;
 }
 

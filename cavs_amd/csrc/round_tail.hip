@@ -15,8 +15,8 @@
 //     which is what makes an agent-scope barrier across XCDs cost as much as a launch (the
 //     invalidate alone, buffer_inv sc1, was measured at 15 us for 32 workgroups).  Groups never
 //     wait for each other;
-//   * arrival is one atomic add per workgroup and round on the group's counter in that L2; the wait
-//     polls it with a bound and gives up into a status word the host reads (every wave then leaves);
+//   * arrival is one store per workgroup and round to a word of its own in that L2; every wavefront polls
+//     all of them with a bound and gives up into a status word the host reads (every wave then leaves);
 //   * the weights never move again: a wavefront owns one eighth of K (64 k at H = 512) of its
 //     workgroup's sixteen columns, i.e. sixteen float4 of the tile-major weights, and keeps them in
 //     registers for the whole launch.  A round then fetches only its operand rows;
@@ -26,6 +26,8 @@
 // / treelstm_round_bwd_children_kernel with ROWS4): the same MFMAs on the same operands in the
 // same order, the same order of sums, the same gate function -- and a row's result does not
 // depend on which rows share its tile -- so the results equal the per-round launches' bit for bit.
+#include <algorithm>
+
 #include "round_sync.h"
 
 namespace cavs {
@@ -44,7 +46,7 @@ constexpr size_t kTailTabBytes = 5 * sizeof(int) * kTailMaxRounds * kTailRows;
 // the rest -- how many of the group's arrivals must be in before the list starts (0: none, e.g. the
 // second slice of a round that does not fit one list).
 struct TailPlan {
-  int nrounds[kTailGroups], arrivals[kTailGroups];
+  int nrounds[kTailGroups];
   int start[kTailGroups][kTailMaxRounds];
   short count[kTailGroups][kTailMaxRounds], flags[kTailGroups][kTailMaxRounds];
 };
@@ -128,8 +130,9 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_fwd_kernel(TailFwdArgs a
   float bias[4];
 #pragma unroll
   for (int k = 0; k < 4; k++) bias[k] = a.bias[k * H + ej];
-  const unsigned total = (unsigned)a.plan.arrivals[grp] * a.expect;
-  if (tid == 0 && total > 0) __hip_atomic_fetch_or(gsync + TAIL_XCC, 1u << xcc_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  unsigned arrived = 0;
+  if (tid == 0) s_bail = 0;
+  if (tid == 0) __hip_atomic_fetch_or(gsync + TAIL_XCC, 1u << xcc_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   bool first_wait = true;
   __syncthreads();
 
@@ -149,10 +152,8 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_fwd_kernel(TailFwdArgs a
       for (int k = 0; k < 4; k++) xw[k] = p[k * H];
     }
     if (need > 0) {
-      if (!tail_wait(status, gsync, (unsigned)need * a.expect, a.spin_max, first_wait, &s_bail)) return;
+      tail_wait(status, gsync, (unsigned)need, a.expect, a.spin_max, first_wait, &s_bail);
       first_wait = false;
-    } else {
-      __syncthreads();
     }
 
     // the epilogue's children
@@ -243,6 +244,7 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_fwd_kernel(TailFwdArgs a
       park(T - 1);
     }
     __syncthreads();
+    if (s_bail) return;
 
     TreeLstmCell q{};
     if (eon) {
@@ -262,7 +264,7 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_fwd_kernel(TailFwdArgs a
         a.pool[(long)e_dst * H2 + H + ej] = q.c;
       }
     }
-    if (arrives) tail_arrive(gsync, total);
+    if (arrives) tail_arrive(gsync, ct, ++arrived);
     else __syncthreads();
     if (eon) {  // what the backward pass and the caller read: on its way while the next round starts
       const long b = erow;
@@ -278,6 +280,7 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_fwd_kernel(TailFwdArgs a
       a.hlr[b * H + ej] = e_hl + e_hr;
     }
   }
+  tail_leave(gsync, H / 16);
 }
 
 // ------------------------------------------------------------------ backward
@@ -344,8 +347,9 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_bwd_kernel(TailBwdArgs a
   }
   const int ej = j0 + x;
   if (ks < 4) __builtin_amdgcn_s_setprio(2);  // (see the forward kernel)
-  const unsigned total = (unsigned)a.plan.arrivals[grp] * a.expect;
-  if (tid == 0 && total > 0) __hip_atomic_fetch_or(gsync + TAIL_XCC, 1u << xcc_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  unsigned arrived = 0;
+  if (tid == 0) s_bail = 0;
+  if (tid == 0) __hip_atomic_fetch_or(gsync + TAIL_XCC, 1u << xcc_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   bool first_wait = true;
   __syncthreads();
 
@@ -391,10 +395,8 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_bwd_kernel(TailBwdArgs a
       }
     }
     if (need > 0) {
-      if (!tail_wait(status, gsync, (unsigned)need * a.expect, a.spin_max, first_wait, &s_bail)) return;
+      tail_wait(status, gsync, (unsigned)need, a.expect, a.spin_max, first_wait, &s_bail);
       first_wait = false;
-    } else {
-      __syncthreads();
     }
     const float pdc = eon ? ld_row(a.dc + erow * H + ej) : 0.f;
 
@@ -490,6 +492,7 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_bwd_kernel(TailBwdArgs a
       park(T - 1);
     }
     __syncthreads();
+    if (s_bail) return;
 
     if (eon) {
       const float *pre = red + (ks * 8 * (NP * 4) + (lane >> 4)) * 16 + x;
@@ -516,9 +519,10 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_bwd_kernel(TailBwdArgs a
         }
       }
     }
-    if (arrives) tail_arrive(gsync, total);
+    if (arrives) tail_arrive(gsync, ct, ++arrived);
     else __syncthreads();
   }
+  tail_leave(gsync, H / 16);
 }
 
 // the barrier alone, on the footprint of the kernels above (one workgroup per CU: the LDS sees to that)
@@ -528,11 +532,15 @@ __global__ __launch_bounds__(512, 1) void tail_probe_kernel(unsigned *sync, int 
   unsigned *status = sync + TAIL_STATUS, *gsync = sync + TAIL_GROUP_WORDS * ((blockIdx.x & 7) + 1);
   red[threadIdx.x] = 0.f;
   if (threadIdx.x == 0) __hip_atomic_fetch_or(gsync + TAIL_XCC, 1u << xcc_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const unsigned total = 3u * expect;
+  if (threadIdx.x == 0) s_bail = 0;
+  __syncthreads();
   for (int r = 0; r < 3; r++) {
-    if (r > 0 && !tail_wait(status, gsync, (unsigned)r * expect, spin_max, r == 1, &s_bail)) return;
-    tail_arrive(gsync, total);
+    if (r > 0) tail_wait(status, gsync, r, expect, spin_max, r == 1, &s_bail);
+    __syncthreads();
+    if (s_bail) return;
+    tail_arrive(gsync, blockIdx.x >> 3, r + 1);
   }
+  tail_leave(gsync, expect);
 }
 
 // Copies the caller's description of the groups and checks it (host arrays: group g runs
@@ -561,10 +569,6 @@ static int tail_plan(const char *who, int ngroups, const int *nrounds, const int
       out->flags[g][i] = (short)f;
       arrived += f & 1;
     }
-    // (the last arrival of a launch clears the counter: nobody may still be waiting on it then)
-    for (int i = nrounds[g] - 1; i >= 0 && !(out->flags[g][i] & 1); i--)
-      CAVS_REQUIRE((out->flags[g][i] >> 1) == 0, "%s: group %d list %d waits, but no list from it on arrives", who, g, i);
-    out->arrivals[g] = arrived;
   }
   return any > 0 ? 1 : 0;  // 0: nothing to do
 }
@@ -609,7 +613,7 @@ int cavs_treelstm_tail_fwd(float *pool, const int *child, const int *pair, const
   CAVS_REQUIRE(!graph_out || out_rows, "cavs_treelstm_tail_fwd: graph_out needs out_rows");
   CAVS_REQUIRE(spin_max >= 0 && extra_arrivals >= 0, "cavs_treelstm_tail_fwd: bad wait bound");
   TailFwdArgs a{pool, child, pair, xW, ld_xw, Upk, bias, G, hlr, gates, msg, graph_out, out_rows, rows, sync, spin_max,
-                H / 16 + extra_arrivals, {}};
+                std::min(H / 16 + extra_arrivals, 64), {}};
   const int todo = tail_plan("cavs_treelstm_tail_fwd", ngroups, nrounds, start, count, flags, max_rounds, &a.plan);
   if (todo <= 0) return todo;
   constexpr size_t lds = kTailFwdRed * sizeof(float) + kTailTabBytes;
@@ -634,7 +638,7 @@ int cavs_treelstm_tail_bwd(float *dxW, int ld_dxw, float *dF, float *dc, const f
   CAVS_REQUIRE(aligned16(dxW) && aligned16(dF) && aligned16(UTp), "cavs_treelstm_tail_bwd: dxW, dF and UTp must be 16-byte aligned");
   CAVS_REQUIRE(spin_max >= 0 && extra_arrivals >= 0, "cavs_treelstm_tail_bwd: bad wait bound");
   TailBwdArgs a{dxW, ld_dxw, dF, dc, UTp, child_rows, gates, G, dret, dret_rows, rows, sync, leaf_rows, spin_max,
-                H / 16 + extra_arrivals, {}};
+                std::min(H / 16 + extra_arrivals, 64), {}};
   const int todo = tail_plan("cavs_treelstm_tail_bwd", ngroups, nrounds, start, count, flags, max_rounds, &a.plan);
   if (todo <= 0) return todo;
   constexpr size_t lds = kTailBwdRed * sizeof(float) + kTailTabBytes;
