@@ -54,9 +54,13 @@ __device__ inline void tail_wait(unsigned *status, unsigned *gsync, unsigned tar
 }
 
 // This workgroup waits no more (behind a barrier of its own).  The last of the group's `wgs` to say so leaves
-// the group's words as the next launch expects them.
+// the group's words as the next launch expects them: zero.  So a workgroup's own arrivals, stored by its first
+// wavefront (the last list arrives too), have to be in the L2 before it counts as gone -- one still under way
+// then would land on top of the zero, and the next launch's waits would pass early.  Stores and atomics of
+// a wavefront are not ordered by themselves: the wait (once a launch) does it.
 __device__ inline void tail_leave(unsigned *gsync, int wgs) {
   if (threadIdx.x >= 64) return;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   unsigned old = 0;
   if (threadIdx.x == 0) old = __hip_atomic_fetch_add(gsync + TAIL_LEFT, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (__builtin_amdgcn_readfirstlane(old) + 1 != (unsigned)wgs) return;
