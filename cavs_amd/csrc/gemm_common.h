@@ -81,10 +81,9 @@ __device__ inline void tile_k_range(const GemmArgs &g, int m0, int n0, int z, in
   *end = kend;
 }
 
-// Stores the TM x TN accumulators of a wavefront whose first row and column are m0 and n0; `more`: adds them
-// to what the same wavefront has stored before.
+// Stores the TM x TN accumulators of a wavefront whose first row and column are m0 and n0.
 template <int TM, int TN>
-__device__ inline void store_tile(const GemmArgs &g, const floatx16 (&acc)[TM][TN], int m0, int n0, int z, int lane, bool more) {
+__device__ inline void store_tile(const GemmArgs &g, const floatx16 (&acc)[TM][TN], int m0, int n0, int z, int lane) {
   const int khalf = lane >> 5;
   // C layout of the 32x32 accumulator: element r of lane l is row 8*(r/4) + 4*(l/32) + r%4,
   // column l%32.
@@ -95,17 +94,6 @@ __device__ inline void store_tile(const GemmArgs &g, const floatx16 (&acc)[TM][T
       const int col = n0 + 32 * j + (lane & 31);
       if (col >= g.N) continue;
       const int rbase = m0 + 32 * i + 4 * khalf;
-      if (more) {
-        float *c = g.ws ? g.ws + (long)z * g.M * g.N + col : g.C + col;
-        const long ld = g.ws ? g.N : g.ldc;
-        const float alpha = g.ws ? 1.f : g.alpha;
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int row = rbase + 8 * (r / 4) + (r % 4);
-          if (row < g.M) c[row * ld] += alpha * acc[i][j][r];
-        }
-        continue;
-      }
       // the three forms of the store are chosen once per tile (the conditions are the same
       // for every lane), not once per element
       if (g.ws) {  // split K: park the partial sum, the reduce kernel finishes the job

@@ -53,10 +53,10 @@ __global__ __launch_bounds__(kThreads, 4) void sgemm_group_kernel(GemmGroup G) {
   const int t = w % tiles, z = w / tiles;
   const int tilesN = (g.N + BN - 1) / BN, m0 = t / tilesN * BM, n0 = t % tilesN * BN;
   switch (G.form[p]) {
-    case 0: split_tile<BM, BN, BK, false, false, VEC>(g, m0, n0, z, S); break;
-    case 1: split_tile<BM, BN, BK, false, true, VEC>(g, m0, n0, z, S); break;
-    case 2: split_tile<BM, BN, BK, true, false, VEC>(g, m0, n0, z, S); break;
-    default: split_tile<BM, BN, BK, true, true, VEC>(g, m0, n0, z, S); break;
+    case 0: split_tile<BM, BN, BK, false, false, VEC, true>(g, m0, n0, z, S); break;
+    case 1: split_tile<BM, BN, BK, false, true, VEC, true>(g, m0, n0, z, S); break;
+    case 2: split_tile<BM, BN, BK, true, false, VEC, true>(g, m0, n0, z, S); break;
+    default: split_tile<BM, BN, BK, true, true, VEC, true>(g, m0, n0, z, S); break;
   }
 }
 
@@ -319,13 +319,14 @@ static GemmPlan plan_gemm(int tA, int tB, int M, int N, int K, bool skinny_allow
     }
     return p;
   };
-  // A CU holds three workgroups of the large tile; from two per CU on it is the faster one (4700 x 2048 x
+  // A CU holds two or three workgroups of the large tile; from two per CU on it is the faster one (4700 x 2048 x
   // 300, 592 tiles: 44.6 us against 49.8; 2368 rows, 304 tiles: 31.1 against 27.3).
   if (large_ok && t128 >= 2 * cus) return split(GemmPlan::TILE128, t128, 1);
-  // Fewer large tiles: K is split until about three share a CU, if that leaves each split at least 512 of K
-  // (4000 x 1024 x 3072: 150 us against 170 on the small tile).
+  // Fewer large tiles: K is split until about two share a CU -- what one holds beyond 512 of K (gemm_split.h) -- if
+  // that leaves each split at least 512 of K (4000 x 1024 x 3072: 150 us against 170 on the small tile; TN 1024 x 4096
+  // x 73000 3402 us against 3499 for three a CU, 512 x 2048 x 7088 92 against 97).
   if (large_ok && allow_split && 4 * t128 >= cus && K >= 2048) {
-    long s = (3 * cus + t128 - 1) / t128;
+    long s = (2 * cus + t128 - 1) / t128;
     // one or two more splits when they even out the workgroups per CU; ties keep the fewer splits
     // (less partial traffic)
     auto fill = [&](long sp) {
@@ -402,15 +403,15 @@ static dim3 tile_grid(GemmArgs *g, int BM, int BN, const GemmPlan &p) {
   return grid;
 }
 
-template <int BM, int BN, int BK>
+template <int BM, int BN, int BK, bool FOLD>
 static void launch_split(const GemmArgs &args, int tA, int tB, bool vec, const GemmPlan &p, hipStream_t st) {
   GemmArgs g = args;
   const dim3 grid = tile_grid(&g, BM, BN, p), block(kThreads);
 #define CAVS_GEMM_CASE(TA, TB)                                                                                \
   if (vec)                                                                                                    \
-    launch(sgemm_split_kernel<BM, BN, BK, TA, TB, true>, grid, block, t_lds_pad, st, g);                      \
+    launch(sgemm_split_kernel<BM, BN, BK, TA, TB, true, FOLD>, grid, block, t_lds_pad, st, g);                \
   else                                                                                                        \
-    launch(sgemm_split_kernel<BM, BN, BK, TA, TB, false>, grid, block, t_lds_pad, st, g)
+    launch(sgemm_split_kernel<BM, BN, BK, TA, TB, false, FOLD>, grid, block, t_lds_pad, st, g)
   if (!tA && !tB) { CAVS_GEMM_CASE(false, false); }
   else if (!tA && tB) { CAVS_GEMM_CASE(false, true); }
   else if (tA && !tB) { CAVS_GEMM_CASE(true, false); }
@@ -503,12 +504,13 @@ static int run_gemm(const char *who, int tA, int tB, int M, int N, int K, float 
   bool vec = vec_path_ok(g, tA, tB);
   if (pull) {
     const dim3 grid = tile_grid(&g, 64, 64, p), block(kThreads);
-    if (vec) launch(sgemm_split_kernel<64, 64, 16, false, false, true, true>, grid, block, 0, st, g);
-    else launch(sgemm_split_kernel<64, 64, 16, false, false, false, true>, grid, block, 0, st, g);
+    if (vec) launch(sgemm_split_kernel<64, 64, 16, false, false, true, true, true>, grid, block, 0, st, g);
+    else launch(sgemm_split_kernel<64, 64, 16, false, false, false, true, true>, grid, block, 0, st, g);
   } else if (p.kind == GemmPlan::TILE128) {
-    launch_split<128, 128, 16>(g, tA, tB, vec, p, st);
+    if (K > 2 * kSplitChain) launch_split<128, 128, 16, true>(g, tA, tB, vec, p, st);
+    else launch_split<128, 128, 16, false>(g, tA, tB, vec, p, st);
   } else {
-    launch_split<64, 64, 16>(g, tA, tB, vec, p, st);
+    launch_split<64, 64, 16, true>(g, tA, tB, vec, p, st);
   }
   CAVS_LAUNCH_CHECK();
   if (p.splits > 1) {
@@ -750,7 +752,10 @@ int cavs_sgemm_group(int count, const cavs_gemm_desc *products, void *workspace,
 
 int cavs_sgemm_group_beside(int count, const cavs_gemm_desc *products, void *workspace, size_t workspace_bytes,
                             void *stream) {
-  t_lds_pad = 10u << 10;  // with the 48 KB of a large tile's panels: two workgroups per CU
+  // With the 48 KB of a large tile's panels more than half of a CU's LDS: one workgroup to a CU.  (Two of them, at
+  // 232 registers, leave no room for the chain's wavefronts.  Training steps of chain LSTMs with a head of 10000
+  // at H = 640, 768, 1024: 2.97, 4.70, 6.03 ms against 3.16, 5.00, 6.20.)
+  t_lds_pad = 34u << 10;
   const int rc = run_group(count, products, workspace, workspace_bytes, nullptr, stream);
   t_lds_pad = 0;
   return rc;

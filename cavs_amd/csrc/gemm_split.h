@@ -3,30 +3,47 @@
 // The fp32 MFMA does 256 multiply-adds x 2 per clock and CU, the bf16 one sixteen times that.  A
 // float is exactly the sum of three bf16 numbers: h = bf16(x), m = bf16(x - h), l = x - h - m (both
 // differences are exact, eight significant bits each), so a product is the sum of nine bf16 products,
-// each of them exact in the fp32 accumulator.  The six of weight 2^-16 and above are added up; the
+// each of them exact in the fp32 accumulator.  (Splitting a number into a sum of shorter ones whose
+// products are exact: Dekker, "A floating-point technique for extending the available precision", 1971;
+// into bf16 parts for matrix units: Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial intelligence
+// datatype for higher-precision computations", 2019.)  The six of weight 2^-16 and above are added up; the
 // other three are below 2^-26 of the product, a quarter of the rounding that one fp32 addition
 // makes.  Six bf16 MFMAs take 6/16 of the matrix pipe's time for the fp32 product, and because an
 // instruction adds 16 values of k before it rounds, the sum rounds less often than the fp32 chain.
-// (Infinite operands: infinity - infinity is taken while splitting, so they give NaN.)
+//
+// What the pipe drops: it rounds a sum to nearest, but an addend of less than about an eighth of the
+// accumulator's last place is lost in it (1 + 16 x 2^-27 is 1), and the parts m and l of a long sum's
+// terms are such addends.  Where they all push one way -- constants, values on a grid -- a chain of 2048
+// of K was up to seven times further off than the fp32 pipe.  So a chain of additions ends after kSplitChain = 256
+// of K and goes into a second set of accumulators by ordinary additions; a product of up to 512 of K on
+// the large tile is one chain, which is no further off than the fp32 pipe there.  The second set costs the
+// large tile its third workgroup per CU (232 registers instead of 167) and 1 to 5 % of its rate; storing
+// and reloading C between chains instead cost 20 %.
+//
+// (Infinite operands: infinity - infinity is taken while splitting, so they give NaN.)  Parts below 2^-133
+// are no bf16 numbers: of an operand below 2^-110 bits of that weight are lost.
 //
 // A workgroup of 4 wavefronts (2 x 2) computes a BM x BN tile, BK of k at a time (two LDS buffers, one
 // barrier per step).  Operands are split on their way into LDS: row x of an operand tile is 2 BK bytes
 // per part, its 16-byte pieces permuted by x so that sixteen lanes reading the same k of sixteen rows
 // touch all 64 banks once (without it: a third of the LDS time).  While a step multiplies, the values of
 // the next one are converted and those of the one behind it are under way; the conversions (4.5
-// vector instructions a value) run in the shadow of the MFMAs of the three workgroups a CU holds.
+// vector instructions a value) run in the shadow of the MFMAs of the two or three workgroups a CU holds.
 // What bounds it is the matrix pipe at the clock it is given: bf16 MFMAs alone, from registers, sustain
 // 1.63 - 1.88 PFLOP/s here (1.75 GHz), i.e. 270 - 310 TFLOP/s of these products.
 //
 // us (TFLOP/s)                  fp32 MFMA, 128 x 128 x 16      this
-//   NN  8192 x  8192 x  8192    8277 (133)                     5685 (193)
-//   NT 73000 x  1024 x  4096    4712 (130)                     3055 (200)
-//   TN  1024 x  4096 x 73000    4791 (128)                     3655 (168)
-//   NN  7088 x 10000 x   512     617 (118)                      409 (178)
-//   NN  2368 x  2048 x   300    34.2 (85)    (64 x 64 tiles)   27.7 (105)
-//   TN   304 x  2048 x  2368    43.7 (67)                      35.8 (82)
-// Relative error against double, same rows: 1.62e-6 / 1.44e-6, 1.15e-6 / 1.00e-6, 2.79e-6 / 1.32e-6,
-// 4.1e-7 / 3.4e-7, 3.1e-7 / 2.6e-7, 3.9e-7 / 3.3e-7.
+//   NN  8192 x  8192 x  8192    8198 (134)                     5766 (191)
+//   NT 73000 x  1024 x  4096    4763 (129)                     3056 (200)
+//   TN  1024 x  4096 x 73000    4664 (131)                     3402 (180)
+//   NN  7088 x 10000 x   512     688 (105)                      407 (178)
+//   NN  2368 x  2048 x   300    34.2 (85)    (64 x 64 tiles)   27.1 (107)
+//   TN   304 x  2048 x  2368    43.2 (68)                      34.7 (85)
+// 2-norm of the error against 64 bits over that of the product, fp32 MFMA / this, 1e-7: operands from U(-1, 1),
+// from U(0, 1), and all of the form (eight bits) (1 + 2^-10 + 2^-11):
+//   NN  8192    16.2 / 2.7   11.9 / 0.8   11.8 / 1.4        NT 73000    11.5 / 2.5   8.5 / 0.7    8.4 / 1.3
+//   TN  1024    27.9 / 3.8   13.7 / 1.3   16.6 / 1.7        NN  7088     4.1 / 3.4   3.1 / 2.4    3.0 / 3.3
+//   NN  2368     3.1 / 2.2    2.6 / 1.6    2.7 / 1.6        TN   304     3.9 / 2.4   1.4 / 0.7    1.4 / 1.2
 #pragma once
 #include <type_traits>
 
@@ -181,11 +198,15 @@ struct SplitLoader {
   }
 };
 
+// K of one chain of additions on the bf16 pipe (see above)
+constexpr int kSplitChain = 256;
+
 // two buffers of three parts
 constexpr int split_lds_bytes(int BM, int BN, int BK) { return 2 * 3 * 2 * BK * (BM + BN); }
 
-// The BM x BN tile at (m0, n0) of split `z` by the calling workgroup; S: split_lds_bytes of LDS.
-template <int BM, int BN, int BK, bool TA, bool TB, bool VEC, bool PULL = false>
+// The BM x BN tile at (m0, n0) of split `z` by the calling workgroup; S: split_lds_bytes of LDS.  FOLD: chains of
+// additions end after kSplitChain of K.
+template <int BM, int BN, int BK, bool TA, bool TB, bool VEC, bool FOLD, bool PULL = false>
 __device__ __forceinline__ void split_tile(const GemmArgs &g, int m0, int n0, int z, char *__restrict__ S) {
   constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
   constexpr int PA = 2 * BK * BM, PB = 2 * BK * BN, BUF = 3 * (PA + PB);
@@ -209,9 +230,29 @@ __device__ __forceinline__ void split_tile(const GemmArgs &g, int m0, int n0, in
   lb.prepare(g.ldb, n0, g.N, tid);
   const float *A = PULL ? g.A : TA ? g.A + m0 : g.A + (long)m0 * g.lda, *B = TB ? g.B + (long)n0 * g.ldb : g.B + n0;
 
-  floatx16 acc[TM][TN];
-  int nk, whole;  // steps of the chain of additions that begins at kbeg: all, those wholly inside it
+  floatx16 acc[TM][TN], sum[FOLD ? TM : 1][FOLD ? TN : 1];
+  const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;  // steps: all, those wholly inside the range
+  const int whole = kend > kbeg ? (kend - kbeg) / BK : 0;
   const int ar = wm * WM + (lane & 31), br = wn * WN + (lane & 31), half = lane >> 5;
+  auto clear = [&](auto &v) {
+    for (auto &row : v)
+      for (floatx16 &c : row)
+#pragma unroll
+        for (int r = 0; r < 16; r++) c[r] = 0.f;
+  };
+  clear(acc);
+  clear(sum);
+  auto fold = [&] {
+    if constexpr (FOLD) {
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) sum[i][j][r] += acc[i][j][r];
+      clear(acc);
+    }
+  };
   struct Regs {
     float a[LA::NU][LA::U], b[LB::NU][LB::U];
   } r0, r1;
@@ -254,57 +295,42 @@ __device__ __forceinline__ void split_tile(const GemmArgs &g, int m0, int n0, in
   };
   // step kt multiplies what is in LDS, converts step kt + 1's values, which came while step kt - 1
   // multiplied, and asks for those of step kt + 2
-  // The bf16 pipe truncates what it adds: over a long K that is a drift the fp32 pipe does not have (1024 x
-  // 1024 x 73000 in 12 splits, error against double: 1.61e-6, with chains of 4096 1.0e-6, the fp32 pipe
-  // 1.40e-6; the two meet near K = 37000).  Long products are added up 4096 of K at a time.
-  const int last = kend, chain = g.K > 16384 ? 4096 : 16384;
-  bool more = false;
-  do {
-    kend = min(last, kbeg + chain);
-    nk = (kend - kbeg + BK - 1) / BK;
-    whole = kend > kbeg ? (kend - kbeg) / BK : 0;
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int j = 0; j < TN; j++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
-    if (nk > 0) {
-      fetch(r0, 0);
-      fetch(r1, 1);
-      put(r0, 0);
-    }
+  if (nk > 0) {
+    fetch(r0, 0);
+    fetch(r1, 1);
+    put(r0, 0);
+  }
+  __syncthreads();
+  int kt = 0;
+  for (; kt + 3 < whole; kt += 2) {  // every fetch in here is whole
+    la.template load<true>(r0.a, A, g.lda, kbeg + (kt + 2) * BK, kend);
+    lb.template load<true>(r0.b, B, g.ldb, kbeg + (kt + 2) * BK, kend);
+    multiply(kt);
+    put(r1, kt + 1);
     __syncthreads();
-    int kt = 0;
-    for (; kt + 3 < whole; kt += 2) {  // every fetch in here is whole
-      la.template load<true>(r0.a, A, g.lda, kbeg + (kt + 2) * BK, kend);
-      lb.template load<true>(r0.b, B, g.ldb, kbeg + (kt + 2) * BK, kend);
-      multiply(kt);
-      put(r1, kt + 1);
-      __syncthreads();
-      la.template load<true>(r1.a, A, g.lda, kbeg + (kt + 3) * BK, kend);
-      lb.template load<true>(r1.b, B, g.ldb, kbeg + (kt + 3) * BK, kend);
-      multiply(kt + 1);
-      put(r0, kt + 2);
-      __syncthreads();
-    }
-    for (; kt < nk; kt += 2) {
-      fetch(r0, kt + 2);
-      multiply(kt);
-      if (kt + 1 < nk) put(r1, kt + 1);
-      __syncthreads();
-      if (kt + 1 >= nk) break;
-      fetch(r1, kt + 3);
-      multiply(kt + 1);
-      if (kt + 2 < nk) put(r0, kt + 2);
-      __syncthreads();
-    }
-    int row = m0 + wm * WM, col = n0 + wn * WN, l = lane;
-    asm volatile("" : "+v"(row), "+v"(col), "+v"(l));  // (or the addresses of the stores are kept through the loops above)
-    store_tile<TM, TN>(g, acc, row, col, z, l, more);
-    more = true;
-    kbeg = kend;
-  } while (kbeg < last);
+    la.template load<true>(r1.a, A, g.lda, kbeg + (kt + 3) * BK, kend);
+    lb.template load<true>(r1.b, B, g.ldb, kbeg + (kt + 3) * BK, kend);
+    multiply(kt + 1);
+    put(r0, kt + 2);
+    if (FOLD && (kt + 2) % (kSplitChain / BK) == 0) fold();
+    __syncthreads();
+  }
+  for (; kt < nk; kt += 2) {
+    fetch(r0, kt + 2);
+    multiply(kt);
+    if (kt + 1 < nk) put(r1, kt + 1);
+    __syncthreads();
+    if (kt + 1 >= nk) break;
+    fetch(r1, kt + 3);
+    multiply(kt + 1);
+    if (kt + 2 < nk) put(r0, kt + 2);
+    __syncthreads();
+  }
+  fold();
+  int row = m0 + wm * WM, col = n0 + wn * WN, l = lane;
+  asm volatile("" : "+v"(row), "+v"(col), "+v"(l));  // (or the addresses of the stores are kept through the loops above)
+  if constexpr (FOLD) store_tile<TM, TN>(g, sum, row, col, z, l);
+  else store_tile<TM, TN>(g, acc, row, col, z, l);
 }
 
 // Tile `t` of a launch over row tiles [row0, row0 + rows): eight row tiles at a time, down each column
@@ -316,8 +342,8 @@ __device__ inline void split_tile_at(int t, int row0, int rows, int tilesN, int 
   *tn = in / high;
 }
 
-template <int BM, int BN, int BK, bool TA, bool TB, bool VEC, bool PULL = false>
-__global__ __launch_bounds__(kThreads, 3) void sgemm_split_kernel(GemmArgs g) {
+template <int BM, int BN, int BK, bool TA, bool TB, bool VEC, bool FOLD, bool PULL = false>
+__global__ __launch_bounds__(kThreads, BM == 128 && FOLD ? 2 : 3) void sgemm_split_kernel(GemmArgs g) {
   __shared__ __attribute__((aligned(16))) char S[split_lds_bytes(BM, BN, BK)];
   apply_live(g, TA, gridDim.y);
   const int tilesN = (g.N + BN - 1) / BN, tilesM = (g.M + BM - 1) / BM;
@@ -348,7 +374,7 @@ __global__ __launch_bounds__(kThreads, 3) void sgemm_split_kernel(GemmArgs g) {
   }
   int tm, tn;
   split_tile_at(t, row0, rows, tilesN, &tm, &tn);
-  split_tile<BM, BN, BK, TA, TB, VEC, PULL>(g, tm * BM, tn * BN, blockIdx.y, S);
+  split_tile<BM, BN, BK, TA, TB, VEC, FOLD, PULL>(g, tm * BM, tn * BN, blockIdx.y, S);
 }
 
 }  // namespace cavs

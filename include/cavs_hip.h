@@ -210,8 +210,8 @@ int cavs_sgemm_group(int count, const cavs_gemm_desc *products, void *workspace,
 /* cavs_sgemm_group for a caller that enqueues the products on a second stream beside a chain of short
  * dependent launches (the weight gradient of a wide classifier head under the backward rounds,
  * cavs/midend/statement.cc:106-111): the tile launches of products that run alone ask for LDS they do
- * not use, so that at most two of their workgroups share a CU and the chain's workgroups find room
- * on every CU.  Same results. */
+ * not use, so that a CU holds one of their workgroups and the chain's find room on every CU.  Same
+ * results. */
 int cavs_sgemm_group_beside(int count, const cavs_gemm_desc *products, void *workspace, size_t workspace_bytes,
                             void *stream);
 /* cavs_sgemm_group followed by cavs_embed_bwd(dtable, ids, C_k, ldc_k, M_k, N_k) on the result of

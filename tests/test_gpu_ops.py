@@ -1794,6 +1794,38 @@ def test_sgemm_keeps_every_bit_of_its_operands(g, tA, tB, M, N, K, ld):
     assert np.abs(g.host(Cd) - exact).max() <= 2.0 ** -24 * (K + 16)
 
 
+def _on_grid(r, n, low):
+    """Values of eight significant bits times 1 + low: what lies below the first eight bits has one sign."""
+    x = (0.5 + r.bulk_uniform(n)).astype(np.float32)
+    return ((x.view(np.int32) & ~0xffff).view(np.float32) * np.float32(1 + low)).astype(np.float32)
+
+
+@pytest.mark.parametrize("tA,tB,M,N,K", [(0, 1, 200, 300, 512), (0, 0, 64, 4096, 2048), (1, 0, 72, 260, 20000), (0, 1, 1100, 8200, 513), (0, 1, 1088, 8192, 2064),
+                                         (1, 0, 1088, 8192, 4100)])
+def test_sums_of_one_sign_are_no_worse_than_a_chain_of_fp32_additions(g, tA, tB, M, N, K):
+    """Operands all of whose low bits push the same way, and constants: a sum that drops what is small beside it drifts
+    here.  The bar is a chain of K fp32 additions, each off by at most half a unit in the last place of the running sum
+    (a k-th of the way to the end: k / K of it), with nothing but chance in the signs."""
+    import torch
+
+    r = rng(M + N + K)
+    draws = dict(positive=lambda n: r.bulk_uniform(n).astype(np.float32), third=lambda n: np.full(n, 1 / 3, np.float32),
+                 ones=lambda n: np.ones(n, np.float32), grid10=lambda n: _on_grid(r, n, 2.0 ** -10 + 2.0 ** -11),
+                 grid18=lambda n: _on_grid(r, n, 2.0 ** -18 + 2.0 ** -19))
+    bar = 2.0 ** -24 * np.sqrt(K / 3)
+    for a, b in (("positive", "positive"), ("third", "positive"), ("grid10", "ones"), ("grid10", "grid10"), ("grid18", "grid18")):
+        A, B = draws[a](M * K).reshape((K, M) if tA else (M, K)), draws[b](K * N).reshape((N, K) if tB else (K, N))
+        Ad, Bd, Cd = g.devf(A), g.devf(B), g.zeros(M, N, fill=float("nan"))
+        g.call("cavs_sgemm", tA, tB, M, N, K, 1.0, g.P(Ad), A.shape[1], g.P(Bd), B.shape[1], 0.0, g.P(Cd), N, g.stream())
+        exact = (Ad.double().t() if tA else Ad.double()) @ (Bd.double().t() if tB else Bd.double())
+        err = float((Cd.double() - exact).norm() / exact.norm())
+        print(f"{a} x {b}: {err:.2e} of {bar:.2e}", flush=True)
+        assert err <= bar, (a, b)
+        del exact
+        g.release()
+        torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("n,V,E,w,leaf_rows", [(1, 5, 8, 4, 1), (63, 4, 12, 260, 40), (64, 255, 4, 256, 0), (65, 256, 20, 8, 65), (2368, 21701, 300, 512, 1216),
                                                (4096, 70000, 8, 12, 100), (4097, 65535, 8, 300, 4000), (9000, 300, 16, 64, 5000), (16384, 1000, 8, 16, 9000),
                                                (16385, 1000, 8, 16, 9000)])
