@@ -20,7 +20,9 @@
 // large tile its third workgroup per CU (232 registers instead of 167) and 1 to 5 % of its rate; storing
 // and reloading C between chains instead cost 20 %.
 //
-// (Infinite operands: infinity - infinity is taken while splitting, so they give NaN.)  Parts below 2^-133
+// An infinite operand (infinity - infinity while splitting) or a finite one whose h rounds to infinity makes
+// NaN; so do NaN operands.  A wavefront whose results are not all finite computes them again on the fp32 MFMA
+// (unsplit_tile): 8192^3 with a NaN in every row takes 26 ms, with one 17, without 6.  Parts below 2^-133
 // are no bf16 numbers: of an operand below 2^-110 bits of that weight are lost.
 //
 // A workgroup of 4 wavefronts (2 x 2) computes a BM x BN tile, BK of k at a time (two LDS buffers, one
@@ -201,6 +203,59 @@ struct SplitLoader {
 // K of one chain of additions on the bf16 pipe (see above)
 constexpr int kSplitChain = 256;
 
+// What the fp32 pipe makes of a wavefront's TM x TN tiles over [kbeg, kend): the operands as they are, straight
+// from memory.  Only for results that came out infinite or NaN (split_tile).
+template <int TM, int TN, bool TA, bool TB, bool PULL>
+__device__ inline void unsplit_tile(const GemmArgs &g, int row, int col, int kbeg, int kend, int lane, floatx16 (&acc)[TM][TN]) {
+  const int x = lane & 31, half = lane >> 5;
+  const float *pa[TM], *pb[TN];
+  bool on[TM];
+#pragma unroll
+  for (int i = 0; i < TM; i++) {
+    const int m = min(row + 32 * i + x, g.M - 1);
+    on[i] = true;
+    if constexpr (PULL) {
+      const long off = (long)(int)(g.pull_x[g.pull_rows[m]] * (float)g.K);
+      on[i] = off >= 0;
+      pa[i] = g.A + (on[i] ? off : 0);
+    } else {
+      pa[i] = TA ? g.A + m : g.A + (long)m * g.lda;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < TN; j++) {
+    const int n = min(col + 32 * j + x, g.N - 1);
+    pb[j] = TB ? g.B + (long)n * g.ldb : g.B + n;
+  }
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+  constexpr int U = 8;  // pairs of k in flight
+  for (int k0 = kbeg; k0 < kend; k0 += 2 * U) {
+    float a[U][TM], b[U][TN];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int k = k0 + 2 * u + half, kc = min(k, kend - 1);
+#pragma unroll
+      for (int i = 0; i < TM; i++) a[u][i] = pa[i][TA ? (long)kc * g.lda : kc];
+#pragma unroll
+      for (int j = 0; j < TN; j++) b[u][j] = pb[j][TB ? kc : (long)kc * g.ldb];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const bool in = k0 + 2 * u + half < kend;
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(in && on[i] ? a[u][i] : 0.f, in ? b[u][j] : 0.f, acc[i][j], 0, 0, 0);
+    }
+  }
+}
+
 // two buffers of three parts
 constexpr int split_lds_bytes(int BM, int BN, int BK) { return 2 * 3 * 2 * BK * (BM + BN); }
 
@@ -329,8 +384,21 @@ __device__ __forceinline__ void split_tile(const GemmArgs &g, int m0, int n0, in
   fold();
   int row = m0 + wm * WM, col = n0 + wn * WN, l = lane;
   asm volatile("" : "+v"(row), "+v"(col), "+v"(l));  // (or the addresses of the stores are kept through the loops above)
-  if constexpr (FOLD) store_tile<TM, TN>(g, sum, row, col, z, l);
-  else store_tile<TM, TN>(g, acc, row, col, z, l);
+  auto finish = [&](floatx16 (&out)[TM][TN]) {
+    // An infinite operand, or a finite one whose first part rounds to infinity (beyond 3.39e38), leaves
+    // infinity - infinity in its parts and so NaN here, whatever the product is: the fp32 pipe decides then.
+    float odd = 0.f;  // (0 times a finite number; NaN if one is not)
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) odd = fmaf(out[i][j][r], 0.f, odd);
+    if (__any(!(odd == 0.f))) unsplit_tile<TM, TN, TA, TB, PULL>(g, row, col, kbeg, kend, l, out);
+    store_tile<TM, TN>(g, out, row, col, z, l);
+  };
+  if constexpr (FOLD) finish(sum);
+  else finish(acc);
 }
 
 // Tile `t` of a launch over row tiles [row0, row0 + rows): eight row tiles at a time, down each column

@@ -1826,6 +1826,39 @@ def test_sums_of_one_sign_are_no_worse_than_a_chain_of_fp32_additions(g, tA, tB,
         torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("tA,tB,M,N,K", [(0, 0, 200, 70, 44), (0, 1, 130, 200, 100), (1, 0, 70, 90, 900), (1, 1, 66, 300, 33), (0, 0, 1100, 8200, 40),
+                                         (0, 1, 1100, 8192, 530), (1, 0, 1090, 8192, 48)])
+def test_products_of_infinite_and_very_large_operands(g, tA, tB, M, N, K):
+    """An infinity times a finite number stays one, two of opposite sign and an infinity times zero are NaN, and finite
+    operands up to the largest float (whose first bf16 part is infinite) give their finite product."""
+    import torch
+
+    r = rng(M + N + K)
+    big = np.float32(np.finfo(np.float32).max)
+    A, B = (0.25 + r.bulk_uniform(M * K).reshape(M, K)).astype(np.float32), (0.25 + r.bulk_uniform(K * N).reshape(K, N)).astype(np.float32)
+    A[3, 5] = np.inf            # a row of infinities
+    A[40, [0, K - 1]] = np.inf, -np.inf  # of NaN
+    A[M - 1, K - 1] = -np.inf
+    B[7, N - 2] = np.inf        # a column of them
+    B[K - 1, 11] = np.nan
+    A[50, :] = 0.0
+    A[50, 2] = big
+    B[2, 3] = 2.0 ** -100       # big times this is a number
+    B[2, 4], B[2, 12] = 4.0, 0.0
+    A[60, 7] = 0.0              # and zero times the infinity of B's column is not
+    Ad, Bd, Cd = g.devf(A.T if tA else A), g.devf(B.T if tB else B), g.zeros(M, N, fill=3.0)
+    g.call("cavs_sgemm", tA, tB, M, N, K, 1.0, g.P(Ad), Ad.shape[1], g.P(Bd), Bd.shape[1], 0.0, g.P(Cd), N, g.stream())
+    got = g.host(Cd).astype(np.float64)
+    with np.errstate(all="ignore"):
+        want = (torch.from_numpy(A).double() @ torch.from_numpy(B).double()).numpy()
+        want = np.where(np.abs(want) > float(big), np.sign(want) * np.inf, want)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.where(np.isinf(got), got, 0), np.where(np.isinf(want), want, 0))
+    ok = np.isfinite(want)
+    assert np.isinf(want).sum() > M and np.isnan(want).sum() > N and ok.sum() > M * N // 2
+    np.testing.assert_allclose(got[ok], want[ok], rtol=2.0 ** -24 * (K + 4))
+
+
 @pytest.mark.parametrize("n,V,E,w,leaf_rows", [(1, 5, 8, 4, 1), (63, 4, 12, 260, 40), (64, 255, 4, 256, 0), (65, 256, 20, 8, 65), (2368, 21701, 300, 512, 1216),
                                                (4096, 70000, 8, 12, 100), (4097, 65535, 8, 300, 4000), (9000, 300, 16, 64, 5000), (16384, 1000, 8, 16, 9000),
                                                (16385, 1000, 8, 16, 9000)])
