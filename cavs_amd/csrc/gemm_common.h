@@ -41,7 +41,10 @@ struct GemmArgs {
   // tiles would finish early and the others set the time as before
   int zseg = 0;
   const int *live = nullptr;  // cavs_gemm_desc::live
+  int pad_block = 0, pad_used = 0;  // cavs_gemm_desc::pad_block, pad_used
 };
+
+__device__ inline bool padding_column(const GemmArgs &g, int col) { return g.pad_block > 0 && col % g.pad_block >= g.pad_used; }
 
 // The sizes a launch with `live` runs at: rows of C (TA = false) or K (TA = true), the known block's rows.
 __device__ inline void apply_live(GemmArgs &g, bool TA, int splits) {

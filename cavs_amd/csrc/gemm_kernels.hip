@@ -280,7 +280,7 @@ __global__ __launch_bounds__(W * 64) void sgemm_skinny_kernel(GemmArgs g) {
     const int l2 = e & 63, r = (e >> 6) & 15, t = e >> 10;
     const int row = m0 + 32 * t + 8 * (r / 4) + 4 * (l2 >> 5) + (r % 4), col = n0 + (l2 & 31);
     if (row >= g.M || col >= g.N) continue;
-    float v = g.alpha * red[e];
+    float v = padding_column(g, col) ? 0.f : g.alpha * red[e];
     if (g.beta != 0.f) v += g.beta * g.C[row * g.ldc + col];
     if (g.D) v += g.D[(long)(row >> g.dshift) * g.ldd + col];
     g.C[row * g.ldc + col] = v;
@@ -469,10 +469,15 @@ struct BlockHint {
   }
 };
 
+// cavs_gemm_desc::pad_block, pad_used
+struct Padding {
+  int block = 0, used = 0;
+};
+
 static int run_gemm(const char *who, int tA, int tB, int M, int N, int K, float alpha, const float *A,
                     int lda, const float *B, int ldb, float beta, float *C, int ldc, const float *D,
                     int ldd, int dshift, void *ws, size_t ws_bytes, void *stream, const PullRows *pull = nullptr,
-                    const BlockHint *hint = nullptr, const int *live = nullptr, int live_expect = 0) {
+                    const BlockHint *hint = nullptr, const int *live = nullptr, int live_expect = 0, Padding pad = {}) {
   int rc = check_gemm(who, tA, tB, M, N, K, A, lda, B, ldb, C, ldc);
   if (rc || M == 0 || N == 0) return rc;
   // Looked-up rows: up to 128 of them the skinny kernel, beyond it the 64 x 64 tiles (M x 2048 x 300..512: 21
@@ -483,6 +488,8 @@ static int run_gemm(const char *who, int tA, int tB, int M, int N, int K, float 
   hipStream_t st = as_stream(stream);
   GemmArgs g{M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, D, ldd, dshift, p.kchunk, nullptr};
   g.live = live;
+  g.pad_block = pad.block;
+  g.pad_used = pad.used;
   if (hint) hint->set(&g, tA, tB, beta == 0.f && !D);
   if (pull) {
     g.pull_rows = pull->rows;
@@ -558,6 +565,7 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
       if (rc) return rc;
     }
     CAVS_REQUIRE(q.M >= 0 && q.N >= 0 && q.K >= 0, "cavs_sgemm_group: negative dimension in product %d", p);
+    CAVS_REQUIRE(q.pad_block >= 0 && q.pad_used >= 0, "cavs_sgemm_group: bad padding in product %d (block %d, used %d)", p, q.pad_block, q.pad_used);
     CAVS_REQUIRE(q.zero_kind >= 0 && q.zero_kind <= CAVS_GEMM_B_ZERO && q.zero_rows >= 0 && q.zero_col >= 0,
                  "cavs_sgemm_group: bad block hint in product %d (kind %d, rows %d, col %d)", p, q.zero_kind, q.zero_rows, q.zero_col);
     tiles[p] = (long)((q.M + 63) / 64) * ((q.N + 63) / 64);
@@ -612,6 +620,8 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
     int splits = K > 0 ? (K + kchunk - 1) / kchunk : 1;
     GemmArgs g{q.M, q.N, q.K, q.A, q.lda, q.B, q.ldb, q.C, q.ldc, q.alpha, q.beta, nullptr, 0, 0, kchunk, nullptr};
     g.live = q.live;
+    g.pad_block = q.pad_block;
+    g.pad_used = q.pad_used;
     BlockHint{q.zero_kind, q.live ? 1 : q.zero_rows, q.zero_col}.set(&g, q.transA, q.transB, q.beta == 0.f);
     if (splits > 1) {
       if (ws) g.ws = reinterpret_cast<float *>(static_cast<char *>(ws) + need);
@@ -654,7 +664,7 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
     if (q.M == 0 || q.N == 0 || !alone[p]) continue;
     const BlockHint hint{q.zero_kind, q.live ? 1 : q.zero_rows, q.zero_col};
     int rc = run_gemm("cavs_sgemm_group", q.transA, q.transB, q.M, q.N, q.K, q.alpha, q.A, q.lda, q.B, q.ldb, q.beta,
-                      q.C, q.ldc, nullptr, 0, 0, ws, ws_bytes, stream, nullptr, &hint, q.live, q.live_expect);
+                      q.C, q.ldc, nullptr, 0, 0, ws, ws_bytes, stream, nullptr, &hint, q.live, q.live_expect, {q.pad_block, q.pad_used});
     if (rc) return rc;
   }
   hipStream_t st = as_stream(stream);
@@ -770,7 +780,14 @@ int cavs_sgemm_group_embed_bwd(int count, const cavs_gemm_desc *products, int em
 int cavs_embed_pull_sgemm(float *C, int ldc, float *e_out, int ld_e, float *ids_out, const float *x, const int *rows,
                           const float *table, int n, int E, const float *B, int ldb, int N, int unused_rows, int unused_col,
                           void *stream) {
+  return cavs_embed_pull_sgemm_padded(C, ldc, e_out, ld_e, ids_out, x, rows, table, n, E, B, ldb, N, unused_rows, unused_col, 0, 0, stream);
+}
+
+int cavs_embed_pull_sgemm_padded(float *C, int ldc, float *e_out, int ld_e, float *ids_out, const float *x, const int *rows,
+                                 const float *table, int n, int E, const float *B, int ldb, int N, int unused_rows, int unused_col,
+                                 int pad_block, int pad_used, void *stream) {
   CAVS_REQUIRE(n >= 0 && E > 0 && N >= 0 && ld_e >= E, "cavs_embed_pull_sgemm: bad shape n=%d E=%d N=%d ld_e=%d", n, E, N, ld_e);
+  CAVS_REQUIRE(pad_block >= 0 && pad_used >= 0, "cavs_embed_pull_sgemm: bad padding (block %d, used %d)", pad_block, pad_used);
   CAVS_REQUIRE(unused_rows >= 0 && unused_col >= 0, "cavs_embed_pull_sgemm: bad unused block (rows %d, col %d)", unused_rows, unused_col);
   const BlockHint hint{CAVS_GEMM_C_UNUSED, unused_rows, unused_col};
   if (n == 0) return CAVS_OK;
@@ -783,11 +800,11 @@ int cavs_embed_pull_sgemm(float *C, int ldc, float *e_out, int ld_e, float *ids_
     int rc = cavs_embed_pull_fwd(e_out, ld_e, ids_out, x, rows, table, n, E, stream);
     if (rc || N == 0) return rc;
     return run_gemm("cavs_embed_pull_sgemm", 0, 0, n, N, E, 1.f, e_out, ld_e, B, ldb, 0.f, C, ldc, nullptr, 0, 0, nullptr, 0, stream,
-                    nullptr, &hint);
+                    nullptr, &hint, nullptr, 0, {pad_block, pad_used});
   }
   const PullRows pull{rows, x, e_out, ld_e, ids_out};
   return run_gemm("cavs_embed_pull_sgemm", 0, 0, n, N, E, 1.f, table, E, B, ldb, 0.f, C, ldc, nullptr, 0, 0, nullptr, 0, stream, &pull,
-                  &hint);
+                  &hint, nullptr, 0, {pad_block, pad_used});
 }
 
 int cavs_sgemm(int transA, int transB, int M, int N, int K, float alpha, const float *A, int lda,

@@ -254,6 +254,13 @@ __device__ inline void unsplit_tile(const GemmArgs &g, int row, int col, int kbe
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(in && on[i] ? a[u][i] : 0.f, in ? b[u][j] : 0.f, acc[i][j], 0, 0, 0);
     }
   }
+#pragma unroll
+  for (int j = 0; j < TN; j++)
+    if (padding_column(g, col + 32 * j + x))
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
 }
 
 // two buffers of three parts

@@ -39,7 +39,8 @@ class GemmDesc(C.Structure):
     """cavs_gemm_desc: one product of cavs_sgemm_group"""
     _fields_ = [("transA", _I), ("transB", _I), ("M", _I), ("N", _I), ("K", _I), ("alpha", _F), ("beta", _F),
                 ("A", _P), ("lda", _I), ("B", _P), ("ldb", _I), ("C", _P), ("ldc", _I),
-                ("zero_kind", _I), ("zero_rows", _I), ("zero_col", _I), ("live", _P), ("live_expect", _I)]
+                ("zero_kind", _I), ("zero_rows", _I), ("zero_col", _I), ("live", _P), ("live_expect", _I),
+                ("pad_block", _I), ("pad_used", _I)]
 
 
 class BlockCopy(C.Structure):
@@ -99,6 +100,7 @@ _SIGS = {
     "cavs_embed_fwd": [_P, _I, _P, _P, _I, _I, _P],
     "cavs_embed_pull_fwd": [_P, _I, _P, _P, _P, _P, _I, _I, _P],
     "cavs_embed_pull_sgemm": [_P, _I, _P, _I, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _I, _P],
+    "cavs_embed_pull_sgemm_padded": [_P, _I, _P, _I, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _I, _I, _I, _P],
     "cavs_embed_index": [_P, _P, _P, _P, _I, _I, _I, _P, _Z, _P],
     "cavs_embed_words": [_P, _I, _P, _P, _I, _I, _P],
     "cavs_embed_words_bwd": [_P, _P, _P, _I, _I, _I, _P],

@@ -112,7 +112,8 @@ Engine::Engine(const cavs_session_config &cfg, void *external_stream, std::share
 // multiple (cfg_.H, E_; the declared ones stay in uH_, uE_).  A padding column stays zero: its weights
 // and biases are zero, so u = tanh(0) = 0, c = i u + f c' = 0 and h = o tanh(c) = 0, and with d h = 0
 // from the head and from the rounds above every gate gradient and every weight gradient of the
-// column is a product with a zero.  Without it such a size runs a round as six to ten separate launches
+// column is a product with a zero.  (An infinite embedding times the zero weights would be a NaN: the product x W
+// is told which columns are padding and leaves zeros there; the rows every other product reads are bounded.)  Without it such a size runs a round as six to ten separate launches
 // (Tree-LSTM, H = 150, 25 trees: 0.78 ms per step, 0.24 padded).
 // A caller's own tensors (bind_param) keep their layout: they are copied block by block into the stored
 // one when a forward pass begins, and the gradients back when a backward pass ends; the embedding
@@ -704,7 +705,7 @@ void Engine::words_forward(const float *W, int w, int leaf_w) {
     check(cavs_embed_words(e_.get(), ld_e_, d_words_index_, param("Emb").w, N, E_, stream_));
   }
   gemm_group({{0, 0, N, w, E_, 1.f, 0.f, e_.get(), ld_e_, W, w, xW_words_.get(), w, lp > 0 ? CAVS_GEMM_C_UNUSED : 0, lp, leaf_w, d_words_index_,
-               words_expected()}});
+               words_expected(), pad_block(), uH_}});
   ProfScope ps(this, K_GATHER);
   check(cavs_spread_rows(xW_.get(), w, xW_words_.get(), w, d_words_index_, N, w, lp, leaf_w, ids, xs_.get(), stream_));
   c_launches_ += 3;
@@ -1474,8 +1475,8 @@ void Engine::treelstm_forward() {
   } else {  // Pull of the word id, the lookup and x * W: one launch
     ProfScope ps(this, K_GEMM);
     // (a leaf gathers zero rows, so its forget gates multiply zero: their columns of x * W are not wanted)
-    check(cavs_embed_pull_sgemm(xW_.get(), 4 * H, e_.get(), ld_e_, xs_.get(), d_x_, d_t2j_, param("Emb").w, N, E, W, 4 * H, 4 * H,
-                                sched_->leaf_prefix, 3 * H, stream_));
+    check(cavs_embed_pull_sgemm_padded(xW_.get(), 4 * H, e_.get(), ld_e_, xs_.get(), d_x_, d_t2j_, param("Emb").w, N, E, W, 4 * H, 4 * H,
+                                       sched_->leaf_prefix, 3 * H, pad_block(), uH_, stream_));
     c_gemm_flops_ += 2.0 * N * 4 * H * E;
     c_gemm_flops_hinted_ += 2.0 * sched_->leaf_prefix * H * E;
     c_launches_ += 1;
@@ -1888,8 +1889,8 @@ void Engine::lstm_forward() {
     words_forward(Wx, 4 * H, 4 * H);
   } else {  // Pull of the token id, the lookup and x * W_x: one launch
     ProfScope ps(this, K_GEMM);
-    check(cavs_embed_pull_sgemm(xW_.get(), 4 * H, e_.get(), E, xs_.get(), d_x_, d_t2j_, param("Emb").w, N, E, Wx, 4 * H, 4 * H, 0, 0,
-                                stream_));
+    check(cavs_embed_pull_sgemm_padded(xW_.get(), 4 * H, e_.get(), E, xs_.get(), d_x_, d_t2j_, param("Emb").w, N, E, Wx, 4 * H, 4 * H, 0, 0,
+                                       pad_block(), uH_, stream_));
     c_gemm_flops_ += 2.0 * N * 4 * H * E;
     c_launches_ += 1;
   }

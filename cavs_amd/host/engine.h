@@ -413,6 +413,7 @@ class Engine {
   bool trains_ = true;  // a backward pass follows
   const int *d_words_index_ = nullptr;
   DeviceArray<float> xW_words_, d_words_, word_parts_;
+  int pad_block() const { return uH_ != cfg_.H ? cfg_.H : 0; }  // padding of x * W (cavs_gemm_desc::pad_block, uH_ used)
   bool words_wanted(bool beside) const;
   int words_expected() const;
   void words_index(int leaf_rows);

@@ -202,6 +202,10 @@ typedef struct cavs_gemm_desc {
    * live_expect: the caller's guess of live[0], which only the plan reads.  Null: all of them. */
   const int *live;
   int live_expect;
+  /* Optional: the columns of C come in blocks of pad_block, of which only the first pad_used are anything
+   * but padding (B is zero in the others).  Padding comes out as zero whatever A holds, also
+   * where an infinity or a NaN of A meets the zeros.  0: none. */
+  int pad_block, pad_used;
 } cavs_gemm_desc;
 enum { CAVS_GEMM_C_UNUSED = 1, CAVS_GEMM_A_ZERO = 2, CAVS_GEMM_B_ZERO = 3 };
 size_t cavs_sgemm_group_workspace(int count, const cavs_gemm_desc *products);
@@ -256,6 +260,10 @@ int cavs_embed_pull_fwd(float *out, int ld_out, float *ids_out, const float *x, 
 int cavs_embed_pull_sgemm(float *C, int ldc, float *e_out, int ld_e, float *ids_out, const float *x,
                           const int *rows, const float *table, int n, int E, const float *B, int ldb,
                           int N, int unused_rows, int unused_col, void *stream);
+/* The same with columns that are padding (cavs_gemm_desc::pad_block, pad_used). */
+int cavs_embed_pull_sgemm_padded(float *C, int ldc, float *e_out, int ld_e, float *ids_out, const float *x,
+                                 const int *rows, const float *table, int n, int E, const float *B, int ldb,
+                                 int N, int unused_rows, int unused_col, int pad_block, int pad_used, void *stream);
 /* The words of a batch, each once, so that what depends on the word alone is done once per word
  * (cavs/backend/op_impl_embedding_lookup.cu:37-148 looks a row up, and adds a gradient row, per vertex).
  * cavs_embed_index: ids_out[b] = x[rows[b]] for b < n, and in `index` (cavs_embed_index_ints(n) ints)

@@ -705,3 +705,38 @@ def test_sizes_that_are_no_multiple_of_a_tile(oracle, model, loss, kw, H, E):
             p[k[1:]] = (p[k[1:]].ravel() - lr * np.asarray(v, np.float32).ravel()).reshape(p[k[1:]].shape)
             close(s.param(k[1:], p[k[1:]].shape), p[k[1:]], k[1:])
     s.close()
+
+
+@pytest.mark.parametrize("model,H,E,B", [("treelstm", 150, 60, 2), ("treelstm", 100, 64, 25), ("treelstm", 70, 300, 90), ("treelstm", 200, 2048, 90), ("lstm", 50, 50, 3), ("lstm", 200, 200, 40),
+                                         ("lstm", 72, 72, 160)])
+def test_an_infinite_embedding_saturates_gates_and_nothing_else_at_sizes_stored_with_padding(model, H, E, B):
+    """Hidden sizes that are stored in whole tiles: an infinity in a looked-up row saturates the gates of its vertex, as it
+    does where sizes are stored as declared (fused_round_rows < 0), and makes no NaN in the padding.  The batches take
+    the three ways x * W is computed: a few rows, hundreds, by words."""
+    V, rng = 500, synth.SplitMix64(H + B)
+    r = 2.0 / np.sqrt(H)
+    u = lambda *s: rng.bulk_uniform(int(np.prod(s)), -r, r).reshape(s).astype(np.float32)  # noqa: E731
+    Emb = u(V, E)
+    Emb[7, 1], Emb[8, 0] = np.inf, -np.inf
+    if model == "treelstm":
+        trees = [synth.random_binary_tree(rng, rng.randint(8, 24)) for _ in range(B)]
+        graph, sizes = synth.pack_graph(trees, 47), [len(t) for t in trees]
+        params = dict(Emb=Emb, W=u(E, 4 * H), U=u(4 * H * H), Bv=u(4 * H))
+    else:
+        sizes = [rng.randint(4, 30) for _ in range(B)]
+        graph = synth.pack_graph([synth.chain(n) for n in sizes], 30)
+        params = dict(Emb=Emb, W=u(8 * H * H), Bv=u(4 * H))
+    params.update(Wfc=u(5, H), bfc=u(5))
+    N = sum(sizes)
+    x, labels = np.floor(rng.bulk_uniform(N) * V).astype(np.float32), np.floor(rng.bulk_uniform(N) * 5).astype(np.float32)
+    x[::9], x[4::11] = 7.0, 8.0
+    out = []
+    for rows in (0, -1):
+        s = session.Session(model, H=H, E=E, V=V, C_=5, fused_round_rows=rows)
+        s.set_params(params)
+        s.step(graph, x, labels, backward=False)
+        out.append((s.fetch("graph_out"), s.fetch("loss")))
+        s.close()
+    assert np.isfinite(out[1][0]).all() and np.isfinite(out[1][1]).all()
+    close(out[0][0], out[1][0].astype(np.float64), "graph_out")
+    close(out[0][1], out[1][1].astype(np.float64), "loss")
