@@ -2535,7 +2535,9 @@ void Engine::head_forward_backward(bool backward) {
         gemm_group({dGd});
         check(cavs_event_record(aux_fork_ev_, stream_));
         check(cavs_stream_wait_event(aux_stream_, aux_fork_ev_));
-        check(cavs_sgemm_group_beside(1, &dWd, ws_aux_.get(), ws_aux_.capacity() * 4, aux_stream_));
+        // (beside the resident launch, one workgroup to a CU with 86 KB of its LDS, plain workgroups find room; with
+        // more LDS they would come after it: C4 2.71 and 2.93 ms)
+        check((group_.first >= 0 ? cavs_sgemm_group : cavs_sgemm_group_beside)(1, &dWd, ws_aux_.get(), ws_aux_.capacity() * 4, aux_stream_));
         c_gemm_flops_ += 2.0 * dWd.M * dWd.N * dWd.K;
         c_launches_ += 1;
         bias_gradient("bfc", dlogits_.get(), N, C, head_bias_parts_, aux_stream_);
