@@ -34,6 +34,7 @@ struct GroupPlan {
   const int4 *recs;    // [*][2]
   unsigned *sync;
   int ngroups, wgs, spin_max, expect;
+  bool whole_lines;  // of the rows the launch writes and reads (ld_row)
 };
 
 template <int I, int N, class F>
@@ -89,7 +90,7 @@ struct GroupWalk {
   // sets *s_bail, looked at behind the barrier that completes the partial sums)
   __device__ inline void wait(const GroupPlan &p, int *s_bail) {
     if (cur.z <= 0) return;
-    tail_wait(status, gsync, (unsigned)cur.z, p.expect, p.spin_max, first_wait, s_bail);
+    tail_wait(status, gsync, (unsigned)cur.z, p.expect, p.spin_max, first_wait, p.whole_lines, s_bail);
     first_wait = false;
   }
   // before the barrier that completes the list's partial sums
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
     }
     w.wait(a.plan, &s_bail);
 
-    // Operand rows, one float4 per child and tile, unconditionally (a missing child reads row 0 and is
+    // Operand rows, one float4 per child and tile, unconditionally (a missing child reads weights and is
     // masked); the next tile's are on their way while a tile is multiplied.
     struct Opnd {
       float4 v[NC];
@@ -216,7 +217,7 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
       for (int k = 0; k < NC; k++) {
         const int row = k == 0 ? c.y : c.z;
         o.on[k] = row >= 0;
-        o.v[k] = ld4(a.pool + (row >= 0 ? row : 0) * MW + ka);
+        o.v[k] = ld4((row >= 0 ? a.pool + row * MW : a.Wp) + ka);
       }
     };
     Opnd o, nx;
@@ -530,14 +531,14 @@ static int group_lds(const void *kernel) {
   return CAVS_OK;
 }
 
-static int group_plan(const char *who, const cavs_group_plan *p, int H, GroupPlan *out) {
+static int group_plan(const char *who, const cavs_group_plan *p, int H, bool whole_lines, GroupPlan *out) {
   CAVS_REQUIRE(cavs_group_rounds_ok(H), "%s: H=%d (multiples of 32 up to %d)", who, H, kGroupMaxH);
   CAVS_REQUIRE(p && p->groups && p->lists && p->recs && p->sync, "%s: null plan", who);
   CAVS_REQUIRE(aligned16(p->groups) && aligned16(p->lists) && aligned16(p->recs), "%s: the plan must be 16-byte aligned", who);
   CAVS_REQUIRE(p->ngroups >= 1 && p->ngroups <= cavs_group_max_groups(H) && p->spin_max >= 0 && p->extra_arrivals >= 0,
                "%s: bad plan (1..%d groups)", who, cavs_group_max_groups(H));
   *out = GroupPlan{reinterpret_cast<const int4 *>(p->groups), reinterpret_cast<const int4 *>(p->lists), reinterpret_cast<const int4 *>(p->recs),
-                   p->sync, p->ngroups, H / 16, p->spin_max, std::min(H / 16 + p->extra_arrivals, 64)};
+                   p->sync, p->ngroups, H / 16, p->spin_max, std::min(H / 16 + p->extra_arrivals, 64), whole_lines};
   return CAVS_OK;
 }
 
@@ -602,7 +603,7 @@ int cavs_group_rows(void) { return kGroupRows; }
 int cavs_treelstm_group_fwd(float *pool, const float *xW, int ld_xw, const float *Upk, const float *bias, float *G, float *hlr,
                             float *gates, float *msg, float *graph_out, int H, const cavs_group_plan *plan, void *stream) {
   GroupFwdArgs a{pool, xW, ld_xw, Upk, bias, G, hlr, gates, msg, graph_out, H, 0, {}};
-  if (int rc = group_plan("cavs_treelstm_group_fwd", plan, H, &a.plan)) return rc;
+  if (int rc = group_plan("cavs_treelstm_group_fwd", plan, H, line_rows(pool, 2 * H), &a.plan)) return rc;
   CAVS_REQUIRE(pool && xW && Upk && bias && G && hlr && gates && ld_xw >= 4 * H, "cavs_treelstm_group_fwd: null pointer or ld_xw=%d", ld_xw);
   CAVS_REQUIRE(aligned16(pool) && aligned16(Upk), "cavs_treelstm_group_fwd: pool and Upk must be 16-byte aligned");
   return group_fwd<GROUP_TREELSTM>(a, stream);
@@ -611,7 +612,7 @@ int cavs_treelstm_group_fwd(float *pool, const float *xW, int ld_xw, const float
 int cavs_lstm_group_fwd(float *pool, const float *xW, int ld_xw, const float *Whp, const float *bias, float *G, float *gates, float *msg,
                         float *graph_out, int H, const cavs_group_plan *plan, void *stream) {
   GroupFwdArgs a{pool, xW, ld_xw, Whp, bias, G, nullptr, gates, msg, graph_out, H, 0, {}};
-  if (int rc = group_plan("cavs_lstm_group_fwd", plan, H, &a.plan)) return rc;
+  if (int rc = group_plan("cavs_lstm_group_fwd", plan, H, line_rows(pool, 2 * H), &a.plan)) return rc;
   CAVS_REQUIRE(pool && xW && Whp && bias && G && gates && ld_xw >= 4 * H, "cavs_lstm_group_fwd: null pointer or ld_xw=%d", ld_xw);
   CAVS_REQUIRE(aligned16(pool) && aligned16(Whp), "cavs_lstm_group_fwd: pool and Whp must be 16-byte aligned");
   return group_fwd<GROUP_LSTM>(a, stream);
@@ -620,7 +621,7 @@ int cavs_lstm_group_fwd(float *pool, const float *xW, int ld_xw, const float *Wh
 int cavs_treefc_group_fwd(float *pool, const float *x, const float *Wp, const float *bias, float *G, float *msg, float *graph_out, int H,
                           int act, const cavs_group_plan *plan, void *stream) {
   GroupFwdArgs a{pool, x, H, Wp, bias, G, nullptr, nullptr, msg, graph_out, H, act, {}};
-  if (int rc = group_plan("cavs_treefc_group_fwd", plan, H, &a.plan)) return rc;
+  if (int rc = group_plan("cavs_treefc_group_fwd", plan, H, line_rows(pool, H), &a.plan)) return rc;
   CAVS_REQUIRE(pool && Wp && G && msg && (act == 0 || act == 1), "cavs_treefc_group_fwd: null pointer or act=%d", act);
   CAVS_REQUIRE(aligned16(pool) && aligned16(Wp), "cavs_treefc_group_fwd: pool and Wp must be 16-byte aligned");
   return group_fwd<GROUP_TREEFC>(a, stream);
@@ -629,7 +630,7 @@ int cavs_treefc_group_fwd(float *pool, const float *x, const float *Wp, const fl
 int cavs_treelstm_group_bwd(float *dxW, int ld_dxw, float *dF, float *dc, const float *UTp, const float *gates, const float *G,
                             const float *dret, int leaf_rows, int H, const cavs_group_plan *plan, void *stream) {
   GroupBwdArgs a{dxW, ld_dxw, dF, dc, UTp, gates, G, nullptr, dret, H, leaf_rows, 0, {}};
-  if (int rc = group_plan("cavs_treelstm_group_bwd", plan, H, &a.plan)) return rc;
+  if (int rc = group_plan("cavs_treelstm_group_bwd", plan, H, line_rows(dxW, ld_dxw) && line_rows(dF, H) && line_rows(dc, H), &a.plan)) return rc;
   CAVS_REQUIRE(dxW && dF && dc && UTp && gates && G && dret && ld_dxw >= 4 * H && ld_dxw % 4 == 0 && leaf_rows >= 0,
                "cavs_treelstm_group_bwd: null pointer or ld=%d", ld_dxw);
   CAVS_REQUIRE(aligned16(dxW) && aligned16(dF) && aligned16(UTp), "cavs_treelstm_group_bwd: dxW, dF and UTp must be 16-byte aligned");
@@ -639,7 +640,7 @@ int cavs_treelstm_group_bwd(float *dxW, int ld_dxw, float *dF, float *dc, const 
 int cavs_lstm_group_bwd(float *da, int ld_da, float *dc, const float *WhTp, const float *gates, const float *G, const float *dret,
                         int leaf_rows, int H, const cavs_group_plan *plan, void *stream) {
   GroupBwdArgs a{da, ld_da, nullptr, dc, WhTp, gates, G, nullptr, dret, H, leaf_rows, 0, {}};
-  if (int rc = group_plan("cavs_lstm_group_bwd", plan, H, &a.plan)) return rc;
+  if (int rc = group_plan("cavs_lstm_group_bwd", plan, H, line_rows(da, ld_da) && line_rows(dc, H), &a.plan)) return rc;
   CAVS_REQUIRE(da && dc && WhTp && gates && G && dret && ld_da >= 4 * H && ld_da % 4 == 0 && leaf_rows >= 0,
                "cavs_lstm_group_bwd: null pointer or ld=%d", ld_da);
   CAVS_REQUIRE(aligned16(da) && aligned16(WhTp), "cavs_lstm_group_bwd: da and WhTp must be 16-byte aligned");
@@ -649,7 +650,7 @@ int cavs_lstm_group_bwd(float *da, int ld_da, float *dc, const float *WhTp, cons
 int cavs_treefc_group_bwd(float *dz, const float *WTp, const float *h, const float *dret, int H, int act, const cavs_group_plan *plan,
                           void *stream) {
   GroupBwdArgs a{dz, H, nullptr, nullptr, WTp, nullptr, nullptr, h, dret, H, 0, act, {}};
-  if (int rc = group_plan("cavs_treefc_group_bwd", plan, H, &a.plan)) return rc;
+  if (int rc = group_plan("cavs_treefc_group_bwd", plan, H, line_rows(dz, H), &a.plan)) return rc;
   CAVS_REQUIRE(dz && WTp && h && dret && (act == 0 || act == 1), "cavs_treefc_group_bwd: null pointer or act=%d", act);
   CAVS_REQUIRE(aligned16(dz) && aligned16(WTp), "cavs_treefc_group_bwd: dz and WTp must be 16-byte aligned");
   return group_bwd<GROUP_TREEFC>(a, stream);

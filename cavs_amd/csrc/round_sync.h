@@ -31,8 +31,9 @@ __device__ inline void tail_arrive(unsigned *gsync, int wg, unsigned arrivals) {
 // Waits until the group's first `expect` (at most 64) workgroups have arrived `target` times; no barrier of the
 // workgroup.  Where the wait gives up (spin_max polls, or another workgroup already did, or the group's
 // workgroups turned out to sit on more than one XCD: the status word says why) *s_bail is set, and the
-// workgroup leaves behind its next barrier.
-__device__ inline void tail_wait(unsigned *status, unsigned *gsync, unsigned target, int expect, int spin_max, bool check_xcc, int *s_bail) {
+// workgroup leaves behind its next barrier.  `whole_lines`: see ld_row.
+__device__ inline void tail_wait(unsigned *status, unsigned *gsync, unsigned target, int expect, int spin_max, bool check_xcc, bool whole_lines,
+                                 int *s_bail) {
   const int lane = threadIdx.x & 63;
   unsigned why = 0;
   bool in = false;
@@ -50,6 +51,7 @@ __device__ inline void tail_wait(unsigned *status, unsigned *gsync, unsigned tar
     __hip_atomic_store(status, why, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     *s_bail = 1;
   }
+  if (!whole_lines) asm volatile("buffer_inv sc1" ::: "memory");
   asm volatile("" ::: "memory");  // (what the others wrote is read after this)
 }
 
@@ -68,11 +70,21 @@ __device__ inline void tail_leave(unsigned *gsync, int wgs) {
   if (threadIdx.x < 2) __hip_atomic_store(gsync + TAIL_XCC + threadIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// A row another workgroup of the group wrote in an earlier round.  No line of such a row can be in
-// this CU's L1 when the load is issued: the L1 starts a kernel empty, rows are whole cache lines,
-// and a row is first read after the barrier that follows its round.  So an ordinary load is served by the L2 the writers share.  (Loads
-// that bypass the L1 by scope -- agent-scope atomic loads -- were measured at about sixty cycles per
-// wavefront and access here, one request per lane: three times the MFMA time of a tile.)
+// A row another workgroup of the group wrote in an earlier round, by an ordinary load, which may be served by
+// this CU's L1.  A line that is in there is not updated by another CU's store, and what the workgroups share is
+// the L2; so no line of such a row may have been loaded before the barrier that follows the row's round:
+//   * the L1 starts a kernel empty, and a store does not leave its line in there;
+//   * a row is read only behind that barrier: loads for a missing child, which are issued all the same and
+//     masked, go to the weights (to row 0 of the pool they could meet a row of this launch);
+//   * rows are whole lines of 128 bytes, so that no row's line holds a piece of one written in another round.
+//     The launching side looks (whole_lines: pointers and row strides); where they are not, every wait drops
+//     the L1's lines (buffer_inv sc1, about 15 us a round for 32 workgroups).
+// Measured, a line loaded, stored to by another CU of the XCD, loaded again: the old value by an ordinary load, by
+// a load with sc0, and by one behind buffer_inv sc0; the new one behind buffer_inv sc1, by a load with sc1, and
+// after a store of one's own to the line.  Loads that bypass the L1 by scope (agent-scope atomic loads) cost
+// about sixty cycles per wavefront and access here, one request per lane: three times the MFMA time of a tile.
+constexpr int kLineBytes = 128;
+inline bool line_rows(const void *p, long ld_floats) { return reinterpret_cast<uintptr_t>(p) % kLineBytes == 0 && ld_floats * 4 % kLineBytes == 0; }
 __device__ inline float ld_row(const float *p) { return *p; }
 
 // The four k slots of an element added up across the wavefront, for the four rows of NP products

@@ -65,6 +65,7 @@ struct TailFwdArgs {
   const int *rows;      // the groups' lists of slab rows
   unsigned *sync;
   int spin_max, expect;
+  bool whole_lines;  // of the pool (ld_row)
   TailPlan plan;
 };
 
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_fwd_kernel(TailFwdArgs a
       for (int k = 0; k < 4; k++) xw[k] = p[k * H];
     }
     if (need > 0) {
-      tail_wait(status, gsync, (unsigned)need, a.expect, a.spin_max, first_wait, &s_bail);
+      tail_wait(status, gsync, (unsigned)need, a.expect, a.spin_max, first_wait, a.whole_lines, &s_bail);
       first_wait = false;
     }
 
@@ -169,12 +170,13 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_fwd_kernel(TailFwdArgs a
     }
 
     // Operand rows: one float4 per child and tile (see CAVS_MMA4), unconditionally (a missing child
-    // reads row 0 and is masked where the operand is used; past the last tile the last one is fetched
+    // reads weights and is masked where the operand is used; past the last tile the last one is fetched
     // again).  A tile's instruction stream carries, between the four k-groups of its MFMAs, the two
     // loads of the next tile and the slot sums of the tile before it: a wavefront stalled in a load's
     // issue or busy on the vector ALU issues no MFMAs, and with every wavefront of the CU in the
     // same phase the matrix pipes idled through both (measured: the three costs simply added up).
     const int ka = kb + 16 * ((lane >> 2) & 3) + 4 * slot;
+    auto child_row = [&](int c) { return (c >= 0 ? a.pool + (long)c * H2 : a.Upk) + ka; };
     struct Opnd {
       float4 l, r;
       int cl, cr;
@@ -206,7 +208,7 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_fwd_kernel(TailFwdArgs a
       nx.cr = child_of(t + 1, 1);
       CAVS_FWD_GROUP(0)
       __builtin_amdgcn_sched_barrier(0);
-      nx.l = ld4(a.pool + (long)(nx.cl >= 0 ? nx.cl : 0) * H2 + ka);
+      nx.l = ld4(child_row(nx.cl));
       if constexpr (PREV) sums.stage_a();
       __builtin_amdgcn_sched_barrier(0);
       CAVS_FWD_GROUP(1)
@@ -215,7 +217,7 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_fwd_kernel(TailFwdArgs a
       __builtin_amdgcn_sched_barrier(0);
       CAVS_FWD_GROUP(2)
       __builtin_amdgcn_sched_barrier(0);
-      nx.r = ld4(a.pool + (long)(nx.cr >= 0 ? nx.cr : 0) * H2 + ka);
+      nx.r = ld4(child_row(nx.cr));
       if constexpr (PREV) sums.stage_c();
       __builtin_amdgcn_sched_barrier(0);
       CAVS_FWD_GROUP(3)
@@ -233,8 +235,8 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_fwd_kernel(TailFwdArgs a
       Opnd oa, ob;
       oa.cl = child_of(0, 0);
       oa.cr = child_of(0, 1);
-      oa.l = ld4(a.pool + (long)(oa.cl >= 0 ? oa.cl : 0) * H2 + ka);
-      oa.r = ld4(a.pool + (long)(oa.cr >= 0 ? oa.cr : 0) * H2 + ka);
+      oa.l = ld4(child_row(oa.cl));
+      oa.r = ld4(child_row(oa.cr));
       tile(std::false_type{}, 0, oa, ob);
       for (int t = 1; t < T; t += 2) {
         tile(std::true_type{}, t, ob, oa);
@@ -295,6 +297,7 @@ struct TailBwdArgs {
   const int *rows;      // the groups' lists of slab rows
   unsigned *sync;
   int leaf_rows, spin_max, expect;
+  bool whole_lines;  // of dxW, dF and dc (ld_row)
   TailPlan plan;
 };
 
@@ -395,7 +398,7 @@ __global__ __launch_bounds__(512, 1) void treelstm_tail_bwd_kernel(TailBwdArgs a
       }
     }
     if (need > 0) {
-      tail_wait(status, gsync, (unsigned)need, a.expect, a.spin_max, first_wait, &s_bail);
+      tail_wait(status, gsync, (unsigned)need, a.expect, a.spin_max, first_wait, a.whole_lines, &s_bail);
       first_wait = false;
     }
     const float pdc = eon ? ld_row(a.dc + erow * H + ej) : 0.f;
@@ -535,7 +538,7 @@ __global__ __launch_bounds__(512, 1) void tail_probe_kernel(unsigned *sync, int 
   if (threadIdx.x == 0) s_bail = 0;
   __syncthreads();
   for (int r = 0; r < 3; r++) {
-    if (r > 0) tail_wait(status, gsync, r, expect, spin_max, r == 1, &s_bail);
+    if (r > 0) tail_wait(status, gsync, r, expect, spin_max, r == 1, true, &s_bail);
     __syncthreads();
     if (s_bail) return;
     tail_arrive(gsync, blockIdx.x >> 3, r + 1);
@@ -613,7 +616,7 @@ int cavs_treelstm_tail_fwd(float *pool, const int *child, const int *pair, const
   CAVS_REQUIRE(!graph_out || out_rows, "cavs_treelstm_tail_fwd: graph_out needs out_rows");
   CAVS_REQUIRE(spin_max >= 0 && extra_arrivals >= 0, "cavs_treelstm_tail_fwd: bad wait bound");
   TailFwdArgs a{pool, child, pair, xW, ld_xw, Upk, bias, G, hlr, gates, msg, graph_out, out_rows, rows, sync, spin_max,
-                std::min(H / 16 + extra_arrivals, 64), {}};
+                std::min(H / 16 + extra_arrivals, 64), line_rows(pool, 2 * H), {}};
   const int todo = tail_plan("cavs_treelstm_tail_fwd", ngroups, nrounds, start, count, flags, max_rounds, &a.plan);
   if (todo <= 0) return todo;
   constexpr size_t lds = kTailFwdRed * sizeof(float) + kTailTabBytes;
@@ -638,7 +641,7 @@ int cavs_treelstm_tail_bwd(float *dxW, int ld_dxw, float *dF, float *dc, const f
   CAVS_REQUIRE(aligned16(dxW) && aligned16(dF) && aligned16(UTp), "cavs_treelstm_tail_bwd: dxW, dF and UTp must be 16-byte aligned");
   CAVS_REQUIRE(spin_max >= 0 && extra_arrivals >= 0, "cavs_treelstm_tail_bwd: bad wait bound");
   TailBwdArgs a{dxW, ld_dxw, dF, dc, UTp, child_rows, gates, G, dret, dret_rows, rows, sync, leaf_rows, spin_max,
-                std::min(H / 16 + extra_arrivals, 64), {}};
+                std::min(H / 16 + extra_arrivals, 64), line_rows(dxW, ld_dxw) && line_rows(dF, H) && line_rows(dc, H), {}};
   const int todo = tail_plan("cavs_treelstm_tail_bwd", ngroups, nrounds, start, count, flags, max_rounds, &a.plan);
   if (todo <= 0) return todo;
   constexpr size_t lds = kTailBwdRed * sizeof(float) + kTailTabBytes;

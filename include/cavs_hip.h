@@ -477,6 +477,9 @@ int cavs_treelstm_round_leaves_fwd(float *pool, const int *pair, const float *xW
  *   spin_max polls: a group's workgroups were not all resident at once) or CAVS_TAIL_SPREAD (they
  *   did not share one XCD).  With a non-zero status every wave has left the kernel, the results of
  *   the launch are undefined, and the caller must clear the block before the next launch.
+ *   The rows that pass from round to round (forward: pool; backward: dxW, dF, dc) are best whole 128-byte
+ *   lines, i.e. pointers and row strides multiples of 128 bytes; where they are not, every round takes
+ *   some fifteen microseconds longer.
  *   Launches on one block must not overlap.  extra_arrivals > 0 makes every wait expect that many
  *   more arrivals than there are workgroups: the way to see the give-up path from a test.
  * For H = 512 (cavs_tail_rounds_ok); at most cavs_tail_max_rounds() lists per group. */

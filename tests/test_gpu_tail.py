@@ -209,6 +209,76 @@ def test_backward_tail_equals_the_per_round_launches_bit_for_bit(g, sizes, base,
     assert (outs[1][0][kid_rows] != -3.0).all()
 
 
+def shifted(g, a, floats):
+    """`a` on the device, `floats` floats past a line of 128 bytes"""
+    t = g.zeros(a.size + 64)
+    v = t[floats: floats + a.size].view(*a.shape)
+    v.copy_(g.devf(a))
+    return v
+
+
+@pytest.mark.parametrize("shift", [0, 4, 20])
+def test_rows_that_pass_between_rounds_are_never_read_from_a_stale_line(g, shift):
+    """Forward: pool row 0 belongs to a vertex of the launch (a load for a missing child must not bring it in before it
+    is written), and rows that start in the middle of a line share it with rows written in other rounds.  Backward:
+    the same for dxW, dF and dc, at a row stride that is no whole number of lines."""
+    sizes, base = (30, 22, 13, 6, 3, 1, 1), 90
+    r = rng(77 + shift)
+    U = (r.bulk_normal(4 * H * H) / np.sqrt(H)).astype(np.float32)
+    d_U, Upk, UTp = packed_weights(g, U)
+    offs, child, N = forest(r, base, sizes)
+    perm = np.arange(N)
+    perm[[0, offs[0]]] = offs[0], 0  # the first vertex of the first round writes pool row 0
+    pair, pchild = perm.astype(np.int32), np.where(child >= 0, perm[child], -1).astype(np.int32)
+    pair[offs[-1]] = -1
+    pool0 = (r.bulk_normal(N * 2 * H).reshape(N, 2 * H) * 0.5).astype(np.float32)
+    d_child, d_kids, d_pair, d_rows = g.devi(pchild), g.devi(child), g.devi(pair), g.devi(np.argsort(r.bulk_normal(N)).astype(np.int32))
+    d_xW, d_bias = g.devf(r.bulk_normal(N * 4 * H)), g.devf(r.bulk_normal(4 * H) * 0.1)
+    fwd, bwd = plan_groups(offs, sizes, child, 1), plan_groups(offs[::-1], sizes[::-1], child, 1, backward=True)
+    outs = []
+    for tail in (False, True):
+        pool = shifted(g, pool0, shift)
+        G, hlr, gates, go = g.zeros(2 * N, 2 * H), g.zeros(N, H), g.zeros(N, 6 * H), g.zeros(N, H)
+        if tail:
+            rows, nrounds, start, count, flags, maxr = fwd
+            sync = sync_block(g)
+            g.call("cavs_treelstm_tail_fwd", g.P(pool), g.P(d_child), g.P(d_pair), g.P(d_xW), 4 * H, g.P(Upk), g.P(d_bias), g.P(G), g.P(hlr),
+                   g.P(gates), None, g.P(go), g.P(d_rows), g.P(g.devi(rows)), 1, nrounds.ctypes.data, start.ctypes.data, count.ctypes.data,
+                   flags.ctypes.data, maxr, H, g.P(sync), 1 << 20, 0, g.stream())
+            assert not g.host(sync).any()
+        else:
+            for off, n in chunks(offs, sizes):
+                g.call("cavs_treelstm_round_fwd_packed", g.P(pool), g.P(d_child) + 4 * 2 * off, g.P(d_pair) + 4 * off, g.P(d_xW) + 4 * off * 4 * H,
+                       4 * H, g.P(d_U), g.P(Upk), g.P(d_bias), g.P(G) + 4 * 2 * off * 2 * H, g.P(hlr) + 4 * off * H, g.P(gates) + 4 * off * 6 * H,
+                       None, g.P(go), g.P(d_rows) + 4 * off, n, H, g.stream())
+        outs.append([g.host(t) for t in (pool, G, hlr, gates, go)])
+    for a, b, what in zip(*outs, ("pool", "G", "hlr", "gates", "graph_out")):
+        np.testing.assert_array_equal(a, b, err_msg=what)
+
+    d_gates, d_G, d_dgo = g.devf(np.tanh(r.bulk_normal(N * 6 * H)).astype(np.float32)), g.devf(r.bulk_normal(2 * N * 2 * H) * 0.5), g.devf(r.bulk_normal(N * H))
+    taken = set(int(k) for k in child if k >= 0)
+    d_orph = g.devi(np.array([v for v in range(N) if v not in taken], np.int32))
+    ld, outs = 4 * H + shift, []
+    for tail in (False, True):
+        dxW, dF, dc = (shifted(g, np.zeros(s, np.float32), shift) for s in ((N, ld), (2 * N, H), (N, H)))
+        g.call("cavs_treelstm_bwd_gates_rows", g.P(d_orph), d_orph.numel(), g.P(d_dgo), g.P(d_rows), g.P(d_gates), g.P(d_G), g.P(dxW), ld, g.P(dF),
+               g.P(dc), base, H, g.stream())
+        if tail:
+            rows, nrounds, start, count, flags, maxr = bwd
+            sync = sync_block(g)
+            g.call("cavs_treelstm_tail_bwd", g.P(dxW), ld, g.P(dF), g.P(dc), g.P(UTp), g.P(d_kids), g.P(d_gates), g.P(d_G), g.P(d_dgo), g.P(d_rows),
+                   base, g.P(g.devi(rows)), 1, nrounds.ctypes.data, start.ctypes.data, count.ctypes.data, flags.ctypes.data, maxr, H, g.P(sync),
+                   1 << 20, 0, g.stream())
+            assert not g.host(sync).any()
+        else:
+            for off, n in chunks(offs[::-1], sizes[::-1]):
+                g.call("cavs_treelstm_round_bwd_children_gates_packed", g.P(dxW), ld, g.P(dF), g.P(dc), g.P(UTp), g.P(d_kids) + 4 * 2 * off,
+                       g.P(d_gates), g.P(d_G), g.P(d_dgo), g.P(d_rows), off, n, base, H, g.stream())
+        outs.append([g.host(t) for t in (dxW, dF, dc)])
+    for a, b, what in zip(*outs, ("dxW", "dF", "dc")):
+        np.testing.assert_array_equal(a, b, err_msg=what)
+
+
 def test_a_wait_that_cannot_complete_gives_up_and_every_wave_leaves(g):
     """extra_arrivals = 1: every wait expects one arrival more than there are workgroups, so the
     first wait runs into its bound.  The launch must end by itself with the status word set; after
