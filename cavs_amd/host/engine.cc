@@ -268,7 +268,6 @@ Engine::~Engine() {
     if (e) cavs_event_destroy(e);
   for (auto &m : marks_)
     if (m.ev) cavs_event_destroy(m.ev);
-  if (word_ev_) cavs_event_destroy(word_ev_);
   if (own_stream_) cavs_stream_destroy(stream_);
 }
 
@@ -606,10 +605,7 @@ void Engine::reserve_edges() {
     R(dxW_, cap * H);
     R(r_z_, rc * H);
   }
-  // (beside: on the scheduler's stream, while the kernels of the last step run)
-  // (not while the lists of a cached plan are still being copied)
-  words_beside_ = own_stream_ && !direct_ && !cfg_.graph_replay && (cfg_.plan_cache == 0 || (hit_plan_ && hit_plan_->made <= done_step_));
-  words_ = words_wanted(words_beside_);
+  words_ = words_wanted();
   if (words_) {
     const size_t w = cell_ ? (size_t)cell_->NX * H : 4 * H;
     size_t most = cell_ ? 0 : w;
@@ -621,13 +617,12 @@ void Engine::reserve_edges() {
     R(xW_words_, cap * w);
     if (!cell_) R(d_words_, cap * w);
     R(word_parts_, cavs_gather_sums_workspace((int)cap, (int)most) / 4);
-    for (WordIndex &wi : word_index_) {
-      const size_t ints = cavs_embed_index_ints((int)cap);
-      if (wi.index.capacity() >= ints) continue;
+    const size_t ints = cavs_embed_index_ints((int)cap);
+    if (word_index_.capacity() < ints) {
       check(cavs_stream_sync(stream_));
-      wi.index.reserve(ints);
-      wi.ids.reserve(cap);
-      wi.scratch.reserve(cavs_embed_index_workspace((int)cap) / 4);
+      word_index_.reserve(ints);
+      word_ids_.reserve(cap);
+      word_scratch_.reserve(cavs_embed_index_workspace((int)cap) / 4);
     }
   }
   if (fused_rows() > 0 && !cell_) R(UT_, (size_t)(cfg_.model == CAVS_MODEL_TREEFC ? 2 : 4) * H * H);
@@ -658,16 +653,20 @@ void Engine::reserve_edges() {
 
 // Whether x * W and its gradients go by words: every different id of the batch once (cavs_embed_index).
 // Saved: the products' rows of the ids met before (a parse tree's inner vertices all look up one word), at
-// 140 TFLOP/s.  Paid: the index where the step has to wait for it (2368 vertices 15 us, 16000 65, 73000
-// 360), spreading the rows (5 / 24 / 256 us at 2048, 2048, 4096 columns), in the backward pass adding up
-// their gradients (10 / 36 / 345 us).
-bool Engine::words_wanted(bool beside) const {
+// 140 TFLOP/s.  Paid: the index (2368 vertices 15 us, 16000 65, 73000 360), spreading the rows (5 / 24 / 256 us
+// at 2048, 2048, 4096 columns), in the backward pass adding up their gradients (10 / 36 / 345 us).  The line is
+// at 1.5 because both are estimates: of 72 sessions (Tree-LSTMs and chains, H = 128 .. 1024, 1200 .. 19000 vertices,
+// with and without a backward pass) all 25 above it gain, 5 us (260 a step) to 1.2 ms (4.85), and of those
+// below it the six that would are between 0.59 and 1.45, by 50 us at most, beside others that would lose as much.
+// (The index on another stream while the kernels of the step before run, which takes it off this account,
+// gained nothing: 10 to 16 us more a step than in line, 1200 to 19000 vertices.)
+bool Engine::words_wanted() const {
   if (N_ < 2048 || cfg_.V <= 0 || cfg_.V >= 1 << 24) return false;
   if (cell_ ? cell_->NX == 0 || cfg_.H % 4 : cfg_.model != CAVS_MODEL_TREELSTM && cfg_.model != CAVS_MODEL_LSTM) return false;
   const double n = N_, w = (double)(cell_ ? cell_->NX : 4) * cfg_.H;
   const double saved = 2.0 * (n - words_expected()) * w * E_ * (trains_ ? 3 : 1) / 140e6;
-  const double paid = (beside ? 0.0 : 8.0 + 0.004 * n) + 6.0 + n * w / 1e6 + (trains_ ? 6.0 + n * w / 0.8e6 : 0.0);
-  return saved > 1.5 * paid;  // (2368 vertices, 2048 columns: 31 against 23 us on paper, no difference measured)
+  const double paid = 8.0 + 0.004 * n + 6.0 + n * w / 1e6 + (trains_ ? 6.0 + n * w / 0.8e6 : 0.0);
+  return saved > 1.5 * paid;
 }
 
 // How many different ids to expect (plans and flop counts only): the leaves' of a tree, half of a text's.
@@ -676,29 +675,16 @@ int Engine::words_expected() const {
   return std::max(1, (int)(V * (1.0 - std::exp(-n / V))));
 }
 
+// On the session's stream, like everything that reads the feeds: a caller may have ordered its own work there.
 void Engine::words_index(int leaf_rows) {
-  WordIndex &wi = word_index_[word_slot_];
-  word_slot_ ^= 1;
-  d_words_index_ = wi.index.get();
-  if (words_beside_) {
-    wait_step(wi.used);  // (the step before last)
-    if (!sched_stream_) check(cavs_stream_create(&sched_stream_));
-    if (!word_ev_) check(cavs_event_create(&word_ev_));
-  }
-  wi.used = steps_;
-  buffers_used_ = true;
-  check(cavs_embed_index(wi.index.get(), wi.ids.get(), d_x_, d_t2j_, N_, cfg_.V, leaf_rows, wi.scratch.get(), wi.scratch.capacity() * 4,
-                         words_beside_ ? sched_stream_ : stream_));
-  if (words_beside_) {
-    check(cavs_event_record(word_ev_, sched_stream_));
-    check(cavs_event_sync(word_ev_));
-  }
+  d_words_index_ = word_index_.get();
+  check(cavs_embed_index(word_index_.get(), word_ids_.get(), d_x_, d_t2j_, N_, cfg_.V, leaf_rows, word_scratch_.get(),
+                         word_scratch_.capacity() * 4, stream_));
 }
 
 // xW_ [N, w] = looked-up rows times W; rows of leaves are only wanted below column leaf_w
 void Engine::words_forward(const float *W, int w, int leaf_w) {
   const int N = N_, lp = leaf_w < w ? sched_->leaf_prefix : 0;
-  const float *ids = word_index_[word_slot_].ids.get();
   words_index(lp);
   {
     ProfScope ps(this, K_GATHER);
@@ -707,7 +693,7 @@ void Engine::words_forward(const float *W, int w, int leaf_w) {
   gemm_group({{0, 0, N, w, E_, 1.f, 0.f, e_.get(), ld_e_, W, w, xW_words_.get(), w, lp > 0 ? CAVS_GEMM_C_UNUSED : 0, lp, leaf_w, d_words_index_,
                words_expected(), pad_block(), uH_}});
   ProfScope ps(this, K_GATHER);
-  check(cavs_spread_rows(xW_.get(), w, xW_words_.get(), w, d_words_index_, N, w, lp, leaf_w, ids, xs_.get(), stream_));
+  check(cavs_spread_rows(xW_.get(), w, xW_words_.get(), w, d_words_index_, N, w, lp, leaf_w, word_ids_.get(), xs_.get(), stream_));
   c_launches_ += 3;
 }
 
@@ -821,7 +807,6 @@ void Engine::remember_plan(const int *graph, int B, int maxlen, uint64_t hash) {
   }
   const size_t N = N_, nk = (size_t)nch_ * N;
   p->hash = hash;
-  p->made = steps_;
   p->B = B;
   p->maxlen = maxlen;
   p->pairing = cfg_.pairing;

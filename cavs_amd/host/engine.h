@@ -350,7 +350,6 @@ class Engine {
     bool graph_off = false;  // recording failed once: ordinary steps from then on
     int recordings = 0;
     uint64_t hash = 0;
-    uint64_t made = 0;  // the step whose stream work fills the lists
     int B = 0, maxlen = 0, pairing = 0;
     std::vector<int32_t> graph;
     std::shared_ptr<Schedule> sched;
@@ -401,20 +400,14 @@ class Engine {
   // e^T * dxW yields the bias gradient (column sums of dxW) as row E of dW for free
   int ld_e_ = 0;
   // x * W and its gradients by words (words_wanted): the index, the products' rows, the gradients' sums
-  struct WordIndex {
-    DeviceArray<int> index;
-    DeviceArray<float> ids, scratch;
-    uint64_t used = 0;  // the last step that reads it
-  };
-  WordIndex word_index_[2];  // of this step and the last: the index is made beside the last step's kernels
-  int word_slot_ = 0;
-  void *word_ev_ = nullptr;
-  bool words_ = false, words_beside_ = false;
+  DeviceArray<int> word_index_;
+  DeviceArray<float> word_ids_, word_scratch_;
+  bool words_ = false;
   bool trains_ = true;  // a backward pass follows
   const int *d_words_index_ = nullptr;
   DeviceArray<float> xW_words_, d_words_, word_parts_;
   int pad_block() const { return uH_ != cfg_.H ? cfg_.H : 0; }  // padding of x * W (cavs_gemm_desc::pad_block, uH_ used)
-  bool words_wanted(bool beside) const;
+  bool words_wanted() const;
   int words_expected() const;
   void words_index(int leaf_rows);
   void words_forward(const float *W, int w, int leaf_w);

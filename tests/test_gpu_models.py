@@ -740,3 +740,48 @@ def test_an_infinite_embedding_saturates_gates_and_nothing_else_at_sizes_stored_
     assert np.isfinite(out[1][0]).all() and np.isfinite(out[1][1]).all()
     close(out[0][0], out[1][0].astype(np.float64), "graph_out")
     close(out[0][1], out[1][1].astype(np.float64), "loss")
+
+
+@pytest.mark.parametrize("model,H,E", [("treelstm", 128, 1024), ("lstm", 384, 384)])
+def test_a_device_feed_written_on_the_sessions_stream_is_read_behind_that(model, H, E):
+    """cavs_session_stream is there for callers that order their own work with a session's: a feed that is written on
+    it before a step is the feed that step reads, also where the step looks at its words (batches of thousands)
+    and the kernels of the step before are still running."""
+    import torch
+
+    V, rng = 300, synth.SplitMix64(H)
+    u = lambda *s: rng.bulk_uniform(int(np.prod(s)), -0.1, 0.1).reshape(s).astype(np.float32)  # noqa: E731
+    if model == "treelstm":
+        trees = [synth.random_binary_tree(rng, 20) for _ in range(90)]
+        graph, N, params = synth.pack_graph(trees, 39), 90 * 39, dict(Emb=u(V, E), W=u(E, 4 * H), U=u(4 * H * H), Bv=u(4 * H))
+    else:
+        graph, N, params = synth.pack_graph([synth.chain(40)] * 120, 40), 120 * 40, dict(Emb=u(V, E), W=u(8 * H * H), Bv=u(4 * H))
+    params.update(Wfc=u(5, H), bfc=u(5))
+    feeds = [np.floor(rng.bulk_uniform(N) * V).astype(np.float32) for _ in range(4)]
+    labels = torch.from_numpy(np.floor(rng.bulk_uniform(N) * 5).astype(np.float32)).cuda()
+    big = torch.rand(4096, 4096, device="cuda")
+    out = []
+    for late in (False, True):
+        s = session.Session(model, H=H, E=E, V=V, C_=5)
+        s.set_params(params)
+        mine = torch.cuda.ExternalStream(session.lib().cavs_session_stream(s._h))
+        x, staged = torch.from_numpy(feeds[0]).cuda(), [torch.from_numpy(f).cuda() for f in feeds]
+        torch.cuda.synchronize()
+        for f in staged:
+            if late:
+                with torch.cuda.stream(mine):
+                    for _ in range(8):  # milliseconds of work in front of the copy
+                        big @ big
+                    x.copy_(f)
+            else:
+                x.copy_(f)
+                torch.cuda.synchronize()
+            s.step(graph, x, labels, backward=True, lr=0.1)
+            if not late:
+                s.sync()
+        out.append((s.fetch("loss"), {k: s.param(k, v.shape) for k, v in params.items()}))
+        torch.cuda.synchronize()
+        s.close()
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    for k in params:
+        np.testing.assert_array_equal(out[0][1][k], out[1][1][k], err_msg=k)
