@@ -1099,9 +1099,9 @@ void Engine::begin_step(const int *graph, int B, int maxlen) {
   parse_ms_ = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
 
-void Engine::forward_only(const int *graph, int B, int maxlen, const float *x_dev, float *graph_out) {
+void Engine::forward_only(const int *graph, int B, int maxlen, const float *x_dev, float *graph_out, bool trains) {
   state_epoch_++;
-  trains_ = true;
+  trains_ = trains;
   begin_step(graph, B, maxlen);
   const bool reads_x = cell_ ? cell_->NX > 0 || cell_->XD > 0 : (cfg_.model != CAVS_MODEL_TREEFC || cfg_.use_x);
   if (reads_x && !x_dev) fail(CAVS_EINVAL, "vertex input feed is null");

@@ -68,8 +68,8 @@ class Engine {
   bool update_jobs(float *w, float *g, float lr, std::vector<cavs_task> *out);
   float *graph_out_ptr() const { return uH_ == cfg_.H ? GO_.get() : go_user_.get(); }
   // The two halves of step() for a caller that runs the loss head itself: forward F into
-  // graph_out [N,H] (vertex order), then backward F from d graph_out.
-  void forward_only(const int *graph, int B, int maxlen, const float *x_dev, float *graph_out);
+  // graph_out [N,H] (vertex order), then backward F from d graph_out.  trains: whether that follows.
+  void forward_only(const int *graph, int B, int maxlen, const float *x_dev, float *graph_out, bool trains);
   // settle_biases = false leaves the bias gradients that exist as rows still to be added up
   // (row E of dW, chunk sums) pending: the caller then takes them with update_bias_jobs() into the
   // launch that applies its parameter updates, instead of a launch of their own here.

@@ -826,6 +826,7 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
   // when nothing between that pass and the update reads them (no clipping, every later gradient op
   // planned away), the engine's pending bias gradients (into the launch that applies the updates).
   head_defer_ = defer_bias_ = false;
+  trains_ = train;
   if (train && lowered_) {
     int at = -1;
     const std::vector<char> &skip = it->second.skip_bwd;

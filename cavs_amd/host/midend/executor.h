@@ -92,6 +92,7 @@ class Executor {
   // with the backward rounds split as for a batch whose message flow is no forest
   int lowering_mode_ = 1;
   bool lowered_ = false;
+  bool trains_ = false;  // this Run has a backward pass
   int pairing_ = 0;
   std::map<std::string, std::unique_ptr<Tensor>> tensors_;
   std::map<std::string, FeedStage> feed_stages_;

@@ -379,7 +379,7 @@ void Executor::lowered_forward(const int32_t *graph, int B, int maxlen, float *)
     Tensor &t = tensor(lw.roles.at(kv.first));
     engine_->bind_param(s.param, t.base - s.offset, nullptr);
   }
-  engine_->forward_only(graph, B, maxlen, func_arg_, nullptr);
+  engine_->forward_only(graph, B, maxlen, func_arg_, nullptr, trains_);
   N_ = engine_->total_length();
   Tensor &go = tensor(global_graph().graph_output);
   go.base = engine_->graph_out_ptr();
