@@ -2,6 +2,8 @@
 
 #include <algorithm>
 #include <cstring>
+#include <string>
+#include <system_error>
 
 namespace cavs {
 
@@ -31,7 +33,10 @@ std::shared_ptr<ReadbackPool> ReadbackPool::shared() {
 ReadbackPool::ReadbackPool() {
   ring_.reserve(kSlot * kSlots);
   const int spare = std::max(1, (int)std::thread::hardware_concurrency() - 1);
-  for (int i = 0; i < std::min(kThreads, spare); i++) threads_.emplace_back([this] { thread_main(); });
+  try {
+    for (int i = 0; i < std::min(kThreads, spare); i++) threads_.emplace_back([this] { thread_main(); });
+  } catch (const std::system_error &) {  // (no more to be had: those there are and the caller's carry on)
+  }
 }
 
 ReadbackPool::~ReadbackPool() {
@@ -39,49 +44,51 @@ ReadbackPool::~ReadbackPool() {
     std::lock_guard<std::mutex> lock(m_);
     stop_ = true;
   }
-  wake_.notify_all();
+  more_.notify_all();
   for (std::thread &t : threads_) t.join();
 }
 
-// Takes pieces in order until there are none left.  The caller's own turn ends early when the next piece
-// is not on its way yet: queueing it is the caller's work.
-void ReadbackPool::work(Job &j, bool caller) {
-  constexpr long per = kSlot / kPiece;
-  for (;;) {
-    long i = j.next.load(std::memory_order_relaxed);
-    if (i >= j.pieces) return;
-    const long chunk = i / per;
-    if (chunk >= j.queued.load(std::memory_order_acquire)) {
-      if (caller || j.failed.load(std::memory_order_relaxed)) return;
-      std::this_thread::yield();
+// Takes one piece on; call with j.can_take().  Pieces are taken in order, and one thread at a time waits for the
+// link, for the first chunk that is not known to have arrived.
+void ReadbackPool::carry(std::unique_lock<std::mutex> &lock, Job &j) {
+  const long i = j.next++, chunk = i / (long)(kSlot / kPiece);
+  const int slot = (int)(chunk % kSlots);
+  while (j.arrived <= chunk && !j.failed) {
+    if (j.waits) {
+      progress_.wait(lock);
       continue;
     }
-    if (!j.next.compare_exchange_weak(i, i + 1)) continue;
-    const int slot = (int)(chunk % kSlots);
-    if (j.arrived.load(std::memory_order_acquire) <= chunk) {
-      if (cavs_event_sync((*j.events)[slot]) != CAVS_OK) j.failed = true;
-      long seen = j.arrived.load(std::memory_order_relaxed);
-      // (chunks of one stream arrive in order, but the other stream's last one may still be under way)
-      if (seen == chunk) j.arrived.compare_exchange_strong(seen, chunk + 1, std::memory_order_release);
-    }
-    const size_t at = (size_t)i * kPiece;
-    std::memcpy(j.host + at, ring_.get() + slot * kSlot + at % kSlot, std::min(kPiece, j.bytes - at));
-    j.slot_pieces[slot].fetch_add(1, std::memory_order_release);
-    j.done.fetch_add(1, std::memory_order_release);
+    j.waits = true;
+    void *event = (*j.events)[j.arrived % kSlots];
+    lock.unlock();
+    const int rc = cavs_event_sync(event);
+    lock.lock();
+    j.waits = false;
+    j.arrived++;
+    if (rc != CAVS_OK) j.failed = true;
+    progress_.notify_all();
   }
+  if (!j.failed) {
+    const size_t at = (size_t)i * kPiece;
+    lock.unlock();
+    std::memcpy(j.host + at, ring_.get() + slot * kSlot + at % kSlot, std::min(kPiece, j.bytes - at));
+    lock.lock();
+  }
+  j.slot_pieces[slot]++;
+  j.done++;
+  progress_.notify_all();
 }
 
 void ReadbackPool::thread_main() {
   std::unique_lock<std::mutex> lock(m_);
   for (;;) {
-    wake_.wait(lock, [this] { return stop_ || (job_ && job_->next.load() < job_->pieces); });
+    more_.wait(lock, [this] { return stop_ || (job_ && job_->can_take()); });
     if (stop_) return;
-    Job *j = job_;
+    Job &j = *job_;
     inside_++;
-    lock.unlock();
-    work(*j, false);
-    lock.lock();
-    if (--inside_ == 0) idle_.notify_all();
+    while (j.can_take()) carry(lock, j);
+    inside_--;
+    progress_.notify_all();
   }
 }
 
@@ -92,34 +99,39 @@ void ReadbackPool::read(char *host, const char *dev, size_t bytes, void *const s
   j.bytes = bytes;
   j.pieces = (long)((bytes + kPiece - 1) / kPiece);
   j.events = &events;
-  for (auto &s : j.slot_pieces) s = 0;
-  {
-    std::lock_guard<std::mutex> lock(m_);
-    job_ = &j;
-  }
-  wake_.notify_all();
   int rc = CAVS_OK;
   const long chunks = (long)((bytes + kSlot - 1) / kSlot);
+  std::unique_lock<std::mutex> lock(m_);
+  job_ = &j;
+  // (the caller carries pieces on as well, but queueing the next chunk comes first)
+  auto work_until = [&](auto over) {
+    while (!over()) {
+      if (j.can_take()) carry(lock, j);
+      else progress_.wait(lock);
+    }
+  };
   for (long i = 0; i < chunks && rc == CAVS_OK; i++) {
     const int slot = (int)(i % kSlots);
     // (only the last chunk of a read is shorter than its slot)
-    while (j.slot_pieces[slot].load(std::memory_order_acquire) < i / kSlots * (long)(kSlot / kPiece) && !j.failed.load(std::memory_order_relaxed))
-      work(j, true);
+    work_until([&] { return j.failed || j.slot_pieces[slot] >= i / kSlots * (long)(kSlot / kPiece); });
+    if (j.failed) break;
+    lock.unlock();
     const size_t at = (size_t)i * kSlot;
     rc = cavs_memcpy_d2h(ring_.get() + slot * kSlot, dev + at, std::min(kSlot, bytes - at), streams[i & 1]);
     if (rc == CAVS_OK) rc = cavs_event_record(events[slot], streams[i & 1]);
-    if (rc == CAVS_OK) j.queued.store(i + 1, std::memory_order_release);
+    lock.lock();
+    if (rc == CAVS_OK) j.queued = i + 1;
+    else j.failed = true;
+    more_.notify_all();
   }
-  if (rc != CAVS_OK) j.failed = true;
-  work(j, true);
-  while (j.done.load(std::memory_order_acquire) < (rc == CAVS_OK ? j.pieces : j.next.load())) std::this_thread::yield();
-  {
-    std::unique_lock<std::mutex> lock(m_);
-    job_ = nullptr;
-    idle_.wait(lock, [this] { return inside_ == 0; });
-  }
-  if (rc != CAVS_OK) check(rc);
-  if (j.failed) fail(CAVS_EHIP, "reading device memory back failed");
+  work_until([&] { return j.failed || j.done == j.pieces; });
+  job_ = nullptr;
+  progress_.wait(lock, [this] { return inside_ == 0; });
+  lock.unlock();
+  if (!j.failed) return;
+  const std::string why = rc != CAVS_OK ? cavs_last_error() : "";
+  for (int k = 0; k < 2; k++) (void)cavs_stream_sync(streams[k]);  // (nothing of it still on its way into the ring)
+  fail(rc != CAVS_OK ? rc : CAVS_EHIP, "reading device memory back failed" + (why.empty() ? why : ": " + why));
 }
 
 Readback::~Readback() {
@@ -141,7 +153,15 @@ void Readback::read(void *host, const void *dev, size_t bytes, void *stream) {
     check(cavs_stream_sync(stream));
     return;
   }
-  if (!pool_) pool_ = ReadbackPool::shared();
+  if (!pool_) {
+    try {
+      pool_ = ReadbackPool::shared();
+    } catch (const Error &) {  // no pinned memory for a ring: a plain copy will do
+      check(cavs_memcpy_d2h(host, dev, bytes, stream));
+      check(cavs_stream_sync(stream));
+      return;
+    }
+  }
   while (events_.size() < (size_t)ReadbackPool::kSlots) {
     void *e = nullptr;
     check(cavs_event_create(&e));

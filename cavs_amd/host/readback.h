@@ -8,7 +8,6 @@
 #ifndef CAVS_HOST_READBACK_H_
 #define CAVS_HOST_READBACK_H_
 
-#include <atomic>
 #include <condition_variable>
 #include <cstddef>
 #include <memory>
@@ -34,26 +33,30 @@ class ReadbackPool {
 
  private:
   ReadbackPool();
+  // One read.  Everything in here is guarded by m_; a piece takes some hundred microseconds.
   struct Job {
     char *host = nullptr;
     size_t bytes = 0;
     long pieces = 0;
     const std::vector<void *> *events = nullptr;
-    std::atomic<long> queued{0}, arrived{0}, next{0}, done{0};  // chunks queued, known to have arrived; pieces taken, carried on
-    std::atomic<long> slot_pieces[kSlots];                      // pieces of this slot carried on so far
-    std::atomic<bool> failed{false};
+    long queued = 0, arrived = 0;         // chunks on their way, chunks known to be in their slots
+    long next = 0, done = 0;              // pieces taken, carried on
+    long slot_pieces[kSlots] = {};        // pieces of this slot carried on so far
+    bool waits = false;                   // somebody waits for chunk `arrived` already
+    bool failed = false;
+    bool can_take() const { return !failed && next < pieces && next / (long)(kSlot / kPiece) < queued; }
   };
-  void work(Job &j, bool caller);
+  void carry(std::unique_lock<std::mutex> &lock, Job &j);
   void thread_main();
 
   std::mutex one_read_;  // the ring serves one read at a time
   std::mutex m_;
-  std::condition_variable wake_, idle_;
-  Job *job_ = nullptr;   // guarded by m_
+  std::condition_variable more_, progress_;  // there may be pieces to take; pieces were carried on, a chunk has arrived
+  Job *job_ = nullptr;
   int inside_ = 0;       // threads that hold job_
   bool stop_ = false;
   PinnedArray<char> ring_;
-  std::vector<std::thread> threads_;
+  std::vector<std::thread> threads_;  // as many as could be had: none is enough
 };
 
 // What one engine or executor reads through.
