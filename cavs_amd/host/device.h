@@ -88,6 +88,11 @@ class PinnedArray {
     p_ = static_cast<T *>(q);
     cap_ = n;
   }
+  void release() {
+    cavs_host_free(p_);
+    p_ = nullptr;
+    cap_ = 0;
+  }
   T *get() const { return p_; }
   size_t capacity() const { return cap_; }
 

@@ -386,7 +386,7 @@ void Engine::get_param(const std::string &name, float *host, size_t n, bool grad
     copy_blocks(jobs);
     src = pad_stage_.get();
   }
-  readback_.read(host, src, n * 4, stream_);
+  readback_.read(host, src, n * 4, stream_, sched_stream_);
   stream_idle();
 }
 
@@ -2729,7 +2729,7 @@ void Engine::fetch(const std::string &what, float *host, size_t n) {
   if (N == 0) fail(CAVS_EINVAL, "no step has run yet");
   if (n != want || !host) fail(CAVS_EINVAL, "'" + what + "' holds " + std::to_string(want) + " floats, got " + std::to_string(n));
   if (blocks > 0) src = user_rows(src, N, blocks);
-  readback_.read(host, src, want * 4, stream_);
+  readback_.read(host, src, want * 4, stream_, sched_stream_);
   stream_idle();
   tail_check();
 }

@@ -929,7 +929,7 @@ long Executor::read_tensor(const std::string &name, float *out, size_t cap) {
   if (e && e->src && e->src->def.name() == "Placeholder" && e->src->def.device() == CPU) return 0;
   size_t n = t->count();
   if (!out || cap < n) return -(long)n;
-  readback_.read(out, t->base, n * 4, stream_);
+  readback_.read(out, t->base, n * 4, stream_, copy_stream_);
   if (engine_) engine_->tail_check();
   return (long)n;
 }

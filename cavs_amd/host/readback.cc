@@ -1,9 +1,12 @@
 #include "readback.h"
 
 #include <algorithm>
+#include <chrono>
+#include <cstdlib>
 #include <cstring>
 #include <string>
 #include <system_error>
+#include <thread>
 
 namespace cavs {
 
@@ -14,38 +17,63 @@ constexpr size_t kPlain = size_t(1) << 20;
 // price of one more wait (one Tree-LSTM sentence, graph_out back: 127 us; 114 with this and the feeds on the
 // idle stream).
 constexpr size_t kSmall = size_t(256) << 10;
-// Threads besides the caller's: a core copies and faults in about 10 GB/s, the link does 55.
-constexpr int kThreads = 11;
+// Threads besides the caller's: a core copies and faults in about 10 GB/s, the link does 55 (89 MB with eleven
+// 2.20 ms, with five 2.23).
+constexpr int kThreads = 5;
+// A plain copy takes about 0.07 ms a megabyte longer: from here on a process has paid what the ring costs.
+constexpr size_t kWorth = size_t(128) << 20;
+// How long the ring stays without anybody attached to it.
+constexpr auto kKeep = std::chrono::seconds(2);
 }  // namespace
 
-std::shared_ptr<ReadbackPool> ReadbackPool::shared() {
-  static std::mutex m;
-  static std::weak_ptr<ReadbackPool> pool;
-  std::lock_guard<std::mutex> lock(m);
-  std::shared_ptr<ReadbackPool> p = pool.lock();
-  if (!p) {
-    p.reset(new ReadbackPool);
-    pool = p;
-  }
-  return p;
+ReadbackPool &ReadbackPool::instance() {
+  static ReadbackPool *pool = [] {
+    auto *p = new ReadbackPool;  // (its threads may outlive every static object)
+    std::atexit([] {
+      ReadbackPool &q = instance();
+      std::lock_guard<std::mutex> lock(q.m_);
+      q.exiting_ = true;
+    });
+    return p;
+  }();
+  return *pool;
 }
 
-ReadbackPool::ReadbackPool() {
-  ring_.reserve(kSlot * kSlots);
+bool ReadbackPool::attach(size_t bytes) {
+  std::lock_guard<std::mutex> lock(m_);
+  if (exiting_) return false;
+  if (ring_.capacity() == 0) {
+    if (plain_ + bytes <= kWorth) {
+      plain_ += bytes;
+      return false;
+    }
+    try {
+      ring_.reserve(kSlot * kSlots);
+    } catch (const Error &) {  // no pinned memory for a ring: a plain copy will do
+      return false;
+    }
+  }
+  users_++;
+  return true;
+}
+
+void ReadbackPool::detach() {
+  std::lock_guard<std::mutex> lock(m_);
+  if (--users_ > 0) return;
+  if (threads_ == 0 && !exiting_) ring_.release();  // (else the threads see to it)
+  more_.notify_all();
+}
+
+// Call with m_ held.  Threads for so many pieces, as far as they can be had.
+void ReadbackPool::staff(long pieces) {
   const int spare = std::max(1, (int)std::thread::hardware_concurrency() - 1);
   try {
-    for (int i = 0; i < std::min(kThreads, spare); i++) threads_.emplace_back([this] { thread_main(); });
-  } catch (const std::system_error &) {  // (no more to be had: those there are and the caller's carry on)
+    while (threads_ < std::min<long>({kThreads, spare, pieces - 1})) {
+      std::thread([this] { thread_main(); }).detach();
+      threads_++;
+    }
+  } catch (const std::system_error &) {
   }
-}
-
-ReadbackPool::~ReadbackPool() {
-  {
-    std::lock_guard<std::mutex> lock(m_);
-    stop_ = true;
-  }
-  more_.notify_all();
-  for (std::thread &t : threads_) t.join();
 }
 
 // Takes one piece on; call with j.can_take().  Pieces are taken in order, and one thread at a time waits for the
@@ -82,14 +110,17 @@ void ReadbackPool::carry(std::unique_lock<std::mutex> &lock, Job &j) {
 void ReadbackPool::thread_main() {
   std::unique_lock<std::mutex> lock(m_);
   for (;;) {
-    more_.wait(lock, [this] { return stop_ || (job_ && job_->can_take()); });
-    if (stop_) return;
+    // (the system's clock: gcc 11's thread sanitizer does not know the wait by the steady one)
+    const bool more = more_.wait_until(lock, std::chrono::system_clock::now() + kKeep, [this] { return job_ && job_->can_take(); });
+    if (!more && users_ > 0) continue;
+    if (!more) break;
     Job &j = *job_;
     inside_++;
     while (j.can_take()) carry(lock, j);
     inside_--;
     progress_.notify_all();
   }
+  if (--threads_ == 0 && !exiting_) ring_.release();
 }
 
 void ReadbackPool::read(char *host, const char *dev, size_t bytes, void *const streams[2], const std::vector<void *> &events) {
@@ -102,6 +133,7 @@ void ReadbackPool::read(char *host, const char *dev, size_t bytes, void *const s
   int rc = CAVS_OK;
   const long chunks = (long)((bytes + kSlot - 1) / kSlot);
   std::unique_lock<std::mutex> lock(m_);
+  staff(j.pieces);
   job_ = &j;
   // (the caller carries pieces on as well, but queueing the next chunk comes first)
   auto work_until = [&](auto over) {
@@ -138,9 +170,10 @@ Readback::~Readback() {
   for (void *e : events_) cavs_event_destroy(e);
   if (begin_) cavs_event_destroy(begin_);
   if (side_) cavs_stream_destroy(side_);
+  if (attached_) ReadbackPool::instance().detach();
 }
 
-void Readback::read(void *host, const void *dev, size_t bytes, void *stream) {
+void Readback::read(void *host, const void *dev, size_t bytes, void *stream, void *second) {
   if (bytes <= kSmall) {
     small_.reserve(bytes < 4096 ? 4096 : 2 * bytes < kSmall ? 2 * bytes : kSmall);
     check(cavs_memcpy_d2h(small_.get(), dev, bytes, stream));
@@ -148,19 +181,12 @@ void Readback::read(void *host, const void *dev, size_t bytes, void *stream) {
     std::memcpy(host, small_.get(), bytes);
     return;
   }
-  if (bytes < kPlain) {
+  ReadbackPool &pool = ReadbackPool::instance();
+  if (bytes >= kPlain && !attached_) attached_ = pool.attach(bytes);
+  if (bytes < kPlain || !attached_) {
     check(cavs_memcpy_d2h(host, dev, bytes, stream));
     check(cavs_stream_sync(stream));
     return;
-  }
-  if (!pool_) {
-    try {
-      pool_ = ReadbackPool::shared();
-    } catch (const Error &) {  // no pinned memory for a ring: a plain copy will do
-      check(cavs_memcpy_d2h(host, dev, bytes, stream));
-      check(cavs_stream_sync(stream));
-      return;
-    }
   }
   while (events_.size() < (size_t)ReadbackPool::kSlots) {
     void *e = nullptr;
@@ -169,13 +195,13 @@ void Readback::read(void *host, const void *dev, size_t bytes, void *stream) {
   }
   void *streams[2] = {stream, stream};
   if (bytes > ReadbackPool::kSlot) {
-    if (!side_) check(cavs_stream_create(&side_));
+    if (!second && !side_) check(cavs_stream_create(&side_));
     if (!begin_) check(cavs_event_create(&begin_));
+    streams[1] = second ? second : side_;
     check(cavs_event_record(begin_, stream));
-    check(cavs_stream_wait_event(side_, begin_));
-    streams[1] = side_;
+    check(cavs_stream_wait_event(streams[1], begin_));
   }
-  pool_->read(static_cast<char *>(host), static_cast<const char *>(dev), bytes, streams, events_);
+  pool.read(static_cast<char *>(host), static_cast<const char *>(dev), bytes, streams, events_);
 }
 
 }  // namespace cavs

@@ -3,16 +3,16 @@
 // which also takes the page faults of a freshly allocated destination: 12 GB/s on one MI355X host, where
 // the link does 55.  Here the link fills a small ring of pinned slots and a few threads carry them on,
 // so that copying and first touch of the destination run beside the transfer and beside each other.
-// One ring and one set of threads per process, made by the first large read and gone with the last
-// object that holds them.
+// One ring and one set of threads per process.  Making them costs some 10 ms (the runtime's first copy to pinned
+// memory alone 6), so they are made once a process has read as much by plain copies as would have paid for them,
+// and sessions that follow each other find them there; some time after the last of these the memory goes back
+// and the threads end.
 #ifndef CAVS_HOST_READBACK_H_
 #define CAVS_HOST_READBACK_H_
 
 #include <condition_variable>
 #include <cstddef>
-#include <memory>
 #include <mutex>
-#include <thread>
 #include <vector>
 
 #include "device.h"
@@ -21,8 +21,11 @@ namespace cavs {
 
 class ReadbackPool {
  public:
-  static std::shared_ptr<ReadbackPool> shared();
-  ~ReadbackPool();
+  static ReadbackPool &instance();  // (lives until the process ends)
+  // Who reads through the pool attaches to it first: false where a plain copy is the better choice so far, `bytes`
+  // being what the caller is about to read.
+  bool attach(size_t bytes);
+  void detach();
   // `events`: one per slot, of the device the stream belongs to
   void read(char *host, const char *dev, size_t bytes, void *const streams[2], const std::vector<void *> &events);
   // Four megabytes per slot, carried on in pieces of one: a copy and its event cost about 15 us besides the
@@ -32,7 +35,7 @@ class ReadbackPool {
   static constexpr int kSlots = 8;
 
  private:
-  ReadbackPool();
+  ReadbackPool() = default;
   // One read.  Everything in here is guarded by m_; a piece takes some hundred microseconds.
   struct Job {
     char *host = nullptr;
@@ -48,26 +51,30 @@ class ReadbackPool {
   };
   void carry(std::unique_lock<std::mutex> &lock, Job &j);
   void thread_main();
+  void staff(long pieces);
 
   std::mutex one_read_;  // the ring serves one read at a time
   std::mutex m_;
   std::condition_variable more_, progress_;  // there may be pieces to take; pieces were carried on, a chunk has arrived
   Job *job_ = nullptr;
   int inside_ = 0;       // threads that hold job_
-  bool stop_ = false;
+  int threads_ = 0;      // as many as could be had: none is enough
+  int users_ = 0;        // who has attached
+  size_t plain_ = 0;     // bytes of large reads that went by plain copies
+  bool exiting_ = false; // the process is on its way out: no more calls into the runtime
   PinnedArray<char> ring_;
-  std::vector<std::thread> threads_;  // as many as could be had: none is enough
 };
 
 // What one engine or executor reads through.
 class Readback {
  public:
   ~Readback();
-  // `bytes` of `dev` are at `host` when this returns; waits for what `stream` holds before it.
-  void read(void *host, const void *dev, size_t bytes, void *stream);
+  // `bytes` of `dev` are at `host` when this returns; waits for what `stream` holds before it.  `second`: another
+  // stream of the caller's with nothing on it (null: large reads make one; a stream more costs up to 3 ms).
+  void read(void *host, const void *dev, size_t bytes, void *stream, void *second);
 
  private:
-  std::shared_ptr<ReadbackPool> pool_;
+  bool attached_ = false;
   std::vector<void *> events_;
   void *side_ = nullptr, *begin_ = nullptr;  // every other chunk of a large read
   PinnedArray<char> small_;

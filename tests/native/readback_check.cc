@@ -4,6 +4,7 @@
 #include <dlfcn.h>
 #include <pthread.h>
 
+#include <atomic>
 #include <cerrno>
 #include <chrono>
 #include <condition_variable>
@@ -82,6 +83,7 @@ struct Event {
 };
 std::mutex g_m;
 long g_fail_copy = -1, g_fail_sync = -1, g_fail_alloc = 0;  // countdown to the call that fails (-1: none)
+std::atomic<long> g_pinned{0};  // allocations of pinned memory that stand
 bool counts_down(long &n) {
   std::lock_guard<std::mutex> lock(g_m);
   return n >= 0 && n-- == 0;
@@ -98,9 +100,11 @@ const char *cavs_last_error(void) { return "told to fail"; }
 int cavs_host_alloc(void **p, size_t n) {
   if (g_fail_alloc) return CAVS_ENOMEM;
   *p = std::malloc(n);
+  g_pinned++;
   return CAVS_OK;
 }
 int cavs_host_free(void *p) {
+  if (p) g_pinned--;
   std::free(p);
   return CAVS_OK;
 }
@@ -174,7 +178,8 @@ bool reads(cavs::Readback &r, size_t n, unsigned seed) {
   Stream s;
   const std::vector<char> dev = pattern(n, seed);
   std::vector<char> host(n, 1);
-  r.read(host.data(), dev.data(), n, &s);
+  Stream second;
+  r.read(host.data(), dev.data(), n, &s, seed & 1 ? &second : nullptr);
   return host == dev;
 }
 bool fails(cavs::Readback &r, size_t n) {
@@ -191,7 +196,10 @@ int main(int argc, char **argv) {
   const size_t M = size_t(1) << 20;
   g_fail_alloc = ringless;
   g_no_threads = threadless;
+  {
   cavs::Readback a, b;
+  expect(reads(a, 100 * M + 8, 2) && g_pinned == 0, "plain copies first");
+  expect(reads(a, 30 * M, 2) && g_pinned == (ringless ? 0 : 1), "the ring when it would have paid");
   if (!ringless) {
     expect(reads(a, 1, 1) && reads(a, 100, 1) && reads(a, 256 << 10, 2), "small");
   }
@@ -215,11 +223,14 @@ int main(int argc, char **argv) {
     set(-1, -1);
     expect(reads(a, 37 * M, 60), "and a read after it");
   }
-  if (!threadless) {  // the last reader goes, the next one starts afresh
-    for (int i = 0; i < 3; i++) {
-      cavs::Readback c;
-      expect(reads(c, 9 * M, 70 + i), "a reader of its own");
-    }
+  for (int i = 0; i < 3; i++) {
+    cavs::Readback c;
+    expect(reads(c, 9 * M, 70 + i), "a reader of its own");
   }
+  }
+  for (int i = 0; i < 300 && g_pinned > 0; i++) std::this_thread::sleep_for(std::chrono::milliseconds(20));
+  expect(g_pinned == 0, "the ring goes back when nobody reads any more");
+  cavs::Readback d;
+  expect(reads(d, 40 * M, 80) && g_pinned == 1, "and comes again");
   return 0;
 }
