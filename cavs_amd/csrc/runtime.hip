@@ -170,6 +170,12 @@ int cavs_device_name(char *buf, size_t len) {
   return CAVS_OK;
 }
 
+int cavs_device_bus_id(int device, char *buf, size_t len) {
+  CAVS_REQUIRE(buf && len >= 13, "cavs_device_bus_id: a buffer of 13 bytes needed");
+  CAVS_HIP_TRY(hipDeviceGetPCIBusId(buf, (int)len, device));
+  return CAVS_OK;
+}
+
 int cavs_malloc(void **ptr, size_t bytes) {
   CAVS_REQUIRE(ptr, "cavs_malloc: null out pointer");
   *ptr = nullptr;

@@ -60,6 +60,7 @@ class GroupPlan(C.Structure):
 _SIGS = {
     "cavs_init": [_I],
     "cavs_device_name": [C.c_char_p, _Z],
+    "cavs_device_bus_id": [_I, C.c_char_p, _Z],
     "cavs_malloc": [C.POINTER(_P), _Z],
     "cavs_free": [_P],
     "cavs_host_alloc": [C.POINTER(_P), _Z],

@@ -144,7 +144,7 @@ const float *Engine::user_rows(const float *src, size_t n, int blocks) {
 void Engine::tail_setup() {
   static std::mutex m;
   static std::map<int, bool> known;
-  tail_ready_ = false;
+  tail_ready_ = probe_due_ = false;
   if (cell_ || !(cfg_.opt & CAVS_OPT_BATCHING) || cfg_.tail_rows < 0 || !cavs_group_rounds_ok(cfg_.H)) return;
   const size_t words = cavs_tail_sync_bytes() / sizeof(int);
   tail_sync_.reserve(words);
@@ -152,10 +152,13 @@ void Engine::tail_setup() {
   std::lock_guard<std::mutex> lock(m);
   auto it = known.find(cfg_.device);
   if (it == known.end()) {
+    probe_due_ = !claim_.take(cfg_.device);  // (beside another process's launches it would say nothing: a later step asks)
+    if (probe_due_) return;
     check(cavs_tail_probe(reinterpret_cast<unsigned *>(tail_sync_.get()), 512, kTailSpins, stream_));
     int head[4] = {0, 0, 0, 0};
     check(cavs_memcpy_d2h(head, tail_sync_.get(), sizeof(head), stream_));
     check(cavs_stream_sync(stream_));
+    claim_.give();
     it = known.emplace(cfg_.device, head[1] == 0).first;
     if (!it->second) check(cavs_zero(tail_sync_.get(), words * sizeof(int), stream_));
   }
@@ -163,7 +166,7 @@ void Engine::tail_setup() {
 }
 
 int Engine::tail_limit() const {
-  if (!tail_ready_ || fused_rows() <= 0 || cfg_.model != CAVS_MODEL_TREELSTM || !cavs_tail_rounds_ok(1, cfg_.H)) return 0;
+  if (!resident_ || fused_rows() <= 0 || cfg_.model != CAVS_MODEL_TREELSTM || !cavs_tail_rounds_ok(1, cfg_.H)) return 0;
   // a round whose rows are dealt so that some group gets more than this stays a launch of its own
   // (the launches take a group's share of a round in slices of at most 32 rows).  64 takes in every
   // round above the leaves of a batch of 64 parse trees: measured 0.363 ms per step against 0.366
@@ -173,7 +176,7 @@ int Engine::tail_limit() const {
 
 // A group takes a round of up to this many rows (in slices of 32); larger rounds are launches of their own.
 int Engine::group_limit() const {
-  if (!tail_ready_ || fused_rows() <= 0 || cell_ || !cavs_group_rounds_ok(cfg_.H)) return 0;
+  if (!resident_ || fused_rows() <= 0 || cell_ || !cavs_group_rounds_ok(cfg_.H)) return 0;
   if (cfg_.model == CAVS_MODEL_TREELSTM && cavs_tail_rounds_ok(1, cfg_.H)) return 0;  // (the tail launches are tuned for that size)
   return cfg_.tail_rows > 0 ? cfg_.tail_rows : 64;
 }
@@ -223,6 +226,7 @@ void Engine::build_tail_plan(const int *kid_rows, int *rows_out) {
 }
 
 void Engine::tail_check() {
+  claim_.give();
   if (!tail_pending_) return;
   tail_pending_ = false;
   int words[4] = {0, 0, 0, 0};
@@ -388,6 +392,7 @@ void Engine::get_param(const std::string &name, float *host, size_t n, bool grad
   }
   readback_.read(host, src, n * 4, stream_, sched_stream_);
   stream_idle();
+  tail_check();
 }
 
 // ------------------------------------------------------------------ profiling
@@ -1055,6 +1060,8 @@ void Engine::begin_step(const int *graph, int B, int maxlen) {
     hit = find_plan(graph, B, maxlen, hash);
   }
   hit_plan_ = hit;
+  if (probe_due_) tail_setup();
+  resident_ = tail_ready_ && fused_rows() > 0 && claim_.take(cfg_.device);
   if (hit) {
     // a batch structure seen before: its schedule and its lists are where the last such step left them
     hit->last_used = ++plan_clock_;
@@ -1092,7 +1099,7 @@ void Engine::begin_step(const int *graph, int B, int maxlen) {
     scheduler_used_ = on_device ? 1 : 0;
     if (cfg_.plan_cache > 0) {
       c_plan_misses_ += 1;
-      remember_plan(graph, B, maxlen, hash);
+      if (resident_ || !(tail_ready_ || probe_due_)) remember_plan(graph, B, maxlen, hash);  // (else its rounds would stay launches of their own)
     }
   }
   reserve_edges();
@@ -1195,6 +1202,7 @@ Engine::StepSig Engine::step_signature(const void *x, const void *labels, bool b
   g.xs = xs_.get();
   g.xs_prev = xs_prev_.get();
   g.backward = backward;
+  g.resident = resident_;
   g.emb_sparse_valid = emb_sparse_valid_;
   g.emb_cleared = emb_cleared_;
   g.upk_valid = upk_valid_;

@@ -18,6 +18,7 @@
 #include "cell.h"
 #include "device.h"
 #include "readback.h"
+#include "resident.h"
 #include "scheduler.h"
 
 namespace cavs {
@@ -291,12 +292,12 @@ class Engine {
   // state it left is then put in place as if the launches had been issued one by one.
   struct StepSig {
     const void *x = nullptr, *labels = nullptr, *xs = nullptr, *xs_prev = nullptr;
-    bool backward = false, emb_sparse_valid = false, emb_cleared = false, upk_valid = false, wfct_valid = false;
+    bool backward = false, resident = false, emb_sparse_valid = false, emb_cleared = false, upk_valid = false, wfct_valid = false;
     int emb_dirty_n = 0, pairing = 0;
     size_t e_ones_rows = 0;
     uint64_t alloc_epoch = 0, state_epoch = 0;
     bool operator==(const StepSig &o) const {
-      return x == o.x && labels == o.labels && xs == o.xs && xs_prev == o.xs_prev && backward == o.backward &&
+      return x == o.x && labels == o.labels && xs == o.xs && xs_prev == o.xs_prev && backward == o.backward && resident == o.resident &&
              emb_sparse_valid == o.emb_sparse_valid && emb_cleared == o.emb_cleared && upk_valid == o.upk_valid &&
              wfct_valid == o.wfct_valid && emb_dirty_n == o.emb_dirty_n && pairing == o.pairing && e_ones_rows == o.e_ones_rows &&
              alloc_epoch == o.alloc_epoch && state_epoch == o.state_epoch;
@@ -444,6 +445,9 @@ class Engine {
   const int *d_tail_rows_ = nullptr;
   DeviceArray<int> tail_sync_;  // the launches' sync block
   bool tail_ready_ = false;     // the device ran the probe's workgroups all at once, each group on one XCD
+  bool probe_due_ = false;      // nobody could ask yet: another process was at it
+  bool resident_ = false;       // this step may launch them: no other process is at it
+  ResidentClaim claim_;
   bool tail_pending_ = false;   // a tail launch was enqueued since the status word was last read
   double c_tail_rounds_ = 0, c_tail_launches_ = 0;
   int tail_limit() const;       // rows per group and round a tail launch may take (0: no tail launches)
@@ -452,7 +456,7 @@ class Engine {
   // the children-by-slab-row lists of a batch whose message flow is a forest
   void build_tail_plan(const int *kid_rows, int *rows_out);
  public:
-  // After the stream has drained: reads the status word of the tail launches.  A launch that gave
+  // After the stream has drained: gives the claim back and reads the status word of the tail launches.  A launch that gave
   // up leaves the results of the steps since undefined (their parameter updates were skipped: they
   // watch the word); the session goes on with one launch per round and this call fails.
   void tail_check();

@@ -45,6 +45,7 @@ int cavs_abi_version(void);
  * (cavs/util/stream_event_handle_pool.h:8-65) and Timing (cavs/util/timing.h:10-67). */
 int cavs_init(int device);
 int cavs_device_name(char *buf, size_t len);
+int cavs_device_bus_id(int device, char *buf, size_t len); /* PCI bus id, as in 0000:05:00.0 */
 int cavs_malloc(void **ptr, size_t bytes);
 int cavs_free(void *ptr);
 int cavs_host_alloc(void **ptr, size_t bytes); /* pinned host memory */

@@ -66,15 +66,20 @@ typedef struct {
    * graph feeds, keyed by the feed's bytes; a step on a feed seen before skips the scheduler and
    * the upload.  0 = off. */
   int plan_cache;
-  /* Tree-LSTM, H = 512, batches whose message flow is a forest: the rounds from the first one on
-   * whose rows can be dealt to eight groups, whole trees of the message flow per group, with at
-   * most this many rows per group (the last forward rounds, the first backward rounds) run as one launch per
-   * direction (cavs_treelstm_tail_fwd / _bwd) instead of one launch per round
-   * (cavs/midend/statement.cc:69-76,106-111).  0 = default (64, which at 64 trees per batch takes in
-   * every round above the leaves; a group's share of a round runs in slices of at most 32 rows),
-   * negative = never.  The session
-   * checks once, when it is created, that the device runs such a launch's workgroups all at once,
-   * each group on one XCD, and keeps to one launch per round if not. */
+  /* Hidden sizes up to 512 (as stored: in whole tiles of 32), batches whose message flow is a forest: the
+   * rounds from the first one on whose rows can be dealt to groups of workgroups, whole trees of the
+   * message flow per group, with at most this many rows per group (the last forward rounds, the first
+   * backward rounds) run as one launch per direction (cavs_treelstm_tail_fwd / _bwd, cavs_*_group_fwd /
+   * _bwd) instead of one launch per round (cavs/midend/statement.cc:69-76,106-111).  0 = default (64; a
+   * group's share of a round runs in slices of at most 32 rows), negative = never.
+   * Such a launch needs all its workgroups on the GPU at once.  The session checks once, when it is created,
+   * that the device runs them so, each group on one XCD, and keeps to one launch per round if not.  Among
+   * sessions of one process the launches are put in order.  Among processes that share a GPU, one at a time
+   * uses them: it holds an advisory lock from its first such step until it has waited for its work
+   * (cavs_session_sync, _fetch, _get_param), and the others' steps run one launch per round
+   * meanwhile.  Programs that keep workgroups of their own resident know nothing of the lock: a launch
+   * that waits for room beyond its bound gives up, the parameters stay those of the last good step, and the
+   * next call that waits for the session fails; with such a program on the GPU use a negative value. */
   int tail_rows;
   /* With a plan cache: 1 = a step on a batch structure seen before, with the same input buffers
    * (inputs_on_device) and the session in the same state as the last time, enqueues its forward

@@ -1,0 +1,130 @@
+"""Launches that keep all their workgroups on the GPU: sessions of one process are put in order, processes that share
+a GPU take turns."""
+import contextlib
+import ctypes as C
+import fcntl
+import subprocess
+import sys
+import threading
+
+import numpy as np
+import pytest
+
+from cavs_amd import hip, session, synth
+from test_oracle_models import small_workload
+from tolerance import close
+
+pytestmark = pytest.mark.gpu
+
+
+@contextlib.contextmanager
+def another_process():
+    """Holds the lock as another process would: by a file description of its own."""
+    hip.call("cavs_init", 0)
+    bus = C.create_string_buffer(32)
+    hip.call("cavs_device_bus_id", 0, bus, 32)
+    with open(f"/sys/bus/pci/devices/{bus.value.decode().lower()}/vendor") as f:
+        fcntl.flock(f, fcntl.LOCK_EX | fcntl.LOCK_NB)
+        yield
+        fcntl.flock(f, fcntl.LOCK_UN)
+
+
+def _session(model, H, w, **kw):
+    if model == "treefc":
+        kw.update(loss="root_sq", act=1, use_bias=True, use_x=True)
+    s = session.Session(model, H=H, E=12 if model == "treelstm" else H, V=31, C_=5, **kw)
+    # (W from U(-0.4, 0.4) times this: a level of a Tree-FC tree multiplies the differences in its inputs by about
+    # 0.4 / sqrt(3) times this times sqrt(2 H), 0.65 with the second form at every H, 1.3 at H = 256 with the first)
+    spread = np.float32(0.25 * np.sqrt(64 / H) if model == "treefc" else 0.25)
+    s.set_params({k: v * spread if k == "W" else v for k, v in w["params"].items() if model != "treefc" or not k.endswith("fc")})
+    return s
+
+
+@pytest.mark.parametrize("models", [(("treelstm", 512), ("lstm", 512)), (("treelstm", 512), ("treelstm", 512)), (("treefc", 256), ("lstm", 96))])
+def test_sessions_on_threads_and_streams_of_their_own(models):
+    """Two sessions train at a time, each on a thread and a stream of its own; every launch of either wants the whole
+    GPU.  Each gives what it gives alone."""
+    ws = [small_workload(m, 90 + i, B=60, H=H, E=12, V=31, C=5) for i, (m, H) in enumerate(models)]
+
+    def train(i, out):
+        (m, H), w = models[i], ws[i]
+        s = _session(m, H, w)
+        for k in range(30):
+            s.step(w["graph"], w["x"], w["labels"], backward=True, lr=1e-4 if m == "treefc" else 1e-2)
+            if k % 7 == i:
+                s.sync()
+        assert s.counter("tail_rounds") > 0
+        out[i] = dict(loss=s.fetch("loss"), go=s.fetch("graph_out"), **s.grads())
+        s.close()
+
+    alone, together = [None, None], [None, None]
+    for i in range(2):
+        train(i, alone)
+    threads = [threading.Thread(target=train, args=(i, together)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for a, b in zip(alone, together):
+        for k in a:
+            close(b[k], a[k], k)
+
+
+@pytest.mark.parametrize("model,H,kw", [("treelstm", 512, {}), ("lstm", 128, {}), ("treefc", 256, dict(plan_cache=4, graph_replay=True)),
+                                        ("treelstm", 96, dict(plan_cache=4)), ("treelstm", 64, dict(schedule="device"))])
+def test_while_another_process_is_at_it_rounds_are_launches_of_their_own(model, H, kw):
+    import torch
+
+    w = small_workload(model, 12, B=50, H=H, E=12, V=31, C=5)
+    feed = (w["graph"], torch.from_numpy(np.ascontiguousarray(w["x"], np.float32)).cuda(), torch.from_numpy(w["labels"]).cuda())
+    torch.cuda.synchronize()
+    s, plain = _session(model, H, w, **kw), _session(model, H, w, tail_rows=-1)
+    free = contextlib.nullcontext
+    # (the gradients of the sum of squares reach the tens: steps of 1e-2 would take W where the bound above no longer holds)
+    lr = 1e-4 if model == "treefc" else 1e-2
+    for k, turn in enumerate((another_process, another_process, free, free, free, another_process, free, free)):
+        with turn():
+            for one in (s, plain):
+                one.step(*feed, backward=True, lr=lr)
+            assert (s.counter("tail_rounds") > 0) == (turn is free), k
+            for what in ("loss", "graph_out"):
+                close(s.fetch(what), plain.fetch(what), what)
+    for k, v in plain.grads().items():
+        close(s.grads()[k], v, k)
+    if "graph_replay" in kw:
+        assert s.counter("graph_replays") > 0
+    s.step(*feed, backward=True, lr=0.0)  # from here until somebody waits the lock is this process's
+    with pytest.raises(BlockingIOError):
+        with another_process():
+            pass
+    s.sync()
+    with another_process():
+        pass
+    s.close()
+    plain.close()
+
+
+def test_a_session_made_while_another_process_is_at_it():
+    """The device is asked once per process whether it runs such launches; a session made while that cannot be asked
+    asks later.  In a process of its own, since this one has asked."""
+    code = """
+import sys
+sys.path[:0] = sys.argv[1:]
+from test_gpu_resident import another_process, _session, small_workload
+w = small_workload("lstm", 12, B=50, H=64, E=12, V=31, C=5)
+with another_process():
+    s = _session("lstm", 64, w)
+    s.step(w["graph"], w["x"], w["labels"], backward=True, lr=1e-2)
+    s.sync()
+    assert s.counter("tail_rounds") == 0 and s.counter("tail_ready") == 0
+s.step(w["graph"], w["x"], w["labels"], backward=True, lr=1e-2)
+s.sync()
+assert s.counter("tail_rounds") > 0 and s.counter("tail_ready") == 1
+print("done")
+"""
+    import os
+
+    here = os.path.dirname(os.path.abspath(__file__))
+    r = subprocess.run([sys.executable, "-c", code, os.path.dirname(here), here, os.path.join(os.path.dirname(here), "oracle")], capture_output=True,
+                       text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.endswith("done\n"), r.stdout + r.stderr
