@@ -2624,9 +2624,13 @@ void Engine::plan_head_chunks(const int *orphans_host) {
   if (cfg_.head_chunks < 0 || cfg_.model != CAVS_MODEL_LSTM || !wide_head() || !s.batching || !forest_ || cfg_.graph_replay || R < 8 ||
       N < 256)
     return;
-  // Where the rounds are one launch per direction, a head whose products fill the chip by themselves runs in
-  // one piece: beside them the rounds take three times as long (C4: 3.32 ms per step, in one piece 3.26).
-  if (cfg_.head_chunks == 0 && group_.first >= 0 && (double)N * cfg_.C >= 512.0 * 128 * 128) return;
+  // Where the rounds are one launch per direction, chunks cost more than they cover: the backward rounds become
+  // launches of their own again, and the forward launch keeps the chip to itself.  Of 54 sessions (H = 128, 256,
+  // 512, 1012 to 9765 vertices in chains of 20 to 200, 2200 to 12000 classes) one piece is faster in 52, by 5 to 71 %
+  // (1012 vertices of 10 .. 100, H = 256, 5000 classes: 0.56 ms against 0.87; C4 2.89 against 2.88), and as fast in
+  // the others; H = 96 the same, 5 to 58 %.  Up to H = 64, where a step takes 0.25 to 0.5 ms either way (0.24 against
+  // 0.30, 0.42 against 0.46), small heads keep the two chunks that 0 stands for.
+  if (cfg_.head_chunks == 0 && group_.first >= 0 && (cfg_.H > 64 || (double)N * cfg_.C >= 512.0 * 128 * 128)) return;
   const int K = cfg_.head_chunks > 0 ? std::min(cfg_.head_chunks, (int)kHeadChunks) : 2;
   int k = 0;
   for (int c = 0; c < K; c++) {

@@ -94,8 +94,9 @@ typedef struct {
    * scheduler, message flow a forest: the head runs over chunks of the rounds on a second stream
    * beside the backward rounds (cavs/midend/statement.cc:69-76,106-111 run them one
    * after the other): the chunks last first, each one's d h releasing the backward rounds of its
-   * rows while the next chunk's is computed.  0 = default (two chunks), 2..4 = that many, negative =
-   * off: the head in one piece between the two passes.  The counter "head_chunks" says in how many
+   * rows while the next chunk's is computed.  0 = default (two chunks; in one piece beside rounds that
+   * are one launch per direction, except for small heads up to H = 64), 2..4 = that many, negative = off:
+   * the head in one piece between the two passes.  The counter "head_chunks" says in how many
    * chunks the last step's head ran (0: in one piece). */
   int head_chunks;
 } cavs_session_config;

@@ -785,3 +785,25 @@ def test_a_device_feed_written_on_the_sessions_stream_is_read_behind_that(model,
     np.testing.assert_array_equal(out[0][0], out[1][0])
     for k in params:
         np.testing.assert_array_equal(out[0][1][k], out[1][1][k], err_msg=k)
+
+
+@pytest.mark.parametrize("H,V,chunks", [(96, 3000, 0), (256, 1100, 0), (544, 600, 2)])
+def test_in_how_many_pieces_a_wide_head_runs_by_default(H, V, chunks):
+    """One piece beside rounds that are one launch per direction, two chunks beside rounds that are launches of their own
+    (H above 512); the results are those of the other way."""
+    graph, lens, rng = synth.chain_batch(7, 24, 8, 40, 40)
+    N = sum(lens)
+    x, labels = np.floor(rng.bulk_uniform(N) * V).astype(np.float32), np.floor(rng.bulk_uniform(N) * V).astype(np.float32)
+    r = 2.0 / np.sqrt(H)
+    u = lambda *s: rng.bulk_uniform(int(np.prod(s)), -r, r).reshape(s).astype(np.float32)  # noqa: E731
+    params = dict(Emb=u(V, H), W=u(8 * H * H), Bv=u(4 * H), Wfc=u(V, H), bfc=u(V))
+    out = []
+    for hc in (0, -1 if chunks else 2):
+        s = session.Session("lstm", H=H, E=H, V=V, C_=V, head_chunks=hc)
+        s.set_params(params)
+        s.step(graph, x, labels, backward=True, lr=0.1)
+        assert s.counter("head_chunks") == (chunks if hc == 0 else max(hc, 0))
+        out.append(dict(loss=s.fetch("loss"), **{k: s.param(k, v.shape) for k, v in params.items()}))
+        s.close()
+    for k in out[0]:
+        close(out[0][k], out[1][k].astype(np.float64), k)
