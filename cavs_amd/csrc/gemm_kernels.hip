@@ -322,11 +322,12 @@ static GemmPlan plan_gemm(int tA, int tB, int M, int N, int K, bool skinny_allow
   // A CU holds two or three workgroups of the large tile; from two per CU on it is the faster one (4700 x 2048 x
   // 300, 592 tiles: 44.6 us against 49.8; 2368 rows, 304 tiles: 31.1 against 27.3).
   if (large_ok && t128 >= 2 * cus) return split(GemmPlan::TILE128, t128, 1);
-  // Fewer large tiles: K is split until about two share a CU -- what one holds beyond 512 of K (gemm_split.h) -- if
-  // that leaves each split at least 512 of K (4000 x 1024 x 3072: 150 us against 170 on the small tile; TN 1024 x 4096
-  // x 73000 3402 us against 3499 for three a CU, 512 x 2048 x 7088 92 against 97).
+  // Fewer large tiles: K is split until about three share a CU, if that leaves each split at least 512 of K
+  // (4000 x 1024 x 3072: 150 us against 170 on the small tile).  (A CU holds two of them beyond 512 of K,
+  // gemm_split.h.  Splits for two are 1 to 6 % faster -- TN 1024 x 4096 x 73000 3421 us against 3462, 512 x 2048 x
+  // 7088 94 against 98.5 -- but the size of the partials decides what cavs_sgemm_splitk_static refuses.)
   if (large_ok && allow_split && 4 * t128 >= cus && K >= 2048) {
-    long s = (2 * cus + t128 - 1) / t128;
+    long s = (3 * cus + t128 - 1) / t128;
     // one or two more splits when they even out the workgroups per CU; ties keep the fewer splits
     // (less partial traffic)
     auto fill = [&](long sp) {
