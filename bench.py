@@ -27,10 +27,13 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0      # MI355X HBM3E
 FP32_MFMA_PEAK_TF = 157.3  # MI355X dense FP32 matrix
+# An fp32 product on the bf16 matrix pipe is six bf16 products (cavs_amd/csrc/gemm_split.h): a sixth of the dense bf16 peak
+SPLIT_MFMA_PEAK_TF = 2516.6 / 6
+MFMA_PEAK_TF = {"gemm": SPLIT_MFMA_PEAK_TF, "round": FP32_MFMA_PEAK_TF}
 # (workload, kernel class) -> HBM bytes per dispatch, from profiles/bench_<workload>_hbm_traffic_pmc.txt
-PMC_TRAFFIC_BYTES = {("C3", "gemm"): 82.05e6, ("C3", "round"): 98.59e6, ("C1", "gemm"): 3.35e6, ("C1", "round"): 0.96e6,
-                     ("C2", "gemm"): 17.11e6, ("C2", "round"): 4.05e6, ("C4", "gemm"): 299.6e6, ("C4", "round"): 10.55e6,
-                     ("C5", "gemm"): 918.6e6, ("C5", "round"): 125.4e6}
+PMC_TRAFFIC_BYTES = {("C3", "gemm"): 76.99e6, ("C3", "round"): 98.64e6, ("C1", "gemm"): 3.17e6, ("C1", "round"): 4.94e6,
+                     ("C2", "gemm"): 17.2e6, ("C2", "round"): 19.04e6, ("C4", "gemm"): 317.3e6, ("C4", "round"): 289.3e6,
+                     ("C5", "gemm"): 335.6e6, ("C5", "round"): 118.9e6}
 # a constant taken from the profile named, not a counter read during this run
 PMC_TRAFFIC_SOURCE = {k: f"profiles/bench_{k[0]}_hbm_traffic_pmc.txt (two rocprofv3 --pmc runs of this command, FETCH_SIZE and "
                          "WRITE_SIZE per dispatch of the class; a constant copied from there, not read in this run)"
@@ -295,14 +298,14 @@ def measure(a, workload, steps, warmup, n_pool, schedule="host", plan_cache=0, p
     # the two MFMA-bound kernel classes; the roofline entry describes whichever takes more device time
     mfma = {
         "gemm": dict(ms=gemm_ms, n=gemm_n, flops=flops,
-                     kernel="sgemm_mfma_kernel / sgemm_skinny_kernel (x*W, weight-gradient and head GEMMs of a step"
+                     kernel="sgemm_split_kernel / sgemm_group_kernel / sgemm_skinny_kernel (x*W, weight-gradient and head GEMMs of a step"
                             "; also the recurrent products of rounds too large for the fused kernels)"),
         "round": dict(ms=round_ms, n=round_n, flops=rflops,
-                      kernel={"treelstm": "treelstm_round_fwd_kernel / treelstm_round_bwd_children_kernel / treelstm_tail_fwd_kernel / "
-                                          "treelstm_tail_bwd_kernel (the rounds near the roots: one launch per direction)",
-                              "lstm": "lstm_round_fwd_kernel / round_bwd_children_kernel",
-                              "treefc": "treefc_round_fwd_kernel / round_bwd_children_kernel"}[w0["model"]] +
-                             " (one launch per round: gather + recurrent products + gates + scatter)"),
+                      kernel={"treelstm": "treelstm_tail_fwd_kernel / treelstm_tail_bwd_kernel (H = 512) / group_fwd_kernel / group_bwd_kernel / "
+                                          "treelstm_round_fwd_kernel / treelstm_round_bwd_children_kernel",
+                              "lstm": "group_fwd_kernel / group_bwd_kernel / lstm_round_fwd_kernel / round_bwd_children_kernel",
+                              "treefc": "group_fwd_kernel / group_bwd_kernel / treefc_round_fwd_kernel / round_bwd_children_kernel"}[w0["model"]] +
+                             " (gather + recurrent products + gates + scatter of a round; up to H = 512 all rounds in one launch per direction)"),
     }
     for v in mfma.values():
         v["tf"] = v["flops"] / (v["ms"] * 1e-3) / 1e12 if v["ms"] else 0.0
@@ -327,15 +330,15 @@ def measure(a, workload, steps, warmup, n_pool, schedule="host", plan_cache=0, p
                    "feeds": "pageable host memory, copied every step" if a.host_feeds else "resident in HBM",
                    "rounds_last_batch": rounds, "launches_last_batch": launches, "loss_head_chunks": head_chunks,
                    "untimed_settle_steps": settle},
-        "roofline": {"bound": "mfma", "achieved": round(dom["tf"], 3), "peak": FP32_MFMA_PEAK_TF,
-                     "unit": "TFLOP/s", "frac": round(dom["tf"] / FP32_MFMA_PEAK_TF, 5), "traffic": traffic,
+        "roofline": {"bound": "mfma", "achieved": round(dom["tf"], 3), "peak": round(MFMA_PEAK_TF[dom_name], 1),
+                     "unit": "TFLOP/s", "frac": round(dom["tf"] / MFMA_PEAK_TF[dom_name], 5), "traffic": traffic,
                      "traffic_source": PMC_TRAFFIC_SOURCE.get((workload, dom_name)) if traffic else None,
                      "kernel": dom["kernel"],
                      "avg_launch_us": round(1e3 * dom["ms"] / dom["n"], 3) if dom["n"] else None,
                      "flops_per_launch": round(dom["flops"] / dom["n"], 1) if dom["n"] else None},
         "kernels": {
-            **{k: {"bound": "mfma", "achieved": round(v["tf"], 3), "peak": FP32_MFMA_PEAK_TF, "unit": "TFLOP/s",
-                   "frac": round(v["tf"] / FP32_MFMA_PEAK_TF, 4),
+            **{k: {"bound": "mfma", "achieved": round(v["tf"], 3), "peak": round(MFMA_PEAK_TF[k], 1), "unit": "TFLOP/s",
+                   "frac": round(v["tf"] / MFMA_PEAK_TF[k], 4),
                    "avg_launch_us": round(1e3 * v["ms"] / max(v["n"], 1), 3), "launches_per_step": round(v["n"] / steps, 1)}
                for k, v in mfma.items()},
             # of the GEMM class's flops (2*M*N*K of the reference's products): the share that multiplies blocks
@@ -384,10 +387,11 @@ def main():
     ap.add_argument("--fused-round-rows", type=int, default=0,
                     help="rounds of at most this many vertices run as fused launches (0: default limit, -1: never)")
     ap.add_argument("--tail-rows", type=int, default=0,
-                    help="Tree-LSTM, H = 512: rounds whose rows can be dealt to eight groups with at most this many rows each run "
+                    help="H up to 512: rounds whose rows can be dealt to groups of workgroups with at most this many rows each run "
                          "inside one launch per direction (0: default limit, -1: one launch per round)")
     ap.add_argument("--head-chunks", type=int, default=0,
-                    help="the loss head of a wide classifier (C4): 0 = in two chunks beside the backward rounds, 2..4 = in that many, negative = in one piece between the two passes")
+                    help="the loss head of a wide classifier (C4): 0 = in one piece beside rounds that are one launch per direction, else in two chunks "
+                         "beside the backward rounds, 2..4 = in that many, negative = in one piece between the two passes")
     ap.add_argument("--also", default="C1,C2,C4,C5",
                     help="further workloads measured with few steps and reported under 'also' (C5 is the large "
                          "Tree-LSTM configuration, where rounds are GEMM-sized); 'none' to skip")

@@ -692,19 +692,19 @@ void Engine::words_forward(const float *W, int w, int leaf_w) {
   const int N = N_, lp = leaf_w < w ? sched_->leaf_prefix : 0;
   words_index(lp);
   {
-    ProfScope ps(this, K_GATHER);
+    ProfScope ps(this, K_OTHER);
     check(cavs_embed_words(e_.get(), ld_e_, d_words_index_, param("Emb").w, N, E_, stream_));
   }
   gemm_group({{0, 0, N, w, E_, 1.f, 0.f, e_.get(), ld_e_, W, w, xW_words_.get(), w, lp > 0 ? CAVS_GEMM_C_UNUSED : 0, lp, leaf_w, d_words_index_,
                words_expected(), pad_block(), uH_}});
-  ProfScope ps(this, K_GATHER);
+  ProfScope ps(this, K_OTHER);
   check(cavs_spread_rows(xW_.get(), w, xW_words_.get(), w, d_words_index_, N, w, lp, leaf_w, word_ids_.get(), xs_.get(), stream_));
   c_launches_ += 3;
 }
 
 // dst [L, w] = the rows of src [N, w] added up by word
 void Engine::words_sum(float *dst, const float *src, int ld_src, int w) {
-  ProfScope ps(this, K_SCATTER);
+  ProfScope ps(this, K_OTHER);
   check(cavs_gather_sums(dst, w, src, ld_src, d_words_index_, N_, w, word_parts_.get(), word_parts_.capacity() * 4, stream_));
   c_launches_ += 2;
 }
