@@ -20,7 +20,7 @@ constexpr size_t kSmall = size_t(256) << 10;
 // Threads besides the caller's: a core copies and faults in about 10 GB/s, the link does 55 (89 MB with eleven
 // 2.20 ms, with five 2.23).
 constexpr int kThreads = 5;
-// A plain copy takes about 0.07 ms a megabyte longer: from here on a process has paid what the ring costs.
+// A plain copy takes 0.03 (11 MB) to 0.07 ms a megabyte longer: from here on a process has paid what the ring costs.
 constexpr size_t kWorth = size_t(128) << 20;
 // How long the ring stays without anybody attached to it.
 constexpr auto kKeep = std::chrono::seconds(2);
