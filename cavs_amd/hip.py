@@ -53,7 +53,8 @@ GEMM_C_UNUSED, GEMM_A_ZERO, GEMM_B_ZERO = 1, 2, 3
 
 class GroupPlan(C.Structure):
     """cavs_group_plan"""
-    _fields_ = [("groups", _P), ("lists", _P), ("recs", _P), ("ngroups", _I), ("sync", _P), ("spin_max", _I), ("extra_arrivals", _I)]
+    _fields_ = [("groups", _P), ("lists", _P), ("recs", _P), ("ngroups", _I), ("sync", _P), ("spin_max", _I), ("extra_arrivals", _I),
+                ("tile_rows", _I)]
 
 
 # name -> argtypes (every function returns int unless listed in _RESTYPE)

@@ -177,12 +177,19 @@ int Engine::tail_limit() const {
 // A group takes a round of up to this many rows (in slices of 32); larger rounds are launches of their own.
 int Engine::group_limit() const {
   if (!resident_ || fused_rows() <= 0 || cell_ || !cavs_group_rounds_ok(cfg_.H)) return 0;
-  if (cfg_.model == CAVS_MODEL_TREELSTM && cavs_tail_rounds_ok(1, cfg_.H)) return 0;  // (the tail launches are tuned for that size)
-  return cfg_.tail_rows > 0 ? cfg_.tail_rows : 64;
+  if (cfg_.tail_rows > 0) return tail_limit() > 0 ? 0 : cfg_.tail_rows;
+  return 64;
+}
+
+// Lists of the group launches for the batch whose index lists are given, and the tiles they run in.
+void Engine::build_group_plan(const int *t2j, const int *pair, const int *child, const int *kid_rows, int *block) {
+  build_group_lists(*sched_, nch_, t2j, pair, child, kid_rows, group_limit(), cavs_group_max_groups(cfg_.H), cavs_group_rows(), &group_, block);
+  if (group_.first >= 0 && group_.tile_rows == 4 && tail_limit() > 0) group_ = GroupLists();  // (the tail launches are tuned for that)
 }
 
 cavs_group_plan Engine::group_plan(const GroupLists::Launch &l) const {
-  return {d_group_ + l.groups, d_group_ + l.lists, d_group_ + l.recs, group_.ngroups, reinterpret_cast<unsigned *>(tail_sync_.get()), kTailSpins, 0};
+  return {d_group_ + l.groups, d_group_ + l.lists, d_group_ + l.recs, group_.ngroups, reinterpret_cast<unsigned *>(tail_sync_.get()), kTailSpins, 0,
+          group_.tile_rows};
 }
 
 void Engine::group_launched() {
@@ -750,10 +757,9 @@ void Engine::upload_index_arena() {
   forest_ = want_forest && build_forest_lists(s, nch_, fused_rows(), pair, child, roots + s.B, roots + s.B + (size_t)nch_ * N, &n_orphans_);
   tail_ = TailPlan();
   int *tail_rows = roots + s.B + (size_t)N * (nch_ + 1);
-  if (want_tail && forest_) build_tail_plan(roots + s.B, tail_rows);
   group_ = GroupLists();
-  if (group_lim > 0 && forest_)
-    build_group_lists(s, nch_, t2j, pair, child, roots + s.B, group_lim, ngroups, cavs_group_rows(), &group_, h.host.get() + group_at);
+  if (group_lim > 0 && forest_) build_group_plan(t2j, pair, child, roots + s.B, h.host.get() + group_at);
+  if (want_tail && forest_ && group_.first < 0) build_tail_plan(roots + s.B, tail_rows);
   d_group_ = h.dev.get() + group_at;
   plan_head_chunks(roots + s.B + (size_t)nch_ * N);
   check(cavs_memcpy_h2d(h.dev.get(), h.host.get(), (group_.first >= 0 ? group_at + group_.ints : total) * sizeof(int),
@@ -958,10 +964,28 @@ void Engine::schedule_on_device(const int *graph, int B, int maxlen) {
   n_orphans_ = B;
   forest_ = !cfg_.split_backward_rounds && fused_rows() > 0;
   for (int r = 1; r < R && forest_; r++) forest_ = s.rounds[r].n <= fused_rows();
+  tail_ = TailPlan();
+  group_ = GroupLists();
+  // The group launches' block is host work on all of the lists: they come back, the block goes up.
+  if (forest_ && group_limit() > 0 && N > 0) {
+    const size_t all = BM * (2 + 2 * (size_t)nch_);
+    const int ngroups = cavs_group_max_groups(cfg_.H);
+    d.kid_host.reserve(all);
+    d.tail_host.reserve(group_lists_bound(N, ngroups));
+    check(cavs_memcpy_d2h(d.kid_host.get(), t2j, all * sizeof(int), sched_stream_));
+    check(cavs_stream_sync(sched_stream_));
+    const int *h = d.kid_host.get();
+    build_group_plan(h, h + BM, h + 2 * BM, h + (2 + nch_) * BM, d.tail_host.get());
+    if (group_.first >= 0) {
+      d.tail_dev.reserve(grow(group_.ints, d.tail_dev.capacity()));
+      check(cavs_memcpy_h2d(d.tail_dev.get(), d.tail_host.get(), group_.ints * sizeof(int), sched_stream_));
+      check(cavs_stream_sync(sched_stream_));
+      d_group_ = d.tail_dev.get();
+    }
+  }
   // The tail launches want whole trees of the message flow dealt to their groups, which is host
   // work on the children-by-slab-row list: it comes back (2N ints), the groups' row lists go up.
-  tail_ = TailPlan();
-  if (forest_ && nch_ == 2 && tail_limit() > 0 && N > 0) {
+  if (forest_ && nch_ == 2 && tail_limit() > 0 && N > 0 && group_.first < 0) {
     d.kid_host.reserve(2 * (size_t)N);
     d.tail_host.reserve(N);
     check(cavs_memcpy_d2h(d.kid_host.get(), kid, 2 * (size_t)N * sizeof(int), sched_stream_));
@@ -972,23 +996,6 @@ void Engine::schedule_on_device(const int *graph, int B, int maxlen) {
       check(cavs_memcpy_h2d(d.tail_dev.get(), d.tail_host.get(), tail_.rows * sizeof(int), sched_stream_));
       check(cavs_stream_sync(sched_stream_));
       d_tail_rows_ = d.tail_dev.get();
-    }
-  }
-  // The group launches' block is host work on all of the lists: they come back, the block goes up.
-  if (forest_ && group_limit() > 0 && N > 0) {
-    const size_t all = BM * (2 + 2 * (size_t)nch_);
-    const int ngroups = cavs_group_max_groups(cfg_.H);
-    d.kid_host.reserve(all);
-    d.tail_host.reserve(group_lists_bound(N, ngroups));
-    check(cavs_memcpy_d2h(d.kid_host.get(), t2j, all * sizeof(int), sched_stream_));
-    check(cavs_stream_sync(sched_stream_));
-    const int *h = d.kid_host.get();
-    build_group_lists(s, nch_, h, h + BM, h + 2 * BM, h + (2 + nch_) * BM, group_limit(), ngroups, cavs_group_rows(), &group_, d.tail_host.get());
-    if (group_.first >= 0) {
-      d.tail_dev.reserve(grow(group_.ints, d.tail_dev.capacity()));
-      check(cavs_memcpy_h2d(d.tail_dev.get(), d.tail_host.get(), group_.ints * sizeof(int), sched_stream_));
-      check(cavs_stream_sync(sched_stream_));
-      d_group_ = d.tail_dev.get();
     }
   }
   sched_ms_ = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count();

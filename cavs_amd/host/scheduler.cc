@@ -408,6 +408,27 @@ size_t group_lists_bound(size_t N, int groups) {
   return N * (16 + 8) + 2 * (size_t)groups * 4;
 }
 
+// What the group with the most work spends on tiles when its lists run in tiles of four rows, and when they run in
+// tiles of sixteen as far as they have more than eight rows.  In units of a tile of four rows, measured inside the
+// launches at H = 512 (cycles): a tile of four 2580 forward and 2750 backward, of sixteen 6700 and 7000; the kernel with
+// both kinds of tiles takes 0.15 longer over a list, so a batch whose lists are all short keeps the other one (chains of
+// one row a group, H = 128: 2.88 against 3.02 ms per 16 steps; trees at H = 256, lists of 42, 27, 20 .. 1 rows: 2.57 against 2.39).
+static int group_tile_rows(const std::vector<int> &per, int rounds, int slice) {
+  double four = 0, wide = 0;
+  for (size_t i = 0; i < per.size(); i += rounds) {
+    double f = 0, w = 0;
+    for (int k = 0; k < rounds; k++)
+      for (int c = per[i + k]; c > 0; c -= slice) {
+        const int n = std::min(c, slice), w16 = (n + 7) / 16;
+        f += (n + 3) / 4;
+        w += 0.15 + 2.6 * w16 + (std::max(0, n - 16 * w16) + 3) / 4;
+      }
+    four = std::max(four, f);
+    wide = std::max(wide, w);
+  }
+  return wide < four ? 16 : 4;
+}
+
 void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pair, const int *child, const int *kid_rows, int lim, int groups,
                        int slice, GroupLists *out, int *block) {
   *out = GroupLists();
@@ -493,6 +514,7 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
       end = l.lists + 4 * (size_t)nl;
     }
     t.ints = end;
+    t.tile_rows = group_tile_rows(per, nr, slice);
     return;
   }
 }

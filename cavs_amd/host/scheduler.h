@@ -98,6 +98,7 @@ struct GroupLists {
   int first = -1, ngroups = 0;
   Launch fwd, bwd;
   size_t ints = 0, rows = 0;
+  int tile_rows = 4;  // cavs_group_plan::tile_rows
 };
 // ints the block may take for N vertices
 size_t group_lists_bound(size_t N, int groups);

@@ -518,6 +518,7 @@ typedef struct {
   int ngroups;
   unsigned *sync;
   int spin_max, extra_arrivals;
+  int tile_rows;  /* 0 or 4: a list runs in tiles of four rows; 16: in tiles of sixteen as far as it has them */
 } cavs_group_plan;
 int cavs_group_rounds_ok(int H);
 int cavs_group_max_groups(int H);
