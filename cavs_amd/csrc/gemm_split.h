@@ -31,7 +31,8 @@
 // touch all 64 banks once (without it: a third of the LDS time).  While a step multiplies, the values of
 // the next one are converted and those of the one behind it are under way; the conversions (4.5
 // vector instructions a value) run in the shadow of the MFMAs of the two or three workgroups a CU holds.
-// What bounds it is the matrix pipe at the clock it is given: bf16 MFMAs alone, from registers, sustain
+// What bounds it is power: with random operands the clock falls to 1.63 - 1.77 GHz (NN and NT below; 2.0 for TN), with
+// operands of zeros the same instructions run at 2.39 GHz and 262 - 290 TFLOP/s.  bf16 MFMAs alone, from registers, sustain
 // 1.63 - 1.88 PFLOP/s here (1.75 GHz), i.e. 270 - 310 TFLOP/s of these products.
 //
 // us (TFLOP/s)                  fp32 MFMA, 128 x 128 x 16      this
@@ -41,6 +42,10 @@
 //   NN  7088 x 10000 x   512     688 (105)                      407 (178)
 //   NN  2368 x  2048 x   300    34.2 (85)    (64 x 64 tiles)   27.1 (107)
 //   TN   304 x  2048 x  2368    43.2 (68)                      34.7 (85)
+// Operands that are not k-contiguous cost instructions (a load per value, 230 a step and wavefront with their
+// addresses): read through buffer descriptors, on one card, us before / now: NN 8192 5920 / 5681, NN 73000 x 4096 x 1024
+// 3365 / 3226, NN 7088 409 / 391, TN 73000 3470 / 3335; NT, which has none, 3132 / 3125.  Tried: parts read a
+// step ahead from three buffers (NN + 2 %, NT + 2 %, TN - 4 %: a third of the cycles less, a clock as much lower).
 // 2-norm of the error against 64 bits over that of the product, fp32 MFMA / this, 1e-7: operands from U(-1, 1),
 // from U(0, 1), and all of the form (eight bits) (1 + 2^-10 + 2^-11):
 //   NN  8192    16.2 / 2.7   11.9 / 0.8   11.8 / 1.4        NT 73000    11.5 / 2.5   8.5 / 0.7    8.4 / 1.3
@@ -73,10 +78,13 @@ __device__ inline void split_pair(float x, float y, unsigned *h, unsigned *m, un
   *l = bf16_pair(x, y);
 }
 
-// where the 16-byte piece of row x that holds k = 8 oct .. 8 oct + 7 lies in a part of a tile BK deep
-template <int BK>
+// where the 16-byte piece of row x that holds k = 8 oct .. 8 oct + 7 lies in a part of a tile BK deep.  Rows of 32 bytes: reads
+// take 4.2 cycles a wavefront and instruction with either rule (8.0 unpermuted); eight values of k written by
+// 64 rows at once take 13 with the second and 16 with the first.
+template <int BK, bool KC>
 __device__ inline int split_at(int x, int oct) {
-  return BK == 16 ? x * 32 + ((oct ^ ((x >> 3) & 1)) << 4) : x * 64 + ((oct ^ ((x >> 2) & 3)) << 4);
+  if (BK == 16) return x * 32 + ((oct ^ ((x >> 3) & 1) ^ (KC ? 0 : (x >> 2) & 1)) << 4);
+  return x * 64 + ((oct ^ ((x >> 2) & 3)) << 4);
 }
 
 // Loader of one BX x BK operand tile: units of one x and U values of k, NU per thread.  KC: k is the
@@ -84,7 +92,7 @@ __device__ inline int split_at(int x, int oct) {
 // column.  An x outside the operand reads the last one instead (what it leads to is not stored);
 // only k is checked, and only where the step is not wholly inside the k range.
 // PULL (k-contiguous): rows are looked up (GemmArgs::pull_*), and those a workgroup reads go on into pull_copy.
-template <int BX, int BK, bool KC, bool VEC, bool PULL = false>
+template <int BX, int BK, bool KC, bool VEC, bool DESC, bool PULL = false>
 struct SplitLoader {
   static constexpr int U = KC || BX * BK < 8 * kThreads ? 4 : 8, NU = BX * BK / U / kThreads, PER = BK / U;
   using Off = std::conditional_t<BX == 64, size_t, unsigned>;  // (the large tile's registers are full: its rows are below 32 MB)
@@ -99,11 +107,11 @@ struct SplitLoader {
         const int u = tid + kThreads * i;
         unit[i] = u % PER;
         boff[i] = (Off)min(u / PER, X - 1 - x0) * (Off)(ld * 4) + 16u * unit[i];
-        at[i] = split_at<BK>(u / PER, unit[i] >> 1) + 8 * (unit[i] & 1);
+        at[i] = split_at<BK, KC>(u / PER, unit[i] >> 1) + 8 * (unit[i] & 1);
       } else {
         unit[i] = __builtin_amdgcn_readfirstlane(tid / BX + (kThreads / BX) * i);  // (BX is a multiple of 64)
         boff[i] = 4u * (unsigned)min(tid % BX, X - 1 - x0);
-        at[i] = split_at<BK>(tid % BX, unit[i] * U / 8) + (U == 4 ? 8 * (unit[i] & 1) : 0);
+        at[i] = split_at<BK, KC>(tid % BX, unit[i] * U / 8) + (U == 4 ? 8 * (unit[i] & 1) : 0);
       }
     }
   }
@@ -121,7 +129,7 @@ struct SplitLoader {
     for (int i = 0; i < NU; i++) {
       const int u = tid + kThreads * i, x = u / PER, gx = x0 + x;
       unit[i] = u % PER;
-      at[i] = split_at<BK>(x, unit[i] >> 1) + 8 * (unit[i] & 1);
+      at[i] = split_at<BK, KC>(x, unit[i] >> 1) + 8 * (unit[i] & 1);
       long off = -1;
       if (gx < g.M) {
         const float id = g.pull_x[g.pull_rows[gx]];
@@ -134,9 +142,28 @@ struct SplitLoader {
     }
   }
 
-  // P: the tile's first element at k = 0; k0 and kend are wave-uniform
+  // P: the tile's first element at k = 0; k0 and kend are wave-uniform.  DESC: a whole step is read through a buffer descriptor, the
+  // step's address in scalar registers and a row's offset in a vector register that never changes: no vector
+  // instructions for addresses.
   template <bool WHOLE>
   __device__ inline void load(float (&v)[NU][U], const float *__restrict__ P, long ld, int k0, int kend) const {
+    if constexpr (WHOLE && DESC && !PULL && (!KC || VEC)) {
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(P + (KC ? (long)k0 : (long)k0 * ld)), 0, 0xffffffffu, 0x00020000);
+#pragma unroll
+      for (int i = 0; i < NU; i++) {
+        if constexpr (KC) {
+          typedef float f4 __attribute__((ext_vector_type(4)));
+          const f4 a = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)boff[i], 0, 0));
+#pragma unroll
+          for (int j = 0; j < 4; j++) v[i][j] = a[j];
+        } else {
+#pragma unroll
+          for (int j = 0; j < U; j++)
+            v[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)boff[i], (int)((U * unit[i] + j) * (unsigned)(ld * 4)), 0));
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < NU; i++) {
       if constexpr (KC) {
@@ -277,8 +304,10 @@ __device__ __forceinline__ void split_tile(const GemmArgs &g, int m0, int n0, in
   int kbeg, kend;
   tile_k_range<BM, BN, TA, TB>(g, m0, n0, z, &kbeg, &kend);
 
-  using LA = SplitLoader<BM, BK, !TA, VEC, PULL>;
-  using LB = SplitLoader<BN, BK, TB, VEC>;
+  // (large tile: measured 3 % faster with descriptors for both operands where one of them is not k-contiguous, 4 % slower where both are)
+  constexpr bool DESC = BM == 128 && BN == 128 && (TA || !TB);
+  using LA = SplitLoader<BM, BK, !TA, VEC, DESC, PULL>;
+  using LB = SplitLoader<BN, BK, TB, VEC, DESC>;
   LA la;
   LB lb;
   if constexpr (PULL) {
@@ -341,9 +370,9 @@ __device__ __forceinline__ void split_tile(const GemmArgs &g, int m0, int n0, in
 #pragma unroll
       for (int p = 0; p < 3; p++) {
 #pragma unroll
-        for (int i = 0; i < TM; i++) a[i][p] = *reinterpret_cast<const bf16x8 *>(SA + p * PA + split_at<BK>(ar + 32 * i, 2 * s + half));
+        for (int i = 0; i < TM; i++) a[i][p] = *reinterpret_cast<const bf16x8 *>(SA + p * PA + split_at<BK, !TA>(ar + 32 * i, 2 * s + half));
 #pragma unroll
-        for (int j = 0; j < TN; j++) b[j][p] = *reinterpret_cast<const bf16x8 *>(SB + p * PB + split_at<BK>(br + 32 * j, 2 * s + half));
+        for (int j = 0; j < TN; j++) b[j][p] = *reinterpret_cast<const bf16x8 *>(SB + p * PB + split_at<BK, TB>(br + 32 * j, 2 * s + half));
       }
       // the small products first
       constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 1, 2, 0, 1, 0};
