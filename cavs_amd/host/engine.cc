@@ -47,7 +47,7 @@ Engine::Engine(const cavs_session_config &cfg, void *external_stream, std::share
     const CellSpec *tail = cell_.get();
     while (tail->next) tail = tail->next.get();
     if (tail->S != cell_->SI) fail(CAVS_EINVAL, "the last cell of the chain does not write what the first one gathers");
-    mw_ = tail->S * cfg.H;
+    mw_ = tail->S * cfg_.H;  // (the stored width: the rows of the pool hold padded blocks)
     nch_ = cell_->K;
   }
   const bool reads_x = cell_ ? cell_->NX > 0 : cfg.model != CAVS_MODEL_TREEFC;

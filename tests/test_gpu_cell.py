@@ -97,6 +97,15 @@ def test_a_tree_lstm_with_a_forget_matrix_per_child(oracle, H, pairing):
     compare(run_generated("treelstm2", w, pairing, mode=0), want)
 
 
+def test_a_padded_function_fills_a_message_pool_of_its_stored_width(oracle):
+    """H = 100 is stored as 128 columns, and so are the rows of the pool: by the declared width the last fifth of them lay behind the
+    buffer.  A batch whose pool spans many pages, so that the place behind it need not be another buffer's slack."""
+    w = small_workload("treelstm2", 187, B=60, H=100, E=12, V=29, C=5)
+    for k in ("U", "W"):  # (the gain of a level stays below one)
+        w["params"][k] = w["params"][k] * np.float32(0.3)
+    compare(run_generated("treelstm2", w, "rowid", mode=1), oracle_step(oracle, w, "treelstm2", pairing="rowid"))
+
+
 def test_a_gated_cell_with_one_state_block_against_fp64_autograd():
     """Children's states enter through products (one of them over their concatenation) and
     elementwise; the message has one block.  No oracle restatement: held to the per-sample fp64
