@@ -2,6 +2,8 @@
 // the HIP runtime compiler for gfx950 and launches it over a 1-D grid.  The source
 // dialect (extern "C" __global__, blockIdx/threadIdx, atomicAdd, expf/tanhf) is the
 // one the reference's generator emits and is valid HIP as is.
+#include <cstring>
+#include <algorithm>
 #include <hip/hiprtc.h>
 
 #include <map>
@@ -141,8 +143,7 @@ int cavs_fused_release(void *handle) {
   return CAVS_OK;
 }
 
-int cavs_cell_compile(const char *source, void **handle) {
-  CAVS_REQUIRE(source && handle, "cavs_cell_compile: null argument");
+static int cell_compile(const char *source, const char *const *names, int kernels, void **handle) {
   *handle = nullptr;
   std::lock_guard<std::mutex> lock(cell_mutex());
   auto it = cell_modules().find(source);
@@ -155,7 +156,7 @@ int cavs_cell_compile(const char *source, void **handle) {
   if (int rc = rtc_compile("cell", source, &code)) return rc;
   CellModule *m = new CellModule;
   hipError_t e = hipModuleLoadData(&m->module, code.data());
-  for (int i = 0; i < kCellKernels && e == hipSuccess; i++) e = hipModuleGetFunction(&m->fn[i], m->module, kCellKernelNames[i]);
+  for (int i = 0; i < kernels && e == hipSuccess; i++) e = hipModuleGetFunction(&m->fn[i], m->module, names[i]);
   if (e != hipSuccess) {
     if (m->module) (void)hipModuleUnload(m->module);
     delete m;
@@ -166,6 +167,50 @@ int cavs_cell_compile(const char *source, void **handle) {
   m->source = source;
   cell_modules()[m->source] = m;
   *handle = m;
+  return CAVS_OK;
+}
+
+int cavs_cell_compile(const char *source, void **handle) {
+  CAVS_REQUIRE(source && handle, "cavs_cell_compile: null argument");
+  return cell_compile(source, kCellKernelNames, kCellKernels, handle);
+}
+
+int cavs_cell_rounds_compile(const char *source, void **handle) {
+  CAVS_REQUIRE(source && handle, "cavs_cell_rounds_compile: null argument");
+  static const char *const names[] = {"rounds_fwd", "rounds_bwd"};
+  return cell_compile(source, names, 2, handle);
+}
+
+int cavs_cell_rounds_launch(void *handle, int back, int H, const cavs_group_plan *p, const void *cells, size_t cells_bytes, int whole_lines, void *stream) {
+  CAVS_REQUIRE(handle && cells && cells_bytes > 0 && cells_bytes % 8 == 0 && cells_bytes <= 3072, "cavs_cell_rounds_launch: bad arguments (%zu bytes)", cells_bytes);
+  CAVS_REQUIRE(cavs_group_rounds_ok(H), "cavs_cell_rounds_launch: H=%d (multiples of 32 up to 512)", H);
+  CAVS_REQUIRE(p && p->groups && p->lists && p->recs && p->sync, "cavs_cell_rounds_launch: null plan");
+  CAVS_REQUIRE(aligned16(p->groups) && aligned16(p->lists) && aligned16(p->recs), "cavs_cell_rounds_launch: the plan must be 16-byte aligned");
+  CAVS_REQUIRE(p->ngroups >= 1 && p->ngroups <= cavs_group_max_groups(H) && p->spin_max >= 0 && p->extra_arrivals >= 0,
+               "cavs_cell_rounds_launch: bad plan (1..%d groups)", cavs_group_max_groups(H));
+  // the arguments of the cells, then what struct RoundsPlan of the generated source holds
+  struct {
+    const void *groups, *lists, *recs;
+    void *sync;
+    long long ngroups, spin_max, expect, whole_lines;
+  } plan = {p->groups, p->lists, p->recs, p->sync, p->ngroups, p->spin_max, std::min(H / 16 + p->extra_arrivals, 64), whole_lines};
+  alignas(16) char args[3072 + sizeof plan];
+  std::memcpy(args, cells, cells_bytes);
+  std::memcpy(args + cells_bytes, &plan, sizeof plan);
+  size_t bytes = cells_bytes + sizeof plan;
+  void *config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, args, HIP_LAUNCH_PARAM_BUFFER_SIZE, &bytes, HIP_LAUNCH_PARAM_END};
+  CellModule *m = static_cast<CellModule *>(handle);
+  const unsigned grid = 8 * (H / 16) * ((p->ngroups + 7) / 8), block = 512;
+  ResidentOrder order(as_stream(stream));
+  if (order.rc()) return order.rc();
+  LaunchProbe &probe = launch_probe();
+  if (probe.armed) {
+    hipEvent_t s = probe.started ? nullptr : probe.start;
+    probe.started = true;
+    CAVS_HIP_TRY(hipExtModuleLaunchKernel(m->fn[back ? 1 : 0], grid * block, 1, 1, block, 1, 1, 0, as_stream(stream), nullptr, config, s, probe.stop, 0));
+  } else {
+    CAVS_HIP_TRY(hipModuleLaunchKernel(m->fn[back ? 1 : 0], grid, 1, 1, block, 1, 1, 0, as_stream(stream), nullptr, config));
+  }
   return CAVS_OK;
 }
 

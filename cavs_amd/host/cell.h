@@ -79,6 +79,9 @@ struct CellSpec {
   int NSV = 0;                  // blocks a vertex saves for the backward pass
   int waves = 0;                // wavefronts per workgroup of the round kernels (they split the k range)
   std::string source;           // the kernels (equal sources share a compiled module)
+  // (the head of a chain) the kernels that run the whole chain over many rounds in one launch per direction; empty where its weights
+  // do not fit the registers of sixteen columns or its sums the LDS
+  std::string rounds;
   // A vertex function of several stages -- a product whose left operand depends on another product
   // of the same vertex -- runs as a chain of such cells: every cell but the last writes, per vertex,
   // a row of intermediate blocks (the next stage's left operands and whatever later stages read of

@@ -145,7 +145,7 @@ void Engine::tail_setup() {
   static std::mutex m;
   static std::map<int, bool> known;
   tail_ready_ = probe_due_ = false;
-  if (cell_ || !(cfg_.opt & CAVS_OPT_BATCHING) || cfg_.tail_rows < 0 || !cavs_group_rounds_ok(cfg_.H)) return;
+  if ((cell_ && cell_->rounds.empty()) || !(cfg_.opt & CAVS_OPT_BATCHING) || cfg_.tail_rows < 0 || !cavs_group_rounds_ok(cfg_.H)) return;
   const size_t words = cavs_tail_sync_bytes() / sizeof(int);
   tail_sync_.reserve(words);
   check(cavs_zero(tail_sync_.get(), words * sizeof(int), stream_));
@@ -163,6 +163,7 @@ void Engine::tail_setup() {
     if (!it->second) check(cavs_zero(tail_sync_.get(), words * sizeof(int), stream_));
   }
   tail_ready_ = it->second;
+  if (tail_ready_ && cell_ && !cell_rounds_) check(cavs_cell_rounds_compile(cell_->rounds.c_str(), &cell_rounds_));
 }
 
 int Engine::tail_limit() const {
@@ -176,7 +177,7 @@ int Engine::tail_limit() const {
 
 // A group takes a round of up to this many rows (in slices of 32); larger rounds are launches of their own.
 int Engine::group_limit() const {
-  if (!resident_ || fused_rows() <= 0 || cell_ || !cavs_group_rounds_ok(cfg_.H)) return 0;
+  if (!resident_ || fused_rows() <= 0 || (cell_ && cell_->rounds.empty()) || !cavs_group_rounds_ok(cfg_.H)) return 0;
   if (cfg_.tail_rows > 0) return tail_limit() > 0 ? 0 : cfg_.tail_rows;
   return 64;
 }
@@ -193,7 +194,12 @@ cavs_group_plan Engine::group_plan(const GroupLists::Launch &l) const {
 }
 
 void Engine::group_launched() {
-  const double rows = (double)group_.rows, per = cfg_.model == CAVS_MODEL_TREELSTM ? 5.0 : cfg_.model == CAVS_MODEL_LSTM ? 4.0 : 2.0;
+  const double rows = (double)group_.rows;
+  double per = cfg_.model == CAVS_MODEL_TREELSTM ? 5.0 : cfg_.model == CAVS_MODEL_LSTM ? 4.0 : 2.0;
+  if (cell_) {
+    per = 0;
+    for (const CellStage &st : cells_) per += st.spec->terms();
+  }
   c_round_flops_ += 2.0 * rows * cfg_.H * per * cfg_.H;
   c_gather_rows_ += nch_ * rows;
   c_scatter_rows_ += rows;
@@ -257,6 +263,7 @@ void Engine::tail_check() {
 Engine::~Engine() {
   cavs_stream_sync(stream_);
   for (CellStage &st : cells_) cavs_cell_release(st.module);
+  cavs_cell_release(cell_rounds_);
   for (auto &e : ev_) cavs_event_destroy(e);
   for (auto &h : hlists_) {
     if (h.up_ev) cavs_event_destroy(h.up_ev);
@@ -641,7 +648,7 @@ void Engine::reserve_edges() {
   if (fused_rows() > 0 && ((cfg_.model == CAVS_MODEL_TREELSTM && (cavs_round_packed_ok(1, H) || cavs_round_packed_ok(65, H))) ||
                            (cfg_.model == CAVS_MODEL_LSTM && (cavs_lstm_round_packed_ok(1, H) || cavs_lstm_round_packed_ok(65, H)))))
     R(Upk_, (size_t)4 * H * H);
-  if (group_.first >= 0) {
+  if (group_.first >= 0 && !cell_) {
     R(Upk_, (size_t)(cfg_.model == CAVS_MODEL_TREEFC ? 2 : 4) * H * H);
     R(UTp_, (size_t)(cfg_.model == CAVS_MODEL_TREEFC ? 2 : 4) * H * H);
   }
@@ -2192,14 +2199,10 @@ void Engine::treefc_backward() {
 // their elementwise part; anything else two launches per round and cell, with the message
 // gradients going through the gradients of the rows the cells write.  Then the weight gradients as
 // products over all rows.
-void Engine::cell_launch(int ci, int k, unsigned gx, unsigned gy, unsigned gz, unsigned block, long off, long n, const int *rows, const float *go) {
+void Engine::cell_args(int ci, const float *go, CellSlot (&a)[CA_SLOTS]) {
   CellStage &st = cells_[ci];
   const CellSpec &c = *st.spec;
   const bool first = ci == 0, last = ci + 1 == (int)cells_.size();
-  union Slot {
-    const void *p;
-    long long i;
-  } a[CA_SLOTS];
   std::memset(a, 0, sizeof a);
   // a cell in the middle of a chain gathers row v of the cell before and writes row v of its own
   a[CA_POOL].p = last ? pool_.get() : st.rows.get();
@@ -2221,7 +2224,6 @@ void Engine::cell_launch(int ci, int k, unsigned gx, unsigned gy, unsigned gz, u
     a[CA_FT_KIDS].p = pi == 0 ? d_kid_rows_ : cell_iota_.get();
   }
   a[CA_T2J].p = d_t2j_;
-  a[CA_ROWS].p = rows;
   a[CA_XW].p = xW_.get();
   a[CA_SV].p = st.sv.get();
   a[CA_ASRC].p = st.asrc.get();
@@ -2231,15 +2233,43 @@ void Engine::cell_launch(int ci, int k, unsigned gx, unsigned gy, unsigned gz, u
   a[CA_BT].p = st.bt.get();
   a[CA_COLSUM].p = st.colsum.get();
   a[CA_X].p = d_x_;
-  a[CA_OFF].i = off;
-  a[CA_N].i = n;
   for (size_t i = 0; i < c.params.size(); i++) {
     const Param &p = param(c.params[i].name);
     a[CA_PARAM0 + i].p = p.w;
     a[CA_PARAM0 + CA_MAX_PARAMS + i].p = p.g;
   }
-  check(cavs_cell_launch(st.module, k, gx, gy, gz, block, a, sizeof a, stream_));
+}
+
+void Engine::cell_launch(int ci, int k, unsigned gx, unsigned gy, unsigned gz, unsigned block, long off, long n, const int *rows, const float *go) {
+  CellSlot a[CA_SLOTS];
+  cell_args(ci, go, a);
+  a[CA_ROWS].p = rows;
+  a[CA_OFF].i = off;
+  a[CA_N].i = n;
+  check(cavs_cell_launch(cells_[ci].module, k, gx, gy, gz, block, a, sizeof a, stream_));
   c_launches_ += 1;
+}
+
+// The rounds of the batch's group lists in one launch, every cell of the chain in it.
+void Engine::cell_rounds_launch(bool back, const float *go) {
+  std::vector<CellSlot> args(cells_.size() * CA_SLOTS);
+  bool whole_lines = true;
+  auto lines = [&](const void *p) { whole_lines = whole_lines && reinterpret_cast<uintptr_t>(p) % 128 == 0; };  // (rows are multiples of 32 floats)
+  for (size_t ci = 0; ci < cells_.size(); ci++) {
+    CellSlot a[CA_SLOTS];
+    cell_args((int)ci, go, a);
+    std::memcpy(&args[ci * CA_SLOTS], a, sizeof a);
+    lines(a[CA_POOL].p);
+    lines(a[CA_POOL_IN].p);
+    lines(a[CA_D].p);
+    lines(a[CA_DS].p);
+  }
+  const cavs_group_plan plan = group_plan(back ? group_.bwd : group_.fwd);
+  {
+    ProfScope ps(this, K_ROUND);
+    check(cavs_cell_rounds_launch(cell_rounds_, back, cfg_.H, &plan, args.data(), args.size() * sizeof(CellSlot), whole_lines, stream_));
+  }
+  group_launched();
 }
 
 void Engine::cell_forward() {
@@ -2263,7 +2293,12 @@ void Engine::cell_forward() {
     const CellSpec &c = *cells_[ci].spec;
     cell_launch((int)ci, CK_PACK, (unsigned)(((size_t)2 * c.blocks() * H * H / 4 + 255) / 256), 1, 1, 256, 0, 0, nullptr, fwd_out_);
   }
-  for (const Round &r : sched_->rounds)
+  for (size_t rk = 0; rk < sched_->rounds.size(); rk++) {
+    const Round &r = sched_->rounds[rk];
+    if (group_.first >= 0 && (int)rk == group_.first) {
+      cell_rounds_launch(false, fwd_out_);
+      break;
+    }
     for (size_t ci = 0; ci < cells_.size(); ci++) {
       const CellSpec &c = *cells_[ci].spec;
       if (ci == 0 && leaf_round(r)) {  // (a later cell's one child is the vertex itself: it always has it)
@@ -2277,6 +2312,7 @@ void Engine::cell_forward() {
       }
       c_scatter_rows_ += r.n;
     }
+  }
 }
 
 void Engine::cell_backward() {
@@ -2315,8 +2351,11 @@ void Engine::cell_backward() {
       ProfScope ps(this, K_GATES);
       cell_launch(L - 1, CK_BWD_ROWS, (unsigned)(((size_t)n_orphans_ * H + 255) / 256), 1, 1, 256, 0, n_orphans_, d_orphans_, d_dgo_);
     }
+    // (the backward order is the forward order reversed: the rounds of the group lists come first)
+    if (group_.first >= 0 && !head_chunked_) cell_rounds_launch(true, d_dgo_);
     for (int k : sched_->bwd_rounds) {
       const Round &r = sched_->rounds[k];
+      if (group_backward(k)) continue;
       c_gather_rows_ += r.n;
       for (int ci = L - 1; ci >= 0; ci--) {
         if (ci == 0 && leaf_round(r)) continue;

@@ -511,6 +511,13 @@ class Engine {
   DeviceArray<int> cell_iota_;  // 0, 1, 2, ...: "the child of slab row v is slab row v" (also: "d h of slab row v is row v")
   size_t cell_iota_n_ = 0;
   void ensure_iota(size_t n);
+  void *cell_rounds_ = nullptr;  // the module of the resident kernels
+  union CellSlot {
+    const void *p;
+    long long i;
+  };
+  void cell_args(int ci, const float *go, CellSlot (&a)[CA_SLOTS]);
+  void cell_rounds_launch(bool back, const float *go);
   // one launch of kernel `k` of cell `ci`'s module
   void cell_launch(int ci, int k, unsigned gx, unsigned gy, unsigned gz, unsigned block, long off, long n, const int *rows, const float *go);
   void embedding_backward_rows();

@@ -168,7 +168,8 @@ size_t C_DumpCell(char *buf, size_t cap, int what) {
     auto m = cavs::mid::match_cell(cavs::mid::global_graph(), &why);
     std::shared_ptr<cavs::CellSpec> spec = m ? m->spec : nullptr;
     for (int i = 0; i < stage && spec; i++) spec = spec->next;
-    d = spec ? spec->source : m ? std::string("// no such stage\n") : "// not a cell: " + why + "\n";
+    if (spec && what % 10 == 2) d = spec->rounds;
+    else d = spec ? spec->source : m ? std::string("// no such stage\n") : "// not a cell: " + why + "\n";
   }
   if (buf && cap) {
     size_t n = std::min(cap - 1, d.size());

@@ -18,6 +18,9 @@ namespace {
 const char kTemplate[] =
 #include "cell_template.inc"
     ;
+const char kRoundsTemplate[] =
+#include "cell_rounds.inc"
+    ;
 
 // ---------------------------------------------------------------- the elementwise part as a DAG
 // One node per value of one hidden unit of one vertex.  Nodes are created in evaluation order, so an
@@ -535,6 +538,10 @@ struct Writer {
       << "\n#define CELL_ND " << s.ND << "\n#define CELL_NSV " << s.NSV << "\n#define CELL_KS " << s.waves << "\n#define CELL_DS_MASK "
       << dv.ds_mask << "\n#define CELL_BWD_CS " << (dv.reads_cs ? 1 : 0) << "\n";
     o << "typedef float f4 __attribute__((ext_vector_type(4)));\n";
+    args();
+  }
+
+  void args() {
     o << "struct CellArgs {\n  float *pool;\n  const int *child, *pair, *kids, *t2j, *rows;\n  const float *xw;\n"
          "  float *sv, *asrc, *go, *d, *ds, *bt, *colsum, *dpool;\n  const float *x;\n  float *pool_in, *dpool_in;\n"
          "  float *ft_sv, *ft_d, *ft_ds;\n  const float *ft_pool_in;\n  const int *ft_child, *ft_kids;\n  long off, n;\n  float *p["
@@ -652,6 +659,124 @@ struct Writer {
     o << "extern \"C\" __global__ void cell_bias(CellArgs a) {\n  const int j = blockIdx.x * 256 + threadIdx.x;\n  if (j >= CELL_H) return;\n";
     for (const CellBias &b : s.biases) o << "  " << param_ptr(b.ref, true) << "[j] " << (b.add ? "+=" : "=") << " a.colsum[" << (long)b.dcol * H << " + j];\n";
     o << "}\n";
+  }
+};
+
+// ---------------------------------------------------------------- many rounds in one launch
+// What the resident kernels name of one cell (cell_rounds.inc): sizes, elementwise part and the products over tiles of four rows, k-group
+// by k-group of the weights a wavefront keeps in registers.
+struct RoundsWriter : Writer {
+  RoundsWriter(const Body &rd, const Derived &d) : Writer(rd, d, true) {}
+
+  struct Blk {
+    int param, ldb;
+    long at;
+    bool operator==(const Blk &b) const { return param == b.param && ldb == b.ldb && at == b.at; }
+  };
+  std::vector<Blk> blks;
+  std::vector<int> term_blk, dcols;
+  std::vector<std::pair<int, int>> raw;  // (child, block) rows the left operands read
+
+  void collect() {
+    for (const CellProduct &p : s.products) {
+      for (const CellTerm &tm : p.terms) {
+        const Blk b{p.B.param, p.ldb, p.B.offset + tm.brow * p.ldb + p.col};
+        const size_t q = std::find(blks.begin(), blks.end(), b) - blks.begin();
+        if (q == blks.size()) blks.push_back(b);
+        term_blk.push_back((int)q);
+      }
+      if (std::find(dcols.begin(), dcols.end(), p.dcol) == dcols.end()) dcols.push_back(p.dcol);
+    }
+    std::set<std::pair<int, int>> seen;
+    for (const CellASrc &a : s.asrc)
+      for (int k = 0; k < s.K; k++)
+        if (a.mask >> k & 1) seen.insert({k, a.block});
+    raw.assign(seen.begin(), seen.end());
+  }
+
+  // a table of small constants as a function of an index that is known when the loop around it is unrolled
+  void table(const char *name, const std::vector<int> &v) {
+    o << "  static __device__ constexpr int " << name << "(int i) { return ";
+    for (size_t i = 0; i + 1 < v.size(); i++) o << "i == " << i << " ? " << v[i] << " : ";
+    o << v.back() << "; }\n";
+  }
+
+  void cell(int index, int nfwd) {
+    collect();
+    const int NP = (int)s.products.size(), NA = (int)s.asrc.size();
+    const std::string ns = "c" + std::to_string(index);
+    o << "namespace " << ns << " {\n";
+    elementwise(nfwd);
+    o << "}  // namespace " << ns << "\nstruct Cell" << index << " {\n  typedef " << ns << "::FwdIn FwdIn;\n  typedef " << ns << "::FwdOut FwdOut;\n  typedef " << ns
+      << "::BwdIn BwdIn;\n  typedef " << ns << "::BwdOut BwdOut;\n";
+    o << "  static constexpr int K = " << s.K << ", S = " << s.S << ", SI = " << s.SI << ", NX = " << s.NX << ", XD = " << s.XD << ", NP = " << NP << ", NA = " << NA
+      << ", ND = " << s.ND << ", NSV = " << s.NSV << ", DS_MASK = " << dv.ds_mask << ", NBK = " << blks.size() << ", NRAW = " << raw.size() << ", NDC = " << dcols.size()
+      << ";\n  static constexpr bool HAS_RET = " << (s.has_ret ? "true" : "false") << ", BWD_CS = " << (dv.reads_cs ? "true" : "false") << ";\n";
+    o << "  static __device__ inline void forward(const FwdIn &in, FwdOut &out) { " << ns << "::cell_forward(in, out); }\n";
+    o << "  static __device__ inline void backward(const BwdIn &in, BwdOut &out) { " << ns << "::cell_backward(in, out); }\n";
+    std::vector<int> rc, rb;
+    for (auto &kb : raw) {
+      rc.push_back(kb.first);
+      rb.push_back(kb.second);
+    }
+    table("raw_child", rc);
+    table("raw_block", rb);
+    table("dcol", dcols);
+    o << "  static __device__ inline void load_bias(const CellArgs &a, int j, FwdIn &in) {\n";
+    for (size_t i = 0; i < s.biases.size(); i++) o << "    in.bias[" << i << "] = " << param_ptr(s.biases[i].ref) << "[j];\n";
+    o << "  }\n  static __device__ inline void store_asrc(float *dst, const FwdIn &in) {\n";
+    for (int q = 0; q < NA; q++) {
+      o << "    dst[" << (long)q * s.H << "] = ";
+      bool first = true;
+      for (int k = 0; k < s.K; k++)
+        if (s.asrc[q].mask >> k & 1) {
+          o << (first ? "" : " + ") << "in.cs[" << k << "][" << s.asrc[q].block << "]";
+          first = false;
+        }
+      o << ";\n";
+    }
+    o << "  }\n  static __device__ inline void add_products(float (&dst)[SI], const float (&s)[NA], int k) {\n";
+    for (int k = 0; k < s.K; k++) {
+      o << "    if (k == " << k << ") {\n";
+      for (int q = 0; q < NA; q++)
+        if (s.asrc[q].mask >> k & 1) o << "      dst[" << s.asrc[q].block << "] += s[" << q << "];\n";
+      o << "    }\n";
+    }
+    o << "  }\n";
+    products("forward_products", "raw[NRAW]", NP, true);
+    products("backward_products", "d[NDC]", NA, false);
+    o << "};\n";
+  }
+
+  void products(const char *fn, const char *operands, int nacc, bool fwd) {
+    const int GPW = (s.H + 127) / 128;
+    o << "  static __device__ inline void " << fn << "(const f4 (&" << std::string(operands).substr(0, std::string(operands).find('[')) << ")"
+      << std::string(operands).substr(std::string(operands).find('[')) << ", const f4 (&w)[NBK][" << GPW << "], f4 (&acc)[" << nacc << "]) {\n";
+    if (fwd)
+      for (size_t q = 0; q < s.asrc.size(); q++) {
+        std::string e;
+        for (int k = 0; k < s.K; k++)
+          if (s.asrc[q].mask >> k & 1) {
+            const size_t i = std::find(raw.begin(), raw.end(), std::make_pair(k, s.asrc[q].block)) - raw.begin();
+            const std::string v = "raw[" + std::to_string(i) + "]";
+            e = e.empty() ? v : e + " + " + v;
+          }
+        o << "    const f4 a" << q << " = " << e << ";\n";
+      }
+    for (int g = 0; g < GPW; g++)
+      for (int c = 0; c < 4; c++) {
+        int t = 0;
+        for (size_t p = 0; p < s.products.size(); p++) {
+          const size_t ai = std::find(dcols.begin(), dcols.end(), s.products[p].dcol) - dcols.begin();
+          for (const CellTerm &tm : s.products[p].terms) {
+            const int to = fwd ? (int)p : tm.asrc;
+            o << "    acc[" << to << "] = __builtin_amdgcn_mfma_f32_4x4x1f32(" << (fwd ? "a" + std::to_string(tm.asrc) : "d[" + std::to_string(ai) + "]") << "[" << c
+              << "], w[" << term_blk[t] << "][" << g << "][" << c << "], acc[" << to << "], 2, " << g << ", 0);\n";
+            t++;
+          }
+        }
+      }
+    o << "  }\n";
   }
 };
 
@@ -924,6 +1049,55 @@ void write_cell(Body &c, const Derived &d, int nfwd, const Body *ft, const Deriv
   s.source = w.o.str();
 }
 
+// The source of the resident kernels of a whole chain (empty: they would not fit).
+std::string write_rounds(const Chain &b) {
+  const int L = (int)b.cells.size(), H = b.cells[0].spec.H;
+  // Sixteen columns of every block in the registers of eight wavefronts, four registers per k-group (of 256; the four-row tiles need
+  // about a hundred), and the partial sums of 32 rows in LDS.
+  int blocks = 0, sums = 1;
+  for (const Body &c : b.cells) {
+    blocks += c.spec.blocks();
+    sums = std::max({sums, (int)c.spec.products.size(), (int)c.spec.asrc.size()});
+    if (c.spec.products.empty() || c.spec.asrc.empty() || c.spec.K > 2) return "";
+  }
+  if (H > 512 || H % 32 || blocks * ((H + 127) / 128) > 32 || sums > 8) return "";
+  std::ostringstream o;
+  o << "#define ROUNDS_H " << H << "\n#define ROUNDS_UH " << b.cells[0].spec.uH << "\n";
+  o << "typedef float f4 __attribute__((ext_vector_type(4)));\n";
+  for (int i = 0; i < L; i++) {
+    RoundsWriter w(b.cells[i], b.derived[i]);
+    if (i == 0) {
+      w.args();
+      o << w.o.str();
+      w.o.str("");
+    }
+    w.cell(i, b.nfwd[i]);
+    o << w.o.str();
+  }
+  o << kRoundsTemplate;
+  o << "struct RoundsArgs {\n  CellArgs a[" << L << "];\n  RoundsPlan plan;\n};\n";
+  const int floats = std::max(sums * 4096, 84 * 256);  // (more than half of a CU's LDS: workgroups land one to a CU)
+  for (int back = 0; back < 2; back++) {
+    o << "extern \"C\" __global__ __launch_bounds__(512, 1) void " << (back ? "rounds_bwd" : "rounds_fwd")
+      << "(RoundsArgs A) {\n  __shared__ __attribute__((aligned(16))) float red[" << floats
+      << "];\n  __shared__ i4 s_rec[2][2 * ROWS];\n  __shared__ int s_bail;\n  Walk wk;\n  if (!wk.start(A.plan, s_rec, &s_bail)) return;\n";
+    for (int i = 0; i < L; i++)
+      o << "  f4 w" << i << "[Cell" << i << "::NBK][GPW];\n  rounds_weights<Cell" << i << "::NBK>(A.a[" << i << "], " << back << ", wk.ct, w" << i << ");\n";
+    o << "  if ((threadIdx.x >> 6) < 4) __builtin_amdgcn_s_setprio(2);\n  __syncthreads();\n  for (int r = 0; r < wk.nlists; r++) {\n"
+         "    const i4 *rt = s_rec[r & 1];\n    const int n = wk.cur[1] < ROWS ? wk.cur[1] : ROWS;\n    wk.fetch_next(r);\n";
+    // (a list whose plan says it waits for nothing reads nothing an earlier list of this launch wrote that the one before it did not wait for)
+    for (int s = 0; s < L; s++) {
+      const int i = back ? L - 1 - s : s, f = (i + L - 1) % L;
+      const std::string target = s == 0 ? "wk.cur[2] > 0 ? (unsigned)r * " + std::to_string(L) + "u : 0u" : "(unsigned)r * " + std::to_string(L) + "u + " + std::to_string(s) + "u";
+      o << "    if (!" << (back ? "rounds_backward<Cell" : "rounds_forward<Cell") << i << ", "
+        << (back ? "Cell" + std::to_string(f) + ", " + (i == 0 ? "true" : "false") : std::string(i == 0 ? "true" : "false") + ", " + (i == L - 1 ? "true" : "false"))
+        << ">(A.a[" << i << "], w" << i << ", wk, rt, n, " << target << ", " << (s == L - 1 ? "true" : "false") << ", r, s_rec, &s_bail, red)) return;\n";
+    }
+    o << "    wk.advance();\n  }\n  wk.leave();\n}\n";
+  }
+  return o.str();
+}
+
 }  // namespace
 
 Resolved resolve_external(const Edge *e) {
@@ -967,6 +1141,7 @@ std::unique_ptr<CellMatch> match_cell(const Graph &g, std::string *why) {
       else head = spec;
       tail = spec;
     }
+    head->rounds = write_rounds(b);
     auto m = std::make_unique<CellMatch>();
     m->spec = head;
     m->roles = b.reader.roles;

@@ -722,6 +722,13 @@ int cavs_cell_compile(const char *source, void **handle);
 int cavs_cell_launch(void *handle, int kernel, unsigned grid_x, unsigned grid_y, unsigned grid_z,
                      unsigned block, const void *args, size_t args_bytes, void *stream);
 int cavs_cell_release(void *handle);
+/* The same for many rounds in one launch per direction, the whole chain of cells in it: `source` defines rounds_fwd and rounds_bwd, which
+ * take the argument structs of the chain's cells, in order, and the plan.  Lists and records as for the group launches (whose sync
+ * block it shares): a forward record names the pool rows of the children of the first cell, a backward one their
+ * slab rows.  whole_lines: every row the launch writes and reads begins on a line of 128 bytes and is whole lines. */
+int cavs_cell_rounds_compile(const char *source, void **handle);
+int cavs_cell_rounds_launch(void *handle, int back, int H, const cavs_group_plan *plan, const void *cells, size_t cells_bytes,
+                            int whole_lines, void *stream);
 
 /* ------------------------------------------------------------------ device schedule
  * The level-wise ready frontier of BatchGraphScheduler::Initialize/ActivateNext
