@@ -42,6 +42,7 @@ struct GemmArgs {
   int zseg = 0;
   const int *live = nullptr;  // cavs_gemm_desc::live
   int pad_block = 0, pad_used = 0;  // cavs_gemm_desc::pad_block, pad_used
+  bool through = false;             // partial sums past this XCD's L2: a workgroup anywhere may read them in the same launch
 };
 
 __device__ inline bool padding_column(const GemmArgs &g, int col) { return g.pad_block > 0 && col % g.pad_block >= g.pad_used; }
@@ -101,6 +102,14 @@ __device__ inline void store_tile(const GemmArgs &g, const floatx16 (&acc)[TM][T
       // for every lane), not once per element
       if (g.ws) {  // split K: park the partial sum, the reduce kernel finishes the job
         float *w = g.ws + (long)z * g.M * g.N + col;
+        if (g.through) {
+#pragma unroll
+          for (int r = 0; r < 16; r++) {
+            const int row = rbase + 8 * (r / 4) + (r % 4);
+            if (row < g.M) __hip_atomic_store(w + (long)row * g.N, acc[i][j][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+          continue;
+        }
 #pragma unroll
         for (int r = 0; r < 16; r++) {
           const int row = rbase + 8 * (r / 4) + (r % 4);

@@ -13,6 +13,7 @@
 #include <atomic>
 
 #include "bench_probes.h"
+#include "colsum_common.h"
 #include "common.h"
 #include "embed_common.h"
 #include "gemm_common.h"
@@ -36,10 +37,78 @@ struct GemmGroup {
   int count;
 };
 
+// The embedding gradient behind one product of a group (cavs_sgemm_group_embed_bwd): the rows of
+// that product's result are scatter-added into the table by extra workgroups of the launch that
+// reduces the other products' K splits, reading the product's own partials directly.
+struct EmbedTail {
+  float *dtable;
+  const float *ids;
+  const float *dy;   // the result, or the first of `parts` partial results `part_stride` floats apart
+  long ld_dy, part_stride;
+  int parts;
+  float *copy;       // where the summed result goes as well (the product's C) when parts > 1
+  long ld_copy;
+  int n, E, gx;      // gx row chunks of 64
+  const int *live;   // cavs_gemm_desc::live of the product
+};
+
+// What a group's launch finishes by itself where it has counters: the workgroup that arrives last at a tile of a product whose K
+// is split adds up the tile's partial sums, in the order of the splits whoever is last, and scatters the tile of the
+// product that feeds the embedding's gradient.  Partial sums go past the L2 (GemmArgs::through), and the count behind
+// them; the last one puts the counter back to zero.  Column sums come along as workgroups behind the products'.
+// As launches of their own these were latency, not work -- ids, parts and atomic adds one behind the other, 4.5 us between
+// two launches.  What bounds the end of the launch now are those trips: so all parts of a tile are in flight at once (one
+// after the other: 24.6 us where it takes 19.6), and the ids are looked up in front of the product.
+//   us, products + reduction (+ scatter) (+ column sums) -> one launch, gaps not counted
+//   64 trees, H = 512 (2370 vertices): 74.0 + 15.6 -> 77.9        25 trees, H = 150: 15.6 + 13.4 -> 19.9
+//   16 chains of 20, H = 128, 1000 classes: 11.9 + 4.1 + 6.1 and 11.9 + 12.0 + 6.1 -> 27.3 together
+struct GroupFold {
+  int *counters;          // one per tile of a split product, zero; null: a launch behind this one adds up
+  int first[kGroupMax];   // the product's first
+  int embed;              // product whose tiles are scattered, or -1
+  EmbedTail tail;
+  ColsumParts sums;       // chunks > 0: its column sums by the workgroups behind the products'
+};
+
+// the partial sums of tile (m0, n0) of a product added up; thread: column lane of rows 16 wave ..
+__device__ inline void fold_tile(const GemmArgs &g, int splits, int m0, int n0) {
+  const int lane = threadIdx.x & 63, row0 = __builtin_amdgcn_readfirstlane(m0 + 16 * (threadIdx.x >> 6)), c = n0 + lane;
+  if (row0 >= g.M || c >= g.N) return;
+  const long stride = (long)g.M * g.N;
+  float acc[16];
+#pragma unroll
+  for (int u = 0; u < 16; u++) acc[u] = 0.f;
+  const ThroughRows rows{g.N, g.M - 1 - row0, 4 * c};
+  const float *p = g.ws + (long)row0 * g.N;
+  for (int z = 0; z < splits; z += 4, p += 4 * stride) {  // four parts in flight: one at a time, each is a trip to memory
+    float v[4][16];
+#pragma unroll
+    for (int k = 0; k < 4; k++) rows.load(p + (z + k < splits ? k : 0) * stride, v[k]);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if (z + k >= splits) break;
+#pragma unroll
+      for (int u = 0; u < 16; u++) acc[u] += v[k][u];
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 16; u++) {
+    if (row0 + u >= g.M) continue;
+    float *to = g.C + (row0 + u) * g.ldc + c;
+    float v = g.alpha * acc[u];
+    if (g.beta != 0.f) v += g.beta * *to;
+    *to = v;
+  }
+}
+
 template <bool VEC>
-__global__ __launch_bounds__(kThreads, 4) void sgemm_group_kernel(GemmGroup G) {
+__global__ __launch_bounds__(kThreads, 4) void sgemm_group_kernel(GemmGroup G, GroupFold F) {
   constexpr int BM = 64, BN = 64, BK = 16;
   __shared__ __attribute__((aligned(16))) char S[split_lds_bytes(BM, BN, BK)];
+  if ((int)blockIdx.x >= G.first[G.count]) {
+    const int b = blockIdx.x - G.first[G.count], across = (F.sums.w + 63) / 64;
+    return colsum_part_block(F.sums, b % across, b / across, reinterpret_cast<float(*)[64]>(S));
+  }
   int p = 0;
   while (p + 1 < G.count && (int)blockIdx.x >= G.first[p + 1]) p++;
   const int local = blockIdx.x - G.first[p];
@@ -50,15 +119,42 @@ __global__ __launch_bounds__(kThreads, 4) void sgemm_group_kernel(GemmGroup G) {
   if (local >= padded) return;
   const int w = xcd_remap(local, padded);
   if (w >= share) return;
-  const int t = w % tiles, z = w / tiles;
-  const int tilesN = (g.N + BN - 1) / BN, m0 = t / tilesN * BM, n0 = t % tilesN * BN;
+  int t = w % tiles;
+  const int z = w / tiles, tilesN = (g.N + BN - 1) / BN, m0 = t / tilesN * BM, n0 = t % tilesN * BN;
+  int mine = -1;  // (asked for in front of the product, looked at behind it)
+  if (F.counters && F.embed == p && m0 < min(F.tail.n, g.M)) mine = embed_row(F.tail.ids, min(F.tail.n, g.M), F.tail.E, m0 / kEmbedRows);
   switch (G.form[p]) {
     case 0: split_tile<BM, BN, BK, false, false, VEC, true>(g, m0, n0, z, S); break;
     case 1: split_tile<BM, BN, BK, false, true, VEC, true>(g, m0, n0, z, S); break;
     case 2: split_tile<BM, BN, BK, true, false, VEC, true>(g, m0, n0, z, S); break;
     default: split_tile<BM, BN, BK, true, true, VEC, true>(g, m0, n0, z, S); break;
   }
+  if (!F.counters) return;
+  asm volatile("" : "+s"(p), "+s"(t));  // (what follows reads its sizes again: kept over the product they cost registers)
+  const int splits = G.splits[p];
+  const bool scatter = F.embed == p;
+  if (splits == 1 && !scatter) return;
+  EmbedHot hot{0, false};
+  if (scatter) hot = embed_hot(mine);  // while the stores are on their way
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this workgroup's part of the tile has arrived
+  __syncthreads();
+  if (splits > 1) {
+    int *count = F.counters + F.first[p] + t, *last = reinterpret_cast<int *>(S);
+    if (threadIdx.x == 0) *last = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (*last != splits - 1) return;
+    if (threadIdx.x == 0) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  GemmArgs h = G.g[p];
+  apply_live(h, G.form[p] >= 2, splits);
+  const int across = (h.N + BN - 1) / BN, tm = t / across, tn = t % across;
+  if (!scatter) return fold_tile(h, splits, tm * BM, tn * BN);
+  const EmbedTail &e = F.tail;
+  const int n = min(e.n, h.M);
+  if (tm * BM >= n) return;
+  embed_bwd_rows<true>(e.dtable, mine, [&] { return hot; }, e.dy, e.ld_dy, e.parts, (long)h.M * h.N, e.copy, e.ld_copy, n, e.E, tm, tn);
 }
+static_assert(kEmbedRows == 64 && kEmbedCols == 64, "a tile of a group is a block of the scatter-add");
 
 // p[0] + p[stride] + ... in that order, four loads in flight at a time (one at a time, a reduction over
 // four splits was four trips to memory in a row)
@@ -113,21 +209,6 @@ __global__ __launch_bounds__(256) void mfma_probe_kernel(float *__restrict__ out
     for (int r = 0; r < 16; r++) s += acc[i][r];
   out[(long)blockIdx.x * blockDim.x + threadIdx.x] = s;
 }
-
-// The embedding gradient behind one product of a group (cavs_sgemm_group_embed_bwd): the rows of
-// that product's result are scatter-added into the table by extra workgroups of the launch that
-// reduces the other products' K splits, reading the product's own partials directly.
-struct EmbedTail {
-  float *dtable;
-  const float *ids;
-  const float *dy;   // the result, or the first of `parts` partial results `part_stride` floats apart
-  long ld_dy, part_stride;
-  int parts;
-  float *copy;       // where the summed result goes as well (the product's C) when parts > 1
-  long ld_copy;
-  int n, E, gx;      // gx row chunks of 64
-  const int *live;   // cavs_gemm_desc::live of the product
-};
 
 __global__ __launch_bounds__(256) void splitk_reduce_group_embed_kernel(GemmGroup R, EmbedTail e) {
   const int nred = R.first[R.count];
@@ -533,8 +614,9 @@ static int run_gemm(const char *who, int tA, int tB, int M, int N, int K, float 
 // together are about four per CU (what a CU holds at once; inside a training step eight per CU
 // measured no better, though it is in a back-to-back loop), each with at least 256 of K.
 // `tail_product` >= 0: that product's result is handed on to the embedding scatter-add (dtable, ids)
+// and `counters` [n_counters]: the group's launch adds up its splits itself where they are enough (GroupFold)
 static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_bytes, size_t *need_out, void *stream,
-                     int tail_product = -1, float *dtable = nullptr, const float *ids = nullptr) {
+                     int tail_product = -1, float *dtable = nullptr, const float *ids = nullptr, int *counters = nullptr, int n_counters = 0, const cavs_colsum_desc *sums = nullptr) {
   CAVS_REQUIRE(count >= 0 && count <= kGroupMax, "cavs_sgemm_group: %d products, at most %d", count, kGroupMax);
   CAVS_REQUIRE(count == 0 || d, "cavs_sgemm_group: null descriptors");
   EmbedTail tail{};
@@ -548,6 +630,9 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
                      q.live};
   }
   GemmGroup G{}, R{};
+  GroupFold F{};
+  F.embed = -1;
+  long split_tiles = 0;
   // K as the plan sees it, and the number of tiles it expects (cavs_gemm_desc::live)
   auto plan_K = [](const cavs_gemm_desc &q) { return q.live && q.transA ? std::min(q.K, std::max(q.live_expect, 1)) : q.K; };
   auto plan_tiles = [](const cavs_gemm_desc &q) {
@@ -577,8 +662,9 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
   for (int p = 0; p < count; p++) {
     const cavs_gemm_desc &q = d[p];
     if (q.M == 0 || q.N == 0) continue;
-    if (!alone[p] && grouped >= 2) {
+    if (!alone[p] && (grouped >= 2 || counters || need_out)) {
       work += (double)plan_tiles(q) * plan_K(q);
+      if (grouped < 2 && need_out) most = std::max(most, plan_workspace(plan_product(q), q.M, q.N));  // (for either way)
       continue;
     }
     alone[p] = true;
@@ -608,6 +694,9 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
   };
   if (launch_size(1L << 30) <= slots)
     while (launch_size(kc) > slots) kc += 32;
+  // Few workgroups: a step of K is a latency then, not work (the head of 840 vertices, H = 224, 23 classes, 72 workgroups: 14.7 us in
+  // chunks of 256, 12.4 in chunks of 128)
+  while (kc > 128 && launch_size(kc / 2) <= 2 * num_cus()) kc /= 2;
   size_t need = 0;
   bool vec = true;
   int n = 0, nr = 0;
@@ -634,6 +723,11 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
     G.splits[n] = splits;
     G.form[n] = (q.transA ? 2 : 0) + (q.transB ? 1 : 0);
     G.first[n + 1] = G.first[n] + (int)((tiles[p] * splits + 7) / 8 * 8);
+    if (splits > 1) {
+      F.first[n] = (int)split_tiles;
+      split_tiles += tiles[p];
+    }
+    if (p == tail_product) F.embed = n;
     n++;
     if (splits > 1 && p == tail_product && !need_out) {
       // the scatter-add sums this product's partials itself (and leaves the sum in C as well)
@@ -669,12 +763,29 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
     if (rc) return rc;
   }
   hipStream_t st = as_stream(stream);
+  bool with_tail = tail_product >= 0 && tail.n > 0 && tail.E > 0;
+  if (counters && n > 0 && split_tiles <= n_counters) {
+    F.counters = counters;
+    F.tail = tail;
+    if (!with_tail) F.embed = -1;
+    if (F.embed >= 0) with_tail = false;
+    for (int p = 0; p < n; p++) G.g[p].through = G.splits[p] > 1;
+    nr = R.count = 0;
+  }
+  unsigned grid = G.first[n];
+  if (sums && sums->n > 0 && n > 0) {
+    F.sums = colsum_job(sums->parts, sums->inp, sums->ld, sums->n, sums->w);
+    grid += (unsigned)((sums->w + 63) / 64 * F.sums.chunks);
+  } else if (sums) {
+    int rc = cavs_colsum_blocks(nullptr, sums->inp, sums->ld, sums->n, sums->w, 1, nullptr, sums->parts,
+                                cavs_colsum_blocks_workspace(sums->n, sums->w, 1), stream);
+    if (rc) return rc;
+  }
   if (n > 0) {
-    if (vec) launch(sgemm_group_kernel<true>, (unsigned)G.first[n], kThreads, 0, st, G);
-    else launch(sgemm_group_kernel<false>, (unsigned)G.first[n], kThreads, 0, st, G);
+    if (vec) launch(sgemm_group_kernel<true>, grid, kThreads, 0, st, G, F);
+    else launch(sgemm_group_kernel<false>, grid, kThreads, 0, st, G, F);
     CAVS_LAUNCH_CHECK();
   }
-  const bool with_tail = tail_product >= 0 && tail.n > 0 && tail.E > 0;
   if (with_tail) {
     const int gy = (tail.E + kEmbedCols - 1) / kEmbedCols;
     launch(splitk_reduce_group_embed_kernel, (unsigned)(R.first[nr] + tail.gx * gy), 256, 0, st, R, tail);
@@ -759,6 +870,14 @@ size_t cavs_sgemm_group_workspace(int count, const cavs_gemm_desc *products) {
 int cavs_sgemm_group(int count, const cavs_gemm_desc *products, void *workspace, size_t workspace_bytes,
                      void *stream) {
   return run_group(count, products, workspace, workspace_bytes, nullptr, stream);
+}
+
+int cavs_sgemm_group_once(int count, const cavs_gemm_desc *products, int embed_product, float *dtable, const float *ids, void *workspace,
+                          size_t workspace_bytes, int *counters, int n_counters, const cavs_colsum_desc *sums, void *stream) {
+  CAVS_REQUIRE(counters && n_counters >= 0, "cavs_sgemm_group_once: null counters");
+  CAVS_REQUIRE(!sums || (sums->n >= 0 && sums->w > 0 && sums->ld >= sums->w && sums->parts && (sums->inp || sums->n == 0)),
+               "cavs_sgemm_group_once: bad column sums");
+  return run_group(count, products, workspace, workspace_bytes, nullptr, stream, embed_product, dtable, ids, counters, n_counters, sums);
 }
 
 int cavs_sgemm_group_beside(int count, const cavs_gemm_desc *products, void *workspace, size_t workspace_bytes,

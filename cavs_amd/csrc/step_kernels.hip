@@ -6,6 +6,7 @@
 // launches their fixed costs add up to more than a round of the vertex function.
 #include <vector>
 
+#include "colsum_common.h"
 #include "common.h"
 #include "round_common.h"
 
@@ -416,24 +417,9 @@ struct BlockMap {
   int dst[8];
 };
 
-__global__ __launch_bounds__(256) void colsum_part_kernel(float *__restrict__ part, const float *__restrict__ inp,
-                                                          long ld, int n, int w, int rows_per_chunk) {
-  __shared__ float s[4][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int col = blockIdx.x * 64 + lane;
-  const int r0 = blockIdx.y * rows_per_chunk, r1 = min(n, r0 + rows_per_chunk);
-  float a0 = 0.f, a1 = 0.f;
-  if (col < w) {
-    int r = r0 + wave;
-    for (; r + 4 < r1; r += 8) {
-      a0 += inp[(long)r * ld + col];
-      a1 += inp[(long)(r + 4) * ld + col];
-    }
-    for (; r < r1; r += 4) a0 += inp[(long)r * ld + col];
-  }
-  s[wave][lane] = a0 + a1;
-  __syncthreads();
-  if (wave == 0 && col < w) part[(long)blockIdx.y * w + col] = (s[0][lane] + s[1][lane]) + (s[2][lane] + s[3][lane]);
+__global__ __launch_bounds__(256) void colsum_part_kernel(ColsumParts s) {
+  __shared__ float lds[4][64];
+  colsum_part_block(s, blockIdx.x, blockIdx.y, lds);
 }
 
 __global__ __launch_bounds__(256) void colsum_blocks_reduce_kernel(float *__restrict__ out, const float *__restrict__ part,
@@ -447,11 +433,6 @@ __global__ __launch_bounds__(256) void colsum_blocks_reduce_kernel(float *__rest
   s[q][o] = a;
   __syncthreads();
   if (q == 0 && col < w) out[map.dst[col / bw] * bw + col % bw] = (s[0][o] + s[1][o]) + (s[2][o] + s[3][o]);
-}
-
-static int colsum_chunks(int n) {
-  int c = (n + 127) / 128;
-  return c < 1 ? 1 : (c > 32 ? 32 : c);
 }
 
 }  // namespace cavs
@@ -681,10 +662,9 @@ int cavs_colsum_blocks(float *out, const float *inp, int ld, int n, int bw, int 
   if (n == 0) return out ? cavs_zero(out, (size_t)w * 4, stream) : (workspace ? cavs_zero(workspace, need, stream) : CAVS_OK);
   CAVS_REQUIRE(inp, "cavs_colsum_blocks: null input");
   CAVS_REQUIRE(workspace && workspace_bytes >= need, "cavs_colsum_blocks: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
-  const int rpc = ((n + chunks - 1) / chunks + 3) / 4 * 4;
   hipStream_t st = as_stream(stream);
   float *part = static_cast<float *>(workspace);
-  launch(colsum_part_kernel, dim3((w + 63) / 64, chunks), 256, 0, st, part, inp, ld, n, w, rpc);
+  launch(colsum_part_kernel, dim3((w + 63) / 64, chunks), 256, 0, st, colsum_job(part, inp, ld, n, w));
   CAVS_LAUNCH_CHECK();
   if (!out) return CAVS_OK;  // the chunk sums stay in the workspace
   launch(colsum_blocks_reduce_kernel, (w + 63) / 64, 256, 0, st, out, part, chunks, w, bw, map);

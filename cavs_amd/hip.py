@@ -35,6 +35,12 @@ TASK_SGD_TRANSPOSE = 9
 TASK_GUARD = 10
 
 
+class ColsumDesc(C.Structure):
+    """cavs_colsum_desc: column sums that ride in a launch of products"""
+
+    _fields_ = [("parts", C.c_void_p), ("inp", C.c_void_p), ("ld", C.c_int), ("n", C.c_int), ("w", C.c_int)]
+
+
 class GemmDesc(C.Structure):
     """cavs_gemm_desc: one product of cavs_sgemm_group"""
     _fields_ = [("transA", _I), ("transB", _I), ("M", _I), ("N", _I), ("K", _I), ("alpha", _F), ("beta", _F),
@@ -96,6 +102,7 @@ _SIGS = {
     "cavs_sgemm_group": [_I, C.POINTER(GemmDesc), _P, _Z, _P],
     "cavs_sgemm_group_beside": [_I, C.POINTER(GemmDesc), _P, _Z, _P],
     "cavs_sgemm_group_embed_bwd": [_I, C.POINTER(GemmDesc), _I, _P, _P, _P, _Z, _P],
+    "cavs_sgemm_group_once": [_I, C.POINTER(GemmDesc), _I, _P, _P, _P, _Z, _P, _I, C.POINTER(ColsumDesc), _P],
     "cavs_sgemm_splitk": [_I, _I, _I, _I, _I, _F, _P, _I, _P, _I, _F, _P, _I, _P, _Z, _P],
     "cavs_sgemm_splitk_static": [_I, _I, _I, _I, _I, _F, _P, _I, _P, _I, _F, _P, _I, _P],
     "cavs_colsum": [_P, _P, _I, _I, _I, _I, _P],

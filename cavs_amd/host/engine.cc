@@ -490,21 +490,22 @@ static double hinted_flops(const cavs_gemm_desc &q) {
   return 2.0 * mnk;
 }
 
-void Engine::gemm_group(const std::vector<cavs_gemm_desc> &products) {
+// of the grouped products on stream_: a list has at most 4 x 256 workgroups, or is whole tiles
+int *Engine::group_counters() {
+  if (gemm_counters_.reserve(kGroupCounters)) check(cavs_zero(gemm_counters_.get(), kGroupCounters * sizeof(int), stream_));
+  return gemm_counters_.get();
+}
+
+void Engine::gemm_group(const std::vector<cavs_gemm_desc> &products, const cavs_colsum_desc *sums) {
   const int count = (int)products.size();
   float *ws = workspace(cavs_sgemm_group_workspace(count, products.data()));
   ProfScope ps(this, K_GEMM);
-  check(cavs_sgemm_group(count, products.data(), ws, ws_.capacity() * 4, stream_));
+  check(cavs_sgemm_group_once(count, products.data(), -1, nullptr, nullptr, ws, ws_.capacity() * 4, group_counters(), kGroupCounters, sums, stream_));
   for (const cavs_gemm_desc &q : products) {
     c_gemm_flops_ += desc_flops(q);
     c_gemm_flops_hinted_ += hinted_flops(q);
   }
   c_launches_ += 1;
-}
-
-void Engine::gemm_splitk(int tA, int tB, int M, int N, int K, const float *A, int lda,
-                         const float *B, int ldb, float *C, int ldc) {
-  gemm(tA, tB, M, N, K, A, lda, B, ldb, 0.f, C, ldc);
 }
 
 void Engine::gather(float *out, int ld_out, const float *src, int ld_src, const int *ids, int n,
@@ -1779,16 +1780,22 @@ bool Engine::bias_row_ok() const {
   return w.g == w.own_g.get();
 }
 
-// One launch leaves the chunk sums; the job that ends the step adds them up in index order.
-void Engine::bias_gradient(const std::string &name, const float *inp, int n, int w, DeviceArray<float> &parts, void *stream) {
+// Chunk sums, for a launch to leave behind (bias_gradient, or one of products); the job that ends the step adds them up in
+// index order.
+cavs_colsum_desc Engine::bias_sums(const std::string &name, const float *inp, int n, int w, DeviceArray<float> &parts) {
   const size_t bytes = cavs_colsum_blocks_workspace(n, w, 1);
   if (parts.capacity() * 4 < bytes) {
     check(cavs_stream_sync(stream_));
     parts.reserve(bytes / 4 + 1);
   }
-  check(cavs_colsum_blocks(nullptr, inp, w, n, w, 1, nullptr, parts.get(), parts.capacity() * 4, stream ? stream : stream_));
-  c_launches_ += 1;
   bias_jobs_.push_back({name, parts.get(), cavs_colsum_parts(n), w, 1, 0});
+  return {parts.get(), inp, w, n, w};
+}
+
+void Engine::bias_gradient(const std::string &name, const float *inp, int n, int w, DeviceArray<float> &parts, void *stream) {
+  const cavs_colsum_desc s = bias_sums(name, inp, n, w, parts);
+  check(cavs_colsum_blocks(nullptr, inp, w, n, w, 1, nullptr, s.parts, parts.capacity() * 4, stream));
+  c_launches_ += 1;
 }
 
 // out [w] = column sums of inp [n, w], chunks of rows added in index order
@@ -1859,7 +1866,7 @@ void Engine::backward_prologue(std::vector<cavs_task> tasks, bool with_embedding
 
 // `products[0]` is de = dxW * W^T; its rows go on into the embedding gradient in the launch that
 // reduces the group's K splits (cavs_sgemm_group_embed_bwd).
-void Engine::gemm_group_embedding_backward(const std::vector<cavs_gemm_desc> &products, int E) {
+void Engine::gemm_group_embedding_backward(const std::vector<cavs_gemm_desc> &products, int E, const cavs_colsum_desc *sums) {
   Param &emb = param("Emb");
   const bool owned = emb.g == emb.own_g.get();
   if (emb_cleared_) {
@@ -1876,13 +1883,13 @@ void Engine::gemm_group_embedding_backward(const std::vector<cavs_gemm_desc> &pr
   {
     ProfScope ps(this, K_GEMM);
     const float *ids = words_ ? reinterpret_cast<const float *>(d_words_index_ + 4 + 3 * (size_t)N_) : xs_.get();
-    check(cavs_sgemm_group_embed_bwd(count, products.data(), 0, emb.g, ids, ws, ws_.capacity() * 4, stream_));
+    check(cavs_sgemm_group_once(count, products.data(), 0, emb.g, ids, ws, ws_.capacity() * 4, group_counters(), kGroupCounters, sums, stream_));
   }
   for (const cavs_gemm_desc &q : products) {
     c_gemm_flops_ += desc_flops(q);
     c_gemm_flops_hinted_ += hinted_flops(q);
   }
-  c_launches_ += 2;
+  c_launches_ += 1;
   xs_.swap(xs_prev_);  // this step's ids: the rows that are dirty now
   emb_dirty_n_ = N_;
   emb_sparse_valid_ = owned;
@@ -2054,13 +2061,13 @@ void Engine::lstm_backward() {
     dx = d_words_.get();
     live = d_words_index_;
   }
-  gemm_group_embedding_backward({
+  const cavs_colsum_desc sums = bias_sums("Bv", dxW_.get(), N, 4 * H, bias_parts_);
+  last_launch(3, true, [&] { gemm_group_embedding_backward({
       {0, 1, N, E, 4 * H, 1.f, 0.f, dx, 4 * H, Wx, 4 * H, de_.get(), E, 0, 0, 0, live, words_expected()},
       {1, 0, E, 4 * H, N, 1.f, 0.f, e_.get(), E, dx, 4 * H, dW, 4 * H, 0, 0, 0, live, words_expected()},
       {1, 0, H, 4 * H, N - lp, 1.f, 0.f, G_.at((size_t)lp * 2 * H), 2 * H, dxW_.at((size_t)lp * 4 * H), 4 * H,
        dW + (size_t)4 * H * E, 4 * H},
-  }, E);
-  last_launch(3, true, [&] { bias_gradient("Bv", dxW_.get(), N, 4 * H, bias_parts_); });
+  }, E, &sums); });
 }
 
 // ------------------------------------------------------------------ Tree-FC
@@ -2184,11 +2191,10 @@ void Engine::treefc_backward() {
     scatter(dpool_.get(), H, d_child_ + 2 * off, r_dG_.get(), H, 2 * r.n, H);
   }
   const int lp = sched_->leaf_prefix;
-  gemm_splitk(1, 0, 2 * H, H, N - lp, G_.at((size_t)2 * lp * H), 2 * H, dxW_.at((size_t)lp * H), H,
-              param("W").g, H);
-  if (cfg_.use_bias) {
-    last_launch(3, true, [&] { bias_gradient("Bv", dxW_.get(), N, H, bias_parts_); });
-  }
+  const cavs_gemm_desc dW{1, 0, 2 * H, H, N - lp, 1.f, 0.f, G_.at((size_t)2 * lp * H), 2 * H, dxW_.at((size_t)lp * H), H, param("W").g, H};
+  cavs_colsum_desc sums;
+  if (cfg_.use_bias) sums = bias_sums("Bv", dxW_.get(), N, H, bias_parts_);
+  last_launch(3, true, [&] { gemm_group({dW}, cfg_.use_bias ? &sums : nullptr); });
 }
 
 // ------------------------------------------------------------------ a vertex function on generated kernels
@@ -2585,8 +2591,8 @@ void Engine::head_forward_backward(bool backward) {
         aux_pending_ = true;
       } else {
         // both read d logits and write different outputs: one launch when they are small
-        gemm_group({dWd, dGd});
-        last_launch(2, true, [&] { bias_gradient("bfc", dlogits_.get(), N, C, head_bias_parts_); });
+        const cavs_colsum_desc sums = bias_sums("bfc", dlogits_.get(), N, C, head_bias_parts_);
+        last_launch(2, true, [&] { gemm_group({dWd, dGd}, &sums); });
       }
     }
     return;

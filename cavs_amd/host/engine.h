@@ -134,10 +134,8 @@ class Engine {
   void gemm(int tA, int tB, int M, int N, int K, const float *A, int lda, const float *B, int ldb,
             float beta, float *C, int ldc);
   // independent products in one launch (cavs_sgemm_group)
-  void gemm_group(const std::vector<cavs_gemm_desc> &products);
+  void gemm_group(const std::vector<cavs_gemm_desc> &products, const cavs_colsum_desc *sums = nullptr);
   void backward_prologue(std::vector<cavs_task> tasks, bool with_embedding);
-  void gemm_splitk(int tA, int tB, int M, int N, int K, const float *A, int lda, const float *B,
-                   int ldb, float *C, int ldc);
   void gather(float *out, int ld_out, const float *src, int ld_src, const int *ids, int n, int w);
   void scatter(float *dst, int ld_dst, const int *ids, const float *inp, int ld_inp, int n, int w);
   bool leaf_round(const Round &r) const {
@@ -422,12 +420,13 @@ class Engine {
   std::vector<BiasJob> bias_jobs_;
   DeviceArray<float> bias_parts_, head_bias_parts_;
   // column sums of inp [n, w] as the gradient of `name`, in a fixed order
-  void bias_gradient(const std::string &name, const float *inp, int n, int w, DeviceArray<float> &parts, void *stream = nullptr);
+  cavs_colsum_desc bias_sums(const std::string &name, const float *inp, int n, int w, DeviceArray<float> &parts);
+  void bias_gradient(const std::string &name, const float *inp, int n, int w, DeviceArray<float> &parts, void *stream);
   void colsum_fixed(float *out, const float *inp, int n, int w);
   bool has_bias_job(const std::string &name) const;
   void settle_bias_jobs(float lr, std::vector<cavs_task> *tasks);
   DeviceArray<float> head_parts_;         // weight-gradient partials of the classifier head
-  void gemm_group_embedding_backward(const std::vector<cavs_gemm_desc> &products, int E);
+  void gemm_group_embedding_backward(const std::vector<cavs_gemm_desc> &products, int E, const cavs_colsum_desc *sums = nullptr);
   DeviceArray<float> UT_;  // transposed recurrent weights for the fused backward rounds
   // The recurrent weights (Tree-LSTM: U; chain LSTM: W') tile-major for the packed forward rounds.
   // Written by the job that applies their SGD update; current while nobody else has written them
@@ -472,6 +471,9 @@ class Engine {
   // the update launch (or whoever reads the gradients first) waits for.
   void *aux_stream_ = nullptr, *aux_fork_ev_ = nullptr, *aux_join_ev_ = nullptr;
   bool aux_pending_ = false;   // work on the side stream that the session's stream has not waited for yet
+  static constexpr int kGroupCounters = 1024;
+  DeviceArray<int> gemm_counters_;
+  int *group_counters();
   DeviceArray<float> ws_aux_;  // its products' split-K workspace
   void aux_join();
   void aux_open();  // creates the side stream and its events

@@ -236,6 +236,20 @@ int cavs_sgemm_group_beside(int count, const cavs_gemm_desc *products, void *wor
 int cavs_sgemm_group_embed_bwd(int count, const cavs_gemm_desc *products, int embed_product,
                                float *dtable, const float *ids, void *workspace,
                                size_t workspace_bytes, void *stream);
+/* cavs_sgemm_group_embed_bwd (embed_product < 0: cavs_sgemm_group) with what adds up the K splits and scatters in the
+ * products' own launch: the workgroup that is last at a tile does it.  counters: n_counters ints of device memory
+ * that are zero before the first call and zero again behind each; one set serves the calls on one stream.  Lists with more
+ * split tiles than counters, and products that run alone, take the launches of the entry points above.  Same results
+ * bit for bit, but for the order of the scatter's atomic adds and where a list of one product is cut.
+ * sums (may be null): the chunk sums that cavs_colsum_blocks(out = null) leaves of `inp` [n, w], in the same launch. */
+typedef struct {
+  float *parts;  /* cavs_colsum_parts(n) rows of w */
+  const float *inp;
+  int ld, n, w;
+} cavs_colsum_desc;
+int cavs_sgemm_group_once(int count, const cavs_gemm_desc *products, int embed_product, float *dtable, const float *ids,
+                          void *workspace, size_t workspace_bytes, int *counters, int n_counters, const cavs_colsum_desc *sums,
+                          void *stream);
 /* C[r,:] = op(A)*op(B) + D[r >> d_shift, :]: the GEMM and the Accumulate that
  * follows it in the backward of a Mirror'ed operand
  * (cavs/backend/op_decl_slice_join.cc:173-182) in one pass.  Workspace as above. */

@@ -481,6 +481,57 @@ def test_sgemm_group_with_the_embedding_gradient_behind_one_product(g, name, k):
         g.call("cavs_sgemm_group_embed_bwd", len(shapes), descs, k, g.P(table), g.P(d_ids), g.P(ws), nbytes, g.stream())
 
 
+@pytest.mark.parametrize("room", [1024, 0])
+@pytest.mark.parametrize("name,k", [("treelstm_step", 0), ("treelstm_step", -1), ("ragged", 0), ("mixed", 1), ("mixed", 0), ("mixed", -1)])
+def test_a_group_that_adds_up_its_own_splits(g, name, k, room):
+    """cavs_sgemm_group_once: column sums ride along; the last workgroup at a tile reduces it, in the order of the launch behind cavs_sgemm_group (the same
+    bits), and scatters the product that feeds the table; the counters are zero again, so the next call finds them so.  With
+    room for no counter it is the launches of the other entry points."""
+    import torch
+
+    shapes = GROUPS[name]
+    r = rng(len(name) * 11 + k + 2)
+    descs = (hip.GemmDesc * len(shapes))()
+    keep, outs = [], []
+    for p, (tA, tB, M, N, K) in enumerate(shapes):
+        A, B = r.bulk_uniform(max(M * K, 1), -1, 1), r.bulk_uniform(max(N * K, 1), -1, 1)
+        keep += [g.devf(A), g.devf(B)]
+        outs.append(torch.empty((max(M, 1), N + 4), dtype=torch.float32, device="cuda"))
+        descs[p] = hip.GemmDesc(tA, tB, M, N, K, 1.0, 0.0, g.P(keep[-2]), max(M if tA else K, 1), g.P(keep[-1]), max(K if tB else N, 1), g.P(outs[p]), N + 4)
+    n, E, V = (shapes[k][2], shapes[k][3], 97) if k >= 0 else (0, 1, 1)
+    ids = np.floor(r.bulk_uniform(max(n, 1)) * V).astype(np.float32)
+    ids[:n // 2] = 3.0
+    d_ids = g.devf(ids)
+    nbytes = hip.lib().cavs_sgemm_group_workspace(len(shapes), descs)
+    ws = torch.empty(max(nbytes // 4, 1), dtype=torch.float32, device="cuda")
+    counters = torch.zeros(1024, dtype=torch.int32, device="cuda")
+    sn, sw = (1300, 130) if room else (7, 64)
+    d_sum = g.devf(r.bulk_uniform(sn * sw, -1, 1))
+    nparts = hip.lib().cavs_colsum_parts(sn)
+    want_parts, parts = (torch.zeros(nparts * sw, dtype=torch.float32, device="cuda") for _ in range(2))
+    g.call("cavs_colsum_blocks", None, g.P(d_sum), sw, sn, sw, 1, None, g.P(want_parts), nparts * sw * 4, g.stream())
+    sums = hip.ColsumDesc(g.P(parts), g.P(d_sum), sw, sn, sw)
+    g.call("cavs_sgemm_group", len(shapes), descs, g.P(ws), nbytes, g.stream())
+    want = [g.host(o) for o in outs]
+    for turn in range(3):
+        table0 = r.bulk_normal(V * E).reshape(V, E)
+        table = g.devf(table0)
+        for o in outs:
+            o.fill_(float("nan"))
+        g.call("cavs_sgemm_group_once", len(shapes), descs, k, g.P(table), g.P(d_ids), g.P(ws), nbytes, g.P(counters), room,
+               sums if turn else None, g.stream())
+        assert not turn or torch.equal(parts, want_parts)
+        parts.zero_()
+        for p, (_, _, M, N, _) in enumerate(shapes):
+            if M:
+                np.testing.assert_array_equal(g.host(outs[p])[:, :N], want[p][:, :N])
+        assert not counters.any()
+        if n:
+            ref = table0.astype(np.float64)
+            np.add.at(ref, ids.astype(np.int64), want[k][:n, :E].astype(np.float64))
+            close(g.host(table), ref, "table")
+
+
 @pytest.mark.parametrize("tA,tB,M,N,K", [(0, 0, 30, 1536, 512), (0, 1, 8, 512, 1536), (0, 1, 130, 512, 512),
                                           (0, 0, 1, 64, 4096), (1, 1, 40, 72, 640), (0, 0, 33, 40, 300),
                                           (0, 1, 65, 33, 68), (0, 0, 600, 1536, 512), (0, 1, 1200, 512, 1536),
