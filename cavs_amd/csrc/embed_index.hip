@@ -2,8 +2,8 @@
 // parse tree looks up row 0, text repeats its frequent words) is multiplied by W once, the gradients
 // of the vertices that read it are added up first, and the products of the backward pass run over words
 // instead of vertices.
-//   cavs_embed_index   sorts the vertices by id, in one workgroup: three to four sweeps of a radix sort
-//                      with stable ranks, then the segments of equal ids
+//   cavs_embed_index   sorts the vertices by id: up to three sweeps of a radix sort with stable ranks,
+//                      then the segments of equal ids; in one workgroup while it all fits LDS
 //   cavs_embed_words   the table rows of the words
 //   cavs_spread_rows   a word's row of x * W to every vertex that looked it up
 //   cavs_gather_sums   a word's gradient row: the sum over its vertices, in vertex order
@@ -14,9 +14,9 @@
 namespace cavs {
 
 constexpr int kIndexThreads = 1024, kIndexWaves = kIndexThreads / 64;
-// Up to kIndexLds rows (and ids below kIndexKeys) are sorted in LDS, id and row packed in a word; more go
-// through memory (the L2 of one XCD).
-constexpr int kIndexLds = 16384, kIndexKeys = 1 << 18;
+// Up to kIndexLds rows (and ids below kIndexKeys) are sorted in LDS, id and row packed in a word, in one launch; more
+// by the launches of index_sort_* and index_words_*.  us, one launch / seven: 4096 rows 20.6 / 29.3, 7088 31.9 / 30.7, 9000 39.0 / 31.8.
+constexpr int kIndexLds = 8192, kIndexKeys = 1 << 19;
 
 // Lanes of `active` whose low `bits` bits of d equal this lane's.
 __device__ inline unsigned long long match_lanes(unsigned d, unsigned long long active) {
@@ -52,31 +52,28 @@ __device__ inline unsigned block_scan(unsigned v, unsigned *wave_sums, unsigned 
   return base + incl - v;
 }
 
+// a row whose id is no whole number in [0, V) is a word of its own
+__device__ inline unsigned word_key(float id, int V) {
+  const int k = (int)id;
+  return (id >= 0.f && id < (float)V && (float)k == id) ? k : V;
+}
+
 // One workgroup.  A row whose id is no whole number in [0, V) is a word of its own (key V).  What bounds
 // it is the chain of sweeps (about 1 us each), not the work: every wavefront takes one stretch of the rows in
 // order, so that ranks are stable without a second pass.
-template <bool SMALL>
 __global__ __launch_bounds__(kIndexThreads) void embed_index_kernel(int *__restrict__ index, float *__restrict__ ids_out,
                                                                     const float *__restrict__ x, const int *__restrict__ rows, int n, int V,
-                                                                    int leaf_rows, int passes, unsigned *__restrict__ scratch) {
-  __shared__ unsigned lds[SMALL ? 2 * kIndexLds : 1];
+                                                                    int leaf_rows, int passes) {
+  __shared__ unsigned lds[2 * kIndexLds];
   __shared__ unsigned hist[kIndexWaves][256];
   __shared__ unsigned wave_sums[kIndexWaves], first_sums[kIndexWaves], leaf_sums[kIndexWaves];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const unsigned long long below = (1ull << lane) - 1;
   // row i: id key(i), vertex row val(i)
-  unsigned *ka = SMALL ? lds : scratch, *va = scratch + n;
-  unsigned *kb = SMALL ? lds + kIndexLds : scratch + 2 * (long)n, *vb = scratch + 3 * (long)n;
-  auto key = [&](int i) { return SMALL ? ka[i] / kIndexLds : ka[i]; };
-  auto val = [&](int i) { return SMALL ? ka[i] % kIndexLds : va[i]; };
-  auto put = [&](unsigned *k, unsigned *v, int i, unsigned id, unsigned row) {
-    if constexpr (SMALL) {
-      k[i] = id * kIndexLds + row;
-    } else {
-      k[i] = id;
-      v[i] = row;
-    }
-  };
+  unsigned *ka = lds, *kb = lds + kIndexLds;
+  auto key = [&](int i) { return ka[i] / kIndexLds; };
+  auto val = [&](int i) { return ka[i] % kIndexLds; };
+  auto put = [&](unsigned *k, int i, unsigned id, unsigned row) { k[i] = id * kIndexLds + row; };
   int *slot = index + 4, *order = slot + n, *at = order + n;
   float *word = reinterpret_cast<float *>(at + n);
   const int per = ((n + kIndexWaves - 1) / kIndexWaves + 63) / 64 * 64;
@@ -85,9 +82,8 @@ __global__ __launch_bounds__(kIndexThreads) void embed_index_kernel(int *__restr
 #pragma unroll 4
   for (int i = beg + lane; i < end; i += 64) {
     const float id = x[rows[i]];
-    const int k = (int)id;
     ids_out[i] = id;
-    put(ka, va, i, (id >= 0.f && id < (float)V && (float)k == id) ? k : V, i);
+    put(ka, i, word_key(id, V), i);
   }
   for (int pass = 0; pass < passes; pass++) {
     const int shift = 8 * pass;
@@ -116,13 +112,12 @@ __global__ __launch_bounds__(kIndexThreads) void embed_index_kernel(int *__restr
       if (in) {
         const int rank = __popcll(m & below);
         const unsigned pos = hist[wave][d] + rank;
-        put(kb, vb, pos, k, v);
+        put(kb, pos, k, v);
         if ((m & ~below & ~(1ull << lane)) == 0) hist[wave][d] = pos + 1;  // (the last of its digit in this step)
       }
     }
     __syncthreads();
     unsigned *t = ka; ka = kb; kb = t;
-    t = va; va = vb; vb = t;
   }
   // Segments of equal ids.  The words no inner vertex looked up come first (their rows of the f columns are
   // zero, as those of the leaves): rows of a segment ascend, so its last one tells.
@@ -179,6 +174,189 @@ __global__ __launch_bounds__(kIndexThreads) void embed_index_kernel(int *__restr
       }
     }
     __syncthreads();
+  }
+}
+
+// The same over many workgroups: a launch per dependent step.  Workgroup g has one stretch of the rows (SortWork), its wavefronts
+// parts of it in order; a digit's rows go behind those of the digits before and of the stretches before, both
+// counted from the table of counts that the launch before left.  Bound by the launches, 5 us each: 16384 rows 33 us, 73000 37,
+// 300000 55, where one workgroup, its rows in memory, took 65, 363 (540 inside a step) and 2090.
+struct SortWork {
+  unsigned *ka, *va, *kb, *vb;  // [n] ids and rows, from and to
+  unsigned *counts;             // [groups][256] rows of a digit in a stretch; then [groups][2] words that begin, words of leaves only
+  int n, per, groups;           // rows of a stretch: a multiple of 1024
+  __device__ inline void stretch(int *beg, int *end) const {
+    const int own = per / kIndexWaves;
+    *beg = min(n, (int)blockIdx.x * per + (int)(threadIdx.x >> 6) * own);
+    *end = min(n, *beg + own);
+  }
+};
+constexpr int kSortGroups = 256;
+static int sort_per(int n) { return std::max(1, (n + kSortGroups * 1024 - 1) / (kSortGroups * 1024)) * 1024; }
+static int sort_groups(int n) { return (n + sort_per(n) - 1) / sort_per(n); }
+
+template <bool FIRST>
+__global__ __launch_bounds__(kIndexThreads) void index_sort_count_kernel(SortWork s, float *__restrict__ ids_out, const float *__restrict__ x,
+                                                                         const int *__restrict__ rows, int V, int shift) {
+  __shared__ unsigned hist[256];
+  if (threadIdx.x < 256) hist[threadIdx.x] = 0;
+  __syncthreads();
+  int beg, end;
+  s.stretch(&beg, &end);
+#pragma unroll 4
+  for (int i = beg + (threadIdx.x & 63); i < end; i += 64) {
+    unsigned k;
+    if constexpr (FIRST) {
+      const float id = x[rows[i]];
+      ids_out[i] = id;
+      k = word_key(id, V);
+      s.ka[i] = k;
+      s.va[i] = i;
+    } else {
+      k = s.ka[i];
+    }
+    atomicAdd(&hist[(k >> shift) & 255], 1u);
+  }
+  __syncthreads();
+  if (threadIdx.x < 256) s.counts[blockIdx.x * 256 + threadIdx.x] = hist[threadIdx.x];
+}
+
+__global__ __launch_bounds__(kIndexThreads) void index_sort_place_kernel(SortWork s, int shift) {
+  __shared__ unsigned hist[kIndexWaves][256];
+  __shared__ unsigned wave_sums[kIndexWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = blockIdx.x;
+  const unsigned long long below = (1ull << lane) - 1;
+  int beg, end;
+  s.stretch(&beg, &end);
+  for (int i = tid; i < kIndexWaves * 256; i += kIndexThreads) (&hist[0][0])[i] = 0;
+  const int d = tid >> 2, part = tid & 3;  // four lanes a digit
+  unsigned all = 0, before = 0;
+#pragma unroll 8
+  for (int h = part; h < s.groups; h += 4) {
+    const unsigned c = s.counts[h * 256 + d];
+    all += c;
+    before += h < g ? c : 0;
+  }
+  __syncthreads();
+  for (int i = beg + lane; i < end; i += 64) atomicAdd(&hist[wave][(s.ka[i] >> shift) & 255], 1u);
+  __syncthreads();
+  {
+    unsigned total;
+    unsigned base = block_scan(all, wave_sums, &total);  // (of the digit's first lane: the digits before)
+    base = __shfl(base, lane & ~3, 64);
+#pragma unroll
+    for (int o = 1; o < 4; o <<= 1) before += __shfl_xor(before, o, 64);
+    unsigned v[4], sum = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      v[j] = sum;
+      sum += hist[4 * part + j][d];
+    }
+    unsigned incl = sum;  // over the digit's four lanes
+#pragma unroll
+    for (int o = 1; o < 4; o <<= 1) {
+      const unsigned u = __shfl_up(incl, o, 4);
+      if (part >= o) incl += u;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) hist[4 * part + j][d] = base + before + (incl - sum) + v[j];
+  }
+  __syncthreads();
+  for (int i0 = beg; i0 < end; i0 += 64) {
+    const int i = i0 + lane;
+    const bool in = i < end;
+    const unsigned k = in ? s.ka[i] : 0, v = in ? s.va[i] : 0, q = (k >> shift) & 255;
+    const unsigned long long m = match_lanes(q, __ballot(in));
+    if (in) {
+      const unsigned pos = hist[wave][q] + __popcll(m & below);
+      s.kb[pos] = k;
+      s.vb[pos] = v;
+      if ((m & ~below & ~(1ull << lane)) == 0) hist[wave][q] = pos + 1;  // (the last of its digit in this step)
+    }
+  }
+}
+
+// Segments of equal ids (s.ka, s.va: sorted), as in embed_index_kernel.  STEP 0: a stretch's words; 1: the words' places, by
+// segment, in s.kb; 2: the words of the rows.
+template <int STEP>
+__global__ __launch_bounds__(kIndexThreads) void index_words_kernel(SortWork s, int *__restrict__ index, const float *__restrict__ ids, int V, int leaf_rows) {
+  __shared__ unsigned own[kIndexWaves][2], others[kIndexWaves][4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = blockIdx.x, n = s.n;
+  const unsigned long long below = (1ull << lane) - 1;
+  unsigned *counts = s.counts + s.groups * 256;
+  int beg, end;
+  s.stretch(&beg, &end);
+  auto bounds = [&](int p, bool *first, bool *last, bool *leaves) {
+    const unsigned k = s.ka[p];
+    *first = p == 0 || k == (unsigned)V || s.ka[p - 1] != k;
+    *last = p == n - 1 || k == (unsigned)V || s.ka[p + 1] != k;
+    *leaves = *last && (int)s.va[p] < leaf_rows;
+  };
+  unsigned nf = 0, nl = 0;
+  for (int i0 = beg; i0 < end; i0 += 64) {
+    bool f = false, l = false, z = false;
+    if (i0 + lane < end) bounds(i0 + lane, &f, &l, &z);
+    nf += __popcll(__ballot(f));
+    nl += __popcll(__ballot(z));
+  }
+  if (lane == 0) own[wave][0] = nf, own[wave][1] = nl;
+  unsigned c[4] = {0, 0, 0, 0};  // words and words of leaves: of the stretches before, of all
+  if (STEP > 0 && tid < s.groups) {
+    c[2] = counts[2 * tid];
+    c[3] = counts[2 * tid + 1];
+    if (tid < g) c[0] = c[2], c[1] = c[3];
+  }
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) c[j] += __shfl_xor(c[j], o, 64);
+    if (lane == 0) others[wave][j] = c[j];
+  }
+  __syncthreads();
+  if constexpr (STEP == 0) {
+    if (tid < 2) {
+      unsigned sum = 0;
+      for (int w = 0; w < kIndexWaves; w++) sum += own[w][tid];
+      counts[2 * g + tid] = sum;
+    }
+    return;
+  }
+  unsigned fcount = 0, zcount = 0, words = 0, leaf_words = 0;
+  for (int w = 0; w < kIndexWaves; w++) {
+    fcount += others[w][0] + (w < wave ? own[w][0] : 0);
+    zcount += others[w][1] + (w < wave ? own[w][1] : 0);
+    words += others[w][2];
+    leaf_words += others[w][3];
+  }
+  if (STEP == 1 && g == 0 && tid == 0) {
+    index[0] = words;
+    index[1] = leaf_words;
+    index[2] = index[3] = 0;
+  }
+  int *slot = index + 4, *order = slot + n, *at = order + n;
+  float *word = reinterpret_cast<float *>(at + n);
+  for (int i0 = beg; i0 < end; i0 += 64) {
+    const int p = i0 + lane;
+    bool f = false, l = false, z = false;
+    if (p < end) bounds(p, &f, &l, &z);
+    const unsigned long long fm = __ballot(f), zm = __ballot(z);
+    const unsigned seg = fcount + __popcll(fm & (below | 1ull << lane)) - 1, leaves_before = zcount + __popcll(zm & below);
+    fcount += __popcll(fm);
+    zcount += __popcll(zm);
+    if (p >= end) continue;
+    const int row = s.va[p];
+    if constexpr (STEP == 1) {
+      if (l) {
+        const unsigned q = z ? leaves_before : leaf_words + (seg - leaves_before);
+        s.kb[seg] = q;
+        word[q] = ids[row];
+      }
+    } else {
+      const int q = s.kb[seg];
+      slot[row] = q;
+      order[p] = row;
+      at[p] = q;
+    }
   }
 }
 
@@ -319,7 +497,8 @@ extern "C" {
 
 size_t cavs_embed_index_ints(int n) { return 4 + 4 * (size_t)std::max(n, 0); }
 
-size_t cavs_embed_index_workspace(int n) { return 4 * sizeof(unsigned) * (size_t)std::max(n, 0); }
+// (no less than for any smaller n)
+size_t cavs_embed_index_workspace(int n) { return n <= 0 ? 0 : 4 * sizeof(unsigned) * (size_t)n + sizeof(unsigned) * 258 * (size_t)std::min((n + 1023) / 1024, kSortGroups); }
 
 int cavs_embed_index(int *index, float *ids_out, const float *x, const int *rows, int n, int V, int leaf_rows, void *workspace,
                      size_t workspace_bytes, void *stream) {
@@ -329,11 +508,24 @@ int cavs_embed_index(int *index, float *ids_out, const float *x, const int *rows
   const size_t need = cavs_embed_index_workspace(n);
   CAVS_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), "cavs_embed_index: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
   const int passes = V < (1 << 8) ? 1 : V < (1 << 16) ? 2 : 3;  // (keys 0 .. V)
-  if (n <= kIndexLds && V < kIndexKeys)
-    launch(embed_index_kernel<true>, 1, kIndexThreads, 0, as_stream(stream), index, ids_out, x, rows, n, V, leaf_rows, passes, nullptr);
-  else
-    launch(embed_index_kernel<false>, 1, kIndexThreads, 0, as_stream(stream), index, ids_out, x, rows, n, V, leaf_rows, passes,
-           static_cast<unsigned *>(workspace));
+  hipStream_t st = as_stream(stream);
+  if (n <= kIndexLds && V < kIndexKeys) {
+    launch(embed_index_kernel, 1, kIndexThreads, 0, st, index, ids_out, x, rows, n, V, leaf_rows, passes);
+    CAVS_LAUNCH_CHECK();
+    return CAVS_OK;
+  }
+  unsigned *w = static_cast<unsigned *>(workspace);
+  SortWork s{w, w + n, w + 2 * (size_t)n, w + 3 * (size_t)n, w + 4 * (size_t)n, n, sort_per(n), sort_groups(n)};
+  for (int pass = 0; pass < passes; pass++) {
+    if (pass == 0) launch(index_sort_count_kernel<true>, s.groups, kIndexThreads, 0, st, s, ids_out, x, rows, V, 0);
+    else launch(index_sort_count_kernel<false>, s.groups, kIndexThreads, 0, st, s, nullptr, nullptr, nullptr, V, 8 * pass);
+    launch(index_sort_place_kernel, s.groups, kIndexThreads, 0, st, s, 8 * pass);
+    std::swap(s.ka, s.kb);
+    std::swap(s.va, s.vb);
+  }
+  launch(index_words_kernel<0>, s.groups, kIndexThreads, 0, st, s, index, ids_out, V, leaf_rows);
+  launch(index_words_kernel<1>, s.groups, kIndexThreads, 0, st, s, index, ids_out, V, leaf_rows);
+  launch(index_words_kernel<2>, s.groups, kIndexThreads, 0, st, s, index, ids_out, V, leaf_rows);
   CAVS_LAUNCH_CHECK();
   return CAVS_OK;
 }

@@ -42,7 +42,6 @@ struct GemmArgs {
   int zseg = 0;
   const int *live = nullptr;  // cavs_gemm_desc::live
   int pad_block = 0, pad_used = 0;  // cavs_gemm_desc::pad_block, pad_used
-  bool through = false;             // partial sums past this XCD's L2: a workgroup anywhere may read them in the same launch
 };
 
 __device__ inline bool padding_column(const GemmArgs &g, int col) { return g.pad_block > 0 && col % g.pad_block >= g.pad_used; }
@@ -85,8 +84,9 @@ __device__ inline void tile_k_range(const GemmArgs &g, int m0, int n0, int z, in
   *end = kend;
 }
 
-// Stores the TM x TN accumulators of a wavefront whose first row and column are m0 and n0.
-template <int TM, int TN>
+// Stores the TM x TN accumulators of a wavefront whose first row and column are m0 and n0.  THROUGH: partial sums past this
+// XCD's L2, for workgroups anywhere in the same launch to read.
+template <int TM, int TN, bool THROUGH = false>
 __device__ inline void store_tile(const GemmArgs &g, const floatx16 (&acc)[TM][TN], int m0, int n0, int z, int lane) {
   const int khalf = lane >> 5;
   // C layout of the 32x32 accumulator: element r of lane l is row 8*(r/4) + 4*(l/32) + r%4,
@@ -102,7 +102,7 @@ __device__ inline void store_tile(const GemmArgs &g, const floatx16 (&acc)[TM][T
       // for every lane), not once per element
       if (g.ws) {  // split K: park the partial sum, the reduce kernel finishes the job
         float *w = g.ws + (long)z * g.M * g.N + col;
-        if (g.through) {
+        if constexpr (THROUGH) {
 #pragma unroll
           for (int r = 0; r < 16; r++) {
             const int row = rbase + 8 * (r / 4) + (r % 4);

@@ -54,7 +54,7 @@ struct EmbedTail {
 
 // What a group's launch finishes by itself where it has counters: the workgroup that arrives last at a tile of a product whose K
 // is split adds up the tile's partial sums, in the order of the splits whoever is last, and scatters the tile of the
-// product that feeds the embedding's gradient.  Partial sums go past the L2 (GemmArgs::through), and the count behind
+// product that feeds the embedding's gradient.  Partial sums go past the L2 (THROUGH), and the count behind
 // them; the last one puts the counter back to zero.  Column sums come along as workgroups behind the products'.
 // As launches of their own these were latency, not work -- ids, parts and atomic adds one behind the other, 4.5 us between
 // two launches.  What bounds the end of the launch now are those trips: so all parts of a tile are in flight at once (one
@@ -124,10 +124,10 @@ __global__ __launch_bounds__(kThreads, 4) void sgemm_group_kernel(GemmGroup G, G
   int mine = -1;  // (asked for in front of the product, looked at behind it)
   if (F.counters && F.embed == p && m0 < min(F.tail.n, g.M)) mine = embed_row(F.tail.ids, min(F.tail.n, g.M), F.tail.E, m0 / kEmbedRows);
   switch (G.form[p]) {
-    case 0: split_tile<BM, BN, BK, false, false, VEC, true>(g, m0, n0, z, S); break;
-    case 1: split_tile<BM, BN, BK, false, true, VEC, true>(g, m0, n0, z, S); break;
-    case 2: split_tile<BM, BN, BK, true, false, VEC, true>(g, m0, n0, z, S); break;
-    default: split_tile<BM, BN, BK, true, true, VEC, true>(g, m0, n0, z, S); break;
+    case 0: split_tile<BM, BN, BK, false, false, VEC, true, false, true>(g, m0, n0, z, S); break;
+    case 1: split_tile<BM, BN, BK, false, true, VEC, true, false, true>(g, m0, n0, z, S); break;
+    case 2: split_tile<BM, BN, BK, true, false, VEC, true, false, true>(g, m0, n0, z, S); break;
+    default: split_tile<BM, BN, BK, true, true, VEC, true, false, true>(g, m0, n0, z, S); break;
   }
   if (!F.counters) return;
   asm volatile("" : "+s"(p), "+s"(t));  // (what follows reads its sizes again: kept over the product they cost registers)
@@ -769,7 +769,6 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
     F.tail = tail;
     if (!with_tail) F.embed = -1;
     if (F.embed >= 0) with_tail = false;
-    for (int p = 0; p < n; p++) G.g[p].through = G.splits[p] > 1;
     nr = R.count = 0;
   }
   unsigned grid = G.first[n];

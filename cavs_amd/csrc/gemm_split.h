@@ -295,7 +295,7 @@ constexpr int split_lds_bytes(int BM, int BN, int BK) { return 2 * 3 * 2 * BK * 
 
 // The BM x BN tile at (m0, n0) of split `z` by the calling workgroup; S: split_lds_bytes of LDS.  FOLD: chains of
 // additions end after kSplitChain of K.
-template <int BM, int BN, int BK, bool TA, bool TB, bool VEC, bool FOLD, bool PULL = false>
+template <int BM, int BN, int BK, bool TA, bool TB, bool VEC, bool FOLD, bool PULL = false, bool THROUGH = false>
 __device__ __forceinline__ void split_tile(const GemmArgs &g, int m0, int n0, int z, char *__restrict__ S) {
   constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
   constexpr int PA = 2 * BK * BM, PB = 2 * BK * BN, BUF = 3 * (PA + PB);
@@ -431,7 +431,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs &g, int m0, int n0, in
 #pragma unroll
         for (int r = 0; r < 16; r++) odd = fmaf(out[i][j][r], 0.f, odd);
     if (__any(!(odd == 0.f))) unsplit_tile<TM, TN, TA, TB, PULL>(g, row, col, kbeg, kend, l, out);
-    store_tile<TM, TN>(g, out, row, col, z, l);
+    store_tile<TM, TN, THROUGH>(g, out, row, col, z, l);
   };
   if constexpr (FOLD) finish(sum);
   else finish(acc);

@@ -673,12 +673,14 @@ void Engine::reserve_edges() {
 
 // Whether x * W and its gradients go by words: every different id of the batch once (cavs_embed_index).
 // Saved: the products' rows of the ids met before (a parse tree's inner vertices all look up one word), at
-// 140 TFLOP/s.  Paid: the index (2368 vertices 15 us, 16000 65, 73000 360 by itself and 520 inside a step),
+// 140 TFLOP/s.  Paid: the index (2368 vertices 15 us, 8192 36, 73000 37),
 // spreading the rows (5 / 24 / 256 us at 2048, 2048, 4096 columns), in the backward pass adding up their
 // gradients (10 / 36 / 345 us).  The line is
 // at 1.5 because both are estimates: of 72 sessions (Tree-LSTMs and chains, H = 128 .. 1024, 1200 .. 19000 vertices,
 // with and without a backward pass) all 25 above it gain, 5 us (260 a step) to 1.2 ms (4.85), and of those
 // below it the six that would are between 0.59 and 1.45, by 50 us at most, beside others that would lose as much.
+// (The estimate charges the index 0.004 us a vertex beyond 8192 too, as it once cost: with 35 us there, a forward pass over
+// 9500 vertices went by words and took 8 % longer.)
 // (The index on another stream while the kernels of the step before run, which takes it off this account,
 // gained nothing: 10 to 16 us more a step than in line, 1200 to 19000 vertices.)
 bool Engine::words_wanted() const {

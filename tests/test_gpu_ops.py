@@ -1984,6 +1984,12 @@ def test_words_of_a_batch(g, n, V, E, w, leaf_rows):
     np.testing.assert_array_equal(outs[0][words:], 7.0)
 
 
+@pytest.mark.parametrize("n,V,leaf_rows", [(17408, 200, 3), (17409, 255, 17409), (70001, 21701, 36000), (33000, 70000, 0), (262145, 1 << 16, 100000)])
+def test_words_of_a_large_batch(g, n, V, leaf_rows):
+    """Stretches of 1024 and of 2048 rows, whole and not, one to three digits."""
+    test_words_of_a_batch(g, n, V, 4, 4, leaf_rows)
+
+
 @pytest.mark.parametrize("M,N,K,L,Z", [(200, 68, 516, 0, 0), (200, 68, 516, 130, 70), (8000, 1024, 300, 4100, 2000), (3000, 300, 2048, 1290, 1200)])
 def test_products_over_the_words_alone(g, M, N, K, L, Z):
     """cavs_gemm_desc.live: only the first L of the M rows, or of K rows, take part, the known block ends at row Z;
