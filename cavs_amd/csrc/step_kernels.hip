@@ -183,6 +183,48 @@ static bool head_supported(int H, int C) {
   return C >= 1 && C <= 8 && H >= 1 && H <= 1024 && C * head_q(H) <= 64 && (size_t)(4 * C * H + 4 * C) * 4 <= 64 * 1024;
 }
 
+// ------------------------------------------------------------------ sum of squares over the roots
+// A wavefront a row, of d h where it is wanted (a root's 2 h, zero elsewhere; roots ascend, so a search tells), else of the
+// roots alone; a root's wavefront leaves the row's sum.  Bound by writing d h and by its launch: gathering the roots,
+// squares, two sums, the clearing, the doubling and scattering them were seven launches (B = 64, H = 256, 2400
+// vertices: 32 us with the gaps between them, 6 now).
+template <class V>
+__global__ __launch_bounds__(256) void root_sq_kernel(float *__restrict__ parts, V *__restrict__ dgo, const V *__restrict__ go,
+                                                      const int *__restrict__ roots, int B, int N, int q) {
+  constexpr int W = sizeof(V) / sizeof(float);
+  const int i = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  int v = i, root = i;  // (without d h: row i of the roots)
+  if (dgo) {
+    if (v >= N) return;
+    int lo = 0, hi = B;  // the first root not below v
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (roots[mid] < v) lo = mid + 1;
+      else hi = mid;
+    }
+    root = lo < B && roots[lo] == v ? lo : -1;
+  } else {
+    if (i >= B) return;
+    v = roots[i];
+  }
+  float sum = 0.f;
+  for (int c = lane; c < q; c += 64) {
+    V h{};
+    if (root >= 0) h = go[(long)v * q + c];
+    float *e = reinterpret_cast<float *>(&h);
+#pragma unroll
+    for (int k = 0; k < W; k++) {
+      sum += e[k] * e[k];
+      e[k] *= 2.f;
+    }
+    if (dgo) dgo[(long)v * q + c] = h;
+  }
+  if (root < 0) return;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+  if (lane == 0) parts[root] = sum;
+}
+
 // ------------------------------------------------------------------ SGD over several tensors
 constexpr int kMaxTensors = 8;
 struct SgdBatch {
@@ -588,6 +630,20 @@ int cavs_run_tasks(int count, const cavs_task *tasks, void *stream) {
   if (k == 0) return CAVS_OK;
   L.count = k;
   launch(tasks_kernel, (unsigned)L.first[k], 256, 0, as_stream(stream), L);
+  CAVS_LAUNCH_CHECK();
+  return CAVS_OK;
+}
+
+int cavs_root_sq(float *parts, float *dgraph_out, const float *graph_out, const int *roots, int B, int N, int H, void *stream) {
+  CAVS_REQUIRE(B >= 0 && N >= B && H > 0, "cavs_root_sq: bad shape B=%d N=%d H=%d", B, N, H);
+  if (B == 0 && (!dgraph_out || N == 0)) return CAVS_OK;
+  CAVS_REQUIRE(graph_out && (B == 0 || (parts && roots)), "cavs_root_sq: null pointer");
+  const unsigned grid = (unsigned)(((dgraph_out ? N : B) + 3) / 4);
+  hipStream_t st = as_stream(stream);
+  if (H % 4 == 0 && aligned16(graph_out) && aligned16(dgraph_out))
+    launch(root_sq_kernel<float4>, grid, 256, 0, st, parts, reinterpret_cast<float4 *>(dgraph_out), reinterpret_cast<const float4 *>(graph_out), roots, B, N, H / 4);
+  else
+    launch(root_sq_kernel<float>, grid, 256, 0, st, parts, dgraph_out, graph_out, roots, B, N, H);
   CAVS_LAUNCH_CHECK();
   return CAVS_OK;
 }

@@ -2599,19 +2599,17 @@ void Engine::head_forward_backward(bool backward) {
     }
     return;
   }
-  float *tmp = logits_.get(), *colacc = loss_.get() + 1;
+  float *tmp = logits_.get(), *colacc = loss_.get() + 1;  // [B * H + 1]
   if (cfg_.loss == CAVS_LOSS_ROOT_SQ) {
     // sum over roots of h^2; gradient 2h on root rows, zero elsewhere
-    gather(tmp, H, GO_.get(), H, d_roots_, B, H);
-    check(cavs_ew_unary(CAVS_EW_SQUARE, dlogits_.get(), tmp, (size_t)B * H, 0, stream_));
-    colsum_fixed(colacc, dlogits_.get(), B, H);
-    colsum_fixed(loss_.get(), colacc, H, 1);
-    c_launches_ += 1;  // the squares
+    last_launch(2, backward, [&] { check(cavs_root_sq(tmp, backward ? dGO_.get() : nullptr, GO_.get(), d_roots_, B, N, H, stream_)); });
+    c_launches_ += 1;
+    const cavs_task sum{CAVS_TASK_SUM_PARTS, 0.f, B, 1, 1, tmp, loss_.get(), nullptr, nullptr};
     if (backward) {
-      check(cavs_zero(dGO_.get(), (size_t)N * H * 4, stream_));
-      check(cavs_scale(dlogits_.get(), tmp, 2.f, (size_t)B * H, stream_));
-      c_launches_ += 2;
-      scatter(dGO_.get(), H, d_roots_, dlogits_.get(), H, B, H);
+      pending_tasks_.push_back(sum);  // rides in the launch that opens the backward pass
+    } else {
+      check(cavs_run_tasks(1, &sum, stream_));
+      c_launches_ += 1;
     }
   } else {
     // Reduce_sum is a sum of absolute values whose gradient op is a constant fill

@@ -661,6 +661,10 @@ int cavs_treefc_bwd_rows(const int *rows, int n, const float *dret, const int *d
                          float *dz, int H, int act, void *stream);
 /* out [cols,rows] = in [rows,cols]^T */
 int cavs_transpose(float *out, const float *in, int rows, int cols, void *stream);
+/* The sum of the squares of the roots' rows and its gradient (cavs/backend/op_impl_blas1_cublas.cc:62-77 over a Square): parts[i] =
+ * the sum over row roots[i] of graph_out [N, H], for a CAVS_TASK_SUM_PARTS job to add up (n0 = B, n1 = n2 = 1); rows of
+ * dgraph_out [N, H] (may be null): twice graph_out's at the roots, else zero.  roots: ascending. */
+int cavs_root_sq(float *parts, float *dgraph_out, const float *graph_out, const int *roots, int B, int N, int H, void *stream);
 /* Several small jobs that do not depend on each other, in one launch (no counterpart in the
  * reference, where each is an op of its own: cavs/backend/op_impl_sgd.cu,
  * op_impl_embedding_lookup.cu, the transposes cuBLAS does inside its calls).  Results are those

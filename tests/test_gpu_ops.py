@@ -1984,6 +1984,23 @@ def test_words_of_a_batch(g, n, V, E, w, leaf_rows):
     np.testing.assert_array_equal(outs[0][words:], 7.0)
 
 
+@pytest.mark.parametrize("B,N,H", [(1, 1, 1), (1, 3, 33), (3, 9, 30), (5, 64, 256), (64, 700, 36), (7, 50, 1028)])
+def test_squares_of_the_roots(g, B, N, H):
+    """cavs_root_sq: row sums of positive terms (H of them: 2^-24 each, and as much again for the squares), 2 h exactly."""
+    r = rng(B * N + H)
+    roots = np.sort(np.argsort(r.bulk_uniform(N))[:B]).astype(np.int32)
+    roots[-1] = N - 1
+    h = r.bulk_uniform(N * H, -2, 2).reshape(N, H).astype(np.float32)
+    d_h, d_roots = g.devf(h.reshape(-1)), g.devi(roots)
+    for back in (True, False):
+        parts, dgo = g.devf(np.full(B, np.nan)), g.devf(np.full(N * H, np.nan))
+        g.call("cavs_root_sq", g.P(parts), g.P(dgo) if back else None, g.P(d_h), g.P(d_roots), B, N, H, g.stream())
+        np.testing.assert_allclose(g.host(parts), (h[roots].astype(np.float64) ** 2).sum(1), rtol=2.0 ** -23 * (H + 1))
+        want = np.zeros((N, H), np.float32)
+        want[roots] = 2 * h[roots]
+        assert not back or np.array_equal(g.host(dgo).reshape(N, H), want)
+
+
 @pytest.mark.parametrize("n,V,leaf_rows", [(17408, 200, 3), (17409, 255, 17409), (70001, 21701, 36000), (33000, 70000, 0), (262145, 1 << 16, 100000)])
 def test_words_of_a_large_batch(g, n, V, leaf_rows):
     """Stretches of 1024 and of 2048 rows, whole and not, one to three digits."""
