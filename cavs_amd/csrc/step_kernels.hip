@@ -140,17 +140,23 @@ __device__ inline void sum_parts_block(const float *__restrict__ part, int npart
   float a0 = 0.f, a1 = 0.f;
   if (i < total) {
     int p = q;
-    // (eight loads in flight; the same additions in the same order as the loops below)
-    for (; p + 28 < nparts; p += 32) {
-      float v[8];
+    // (32 loads in flight, then eight; the same additions in the same order as the loops below.  296 parts in trips of
+    // eight were most of the launch that opens a backward pass.)
+    auto trip = [&](auto &v) {
+      constexpr int U = sizeof(v) / sizeof(float);
+      for (; p + 4 * (U - 1) < nparts; p += 4 * U) {
 #pragma unroll
-      for (int k = 0; k < 8; k++) v[k] = part[(long)(p + 4 * k) * total + i];
+        for (int k = 0; k < U; k++) v[k] = part[(long)(p + 4 * k) * total + i];
 #pragma unroll
-      for (int k = 0; k < 8; k += 2) {
-        a0 += v[k];
-        a1 += v[k + 1];
+        for (int k = 0; k < U; k += 2) {
+          a0 += v[k];
+          a1 += v[k + 1];
+        }
       }
-    }
+    };
+    float many[32], few[8];
+    trip(many);
+    trip(few);
     for (; p + 4 < nparts; p += 8) {
       a0 += part[(long)p * total + i];
       a1 += part[(long)(p + 4) * total + i];
@@ -250,44 +256,72 @@ __global__ void sgd_multi_kernel(SgdBatch t, float lr) {
 // to raise the row's stamp to this step's epoch owns it.  A workgroup takes kSgdChunk lookups
 // and asks for a row once however often it occurs among them (parse trees look up one and
 // the same row for every internal vertex; one atomic per vertex would serialise on it).
+// Its rows are read while the stamps are on their way and used if it comes to own them: what bounds it is the
+// chain of ids, stamps and rows, now ids and rows.
 constexpr int kSgdChunk = 16;
 struct EmbedSgdLds {
   int row[kSgdChunk];
-  long owned[kSgdChunk];
-  int n_owned;
+  long at[kSgdChunk];  // first element of the row in the table; -1: looked up earlier in the chunk, or nothing
+  int owned[kSgdChunk];
+  int odd;             // a row begins within a float4 (an id that is no whole number)
 };
+
+template <class V>
+__device__ inline void embed_sgd_rows(V *__restrict__ table, const V *__restrict__ dtable, int q, float lr, int *__restrict__ stamp,
+                                      int epoch, EmbedSgdLds &lds) {
+  constexpr int W = sizeof(V) / sizeof(float), U = 5;  // (16 rows of 320 in one turn; with eight it spills)
+  const int tid = threadIdx.x, total = kSgdChunk * q, step = U * blockDim.x;
+  for (int i0 = tid; i0 - tid < total; i0 += step) {
+    V t[U], d[U];
+    long at[U];
+    int r[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = i0 + u * blockDim.x;
+      r[u] = i < total ? i / q : 0;
+      at[u] = i < total ? lds.at[r[u]] : -1;
+      if (at[u] < 0) continue;
+      at[u] = at[u] / W + i % q;
+      t[u] = table[at[u]];
+      d[u] = dtable[at[u]];
+    }
+    if (i0 == tid) {  // the first turn: the stamps
+      if (tid < kSgdChunk) lds.owned[tid] = lds.at[tid] >= 0 && atomicMax(stamp + lds.row[tid], epoch) < epoch;
+      __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (at[u] < 0 || !lds.owned[r[u]]) continue;
+      float *x = reinterpret_cast<float *>(&t[u]), *y = reinterpret_cast<float *>(&d[u]);
+#pragma unroll
+      for (int k = 0; k < W; k++) x[k] -= lr * y[k];
+      table[at[u]] = t[u];
+    }
+  }
+}
 
 __device__ inline void embed_sgd_block(float *__restrict__ table, const float *__restrict__ dtable,
                                        const float *__restrict__ ids, int n, int E, float lr, int *__restrict__ stamp,
                                        int epoch, int block, EmbedSgdLds &lds) {
-  int (&row)[kSgdChunk] = lds.row;
-  long (&owned)[kSgdChunk] = lds.owned;
-  int &n_owned = lds.n_owned;
   const int v0 = block * kSgdChunk, tid = threadIdx.x;
-  if (tid < kSgdChunk) row[tid] = v0 + tid < n ? (int)ids[v0 + tid] : -1 - tid;
-  if (tid == 0) n_owned = 0;
-  __syncthreads();
-  if (tid < kSgdChunk) {
-    bool first = row[tid] >= 0;
-    for (int r = 0; r < tid; r++) first = first && row[r] != row[tid];
-    if (first && atomicMax(stamp + row[tid], epoch) < epoch)
-      owned[atomicAdd(&n_owned, 1)] = (long)(int)(ids[v0 + tid] * (float)E);
+  if (tid < kSgdChunk) {  // (lanes of one wavefront)
+    const float id = v0 + tid < n ? ids[v0 + tid] : 0.f;
+    const int row = v0 + tid < n ? (int)id : -1 - tid;
+    bool first = row >= 0;
+#pragma unroll
+    for (int r = 0; r < kSgdChunk - 1; r++)
+      if (r < tid && __builtin_amdgcn_readlane(row, r) == row) first = false;
+    lds.row[tid] = row;
+    const int at = first ? (int)(id * (float)E) : -1;
+    lds.at[tid] = at;
+    const bool odd = __any(at >= 0 && at % 4 != 0);
+    if (tid == 0) lds.odd = odd;
   }
   __syncthreads();
-  // every owned row of a column is in flight before the first store
-  const int cnt = n_owned;
-  for (int c = tid; c < E; c += blockDim.x) {
-    float t[kSgdChunk], d[kSgdChunk];
-#pragma unroll
-    for (int r = 0; r < kSgdChunk; r++)
-      if (r < cnt) {
-        t[r] = table[owned[r] + c];
-        d[r] = dtable[owned[r] + c];
-      }
-#pragma unroll
-    for (int r = 0; r < kSgdChunk; r++)
-      if (r < cnt) table[owned[r] + c] = t[r] - lr * d[r];
-  }
+  if (E % 4 == 0 && ((reinterpret_cast<uintptr_t>(table) | reinterpret_cast<uintptr_t>(dtable)) & 15) == 0 && !lds.odd)
+    embed_sgd_rows(reinterpret_cast<float4 *>(table), reinterpret_cast<const float4 *>(dtable), E / 4, lr, stamp, epoch, lds);
+  else
+    embed_sgd_rows(table, dtable, E, lr, stamp, epoch, lds);
 }
 
 __global__ void embed_sgd_kernel(float *__restrict__ table, const float *__restrict__ dtable,
@@ -413,6 +447,17 @@ __global__ __launch_bounds__(256) void tasks_kernel(TaskList L) {
       float *__restrict__ w = static_cast<float *>(t.p0);
       const float *__restrict__ g = static_cast<const float *>(t.p1);
       const size_t n = (size_t)t.n0, stride = (size_t)nb * 256;
+      if (n % 4 == 0 && ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(g)) & 15) == 0) {
+        float4 *w4 = reinterpret_cast<float4 *>(w);
+        const float4 *g4 = reinterpret_cast<const float4 *>(g);
+        for (size_t i = (size_t)b * 256 + tid; i < n / 4; i += stride) {
+          float4 v = w4[i];
+          const float4 d = g4[i];
+          v.x -= t.f0 * d.x, v.y -= t.f0 * d.y, v.z -= t.f0 * d.z, v.w -= t.f0 * d.w;
+          w4[i] = v;
+        }
+        break;
+      }
       for (size_t i = (size_t)b * 256 + tid; i < n; i += stride) w[i] -= t.f0 * g[i];
       break;
     }
@@ -429,7 +474,14 @@ __global__ __launch_bounds__(256) void tasks_kernel(TaskList L) {
       for (int i = b * 256 + tid; i < total; i += nb * 256) {
         const int k = i / bw, d = (int)((t.n2 >> (4 * k)) & 15) * bw + i % bw;
         float g = src[i];
-        for (int q = 1; q < parts; q++) g += src[(long)q * total + i];
+        for (int q = 1; q < parts; q += 8) {  // eight loads in flight
+          float v[8];
+#pragma unroll
+          for (int u = 0; u < 8; u++) v[u] = src[(long)min(q + u, parts - 1) * total + i];
+#pragma unroll
+          for (int u = 0; u < 8; u++)
+            if (q + u < parts) g += v[u];
+        }
         if (gout) gout[d] = g;
         if (w) w[d] -= t.f0 * g;
       }
@@ -599,7 +651,7 @@ int cavs_run_tasks(int count, const cavs_task *tasks, void *stream) {
           CAVS_REQUIRE(d < (int)t.n1 && !(seen >> d & 1u), "cavs_run_tasks: job %d: the block map is not a permutation", i);
           seen |= 1u << d;
         }
-        blocks = (t.n0 * t.n1 + 1023) / 1024;
+        blocks = (t.n0 * t.n1 + 255) / 256;
         break;
       }
       case CAVS_TASK_TREELSTM_GATES_ROWS: {
