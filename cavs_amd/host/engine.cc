@@ -1604,7 +1604,8 @@ void Engine::treelstm_backward() {
   // every round hands d h, d c on to its children and does their gate gradients in its epilogue
   const bool folded = forest_;
   // (those of the roots depend on nothing the opening launch writes and ride in it)
-  const bool roots_ride = folded && fused > 0 && H % 4 == 0 && n_orphans_ > 0;
+  const bool roots_grouped = group_.first >= 0;  // (the group launch has lists of them)
+  const bool roots_ride = folded && !roots_grouped && fused > 0 && H % 4 == 0 && n_orphans_ > 0;
   std::vector<cavs_task> opening;
   if (fused > 0) {  // U_iou^T and U_f^T: the B operand of the children products, k-major
     const int kind = packed ? CAVS_TASK_PACK_T : CAVS_TASK_TRANSPOSE;
@@ -1620,7 +1621,7 @@ void Engine::treelstm_backward() {
                        const_cast<int *>(d_orphans_), const_cast<float *>(d_dgo_), const_cast<int *>(d_t2j_), gates_.get(), G_.get(),
                        dxW_.get(), dF_.get(), dc_.get()});
   backward_prologue(opening, true);
-  if (folded && !roots_ride) {
+  if (folded && !roots_grouped && !roots_ride) {
     CAVS_TIMED(K_GATES, cavs_treelstm_bwd_gates_rows(d_orphans_, n_orphans_, d_dgo_, d_t2j_, gates_.get(), G_.get(), dxW_.get(), 4 * H,
                                                      dF_.get(), dc_.get(), sched_->leaf_prefix, H, stream_));
     c_launches_ += 1;
@@ -1983,7 +1984,7 @@ void Engine::lstm_backward() {
   const float *dret = head_chunked_ ? dret_.get() : d_dgo_;
   const int *dret_rows = head_chunked_ ? cell_iota_.get() : d_t2j_;
   int chunk = head_chunked_ ? (int)head_chunks_.size() : 0;
-  if (folded && !head_chunked_) {
+  if (folded && !head_chunked_ && group_.first < 0) {  // (the group launch has lists of them)
     CAVS_TIMED(K_GATES, cavs_lstm_bwd_gates_rows(d_orphans_, n_orphans_, d_dgo_, d_t2j_, gates_.get(), G_.get(), dxW_.get(), 4 * H,
                                                  dc_.get(), sched_->leaf_prefix, H, stream_));
     c_launches_ += 1;
@@ -2148,7 +2149,7 @@ void Engine::treefc_backward() {
     backward_prologue({}, false);
   }
   const bool folded = forest_;  // one launch per round, as in treelstm_backward
-  if (folded) {
+  if (folded && group_.first < 0) {  // (the group launch has lists of them)
     CAVS_TIMED(K_GATES, cavs_treefc_bwd_rows(d_orphans_, n_orphans_, d_dgo_, d_t2j_, msg_.get(), dxW_.get(), H, cfg_.act, stream_));
     c_launches_ += 1;
   }
@@ -2355,7 +2356,7 @@ void Engine::cell_backward() {
     // gathered -- the states of the round's children for the first cell, the rows of the cell before
     // for the others -- and runs the elementwise part of the cell that wrote them at once.  The
     // vertices without a reader go first.
-    if (n_orphans_ > 0) {
+    if (n_orphans_ > 0 && (group_.first < 0 || head_chunked_)) {  // (the group launch has lists of them)
       ProfScope ps(this, K_GATES);
       cell_launch(L - 1, CK_BWD_ROWS, (unsigned)(((size_t)n_orphans_ * H + 255) / 256), 1, 1, 256, 0, n_orphans_, d_orphans_, d_dgo_);
     }

@@ -404,8 +404,8 @@ void build_tail_lists(const Schedule &s, const int *kid_rows, int lim, int group
 }
 
 size_t group_lists_bound(size_t N, int groups) {
-  // two sets of records, forward and backward lists of at least a row each, two tables of groups
-  return N * (16 + 8) + 2 * (size_t)groups * 4;
+  // records forward, backward and of the rows nobody sends a gradient to, lists of at least a row each, two tables of groups
+  return N * (24 + 12) + 2 * (size_t)groups * 4;
 }
 
 // What the group with the most work spends on tiles when its lists run in tiles of four rows, and when they run in
@@ -475,6 +475,17 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
       at[i] = fill;
       fill += per[i];
     }
+    // The rows whose message nobody reads open the backward pass: with the group whose tree they are in, those of earlier
+    // rounds with any.
+    std::vector<int> roots, root_at((size_t)G + 1, 0);
+    for (int b = 0, any = 0; b < N; b++) {
+      if (pair[b] >= 0) continue;
+      const int g = b >= lo ? cell[b - lo] / nr : any++ % G;
+      roots.push_back(b);
+      roots.push_back(g);
+      root_at[g + 1]++;
+    }
+    for (int g = 0; g < G; g++) root_at[g + 1] += root_at[g];
     t.fwd.recs = 0;
     t.bwd.recs = t.rows * 8;
     cur = at;
@@ -488,7 +499,12 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
       std::memcpy(f, fr, sizeof fr);
       std::memcpy(w, br, sizeof br);
     }
-    size_t end = 2 * t.rows * 8;
+    cur.assign(root_at.begin(), root_at.end());
+    for (size_t i = 0; i < roots.size(); i += 2) {
+      const int b = roots[i], r[8] = {b, b, -1, t2j[b], -1, 0, 0, 0};
+      std::memcpy(block + t.bwd.recs + 8 * (t.rows + cur[roots[i + 1]]++), r, sizeof r);
+    }
+    size_t end = (2 * t.rows + roots.size() / 2) * 8;
     // A direction: a group's share of a round as lists of at most `slice` rows; the first waits for the
     // rounds the group has done so far, the last is an arrival.
     for (int back = 0; back < 2; back++) {
@@ -499,6 +515,12 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
       for (int g = 0; g < G; g++) {
         int *gd = block + l.groups + 4 * (size_t)g, done = 0;
         gd[0] = nl;
+        const int alone = back ? root_at[g + 1] - root_at[g] : 0;
+        for (int c0 = 0; c0 < alone; c0 += slice, nl++) {
+          const int row[4] = {(int)t.rows + root_at[g] + c0, std::min(slice, alone - c0), 0, (c0 + slice >= alone) | 2};
+          std::copy(row, row + 4, lists + 4 * (size_t)nl);
+        }
+        done += alone > 0;
         for (int i = 0; i < nr; i++) {
           const int k = back ? nr - 1 - i : i, c = per[(size_t)g * nr + k];
           for (int c0 = 0; c0 < c; c0 += slice, nl++) {

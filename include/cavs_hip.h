@@ -519,7 +519,9 @@ int cavs_tail_probe(unsigned *sync, int H, int spin_max, void *stream);
  * (cavs_group_rounds_ok) and all three vertex functions (the loops of cavs/midend/statement.cc:69-76,
  * 106-111 without the round trips to the host): as the tail launches above, with
  *   groups  [ngroups][4]  first list, number of lists, arrivals of the launch, 0
- *   lists   [*][4]        first record, rows (at most cavs_group_rows()), arrivals that must be in, arrives (0 / 1)
+ *   lists   [*][4]        first record, rows (at most cavs_group_rows()), arrivals that must be in, arrives (0 / 1); backward + 2: rows
+ *                         that get no gradient from a parent, each named as its own child 0: what
+ *                         cavs_*_bwd_rows does with them
  *   recs    [*][8]        forward:  slab row, pool rows of its children (-1: none), pool row its message goes
  *                                   to (-1: none), row of graph_out, 0, 0, 0
  *                         backward: slab row, slab rows of its children, row of dret of child 0, of child 1, 0, 0, 0
