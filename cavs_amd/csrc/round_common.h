@@ -355,5 +355,91 @@ inline bool exact_stages(int H, const RoundPlan &p) {
   return H % (p.waves * 16 * ug * 2) == 0 && H <= 8192;
 }
 
+// Vertices without children (whose rows of gates the backward pass reads all the same), elementwise: W columns of one by a thread.
+struct RoundLeavesArgs {
+  const float *xW;
+  long ld_xw;
+  const float *bias;
+  const int *pair;
+  float *gates, *msg, *pool, *go;
+  const int *out_rows;
+  int n, H;
+};
+
+template <int W>
+__device__ inline void stw(float *p, const float (&v)[W]) {
+  if constexpr (W == 4) {
+    *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < W; k++) p[k] = v[k];
+  }
+}
+
+template <int W>
+__device__ inline void treelstm_leaves_at(const RoundLeavesArgs &a, long idx) {
+  const int H = a.H, hw = H / W;
+  const long H2 = 2L * H;
+  if (idx >= (long)a.n * hw) return;
+  const int r = (int)(idx / hw), j = (int)(idx % hw) * W;
+  const int dst = a.pair[r], out = a.go ? a.out_rows[r] : -1;
+  const float *xw = a.xW + r * a.ld_xw + j;
+  float gi[W], go[W], gu[W], gf[W], gtc[W], mh[W], mc[W];
+#pragma unroll
+  for (int k = 0; k < W; k++) {
+    // same association as with children: (x*W + 0) + bias
+    const float i = sigm_r((xw[k] + 0.f) + a.bias[j + k]);
+    const float o = sigm_r((xw[H + k] + 0.f) + a.bias[3 * H + j + k]);
+    const float u = tanh_r((xw[2 * H + k] + 0.f) + a.bias[2 * H + j + k]);
+    const float f = sigm_r((xw[3 * H + k] + 0.f) + a.bias[H + j + k]);
+    const float c = (i * u + f * 0.f) + f * 0.f;
+    const float tc = tanh_r(c);
+    gi[k] = i; go[k] = o; gu[k] = u; gf[k] = f; gtc[k] = tc; mh[k] = o * tc; mc[k] = c;
+  }
+  auto st = [](float *p, const float (&v)[W]) {
+    if constexpr (W == 4) {
+      *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < W; k++) p[k] = v[k];
+    }
+  };
+  float *g = a.gates + (long)r * 6 * H + j;
+  st(g, gi); st(g + H, go); st(g + 2 * H, gu); st(g + 3 * H, gf); st(g + 4 * H, gf); st(g + 5 * H, gtc);
+  if (a.msg) {
+    float *m = a.msg + r * H2 + j;
+    st(m, mh); st(m + H, mc);
+  }
+  if (dst >= 0) { st(a.pool + dst * H2 + j, mh); st(a.pool + dst * H2 + H + j, mc); }
+  if (out >= 0) st(a.go + (long)out * H + j, mh);
+}
+
+template <int W>
+__device__ inline void lstm_leaves_at(const RoundLeavesArgs &a, long idx) {
+  const int H = a.H, hw = H / W;
+  const long H2 = 2L * H;
+  if (idx >= (long)a.n * hw) return;
+  const int r = (int)(idx / hw), j = (int)(idx % hw) * W;
+  const int dst = a.pair[r], out = a.go ? a.out_rows[r] : -1;
+  const float *xw = a.xW + r * a.ld_xw + j;
+  float gi[W], gf[W], gu[W], go[W], gtc[W], mh[W], mc[W];
+#pragma unroll
+  for (int k = 0; k < W; k++) {
+    const float i = sigm_r((xw[k] + 0.f) + a.bias[j + k]);
+    const float f = sigm_r((xw[H + k] + 0.f) + a.bias[H + j + k]);
+    const float u = tanh_r((xw[2 * H + k] + 0.f) + a.bias[2 * H + j + k]);
+    const float o = sigm_r((xw[3 * H + k] + 0.f) + a.bias[3 * H + j + k]);
+    const float c = i * u + f * 0.f;
+    const float tc = tanh_r(c);
+    gi[k] = i; gf[k] = f; gu[k] = u; go[k] = o; gtc[k] = tc; mh[k] = o * tc; mc[k] = c;
+  }
+  float *g = a.gates + (long)r * 5 * H + j;
+  stw<W>(g, gi); stw<W>(g + H, gf); stw<W>(g + 2 * H, gu); stw<W>(g + 3 * H, go); stw<W>(g + 4 * H, gtc);
+  float *m = a.msg + r * H2 + j;
+  stw<W>(m, mh); stw<W>(m + H, mc);
+  if (dst >= 0) { stw<W>(a.pool + dst * H2 + j, mh); stw<W>(a.pool + dst * H2 + H + j, mc); }
+  if (out >= 0) stw<W>(a.go + (long)out * H + j, mh);
+}
+
 }  // namespace cavs
 #endif

@@ -169,15 +169,6 @@ __device__ inline void sum_regions(float (&v)[NP], const float *red, int lds, in
 }
 
 template <int W>
-__device__ inline void stw(float *p, const float (&v)[W]) {
-  if constexpr (W == 4) {
-    *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
-  } else {
-#pragma unroll
-    for (int k = 0; k < W; k++) p[k] = v[k];
-  }
-}
-template <int W>
 __device__ inline void ldw(const float *p, float (&v)[W]) {
   if constexpr (W == 4) {
     const float4 t = ld4(p);
@@ -287,42 +278,9 @@ __global__ __launch_bounds__(WAVES * 64) void lstm_round_fwd_kernel(LstmFwdArgs 
 
 // first step of every sequence (no predecessor), and the gate gradients of any round:
 // elementwise, with the row movement folded in
-struct LstmLeavesArgs {
-  const float *xW;
-  long ld_xw;
-  const float *bias;
-  const int *pair;
-  float *gates, *msg, *pool, *go;
-  const int *out_rows;
-  int n, H;
-};
-
 template <int W>
-__global__ void lstm_round_leaves_fwd_kernel(LstmLeavesArgs a) {
-  const int H = a.H, hw = H / W;
-  const long H2 = 2L * H;
-  long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)a.n * hw) return;
-  const int r = (int)(idx / hw), j = (int)(idx % hw) * W;
-  const int dst = a.pair[r], out = a.go ? a.out_rows[r] : -1;
-  const float *xw = a.xW + r * a.ld_xw + j;
-  float gi[W], gf[W], gu[W], go[W], gtc[W], mh[W], mc[W];
-#pragma unroll
-  for (int k = 0; k < W; k++) {
-    const float i = sigm_r((xw[k] + 0.f) + a.bias[j + k]);
-    const float f = sigm_r((xw[H + k] + 0.f) + a.bias[H + j + k]);
-    const float u = tanh_r((xw[2 * H + k] + 0.f) + a.bias[2 * H + j + k]);
-    const float o = sigm_r((xw[3 * H + k] + 0.f) + a.bias[3 * H + j + k]);
-    const float c = i * u + f * 0.f;
-    const float tc = tanh_r(c);
-    gi[k] = i; gf[k] = f; gu[k] = u; go[k] = o; gtc[k] = tc; mh[k] = o * tc; mc[k] = c;
-  }
-  float *g = a.gates + (long)r * 5 * H + j;
-  stw<W>(g, gi); stw<W>(g + H, gf); stw<W>(g + 2 * H, gu); stw<W>(g + 3 * H, go); stw<W>(g + 4 * H, gtc);
-  float *m = a.msg + r * H2 + j;
-  stw<W>(m, mh); stw<W>(m + H, mc);
-  if (dst >= 0) { stw<W>(a.pool + dst * H2 + j, mh); stw<W>(a.pool + dst * H2 + H + j, mc); }
-  if (out >= 0) stw<W>(a.go + (long)out * H + j, mh);
+__global__ void lstm_round_leaves_fwd_kernel(RoundLeavesArgs a) {
+  lstm_leaves_at<W>(a, (long)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 struct LstmBwdGatesArgs {
@@ -781,7 +739,7 @@ int cavs_lstm_round_leaves_fwd(float *pool, const int *pair, const float *xW, in
   if (n == 0) return CAVS_OK;
   CAVS_REQUIRE(pool && pair && xW && bias && gates && msg, "cavs_lstm_round_leaves_fwd: null pointer");
   CAVS_REQUIRE(!graph_out || out_rows, "cavs_lstm_round_leaves_fwd: graph_out needs out_rows");
-  LstmLeavesArgs a{xW, ld_xw, bias, pair, gates, msg, pool, graph_out, out_rows, n, H};
+  RoundLeavesArgs a{xW, ld_xw, bias, pair, gates, msg, pool, graph_out, out_rows, n, H};
   const bool vec = H % 4 == 0 && ld_xw % 4 == 0 && all16({pool, xW, bias, gates, msg, graph_out});
   launch_pointwise(a, n, H, vec, as_stream(stream), lstm_round_leaves_fwd_kernel<4>, lstm_round_leaves_fwd_kernel<1>);
   CAVS_LAUNCH_CHECK();

@@ -134,7 +134,8 @@ __global__ __launch_bounds__(256) void fc_xent_kernel(const float *__restrict__ 
 // out[i] = sum over the workgroups' partials: four interleaved slices per output, each added
 // in index order, combined in a fixed order
 __device__ inline void sum_parts_block(const float *__restrict__ part, int nparts, int total, int CH,
-                                       float *__restrict__ dW, float *__restrict__ db, int block, float (&s)[4][64]) {
+                                       float *__restrict__ dW, float *__restrict__ db, int block, float (&s)[4][64], float lr = 0.f,
+                                       float *__restrict__ W = nullptr, float *__restrict__ bias = nullptr) {
   const int o = threadIdx.x & 63, q = threadIdx.x >> 6;
   const int i = block * 64 + o;
   float a0 = 0.f, a1 = 0.f;
@@ -168,6 +169,8 @@ __device__ inline void sum_parts_block(const float *__restrict__ part, int npart
   if (q == 0 && i < total) {
     const float v = (s[0][o] + s[1][o]) + (s[2][o] + s[3][o]);
     if (i < CH) dW[i] = v; else db[i - CH] = v;
+    if (W && i < CH) W[i] -= lr * v;
+    if (bias && i >= CH) bias[i - CH] -= lr * v;
   }
 }
 
@@ -431,6 +434,9 @@ __global__ __launch_bounds__(256) void tasks_kernel(TaskList L) {
       __syncthreads();
       const int tt = tid >> 6, slot = (tid >> 4) & 3, x = tid & 15, col = 16 * tt + x;
       if (16 * (4 * cb + tt) >= N) break;
+      if (t.p3)  // the transpose's: its k-groups are B's column tiles
+        static_cast<float4 *>(t.p3)[(((long)(4 * cb + tt) * (t.n0 / 16) + kg) * 4 + slot) * 16 + x] =
+            make_float4(lds.pk[x][16 * tt + 4 * slot], lds.pk[x][16 * tt + 4 * slot + 1], lds.pk[x][16 * tt + 4 * slot + 2], lds.pk[x][16 * tt + 4 * slot + 3]);
       out[(((long)kg * (N / 16) + 4 * cb + tt) * 4 + slot) * 16 + x] =
           make_float4(lds.pk[4 * slot][col], lds.pk[4 * slot + 1][col], lds.pk[4 * slot + 2][col], lds.pk[4 * slot + 3][col]);
       break;
@@ -489,8 +495,17 @@ __global__ __launch_bounds__(256) void tasks_kernel(TaskList L) {
     }
     case CAVS_TASK_SUM_PARTS:  // p1[i] (i < n2) or p2[i - n2] = sum over p < n0 of p0[p * n1 + i], i < n1
       sum_parts_block(static_cast<const float *>(t.p0), (int)t.n0, (int)t.n1, (int)t.n2, static_cast<float *>(t.p1),
-                      static_cast<float *>(t.p2), b, lds.sums);
+                      static_cast<float *>(t.p2), b, lds.sums, t.f0, static_cast<float *>(t.p3), static_cast<float *>(t.p4));
       break;
+    case CAVS_TASK_TREELSTM_LEAVES:
+    case CAVS_TASK_LSTM_LEAVES: {
+      const RoundLeavesArgs a{static_cast<const float *>(t.p2), (long)t.n2, static_cast<const float *>(t.p3), static_cast<const int *>(t.p1),
+                              static_cast<float *>(t.p4), static_cast<float *>(t.p5), static_cast<float *>(t.p0), static_cast<float *>(t.p6),
+                              static_cast<const int *>(t.p7), (int)t.n0, (int)t.n1};
+      if (t.kind == CAVS_TASK_LSTM_LEAVES) lstm_leaves_at<4>(a, (long)b * 256 + tid);
+      else treelstm_leaves_at<4>(a, (long)b * 256 + tid);
+      break;
+    }
     case CAVS_TASK_TREELSTM_GATES_ROWS: {  // cavs_treelstm_bwd_gates_rows as a job
       const BwdGatesRowsArgs a{static_cast<const int *>(t.p0), static_cast<const float *>(t.p1), static_cast<const int *>(t.p2),
                                static_cast<const float *>(t.p3), static_cast<const float *>(t.p4), static_cast<float *>(t.p5),
@@ -617,7 +632,7 @@ int cavs_run_tasks(int count, const cavs_task *tasks, void *stream) {
                      "cavs_run_tasks: job %d: bad shape to pack (rows and columns multiples of 16)", i);
         if (t.n0 == 0 || t.n1 == 0) continue;
         CAVS_REQUIRE(t.p0 && t.p1 && t.p0 != t.p1 && t.p0 != t.p2, "cavs_run_tasks: job %d: null or aliased pointer", i);
-        CAVS_REQUIRE(aligned16(t.p0) && aligned16(t.p1) && aligned16(t.p2), "cavs_run_tasks: job %d: pack needs 16-byte aligned pointers", i);
+        CAVS_REQUIRE(aligned16(t.p0) && aligned16(t.p1) && aligned16(t.p2) && aligned16(t.p3), "cavs_run_tasks: job %d: pack needs 16-byte aligned pointers", i);
         blocks = (t.n0 / 16) * ((t.n1 + 63) / 64);
         break;
       case CAVS_TASK_ZERO_ROWS:
@@ -663,6 +678,16 @@ int cavs_run_tasks(int count, const cavs_task *tasks, void *stream) {
         blocks = (t.n0 * (t.n1 / 4) + 255) / 256;
         break;
       }
+      case CAVS_TASK_TREELSTM_LEAVES:
+      case CAVS_TASK_LSTM_LEAVES:
+        CAVS_REQUIRE(t.n0 >= 0 && t.n0 < (1 << 24) && t.n1 > 0 && t.n1 < (1 << 20) && t.n1 % 4 == 0 && t.n2 >= 4 * t.n1 && t.n2 % 4 == 0,
+                     "cavs_run_tasks: job %d: bad shape of a round of leaves", i);
+        if (t.n0 == 0) continue;
+        CAVS_REQUIRE(t.p0 && t.p1 && t.p2 && t.p3 && t.p4 && (t.p5 || t.kind == CAVS_TASK_TREELSTM_LEAVES) && (!t.p6 || t.p7), "cavs_run_tasks: job %d: null pointer", i);
+        CAVS_REQUIRE(aligned16(t.p0) && aligned16(t.p2) && aligned16(t.p3) && aligned16(t.p4) && aligned16(t.p5) && aligned16(t.p6),
+                     "cavs_run_tasks: job %d: a round of leaves needs 16-byte aligned pointers", i);
+        blocks = (t.n0 * (t.n1 / 4) + 255) / 256;
+        break;
       case CAVS_TASK_SUM_PARTS:
         CAVS_REQUIRE(t.n0 >= 0 && t.n1 >= 0 && t.n1 < (1 << 30) && t.n0 < (1 << 30) && t.n2 >= 0 && t.n2 <= t.n1,
                      "cavs_run_tasks: job %d: bad shape", i);

@@ -250,7 +250,7 @@ void Engine::tail_check() {
   // word: the parameters are those of the last good step.  From here on: one launch per round.
   tail_ready_ = false;
   state_epoch_++;
-  upk_valid_ = wfct_valid_ = false;
+  upk_valid_ = utp_valid_ = wfct_valid_ = false;
   emb_sparse_valid_ = false;
   check(cavs_zero(tail_sync_.get(), cavs_tail_sync_bytes(), stream_));
   fail(CAVS_EHIP, std::string("a launch over the rounds near the roots gave up (") +
@@ -341,7 +341,7 @@ void Engine::bind_param(const std::string &name, float *w, float *g) {
     p.ug = g ? g : p.own_ug.get();
     return;
   }
-  if (p.w != w) upk_valid_ = wfct_valid_ = false;
+  if (p.w != w) upk_valid_ = utp_valid_ = wfct_valid_ = false;
   p.w = w;
   p.g = g ? g : p.own_g.get();
 }
@@ -361,18 +361,21 @@ bool Engine::update_jobs(float *w, float *g, float lr, std::vector<cavs_task> *o
   }
   if (Upk_.capacity() == 0) return false;
   const long long H = cfg_.H;
+  // the transposed copy as well, where the resident backward launch reads one (a recorded step makes it each time)
+  float *tp = UTp_.capacity() > 0 && !cfg_.graph_replay ? UTp_.get() : nullptr;
   if (cfg_.model == CAVS_MODEL_TREELSTM && w == param("U").w) {
-    out->push_back({CAVS_TASK_SGD_PACK, lr, H, 3 * H, 0, Upk_.get(), w, g, nullptr});
-    out->push_back({CAVS_TASK_SGD_PACK, lr, H, H, 0, Upk_.at((size_t)3 * H * H), w + 3 * H * H, g + 3 * H * H, nullptr});
+    out->push_back({CAVS_TASK_SGD_PACK, lr, H, 3 * H, 0, Upk_.get(), w, g, tp});
+    out->push_back({CAVS_TASK_SGD_PACK, lr, H, H, 0, Upk_.at((size_t)3 * H * H), w + 3 * H * H, g + 3 * H * H, tp ? tp + 3 * H * H : nullptr});
   } else if (cfg_.model == CAVS_MODEL_LSTM && w == param("W").w) {  // [U' | W'], W' with its packed copy
     const long long half = 4 * H * E_;
     out->push_back({CAVS_TASK_SGD, lr, half, 0, 0, w, g, nullptr, nullptr});
-    out->push_back({CAVS_TASK_SGD_PACK, lr, H, 4 * H, 0, Upk_.get(), w + half, g + half, nullptr});
+    out->push_back({CAVS_TASK_SGD_PACK, lr, H, 4 * H, 0, Upk_.get(), w + half, g + half, tp});
   } else if (cfg_.model == CAVS_MODEL_TREEFC && w == param("W").w) {
-    out->push_back({CAVS_TASK_SGD_PACK, lr, 2 * H, H, 0, Upk_.get(), w, g, nullptr});
+    out->push_back({CAVS_TASK_SGD_PACK, lr, 2 * H, H, 0, Upk_.get(), w, g, tp});
   } else {
     return false;
   }
+  utp_valid_ = tp != nullptr;
   upk_valid_ = true;
   return true;
 }
@@ -387,7 +390,7 @@ void Engine::set_param(const std::string &name, const float *host, size_t n) {
   block_jobs(p, pad_stage_.get(), p.w, false, &jobs);
   copy_blocks(jobs);
   check(cavs_stream_sync(stream_));
-  upk_valid_ = wfct_valid_ = false;
+  upk_valid_ = utp_valid_ = wfct_valid_ = false;
   state_epoch_++;
 }
 
@@ -651,7 +654,7 @@ void Engine::reserve_edges() {
     R(Upk_, (size_t)4 * H * H);
   if (group_.first >= 0 && !cell_) {
     R(Upk_, (size_t)(cfg_.model == CAVS_MODEL_TREEFC ? 2 : 4) * H * H);
-    R(UTp_, (size_t)(cfg_.model == CAVS_MODEL_TREEFC ? 2 : 4) * H * H);
+    if (ensure(UTp_, (size_t)(cfg_.model == CAVS_MODEL_TREEFC ? 2 : 4) * H * H)) utp_valid_ = false;
   }
   if (cfg_.model == CAVS_MODEL_TREELSTM) {
     R(hlr_, cap * H);
@@ -1070,6 +1073,7 @@ void Engine::begin_step(const int *graph, int B, int maxlen) {
   bias_jobs_.clear();
   head_chunks_.clear();  // (planned with the host scheduler's lists only)
   pending_tasks_.clear();  // (a step that failed half way may have left a job for a backward pass that never ran)
+  emb_cleared_ = false;
   wait_ms_ = 0.f;
   uint64_t hash = 0;
   Plan *hit = nullptr;
@@ -1127,6 +1131,7 @@ void Engine::begin_step(const int *graph, int B, int maxlen) {
 void Engine::forward_only(const int *graph, int B, int maxlen, const float *x_dev, float *graph_out, bool trains) {
   state_epoch_++;
   trains_ = trains;
+  whole_step_ = false;
   begin_step(graph, B, maxlen);
   const bool reads_x = cell_ ? cell_->NX > 0 || cell_->XD > 0 : (cfg_.model != CAVS_MODEL_TREEFC || cfg_.use_x);
   if (reads_x && !x_dev) fail(CAVS_EINVAL, "vertex input feed is null");
@@ -1141,7 +1146,7 @@ void Engine::forward_only(const int *graph, int B, int maxlen, const float *x_de
     for (auto &kv : params_)
       if (kv.second->uw) block_jobs(*kv.second, kv.second->uw, kv.second->w, false, &jobs);
     copy_blocks(jobs);
-    upk_valid_ = false;
+    upk_valid_ = utp_valid_ = false;
   }
   model_forward();
   pop_ret(fwd_out_);
@@ -1323,7 +1328,9 @@ void Engine::step(const int *graph, int B, int maxlen, const void *x, const void
     ~StepTimer() { e->host_step_ms_ = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count(); }
   } step_timer{this, step_t0};
   trains_ = backward;
+  whole_step_ = false;
   begin_step(graph, B, maxlen);
+  whole_step_ = backward && !cfg_.graph_replay && !profile_;
   const int N = N_;
   const bool needs_x = cfg_.model != CAVS_MODEL_TREEFC || cfg_.use_x;
   const size_t xw = cfg_.model == CAVS_MODEL_TREEFC ? uH_ : 1;
@@ -1403,6 +1410,16 @@ void Engine::step(const int *graph, int B, int maxlen, const void *x, const void
       std::vector<std::string> by_job;
       for (const BiasJob &j : bias_jobs_) by_job.push_back(j.param);
       settle_bias_jobs(lr, &tasks);
+      for (cavs_task &t : pending_tasks_) {
+        if (cfg_.loss == CAVS_LOSS_SOFTMAX) {  // the sums are the gradients of the head
+          t.f0 = lr;
+          t.p3 = param("Wfc").w;
+          t.p4 = param("bfc").w;
+          by_job.insert(by_job.end(), {"Wfc", "bfc"});
+        }
+        tasks.push_back(t);
+      }
+      pending_tasks_.clear();
       for (auto &kv : params_) {
         Param &p = *kv.second;
         if (std::find(by_job.begin(), by_job.end(), kv.first) != by_job.end()) continue;  // updated by the job that delivers its gradient
@@ -1418,7 +1435,10 @@ void Engine::step(const int *graph, int B, int maxlen, const void *x, const void
         // the recurrent weights, a wide head's weights: the update and the copy the kernels read in one job
         if (update_jobs(p.w, p.g, lr, &tasks)) {
           // a caller's own tensor may be written behind the engine's back
-          if (p.w != p.own_w.get()) (kv.first == "Wfc" ? wfct_valid_ : upk_valid_) = false;
+          if (p.w != p.own_w.get()) {
+            (kv.first == "Wfc" ? wfct_valid_ : upk_valid_) = false;
+            utp_valid_ = false;
+          }
           continue;
         }
         tasks.push_back({CAVS_TASK_SGD, lr, (long long)p.n, 0, 0, p.w, p.g, nullptr, nullptr});
@@ -1428,7 +1448,14 @@ void Engine::step(const int *graph, int B, int maxlen, const void *x, const void
       if (end_stamped_) m.step = steps_;
       c_launches_ += 1;
     } else {
-      settle_bias_jobs(0.f, nullptr);
+      std::vector<cavs_task> tasks;
+      settle_bias_jobs(0.f, &tasks);
+      tasks.insert(tasks.end(), pending_tasks_.begin(), pending_tasks_.end());
+      pending_tasks_.clear();
+      if (!tasks.empty()) {
+        check(cavs_run_tasks((int)tasks.size(), tasks.data(), stream_));
+        c_launches_ += 1;
+      }
     }
   }
 }
@@ -1535,8 +1562,11 @@ void Engine::treelstm_forward() {
     // rows themselves nobody reads it and the fused launches skip it
     float *msg = out_folded_ ? nullptr : msg_.at(off * 2 * H);
     if (leaf_round(r) && fused > 0) {  // (elementwise: a round of any size)
-      CAVS_TIMED(K_GATES, cavs_treelstm_round_leaves_fwd(pool_.get(), d_pair_ + off, xW_.at(off * 4 * H), 4 * H, Bv, gates_.at(off * 6 * H),
-                                                         msg, go, d_t2j_ + off, r.n, H, stream_));
+      const cavs_task leaves{CAVS_TASK_TREELSTM_LEAVES, 0.f, r.n, H, 4 * H, pool_.get(), const_cast<int *>(d_pair_ + off), xW_.at(off * 4 * H),
+                             const_cast<float *>(Bv), gates_.at(off * 6 * H), msg, go, const_cast<int *>(d_t2j_ + off)};
+      if (!leaves_with_company(leaves))
+        CAVS_TIMED(K_GATES, cavs_treelstm_round_leaves_fwd(pool_.get(), d_pair_ + off, xW_.at(off * 4 * H), 4 * H, Bv, gates_.at(off * 6 * H),
+                                                           msg, go, d_t2j_ + off, r.n, H, stream_));
       c_scatter_rows_ += r.n;
       c_launches_ += 1;
       continue;
@@ -1607,14 +1637,18 @@ void Engine::treelstm_backward() {
   const bool roots_grouped = group_.first >= 0;  // (the group launch has lists of them)
   const bool roots_ride = folded && !roots_grouped && fused > 0 && H % 4 == 0 && n_orphans_ > 0;
   std::vector<cavs_task> opening;
-  if (fused > 0) {  // U_iou^T and U_f^T: the B operand of the children products, k-major
+  bool rest = group_.first < 0;  // rounds that are launches of their own
+  for (int k = 0; k < group_.first; k++) rest |= !leaf_round(sched_->rounds[k]);
+  const bool grouped_tp = group_.first >= 0 && (!packed || !rest);  // the group launch reads its own copy
+  if (grouped_tp && !utp_valid_) {
+    opening.push_back({CAVS_TASK_PACK_T, 0.f, H, 3 * H, 0, UTp_.get(), const_cast<float *>(U), nullptr, nullptr});
+    opening.push_back({CAVS_TASK_PACK_T, 0.f, H, H, 0, UTp_.at((size_t)3 * H * H), const_cast<float *>(U) + (size_t)3 * H * H, nullptr, nullptr});
+    utp_valid_ = !cfg_.graph_replay && param("U").w == param("U").own_w.get();
+  }
+  if (fused > 0 && rest) {  // U_iou^T and U_f^T: the B operand of the children products, k-major
     const int kind = packed ? CAVS_TASK_PACK_T : CAVS_TASK_TRANSPOSE;
     opening.push_back({kind, 0.f, H, 3 * H, 0, UT_.get(), const_cast<float *>(U), nullptr, nullptr});
     opening.push_back({kind, 0.f, H, H, 0, UT_.at((size_t)3 * H * H), const_cast<float *>(U) + (size_t)3 * H * H, nullptr, nullptr});
-    if (group_.first >= 0 && !packed) {
-      opening.push_back({CAVS_TASK_PACK_T, 0.f, H, 3 * H, 0, UTp_.get(), const_cast<float *>(U), nullptr, nullptr});
-      opening.push_back({CAVS_TASK_PACK_T, 0.f, H, H, 0, UTp_.at((size_t)3 * H * H), const_cast<float *>(U) + (size_t)3 * H * H, nullptr, nullptr});
-    }
   }
   if (roots_ride)
     opening.push_back({CAVS_TASK_TREELSTM_GATES_ROWS, 0.f, n_orphans_, H, (long long)sched_->leaf_prefix | ((long long)(4 * H) << 32),
@@ -1648,7 +1682,7 @@ void Engine::treelstm_backward() {
   }
   if (group_.first >= 0) {
     const cavs_group_plan plan = group_plan(group_.bwd);
-    CAVS_TIMED(K_ROUND, cavs_treelstm_group_bwd(dxW_.get(), 4 * H, dF_.get(), dc_.get(), packed ? UT_.get() : UTp_.get(), gates_.get(), G_.get(),
+    CAVS_TIMED(K_ROUND, cavs_treelstm_group_bwd(dxW_.get(), 4 * H, dF_.get(), dc_.get(), grouped_tp ? UTp_.get() : UT_.get(), gates_.get(), G_.get(),
                                                 d_dgo_, sched_->leaf_prefix, H, &plan, stream_));
     group_launched();
   }
@@ -1845,6 +1879,27 @@ void Engine::settle_bias_jobs(float lr, std::vector<cavs_task> *tasks) {
   }
 }
 
+// The rows of the embedding's gradient that the previous step looked up, as a job of the caller's launch (once a step).
+void Engine::clear_embedding(std::vector<cavs_task> *tasks) {
+  Param &emb = param("Emb");
+  if (emb_cleared_ || emb.g != emb.own_g.get() || !emb_sparse_valid_) return;
+  if (emb_dirty_n_ > 0)
+    tasks->push_back({CAVS_TASK_ZERO_ROWS, 0.f, emb_dirty_n_, (long long)(emb.n / cfg_.V), 0, emb.g, xs_prev_.get(), nullptr, nullptr});
+  emb_cleared_ = true;
+}
+
+// A round of leaves; what has to be done before the backward pass and can be done now rides in its launch.  (With the transposed
+// weights written by the update, the roots in the resident launch and the head's sums in the launch of the updates, nothing opens a
+// backward pass any more: 64 trees, H = 512, 329 -> 324 us a step, 25 trees, H = 150, 189 -> 184.)
+bool Engine::leaves_with_company(cavs_task leaves) {
+  if (!whole_step_ || cfg_.H % 4) return false;
+  std::vector<cavs_task> tasks{leaves};
+  clear_embedding(&tasks);
+  if (tasks.size() == 1) return false;
+  CAVS_TIMED(K_GATES, cavs_run_tasks((int)tasks.size(), tasks.data(), stream_));
+  return true;
+}
+
 // EmbeddingLookup_grad (cavs/backend/op_impl_embedding.cu:58-92): scatter-add of the rows of
 // de into a zeroed table.  The table is kept zero outside the rows of the previous step, so
 // clearing it costs those rows, not the vocabulary.
@@ -1852,16 +1907,11 @@ void Engine::settle_bias_jobs(float lr, std::vector<cavs_task> *tasks) {
 // the embedding gradient (the rows the previous step looked up) do not depend on each other:
 // one launch.
 void Engine::backward_prologue(std::vector<cavs_task> tasks, bool with_embedding) {
+  if (with_embedding) clear_embedding(&tasks);
+  // nothing but sums that the update waits for: they ride in the launch that ends the step
+  if (tasks.empty() && whole_step_) return;
   tasks.insert(tasks.end(), pending_tasks_.begin(), pending_tasks_.end());
   pending_tasks_.clear();
-  if (with_embedding) {
-    Param &emb = param("Emb");
-    if (emb.g == emb.own_g.get() && emb_sparse_valid_) {
-      if (emb_dirty_n_ > 0)
-        tasks.push_back({CAVS_TASK_ZERO_ROWS, 0.f, emb_dirty_n_, (long long)(emb.n / cfg_.V), 0, emb.g, xs_prev_.get(), nullptr, nullptr});
-      emb_cleared_ = true;
-    }
-  }
   if (tasks.empty()) return;
   CAVS_TIMED(K_OTHER, cavs_run_tasks((int)tasks.size(), tasks.data(), stream_));
   c_launches_ += 1;
@@ -1934,8 +1984,11 @@ void Engine::lstm_forward() {
     float *a = xW_.at(off * 4 * H), *msg = msg_.at(off * 2 * H), *G = nullptr;
     if (r.n <= fused) {  // one launch: Gather, h*W', gates, Scatter, Push/PopRet
       if (leaf_round(r)) {
-        CAVS_TIMED(K_GATES, cavs_lstm_round_leaves_fwd(pool_.get(), d_pair_ + off, a, 4 * H, Bv, gates_.at(off * 5 * H), msg, go,
-                                                       d_t2j_ + off, r.n, H, stream_));
+        const cavs_task leaves{CAVS_TASK_LSTM_LEAVES, 0.f, r.n, H, 4 * H, pool_.get(), const_cast<int *>(d_pair_ + off), a, const_cast<float *>(Bv),
+                               gates_.at(off * 5 * H), msg, go, const_cast<int *>(d_t2j_ + off)};
+        if (!leaves_with_company(leaves))
+          CAVS_TIMED(K_GATES, cavs_lstm_round_leaves_fwd(pool_.get(), d_pair_ + off, a, 4 * H, Bv, gates_.at(off * 5 * H), msg, go,
+                                                         d_t2j_ + off, r.n, H, stream_));
       } else {
         const bool pk = any_packed && cavs_lstm_round_packed_ok(r.n, H);
         CAVS_TIMED(K_ROUND, (pk ? cavs_lstm_round_fwd_packed : cavs_lstm_round_fwd)(
@@ -1971,14 +2024,18 @@ void Engine::lstm_backward() {
     if (group_backward((int)k)) break;
     if (!leaf_round(r) && !cavs_lstm_round_packed_ok(r.n, H)) packed = false;
   }
-  if (fused > 0) {  // W'^T: the B operand of d h_prev = da * W'^T, k-major
-    std::vector<cavs_task> opening{{packed ? CAVS_TASK_PACK_T : CAVS_TASK_TRANSPOSE, 0.f, H, 4 * H, 0, UT_.get(), const_cast<float *>(Wh), nullptr,
-                                    nullptr}};
-    if (group_.first >= 0 && !head_chunked_ && !packed) opening.push_back({CAVS_TASK_PACK_T, 0.f, H, 4 * H, 0, UTp_.get(), const_cast<float *>(Wh), nullptr, nullptr});
-    backward_prologue(opening, true);
-  } else {
-    backward_prologue({}, true);
+  const bool resident = group_.first >= 0 && !head_chunked_;
+  bool rest = !resident;  // rounds that are launches of their own
+  for (int k = 0; resident && k < group_.first; k++) rest |= !leaf_round(sched_->rounds[k]);
+  const bool grouped_tp = resident && (!packed || !rest);  // the group launch reads its own copy
+  std::vector<cavs_task> opening;
+  if (fused > 0 && rest)  // W'^T: the B operand of d h_prev = da * W'^T, k-major
+    opening.push_back({packed ? CAVS_TASK_PACK_T : CAVS_TASK_TRANSPOSE, 0.f, H, 4 * H, 0, UT_.get(), const_cast<float *>(Wh), nullptr, nullptr});
+  if (grouped_tp && !utp_valid_) {
+    opening.push_back({CAVS_TASK_PACK_T, 0.f, H, 4 * H, 0, UTp_.get(), const_cast<float *>(Wh), nullptr, nullptr});
+    utp_valid_ = !cfg_.graph_replay && param("W").w == param("W").own_w.get();
   }
+  backward_prologue(opening, true);
   const bool folded = forest_;  // one launch per round, as in treelstm_backward
   // a wide head in chunks: d h comes in slab order, chunk by chunk, the last rounds' first
   const float *dret = head_chunked_ ? dret_.get() : d_dgo_;
@@ -1993,7 +2050,7 @@ void Engine::lstm_backward() {
   // slow each other down more than a launch per round does -- C4 3.89 ms per step against 3.60.)
   if (group_.first >= 0 && !head_chunked_) {
     const cavs_group_plan plan = group_plan(group_.bwd);
-    CAVS_TIMED(K_ROUND, cavs_lstm_group_bwd(dxW_.get(), 4 * H, dc_.get(), packed ? UT_.get() : UTp_.get(), gates_.get(), G_.get(), d_dgo_,
+    CAVS_TIMED(K_ROUND, cavs_lstm_group_bwd(dxW_.get(), 4 * H, dc_.get(), grouped_tp ? UTp_.get() : UT_.get(), gates_.get(), G_.get(), d_dgo_,
                                             sched_->leaf_prefix, H, &plan, stream_));
     group_launched();
   }
@@ -2143,7 +2200,10 @@ void Engine::treefc_backward() {
     bool rest = group_.first < 0;  // rounds that are launches of their own
     for (int k = 0; k < group_.first; k++) rest |= !leaf_round(sched_->rounds[k]);
     if (rest) opening.push_back({CAVS_TASK_TRANSPOSE, 0.f, 2 * H, H, 0, UT_.get(), const_cast<float *>(W), nullptr, nullptr});
-    if (group_.first >= 0) opening.push_back({CAVS_TASK_PACK_T, 0.f, 2 * H, H, 0, UTp_.get(), const_cast<float *>(W), nullptr, nullptr});
+    if (group_.first >= 0 && !utp_valid_) {
+      opening.push_back({CAVS_TASK_PACK_T, 0.f, 2 * H, H, 0, UTp_.get(), const_cast<float *>(W), nullptr, nullptr});
+      utp_valid_ = !cfg_.graph_replay && param("W").w == param("W").own_w.get();
+    }
     backward_prologue(opening, false);
   } else {
     backward_prologue({}, false);

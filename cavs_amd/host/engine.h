@@ -47,7 +47,7 @@ class Engine {
   void bind_param(const std::string &name, float *w, float *g);
   // somebody else has written bound weights: no copy of them is current
   void weights_written() {
-    upk_valid_ = wfct_valid_ = false;
+    upk_valid_ = utp_valid_ = wfct_valid_ = false;
     state_epoch_++;
   }
   // where the next backward pass leaves the gradient of `name` (null: the engine's own buffer)
@@ -403,6 +403,10 @@ class Engine {
   DeviceArray<float> word_ids_, word_scratch_;
   bool words_ = false;
   bool trains_ = true;  // a backward pass follows
+  bool whole_step_ = false;  // ... and the update, in the same call: nobody looks in between
+  bool utp_valid_ = false;   // UTp_ is the weights'
+  void clear_embedding(std::vector<cavs_task> *tasks);
+  bool leaves_with_company(cavs_task leaves);
   const int *d_words_index_ = nullptr;
   DeviceArray<float> xW_words_, d_words_, word_parts_;
   int pad_block() const { return uH_ != cfg_.H ? cfg_.H : 0; }  // padding of x * W (cavs_gemm_desc::pad_block, uH_ used)

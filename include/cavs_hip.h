@@ -677,7 +677,8 @@ int cavs_root_sq(float *parts, float *dgraph_out, const float *graph_out, const 
  *   CAVS_TASK_EMBED_SGD  cavs_embed_sgd(p0 = table, p1 = dtable, p2 = ids, n0 = n, n1 = E,
  *                                       f0 = lr, p3 = stamp, n2 = epoch)
  *   CAVS_TASK_SUM_PARTS  out[i] = sum over p < n0 of p0[p * n1 + i] in a fixed order, i < n1, where
- *                        out[i] is p1[i] for i < n2 and p2[i - n2] above
+ *                        out[i] is p1[i] for i < n2 and p2[i - n2] above; and p3[i], p4[i - n2] -= f0 * it
+ *                        where they are given (the update of what the sums are the gradient of)
  *   CAVS_TASK_BLOCKS_SGD p1 holds n1 (<= 8) blocks of n0 floats; block k goes to block d_k of p2 (if
  *                        given) and p0[d_k block] -= f0 * it (if p0 given); d_k = (n2 >> 4k) & 15, a
  *                        permutation.  A gradient that arrives in another block order than its
@@ -691,7 +692,8 @@ int cavs_root_sq(float *parts, float *dgraph_out, const float *graph_out, const 
  *   CAVS_TASK_SGD_PACK   p1[i] -= f0 * p2[i] (skipped when p2 is null), then p0 = B = p1 ([K = n0, N = n1]
  *                        row-major; both multiples of 16) in the same tile-major layout: the
  *                        parameter update (cavs/backend/op_impl_sgd.cu) and the packed copy the next
- *                        forward pass reads, in one pass over the weights.
+ *                        forward pass reads, in one pass over the weights.  p3 (if given): what CAVS_TASK_PACK_T
+ *                        makes of p1, the copy the next backward pass reads.
  *   CAVS_TASK_SGD_TRANSPOSE  p1[i] -= f0 * p2[i] (skipped when p2 is null), then p0[c][r] = p1[r][c], n0 rows,
  *                        n1 columns: the update of a wide classifier's weights [C, H]
  *                        (cavs/backend/op_impl_fullyconnected_cublas.cc:71-79) and the [H, C] copy the
@@ -700,14 +702,18 @@ int cavs_root_sq(float *parts, float *dgraph_out, const float *graph_out, const 
  *                        dret_rows = p2, gates = p3, G = p4, dxW = p5, ld_dxw = n2 >> 32, dF = p6,
  *                        dc = p7, leaf_rows = n2 & 0xffffffff, H = n1; H a multiple of 4): the gate
  *                        gradients of the roots ride in the launch that opens the backward pass.
+ *   CAVS_TASK_TREELSTM_LEAVES, CAVS_TASK_LSTM_LEAVES  cavs_treelstm_round_leaves_fwd, cavs_lstm_round_leaves_fwd(pool = p0, pair = p1,
+ *                        xW = p2, ld_xw = n2, bias = p3, gates = p4, msg = p5, graph_out = p6, out_rows = p7,
+ *                        n = n0, H = n1 a multiple of 4, pointers 16-byte aligned)
  *   CAVS_TASK_GUARD      not a job: when the int p0 points at is not zero as the launch runs, none of
  *                        its jobs does anything (the parameter updates of a step whose
  *                        cavs_treelstm_tail_* launch gave up: p0 = the status word of its sync block).
  *                        At most one per launch; it does not count towards the 12.
- * p4 .. p7 are read by CAVS_TASK_TREELSTM_GATES_ROWS only and may stay null otherwise. */
+ * p4 .. p7 are read by the jobs that name them only and may stay null otherwise. */
 enum { CAVS_TASK_TRANSPOSE = 0, CAVS_TASK_ZERO_ROWS = 1, CAVS_TASK_SGD = 2, CAVS_TASK_EMBED_SGD = 3,
        CAVS_TASK_SUM_PARTS = 4, CAVS_TASK_BLOCKS_SGD = 5, CAVS_TASK_PACK_T = 6, CAVS_TASK_SGD_PACK = 7,
-       CAVS_TASK_TREELSTM_GATES_ROWS = 8, CAVS_TASK_SGD_TRANSPOSE = 9, CAVS_TASK_GUARD = 10 };
+       CAVS_TASK_TREELSTM_GATES_ROWS = 8, CAVS_TASK_SGD_TRANSPOSE = 9, CAVS_TASK_GUARD = 10,
+       CAVS_TASK_TREELSTM_LEAVES = 11, CAVS_TASK_LSTM_LEAVES = 12 };
 typedef struct cavs_task {
   int kind;
   float f0;

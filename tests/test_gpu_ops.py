@@ -2001,6 +2001,52 @@ def test_squares_of_the_roots(g, B, N, H):
         assert not back or np.array_equal(g.host(dgo).reshape(N, H), want)
 
 
+@pytest.mark.parametrize("n,H", [(1, 16), (5, 32), (70, 96), (33, 512)])
+def test_jobs_that_ride_at_either_end_of_a_step(g, n, H):
+    """A round of leaves as a job: the bits of the launch of its own.  The update of recurrent weights with both packed copies: those of the
+    update and of CAVS_TASK_PACK_T behind it.  Sums with the update of what they are the gradient of: those of the two jobs."""
+    import torch
+
+    r, T = rng(n + H), hip.Task
+    u = lambda *s: g.devf(r.bulk_uniform(int(np.prod(s)), -1, 1))
+    empty = lambda *s: torch.full(s, float("nan"), dtype=torch.float32, device="cuda")
+    run = lambda *jobs: g.call("cavs_run_tasks", len(jobs), (T * len(jobs))(*jobs), g.stream())
+    pair, rows = g.devi(np.where(np.arange(n) % 3 == 1, -1, np.arange(n)[::-1])), g.devi(np.arange(n)[::-1].copy())
+    xW, bias = u(n, 4 * H), u(4 * H)
+    for kind, name, ng in ((hip.TASK_TREELSTM_LEAVES, "treelstm", 6), (hip.TASK_LSTM_LEAVES, "lstm", 5)):
+        res = []
+        for job in (False, True):
+            pool, gates, msg, go = empty(n, 2 * H), empty(n, ng * H), empty(n, 2 * H), empty(n, H)
+            if job:
+                run(T(kind, 0.0, n, H, 4 * H, g.P(pool), g.P(pair), g.P(xW), g.P(bias), g.P(gates), g.P(msg), g.P(go), g.P(rows)))
+            else:
+                g.call(f"cavs_{name}_round_leaves_fwd", g.P(pool), g.P(pair), g.P(xW), 4 * H, g.P(bias), g.P(gates), g.P(msg), g.P(go), g.P(rows), n, H,
+                       g.stream())
+            res.append([g.host(t) for t in (pool, gates, msg, go)])
+        for a, b in zip(*res):
+            np.testing.assert_array_equal(a, b)
+    w, grad, lr = r.bulk_uniform(3 * H * H, -1, 1), u(H, 3 * H), 0.25
+    res = []
+    for both in (False, True):
+        d_w, p, tp = g.devf(w), empty(3 * H * H), empty(3 * H * H)
+        run(T(hip.TASK_SGD_PACK, lr, H, 3 * H, 0, g.P(p), g.P(d_w), g.P(grad), g.P(tp) if both else None))
+        if not both:
+            run(T(hip.TASK_PACK_T, 0.0, H, 3 * H, 0, g.P(tp), g.P(d_w), None, None))
+        res.append([g.host(t) for t in (d_w, p, tp)])
+    for a, b in zip(*res):
+        np.testing.assert_array_equal(a, b)
+    parts, w0, b0 = u(41, H + 3), r.bulk_uniform(H, -1, 1), r.bulk_uniform(3, -1, 1)
+    res = []
+    for both in (False, True):
+        W, b, dW, db = g.devf(w0), g.devf(b0), empty(H), empty(3)
+        run(T(hip.TASK_SUM_PARTS, lr, 41, H + 3, H, g.P(parts), g.P(dW), g.P(db), g.P(W) if both else None, g.P(b) if both else None))
+        if not both:
+            run(T(hip.TASK_SGD, lr, H, 0, 0, g.P(W), g.P(dW), None, None), T(hip.TASK_SGD, lr, 3, 0, 0, g.P(b), g.P(db), None, None))
+        res.append([g.host(t) for t in (W, b, dW, db)])
+    for a, b in zip(*res):
+        np.testing.assert_array_equal(a, b)
+
+
 @pytest.mark.parametrize("n,V,leaf_rows", [(17408, 200, 3), (17409, 255, 17409), (70001, 21701, 36000), (33000, 70000, 0), (262145, 1 << 16, 100000)])
 def test_words_of_a_large_batch(g, n, V, leaf_rows):
     """Stretches of 1024 and of 2048 rows, whole and not, one to three digits."""
