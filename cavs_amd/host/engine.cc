@@ -184,7 +184,8 @@ int Engine::group_limit() const {
 
 // Lists of the group launches for the batch whose index lists are given, and the tiles they run in.
 void Engine::build_group_plan(const int *t2j, const int *pair, const int *child, const int *kid_rows, int *block) {
-  build_group_lists(*sched_, nch_, t2j, pair, child, kid_rows, group_limit(), cavs_group_max_groups(cfg_.H), cavs_group_rows(), &group_, block);
+  build_group_lists(*sched_, nch_, t2j, pair, child, kid_rows, group_limit(), cavs_group_max_groups(cfg_.H), cavs_group_rows(),
+                    may_backward_ || cfg_.plan_cache > 0, &group_, block);
   if (group_.first >= 0 && group_.tile_rows == 4 && tail_limit() > 0) group_ = GroupLists();  // (the tail launches are tuned for that)
 }
 
@@ -652,10 +653,7 @@ void Engine::reserve_edges() {
   if (fused_rows() > 0 && ((cfg_.model == CAVS_MODEL_TREELSTM && (cavs_round_packed_ok(1, H) || cavs_round_packed_ok(65, H))) ||
                            (cfg_.model == CAVS_MODEL_LSTM && (cavs_lstm_round_packed_ok(1, H) || cavs_lstm_round_packed_ok(65, H)))))
     R(Upk_, (size_t)4 * H * H);
-  if (group_.first >= 0 && !cell_) {
-    R(Upk_, (size_t)(cfg_.model == CAVS_MODEL_TREEFC ? 2 : 4) * H * H);
-    if (ensure(UTp_, (size_t)(cfg_.model == CAVS_MODEL_TREEFC ? 2 : 4) * H * H)) utp_valid_ = false;
-  }
+  reserve_group();
   if (cfg_.model == CAVS_MODEL_TREELSTM) {
     R(hlr_, cap * H);
     R(dF_, cap * 2 * H);
@@ -672,6 +670,14 @@ void Engine::reserve_edges() {
     R(logits_, (size_t)sched_->B * H + 1);   // root rows / |h| scratch
     R(dlogits_, std::max<size_t>((size_t)sched_->B * H, cap * H));
   }
+}
+
+// the packed weights of the resident launches
+void Engine::reserve_group() {
+  if (group_.first < 0 || cell_) return;
+  const size_t n = (size_t)(cfg_.model == CAVS_MODEL_TREEFC ? 2 : 4) * cfg_.H * cfg_.H;
+  ensure(Upk_, n);
+  if (ensure(UTp_, n)) utp_valid_ = false;
 }
 
 // Whether x * W and its gradients go by words: every different id of the batch once (cavs_embed_index).
@@ -767,16 +773,16 @@ void Engine::upload_index_arena() {
   int *t2j = h.host.get(), *pair = t2j + N, *child = pair + N, *roots = child + (size_t)nch_ * N;
   std::string err = build_index_lists(s, nch_, cfg_.pairing, t2j, pair, child, roots);
   if (!err.empty()) fail(CAVS_EUNSUPPORTED, err);
-  forest_ = want_forest && build_forest_lists(s, nch_, fused_rows(), pair, child, roots + s.B, roots + s.B + (size_t)nch_ * N, &n_orphans_);
   tail_ = TailPlan();
-  int *tail_rows = roots + s.B + (size_t)N * (nch_ + 1);
   group_ = GroupLists();
-  if (group_lim > 0 && forest_) build_group_plan(t2j, pair, child, roots + s.B, h.host.get() + group_at);
-  if (want_tail && forest_ && group_.first < 0) build_tail_plan(roots + s.B, tail_rows);
+  forest_ = false;
+  group_at_ = group_at;
   d_group_ = h.dev.get() + group_at;
+  lists_later_ = !may_backward_ && cfg_.plan_cache == 0 && want_forest && (group_lim > 0 || want_tail) && N >= kListsLater;
+  if (!lists_later_ && want_forest) build_late_lists(h);
   plan_head_chunks(roots + s.B + (size_t)nch_ * N);
-  check(cavs_memcpy_h2d(h.dev.get(), h.host.get(), (group_.first >= 0 ? group_at + group_.ints : total) * sizeof(int),
-                        direct_ ? stream_ : sched_stream_));
+  const size_t ints = lists_later_ ? (size_t)N * (2 + nch_) + s.B : group_.first >= 0 ? group_at + group_.ints : total;
+  check(cavs_memcpy_h2d(h.dev.get(), h.host.get(), ints * sizeof(int), direct_ ? stream_ : sched_stream_));
   if (!direct_) {
     check(cavs_event_record(h.up_ev, sched_stream_));
     check(cavs_event_sync(h.up_ev));  // a few microseconds; the compute stream is still busy with the previous step
@@ -788,6 +794,40 @@ void Engine::upload_index_arena() {
   d_kid_rows_ = want_forest ? d_roots_ + s.B : nullptr;
   d_orphans_ = want_forest ? d_kid_rows_ + (size_t)nch_ * N : nullptr;
   d_tail_rows_ = want_tail ? d_orphans_ + N : nullptr;
+}
+
+// The lists behind those of the rounds: who wrote what a vertex reads, and the plans of the resident launches.
+void Engine::build_late_lists(HostLists &h) {
+  const Schedule &s = *sched_;
+  const int N = N_;
+  int *t2j = h.host.get(), *pair = t2j + N, *child = pair + N, *kids = child + (size_t)nch_ * N + s.B, *orphans = kids + (size_t)nch_ * N;
+  forest_ = build_forest_lists(s, nch_, fused_rows(), pair, child, kids, orphans, &n_orphans_);
+  if (!forest_) return;
+  if (group_limit() > 0) build_group_plan(t2j, pair, child, kids, h.host.get() + group_at_);
+  if (tail_limit() > 0 && group_.first < 0) build_tail_plan(kids, orphans + N);
+}
+
+// A forward pass over a large batch: the plans of the launches that run its last rounds are built, and go up, while the
+// first product runs (256 trees, H = 512, 9500 vertices: 40 us of host work under 85 us of x * W, 4016 -> 3701 us for 8 passes).  Few
+// vertices keep one upload: a second one costs 10 us.
+void Engine::finish_lists() {
+  if (!lists_later_) return;
+  lists_later_ = false;
+  HostLists &h = hlists_[hlists_slot_ ^ 1];
+  build_late_lists(h);
+  size_t at = 0, ints = 0;
+  if (group_.first >= 0) {
+    at = group_at_;
+    ints = group_.ints;
+  } else if (tail_.first >= 0) {
+    at = (size_t)N_ * (3 + 2 * nch_) + sched_->B;
+    ints = tail_.rows;
+  }
+  if (ints == 0) return;
+  check(cavs_memcpy_h2d(h.dev.get() + at, h.host.get() + at, ints * sizeof(int), sched_stream_));
+  check(cavs_event_record(h.up_ev, sched_stream_));
+  check(cavs_event_sync(h.up_ev));
+  reserve_group();
 }
 
 // ------------------------------------------------------------------ step
@@ -1073,7 +1113,7 @@ void Engine::begin_step(const int *graph, int B, int maxlen) {
   bias_jobs_.clear();
   head_chunks_.clear();  // (planned with the host scheduler's lists only)
   pending_tasks_.clear();  // (a step that failed half way may have left a job for a backward pass that never ran)
-  emb_cleared_ = false;
+  emb_cleared_ = lists_later_ = false;
   wait_ms_ = 0.f;
   uint64_t hash = 0;
   Plan *hit = nullptr;
@@ -1131,6 +1171,7 @@ void Engine::begin_step(const int *graph, int B, int maxlen) {
 void Engine::forward_only(const int *graph, int B, int maxlen, const float *x_dev, float *graph_out, bool trains) {
   state_epoch_++;
   trains_ = trains;
+  may_backward_ = true;  // (a call of its own)
   whole_step_ = false;
   begin_step(graph, B, maxlen);
   const bool reads_x = cell_ ? cell_->NX > 0 || cell_->XD > 0 : (cfg_.model != CAVS_MODEL_TREEFC || cfg_.use_x);
@@ -1327,7 +1368,7 @@ void Engine::step(const int *graph, int B, int maxlen, const void *x, const void
     std::chrono::steady_clock::time_point t0;
     ~StepTimer() { e->host_step_ms_ = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count(); }
   } step_timer{this, step_t0};
-  trains_ = backward;
+  trains_ = may_backward_ = backward;
   whole_step_ = false;
   begin_step(graph, B, maxlen);
   whole_step_ = backward && !cfg_.graph_replay && !profile_;
@@ -1504,10 +1545,6 @@ void Engine::treelstm_forward() {
   const int N = N_, H = cfg_.H, E = E_;
   const float *W = param("W").w, *U = param("U").w, *Bv = param("Bv").w;
   const int fused = fused_rows();
-  bool any_packed = false;
-  if (Upk_.capacity() > 0)
-    for (const Round &r : sched_->rounds) any_packed |= !leaf_round(r) && r.n <= fused && cavs_round_packed_ok(r.n, H);
-  if (any_packed || group_.first >= 0) ensure_packed();
   if (words_) {
     words_forward(W, 4 * H, 3 * H);
   } else {  // Pull of the word id, the lookup and x * W: one launch
@@ -1519,6 +1556,11 @@ void Engine::treelstm_forward() {
     c_gemm_flops_hinted_ += 2.0 * sched_->leaf_prefix * H * E;
     c_launches_ += 1;
   }
+  finish_lists();
+  bool any_packed = false;
+  if (Upk_.capacity() > 0)
+    for (const Round &r : sched_->rounds) any_packed |= !leaf_round(r) && r.n <= fused && cavs_round_packed_ok(r.n, H);
+  if (any_packed || group_.first >= 0) ensure_packed();
   if (!sched_->batching) {  // leaves are interleaved with internal vertices: their child rows must read as zero
     check(cavs_zero(G_.get(), (size_t)N * 2 * 2 * H * 4, stream_));
     check(cavs_zero(hlr_.get(), (size_t)N * H * 4, stream_));
@@ -1962,6 +2004,7 @@ void Engine::lstm_forward() {
     c_gemm_flops_ += 2.0 * N * 4 * H * E;
     c_launches_ += 1;
   }
+  finish_lists();
   if (!sched_->batching) check(cavs_zero(G_.get(), (size_t)N * 2 * H * 4, stream_));
   const int fused = fused_rows();
   bool any_packed = false;
@@ -2138,6 +2181,7 @@ void Engine::treefc_forward() {
   const float *Bv = cfg_.use_bias ? param("Bv").w : nullptr;
   if (cfg_.use_x) gather(xs_.get(), H, d_x_, uH_, d_t2j_, N, uH_);
   if (!sched_->batching) check(cavs_zero(G_.get(), (size_t)N * 2 * H * 4, stream_));
+  finish_lists();
   const int fused = fused_rows();
   out_folded_ = fused > 0 && sched_->max_round <= fused && fwd_out_ != nullptr;
   float *go = out_folded_ ? fwd_out_ : nullptr;
@@ -2354,6 +2398,7 @@ void Engine::cell_forward() {
     c_gemm_flops_ += 2.0 * N * c0.NX * H * E_;
     c_launches_ += 1;
   }
+  finish_lists();
   out_folded_ = true;  // the rounds write the pushed value by vertex id themselves
   for (size_t ci = 0; ci < cells_.size(); ci++) {
     // the weights may have changed since the last step (the caller's optimizer writes them): both

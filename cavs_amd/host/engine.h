@@ -235,6 +235,7 @@ class Engine {
     void *up_ev = nullptr;
     uint64_t used = 0;  // the step that reads them (0: none)
   } hlists_[2];
+  void build_late_lists(HostLists &h);
   int hlists_slot_ = 0;
   const int *d_t2j_ = nullptr, *d_pair_ = nullptr, *d_child_ = nullptr, *d_roots_ = nullptr;
   // Tree-LSTM, message flow of the batch is a forest: children by slab row, and the slab rows
@@ -403,6 +404,12 @@ class Engine {
   DeviceArray<float> word_ids_, word_scratch_;
   bool words_ = false;
   bool trains_ = true;  // a backward pass follows
+  bool may_backward_ = true;  // a backward pass over this batch may come
+  bool lists_later_ = false;  // build_late_lists has yet to run
+  static constexpr int kListsLater = 4096;
+  size_t group_at_ = 0;
+  void finish_lists();
+  void reserve_group();
   bool whole_step_ = false;  // ... and the update, in the same call: nobody looks in between
   bool utp_valid_ = false;   // UTp_ is the weights'
   void clear_embedding(std::vector<cavs_task> *tasks);

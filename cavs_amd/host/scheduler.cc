@@ -430,7 +430,7 @@ static int group_tile_rows(const std::vector<int> &per, int rounds, int slice) {
 }
 
 void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pair, const int *child, const int *kid_rows, int lim, int groups,
-                       int slice, GroupLists *out, int *block) {
+                       int slice, bool back, GroupLists *out, int *block) {
   *out = GroupLists();
   const int R = (int)s.rounds.size(), N = s.N;
   auto leaf_round = [](const Round &r) { return r.gather_begin[0] == r.gather_end[0] && r.gather_begin[1] == r.gather_end[1]; };
@@ -478,7 +478,7 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
     // The rows whose message nobody reads open the backward pass: with the group whose tree they are in, those of earlier
     // rounds with any.
     std::vector<int> roots, root_at((size_t)G + 1, 0);
-    for (int b = 0, any = 0; b < N; b++) {
+    for (int b = 0, any = 0; back && b < N; b++) {
       if (pair[b] >= 0) continue;
       const int g = b >= lo ? cell[b - lo] / nr : any++ % G;
       roots.push_back(b);
@@ -495,8 +495,9 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
       const int *c = child + (size_t)nch * b, *q = kid_rows + (size_t)nch * b;
       const int c1 = nch == 2 ? c[1] : -1, q1 = nch == 2 ? q[1] : -1;
       const int fr[8] = {b, c[0], c1, pair[b], t2j[b], 0, 0, 0};
-      const int br[8] = {b, q[0], q1, q[0] >= 0 ? t2j[q[0]] : -1, q1 >= 0 ? t2j[q1] : -1, 0, 0, 0};
       std::memcpy(f, fr, sizeof fr);
+      if (!back) continue;
+      const int br[8] = {b, q[0], q1, q[0] >= 0 ? t2j[q[0]] : -1, q1 >= 0 ? t2j[q1] : -1, 0, 0, 0};
       std::memcpy(w, br, sizeof br);
     }
     cur.assign(root_at.begin(), root_at.end());
@@ -504,25 +505,25 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
       const int b = roots[i], r[8] = {b, b, -1, t2j[b], -1, 0, 0, 0};
       std::memcpy(block + t.bwd.recs + 8 * (t.rows + cur[roots[i + 1]]++), r, sizeof r);
     }
-    size_t end = (2 * t.rows + roots.size() / 2) * 8;
+    size_t end = ((back ? 2 : 1) * t.rows + roots.size() / 2) * 8;
     // A direction: a group's share of a round as lists of at most `slice` rows; the first waits for the
     // rounds the group has done so far, the last is an arrival.
-    for (int back = 0; back < 2; back++) {
-      GroupLists::Launch &l = back ? t.bwd : t.fwd;
+    for (int dir = 0; dir < (back ? 2 : 1); dir++) {
+      GroupLists::Launch &l = dir ? t.bwd : t.fwd;
       l.groups = end;
       l.lists = end + (size_t)G * 4;
       int *lists = block + l.lists, nl = 0;
       for (int g = 0; g < G; g++) {
         int *gd = block + l.groups + 4 * (size_t)g, done = 0;
         gd[0] = nl;
-        const int alone = back ? root_at[g + 1] - root_at[g] : 0;
+        const int alone = dir ? root_at[g + 1] - root_at[g] : 0;
         for (int c0 = 0; c0 < alone; c0 += slice, nl++) {
           const int row[4] = {(int)t.rows + root_at[g] + c0, std::min(slice, alone - c0), 0, (c0 + slice >= alone) | 2};
           std::copy(row, row + 4, lists + 4 * (size_t)nl);
         }
         done += alone > 0;
         for (int i = 0; i < nr; i++) {
-          const int k = back ? nr - 1 - i : i, c = per[(size_t)g * nr + k];
+          const int k = dir ? nr - 1 - i : i, c = per[(size_t)g * nr + k];
           for (int c0 = 0; c0 < c; c0 += slice, nl++) {
             const int row[4] = {at[(size_t)g * nr + k] + c0, std::min(slice, c - c0), c0 == 0 ? done : 0, c0 + slice >= c};
             std::copy(row, row + 4, lists + 4 * (size_t)nl);
