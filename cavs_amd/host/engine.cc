@@ -184,8 +184,10 @@ int Engine::group_limit() const {
 
 // Lists of the group launches for the batch whose index lists are given, and the tiles they run in.
 void Engine::build_group_plan(const int *t2j, const int *pair, const int *child, const int *kid_rows, int *block) {
+  // (no list of more than eight rows, no tile of sixteen: the tail launches)
+  if (tail_limit() > 0 && std::all_of(sched_->rounds.begin(), sched_->rounds.end(), [&](const Round &r) { return r.n <= 8 || leaf_round(r); })) return;
   build_group_lists(*sched_, nch_, t2j, pair, child, kid_rows, group_limit(), cavs_group_max_groups(cfg_.H), cavs_group_rows(),
-                    may_backward_ || cfg_.plan_cache > 0, &group_, block);
+                    !lists_forward_only(), &group_, block);
   if (group_.first >= 0 && group_.tile_rows == 4 && tail_limit() > 0) group_ = GroupLists();  // (the tail launches are tuned for that)
 }
 
@@ -778,7 +780,7 @@ void Engine::upload_index_arena() {
   forest_ = false;
   group_at_ = group_at;
   d_group_ = h.dev.get() + group_at;
-  lists_later_ = !may_backward_ && cfg_.plan_cache == 0 && want_forest && (group_lim > 0 || want_tail) && N >= kListsLater;
+  lists_later_ = lists_forward_only() && want_forest && (group_lim > 0 || want_tail) && N >= kListsLater;
   if (!lists_later_ && want_forest) build_late_lists(h);
   plan_head_chunks(roots + s.B + (size_t)nch_ * N);
   const size_t ints = lists_later_ ? (size_t)N * (2 + nch_) + s.B : group_.first >= 0 ? group_at + group_.ints : total;
@@ -801,8 +803,10 @@ void Engine::build_late_lists(HostLists &h) {
   const Schedule &s = *sched_;
   const int N = N_;
   int *t2j = h.host.get(), *pair = t2j + N, *child = pair + N, *kids = child + (size_t)nch_ * N + s.B, *orphans = kids + (size_t)nch_ * N;
-  forest_ = build_forest_lists(s, nch_, fused_rows(), pair, child, kids, orphans, &n_orphans_);
-  if (!forest_) return;
+  // (the resident launches of a forward pass read the lists whatever runs the larger rounds)
+  const bool forest = build_forest_lists(s, nch_, lists_forward_only() ? N : fused_rows(), pair, child, kids, orphans, &n_orphans_);
+  forest_ = forest && !lists_forward_only();
+  if (!forest) return;
   if (group_limit() > 0) build_group_plan(t2j, pair, child, kids, h.host.get() + group_at_);
   if (tail_limit() > 0 && group_.first < 0) build_tail_plan(kids, orphans + N);
 }

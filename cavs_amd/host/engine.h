@@ -408,6 +408,7 @@ class Engine {
   bool lists_later_ = false;  // build_late_lists has yet to run
   static constexpr int kListsLater = 4096;
   size_t group_at_ = 0;
+  bool lists_forward_only() const { return !may_backward_ && cfg_.plan_cache == 0; }
   void finish_lists();
   void reserve_group();
   bool whole_step_ = false;  // ... and the update, in the same call: nobody looks in between

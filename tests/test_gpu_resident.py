@@ -128,3 +128,27 @@ print("done")
     r = subprocess.run([sys.executable, "-c", code, os.path.dirname(here), here, os.path.join(os.path.dirname(here), "oracle")], capture_output=True,
                        text=True, timeout=100)
     assert r.returncode == 0 and r.stdout.endswith("done\n"), r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("model,H,B", [("treelstm", 64, 40), ("treelstm", 64, 600), ("treelstm", 512, 600), ("lstm", 96, 1000), ("treefc", 64, 600)])
+def test_a_forward_pass_plans_for_itself(model, H, B):
+    """Without a backward pass only forward lists are made, in a large batch (4096 vertices) under the first product, and larger rounds by
+    products leave the resident launch the others: what a launch per round gives (other orders of the same sums).  The backward pass
+    that follows on the same batch has lists of its own."""
+    w = small_workload(model, 77, B=B, H=H, E=12, V=31, C=5)
+    assert (w["N"] >= 4096) == (B > 40)
+    ref, s = (_session(model, H, w, tail_rows=k) for k in (-1, 0))
+    few = _session(model, H, w, fused_round_rows=300)  # (rounds of more rows: products)
+    for x in (ref, s, few):
+        x.step(w["graph"], w["x"], w["labels"], backward=False)
+    assert ref.counter("tail_rounds") == 0 and s.counter("tail_rounds") > 0 and few.counter("tail_rounds") > 0
+    for x in (s, few):
+        close(x.fetch("graph_out"), ref.fetch("graph_out"), "graph_out")
+        close(x.fetch("loss"), ref.fetch("loss"), "loss")
+    for x in (ref, s):
+        x.step(w["graph"], w["x"], w["labels"], backward=True, lr=1e-3)
+    got, want = s.grads(), ref.grads()
+    for k, v in want.items():
+        close(got[k], v, k)
+    for x in (ref, s, few):
+        x.close()
