@@ -362,6 +362,17 @@ bool Engine::update_jobs(float *w, float *g, float lr, std::vector<cavs_task> *o
     wfct_valid_ = true;
     return true;
   }
+  // the table by the rows that were looked up: its gradient is zero in all others
+  const auto emb = params_.find("Emb");
+  if (emb != params_.end() && w == emb->second->w && g == emb->second->g && g == emb->second->own_g.get() && emb_sparse_valid_ && emb_dirty_n_ == N_ &&
+      !cfg_.graph_replay) {
+    if (emb_stamp_.capacity() < (size_t)cfg_.V) {
+      emb_stamp_.reserve(cfg_.V);
+      check(cavs_zero(emb_stamp_.get(), (size_t)cfg_.V * 4, stream_));
+    }
+    out->push_back({CAVS_TASK_EMBED_SGD, lr, N_, (long long)(emb->second->n / cfg_.V), ++emb_epoch_, w, g, xs_prev_.get(), emb_stamp_.get()});
+    return true;
+  }
   if (Upk_.capacity() == 0) return false;
   const long long H = cfg_.H;
   // the transposed copy as well, where the resident backward launch reads one (a recorded step makes it each time)
@@ -596,7 +607,7 @@ void Engine::reserve_edges() {
       // by row of the round and child (two launches)
       R(st.ds, std::max(cap * k.SI * H, rc * k.K * k.SI * H));
       R(st.bt, (size_t)2 * k.blocks() * H * H);  // the weight blocks tile-major, as they are and transposed
-      R(st.colsum, (size_t)k.ND * H);
+      R(st.colsum, cavs_colsum_blocks_workspace((int)cap, k.ND * (int)H, 1) / 4);
       if (ci + 1 < cells_.size()) {
         R(st.rows, cap * k.S * H);
         R(st.drows, cap * k.S * H);
@@ -2586,25 +2597,34 @@ void Engine::cell_backward() {
   }
   // (overlapping but different blocks of one weight would need more than "the same first element")
   constexpr size_t kGroup = 8;  // products per cavs_sgemm_group launch
+  // the chunk sums of the gradient rows' columns come along with the products, a cell's with a launch
+  std::vector<cavs_colsum_desc> sums;
+  for (CellStage &st : cells_)
+    if (!st.spec->biases.empty()) sums.push_back({st.colsum.get(), st.d.get(), st.spec->ND * H, N, st.spec->ND * H});
+  size_t riders = 0;
+  auto rider = [&]() -> const cavs_colsum_desc * { return riders < sums.size() ? &sums[riders++] : nullptr; };
   bool embedded = false;
   for (size_t wv = 0; wv < waves.size(); wv++) {
     const std::vector<cavs_gemm_desc> &w = waves[wv];
     size_t at = 0;
     if (wv == 0 && c0.NX > 0 && L == 1 && !w.empty()) {  // d e is complete after this launch
       const size_t take = std::min(w.size(), kGroup);
-      gemm_group_embedding_backward(std::vector<cavs_gemm_desc>(w.begin(), w.begin() + take), E_);
+      gemm_group_embedding_backward(std::vector<cavs_gemm_desc>(w.begin(), w.begin() + take), E_, rider());
       at = take;
       embedded = true;
     }
-    for (; at < w.size(); at += kGroup) gemm_group(std::vector<cavs_gemm_desc>(w.begin() + at, w.begin() + std::min(w.size(), at + kGroup)));
+    for (; at < w.size(); at += kGroup) gemm_group(std::vector<cavs_gemm_desc>(w.begin() + at, w.begin() + std::min(w.size(), at + kGroup)), rider());
   }
   if (c0.NX > 0 && !embedded) embedding_backward_rows();
+  while (const cavs_colsum_desc *s = rider()) {
+    check(cavs_colsum_blocks(nullptr, s->inp, s->ld, s->n, s->w, 1, nullptr, s->parts, cavs_colsum_blocks_workspace(s->n, s->w, 1), stream_));
+    c_launches_ += 1;
+  }
   for (size_t ci = 0; ci < cells_.size(); ci++) {
     const CellStage &st = cells_[ci];
     if (st.spec->biases.empty()) continue;
-    colsum_fixed(st.colsum.get(), st.d.get(), N, st.spec->ND * H);
     ProfScope ps(this, K_OTHER);
-    cell_launch((int)ci, CK_BIAS, (H + 255) / 256, 1, 1, 256, 0, 0, nullptr, d_dgo_);
+    cell_launch((int)ci, CK_BIAS, (H + 63) / 64, 1, 1, 256, 0, cavs_colsum_parts(N), nullptr, d_dgo_);
   }
 }
 

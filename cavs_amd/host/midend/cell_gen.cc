@@ -655,9 +655,19 @@ struct Writer {
       }
     }
     o << "  }\n}\n";
-    // the bias gradients out of the column sums of the gradient rows
-    o << "extern \"C\" __global__ void cell_bias(CellArgs a) {\n  const int j = blockIdx.x * 256 + threadIdx.x;\n  if (j >= CELL_H) return;\n";
-    for (const CellBias &b : s.biases) o << "  " << param_ptr(b.ref, true) << "[j] " << (b.add ? "+=" : "=") << " a.colsum[" << (long)b.dcol * H << " + j];\n";
+    // the bias gradients out of the chunk sums of the gradient rows' columns (a.n of them, a quarter to a wavefront)
+    const size_t nb = std::max<size_t>(1, s.biases.size());
+    o << "extern \"C\" __global__ __launch_bounds__(256) void cell_bias(CellArgs a) {\n  __shared__ float s[" << nb << "][4][64];\n"
+         "  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6, j = blockIdx.x * 64 + lane;\n";
+    for (size_t b = 0; b < s.biases.size(); b++)
+      o << "  {\n    float t = 0.f;\n    if (j < CELL_H)\n      for (int c = q; c < (int)a.n; c += 32) {\n        float v[8];\n#pragma unroll\n"
+           "        for (int u = 0; u < 8; u++) v[u] = a.colsum[(long)(c + 4 * u < (int)a.n ? c + 4 * u : q) * (CELL_ND * CELL_H) + "
+        << (long)s.biases[b].dcol * H << " + j];\n#pragma unroll\n        for (int u = 0; u < 8; u++)\n          if (c + 4 * u < (int)a.n) t += v[u];\n      }\n    s[" << b
+        << "][q][lane] = t;\n  }\n";
+    o << "  __syncthreads();\n  if (q != 0 || j >= CELL_H) return;\n";
+    for (size_t b = 0; b < s.biases.size(); b++)
+      o << "  " << param_ptr(s.biases[b].ref, true) << "[j] " << (s.biases[b].add ? "+=" : "=") << " (s[" << b << "][0][lane] + s[" << b << "][1][lane]) + (s["
+        << b << "][2][lane] + s[" << b << "][3][lane]);\n";
     o << "}\n";
   }
 };
