@@ -642,6 +642,7 @@ void Engine::reserve_edges() {
     R(dxW_, cap * H);
     R(r_z_, rc * H);
   }
+  group_counters();  // (not first within a recording, where the zeros would come with each replay only)
   words_ = words_wanted();
   if (words_) {
     const size_t w = cell_ ? (size_t)cell_->NX * H : 4 * H;
