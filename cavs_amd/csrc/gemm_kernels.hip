@@ -708,6 +708,11 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
     if (s < 1) s = 1;
     int kchunk = K > 0 ? (int)(((K + s - 1) / s + 31) / 32 * 32) : 1;
     int splits = K > 0 ? (K + kchunk - 1) / kchunk : 1;
+    if (grouped == 1) {  // as it would be cut by itself
+      const GemmPlan alone_plan = plan_product(q);
+      kchunk = alone_plan.kchunk;
+      splits = alone_plan.splits;
+    }
     GemmArgs g{q.M, q.N, q.K, q.A, q.lda, q.B, q.ldb, q.C, q.ldc, q.alpha, q.beta, nullptr, 0, 0, kchunk, nullptr};
     g.live = q.live;
     g.pad_block = q.pad_block;

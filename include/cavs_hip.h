@@ -240,7 +240,7 @@ int cavs_sgemm_group_embed_bwd(int count, const cavs_gemm_desc *products, int em
  * products' own launch: the workgroup that is last at a tile does it.  counters: n_counters ints of device memory
  * that are zero before the first call and zero again behind each; one set serves the calls on one stream.  Lists with more
  * split tiles than counters, and products that run alone, take the launches of the entry points above.  Same results
- * bit for bit, but for the order of the scatter's atomic adds and where a list of one product is cut.
+ * bit for bit, but for the order of the scatter's atomic adds.
  * sums (may be null): the chunk sums that cavs_colsum_blocks(out = null) leaves of `inp` [n, w], in the same launch. */
 typedef struct {
   float *parts;  /* cavs_colsum_parts(n) rows of w */

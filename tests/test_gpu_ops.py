@@ -482,7 +482,7 @@ def test_sgemm_group_with_the_embedding_gradient_behind_one_product(g, name, k):
 
 
 @pytest.mark.parametrize("room", [1024, 0])
-@pytest.mark.parametrize("name,k", [("treelstm_step", 0), ("treelstm_step", -1), ("ragged", 0), ("mixed", 1), ("mixed", 0), ("mixed", -1)])
+@pytest.mark.parametrize("name,k", [("treelstm_step", 0), ("treelstm_step", -1), ("ragged", 0), ("single", -1), ("single", 0), ("mixed", 1), ("mixed", 0), ("mixed", -1)])
 def test_a_group_that_adds_up_its_own_splits(g, name, k, room):
     """cavs_sgemm_group_once: column sums ride along; the last workgroup at a tile reduces it, in the order of the launch behind cavs_sgemm_group (the same
     bits), and scatters the product that feeds the table; the counters are zero again, so the next call finds them so.  With
