@@ -176,6 +176,45 @@ int cavs_schedule_tail_lists(const int *graph, int B, int maxlen, int pairing, i
   return (int)t.rows;
 }
 
+int cavs_schedule_group_lists(const int *graph, int B, int maxlen, int nchild, int pairing, int rows_limit, int groups, int slice, int forward_only,
+                              int only_wide, int *meta, int *block, int cap) {
+  if (!graph || B <= 0 || maxlen <= 0 || nchild < 1 || nchild > 2 || pairing < 0 || pairing > 1 || rows_limit < 1 || groups < 1 || groups > 128 ||
+      slice < 1 || !meta || cap < 0 || (cap > 0 && !block)) {
+    g_error = "bad arguments";
+    return -1;
+  }
+  cavs::Schedule sch;
+  std::string err = cavs::build_schedule(graph, B, maxlen, true, &sch);
+  if (err.empty() && sch.executed != sch.N) err = "the batch holds a single-vertex sample";
+  const size_t N = err.empty() ? (size_t)sch.N : 0, nk = N * (size_t)nchild;
+  std::vector<int> t2j(N), pair(N), child(nk), roots((size_t)B), kid(nk), orphans(N);
+  if (err.empty()) err = cavs::build_index_lists(sch, nchild, pairing, t2j.data(), pair.data(), child.data(), roots.data());
+  if (!err.empty()) {
+    g_error = err;
+    return -1;
+  }
+  std::fill(meta, meta + 11, 0);
+  meta[0] = -1;
+  int n_orphans = 0;
+  if (!cavs::build_forest_lists(sch, nchild, 1 << 30, pair.data(), child.data(), kid.data(), orphans.data(), &n_orphans)) return 0;
+  const int mark = 0x5a5a5a5a;  // (no value a list holds)
+  std::vector<int> room(cavs::group_lists_bound(sch, N - sch.scatter_ids.size(), groups), mark);
+  cavs::GroupLists t;
+  cavs::build_group_lists(sch, nchild, t2j.data(), pair.data(), child.data(), kid.data(), forward_only ? nullptr : orphans.data(), n_orphans, rows_limit,
+                          groups, slice, only_wide != 0, &t, room.data());
+  const int out[10] = {t.first, t.ngroups, t.tile_rows, (int)t.fwd.groups, (int)t.fwd.lists, (int)t.fwd.recs,
+                       (int)t.bwd.groups, (int)t.bwd.lists, (int)t.bwd.recs, (int)room.size()};
+  std::copy(out, out + 10, meta);
+  meta[10] = (int)(room.size() - (size_t)std::count(room.begin(), room.end(), mark));
+  if (t.first < 0) return 0;
+  if ((size_t)cap < t.ints) {
+    g_error = "the block takes " + std::to_string(t.ints) + " ints";
+    return -1;
+  }
+  std::copy(room.begin(), room.begin() + t.ints, block);
+  return (int)t.ints;
+}
+
 int cavs_schedule_trace_from_lists(int B, int maxlen, int N, int nchild, const int *round2offset, int R, const int *t2j,
                                    const int *pair, const int *child, const int *roots, int with_backward, int *out, int cap) {
   if (B <= 0 || N <= 0 || R < 0 || !round2offset || !t2j || !pair || !child || !roots) {

@@ -183,12 +183,12 @@ int Engine::group_limit() const {
 }
 
 // Lists of the group launches for the batch whose index lists are given, and the tiles they run in.
-void Engine::build_group_plan(const int *t2j, const int *pair, const int *child, const int *kid_rows, int *block) {
+void Engine::build_group_plan(const int *t2j, const int *pair, const int *child, const int *kid_rows, const int *orphans, int *block) {
   // (no list of more than eight rows, no tile of sixteen: the tail launches)
   if (tail_limit() > 0 && std::all_of(sched_->rounds.begin(), sched_->rounds.end(), [&](const Round &r) { return r.n <= 8 || leaf_round(r); })) return;
-  build_group_lists(*sched_, nch_, t2j, pair, child, kid_rows, group_limit(), cavs_group_max_groups(cfg_.H), cavs_group_rows(),
-                    !lists_forward_only(), &group_, block);
-  if (group_.first >= 0 && group_.tile_rows == 4 && tail_limit() > 0) group_ = GroupLists();  // (the tail launches are tuned for that)
+  // (nor where tiles of four are the better ones: the tail launches are tuned for those)
+  build_group_lists(*sched_, nch_, t2j, pair, child, kid_rows, lists_forward_only() ? nullptr : orphans, n_orphans_, group_limit(),
+                    cavs_group_max_groups(cfg_.H), cavs_group_rows(), tail_limit() > 0, &group_, block);
 }
 
 cavs_group_plan Engine::group_plan(const GroupLists::Launch &l) const {
@@ -766,7 +766,7 @@ void Engine::upload_index_arena() {
   const size_t total = (size_t)N * (2 + nch_) + s.B + (want_forest ? (size_t)N * (nch_ + 1) : 0) + (want_tail ? (size_t)N : 0);
   const int group_lim = want_forest ? group_limit() : 0, ngroups = group_lim > 0 ? cavs_group_max_groups(cfg_.H) : 0;
   const size_t group_at = (total + 3) / 4 * 4;  // (16-byte aligned on the device)
-  const size_t room = group_lim > 0 ? group_at + group_lists_bound(N, ngroups) : total;
+  const size_t room = group_lim > 0 ? group_at + group_lists_bound(s, (size_t)N - s.scatter_ids.size(), ngroups) : total;
   // Two sets of buffers (pinned staging + device lists) alternate, and the copy runs on a stream
   // of its own: the lists of step k + 1 are built and uploaded while the kernels of step k run,
   // instead of the copy sitting in the compute stream between two steps.  A set is rewritten only
@@ -819,7 +819,7 @@ void Engine::build_late_lists(HostLists &h) {
   const bool forest = build_forest_lists(s, nch_, lists_forward_only() ? N : fused_rows(), pair, child, kids, orphans, &n_orphans_);
   forest_ = forest && !lists_forward_only();
   if (!forest) return;
-  if (group_limit() > 0) build_group_plan(t2j, pair, child, kids, h.host.get() + group_at_);
+  if (group_limit() > 0) build_group_plan(t2j, pair, child, kids, orphans, h.host.get() + group_at_);
   if (tail_limit() > 0 && group_.first < 0) build_tail_plan(kids, orphans + N);
 }
 
@@ -1037,14 +1037,14 @@ void Engine::schedule_on_device(const int *graph, int B, int maxlen) {
   group_ = GroupLists();
   // The group launches' block is host work on all of the lists: they come back, the block goes up.
   if (forest_ && group_limit() > 0 && N > 0) {
-    const size_t all = BM * (2 + 2 * (size_t)nch_);
+    const size_t all = need;
     const int ngroups = cavs_group_max_groups(cfg_.H);
     d.kid_host.reserve(all);
-    d.tail_host.reserve(group_lists_bound(N, ngroups));
+    d.tail_host.reserve(group_lists_bound(s, B, ngroups));
     check(cavs_memcpy_d2h(d.kid_host.get(), t2j, all * sizeof(int), sched_stream_));
     check(cavs_stream_sync(sched_stream_));
     const int *h = d.kid_host.get();
-    build_group_plan(h, h + BM, h + 2 * BM, h + (2 + nch_) * BM, d.tail_host.get());
+    build_group_plan(h, h + BM, h + 2 * BM, h + (2 + nch_) * BM, h + (2 + 2 * nch_) * BM + B, d.tail_host.get());
     if (group_.first >= 0) {
       d.tail_dev.reserve(grow(group_.ints, d.tail_dev.capacity()));
       check(cavs_memcpy_h2d(d.tail_dev.get(), d.tail_host.get(), group_.ints * sizeof(int), sched_stream_));

@@ -466,7 +466,7 @@ class Engine {
   // fills tail_ and writes the groups' row lists to `rows_out` (room for N ints) from the host copy of
   // the children-by-slab-row lists of a batch whose message flow is a forest
   void build_tail_plan(const int *kid_rows, int *rows_out);
-  void build_group_plan(const int *t2j, const int *pair, const int *child, const int *kid_rows, int *block);
+  void build_group_plan(const int *t2j, const int *pair, const int *child, const int *kid_rows, const int *orphans, int *block);
  public:
   // After the stream has drained: gives the claim back and reads the status word of the tail launches.  A launch that gave
   // up leaves the results of the steps since undefined (their parameter updates were skipped: they

@@ -403,9 +403,11 @@ void build_tail_lists(const Schedule &s, const int *kid_rows, int lim, int group
   }
 }
 
-size_t group_lists_bound(size_t N, int groups) {
-  // records forward, backward and of the rows nobody sends a gradient to, lists of at least a row each, two tables of groups
-  return N * (24 + 12) + 2 * (size_t)groups * 4;
+size_t group_lists_bound(const Schedule &s, size_t alone, int groups) {
+  // records of the rows above the leaves forward and backward, and of the rows nobody sends a gradient to; lists of at least a
+  // row each; two tables of groups
+  const size_t inner = (size_t)(s.N - s.leaf_prefix);
+  return inner * (16 + 8) + alone * (8 + 4) + 2 * (size_t)groups * 4;
 }
 
 // What the group with the most work spends on tiles when its lists run in tiles of four rows, and when they run in
@@ -429,13 +431,14 @@ static int group_tile_rows(const std::vector<int> &per, int rounds, int slice) {
   return wide < four ? 16 : 4;
 }
 
-void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pair, const int *child, const int *kid_rows, int lim, int groups,
-                       int slice, bool back, GroupLists *out, int *block) {
+void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pair, const int *child, const int *kid_rows, const int *orphans,
+                       int n_orphans, int lim, int groups, int slice, bool only_wide, GroupLists *out, int *block) {
+  const bool back = orphans != nullptr;
   *out = GroupLists();
   const int R = (int)s.rounds.size(), N = s.N;
   auto leaf_round = [](const Round &r) { return r.gather_begin[0] == r.gather_end[0] && r.gather_begin[1] == r.gather_end[1]; };
   if (lim <= 0 || groups < 1 || slice < 1 || !s.batching || R < 3) return;
-  int k0 = R;  // the rounds with children that no larger one follows
+  int k0 = R;  // the rounds with children that no larger one follows (never that of the leaves: group_lists_bound)
   while (k0 > 1 && !leaf_round(s.rounds[k0 - 1]) && s.rounds[k0 - 1].n <= (long)groups * lim) k0--;
   std::vector<int> comp, weight, order, group, per, cell;
   for (; R - k0 >= 2; k0++) {
@@ -464,10 +467,13 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
       }
     if (!ok) continue;
 
+    const int tile_rows = group_tile_rows(per, nr, slice);
+    if (only_wide && tile_rows == 4) return;
     GroupLists &t = *out;
     t.first = k0;
     t.ngroups = G;
     t.rows = (size_t)(N - lo);
+    t.tile_rows = tile_rows;
     // the records, group by group, round by round
     std::vector<int> at((size_t)G * nr), cur;
     int fill = 0;
@@ -477,35 +483,36 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
     }
     // The rows whose message nobody reads open the backward pass: with the group whose tree they are in, those of earlier
     // rounds with any.
-    std::vector<int> roots, root_at((size_t)G + 1, 0);
-    for (int b = 0, any = 0; back && b < N; b++) {
-      if (pair[b] >= 0) continue;
-      const int g = b >= lo ? cell[b - lo] / nr : any++ % G;
-      roots.push_back(b);
-      roots.push_back(g);
-      root_at[g + 1]++;
+    std::vector<int> root_group(back ? n_orphans : 0), root_at((size_t)G + 1, 0);
+    for (int i = 0, any = 0; i < (int)root_group.size(); i++) {
+      const int b = orphans[i];
+      root_group[i] = b >= lo ? group[comp[b]] : any++ % G;
+      root_at[root_group[i] + 1]++;
     }
     for (int g = 0; g < G; g++) root_at[g + 1] += root_at[g];
     t.fwd.recs = 0;
     t.bwd.recs = t.rows * 8;
+    // (word by word in place: as arrays that are copied, a record is stored in fours and loaded in sixteens, which the core
+    // cannot forward -- 43 of 67 us for 4200 vertices)
+    auto put = [](int *r, int a, int b, int c, int d, int e) {
+      r[0] = a, r[1] = b, r[2] = c, r[3] = d, r[4] = e, r[5] = r[6] = r[7] = 0;
+    };
     cur = at;
+    int *const fwd = block + t.fwd.recs, *const bwd = block + t.bwd.recs;
     for (int b = lo; b < N; b++) {
-      const int i = cur[cell[b - lo]]++;
-      int *f = block + t.fwd.recs + 8 * (size_t)i, *w = block + t.bwd.recs + 8 * (size_t)i;
+      const size_t i = cur[cell[b - lo]]++;
       const int *c = child + (size_t)nch * b, *q = kid_rows + (size_t)nch * b;
-      const int c1 = nch == 2 ? c[1] : -1, q1 = nch == 2 ? q[1] : -1;
-      const int fr[8] = {b, c[0], c1, pair[b], t2j[b], 0, 0, 0};
-      std::memcpy(f, fr, sizeof fr);
+      put(fwd + 8 * i, b, c[0], nch == 2 ? c[1] : -1, pair[b], t2j[b]);
       if (!back) continue;
-      const int br[8] = {b, q[0], q1, q[0] >= 0 ? t2j[q[0]] : -1, q1 >= 0 ? t2j[q1] : -1, 0, 0, 0};
-      std::memcpy(w, br, sizeof br);
+      const int q0 = q[0], q1 = nch == 2 ? q[1] : -1;
+      put(bwd + 8 * i, b, q0, q1, q0 >= 0 ? t2j[q0] : -1, q1 >= 0 ? t2j[q1] : -1);
     }
     cur.assign(root_at.begin(), root_at.end());
-    for (size_t i = 0; i < roots.size(); i += 2) {
-      const int b = roots[i], r[8] = {b, b, -1, t2j[b], -1, 0, 0, 0};
-      std::memcpy(block + t.bwd.recs + 8 * (t.rows + cur[roots[i + 1]]++), r, sizeof r);
+    for (size_t i = 0; i < root_group.size(); i++) {
+      const int b = orphans[i];
+      put(bwd + 8 * (t.rows + cur[root_group[i]]++), b, b, -1, t2j[b], -1);
     }
-    size_t end = ((back ? 2 : 1) * t.rows + roots.size() / 2) * 8;
+    size_t end = ((back ? 2 : 1) * t.rows + root_group.size()) * 8;
     // A direction: a group's share of a round as lists of at most `slice` rows; the first waits for the
     // rounds the group has done so far, the last is an arrival.
     for (int dir = 0; dir < (back ? 2 : 1); dir++) {
@@ -537,7 +544,6 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
       end = l.lists + 4 * (size_t)nl;
     }
     t.ints = end;
-    t.tile_rows = group_tile_rows(per, nr, slice);
     return;
   }
 }

@@ -54,6 +54,7 @@ def lib():
             "cavs_schedule_trace": [P, I, I, I, I, P, I],
             "cavs_schedule_index_lists": [P, I, I, I, I, I, P, P, P, P, P, P, P],
             "cavs_schedule_tail_lists": [P, I, I, I, I, I, I, I, P, P, P, P, P, P, P, P, P],
+            "cavs_schedule_group_lists": [P, I, I, I, I, I, I, I, I, I, P, P, I],
             "cavs_schedule_trace_from_lists": [I, I, I, I, P, I, P, P, P, P, I, P, I],
             "cavs_session_timing": [P, C.c_char_p, C.POINTER(F)],
             "cavs_session_counter": [P, C.c_char_p, C.POINTER(C.c_double)],
@@ -153,6 +154,26 @@ def tail_lists(graph, pairing="reference", fused_limit=1 << 30, rows_limit=32, g
     names = ("start", "count", "flags", "bstart", "bcount", "bflags")
     out = dict(first=int(meta[0]), M=M, lists_max=int(meta[2]), tiles_max=int(meta[3]), nrounds=nrounds, rows=rows[:n])
     out.update({k: a[: groups * M].reshape(groups, M) for k, a in zip(names, arr)})
+    return out
+
+
+def group_lists(graph, nchild, pairing="reference", rows_limit=64, groups=64, slice_rows=32, forward_only=False, only_wide=False):
+    """Host-only: the lists of the launches that keep many rounds resident.  dict(first, ngroups, tile_rows, room, written,
+    fwd, bwd); fwd and bwd (None where forward_only): dict(groups [ngroups, 4], lists [*, 4], recs [*, 8]).  No two
+    rounds qualify: first is -1."""
+    g = np.ascontiguousarray(graph, np.int32)
+    B, maxlen = g.shape
+    meta, block = np.zeros(11, np.int32), np.zeros(48 * B * maxlen + 8 * groups, np.int32)
+    n = lib().cavs_schedule_group_lists(g.ctypes.data, B, maxlen, nchild, PAIR[pairing], rows_limit, groups, slice_rows, int(forward_only),
+                                        int(only_wide), meta.ctypes.data, block.ctypes.data, block.size)
+    if n < 0:
+        raise hip.CavsError("graph feed rejected: " + lib().cavs_session_error().decode())
+    out = dict(first=int(meta[0]), ngroups=int(meta[1]), tile_rows=int(meta[2]), room=int(meta[9]), written=int(meta[10]), fwd=None, bwd=None)
+    for k, m in (("fwd", meta[3:6]), ("bwd", meta[6:9]))[: 0 if n == 0 else 1 if forward_only else 2]:
+        gr = block[m[0]: m[0] + 4 * meta[1]].reshape(-1, 4)
+        li = block[m[1]: m[1] + 4 * (gr[-1, 0] + gr[-1, 1])].reshape(-1, 4)
+        rows = int((li[:, 0] + li[:, 1]).max())
+        out[k] = dict(groups=gr, lists=li, recs=block[m[2]: m[2] + 8 * rows].reshape(-1, 8))
     return out
 
 

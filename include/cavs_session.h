@@ -159,6 +159,15 @@ int cavs_schedule_index_lists(const int *graph, int B, int maxlen, int nchild, i
 int cavs_schedule_tail_lists(const int *graph, int B, int maxlen, int pairing, int fused_limit, int rows_limit, int groups,
                              int max_lists, int *meta, int *nrounds, int *start, int *count, int *flags, int *bstart,
                              int *bcount, int *bflags, int *rows_out);
+/* Pure host call: the block of the launches that keep many rounds resident (cavs_*_group_fwd / _bwd, cavs_hip.h) as the session
+ * would build it.  rows_limit: most rows of a round a group may get; groups (1..128): what the launches take
+ * (cavs_group_max_groups); slice: most rows of a list (cavs_group_rows); forward_only: no backward lists; only_wide: nothing
+ * where the lists would run in tiles of four rows.  Out: block; meta[0] = first round inside the launches (-1: none),
+ * [1] groups, [2] rows of a tile, [3..5] where groups, lists and records of the forward launch start in the block,
+ * [6..8] of the backward launch, [9] the room set aside for the block, [10] the words of it that were written.  Returns the ints
+ * of the block (0: no two rounds qualify), or -1 with the reason in cavs_session_error(). */
+int cavs_schedule_group_lists(const int *graph, int B, int maxlen, int nchild, int pairing, int rows_limit, int groups, int slice,
+                              int forward_only, int only_wide, int *meta, int *block, int cap);
 int cavs_schedule_trace_from_lists(int B, int maxlen, int N, int nchild, const int *round2offset, int R,
                                    const int *t2j, const int *pair, const int *child, const int *roots,
                                    int with_backward, int *out, int cap);

@@ -179,3 +179,72 @@ def test_the_deal_starts_later_under_a_tighter_limit_and_refuses_what_does_not_f
     chain = synth.chain_batch(5, 6, 4, 9, 9)[0]
     with pytest.raises(hip.CavsError):
         session.tail_lists(chain)
+
+
+@pytest.mark.parametrize("pairing", ["reference", "rowid"])
+@pytest.mark.parametrize("nchild,B,lo,hi", [(2, 64, 2, 64), (2, 25, 2, 50), (2, 200, 8, 40), (1, 128, 10, 100), (1, 16, 20, 20)])
+def test_the_lists_of_the_launches_that_keep_many_rounds_resident(nchild, B, lo, hi, pairing):
+    """Every row above the leaves once per direction, with the neighbours the index lists give it; rows without a parent as the
+    first lists of a backward pass, with the group their tree is in; a list waits for what its group has done."""
+    graph = (synth.tree_batch if nchild == 2 else synth.chain_batch)(900 + B, B, lo, hi)[0]
+    ix = session.index_lists(graph, nchild, pairing)
+    N, kid = ix["N"], ix["kid"].reshape(-1, nchild)
+    child = ix["child"].reshape(-1, nchild)
+    g = session.group_lists(graph, nchild, pairing, rows_limit=64, groups=64)
+    assert g["first"] >= 0
+    lo_row = int(g["fwd"]["recs"][:, 0].min())
+    none = np.full(N, -1)
+    c1, k1 = (child[:, 1], kid[:, 1]) if nchild == 2 else (none, none)
+    t2j = lambda k: np.where(k >= 0, ix["t2j"][np.maximum(k, 0)], -1)  # noqa: E731
+    rows = N - lo_row
+    f = g["fwd"]["recs"][:rows]
+    v = f[:, 0]
+    assert sorted(v) == list(range(lo_row, N))
+    np.testing.assert_array_equal(f[:, 1:5], np.stack([child[v, 0], c1[v], ix["pair"][v], ix["t2j"][v]], 1))
+    b = g["bwd"]["recs"][:rows]
+    v = b[:, 0]
+    assert sorted(v) == list(range(lo_row, N))
+    np.testing.assert_array_equal(b[:, 1:5], np.stack([kid[v, 0], k1[v], t2j(kid[v, 0]), t2j(k1[v])], 1))
+    alone = g["bwd"]["recs"][rows:]
+    assert sorted(alone[:, 0]) == sorted(ix["orphans"])
+    np.testing.assert_array_equal(alone[:, 1:5], np.stack([alone[:, 0], none[: len(alone)], ix["t2j"][alone[:, 0]], none[: len(alone)]], 1))
+    for d in ("fwd", "bwd"):
+        done_rows, seen = {}, np.zeros(len(g[d]["recs"]), int)
+        for grp, (at, n, arrivals, _) in enumerate(g[d]["groups"]):
+            arrived = 0
+            for first, count, wait, flags in g[d]["lists"][at: at + n]:
+                assert 1 <= count <= 32 and wait in (0, arrived)
+                seen[first: first + count] += 1
+                for r in g[d]["recs"][first: first + count]:
+                    if d == "bwd" and flags & 2:
+                        assert wait == 0 and not arrived
+                        done_rows[int(r[0])] = (grp, -1)
+                        continue
+                    # who wrote what this row reads ran in an earlier, waited-for round of the same group
+                    src = [int(k) for k in (kid[r[0]] if d == "fwd" else [])] or [int(r[0])]
+                    for k in src:
+                        if k >= lo_row and (k in done_rows or d == "fwd"):
+                            assert done_rows[k][0] == grp and done_rows[k][1] < arrived
+                    for k in ([int(r[0])] if d == "fwd" else [int(x) for x in kid[r[0]] if x >= 0]):
+                        done_rows[k] = (grp, arrived)
+                arrived += flags & 1
+            assert arrived == arrivals
+        assert (seen == 1).all()
+
+
+@pytest.mark.parametrize("nchild,B,lo,hi", [(2, 64, 2, 64), (2, 25, 2, 50), (2, 256, 32, 256), (1, 128, 10, 100), (1, 16, 20, 20)])
+def test_what_planning_a_new_batch_takes(nchild, B, lo, hi):
+    """Room for the lists (pinned, and copied): by the rows that may be in them, not by all of the batch's.  Where the launches with tiles
+    of four rows run instead, nothing of the block is written."""
+    graph = (synth.tree_batch if nchild == 2 else synth.chain_batch)(900 + B, B, lo, hi)[0]
+    N, leaves = session.index_lists(graph, nchild)["N"], int((session.index_lists(graph, nchild)["child"].reshape(-1, nchild)[:, 0] < 0).sum())
+    g = session.group_lists(graph, nchild)
+    assert g["room"] <= 24 * (N - leaves) + 12 * B + 8 * 64
+    assert g["written"] <= g["room"]
+    few = session.group_lists(graph, nchild, rows_limit=1 << 20, groups=64, only_wide=True)
+    assert few["first"] < 0 or few["tile_rows"] == 16
+    assert few["first"] >= 0 or few["written"] == 0
+    assert session.group_lists(graph, nchild, rows_limit=1 << 20, groups=64)["first"] >= 0
+    fwd = session.group_lists(graph, nchild, forward_only=True)
+    assert fwd["first"] == g["first"] and fwd["bwd"] is None
+    np.testing.assert_array_equal(fwd["fwd"]["recs"], g["fwd"]["recs"])
