@@ -782,8 +782,10 @@ void Engine::upload_index_arena() {
   }
   h.used = steps_;
   buffers_used_ = true;
-  h.host.reserve(grow(room, h.host.capacity()));
-  h.dev.reserve(grow(room, h.dev.capacity()));
+  // (twice what the first batch takes: growing is a wait for the device and 0.35 ms of pinning pages, whatever the size)
+  const size_t want = h.host.capacity() == 0 ? 2 * room : grow(room, h.host.capacity());
+  h.host.reserve(want);
+  h.dev.reserve(want);
   int *t2j = h.host.get(), *pair = t2j + N, *child = pair + N, *roots = child + (size_t)nch_ * N;
   std::string err = build_index_lists(s, nch_, cfg_.pairing, t2j, pair, child, roots);
   if (!err.empty()) fail(CAVS_EUNSUPPORTED, err);
