@@ -31,6 +31,10 @@ def libs():
         a.cavs_app_read_param.restype = C.c_long
         a.cavs_app_read.argtypes = [C.c_char_p, C.c_void_p, C.c_size_t]
         a.cavs_app_read.restype = C.c_long
+        a.cavs_app_counter.argtypes = [C.c_char_p]
+        a.cavs_app_counter.restype = C.c_double
+        a.cavs_app_bound_waits.argtypes = [C.c_int, C.c_int]
+        a.cavs_app_bound_waits.restype = None
         a.cavs_app_var_size.argtypes = [C.c_char_p]
         a.cavs_app_var_size.restype = C.c_long
         _host.C_DumpGraph.restype = C.c_size_t
@@ -155,6 +159,17 @@ class App:
         """Kernels the OPT_FUSION pass generated for the programs compiled so far."""
         a, _ = libs()
         return int(a.cavs_app_generated_kernels())
+
+    def counter(self, name):
+        """A count of the last pass of a lowered vertex function (`Session.counter`'s names)."""
+        a, _ = libs()
+        return float(a.cavs_app_counter(name.encode()))
+
+    def bound_waits(self, spins, extra):
+        """For tests: the waits inside the launches that run many rounds give up after `spins` polls, and wait for `extra` workgroups
+        that do not exist (0, 0: as ever)."""
+        a, _ = libs()
+        a.cavs_app_bound_waits(int(spins), int(extra))
 
     def close(self):
         a, _ = libs()

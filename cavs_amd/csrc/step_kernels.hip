@@ -350,6 +350,8 @@ struct TaskList {
   int first[kMaxTasks + 1];
   int count;
   const int *guard;  // CAVS_TASK_GUARD: when the word it points at is not zero, no job of the launch runs
+  int *report;       // CAVS_TASK_GUARD_REPORT: which such launch was the first
+  int serial;
 };
 
 __global__ __launch_bounds__(256) void tasks_kernel(TaskList L) {
@@ -359,7 +361,11 @@ __global__ __launch_bounds__(256) void tasks_kernel(TaskList L) {
     EmbedSgdLds sgd;
     float sums[4][64];
   } lds;
-  if (L.guard && __hip_atomic_load(L.guard, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
+  if (L.guard && __hip_atomic_load(L.guard, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+    if (L.report && blockIdx.x == 0 && threadIdx.x == 0 && __hip_atomic_load(L.report, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == 0)
+      __hip_atomic_store(L.report, L.serial, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return;
+  }
   int k = 0;
   while (k + 1 < L.count && (int)blockIdx.x >= L.first[k + 1]) k++;
   const cavs_task &t = L.t[k];
@@ -601,9 +607,13 @@ int cavs_run_tasks(int count, const cavs_task *tasks, void *stream) {
   for (int i = 0; i < count; i++) {
     const cavs_task &t = tasks[i];
     long blocks = 0;
-    if (t.kind == CAVS_TASK_GUARD) {
+    if (t.kind == CAVS_TASK_GUARD || t.kind == CAVS_TASK_GUARD_REPORT) {
       CAVS_REQUIRE(t.p0 && !L.guard, "cavs_run_tasks: job %d: a guard needs a word to watch, and a launch takes one guard", i);
       L.guard = static_cast<const int *>(t.p0);
+      if (t.kind == CAVS_TASK_GUARD) continue;
+      CAVS_REQUIRE(t.p1 && t.n0 > 0 && t.n0 < (1ll << 31), "cavs_run_tasks: job %d: a guard that reports needs a word and a positive number", i);
+      L.report = static_cast<int *>(t.p1);
+      L.serial = (int)t.n0;
       continue;
     }
     switch (t.kind) {

@@ -33,7 +33,7 @@ TASK_TRANSPOSE, TASK_ZERO_ROWS, TASK_SGD, TASK_EMBED_SGD, TASK_SUM_PARTS, TASK_B
 TASK_TREELSTM_GATES_ROWS = 8
 TASK_SGD_TRANSPOSE = 9
 TASK_GUARD = 10
-TASK_TREELSTM_LEAVES, TASK_LSTM_LEAVES = 11, 12
+TASK_TREELSTM_LEAVES, TASK_LSTM_LEAVES, TASK_GUARD_REPORT = 11, 12, 13
 
 
 class ColsumDesc(C.Structure):

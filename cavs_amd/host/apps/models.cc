@@ -585,6 +585,10 @@ long cavs_app_var_size(const char *name) {
 }
 
 int cavs_app_uses_fused_path(void) { return g_app ? g_app->sess->FusedPathKind() : 0; }
+double cavs_app_counter(const char *name) { return g_app ? C_SessionCounter(g_app->sess->handle(), name) : -1.0; }
+void cavs_app_bound_waits(int spins, int extra) {
+  if (g_app) C_SessionBoundWaits(g_app->sess->handle(), spins, extra);
+}
 int cavs_app_generated_kernels(void) { return g_app ? g_app->sess->GeneratedKernels() : 0; }
 
 void cavs_app_destroy(void) {

@@ -16,8 +16,6 @@
 namespace cavs {
 
 namespace {
-// polls of a tail launch's bounded wait (a poll is a round trip to the L2 and a short sleep: ~1 us)
-constexpr int kTailSpins = 1 << 19;
 inline size_t grow(size_t need, size_t have) {
   if (need <= have) return have;
   size_t g = have + have / 4;
@@ -192,7 +190,7 @@ void Engine::build_group_plan(const int *t2j, const int *pair, const int *child,
 }
 
 cavs_group_plan Engine::group_plan(const GroupLists::Launch &l) const {
-  return {d_group_ + l.groups, d_group_ + l.lists, d_group_ + l.recs, group_.ngroups, reinterpret_cast<unsigned *>(tail_sync_.get()), kTailSpins, 0,
+  return {d_group_ + l.groups, d_group_ + l.lists, d_group_ + l.recs, group_.ngroups, reinterpret_cast<unsigned *>(tail_sync_.get()), tail_spins_, tail_extra_,
           group_.tile_rows};
 }
 
@@ -241,14 +239,26 @@ void Engine::build_tail_plan(const int *kid_rows, int *rows_out) {
   tail_.flops = 2.0 * tail_.rows * cfg_.H * 5.0 * cfg_.H;
 }
 
+void Engine::bound_waits(int spins, int extra) {
+  tail_spins_ = spins > 0 ? spins : kTailSpins;
+  tail_extra_ = spins > 0 ? std::max(extra, 0) : 0;
+}
+
 void Engine::tail_check() {
+  const std::string why = tail_settle();
+  if (!why.empty())
+    fail(CAVS_EHIP, why + ": the results of the steps since the last synchronisation are undefined and their parameter updates were skipped; "
+                          "the session continues with one launch per round");
+}
+
+std::string Engine::tail_settle() {
   claim_.give();
-  if (!tail_pending_) return;
+  if (!tail_pending_) return "";
   tail_pending_ = false;
   int words[4] = {0, 0, 0, 0};
   check(cavs_memcpy_d2h(words, tail_sync_.get(), sizeof(words), stream_));
   check(cavs_stream_sync(stream_));
-  if (words[1] == 0) return;
+  if (words[1] == 0) return "";
   // every launch since the one that gave up left at once, and every parameter update watched the
   // word: the parameters are those of the last good step.  From here on: one launch per round.
   tail_ready_ = false;
@@ -256,11 +266,8 @@ void Engine::tail_check() {
   upk_valid_ = utp_valid_ = wfct_valid_ = false;
   emb_sparse_valid_ = false;
   check(cavs_zero(tail_sync_.get(), cavs_tail_sync_bytes(), stream_));
-  fail(CAVS_EHIP, std::string("a launch over the rounds near the roots gave up (") +
-                      (words[1] == CAVS_TAIL_TIMEOUT ? "its workgroups were not all resident within the wait's bound"
-                                                     : "its workgroups did not share one XCD") +
-                      "): the results of the steps since the last synchronisation are undefined and their parameter updates were "
-                      "skipped; the session continues with one launch per round");
+  return std::string("a launch over the rounds near the roots gave up (") +
+         (words[1] == CAVS_TAIL_TIMEOUT ? "its workgroups were not all resident within the wait's bound" : "its workgroups did not share one XCD") + ")";
 }
 
 Engine::~Engine() {
@@ -1596,8 +1603,8 @@ void Engine::treelstm_forward() {
         CAVS_TIMED(K_ROUND, cavs_treelstm_tail_fwd(pool_.get(), d_child_, d_pair_, xW_.get(), 4 * H, Upk_.get(), Bv, G_.get(), hlr_.get(),
                                                    gates_.get(), out_folded_ ? nullptr : msg_.get(), go, d_t2j_, d_tail_rows_,
                                                    (int)tail_.nrounds.size(), tail_.nrounds.data(), tail_.start.data(), tail_.count.data(),
-                                                   tail_.flags.data(), tail_.max_rounds, H, reinterpret_cast<unsigned *>(tail_sync_.get()), kTailSpins,
-                                                   0, stream_));
+                                                   tail_.flags.data(), tail_.max_rounds, H, reinterpret_cast<unsigned *>(tail_sync_.get()), tail_spins_,
+                                                   tail_extra_, stream_));
       });
       c_round_flops_ += tail_.flops;
       c_gather_rows_ += 2.0 * tail_.vertices;
@@ -1731,7 +1738,7 @@ void Engine::treelstm_backward() {
     CAVS_TIMED(K_ROUND, cavs_treelstm_tail_bwd(dxW_.get(), 4 * H, dF_.get(), dc_.get(), UT_.get(), d_kid_rows_, gates_.get(), G_.get(), d_dgo_,
                                                d_t2j_, sched_->leaf_prefix, d_tail_rows_, (int)tail_.nrounds.size(), tail_.nrounds.data(),
                                                tail_.bstart.data(), tail_.bcount.data(), tail_.bflags.data(), tail_.max_rounds, H,
-                                               reinterpret_cast<unsigned *>(tail_sync_.get()), kTailSpins, 0, stream_));
+                                               reinterpret_cast<unsigned *>(tail_sync_.get()), tail_spins_, tail_extra_, stream_));
     c_gather_rows_ += tail_.vertices;
     c_round_flops_ += tail_.flops;
     c_scatter_rows_ += 2.0 * tail_.vertices;

@@ -459,6 +459,9 @@ class Engine {
   bool probe_due_ = false;      // nobody could ask yet: another process was at it
   bool resident_ = false;       // this step may launch them: no other process is at it
   ResidentClaim claim_;
+  // polls of a tail launch's bounded wait (a poll is a round trip to the L2 and a short sleep: ~1 us)
+  static constexpr int kTailSpins = 1 << 19;
+  int tail_spins_ = kTailSpins, tail_extra_ = 0;
   bool tail_pending_ = false;   // a tail launch was enqueued since the status word was last read
   double c_tail_rounds_ = 0, c_tail_launches_ = 0;
   int tail_limit() const;       // rows per group and round a tail launch may take (0: no tail launches)
@@ -472,6 +475,11 @@ class Engine {
   // up leaves the results of the steps since undefined (their parameter updates were skipped: they
   // watch the word); the session goes on with one launch per round and this call fails.
   void tail_check();
+  // The same without failing: why a launch gave up (empty: none did).
+  std::string tail_settle();
+  // For tests: the waits of the launches from here on poll `spins` times at most and for `extra` workgroups that do not exist
+  // (0: as ever).
+  void bound_waits(int spins, int extra);
   // the word a parameter-update launch must watch (CAVS_TASK_GUARD), or null
   const int *update_guard() const { return tail_ready_ ? tail_sync_.get() + 1 : nullptr; }
  private:

@@ -193,7 +193,15 @@ long C_ReadTensor(C_Session *s, const char *name, float *out, size_t cap) {
 
 int C_SessionUsesFusedPath(C_Session *s) { return s->exec.fused_path_kind(); }
 int C_SessionGeneratedKernels(C_Session *s) { return s->exec.fused_kernel_count(); }
-void C_SessionAllowFusedPath(C_Session *s, int allow) { s->exec.set_lowering_mode(allow < 0 ? 0 : allow > 3 ? 3 : allow); }
-void C_SessionSetPairing(C_Session *s, int pairing) { s->exec.set_pairing(pairing); }
+double C_SessionCounter(C_Session *s, const char *name) {
+  double v = 0;
+  if (!name || !guarded("C_SessionCounter", [&] { v = s->exec.counter(name); })) return -1.0;
+  return v;
+}
+void C_SessionBoundWaits(C_Session *s, int spins, int extra) { s->exec.bound_waits(spins, extra); }
+void C_SessionAllowFusedPath(C_Session *s, int allow) {
+  must("C_SessionAllowFusedPath", [&] { s->exec.set_lowering_mode(allow < 0 ? 0 : allow > 3 ? 3 : allow); });
+}
+void C_SessionSetPairing(C_Session *s, int pairing) { must("C_SessionSetPairing", [&] { s->exec.set_pairing(pairing); }); }
 
 }  // extern "C"

@@ -88,6 +88,7 @@ void Executor::set_variable(const std::string &name, const float *data, size_t n
   pending_vars_[name].assign(data, data + n);
   Tensor *t = find_tensor(name);
   if (t) {
+    sync_and_settle();  // (Runs before this one read the value as it was)
     check(cavs_memcpy_h2d(t->base, data, n * 4, stream_));
     check(cavs_stream_sync(stream_));
     if (engine_) engine_->weights_written();
@@ -140,6 +141,8 @@ void Executor::init_variables() {
 void Executor::compile() {
   Graph &g = global_graph();
   if (compiled_version_ == g.version) return;
+  if (engine_) sync_and_settle();  // (by the programs as they were)
+  past_[0].live = past_[1].live = false;
   compiled_version_ = g.version;
   nch_ = 0;
   pool_w_ = ret_w_ = arg_w_ = 0;
@@ -733,7 +736,10 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
     check(cavs_event_sync(run_done_ev_[parity]));
     run_busy_[parity] = false;
   }
+  confirm(parity);
   bool uploads = false;
+  if (lowered_ && !run_done_ev_[0])
+    for (void *&e : run_done_ev_) check(cavs_event_create_device(&e));
   for (auto &f : feeds) {
     const Edge *e = g.main.find(f.first);
     if (!e || !e->src || e->src->def.name() != "Placeholder") fail(CAVS_EINVAL, "'" + f.first + "' is not a Placeholder");
@@ -742,14 +748,16 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
     Tensor &t = *slot;
     t.width = numel(e->shape);
     if (f.second->data.size() != (size_t)t.width * 4) fail(CAVS_EINVAL, "feed '" + f.first + "' has the wrong size");
+    if (std::find(fed_.begin(), fed_.end(), std::make_pair(&t, e->src->def.device() == CPU)) == fed_.end())
+      fed_.push_back({&t, e->src->def.device() == CPU});
     if (e->src->def.device() == CPU) {
       t.base = reinterpret_cast<float *>(const_cast<char *>(f.second->data.data()));
     } else {
       if (!copy_stream_) {
         check(cavs_stream_create(&copy_stream_));
         check(cavs_event_create(&feeds_up_ev_));
-        check(cavs_event_create_device(&run_done_ev_[0]));
-        check(cavs_event_create_device(&run_done_ev_[1]));
+        for (void *&ev : run_done_ev_)
+          if (!ev) check(cavs_event_create_device(&ev));
       }
       FeedStage &st = feed_stages_[f.first];
       const size_t bytes = (size_t)t.width * 4;
@@ -759,6 +767,7 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
       if (t.base && t.base == st.dev[parity].get() && run_busy_[parity ^ 1]) {
         check(cavs_event_sync(run_done_ev_[parity ^ 1]));
         run_busy_[parity ^ 1] = false;
+        confirm(parity ^ 1);
       }
       st.slot[parity].reserve(bytes);
       st.dev[parity].reserve(t.width);
@@ -781,7 +790,7 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
       if (on && stamped) e->run_busy_[parity] = true;
       else if (on && cavs_event_record(e->run_done_ev_[parity], e->stream_) == CAVS_OK) e->run_busy_[parity] = true;
     }
-  } mark_done{this, parity, copy_stream_ != nullptr};  // every Run, so that a later one can tell when this one's reads are over
+  } mark_done{this, parity, run_done_ev_[0] != nullptr};  // every Run, so that a later one can tell when this one's reads are over
   bool train = false;
   std::vector<std::string> targets;
   for (auto &o : outputs) {
@@ -794,7 +803,6 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
   }
   std::vector<const Node *> order;
   forward_needed(targets, &order);
-  RoundCtx mainctx{0, 0, false};
   std::string key = train ? "T" : "F";
   for (auto &t : targets) key += "|" + t;
   auto it = main_cache_.find(key);
@@ -815,12 +823,48 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
     }
     it = main_cache_.emplace(key, std::move(mp)).first;
   }
-  binds_ = &it->second.binds;
-  const HeadFuse &head = it->second.head;
   // The optimizer's scope -- the replayed forward ops, the gradients and the update -- runs
   // `iters` times per Run (ScopedNode(s_, name, iters), cavs/midend/graph_util.cc:266-283;
   // BasicBlock::Run, cavs/midend/statement.h:66-75).
   const int passes = train ? std::max(1, g.opt.iters) : 1;
+  if (passes_run_ > (1 << 30)) {  // (before their number runs over: none is left to be told apart)
+    sync_and_settle();
+    passes_run_ = 0;
+  }
+  if (lowered_) remember_run(parity, &it->second, train, passes);
+  run_program(it->second, train, 0, passes, mark_done.on ? run_done_ev_[parity] : nullptr, &mark_done.stamped);
+  results->assign(outputs.size(), nullptr);
+  // A Run that asks for the optimizer only (the training loop of the reference's apps) has
+  // nothing to hand back: it returns with the step still in flight, and the host prepares the
+  // next batch meanwhile.  Whatever reads a value afterwards waits for the stream first.
+  bool reads = false;
+  for (auto &o : outputs)
+    if (!(g.opt.present && o == g.opt.output)) reads = true;
+  if (!reads) {
+    dirty_ = true;
+    return;
+  }
+  sync_and_settle();
+  dirty_ = false;
+  for (size_t i = 0; i < outputs.size(); i++) {
+    if (g.opt.present && outputs[i] == g.opt.output) continue;
+    Tensor &t = tensor(outputs[i]);
+    auto *h = new HostTensor;
+    h->name = outputs[i];
+    h->data.resize(t.count() * 4);
+    check(cavs_memcpy_d2h(h->data.data(), t.base, h->data.size(), stream_));
+    (*results)[i] = h;
+  }
+  check(cavs_stream_sync(stream_));
+}
+
+// `passes` passes of a program from pass `from` on.  done_ev (may be null): recorded by the last launch where that is
+// possible, *stamped says whether.
+void Executor::run_program(const MainProgram &mp, bool train, int from, int passes, void *done_ev, bool *stamped) {
+  Graph &g = global_graph();
+  RoundCtx mainctx{0, 0, false};
+  binds_ = &mp.binds;
+  const HeadFuse &head = mp.head;
   // Launches that can ride in others when the lowered vertex function's backward pass follows in
   // this Run: the sum of the head's gradient partials (into the launch that opens that pass) and,
   // when nothing between that pass and the update reads them (no clipping, every later gradient op
@@ -829,28 +873,28 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
   trains_ = train;
   if (train && lowered_) {
     int at = -1;
-    const std::vector<char> &skip = it->second.skip_bwd;
-    for (size_t i = 0; i < it->second.bwd.size(); i++)
-      if (it->second.bwd[i].name() == "GraphOutput_grad") at = (int)i;
+    const std::vector<char> &skip = mp.skip_bwd;
+    for (size_t i = 0; i < mp.bwd.size(); i++)
+      if (mp.bwd[i].name() == "GraphOutput_grad") at = (int)i;
     if (at >= 0 && head.fc >= 0 && head.fc_grad >= 0 && head.fc_grad < at) head_defer_ = true;
     if (at >= 0 && g.opt.clip <= 0.f) {
       defer_bias_ = true;
-      for (size_t i = at + 1; i < it->second.bwd.size(); i++)
+      for (size_t i = at + 1; i < mp.bwd.size(); i++)
         if (!(i < skip.size() && skip[i])) defer_bias_ = false;
     }
   }
-  for (int pass = 0; pass < passes; pass++) {
+  for (int pass = from; pass < passes; pass++) {
   bool head_fused = false;
-  for (size_t i = 0; i < it->second.fwd.size(); i++) {
-    const OpDef &d = it->second.fwd[i];
-    if ((int)i == head.fc) head_fused = run_fused_head(it->second);
+  for (size_t i = 0; i < mp.fwd.size(); i++) {
+    const OpDef &d = mp.fwd[i];
+    if ((int)i == head.fc) head_fused = run_fused_head(mp);
     if (head_fused && ((int)i == head.fc || (int)i == head.loss)) continue;
     if (d.name() == "GraphOutput") run_graph_output(d); else exec(d, mainctx);
   }
   if (train) {
-    const std::vector<char> &skip = it->second.skip_bwd;
-    for (size_t i = 0; i < it->second.bwd.size(); i++) {
-      const OpDef &d = it->second.bwd[i];
+    const std::vector<char> &skip = mp.skip_bwd;
+    for (size_t i = 0; i < mp.bwd.size(); i++) {
+      const OpDef &d = mp.bwd[i];
       if (i < skip.size() && skip[i]) continue;
       if (head_fused && ((int)i == head.loss_grad || (int)i == head.fc_grad || (int)i == head.seed)) continue;
       if (d.name() == "GraphOutput_grad") run_graph_output_grad(d); else exec(d, mainctx);
@@ -872,7 +916,12 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
     std::vector<const float *> by_bias_job;
     // (the lowered F's launches over the rounds near the roots can give up: no update runs then)
     const int *guard = engine_ ? engine_->update_guard() : nullptr;
-    const cavs_task guard_task{CAVS_TASK_GUARD, 0.f, 0, 0, 0, const_cast<int *>(guard), nullptr, nullptr, nullptr};
+    if (guard && held_back_.capacity() == 0) {
+      held_back_.reserve(1);
+      *held_back_.get() = 0;
+    }
+    passes_run_++;
+    const cavs_task guard_task{CAVS_TASK_GUARD_REPORT, 0.f, passes_run_, 0, 0, const_cast<int *>(guard), held_back_.get(), nullptr, nullptr};
     if (guard) updates.push_back(guard_task);
     if (engine_ && defer_bias_) engine_->update_bias_jobs(g.opt.lr, &updates, &by_bias_job);
     for (auto &v : g.opt.vars) {
@@ -887,39 +936,83 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
       if (engine_ && engine_->update_jobs(w.base, gr.base, g.opt.lr, &updates)) continue;
       updates.push_back({CAVS_TASK_SGD, g.opt.lr, (long long)w.count(), 0, 0, w.base, gr.base, nullptr, nullptr});
     }
-    const bool stamp = mark_done.on && pass + 1 == passes;
-    if (stamp) check(cavs_stop_event_arm(run_done_ev_[parity]));
+    const bool stamp = done_ev && pass + 1 == passes;
+    if (stamp) check(cavs_stop_event_arm(done_ev));
     const int rc = cavs_run_tasks((int)updates.size(), updates.data(), stream_);
     int launched = 0;
     if (stamp) check(cavs_profile_disarm(&launched));
     check(rc);
-    mark_done.stamped = launched != 0;
+    *stamped = launched != 0;
   }
   }  // passes
-  results->assign(outputs.size(), nullptr);
-  // A Run that asks for the optimizer only (the training loop of the reference's apps) has
-  // nothing to hand back: it returns with the step still in flight, and the host prepares the
-  // next batch meanwhile.  Whatever reads a value afterwards waits for the stream first.
-  bool reads = false;
-  for (auto &o : outputs)
-    if (!(g.opt.present && o == g.opt.output)) reads = true;
-  if (!reads) {
-    dirty_ = true;
-    return;
+}
+
+// What a Run read and would read again.
+void Executor::remember_run(int parity, const MainProgram *mp, bool train, int passes) {
+  PastRun &r = past_[parity];
+  r.program = mp;
+  r.train = train;
+  r.passes = passes;
+  r.serial = passes_run_ + 1;
+  r.feeds.clear();
+  size_t hosts = 0;
+  for (auto &f : fed_) {
+    float *base = f.first->base;
+    if (f.second && base) {  // (the caller's memory, which is free again when the Run returns)
+      if (r.host.size() <= hosts) r.host.emplace_back();
+      r.host[hosts].assign(base, base + f.first->width);
+      base = r.host[hosts++].data();
+    }
+    r.feeds.push_back({f.first, base});
   }
+  r.live = true;
+}
+
+// The last Run of this parity is over.  If its update was held back it is made up for now, while its feeds are there.
+void Executor::confirm(int parity) {
+  if (!past_[parity].live) return;
+  if (held_back_.capacity() > 0 && *static_cast<volatile int *>(held_back_.get()) != 0) sync_and_settle();
+  past_[parity].live = false;
+}
+
+// Waits for everything.  Runs that a launch which gave up has undone (their updates watch its status word, as do all those behind)
+// are run again, from the first pass that was held back, with one launch per round.
+void Executor::sync_and_settle() {
   check(cavs_stream_sync(stream_));
-  dirty_ = false;
-  for (size_t i = 0; i < outputs.size(); i++) {
-    if (g.opt.present && outputs[i] == g.opt.output) continue;
-    Tensor &t = tensor(outputs[i]);
-    auto *h = new HostTensor;
-    h->name = outputs[i];
-    h->data.resize(t.count() * 4);
-    check(cavs_memcpy_d2h(h->data.data(), t.base, h->data.size(), stream_));
-    (*results)[i] = h;
+  settle();
+}
+
+void Executor::settle() {
+  const std::string why = engine_ ? engine_->tail_settle() : "";
+  if (!why.empty()) {
+    const int first = held_back_.capacity() > 0 ? *static_cast<volatile int *>(held_back_.get()) : 0;
+    if (first != 0) *held_back_.get() = 0;
+    std::vector<std::pair<Tensor *, float *>> now;
+    for (auto &f : fed_) now.push_back({f.first, f.first->base});
+    const int old = past_[0].live && past_[1].live && past_[1].serial < past_[0].serial ? 1 : 0;
+    // (a Run without an update is the newest one: it was about to be read)
+    for (int k = 0; k < 2; k++) {
+      PastRun &r = past_[(old + k) & 1];
+      if (!r.live || (r.train && (first == 0 || r.serial + r.passes <= first))) continue;
+      for (auto &f : r.feeds) f.first->base = f.second;
+      bool stamped = false;
+      const int serial = passes_run_;
+      run_program(*r.program, r.train, r.train ? std::max(0, first - r.serial) : 0, r.passes, nullptr, &stamped);
+      passes_run_ = serial;
+    }
+    check(cavs_stream_sync(stream_));
+    for (auto &f : now) f.first->base = f.second;
+    std::fprintf(stderr, "cavs: %s; what it held back was run again, and the session continues with one launch per round\n", why.c_str());
   }
-  check(cavs_stream_sync(stream_));
-  if (engine_) engine_->tail_check();
+  past_[0].live = past_[1].live = false;
+}
+
+// Behind a read, which has waited for the stream: whether what it read has changed since.
+bool Executor::settle_read() {
+  if (!engine_) return false;
+  const bool again = held_back_.capacity() > 0 && *static_cast<volatile int *>(held_back_.get()) != 0;
+  settle();
+  return again;
 }
 
 long Executor::read_tensor(const std::string &name, float *out, size_t cap) {
@@ -930,7 +1023,7 @@ long Executor::read_tensor(const std::string &name, float *out, size_t cap) {
   size_t n = t->count();
   if (!out || cap < n) return -(long)n;
   readback_.read(out, t->base, n * 4, stream_, copy_stream_);
-  if (engine_) engine_->tail_check();
+  if (settle_read()) readback_.read(out, t->base, n * 4, stream_, copy_stream_);
   return (long)n;
 }
 

@@ -57,8 +57,10 @@ class Executor {
   bool uses_fused_path() const { return lowered_; }
   int fused_kernel_count() const { return fused_groups_; }
   int fused_path_kind() const;  // 0: F runs op by op; 1: hand-written round kernels; 2: generated ones
-  void set_lowering_mode(int m) { lowering_mode_ = m; compiled_version_ = -1; }
-  void set_pairing(int p) { pairing_ = p; compiled_version_ = -1; }
+  void set_lowering_mode(int m);
+  void set_pairing(int p);
+  double counter(const std::string &name) const { return engine_ ? engine_->counter(name) : 0.0; }
+  void bound_waits(int spins, int extra);  // Engine::bound_waits
 
  private:
   struct RoundCtx {
@@ -147,6 +149,27 @@ class Executor {
     std::vector<GradBind> binds;
     HeadFuse head;
   };
+  void run_program(const MainProgram &mp, bool train, int from, int passes, void *done_ev, bool *stamped);
+  // A lowered F's launches over the rounds near the roots can give up.  Neither the update of such a pass nor any behind it does anything
+  // (CAVS_TASK_GUARD_REPORT), and what the Runs since have read is kept until they are known to have gone through -- the next
+  // Run but one looks before it takes a Run's feed buffers, every reading looks -- so that they can be run again.
+  struct PastRun {
+    const MainProgram *program = nullptr;
+    bool live = false, train = false;
+    int passes = 1, serial = 0;                      // serial of its first pass (passes_run_)
+    std::vector<std::pair<Tensor *, float *>> feeds;  // where its placeholders were
+    std::vector<std::vector<float>> host;            // those that stay in host memory
+  };
+  PastRun past_[2];                            // by parity
+  std::vector<std::pair<Tensor *, bool>> fed_;  // placeholders, and whether they stay in host memory
+  PinnedArray<int> held_back_;                 // [1] the first pass whose update was held back; 0: none
+  int passes_run_ = 0;
+  int spins_ = 0, extra_ = 0;
+  void remember_run(int parity, const MainProgram *mp, bool train, int passes);
+  void confirm(int parity);
+  void sync_and_settle();
+  void settle();
+  bool settle_read();
   void plan_fused_head(MainProgram *mp) const;
   bool run_fused_head(const MainProgram &mp);
   float *output_storage(const std::string &name, long *count);

@@ -352,6 +352,24 @@ std::map<std::string, Slot> role_slots(const Lowering &lw) {
 }
 }  // namespace
 
+void Executor::set_lowering_mode(int m) {
+  if (engine_) sync_and_settle();
+  lowering_mode_ = m;
+  compiled_version_ = -1;
+}
+
+void Executor::set_pairing(int p) {
+  if (engine_) sync_and_settle();
+  pairing_ = p;
+  compiled_version_ = -1;
+}
+
+void Executor::bound_waits(int spins, int extra) {
+  spins_ = spins;
+  extra_ = extra;
+  if (engine_) engine_->bound_waits(spins, extra);
+}
+
 int Executor::fused_path_kind() const { return !lowered_ ? 0 : lowering_->model == CAVS_MODEL_CELL ? 2 : 1; }
 
 void Executor::lowered_forward(const int32_t *graph, int B, int maxlen, float *) {
@@ -369,6 +387,7 @@ void Executor::lowered_forward(const int32_t *graph, int B, int maxlen, float *)
     cfg.use_x = lw.use_x;
     cfg.split_backward_rounds = lowering_mode_ == 3;
     engine_ = std::make_unique<Engine>(cfg, stream_, lw.cell);
+    engine_->bound_waits(spins_, extra_);
   }
   engine_->set_pairing(pairing_);
   // parameters live in the user's Variable tensors; the engine reads them in place

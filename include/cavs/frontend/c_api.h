@@ -53,6 +53,12 @@ long C_ReadTensor(C_Session *s, const char *name, float *out, size_t cap);
 int C_SessionUsesFusedPath(C_Session *s);
 /* Number of kernels the OPT_FUSION pass generated for the programs compiled so far. */
 int C_SessionGeneratedKernels(C_Session *s);
+/* A count of the last pass of a lowered vertex function (cavs_session_counter's names: "tail_rounds", "launches", ..); 0 where it
+ * runs op by op, -1 for a name that does not exist. */
+double C_SessionCounter(C_Session *s, const char *name);
+/* For tests: the waits inside the launches that run many rounds poll `spins` times at most, and for `extra` workgroups that do not
+ * exist, so that they give up (0, 0: as ever).  What such a launch holds back is run again, one launch per round. */
+void C_SessionBoundWaits(C_Session *s, int spins, int extra);
 /* 0 forbids that lowering (op-by-op execution of F, for A/B tests); 1, the default, tries the
  * hand-written kernels first and generated ones next; 2 goes for generated kernels only; 3 does the
  * same and runs the backward rounds the way a batch whose message flow is no forest needs them

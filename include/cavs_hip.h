@@ -709,11 +709,13 @@ int cavs_root_sq(float *parts, float *dgraph_out, const float *graph_out, const 
  *                        its jobs does anything (the parameter updates of a step whose
  *                        cavs_treelstm_tail_* launch gave up: p0 = the status word of its sync block).
  *                        At most one per launch; it does not count towards the 12.
+ *   CAVS_TASK_GUARD_REPORT  CAVS_TASK_GUARD that says so: the int p1, host memory of cavs_host_alloc, gets n0 (positive) if it
+ *                        is zero when a launch holds its jobs back.
  * p4 .. p7 are read by the jobs that name them only and may stay null otherwise. */
 enum { CAVS_TASK_TRANSPOSE = 0, CAVS_TASK_ZERO_ROWS = 1, CAVS_TASK_SGD = 2, CAVS_TASK_EMBED_SGD = 3,
        CAVS_TASK_SUM_PARTS = 4, CAVS_TASK_BLOCKS_SGD = 5, CAVS_TASK_PACK_T = 6, CAVS_TASK_SGD_PACK = 7,
        CAVS_TASK_TREELSTM_GATES_ROWS = 8, CAVS_TASK_SGD_TRANSPOSE = 9, CAVS_TASK_GUARD = 10,
-       CAVS_TASK_TREELSTM_LEAVES = 11, CAVS_TASK_LSTM_LEAVES = 12 };
+       CAVS_TASK_TREELSTM_LEAVES = 11, CAVS_TASK_LSTM_LEAVES = 12, CAVS_TASK_GUARD_REPORT = 13 };
 typedef struct cavs_task {
   int kind;
   float f0;

@@ -6,11 +6,12 @@ import subprocess
 import numpy as np
 import pytest
 
-from cavs_amd import build
+from cavs_amd import apps, build, session
 from test_cell_lowering import _declare, _dump
-from test_gpu_cell import compare, run_generated
+from test_gpu_cell import NAMES, compare, run_generated
 from test_gpu_resident import another_process
 from test_oracle_models import small_workload
+from tolerance import close
 
 
 @pytest.mark.parametrize("model,H", [("treelstm2", 512), ("treegru", 100), ("treedeep", 64)])
@@ -59,3 +60,43 @@ def test_resident_rounds_give_what_a_launch_per_round_gives(model, H):
     assert got[0][3] == got[1][3] == 2
     compare(got[0], dict(loss=got[1][0], graph_out=got[1][1], grads=got[1][2]))
 
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model,H,mode", [("treelstm2", 100, 1), ("treedeep", 64, 1), ("treelstm", 64, 1), ("treelstm", 512, 1), ("lstm", 128, 1)])
+@pytest.mark.parametrize("iters,read", [(1, False), (1, True), (3, False)])
+def test_what_a_launch_that_gives_up_holds_back_is_run_again(model, H, mode, iters, read):
+    """The waits of such a launch are bounded: when one runs out, the updates of that pass and of all behind it are held back.  A
+    training loop that reads nothing, one that reads every step, one of three passes a Run: each ends where the same loop ends whose
+    launches never give up (the rounds run as launches of their own from there on, so sums are ordered otherwise)."""
+    batches = [small_workload(model, 500 + k, B=12, H=H, E=12, V=29, C=5) for k in range(5)]
+    gain = np.float32(0.4 * min(1.0, (64.0 / H) ** 0.5))
+    params = {k: np.asarray(batches[0]["params"][k], np.float32) * (gain if k in ("U", "W") else np.float32(1.0)) for k in NAMES[model]}
+    maxlen = max(w["graph"].shape[1] for w in batches)
+    graphs = [np.pad(w["graph"], ((0, 0), (0, maxlen - w["graph"].shape[1])), constant_values=-1) for w in batches]
+    ends = []
+    for gives_up in (False, True):
+        w0 = batches[0]
+        a = apps.App(model, B=12, maxlen=maxlen, H=H, E=w0["E"], V=w0["V"], C_=w0["C"], opt=session.OPT_BATCHING, lr=0.02, allow_fused=mode, iters=iters)
+        a.set_params(params)
+        seen = []
+        for k, (g, w) in enumerate(zip(graphs, batches)):
+            print(f"[case] {model} H={H} iters={iters} read={read} gives up={gives_up} step {k}", flush=True)
+            if gives_up and k == 1:  # (64 polls, for one workgroup more than there are)
+                a.bound_waits(64, 1)
+            out = a.step(g, w["x"], w["labels"], train=True, fetch=read)
+            if k == 0:
+                assert a.counter("tail_rounds") > 0
+            if read:
+                seen.append(np.asarray(out[0]))
+        values = {k: a.grad(k, np.shape(v), grad=False) for k, v in params.items()}
+        grads = {k: a.grad(k, np.shape(v)) for k, v in params.items()}
+        assert (a.counter("tail_rounds") > 0) == (not gives_up)
+        a.close()
+        ends.append((seen, values, grads))
+    (seen, values, grads), (want_seen, want, want_grads) = ends[1], ends[0]
+    for x, y in zip(seen, want_seen):
+        close(x, y, "loss")
+    for k in params:
+        assert np.abs(want[k] - params[k].reshape(want[k].shape)).max() > 1e-4, f"{k} does not move"
+        close(values[k], want[k], k)
+        close(grads[k], want_grads[k], "d" + k)
