@@ -14,9 +14,9 @@
 namespace cavs {
 
 constexpr int kIndexThreads = 1024, kIndexWaves = kIndexThreads / 64;
-// Up to kIndexLds rows (and ids below kIndexKeys) are sorted in LDS, id and row packed in a word, in one launch; more
+// Up to kIndexLds rows whose ids fit a word beside the row's number are sorted in LDS in one launch; more
 // by the launches of index_sort_* and index_words_*.  us, one launch / seven: 4096 rows 20.6 / 29.3, 7088 31.9 / 30.7, 9000 39.0 / 31.8.
-constexpr int kIndexLds = 8192, kIndexKeys = 1 << 19;
+constexpr int kIndexLds = 8192;
 
 // Lanes of `active` whose low `bits` bits of d equal this lane's.
 __device__ inline unsigned long long match_lanes(unsigned d, unsigned long long active) {
@@ -63,7 +63,7 @@ __device__ inline unsigned word_key(float id, int V) {
 // order, so that ranks are stable without a second pass.
 __global__ __launch_bounds__(kIndexThreads) void embed_index_kernel(int *__restrict__ index, float *__restrict__ ids_out,
                                                                     const float *__restrict__ x, const int *__restrict__ rows, int n, int V,
-                                                                    int leaf_rows, int passes) {
+                                                                    int leaf_rows, int passes, int row_bits) {
   __shared__ unsigned lds[2 * kIndexLds];
   __shared__ unsigned hist[kIndexWaves][256];
   __shared__ unsigned wave_sums[kIndexWaves], first_sums[kIndexWaves], leaf_sums[kIndexWaves];
@@ -71,9 +71,9 @@ __global__ __launch_bounds__(kIndexThreads) void embed_index_kernel(int *__restr
   const unsigned long long below = (1ull << lane) - 1;
   // row i: id key(i), vertex row val(i)
   unsigned *ka = lds, *kb = lds + kIndexLds;
-  auto key = [&](int i) { return ka[i] / kIndexLds; };
-  auto val = [&](int i) { return ka[i] % kIndexLds; };
-  auto put = [&](unsigned *k, int i, unsigned id, unsigned row) { k[i] = id * kIndexLds + row; };
+  auto key = [&](int i) { return ka[i] >> row_bits; };
+  auto val = [&](int i) { return ka[i] & ((1u << row_bits) - 1); };
+  auto put = [&](unsigned *k, int i, unsigned id, unsigned row) { k[i] = id << row_bits | row; };
   int *slot = index + 4, *order = slot + n, *at = order + n;
   float *word = reinterpret_cast<float *>(at + n);
   const int per = ((n + kIndexWaves - 1) / kIndexWaves + 63) / 64 * 64;
@@ -183,7 +183,8 @@ __global__ __launch_bounds__(kIndexThreads) void embed_index_kernel(int *__restr
 // 300000 55, where one workgroup, its rows in memory, took 65, 363 (540 inside a step) and 2090.
 struct SortWork {
   unsigned *ka, *va, *kb, *vb;  // [n] ids and rows, from and to
-  unsigned *counts;             // [groups][256] rows of a digit in a stretch; then [groups][2] words that begin, words of leaves only
+  unsigned *counts;             // [groups][256] rows of a digit in a stretch (where the index goes afterwards)
+  unsigned *words;              // [groups][2] words that begin in a stretch, words of leaves only (where the sort had its rows)
   int n, per, groups;           // rows of a stretch: a multiple of 1024
   __device__ inline void stretch(int *beg, int *end) const {
     const int own = per / kIndexWaves;
@@ -283,7 +284,7 @@ __global__ __launch_bounds__(kIndexThreads) void index_words_kernel(SortWork s, 
   __shared__ unsigned own[kIndexWaves][2], others[kIndexWaves][4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = blockIdx.x, n = s.n;
   const unsigned long long below = (1ull << lane) - 1;
-  unsigned *counts = s.counts + s.groups * 256;
+  unsigned *counts = s.words;
   int beg, end;
   s.stretch(&beg, &end);
   auto bounds = [&](int p, bool *first, bool *last, bool *leaves) {
@@ -497,8 +498,7 @@ extern "C" {
 
 size_t cavs_embed_index_ints(int n) { return 4 + 4 * (size_t)std::max(n, 0); }
 
-// (no less than for any smaller n)
-size_t cavs_embed_index_workspace(int n) { return n <= 0 ? 0 : 4 * sizeof(unsigned) * (size_t)n + sizeof(unsigned) * 258 * (size_t)std::min((n + 1023) / 1024, kSortGroups); }
+size_t cavs_embed_index_workspace(int n) { return 4 * sizeof(unsigned) * (size_t)std::max(n, 0); }
 
 int cavs_embed_index(int *index, float *ids_out, const float *x, const int *rows, int n, int V, int leaf_rows, void *workspace,
                      size_t workspace_bytes, void *stream) {
@@ -509,13 +509,15 @@ int cavs_embed_index(int *index, float *ids_out, const float *x, const int *rows
   CAVS_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), "cavs_embed_index: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
   const int passes = V < (1 << 8) ? 1 : V < (1 << 16) ? 2 : 3;  // (keys 0 .. V)
   hipStream_t st = as_stream(stream);
-  if (n <= kIndexLds && V < kIndexKeys) {
-    launch(embed_index_kernel, 1, kIndexThreads, 0, st, index, ids_out, x, rows, n, V, leaf_rows, passes);
+  int row_bits = 8;  // (up to 256 rows: any id a float counts to)
+  while ((1 << row_bits) < std::min(n, kIndexLds)) row_bits++;
+  if (n <= kIndexLds && (n <= 256 || V < 1 << (32 - row_bits))) {  // (ids 0 .. V)
+    launch(embed_index_kernel, 1, kIndexThreads, 0, st, index, ids_out, x, rows, n, V, leaf_rows, passes, row_bits);
     CAVS_LAUNCH_CHECK();
     return CAVS_OK;
   }
   unsigned *w = static_cast<unsigned *>(workspace);
-  SortWork s{w, w + n, w + 2 * (size_t)n, w + 3 * (size_t)n, w + 4 * (size_t)n, n, sort_per(n), sort_groups(n)};
+  SortWork s{w, w + n, w + 2 * (size_t)n, w + 3 * (size_t)n, reinterpret_cast<unsigned *>(index + 4), nullptr, n, sort_per(n), sort_groups(n)};
   for (int pass = 0; pass < passes; pass++) {
     if (pass == 0) launch(index_sort_count_kernel<true>, s.groups, kIndexThreads, 0, st, s, ids_out, x, rows, V, 0);
     else launch(index_sort_count_kernel<false>, s.groups, kIndexThreads, 0, st, s, nullptr, nullptr, nullptr, V, 8 * pass);
@@ -523,6 +525,7 @@ int cavs_embed_index(int *index, float *ids_out, const float *x, const int *rows
     std::swap(s.ka, s.kb);
     std::swap(s.va, s.vb);
   }
+  s.words = s.vb;
   launch(index_words_kernel<0>, s.groups, kIndexThreads, 0, st, s, index, ids_out, V, leaf_rows);
   launch(index_words_kernel<1>, s.groups, kIndexThreads, 0, st, s, index, ids_out, V, leaf_rows);
   launch(index_words_kernel<2>, s.groups, kIndexThreads, 0, st, s, index, ids_out, V, leaf_rows);

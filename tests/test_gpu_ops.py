@@ -1910,9 +1910,28 @@ def test_products_of_infinite_and_very_large_operands(g, tA, tB, M, N, K):
     np.testing.assert_allclose(got[ok], want[ok], rtol=2.0 ** -24 * (K + 4))
 
 
+@pytest.mark.parametrize("n,V", [(1, 3), (257, (1 << 24) - 1), (8192, 1000), (8193, 1000), (8193, 1 << 20), (70000, 500), (300000, 70000)])
+def test_the_index_of_a_batch_stays_within_four_words_a_row(g, n, V):
+    """The workspace of cavs_embed_index: the sort's rows, twice, and nothing else; its counts lie where the index goes afterwards."""
+    r = rng(n + V)
+    x = np.floor(r.bulk_uniform(n) * min(V, 3 * n)).astype(np.float32)
+    x[:: max(2, n // 7)] = V - 1
+    L = hip.lib()
+    assert L.cavs_embed_index_workspace(n) == 16 * n
+    ws, index = g.devi(np.full(4 * n + 64, 77, np.int32)), g.devi(np.full(L.cavs_embed_index_ints(n) + 64, 77, np.int32))
+    g.call("cavs_embed_index", g.P(index), g.P(g.zeros(n)), g.P(g.devf(x)), g.P(g.devi(np.arange(n))), n, V, n // 2, g.P(ws), 16 * n, g.stream())
+    got = g.host(index)
+    assert (got[-64:] == 77).all() and (g.host(ws)[-64:] == 77).all()
+    slot, order, word = got[4:4 + n], got[4 + n:4 + 2 * n], got[4 + 3 * n:4 + 4 * n].view(np.float32)
+    assert got[0] == len(np.unique(x))
+    np.testing.assert_array_equal(word[slot], x)
+    np.testing.assert_array_equal(order, np.argsort(x, kind="stable"))
+
+
 @pytest.mark.parametrize("n,V,E,w,leaf_rows", [(1, 5, 8, 4, 1), (63, 4, 12, 260, 40), (64, 255, 4, 256, 0), (65, 256, 20, 8, 65), (2368, 21701, 300, 512, 1216),
                                                (4096, 70000, 8, 12, 100), (4097, 65535, 8, 300, 4000), (9000, 300, 16, 64, 5000), (16384, 1000, 8, 16, 9000),
-                                               (16385, 1000, 8, 16, 9000)])
+                                               (16385, 1000, 8, 16, 9000), (8192, 524287, 4, 64, 5000), (8192, 524288, 4, 64, 5000), (8193, 1000, 8, 16, 4000),
+                                               (1, 2200000, 4, 4, 1), (256, 2200000, 4, 64, 100), (1025, 2097151, 4, 64, 500), (1025, 2097152, 4, 64, 500)])
 def test_words_of_a_batch(g, n, V, E, w, leaf_rows):
     """cavs_embed_index and what runs over its words, against numpy: one id shared by most rows (segments over many
     pieces), ids that are no table row, sizes at the edges of a wavefront, of the digits and of the sort in LDS."""
