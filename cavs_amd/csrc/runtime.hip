@@ -148,7 +148,7 @@ using namespace cavs;
 extern "C" {
 
 const char *cavs_last_error(void) { return g_err; }
-int cavs_abi_version(void) { return 2; }
+int cavs_abi_version(void) { return CAVS_ABI_VERSION; }
 
 int cavs_init(int device) {
   CAVS_HIP_TRY(hipSetDevice(device));

@@ -36,7 +36,10 @@ enum {
 };
 
 const char *cavs_last_error(void);
-/* ABI version of this header; bumped on any signature change. */
+/* ABI version of this header; bumped on any change of a signature, a struct or what a call reads.  A caller compares what it was built
+ * with (CAVS_ABI_VERSION) to what the library says.
+ *   3: cavs_group_plan::tile_rows; CAVS_TASK_SUM_PARTS reads f0, p3 and p4, CAVS_TASK_SGD_PACK reads p3 (null: as before) */
+#define CAVS_ABI_VERSION 3
 int cavs_abi_version(void);
 
 /* ------------------------------------------------------------------ runtime

@@ -20,6 +20,15 @@ def test_library_exports_every_declared_symbol():
     assert set(names) == bound, sorted(set(names) ^ bound)
 
 
+def test_the_version_moves_with_the_structs():
+    """A caller built against another layout finds out by the version: sizes and offsets of what the calls read, as version 3 has them."""
+    assert hip.lib().cavs_abi_version() == 3
+    import ctypes as C
+
+    assert (C.sizeof(hip.Task), C.sizeof(hip.GroupPlan), hip.GroupPlan.tile_rows.offset, C.sizeof(hip.ColsumDesc)) == (96, 56, 48, 32)
+    assert re.search(r"#define CAVS_ABI_VERSION 3\b", open(hip.HEADER).read())
+
+
 def test_header_cites_the_reference_for_every_entry_group():
     text = open(hip.HEADER).read()
     assert len(re.findall(r"cavs/(backend|midend|util)/[a-z0-9_./]+:\d+", text)) >= 20
