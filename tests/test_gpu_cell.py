@@ -30,7 +30,7 @@ def oracle_step(oracle, w, model, **kw):
                              Cc=w["C"], precise=True, threads=16, **kw)
 
 
-def run_generated(model, w, pairing, mode=2, lr=0.0, root_mask=None):
+def run_generated(model, w, pairing, mode=2, lr=0.0, root_mask=None, counts=None):
     B, maxlen = w["graph"].shape
     a = apps.App(model, B=B, maxlen=maxlen, H=w["H"], E=w["E"], V=w["V"], C_=w["C"], opt=session.OPT_BATCHING, lr=lr,
                  pairing=pairing, allow_fused=mode)
@@ -39,6 +39,8 @@ def run_generated(model, w, pairing, mode=2, lr=0.0, root_mask=None):
     loss, go = a.step(w["graph"], w["x"], w["labels"], train=True, root_mask=root_mask)
     grads = {"d" + k: a.grad(k, np.shape(w["params"][k])) for k in NAMES[model]}
     kind = a.fused_kind
+    if counts is not None:
+        counts.append({k: a.counter(k) for k in ("tail_rounds", "rounds")})
     a.close()
     return loss, go, grads, kind
 

@@ -52,12 +52,13 @@ def test_resident_rounds_give_what_a_launch_per_round_gives(model, H):
     w = small_workload(model, 187, B=60, H=H, E=12, V=29, C=5)
     for k in ("U", "W"):
         w["params"][k] = w["params"][k] * np.float32(0.4 * min(1.0, (64.0 / H) ** 0.5))
-    got = []
+    got, counts = [], []
     for turn in (contextlib.nullcontext, another_process):
         with turn():
             print(f"[case] {model} H={H} {'resident' if turn is contextlib.nullcontext else 'a launch per round'}", flush=True)
-            got.append(run_generated(model, w, "reference", mode=1))
+            got.append(run_generated(model, w, "reference", mode=1, counts=counts))
     assert got[0][3] == got[1][3] == 2
+    assert counts[0]["tail_rounds"] >= 2 * (counts[0]["rounds"] - 2) and counts[1]["tail_rounds"] == 0, counts
     compare(got[0], dict(loss=got[1][0], graph_out=got[1][1], grads=got[1][2]))
 
 
