@@ -612,7 +612,8 @@ static int run_gemm(const char *who, int tA, int tB, int M, int N, int K, float 
 
 // Plans a group: every product on the 64x64 tile, K split so that all workgroups of the group
 // together are about four per CU (what a CU holds at once; inside a training step eight per CU
-// measured no better, though it is in a back-to-back loop), each with at least 256 of K.
+// measured no better, though it is in a back-to-back loop), each with at least 256 of K; 128 where the workgroups
+// are few even so, and a single product is cut as it would be by itself (plan_product).
 // `tail_product` >= 0: that product's result is handed on to the embedding scatter-add (dtable, ids)
 // and `counters` [n_counters]: the group's launch adds up its splits itself where they are enough (GroupFold)
 static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_bytes, size_t *need_out, void *stream,

@@ -31,7 +31,7 @@ enum { GROUP_TREELSTM = 0, GROUP_LSTM = 1, GROUP_TREEFC = 2 };
 
 struct GroupPlan {
   const int4 *groups;  // [ngroups] first list, lists, arrivals
-  const int4 *lists;   // [*] first record, rows, arrivals to wait for, whether it arrives
+  const int4 *lists;   // [*] first record, rows, arrivals to wait for; 1: it arrives, + 2 (backward): rows without a parent
   const int4 *recs;    // [*][2]
   unsigned *sync;
   int ngroups, wgs, spin_max, expect;

@@ -123,7 +123,7 @@ enum CellArg {
   CA_DS,         // float*  [N, SI*H] elementwise part of a vertex's message gradient by slab row; or, for
                  //         cell_bwd_gates / cell_bwd_pool, [K * n, SI*H] by row of the round and child
   CA_BT,         // float*  tile-major copies of the weight blocks: as they are, then transposed
-  CA_COLSUM,     // float*  [ND*H] column sums of D
+  CA_COLSUM,     // float*  [cavs_colsum_parts(N), ND*H] chunk sums of the columns of D (CK_BIAS: their number in CA_N)
   CA_DPOOL,      // float*  gradient of the rows this cell's state goes to [*, S*H] (cell_bwd_gates reads it)
   CA_X,          // float*  the vertex input by vertex id [*, XD*H]
   CA_POOL_IN,    // float*  the rows this cell gathers its children's states from [*, SI*H] (a function of one stage: CA_POOL)

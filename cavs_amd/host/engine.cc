@@ -2674,7 +2674,7 @@ void Engine::head_forward_backward(bool backward) {
     Param &Wfc = param("Wfc"), &bfc = param("bfc");
     const size_t head_bytes = cavs_fc_softmax_xent_workspace(N, H, C);
     if (head_bytes > 0) {  // few classes: the whole head and its gradients in one launch; the sum of
-                           // its weight-gradient partials rides in the launch that opens backward
+                           // its weight-gradient partials rides in the launch that opens backward, or in the update's
       if (head_parts_.capacity() * 4 < head_bytes) {
         check(cavs_stream_sync(stream_));  // the last step's jobs may still read the old buffer
         head_parts_.reserve(head_bytes / 4 + 1);
@@ -2723,8 +2723,12 @@ void Engine::head_forward_backward(bool backward) {
         gemm_group({dGd});
         check(cavs_event_record(aux_fork_ev_, stream_));
         check(cavs_stream_wait_event(aux_stream_, aux_fork_ev_));
-        // (beside the resident launch, one workgroup to a CU with 86 KB of its LDS, plain workgroups find room; with
-        // more LDS they would come after it: C4 2.71 and 2.93 ms)
+        // (beside a resident launch of one workgroup to a CU with 84 KB of its LDS -- all but the Tree-LSTM's with tiles of
+        // sixteen rows at H = 160 .. 256 and 416 .. 512, 128 KB -- plain workgroups find room; with more LDS they would come
+        // after it: 7000 vertices in chains, H = 512, 10000 classes 2.71 and 2.93 ms.  Beside those of 128 KB nothing finds room: what is placed
+        // first holds the others up.  Plain is the better one there too, us a step plain / with more LDS / on the session's stream / with
+        // tiles of four rows: 64 trees, H = 512, 5000 classes 609 / 640 / 623 / 623, 10000 classes 854 / 883 / 858 / 867, 128 trees 1060 / 1144 /
+        // 1078 / 1065; H = 256, 10000 classes 534 / 552 / 536 / 538, 5000 classes 373 / 398 / 363 / 366, 200 trees 870 / 901 / 884 / 886)
         check((group_.first >= 0 ? cavs_sgemm_group : cavs_sgemm_group_beside)(1, &dWd, ws_aux_.get(), ws_aux_.capacity() * 4, aux_stream_));
         c_gemm_flops_ += 2.0 * dWd.M * dWd.N * dWd.K;
         c_launches_ += 1;
@@ -2746,7 +2750,7 @@ void Engine::head_forward_backward(bool backward) {
     c_launches_ += 1;
     const cavs_task sum{CAVS_TASK_SUM_PARTS, 0.f, B, 1, 1, tmp, loss_.get(), nullptr, nullptr};
     if (backward) {
-      pending_tasks_.push_back(sum);  // rides in the launch that opens the backward pass
+      pending_tasks_.push_back(sum);  // rides in the launch that opens the backward pass, or where none does in the update's
     } else {
       check(cavs_run_tasks(1, &sum, stream_));
       c_launches_ += 1;
