@@ -649,8 +649,8 @@ void Engine::reserve_edges() {
     R(dxW_, cap * H);
     R(r_z_, rc * H);
   }
-  group_counters();  // (not first within a recording, where the zeros would come with each replay only)
   words_ = words_wanted();
+  if (trains_ || words_) group_counters();  // (not first within a recording, where the zeros would come with each replay only)
   if (words_) {
     const size_t w = cell_ ? (size_t)cell_->NX * H : 4 * H;
     size_t most = cell_ ? 0 : w;
@@ -698,7 +698,7 @@ void Engine::reserve_group() {
   if (group_.first < 0 || cell_) return;
   const size_t n = (size_t)(cfg_.model == CAVS_MODEL_TREEFC ? 2 : 4) * cfg_.H * cfg_.H;
   ensure(Upk_, n);
-  if (ensure(UTp_, n)) utp_valid_ = false;
+  if (!lists_forward_only() && ensure(UTp_, n)) utp_valid_ = false;
 }
 
 // Whether x * W and its gradients go by words: every different id of the batch once (cavs_embed_index).
