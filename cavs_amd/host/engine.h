@@ -477,6 +477,7 @@ class Engine {
   void tail_check();
   // The same without failing: why a launch gave up (empty: none did).
   std::string tail_settle();
+  bool tail_pending() const { return tail_pending_; }  // such a launch has been enqueued since
   // For tests: the waits of the launches from here on poll `spins` times at most and for `extra` workgroups that do not exist
   // (0: as ever).
   void bound_waits(int spins, int extra);

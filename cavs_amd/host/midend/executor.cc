@@ -841,6 +841,7 @@ void Executor::run(const std::vector<std::string> &outputs, std::vector<HostTens
   for (auto &o : outputs)
     if (!(g.opt.present && o == g.opt.output)) reads = true;
   if (!reads) {
+    keep_host_feeds(parity);
     dirty_ = true;
     return;
   }
@@ -955,17 +956,23 @@ void Executor::remember_run(int parity, const MainProgram *mp, bool train, int p
   r.passes = passes;
   r.serial = passes_run_ + 1;
   r.feeds.clear();
-  size_t hosts = 0;
-  for (auto &f : fed_) {
-    float *base = f.first->base;
-    if (f.second && base) {  // (the caller's memory, which is free again when the Run returns)
-      if (r.host.size() <= hosts) r.host.emplace_back();
-      r.host[hosts].assign(base, base + f.first->width);
-      base = r.host[hosts++].data();
-    }
-    r.feeds.push_back({f.first, base});
-  }
+  for (auto &f : fed_) r.feeds.push_back({f.first, f.first->base});
   r.live = true;
+}
+
+// Of a Run that returns before it is known to have gone through: the caller's memory is free again then.  (Nothing to keep where no
+// launch that can give up is under way.)
+void Executor::keep_host_feeds(int parity) {
+  PastRun &r = past_[parity];
+  if (!r.live) return;
+  r.live = engine_ && engine_->tail_pending();
+  size_t hosts = 0;
+  for (size_t i = 0; r.live && i < fed_.size(); i++) {
+    if (!fed_[i].second || !r.feeds[i].second) continue;
+    if (r.host.size() <= hosts) r.host.emplace_back();
+    r.host[hosts].assign(r.feeds[i].second, r.feeds[i].second + fed_[i].first->width);
+    r.feeds[i].second = r.host[hosts++].data();
+  }
 }
 
 // The last Run of this parity is over.  If its update was held back it is made up for now, while its feeds are there.

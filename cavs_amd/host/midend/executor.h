@@ -166,6 +166,7 @@ class Executor {
   int passes_run_ = 0;
   int spins_ = 0, extra_ = 0;
   void remember_run(int parity, const MainProgram *mp, bool train, int passes);
+  void keep_host_feeds(int parity);
   void confirm(int parity);
   void sync_and_settle();
   void settle();
