@@ -47,7 +47,7 @@ def libs():
 
 
 class App:
-    """model: treelstm | lstm | treefc | treefc_x | treelstm2 | treegate | cell<seed>.  opt: OPT_* bitmask, or -1 to only
+    """model: treelstm | lstm | treefc | treefc_x | treefc_xr | treelstm2 | treegate | cell<seed>.  opt: OPT_* bitmask, or -1 to only
     declare the program (no device)."""
 
     def __init__(self, model, *, B, maxlen, H, E=0, V=0, C_=0, opt=session.OPT_BATCHING, lr=0.0, clip=0.0,
@@ -97,13 +97,13 @@ class App:
         reference apps' loops do, and reads nothing back."""
         a, _ = libs()
         g = np.ascontiguousarray(graph, np.int32)
-        xw = self.H if self.model == "treefc_x" else 1
+        xw = self.H if self.model in ("treefc_x", "treefc_xr") else 1
         if self.model == "treefc":  # the reference Tree-FC app reads no vertex input and no labels
             x = labels = None
-        elif self.model == "treefc_x":
+        elif self.model in ("treefc_x", "treefc_xr"):
             labels = None
         xb, lb = self._placeholder(x, xw), self._placeholder(labels)
-        mb = self._placeholder(root_mask, self.H) if self.model == "treefc_x" else np.zeros(1, np.float32)
+        mb = self._placeholder(root_mask, self.H) if self.model in ("treefc_x", "treefc_xr") else np.zeros(1, np.float32)
         if train and not fetch:
             n = a.cavs_app_step(g.ctypes.data, xb.ctypes.data, lb.ctypes.data, mb.ctypes.data, 1, None, 0, None, 0)
             if n < 0:

@@ -202,7 +202,7 @@ class SeqLSTM : public GraphSupport {
 
 class TreeFC : public GraphSupport {
  public:
-  // variant 0: the reference app (relu, no bias, no vertex input); variant 1: tanh + bias + Pull'ed input
+  // variant 0: the reference app (relu, no bias, no vertex input); variant 1: tanh + bias + Pull'ed input; 2: the same with relu
   TreeFC(const Sym &graph_ph, const Sym &vertex_ph, const Dims &d, int variant)
       : GraphSupport(graph_ph, vertex_ph), H(d.H), variant_(variant) {
     W = Sym::Variable(DT_FLOAT, {2 * H, H}, Sym::Uniform(-0.1f, 0.1f));
@@ -215,7 +215,8 @@ class TreeFC : public GraphSupport {
     Sym res;
     if (variant_) {
       Sym x = Pull(0, {H});
-      res = (fc + Bv.Mirror() + x).Tanh();
+      Sym pre = fc + Bv.Mirror() + x;
+      res = variant_ == 2 ? pre.Relu() : pre.Tanh();
     } else {
       res = fc.Relu();
     }
@@ -405,7 +406,7 @@ App *g_app = nullptr;
 extern "C" {
 
 // model: "treelstm" | "lstm" | "treefc" (reference app) | "treefc_x" (tanh + bias + input, sum of
-// squares at the roots).  Declares the program and opens a session.  One app per process at a time.
+// squares at the roots; "treefc_xr": relu).  Declares the program and opens a session.  One app per process at a time.
 // gradient clipping threshold of the optimizer the next cavs_app_create declares (0: none)
 static float g_clip = 0.f;
 void cavs_app_set_clip(float clip) { g_clip = clip; }
@@ -423,8 +424,8 @@ int cavs_app_create(const char *model, int B, int maxlen, int V, int E, int H, i
     app->model = model;
     const Dims &d = app->d;
     app->graph = Sym::Placeholder(DT_FLOAT, {B, maxlen}, "CPU");
-    bool fc = app->model == "treefc" || app->model == "treefc_x";
-    app->vertex = Sym::Placeholder(DT_FLOAT, app->model == "treefc_x" ? vector<int>{B * maxlen, H} : vector<int>{B, maxlen});
+    const bool fcx = app->model == "treefc_x" || app->model == "treefc_xr", fc = app->model == "treefc" || fcx;
+    app->vertex = Sym::Placeholder(DT_FLOAT, fcx ? vector<int>{B * maxlen, H} : vector<int>{B, maxlen});
     if (!fc) {
       app->label = Sym::Placeholder(DT_FLOAT, {B, maxlen});
       app->weight = Sym::Variable(DT_FLOAT, {C, H}, Sym::Uniform(-0.1f, 0.1f));
@@ -459,10 +460,10 @@ int cavs_app_create(const char *model, int B, int maxlen, int V, int E, int H, i
       app->gs.reset(m);
       app->vars = {{"Emb", m->embedding}, {"W", m->LSTM_w}, {"Bv", m->LSTM_b}};
     } else if (fc) {
-      auto *m = new TreeFC(app->graph, app->vertex, d, app->model == "treefc_x");
+      auto *m = new TreeFC(app->graph, app->vertex, d, !fcx ? 0 : app->model == "treefc_x" ? 1 : 2);
       app->gs.reset(m);
       app->vars = {{"W", m->W}};
-      if (app->model == "treefc_x") app->vars.push_back({"Bv", m->Bv});
+      if (fcx) app->vars.push_back({"Bv", m->Bv});
     } else {
       return -1;
     }
@@ -474,7 +475,7 @@ int cavs_app_create(const char *model, int B, int maxlen, int V, int E, int H, i
       label_reshape.ControlDependency(app->graph_output);
       app->loss = app->graph_output.FullyConnected(app->weight, app->bias).SoftmaxEntropyLoss(label_reshape);
       app->total = app->loss.Reduce_mean();
-    } else if (app->model == "treefc_x") {
+    } else if (fcx) {
       app->mask = Sym::Placeholder(DT_FLOAT, {B * maxlen, H});
       Sym mask_rows = app->mask.Reshape({-1, H});
       mask_rows.ControlDependency(app->graph_output);
@@ -524,10 +525,10 @@ long cavs_app_step(const int *graph, const float *x, const float *labels, const 
   try {
     App &a = *g_app;
     vector<std::pair<Sym, void *>> feeds = {{a.graph, (void *)graph}};
-    bool fc = a.model == "treefc" || a.model == "treefc_x";
-    if (!fc || a.model == "treefc_x") feeds.push_back({a.vertex, (void *)x});
+    const bool fcx = a.model == "treefc_x" || a.model == "treefc_xr", fc = a.model == "treefc" || fcx;
+    if (!fc || fcx) feeds.push_back({a.vertex, (void *)x});
     if (!fc) feeds.push_back({a.label, (void *)labels});
-    if (a.model == "treefc_x") feeds.push_back({a.mask, (void *)mask});
+    if (fcx) feeds.push_back({a.mask, (void *)mask});
     vector<Sym> outs;
     if (train) outs.push_back(a.train);
     if (train && !loss_out && !go_out) {  // as the reference apps loop: sess.Run({train}, feeds), nothing read back

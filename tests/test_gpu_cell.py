@@ -15,7 +15,7 @@ from tolerance import close
 pytestmark = pytest.mark.gpu
 
 NAMES = {"treelstm": ("Emb", "W", "U", "Bv", "Wfc", "bfc"), "treelstm2": ("Emb", "W", "U", "Bv", "Wfc", "bfc"),
-         "treegate": ("Emb", "W", "U", "Bv", "Wfc", "bfc"), "treegru": ("Emb", "W", "U", "Bv", "Wfc", "bfc"), "treedeep": ("Emb", "W", "U", "Bv", "Wfc", "bfc"), "lstm": ("Emb", "W", "Bv", "Wfc", "bfc"), "treefc": ("W",), "treefc_x": ("W", "Bv")}
+         "treegate": ("Emb", "W", "U", "Bv", "Wfc", "bfc"), "treegru": ("Emb", "W", "U", "Bv", "Wfc", "bfc"), "treedeep": ("Emb", "W", "U", "Bv", "Wfc", "bfc"), "lstm": ("Emb", "W", "Bv", "Wfc", "bfc"), "treefc": ("W",), "treefc_x": ("W", "Bv"), "treefc_xr": ("W", "Bv")}
 
 
 @pytest.fixture(scope="module", autouse=True)

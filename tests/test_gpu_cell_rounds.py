@@ -101,3 +101,42 @@ def test_what_a_launch_that_gives_up_holds_back_is_run_again(model, H, mode, ite
         assert np.abs(want[k] - params[k].reshape(want[k].shape)).max() > 1e-4, f"{k} does not move"
         close(values[k], want[k], k)
         close(grads[k], want_grads[k], "d" + k)
+
+
+def _trees_of_three_rounds(H, B=9):
+    """Vertices of a sample: leaves 0, 1, 3, inner 2 = (0, 1), root 4 = (2, 3)"""
+    graph = np.tile(np.array([2, 2, 4, 4, -1], np.int32), (B, 1))
+    rng = np.random.default_rng(H)
+    params = dict(W=rng.uniform(-0.3, 0.3, (2 * H, H)).astype(np.float32), Bv=rng.uniform(0.1, 0.2, H).astype(np.float32))
+    x, mask = rng.uniform(0.1, 0.5, (5 * B, H)).astype(np.float32), np.zeros((5 * B, H), np.float32)
+    mask[4::5] = 1
+    return dict(graph=graph, x=x, labels=None, params=params, H=H, E=0, V=0, C=0, N=5 * B), mask
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [32, 64, 160, 288])
+@pytest.mark.parametrize("where", ["state", "gradient"])
+def test_an_infinity_reaches_what_multiplies_it_and_nothing_else(where, H):
+    """Hidden sizes at which some wavefronts have no column to multiply, or fewer than others: an infinite state of one leaf (the first
+    column, which such a wavefront reads all the same) makes its parent's row infinite or zero, an infinite gradient at one root
+    an infinite gradient below, and neither a NaN -- as a launch per round has it."""
+    w, mask = _trees_of_three_rounds(H)
+    if where == "state":
+        w["x"][0, 0] = np.inf
+    else:
+        mask[4, 0], w["x"][4, 0] = np.inf, 100.0  # (a column that relu passes)
+    got, counts = [], []
+    for turn in (contextlib.nullcontext, another_process):
+        with turn():
+            print(f"[case] infinite {where} H={H} {'resident' if turn is contextlib.nullcontext else 'a launch per round'}", flush=True)
+            got.append(run_generated("treefc_xr", w, "rowid", mode=2, root_mask=mask, counts=counts))
+    assert got[0][3] == got[1][3] == 2 and counts[0]["tail_rounds"] > 0 == counts[1]["tail_rounds"], counts
+    go = got[0][1].reshape(-1, 5, H)
+    assert not np.isnan(go[0, 2]).any() and np.isfinite(go[1:]).all()
+    if where == "state":
+        assert (go[0, 2] == np.where(w["params"]["W"][0] > 0, np.inf, 0)).all()
+    else:
+        assert not np.isnan(got[0][2]["dW"][:, 1:]).any() and np.isinf(got[0][2]["dW"][:, 1:]).any()
+    for a, b in zip([got[0][1]] + list(got[0][2].values()), [got[1][1]] + list(got[1][2].values())):
+        np.testing.assert_array_equal(np.isnan(a), np.isnan(b))
+        close(np.where(np.isfinite(a), a, np.sign(np.nan_to_num(a, nan=0.0))), np.where(np.isfinite(b), b, np.sign(np.nan_to_num(b, nan=0.0))))
