@@ -161,6 +161,12 @@ struct GroupBwdArgs {
 }  // namespace cavs
 
 namespace cavs {
+// mask: 0 or -1, made where the compiler cannot see which (an empty asm): of values that have just been loaded it would make a
+// select with branches
+__device__ inline float4 and4(int mask, const float4 &v) {
+  return make_float4(__int_as_float(__float_as_int(v.x) & mask), __int_as_float(__float_as_int(v.y) & mask), __int_as_float(__float_as_int(v.z) & mask),
+                     __int_as_float(__float_as_int(v.w) & mask));
+}
 __device__ inline float4 sel4(bool on, const float4 &v) { return on ? v : zero4(); }
 }  // namespace cavs
 
@@ -209,9 +215,11 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
 #pragma unroll
     for (int k = 0; k < (MODEL == GROUP_TREEFC ? 1 : 4); k++) bias[k] = a.bias[k * H + ej];
   }
-  // where this lane's float4 of an operand row is (CAVS_MMA4's layout); lanes of k-groups beyond the wavefront's read the row's start
+  // where this lane's float4 of an operand row is (CAVS_MMA4's layout); lanes of k-groups beyond the wavefront's read the row's start and
+  // drop it (their weights are zero, but zero times an infinity is a NaN)
   const int og = (lane >> 2) & 3, okg = ks * GPW + og;
-  const int ka = og < GPW && okg < KG ? 16 * okg + 4 * slot : 0;
+  const bool inside = og < GPW && okg < KG;
+  const int ka = inside ? 16 * okg + 4 * slot : 0;
   WideFwd<MODEL, GPW> wide(a, __builtin_amdgcn_readfirstlane(ks), lane, red);
   bool begun = false;  // (WIDE) the first tile's rows have been asked for
   __syncthreads();
@@ -248,7 +256,7 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
 #pragma unroll
       for (int k = 0; k < NC; k++) {
         const int row = k == 0 ? c.y : c.z;
-        o.on[k] = row >= 0;
+        o.on[k] = row >= 0 && inside;
         o.v[k] = ld4((row >= 0 ? a.pool + row * MW : a.Wp) + ka);
       }
     };
@@ -405,10 +413,18 @@ __global__ __launch_bounds__(512, 1) void group_bwd_kernel(GroupBwdArgs a) {
   else __builtin_amdgcn_s_setprio(2);
   const int og = (lane >> 2) & 3;
   int kl[Q];  // this lane's float4 of a row of dA
+  int in[Q];  // (a mask: as in the forward kernel)
 #pragma unroll
-  for (int q = 0; q < Q; q++) kl[q] = 4 * q + og < NL && ks * NL + 4 * q + og < LG ? 16 * (ks * NL + 4 * q + og) + 4 * slot : 0;
-  const int kf = og < GPW && ks * GPW + og < KG ? 16 * (ks * GPW + og) + 4 * slot : 0;  // of a row of dF
+  for (int q = 0; q < Q; q++) {
+    in[q] = 4 * q + og < NL && ks * NL + 4 * q + og < LG ? -1 : 0;
+    kl[q] = in[q] ? 16 * (ks * NL + 4 * q + og) + 4 * slot : 0;
+    asm("" : "+v"(in[q]));
+  }
+  int in_f = og < GPW && ks * GPW + og < KG ? -1 : 0;
+  const int kf = in_f ? 16 * (ks * GPW + og) + 4 * slot : 0;  // of a row of dF
+  asm("" : "+v"(in_f));
   WideBwd<MODEL, GPW> wide(a, __builtin_amdgcn_readfirstlane(ks), lane, red);
+  if constexpr (WIDE) wide.clear();
   bool begun = false;  // (as in the forward kernel)
   __syncthreads();
 
@@ -492,6 +508,12 @@ __global__ __launch_bounds__(512, 1) void group_bwd_kernel(GroupBwdArgs a) {
     if (4 * TW < T) fetch(4 * TW, o);
     for (int t = 4 * TW; t < T; t++) {
       fetch(t + 1, nx);
+#pragma unroll
+      for (int q = 0; q < Q; q++) o.l[q] = and4(in[q], o.l[q]);
+      if constexpr (MODEL == GROUP_TREELSTM) {
+        o.f[0] = and4(in_f, o.f[0]);
+        o.f[1] = and4(in_f, o.f[1]);
+      }
       // (the long product in two accumulators: each MFMA would wait for the one before otherwise)
       floatx4 acc[NP], two = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll

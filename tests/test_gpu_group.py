@@ -87,3 +87,35 @@ def test_a_wait_that_gives_up_leaves_the_launch():
                    g.stream())
     finally:
         g.release()
+
+
+@pytest.mark.parametrize("H", [32, 96, 160, 288, 512])
+@pytest.mark.parametrize("trees", [1, 20])
+def test_an_infinity_reaches_what_multiplies_it_and_nothing_else(trees, H):
+    """Tree-FC with relu, whose states have no bound.  Where some wavefronts have no column to multiply, or fewer than others, they read the
+    first ones all the same: an infinite state of a leaf (forward) and an infinite gradient of a root (backward) come out as with a launch per
+    round, in tiles of four rows (a tree a group) and of sixteen."""
+    rng, B = np.random.default_rng(H), min(1900, trees * hip.lib().cavs_group_max_groups(H))
+    graph = np.tile(np.array([2, 2, 4, 4, -1], np.int32), (B, 1))  # leaves 0, 1, 3, inner 2 = (0, 1), root 4 = (2, 3)
+    params = dict(W=rng.uniform(-0.3, 0.3, (2 * H, H)).astype(np.float32), Bv=rng.uniform(0.1, 0.2, H).astype(np.float32))
+    for at in (0, 4):
+        x = rng.uniform(0.1, 0.5, (5 * B, H)).astype(np.float32)
+        x[at, 0] = np.inf
+        out = []
+        for kw in ({}, dict(tail_rows=-1)):
+            print(f"[case] H={H} B={B} infinite {'state' if at == 0 else 'gradient'} {kw}", flush=True)
+            s = session.Session("treefc", H=H, E=0, V=0, C_=0, loss="root_sq", act=0, use_bias=True, use_x=True, **kw)
+            s.set_params(params)
+            s.step(graph, x, None, backward=True)
+            assert (s.counter("tail_rounds") > 0) == (not kw)
+            out.append([s.fetch("graph_out")] + list(s.grads().values()))
+            s.close()
+        go = out[0][0].reshape(B, 5, H)
+        assert np.isfinite(go[1:]).all() and not np.isnan(go[0, 2]).any()
+        if at == 0:
+            assert (go[0, 2] == np.where(params["W"][0] > 0, np.inf, 0)).all()
+        for a, b in zip(*out):
+            np.testing.assert_array_equal(np.isnan(a), np.isnan(b))
+            ok = np.isfinite(b)
+            np.testing.assert_array_equal(np.isfinite(a), ok)
+            close(np.where(ok, a, 0), np.where(ok, b, 0))
