@@ -12,7 +12,7 @@
 //     32 bytes per row, built on the host and fetched a round ahead: no chain of index loads
 //     stands between two rounds;
 //   * the plan is read from memory, so a launch runs any number of rounds (chains of hundreds).
-// A wavefront owns ceil(H / 128) k-groups of 16 of its workgroup's columns; those beyond H multiply by zero weights.
+// A wavefront owns ceil(H / 128) k-groups of 16 of its workgroup's columns; those beyond H are dropped.
 #pragma once
 #include <algorithm>
 #include <type_traits>
