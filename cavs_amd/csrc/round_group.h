@@ -55,6 +55,12 @@ __device__ inline int4 plan_row(const int4 *p) {
   return int4{v[0], v[1], v[2], v[3]};
 }
 
+// A load is waited for here: the wait behind a branch further down would be for everything that may be under way by then
+__device__ inline void arrived(float v) { asm volatile("" ::"v"(v)); }
+// row * ld floats behind p: one multiplication of 32 bits (row >= 0)
+template <class T>
+__device__ inline T *row_at(T *p, int row, unsigned ld) { return p + (size_t)(unsigned)row * ld; }
+
 // What every list of a launch goes through besides its products: the plan, the records of the next
 // list on their way while this one runs, and the group's barrier.
 struct GroupWalk {
@@ -63,6 +69,7 @@ struct GroupWalk {
   int nlists, ct;
   unsigned arrived;
   int4 cur, nxt, ahead, rec;
+  unsigned words;  // the group's, as they were when the list began
   bool first_wait;
   __device__ inline bool start(const GroupPlan &p, int4 (*s_rec)[2 * kGroupRows], int *s_bail) {
     const int idx = blockIdx.x >> 3, grp = (blockIdx.x & 7) + 8 * (idx / p.wgs);  // workgroup b sits on XCD b % 8
@@ -82,36 +89,49 @@ struct GroupWalk {
     if (threadIdx.x == 0) *s_bail = 0;
     cur = plan_row(lists);
     nxt = plan_row(lists + (nlists > 1 ? 1 : 0));
-    if (threadIdx.x < 2 * kGroupRows) s_rec[0][threadIdx.x] = record(cur);
+    put(s_rec[0], cur, record(cur));
     if (threadIdx.x == 0) __hip_atomic_fetch_or(gsync + TAIL_XCC, 1u << xcc_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return true;
   }
+  // half a record to a thread, the same to every wavefront (of a row beyond the list's: its first row's)
   __device__ inline int4 record(const int4 &list) const {
-    const int i = threadIdx.x >> 1;
-    return i < list.y ? recs[2L * (list.x + i) + (threadIdx.x & 1)] : int4{-1, -1, -1, -1};
+    const int i = (threadIdx.x & 63) >> 1;
+    return recs[2L * (list.x + (i < list.y ? i : 0)) + (threadIdx.x & 1)];
   }
-  __device__ inline void fetch_next(int r) {
-    ahead = plan_row(lists + (r + 2 < nlists ? r + 2 : nlists - 1));
-    if (threadIdx.x < 2 * kGroupRows) rec = record(nxt);
+  __device__ inline void put(int4 *to, const int4 &list, const int4 &v) const {
+    if (threadIdx.x < 2 * kGroupRows) to[threadIdx.x] = (int)(threadIdx.x >> 1) < list.y ? v : int4{-1, -1, -1, -1};
+  }
+  // A list begins: the group's words, then what its gate functions and the lists behind it read of the launches before.  Loads come
+  // back in the order they were made, and those go to memory: with the words behind them, the words were another trip; so they are asked
+  // for first and looked at when the addresses are done.  Nothing here is conditional, or the waits, which then have to hold for
+  // either way, would be for everything: a wavefront without rows asks for what the list's first needs.
+  // Cycles from list to list, 16 chains of 20, H = 128: 4200 forward and 3850 backward -> 3550 and 3250 (with the last tile of a list by
+  // itself: 300 of them).  Passes of 16 steps: those chains 2527 -> 2430 us, Tree-FC, 64 trees, H = 256 2152 -> 1968; 37 chains,
+  // H = 200, one step with its gradients 635 -> 616.
+  __device__ inline void begin(const GroupPlan &p, int r) {
+    words = tail_ask(gsync, p.expect);
+    ahead = lists[r + 2 < nlists ? r + 2 : nlists - 1];  // (not by the scalar unit: waits for LDS would be for it too)
+    rec = record(nxt);
   }
   // (where there is nothing to wait for, the barrier at the end of the list before is enough; a wait that gives up
   // sets *s_bail, looked at behind the barrier that completes the partial sums)
   __device__ inline void wait(const GroupPlan &p, int *s_bail) {
     if (cur.z <= 0) return;
-    tail_wait(status, gsync, (unsigned)cur.z, p.expect, p.spin_max, first_wait, p.whole_lines, s_bail);
+    if (first_wait || !p.whole_lines || !__all(words >= (unsigned)cur.z))
+      tail_wait(status, gsync, (unsigned)cur.z, p.expect, p.spin_max, first_wait, p.whole_lines, s_bail);
+    asm volatile("" ::: "memory");  // (what the others wrote is read after this)
     first_wait = false;
   }
   // before the barrier that completes the list's partial sums
-  __device__ inline void keep_next(int r, int4 (*s_rec)[2 * kGroupRows]) const {
-    if (threadIdx.x < 2 * kGroupRows) s_rec[(r + 1) & 1][threadIdx.x] = rec;
-  }
+  __device__ inline void keep_next(int r, int4 (*s_rec)[2 * kGroupRows]) const { put(s_rec[(r + 1) & 1], nxt, rec); }
   __device__ inline void done() {
     if (cur.w & 1) tail_arrive(gsync, ct, ++arrived);
     else __syncthreads();
   }
   __device__ inline void advance() {
     cur = nxt;
-    nxt = ahead;
+    nxt = int4{__builtin_amdgcn_readfirstlane(ahead.x), __builtin_amdgcn_readfirstlane(ahead.y), __builtin_amdgcn_readfirstlane(ahead.z),
+               __builtin_amdgcn_readfirstlane(ahead.w)};
   }
 };
 
@@ -224,26 +244,24 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
   bool begun = false;  // (WIDE) the first tile's rows have been asked for
   __syncthreads();
 
+  const float *x_rows = MODEL == GROUP_TREEFC && !a.xW ? a.Wp : a.xW;
+  const unsigned x_ld = MODEL == GROUP_TREEFC && !a.xW ? 0 : (unsigned)a.ld_xw;
   for (int r = 0; r < w.nlists; r++) {
     const int4 *rt = s_rec[r & 1];
     const int n = w.cur.y < kGroupRows ? w.cur.y : kGroupRows, T = (n + 3) >> 2, TW = WIDE ? wide_tiles(n) : 0;
-    w.fetch_next(r);
-    // what does not depend on the rounds before
+    w.begin(a.plan, r);
+    // what does not depend on the rounds before (a wavefront without rows reads the first one's: see begin())
     const int eb = 4 * ks + slot;
     const bool eon = eb < n;
-    int4 rec{-1, -1, -1, -1};
-    int e_out = -1;
+    int4 rec = rt[eon ? 2 * eb : 0];
+    const int e_out = a.go && eon ? rt[2 * eb + 1].x : -1;
     float xw[4] = {0.f, 0.f, 0.f, 0.f};
-    if (eon) {
-      rec = rt[2 * eb];
-      e_out = a.go ? rt[2 * eb + 1].x : -1;
-      if (MODEL != GROUP_TREEFC || a.xW) {
-        const float *p = a.xW + rec.x * a.ld_xw + ej;
+    {
+      const float *p = row_at(x_rows, max(rec.x, 0), x_ld) + ej;
 #pragma unroll
-        for (int k = 0; k < (MODEL == GROUP_TREEFC ? 1 : 4); k++) xw[k] = p[k * H];
-      }
+      for (int k = 0; k < (MODEL == GROUP_TREEFC ? 1 : 4); k++) xw[k] = p[k * H];
     }
-    w.wait(a.plan, &s_bail);
+    if (!eon) rec = int4{-1, -1, -1, -1};
 
     // Operand rows, one float4 per child and tile, unconditionally (a missing child reads weights and is
     // masked); the next tile's are on their way while a tile is multiplied.
@@ -251,33 +269,21 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
       float4 v[NC];
       bool on[NC];
     };
-    auto fetch = [&](int t, Opnd &o) {
-      const int4 c = rt[2 * (4 * (t < T ? t : T - 1) + (lane & 3))];
+    const float *at[NC], *kid[NC];
+    auto rows = [&](int t, Opnd &o) {
+      const int4 c = rt[2 * (4 * t + (lane & 3))];
 #pragma unroll
       for (int k = 0; k < NC; k++) {
         const int row = k == 0 ? c.y : c.z;
         o.on[k] = row >= 0 && inside;
-        o.v[k] = ld4((row >= 0 ? a.pool + row * MW : a.Wp) + ka);
+        at[k] = (row >= 0 ? row_at(a.pool, row, MW) : a.Wp) + ka;
       }
     };
-    Opnd o, nx;
-    if (WIDE && TW > 0 && !begun) wide.fetch(a, rt, n, 0, MW);
-    if (!WIDE || 4 * TW < T) fetch(4 * TW, o);
-    // the epilogue's children
-    float e_h[NC], e_c[NC];
+    auto fetch = [&](Opnd &o) {
 #pragma unroll
-    for (int k = 0; k < NC; k++) {
-      const int row = k == 0 ? rec.y : rec.z;
-      e_h[k] = e_c[k] = 0.f;
-      if (row >= 0) {
-        e_h[k] = ld_row(a.pool + row * MW + ej);
-        if (MODEL != GROUP_TREEFC) e_c[k] = ld_row(a.pool + row * MW + H + ej);
-      }
-    }
-    if constexpr (WIDE)
-      for (int t = 0; t < TW; t++) wide.tile(a, rt, n, t, t + 1 < TW, MW, wt, red);
-    for (int t = 4 * TW; t < T; t++) {
-      fetch(t + 1, nx);
+      for (int k = 0; k < NC; k++) o.v[k] = ld4(at[k]);
+    };
+    auto multiply = [&](int t, const Opnd &o) {
       floatx4 acc[NP];
 #pragma unroll
       for (int p = 0; p < NP; p++) acc[p] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -306,8 +312,36 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
       sums.take(acc);
       sums.all();
       group_park<NP>(red, sums, t, ks, slot, x);
-      o = nx;
+    };
+    Opnd o, nx;
+    const bool fours = 4 * TW < T;
+    if (fours) rows(4 * TW, o);
+#pragma unroll
+    for (int k = 0; k < NC; k++) {  // the element's children
+      const int row = k == 0 ? rec.y : rec.z;
+      kid[k] = (row >= 0 ? row_at(a.pool, row, MW) : a.Wp) + ej;
     }
+    w.wait(a.plan, &s_bail);
+    if (WIDE && TW > 0 && !begun) wide.fetch(a, rt, n, 0, MW);
+    if (fours) fetch(o);
+    float e_h[NC], e_c[NC];
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+      e_h[k] = ld_row(kid[k]);
+      e_c[k] = MODEL != GROUP_TREEFC ? ld_row(kid[k] + H) : 0.f;
+    }
+    if constexpr (WIDE)
+      for (int t = 0; t < TW; t++) wide.tile(a, rt, n, t, t + 1 < TW, MW, wt, red);
+    if (fours) {
+      for (int t = 4 * TW; t + 1 < T; t++) {
+        rows(t + 1, nx);
+        fetch(nx);
+        multiply(t, o);
+        o = nx;
+      }
+      multiply(T - 1, o);  // (by itself: in the loop it would wait for a fetch of its own successor)
+    }
+    arrived(MODEL != GROUP_TREEFC ? e_c[NC - 1] : e_h[NC - 1]);
     w.keep_next(r, s_rec);
     __syncthreads();
     if (s_bail) return;
@@ -317,6 +351,12 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
       if (begun) wide.fetch(a, s_rec[(r + 1) & 1], w.nxt.y < kGroupRows ? w.nxt.y : kGroupRows, 0, MW);
     }
 
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+      const bool on = (k == 0 ? rec.y : rec.z) >= 0;
+      e_h[k] = on ? e_h[k] : 0.f;
+      e_c[k] = on ? e_c[k] : 0.f;
+    }
     float st[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, h = 0.f, cc = 0.f;  // what the backward pass wants, and the state
     if (eon) {
       float v[NP];
@@ -433,81 +473,71 @@ __global__ __launch_bounds__(512, 1) void group_bwd_kernel(GroupBwdArgs a) {
     // (rows without a parent: nothing to multiply, nothing sent to them)
     const bool alone = w.cur.w & 2;
     const int n = w.cur.y < kGroupRows ? w.cur.y : kGroupRows, T = alone ? 0 : (n + 3) >> 2, TW = WIDE && !alone ? wide_tiles(n) : 0;
-    w.fetch_next(r);
-    // the operands of the children's pointwise part: everything but d c of the parent was written before this launch
+    w.begin(a.plan, r);
+    // the operands of the children's pointwise part: everything but d c of the parent was written before this launch (a wavefront
+    // without rows reads the first one's, a missing child and the states of a leaf's children what is there)
     const int eb = 4 * ks + slot;
     const bool eon = eb < n;
-    int4 rec{-1, -1, -1, -1};
+    const int4 rec = rt[eon ? 2 * eb : 0];
     int kid[NC], kdr[NC];
     float pf[NC];
     struct Kid {
       float g[NG], dr, c[2];
     } kd[NC];
-#pragma unroll
-    for (int k = 0; k < NC; k++) kid[k] = kdr[k] = -1, pf[k] = 0.f;
-    if (eon) {
-      rec = rt[2 * eb];
-      kid[0] = rec.y;
-      kdr[0] = rec.w;
-      if constexpr (NC == 2) {
-        kid[NC - 1] = rec.z;
-        kdr[NC - 1] = rt[2 * eb + 1].x;
-      }
-      if (alone) {
-      } else if constexpr (MODEL == GROUP_TREELSTM) {
-        pf[0] = a.gates[(long)rec.x * 6 * H + 3 * H + ej];
-        pf[NC - 1] = a.gates[(long)rec.x * 6 * H + 4 * H + ej];
-      } else if constexpr (MODEL == GROUP_LSTM) {
-        pf[0] = a.gates[(long)rec.x * 5 * H + H + ej];
-      }
+    kid[0] = rec.y;
+    kdr[0] = rec.w;
+    if constexpr (NC == 2) {
+      kid[NC - 1] = rec.z;
+      kdr[NC - 1] = rt[eon ? 2 * eb + 1 : 1].x;
+    }
+    const int parent = max(rec.x, 0);
+    pf[0] = pf[NC - 1] = 0.f;
+    if constexpr (MODEL == GROUP_TREELSTM) {
+      pf[0] = row_at(a.gates, parent, 6 * H)[3 * H + ej];
+      pf[NC - 1] = row_at(a.gates, parent, 6 * H)[4 * H + ej];
+    } else if constexpr (MODEL == GROUP_LSTM) {
+      pf[0] = row_at(a.gates, parent, 5 * H)[H + ej];
     }
 #pragma unroll
     for (int s = 0; s < NC; s++) {
       Kid &q = kd[s];
-#pragma unroll
-      for (int t = 0; t < NG; t++) q.g[t] = 0.f;
-      q.dr = q.c[0] = q.c[1] = 0.f;
-      const long v = kid[s];
-      if (v < 0) continue;
-      q.dr = a.dret[(long)kdr[s] * H + ej];
+      q.c[0] = q.c[1] = 0.f;
+      const int v = max(kid[s], 0);
+      q.dr = row_at(a.dret, max(kdr[s], 0), H)[ej];
       if constexpr (MODEL == GROUP_TREEFC) {
-        q.g[0] = a.h[v * H + ej];
+        q.g[0] = row_at(a.h, v, H)[ej];
       } else {
+        const float *g = row_at(a.gates, v, NG * H) + ej;
+        long to_c = v >= a.leaf_rows ? reinterpret_cast<const char *>(row_at(a.G, v, NC * 2 * H) + H + ej) - reinterpret_cast<const char *>(g) : 0;
+        asm("" : "+v"(to_c));  // (or it is a branch, and waits with it)
+        const float *c = reinterpret_cast<const float *>(reinterpret_cast<const char *>(g) + to_c);
 #pragma unroll
-        for (int t = 0; t < NG; t++) q.g[t] = a.gates[v * NG * H + (long)t * H + ej];
-        if (v >= a.leaf_rows) {
+        for (int t = 0; t < NG; t++) q.g[t] = g[(long)t * H];
 #pragma unroll
-          for (int t = 0; t < NC; t++) q.c[t] = a.G[(NC * v + t) * 2 * H + H + ej];
-        }
+        for (int t = 0; t < NC; t++) q.c[t] = c[t * (NG == 6 ? 2 * H : 0)];
       }
     }
-    w.wait(a.plan, &s_bail);
-    float pdc = 0.f;
-    if (MODEL != GROUP_TREEFC && eon && !alone) pdc = ld_row(a.dc + (long)rec.x * H + ej);
 
     struct Opnd {
       float4 l[Q], f[2];
     };
-    auto fetch = [&](int t, Opnd &o) {
+    const float *at_l = nullptr, *at_f = nullptr;
+    auto rows = [&](int t) {
       // (rows past the list's end stand for its first row; their results are not written)
-      const int i = 4 * (t < T ? t : T - 1) + (lane & 3);
-      const long row = rt[2 * (i < n ? i : 0)].x;
-      const float *p = a.dA + row * a.ld;
+      const int i = 4 * t + (lane & 3);
+      const int row = rt[2 * (i < n ? i : 0)].x;
+      at_l = row_at(a.dA, row, a.ld);
+      if constexpr (MODEL == GROUP_TREELSTM) at_f = row_at(a.dF, row, 2 * H) + kf;
+    };
+    auto fetch = [&](Opnd &o) {
 #pragma unroll
-      for (int q = 0; q < Q; q++) o.l[q] = ld4(p + kl[q]);
+      for (int q = 0; q < Q; q++) o.l[q] = ld4(at_l + kl[q]);
       if constexpr (MODEL == GROUP_TREELSTM) {
-        o.f[0] = ld4(a.dF + 2 * row * H + kf);
-        o.f[1] = ld4(a.dF + (2 * row + 1) * H + kf);
+        o.f[0] = ld4(at_f);
+        o.f[1] = ld4(at_f + H);
       }
     };
-    Opnd o, nx;
-    if constexpr (WIDE) {
-      if (TW > 0 && !begun) wide.start(a, rt, n);
-      for (int t = 0; t < TW; t++) wide.tile(a, rt, n, t, t + 1 < TW, wl, ws, red);
-    }
-    if (4 * TW < T) fetch(4 * TW, o);
-    for (int t = 4 * TW; t < T; t++) {
-      fetch(t + 1, nx);
+    auto multiply = [&](int t, Opnd &o) {
 #pragma unroll
       for (int q = 0; q < Q; q++) o.l[q] = and4(in[q], o.l[q]);
       if constexpr (MODEL == GROUP_TREELSTM) {
@@ -550,8 +580,32 @@ __global__ __launch_bounds__(512, 1) void group_bwd_kernel(GroupBwdArgs a) {
       sums.take(acc);
       sums.all();
       group_park<NP>(red, sums, t, ks, slot, x);
-      o = nx;
+    };
+    Opnd o, nx;
+    const bool fours = 4 * TW < T;
+    constexpr bool kEarly = !(WIDE && MODEL == GROUP_TREELSTM && GPW == 4);  // (its registers are full)
+    if (kEarly && fours) rows(4 * TW);
+    w.wait(a.plan, &s_bail);
+    if constexpr (WIDE) {
+      if (TW > 0 && !begun) wide.start(a, rt, n);
     }
+    if (!kEarly && fours) rows(4 * TW);
+    if (fours) fetch(o);
+    float pdc = 0.f;
+    if (MODEL != GROUP_TREEFC) pdc = ld_row((alone ? a.gates : row_at(a.dc, parent, H)) + ej);  // (never a row before its round: ld_row)
+    if constexpr (WIDE)
+      for (int t = 0; t < TW; t++) wide.tile(a, rt, n, t, t + 1 < TW, wl, ws, red);
+    if (fours) {
+      for (int t = 4 * TW; t + 1 < T; t++) {
+        rows(t + 1);
+        fetch(nx);
+        multiply(t, o);
+        o = nx;
+      }
+      multiply(T - 1, o);
+    }
+    arrived(MODEL != GROUP_TREEFC ? pdc : kd[NC - 1].g[0]);
+    if (alone) pdc = pf[0] = pf[NC - 1] = 0.f;
     w.keep_next(r, s_rec);
     __syncthreads();
     if (s_bail) return;
@@ -566,25 +620,29 @@ __global__ __launch_bounds__(512, 1) void group_bwd_kernel(GroupBwdArgs a) {
       for (int p = 0; p < NP; p++) v[p] = 0.f;
       if (WIDE && ks < 4 * TW) wide_sum<NP>(red, ks, lane, v);
       else if (!alone) group_sum<NP>(red, ks, slot, x, v);
+      int ee = ej;
+      if (!kEarly) asm volatile("" : "+v"(ee));  // (or the rows' addresses are kept from list to list, in scratch memory)
 #pragma unroll
       for (int s = 0; s < NC; s++) {
-        const long c = kid[s];
+        const int c = kid[s];
         if (c < 0) continue;
-        const Kid &q = kd[s];
-        float *d = a.dA + c * a.ld + ej;
+        Kid &q = kd[s];
+        if (c < a.leaf_rows) q.c[0] = q.c[1] = 0.f;
+        float *d = row_at(a.dA, c, a.ld) + ee;
         if constexpr (MODEL == GROUP_TREELSTM) {
           const GateGrad gg = gate_grad(q.g[0], q.g[1 % NG], q.g[2 % NG], q.g[3 % NG], q.g[4 % NG], q.g[5 % NG], v[0] + v[(1 + s) % NP],
                                         pdc * pf[s], q.dr, q.c[0], q.c[1]);
           d[0] = gg.di; d[H] = gg.d_o; d[2 * H] = gg.du; d[3 * H] = gg.dfl + gg.dfr;
           if (c >= a.leaf_rows) {
-            a.dF[(2 * c) * H + ej] = gg.dfl;
-            a.dF[(2 * c + 1) * H + ej] = gg.dfr;
-            a.dc[c * H + ej] = gg.dc;
+            float *f = row_at(a.dF, c, 2 * H) + ee;
+            f[0] = gg.dfl;
+            f[H] = gg.dfr;
+            row_at(a.dc, c, H)[ee] = gg.dc;
           }
         } else if constexpr (MODEL == GROUP_LSTM) {
           const LstmGateGrad gg = lstm_gate_grad(q.g[0], q.g[1 % NG], q.g[2 % NG], q.g[3 % NG], q.g[4 % NG], v[0], pdc * pf[0], q.dr, q.c[0]);
           d[0] = gg.di; d[H] = gg.df; d[2 * H] = gg.du; d[3 * H] = gg.d_o;
-          if (c >= a.leaf_rows) a.dc[c * H + ej] = gg.dc;
+          if (c >= a.leaf_rows) row_at(a.dc, c, H)[ee] = gg.dc;
         } else {
           d[0] = treefc_dz(v[s % NP] + q.dr, q.g[0], a.act);
         }

@@ -28,6 +28,14 @@ __device__ inline void tail_arrive(unsigned *gsync, int wg, unsigned arrivals) {
   if (threadIdx.x == 0) __hip_atomic_store(gsync + TAIL_FLAGS + wg, arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// The words of the group's first `expect` (at most 64) workgroups, a lane's each (the others': as if there): asked for here,
+// looked at by who has done something else in between.
+__device__ inline unsigned tail_ask(const unsigned *gsync, int expect) {
+  const int lane = threadIdx.x & 63;
+  const unsigned v = __hip_atomic_load(gsync + TAIL_FLAGS + (lane < expect ? lane : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return lane < expect ? v : ~0u;
+}
+
 // Waits until the group's first `expect` (at most 64) workgroups have arrived `target` times; no barrier of the
 // workgroup.  Where the wait gives up (spin_max polls, or another workgroup already did, or the group's
 // workgroups turned out to sit on more than one XCD: the status word says why) *s_bail is set, and the

@@ -126,9 +126,9 @@ template <int MODEL, int GPW>
 struct WideBwd {
   static constexpr int NP = MODEL == GROUP_TREELSTM ? 3 : MODEL == GROUP_LSTM ? 1 : 2;
   // k-groups of the product over a row of dA (K = 3H, 4H, H) and of those over the rows of dF; a tile takes its U
-  // k-groups D at a time
+  // k-groups D at a time (five of the twenty at H = 512: ten spill)
   static constexpr int KL = MODEL == GROUP_TREELSTM ? 3 * GPW : MODEL == GROUP_LSTM ? 4 * GPW : GPW, KF = MODEL == GROUP_TREELSTM ? GPW : 0;
-  static constexpr int U = KL + 2 * KF, D = U <= 10 ? U : U % 2 == 0 ? U / 2 : U / 3;
+  static constexpr int U = KL + 2 * KF, D = U <= 10 ? U : U > 16 && U % 4 == 0 ? U / 4 : U % 2 == 0 ? U / 2 : U / 3;
   static_assert(U % D == 0, "a tile is whole turns");
   static constexpr int NS = MODEL == GROUP_LSTM ? 1 : GPW;
   static constexpr size_t kLds = group_red_bytes(NP) + (size_t)8 * (D * 64 + 1) * sizeof(float4);
