@@ -35,13 +35,17 @@ struct GemmArgs {
   // A block the caller knows about (cavs_gemm_desc::zero_kind and friends): the tiles it covers
   // run a shorter k range, or none
   int zkind = 0, zrows = 0, zcol = 0;
-  // > 0: the launch is two launches back to back, the first zseg tiles (the row tiles inside the
-  // block, whose workgroups do less) and the rest, each padded to a multiple of 8 workgroups and
-  // dealt to the XCDs by itself: with one deal over all tiles the XCDs that hold the first
-  // tiles would finish early and the others set the time as before
-  int zseg = 0;
+  // seg_rows > 0: the launch is several launches back to back, each padded to a multiple of 8 workgroups and dealt to the XCDs by
+  // itself -- with one deal over all tiles the XCDs that hold those with less to do would finish early and the others set the time as
+  // before: the row tiles inside the block up to column tile seg_cols, those up to seg_mixed (partly inside it), the other row
+  // tiles, and what is left of the block (nothing but zeros to store)
+  int seg_rows = 0, seg_cols = 0, seg_mixed = 0;
   const int *live = nullptr;  // cavs_gemm_desc::live
   int pad_block = 0, pad_used = 0;  // cavs_gemm_desc::pad_block, pad_used
+  // an id per row of A as it is stored (of M, or of K where A is transposed): rows with equal ids, none below zero, are equal, and from
+  // ids_from on they may well be
+  const float *row_ids = nullptr;
+  int ids_from = 0;
 };
 
 __device__ inline bool padding_column(const GemmArgs &g, int col) { return g.pad_block > 0 && col % g.pad_block >= g.pad_used; }

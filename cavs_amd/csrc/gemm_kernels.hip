@@ -34,6 +34,10 @@ struct GemmGroup {
   int tiles[kGroupMax];
   int splits[kGroupMax];
   int form[kGroupMax];  // transA * 2 + transB
+  // Tiles and splits whose rows may be all one (GemmArgs::row_ids): those behind the first long_tiles, long_splits.  They are done soon, so
+  // they come behind everything else (from after[p] on) and are dealt to the XCDs by themselves: among the others they left some XCDs
+  // without work.
+  int long_tiles[kGroupMax], long_splits[kGroupMax], after[kGroupMax + 1];
   int count;
 };
 
@@ -105,22 +109,37 @@ template <bool VEC>
 __global__ __launch_bounds__(kThreads, 4) void sgemm_group_kernel(GemmGroup G, GroupFold F) {
   constexpr int BM = 64, BN = 64, BK = 16;
   __shared__ __attribute__((aligned(16))) char S[split_lds_bytes(BM, BN, BK)];
-  if ((int)blockIdx.x >= G.first[G.count]) {
-    const int b = blockIdx.x - G.first[G.count], across = (F.sums.w + 63) / 64;
+  const int end = G.first[G.count] + G.after[G.count];
+  if ((int)blockIdx.x >= end) {
+    const int b = blockIdx.x - end, across = (F.sums.w + 63) / 64;
     return colsum_part_block(F.sums, b % across, b / across, reinterpret_cast<float(*)[64]>(S));
   }
-  int p = 0;
-  while (p + 1 < G.count && (int)blockIdx.x >= G.first[p + 1]) p++;
-  const int local = blockIdx.x - G.first[p];
+  const bool soon = (int)blockIdx.x >= G.first[G.count];
+  int local = blockIdx.x, p = 0;
+  if (soon) {
+    local -= G.first[G.count];
+    while (p + 1 < G.count && local >= G.after[p + 1]) p++;
+    local -= G.after[p];
+  } else {
+    while (p + 1 < G.count && local >= G.first[p + 1]) p++;
+    local -= G.first[p];
+  }
   GemmArgs g = G.g[p];
   apply_live(g, G.form[p] >= 2, G.splits[p]);
   const int tiles = g.live ? (g.M + BM - 1) / BM * ((g.N + BN - 1) / BN) : G.tiles[p];
-  const int share = tiles * G.splits[p], padded = (share + 7) & ~7;
+  const int longT = g.live ? tiles : G.long_tiles[p], longZ = G.long_splits[p];
+  const int share = soon ? tiles * G.splits[p] - longT * longZ : longT * longZ, padded = (share + 7) & ~7;
   if (local >= padded) return;
   const int w = xcd_remap(local, padded);
   if (w >= share) return;
-  int t = w % tiles;
-  const int z = w / tiles, tilesN = (g.N + BN - 1) / BN, m0 = t / tilesN * BM, n0 = t % tilesN * BN;
+  int t = w % longT, z = w / longT;
+  if (soon) {
+    const bool rows = longT < tiles;
+    const int across = rows ? tiles - longT : tiles;
+    t = (rows ? longT : 0) + w % across;
+    z = (rows ? 0 : longZ) + w / across;
+  }
+  const int tilesN = (g.N + BN - 1) / BN, m0 = t / tilesN * BM, n0 = t % tilesN * BN;
   int mine = -1;  // (asked for in front of the product, looked at behind it)
   if (F.counters && F.embed == p && m0 < min(F.tail.n, g.M)) mine = embed_row(F.tail.ids, min(F.tail.n, g.M), F.tail.E, m0 / kEmbedRows);
   switch (G.form[p]) {
@@ -468,7 +487,7 @@ static bool vec_path_ok(const GemmArgs &g, int tA, int tB) {
 // workgroups then take more of a CU than they use, and fewer of them share one
 static thread_local unsigned t_lds_pad = 0;
 
-// The grid of a launch of BM x BN tiles: a known block of whole row tiles becomes a launch of its own (GemmArgs::zseg).
+// The grid of a launch of BM x BN tiles: a known block of whole row tiles becomes a launch of its own (GemmArgs::seg_rows).
 static dim3 tile_grid(GemmArgs *g, int BM, int BN, const GemmPlan &p) {
   dim3 grid((unsigned)p.tiles, p.splits);
   if (g->live) {  // (the kernel counts its tiles; room for two padded launches)
@@ -476,10 +495,15 @@ static dim3 tile_grid(GemmArgs *g, int BM, int BN, const GemmPlan &p) {
     return grid;
   }
   if (g->zkind == CAVS_GEMM_A_ZERO || g->zkind == CAVS_GEMM_C_UNUSED) {
-    const long inside = (long)(std::min(g->zrows, g->M) / BM) * ((g->N + BN - 1) / BN);
-    if (inside > 0 && inside < p.tiles) {
-      g->zseg = (int)inside;
-      grid.x = (unsigned)((inside + 7) / 8 * 8 + (p.tiles - inside + 7) / 8 * 8);
+    const int tilesM = (g->M + BM - 1) / BM, tilesN = (g->N + BN - 1) / BN, rows = std::min(g->zrows, g->M);
+    if (rows / BM > 0 && rows / BM < tilesM) {
+      const bool unused = g->zkind == CAVS_GEMM_C_UNUSED;
+      g->seg_rows = rows / BM;
+      g->seg_cols = unused ? std::min((g->zcol + BN - 1) / BN, tilesN) : tilesN;
+      g->seg_mixed = unused ? (rows + BM - 1) / BM : g->seg_rows;
+      auto whole = [](long n) { return (n + 7) / 8 * 8; };
+      grid.x = (unsigned)(whole((long)g->seg_rows * g->seg_cols) + whole((long)(g->seg_mixed - g->seg_rows) * tilesN) +
+                          whole((long)(tilesM - g->seg_mixed) * tilesN) + whole((long)g->seg_rows * (tilesN - g->seg_cols)));
     }
   }
   return grid;
@@ -559,7 +583,8 @@ struct Padding {
 static int run_gemm(const char *who, int tA, int tB, int M, int N, int K, float alpha, const float *A,
                     int lda, const float *B, int ldb, float beta, float *C, int ldc, const float *D,
                     int ldd, int dshift, void *ws, size_t ws_bytes, void *stream, const PullRows *pull = nullptr,
-                    const BlockHint *hint = nullptr, const int *live = nullptr, int live_expect = 0, Padding pad = {}) {
+                    const BlockHint *hint = nullptr, const int *live = nullptr, int live_expect = 0, Padding pad = {},
+                    const float *row_ids = nullptr) {
   int rc = check_gemm(who, tA, tB, M, N, K, A, lda, B, ldb, C, ldc);
   if (rc || M == 0 || N == 0) return rc;
   // Looked-up rows: up to 128 of them the skinny kernel, beyond it the 64 x 64 tiles (M x 2048 x 300..512: 21
@@ -572,6 +597,7 @@ static int run_gemm(const char *who, int tA, int tB, int M, int N, int K, float 
   g.live = live;
   g.pad_block = pad.block;
   g.pad_used = pad.used;
+  g.row_ids = row_ids;
   if (hint) hint->set(&g, tA, tB, beta == 0.f && !D);
   if (pull) {
     g.pull_rows = pull->rows;
@@ -616,8 +642,12 @@ static int run_gemm(const char *who, int tA, int tB, int M, int N, int K, float 
 // are few even so, and a single product is cut as it would be by itself (plan_product).
 // `tail_product` >= 0: that product's result is handed on to the embedding scatter-add (dtable, ids)
 // and `counters` [n_counters]: the group's launch adds up its splits itself where they are enough (GroupFold)
+struct Lookups {  // bit p: product p is over the rows that the ids looked up, equal where those are (GemmArgs::row_ids)
+  unsigned products = 0;
+  int from = 0;
+};
 static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_bytes, size_t *need_out, void *stream,
-                     int tail_product = -1, float *dtable = nullptr, const float *ids = nullptr, int *counters = nullptr, int n_counters = 0, const cavs_colsum_desc *sums = nullptr) {
+                     int tail_product = -1, float *dtable = nullptr, const float *ids = nullptr, int *counters = nullptr, int n_counters = 0, const cavs_colsum_desc *sums = nullptr, Lookups lookups = {}) {
   CAVS_REQUIRE(count >= 0 && count <= kGroupMax, "cavs_sgemm_group: %d products, at most %d", count, kGroupMax);
   CAVS_REQUIRE(count == 0 || d, "cavs_sgemm_group: null descriptors");
   EmbedTail tail{};
@@ -634,6 +664,10 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
   GroupFold F{};
   F.embed = -1;
   long split_tiles = 0;
+  auto looked_up = [&](int p) {
+    const cavs_gemm_desc &q = d[p];
+    return (lookups.products >> p & 1) && !q.live && (q.transA ? !q.transB : q.transB && p == tail_product);
+  };
   // K as the plan sees it, and the number of tiles it expects (cavs_gemm_desc::live)
   auto plan_K = [](const cavs_gemm_desc &q) { return q.live && q.transA ? std::min(q.K, std::max(q.live_expect, 1)) : q.K; };
   auto plan_tiles = [](const cavs_gemm_desc &q) {
@@ -719,6 +753,15 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
     g.pad_block = q.pad_block;
     g.pad_used = q.pad_used;
     BlockHint{q.zero_kind, q.live ? 1 : q.zero_rows, q.zero_col}.set(&g, q.transA, q.transB, q.beta == 0.f);
+    G.long_tiles[n] = (int)tiles[p];
+    G.long_splits[n] = splits;
+    if (looked_up(p)) {
+      g.row_ids = ids;
+      g.ids_from = lookups.from;
+      const long rows = std::min<long>(((long)lookups.from + 63) / 64 * ((q.N + 63) / 64), tiles[p]);
+      if (q.transA) G.long_splits[n] = (int)std::min<long>(((long)lookups.from + kchunk - 1) / kchunk, splits);
+      else G.long_tiles[n] = (int)rows;
+    }
     if (splits > 1) {
       if (ws) g.ws = reinterpret_cast<float *>(static_cast<char *>(ws) + need);
       need += ((size_t)splits * q.M * q.N * sizeof(float) + 255) / 256 * 256;
@@ -728,7 +771,9 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
     G.tiles[n] = (int)tiles[p];
     G.splits[n] = splits;
     G.form[n] = (q.transA ? 2 : 0) + (q.transB ? 1 : 0);
-    G.first[n + 1] = G.first[n] + (int)((tiles[p] * splits + 7) / 8 * 8);
+    const long first = (long)G.long_tiles[n] * G.long_splits[n];
+    G.first[n + 1] = G.first[n] + (int)((first + 7) / 8 * 8);
+    G.after[n + 1] = G.after[n] + (int)((tiles[p] * splits - first + 7) / 8 * 8);
     if (splits > 1) {
       F.first[n] = (int)split_tiles;
       split_tiles += tiles[p];
@@ -777,7 +822,7 @@ static int run_group(int count, const cavs_gemm_desc *d, void *ws, size_t ws_byt
     if (F.embed >= 0) with_tail = false;
     nr = R.count = 0;
   }
-  unsigned grid = G.first[n];
+  unsigned grid = G.first[n] + G.after[n];
   if (sums && sums->n > 0 && n > 0) {
     F.sums = colsum_job(sums->parts, sums->inp, sums->ld, sums->n, sums->w);
     grid += (unsigned)((sums->w + 63) / 64 * F.sums.chunks);
@@ -885,6 +930,17 @@ int cavs_sgemm_group_once(int count, const cavs_gemm_desc *products, int embed_p
   return run_group(count, products, workspace, workspace_bytes, nullptr, stream, embed_product, dtable, ids, counters, n_counters, sums);
 }
 
+int cavs_sgemm_group_lookups(int count, const cavs_gemm_desc *products, int embed_product, float *dtable, const float *ids, unsigned lookup_products,
+                             int same_from, void *workspace, size_t workspace_bytes, int *counters, int n_counters, const cavs_colsum_desc *sums,
+                             void *stream) {
+  CAVS_REQUIRE(counters && n_counters >= 0, "cavs_sgemm_group_lookups: null counters");
+  CAVS_REQUIRE(embed_product >= 0 && same_from >= 0, "cavs_sgemm_group_lookups: product %d, rows from %d", embed_product, same_from);
+  CAVS_REQUIRE(!sums || (sums->n >= 0 && sums->w > 0 && sums->ld >= sums->w && sums->parts && (sums->inp || sums->n == 0)),
+               "cavs_sgemm_group_lookups: bad column sums");
+  return run_group(count, products, workspace, workspace_bytes, nullptr, stream, embed_product, dtable, ids, counters, n_counters, sums,
+                   {lookup_products, same_from});
+}
+
 int cavs_sgemm_group_beside(int count, const cavs_gemm_desc *products, void *workspace, size_t workspace_bytes,
                             void *stream) {
   // With the 48 KB of a large tile's panels more than half of a CU's LDS: one workgroup to a CU.  (Two of them, at
@@ -925,7 +981,7 @@ int cavs_embed_pull_sgemm_padded(float *C, int ldc, float *e_out, int ld_e, floa
     int rc = cavs_embed_pull_fwd(e_out, ld_e, ids_out, x, rows, table, n, E, stream);
     if (rc || N == 0) return rc;
     return run_gemm("cavs_embed_pull_sgemm", 0, 0, n, N, E, 1.f, e_out, ld_e, B, ldb, 0.f, C, ldc, nullptr, 0, 0, nullptr, 0, stream,
-                    nullptr, &hint, nullptr, 0, {pad_block, pad_used});
+                    nullptr, &hint, nullptr, 0, {pad_block, pad_used}, ids_out);
   }
   const PullRows pull{rows, x, e_out, ld_e, ids_out};
   return run_gemm("cavs_embed_pull_sgemm", 0, 0, n, N, E, 1.f, table, E, B, ldb, 0.f, C, ldc, nullptr, 0, 0, nullptr, 0, stream, &pull,

@@ -91,7 +91,7 @@ __device__ inline int split_at(int x, int oct) {
 // contiguous index in memory and a unit is 16 bytes of it; otherwise a unit is eight rows of one
 // column.  An x outside the operand reads the last one instead (what it leads to is not stored);
 // only k is checked, and only where the step is not wholly inside the k range.
-// PULL (k-contiguous): rows are looked up (GemmArgs::pull_*), and those a workgroup reads go on into pull_copy.
+// PULL (k-contiguous): rows are looked up (GemmArgs::pull_*); a row without an id reads the table's first, and is zero.
 template <int BX, int BK, bool KC, bool VEC, bool DESC, bool PULL = false>
 struct SplitLoader {
   static constexpr int U = KC || BX * BK < 8 * kThreads ? 4 : 8, NU = BX * BK / U / kThreads, PER = BK / U;
@@ -118,13 +118,11 @@ struct SplitLoader {
 
   // Row x0 + r of the operand is the table row that starts at float int(id * K) (EmbeddingLookup's
   // offset), id = px[rows[x0 + r]]; a negative id is a zero row.
-  bool in[PULL ? NU : 1];       // the row is inside the operand and has an id
-  float *copy[PULL ? NU : 1];  // where the unit goes as well, or nullptr
-  int copy_mod = 1, copy_rem = 0;
-  __device__ inline void prepare_pull(const GemmArgs &g, int x0, int tid, float *ids_out, int mod, int rem) {
+  bool in[PULL ? NU : 1];  // the row has an id
+  bool all_in = true;      // every row of this wavefront has
+  long one = -1;  // the row this wavefront's units are all of, if they are; -2: it has none
+  __device__ inline void prepare_pull(const GemmArgs &g, int x0, int tid, float *ids_out) {
     static_assert(!PULL || KC, "looked-up rows are k-contiguous");
-    copy_mod = mod;
-    copy_rem = rem;
 #pragma unroll
     for (int i = 0; i < NU; i++) {
       const int u = tid + kThreads * i, x = u / PER, gx = x0 + x;
@@ -136,9 +134,11 @@ struct SplitLoader {
         off = (long)(int)(id * (float)g.K);
         if (ids_out && unit[i] == 0) ids_out[gx] = id;
       }
-      in[i] = off >= 0;
-      boff[i] = 4 * ((Off)(in[i] ? off : 0) + U * unit[i]);
-      copy[i] = gx < g.M ? g.pull_copy + (long)gx * g.ld_copy + U * unit[i] : nullptr;
+      if (i == 0) one = __builtin_amdgcn_readfirstlane(gx < g.M ? (int)off : -2);  // (rows ascend: beyond the last, all of them are)
+      if (!__all(off == one || gx >= g.M)) one = -1;
+      in[i] = off >= 0 || gx >= g.M;
+      all_in &= __all(in[i]);
+      boff[i] = 4 * ((Off)(off >= 0 ? off : 0) + U * unit[i]);
     }
   }
 
@@ -168,27 +168,7 @@ struct SplitLoader {
     for (int i = 0; i < NU; i++) {
       if constexpr (KC) {
         const float *q = reinterpret_cast<const float *>(reinterpret_cast<const char *>(P + k0) + boff[i]);
-        if constexpr (PULL) {
-          const int left = in[i] ? kend - k0 - U * unit[i] : 0;
-          if constexpr (VEC) {  // (K is a multiple of 4)
-            float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (left > 0) a = *reinterpret_cast<const float4 *>(q);
-            v[i][0] = a.x, v[i][1] = a.y, v[i][2] = a.z, v[i][3] = a.w;
-          } else {
-#pragma unroll
-            for (int j = 0; j < U; j++) v[i][j] = j < left ? q[j] : 0.f;
-          }
-          if (copy[i] && (k0 / BK) % copy_mod == copy_rem) {
-            const int room = kend - k0 - U * unit[i];
-            if constexpr (VEC) {
-              if (room > 0) *reinterpret_cast<float4 *>(copy[i] + k0) = make_float4(v[i][0], v[i][1], v[i][2], v[i][3]);
-            } else {
-#pragma unroll
-              for (int j = 0; j < U; j++)
-                if (j < room) copy[i][k0 + j] = v[i][j];
-            }
-          }
-        } else if constexpr (WHOLE && VEC) {
+        if constexpr (WHOLE && VEC) {
           const float4 a = *reinterpret_cast<const float4 *>(q);
           v[i][0] = a.x, v[i][1] = a.y, v[i][2] = a.z, v[i][3] = a.w;
         } else {
@@ -208,7 +188,15 @@ struct SplitLoader {
     }
   }
 
-  __device__ inline void store(const float (&v)[NU][U], char *__restrict__ S) const {
+  __device__ inline void store(float (&v)[NU][U], char *__restrict__ S) const {
+    if constexpr (PULL) {
+      if (!all_in) {
+#pragma unroll
+        for (int i = 0; i < NU; i++)
+#pragma unroll
+          for (int j = 0; j < U; j++) v[i][j] = in[i] ? v[i][j] : 0.f;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < NU; i++) {
       unsigned h[U / 2], m[U / 2], l[U / 2];
@@ -290,6 +278,234 @@ __device__ inline void unsplit_tile(const GemmArgs &g, int row, int col, int kbe
         for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
 }
 
+// ------------------------------------------------------------------ rows that are all the same
+// The inner vertices of a parse tree carry no word: they all look one table row up, and in a batch's rows they stand together, behind
+// the leaves.  So the lower half of x * W's row tiles hold one and the same row, the d W of those vertices is one row times the
+// sum of their gradients, and what they send to the table is that sum times W^T.  A tile finds out by itself (row_ids: rows
+// with equal ids are equal) and does a vector's work in fp32 where it would do a matrix's:
+//   x * W      one row times its columns of B, written to every row                    (same_rows_product)
+//   A^T * B    the sum of B's rows over its part of K, then one step of K = 1 as MFMA  (in split_tile)
+//   A * B^T    for the table: the sum of A's rows times its columns of B               (summed_rows_product)
+// What bounds such a tile are trips to memory, so its loads are all in flight at once.  64 trees, H = 512 (1217 leaves, 1153 inner
+// vertices), us a launch: x * W 30.4 -> 20.5, the deferred products 75 -> 64; 256 trees x * W 73.5 -> 47; Tree-LSTM steps of 64
+// trees 10250 -> 9550 (32 of them, with the resident rounds' change before).
+// The sums are shorter than the chains they replace, and in pairs.  2-norm of the error against 64 bits over that of the result, 2370 rows of
+// 300, 2048 columns, normal operands / operands from U(0, 1), before and now, 1e-7: x W 2.3 -> 1.9 / 1.7 -> 1.4, d W 2.4 -> 2.0 / 0.9 -> 0.6,
+// the table's gradient 10.3 -> 2.2 / 0.72 -> 0.67.
+
+// Whether ids[first .. end) are one and the same (the whole workgroup asks; every wavefront finds the same)
+__device__ inline bool same_ids(const float *__restrict__ ids, int first, int end) {
+  const float id = ids[first];
+  bool same = id >= 0.f;
+  for (int i = first + (threadIdx.x & 63); i < end; i += 64) same &= ids[i] == id;
+  return __all(same);
+}
+
+// One element of the product's result, or of its part of it
+template <bool THROUGH>
+__device__ inline void put_result(const GemmArgs &g, int z, int row, int col, float v) {
+  if (!g.ws) {
+    g.C[row * g.ldc + col] = g.alpha * v;
+    return;
+  }
+  float *w = g.ws + ((long)z * g.M + row) * g.N + col;
+  if constexpr (THROUGH) __hip_atomic_store(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else *w = v;
+}
+
+constexpr int kSameK = 4096;  // the row has room in the tile's LDS
+
+// C's rows m0 .. m0 + BM, columns n0 .. n0 + BN: `row` (K floats) times B, in every row.  beta = 0, K not split.  A thread has C of the
+// columns and every PARTS-th of K, as many loads in flight as there are registers for: one trip to memory behind the other is all
+// the time this takes.
+template <int BM, int BN, bool VEC>
+__device__ __forceinline__ void same_rows_product(const GemmArgs &g, const float *__restrict__ row, int m0, int n0, char *__restrict__ S) {
+  constexpr int C = VEC ? 4 : 1, ACROSS = BN / C, PARTS = kThreads / ACROSS, U = VEC ? 12 : 32;
+  float *a = reinterpret_cast<float *>(S), *part = a + kSameK;  // [kSameK], [PARTS][BN]
+  const int tid = threadIdx.x, c = C * (tid % ACROSS), q = tid / ACROSS;
+  const float *b = g.B + min(n0 + c, g.N - C);
+  float acc[C] = {}, v[U][C];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const float *at = b + (long)min(k0 + q + u * PARTS, g.K - 1) * g.ldb;
+      if constexpr (VEC) {
+        const float4 t = *reinterpret_cast<const float4 *>(at);
+        v[u][0] = t.x, v[u][1] = t.y, v[u][2] = t.z, v[u][3] = t.w;
+      } else {
+        v[u][0] = *at;
+      }
+    }
+  };
+  load(0);
+  for (int k = tid; k < g.K; k += kThreads) a[k] = row[k];
+  __syncthreads();
+  for (int k0 = 0; k0 < g.K; k0 += U * PARTS) {
+    if (k0 > 0) load(k0);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int k = k0 + q + u * PARTS;
+      const float x = k < g.K ? a[k] : 0.f;
+#pragma unroll
+      for (int j = 0; j < C; j++) acc[j] = k < g.K ? fmaf(x, v[u][j], acc[j]) : acc[j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < C; j++) part[q * BN + c + j] = acc[j];
+  __syncthreads();
+  // the parts' sums, a column to a thread, in their order; then every row
+  if (tid < BN) {
+    float t = 0.f;
+    for (int p = 0; p < PARTS; p++) t += part[p * BN + tid];
+    a[tid] = padding_column(g, n0 + tid) ? 0.f : g.alpha * t;
+  }
+  __syncthreads();
+  for (int r = q; r < BM && m0 + r < g.M; r += PARTS) {
+    float *to = g.C + (long)(m0 + r) * g.ldc + n0 + c;
+    if (VEC && g.ldc % 4 == 0 && n0 + c < g.N && (reinterpret_cast<uintptr_t>(to) & 15) == 0) {
+      *reinterpret_cast<float4 *>(to) = *reinterpret_cast<const float4 *>(a + c);
+    } else {
+#pragma unroll
+      for (int j = 0; j < C; j++)
+        if (n0 + c + j < g.N) to[j] = a[c + j];
+    }
+  }
+}
+
+// The rows of a tile that were looked up, on into pull_copy: the column tiles that run share them, every tilesN-th step of K each.  (Behind
+// the product, when the rows are near: among its loads the stores' conditions had every wait be for everything.)
+template <int BM, int BN, int BK, bool VEC>
+__device__ __forceinline__ void copy_looked_up(const GemmArgs &g, int m0, int n0) {
+  const int tilesN = (g.N + BN - 1) / BN;
+  const int active = (g.zkind == CAVS_GEMM_C_UNUSED && m0 + BM <= g.zrows) ? min(tilesN, (g.zcol + BN - 1) / BN) : tilesN;
+  constexpr int U = VEC ? 4 : 1;
+  const int x = threadIdx.x / (BK / U), k_ = threadIdx.x % (BK / U) * U;
+  for (int k0 = n0 / BN * BK; k0 < g.K; k0 += BK * active)
+    for (int r = x; r < BM; r += kThreads / (BK / U)) {
+      const int row = m0 + r, k = k0 + k_;
+      if (row >= g.M || k >= g.K) continue;
+      const long off = (long)(int)(g.pull_x[g.pull_rows[row]] * (float)g.K);
+      float *to = g.pull_copy + (long)row * g.ld_copy + k;
+      if constexpr (VEC) *reinterpret_cast<float4 *>(to) = off >= 0 ? *reinterpret_cast<const float4 *>(g.A + off + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+      else *to = off >= 0 ? g.A[off + k] : 0.f;
+    }
+}
+
+// sixteen values added up in pairs
+__device__ inline float4 pairs(float4 (&v)[16]) {
+#pragma unroll
+  for (int n = 8; n > 0; n /= 2)
+#pragma unroll
+    for (int i = 0; i < n; i++) v[i].x += v[i + n].x, v[i].y += v[i + n].y, v[i].z += v[i + n].z, v[i].w += v[i + n].w;
+  return v[0];
+}
+
+// Sixteen rows from p on, a float4 of each to a lane at byte `at` of a row: the rows' offsets are scalars
+__device__ inline void sixteen_rows(const float *p, int ld, int last, int at, float4 (&v)[16]) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), 0, 0xffffffffu, 0x00020000);
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const f4 a = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(r, at, max(min(i, last), 0) * ld * 4, 0));
+    v[i] = make_float4(a[0], a[1], a[2], a[3]);
+  }
+}
+
+// Rows m0 .. m0 + 64 of A (M x K) summed, times rows n0 .. n0 + 64 of B (N x K), over [kbeg, kend): the first row of the tile of C, and
+// zeros in the others.  kbeg, kend, lda, ldb are multiples of 4, A and B 16-byte aligned.
+template <bool THROUGH>
+__device__ __forceinline__ void summed_rows_product(const GemmArgs &g, int m0, int n0, int z, int kbeg, int kend, char *__restrict__ S) {
+  constexpr int KB = 1024, ROWS = 16;  // k at a time; rows of A and of B to a wavefront
+  float *s = reinterpret_cast<float *>(S);  // [4][KB], the sums in the first
+  float *out = s + 4 * KB;                  // [64]
+  const int tid = threadIdx.x, lane = tid & 63, q = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ra = min(m0 + ROWS * q, g.M - 1), rb = min(n0 + ROWS * q, g.N - 1);  // (a wavefront beyond the last row adds nothing, or is not stored)
+  const int rows = g.M - (m0 + ROWS * q), cols = g.N - 1 - rb;
+  const float *A = g.A + (long)ra * g.lda, *B = g.B + (long)rb * g.ldb;
+  const int lda = (int)g.lda, ldb = (int)g.ldb;
+  float acc[ROWS];
+#pragma unroll
+  for (int e = 0; e < ROWS; e++) acc[e] = 0.f;
+  for (int k0 = kbeg; k0 < kend; k0 += KB) {
+    const int len = min(KB, kend - k0);
+    __syncthreads();
+    for (int k = 4 * lane; k < len; k += 256) {
+      float4 v[ROWS];
+      sixteen_rows(A + k0, lda, rows - 1, 4 * k, v);
+#pragma unroll
+      for (int r = 0; r < ROWS; r++)
+        if (r >= rows) v[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+      *reinterpret_cast<float4 *>(s + q * KB + k) = pairs(v);
+    }
+    __syncthreads();
+    for (int k = 4 * tid; k < len; k += 4 * kThreads) {
+      float4 t = *reinterpret_cast<const float4 *>(s + k);
+#pragma unroll
+      for (int p = 1; p < 4; p++) {
+        const float4 o = *reinterpret_cast<const float4 *>(s + p * KB + k);
+        t.x += o.x, t.y += o.y, t.z += o.z, t.w += o.w;
+      }
+      *reinterpret_cast<float4 *>(s + k) = t;
+    }
+    __syncthreads();
+    for (int k = 4 * lane; k < len; k += 256) {
+      const float4 t = *reinterpret_cast<const float4 *>(s + k);
+      float4 v[ROWS];
+      sixteen_rows(B + k0, ldb, cols, 4 * k, v);
+#pragma unroll
+      for (int e = 0; e < ROWS; e++) acc[e] = fmaf(t.w, v[e].w, fmaf(t.z, v[e].z, fmaf(t.y, v[e].y, fmaf(t.x, v[e].x, acc[e]))));
+    }
+  }
+  // the lanes' sums of sixteen columns: halves are exchanged until a lane holds one
+#pragma unroll
+  for (int n = ROWS / 2; n > 0; n /= 2)
+#pragma unroll
+    for (int e = 0; e < n; e++) {
+      const bool up = lane & (4 * n);
+      const float give = up ? acc[e] : acc[e + n], keep = up ? acc[e + n] : acc[e];
+      acc[e] = keep + __shfl_xor(give, 4 * n, 64);
+    }
+  acc[0] += __shfl_xor(acc[0], 2, 64);
+  acc[0] += __shfl_xor(acc[0], 1, 64);
+  if ((lane & 3) == 0) out[ROWS * q + (lane >> 2)] = acc[0];
+  __syncthreads();
+  if (n0 + lane >= g.N) return;
+  const float sum = out[lane];
+#pragma unroll 4
+  for (int r = 0; r < ROWS; r++) {
+    const int row = m0 + ROWS * q + r;
+    if (row < g.M) put_result<THROUGH>(g, z, row, n0 + lane, row == m0 ? sum : 0.f);
+  }
+}
+
+// Columns n0 .. n0 + 64 of B (K x N) summed over rows [kbeg, kend), to s[64] in LDS.  N, ldb are multiples of 4, B 16-byte aligned.
+__device__ __forceinline__ void column_sums(const GemmArgs &g, int n0, int kbeg, int kend, float *__restrict__ s) {
+  constexpr int U = 16;
+  const int tid = threadIdx.x, group = tid >> 4, c = n0 + 4 * (tid & 15);
+  const float *b = g.B + (long)kbeg * g.ldb + min(c, g.N - 4);
+  const unsigned ldb = (unsigned)g.ldb;
+  float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int k = kbeg + group; k < kend; k += 16 * U) {
+    float4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) v[u] = *reinterpret_cast<const float4 *>(b + (size_t)(unsigned)(min(k + 16 * u, kend - 1) - kbeg) * ldb);
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (k + 16 * u >= kend) v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 o = pairs(v);
+    t.x += o.x, t.y += o.y, t.z += o.z, t.w += o.w;
+  }
+  *reinterpret_cast<float4 *>(s + 64 + tid * 4) = t;
+  __syncthreads();
+  if (tid < 64) {
+    float v = 0.f;
+#pragma unroll
+    for (int p = 0; p < 16; p++) v += s[64 + p * 64 + tid];
+    s[tid] = n0 + tid < g.N ? v : 0.f;
+  }
+  __syncthreads();
+}
+
 // two buffers of three parts
 constexpr int split_lds_bytes(int BM, int BN, int BK) { return 2 * 3 * 2 * BK * (BM + BN); }
 
@@ -311,12 +527,48 @@ __device__ __forceinline__ void split_tile(const GemmArgs &g, int m0, int n0, in
   LA la;
   LB lb;
   if constexpr (PULL) {
-    // the column tiles of this row tile that do run share the copying
-    const int tilesN = (g.N + BN - 1) / BN, tn = n0 / BN;
-    const int active = (g.zkind == CAVS_GEMM_C_UNUSED && m0 + BM <= g.zrows) ? min(tilesN, (g.zcol + BN - 1) / BN) : tilesN;
-    la.prepare_pull(g, m0, tid, n0 == 0 ? g.pull_ids : nullptr, active, tn);
+    la.prepare_pull(g, m0, tid, n0 == 0 ? g.pull_ids : nullptr);
+    if (g.K <= kSameK && kend > kbeg) {
+      long *one = reinterpret_cast<long *>(S);
+      if (lane == 0) one[wave] = la.one;
+      __syncthreads();
+      const long row = one[0];
+      bool same = row >= 0;
+#pragma unroll
+      for (int w = 1; w < 4; w++) same &= one[w] == row || one[w] == -2;
+      __syncthreads();
+      if (same) {
+        copy_looked_up<BM, BN, BK, VEC>(g, m0, n0);
+        return same_rows_product<BM, BN, VEC>(g, g.A + row, m0, n0, S);
+      }
+    }
   } else {
+    if constexpr (!TA && !TB && !THROUGH) {
+      if (g.row_ids && m0 >= g.ids_from && g.K <= kSameK && kend > kbeg && same_ids(g.row_ids, m0, min(m0 + BM, g.M)))
+        return same_rows_product<BM, BN, VEC>(g, g.A + (long)m0 * g.lda, m0, n0, S);
+    }
+    if constexpr (!TA && TB && VEC && THROUGH) {
+      if (g.row_ids && m0 >= g.ids_from && kend > kbeg && same_ids(g.row_ids, m0, min(m0 + BM, g.M)))
+        return summed_rows_product<THROUGH>(g, m0, n0, z, kbeg, kend, S);
+    }
     la.prepare(g.lda, m0, g.M, tid);
+  }
+  // (A^T B) rows of K from `same` on, if they are equal: the sums of B's before the loops (no accumulator yet), their step behind them
+  int same = kend;
+  const int kall = kend;
+  float one_a = 0.f, one_b = 0.f;
+  if constexpr (TA && !TB && VEC && THROUGH) {
+    if (g.row_ids) {
+      const int from = max(kbeg, kbeg + (g.ids_from - kbeg + BK - 1) / BK * BK);
+      if (from + 2 * BK <= kend && same_ids(g.row_ids, from, kend)) {
+        kend = same = from;
+        float *s = reinterpret_cast<float *>(S);
+        column_sums(g, n0, same, kall, s);
+        one_a = g.A[(long)same * g.lda + m0 + min(tid % BM, g.M - 1 - m0)];
+        one_b = s[tid % BN];
+        __syncthreads();
+      }
+    }
   }
   lb.prepare(g.ldb, n0, g.N, tid);
   const float *A = PULL ? g.A : TA ? g.A + m0 : g.A + (long)m0 * g.lda, *B = TB ? g.B + (long)n0 * g.ldb : g.B + n0;
@@ -357,7 +609,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs &g, int m0, int n0, in
       lb.template load<false>(r.b, B, g.ldb, k0, kend);
     }
   };
-  auto put = [&](const Regs &r, int kt) {
+  auto put = [&](Regs &r, int kt) {
     char *to = S + (kt & 1) * BUF;
     la.store(r.a, to);
     lb.store(r.b, to + 3 * PA);
@@ -417,6 +669,29 @@ __device__ __forceinline__ void split_tile(const GemmArgs &g, int m0, int n0, in
     if (kt + 2 < nk) put(r0, kt + 2);
     __syncthreads();
   }
+  if constexpr (TA && !TB && VEC && THROUGH) {
+    if (same < kall) {
+      // A's row of 64 and the sums, as one step whose other rows of K are zero.  (An infinity meets every gradient by itself, as
+      // it would have: left to unsplit_tile by the NaN it makes here.)
+      constexpr int U = LA::U;
+      Regs r;
+#pragma unroll
+      for (int i = 0; i < LA::NU; i++)
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+          const bool on = U * la.unit[i] + j == 0;
+          r.a[i][j] = on ? one_a : 0.f;
+          r.b[i][j] = on ? one_b : 0.f;
+        }
+      put(r, 0);
+      __syncthreads();
+      multiply(0);
+      kend = kall;
+    }
+  }
+  if constexpr (PULL) {
+    if (kend > kbeg) copy_looked_up<BM, BN, BK, VEC>(g, m0, n0);
+  }
   fold();
   int row = m0 + wm * WM, col = n0 + wn * WN, l = lane;
   asm volatile("" : "+v"(row), "+v"(col), "+v"(l));  // (or the addresses of the stores are kept through the loops above)
@@ -452,32 +727,44 @@ __global__ __launch_bounds__(kThreads, BM == 128 && FOLD ? 2 : 3) void sgemm_spl
   apply_live(g, TA, gridDim.y);
   const int tilesN = (g.N + BN - 1) / BN, tilesM = (g.M + BM - 1) / BM;
   if (g.live && (g.zkind == CAVS_GEMM_A_ZERO || g.zkind == CAVS_GEMM_C_UNUSED)) {
-    const int inside = min(g.zrows, g.M) / BM * tilesN;
-    g.zseg = inside < tilesM * tilesN ? inside : 0;
+    const int inside = min(g.zrows, g.M) / BM;
+    g.seg_rows = g.seg_mixed = inside < tilesM ? inside : 0;
+    g.seg_cols = tilesN;
   }
-  int t, row0 = 0, rows = tilesM;
-  if (g.zseg > 0) {
-    const int first = (g.zseg + 7) & ~7, rest = (tilesM * tilesN - g.zseg + 7) & ~7, b = blockIdx.x;
-    if (b >= first + rest) return;
-    if (b < first) {
-      t = xcd_remap(b, first);
-      rows = g.zseg / tilesN;
-    } else {
-      t = xcd_remap(b - first, rest);
-      row0 = g.zseg / tilesN;
-      rows = tilesM - row0;
+  int t = blockIdx.x, row0 = 0, rows = tilesM, col0 = 0, cols = tilesN;
+  if (g.seg_rows > 0) {
+    for (int seg = 0;; seg++) {
+      if (seg > 3) return;
+      const bool inside = seg == 0 || seg == 3;
+      row0 = inside ? 0 : seg == 1 ? g.seg_rows : g.seg_mixed;
+      rows = (inside ? g.seg_rows : seg == 1 ? g.seg_mixed : tilesM) - row0;
+      col0 = seg == 3 ? g.seg_cols : 0;
+      cols = (seg == 0 ? g.seg_cols : tilesN) - col0;
+      const int n = (rows * cols + 7) & ~7;
+      if (t < n) {
+        t = xcd_remap(t, n);
+        break;
+      }
+      t -= n;
     }
-    if (t >= rows * tilesN) return;
+    if (t >= rows * cols) return;
   } else if (g.live) {
     const int all = (tilesM * tilesN + 7) & ~7;
-    if ((int)blockIdx.x >= all) return;
-    t = xcd_remap(blockIdx.x, all);
+    if (t >= all) return;
+    t = xcd_remap(t, all);
     if (t >= tilesM * tilesN) return;
   } else {
-    t = xcd_remap(blockIdx.x, tilesM * tilesN);
+    t = xcd_remap(t, tilesM * tilesN);
   }
   int tm, tn;
-  split_tile_at(t, row0, rows, tilesN, &tm, &tn);
+  split_tile_at(t, row0, rows, cols, &tm, &tn);
+  tn += col0;
+  if constexpr (!TA && !TB) {
+    if ((PULL || g.row_ids) && g.seg_rows == 0) {  // rows from both halves in turn: those of the second may be done sooner
+      const int half = (tilesM + 1) / 2;
+      tm = tm & 1 ? half + tm / 2 : tm / 2;
+    }
+  }
   split_tile<BM, BN, BK, TA, TB, VEC, FOLD, PULL>(g, tm * BM, tn * BN, blockIdx.y, S);
 }
 

@@ -105,6 +105,7 @@ _SIGS = {
     "cavs_sgemm_group_embed_bwd": [_I, C.POINTER(GemmDesc), _I, _P, _P, _P, _Z, _P],
     "cavs_root_sq": [_P, _P, _P, _P, _I, _I, _I, _P],
     "cavs_sgemm_group_once": [_I, C.POINTER(GemmDesc), _I, _P, _P, _P, _Z, _P, _I, C.POINTER(ColsumDesc), _P],
+    "cavs_sgemm_group_lookups": [_I, C.POINTER(GemmDesc), _I, _P, _P, C.c_uint, _I, _P, _Z, _P, _I, C.POINTER(ColsumDesc), _P],
     "cavs_sgemm_splitk": [_I, _I, _I, _I, _I, _F, _P, _I, _P, _I, _F, _P, _I, _P, _Z, _P],
     "cavs_sgemm_splitk_static": [_I, _I, _I, _I, _I, _F, _P, _I, _P, _I, _F, _P, _I, _P],
     "cavs_colsum": [_P, _P, _I, _I, _I, _I, _P],

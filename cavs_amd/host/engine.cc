@@ -1859,7 +1859,7 @@ void Engine::treelstm_backward() {
       {1, 0, H, H, 2 * (N - lp), 1.f, 0.f, G_.at((size_t)2 * lp * 2 * H), 2 * H, dF_.at((size_t)2 * lp * H), H,
        dU + (size_t)3 * H * H, H},
   };
-  last_launch(3, bias_row, [&] { gemm_group_embedding_backward(products, E); });
+  last_launch(3, bias_row, [&] { gemm_group_embedding_backward(products, E, 3); });
   // bias blocks [i|f|u|o] from dxW columns [i|o|u|f]
   if (bias_row) {
     // settled by the launch that ends the step (or right after this pass); block k of the row
@@ -1986,7 +1986,7 @@ void Engine::backward_prologue(std::vector<cavs_task> tasks, bool with_embedding
 
 // `products[0]` is de = dxW * W^T; its rows go on into the embedding gradient in the launch that
 // reduces the group's K splits (cavs_sgemm_group_embed_bwd).
-void Engine::gemm_group_embedding_backward(const std::vector<cavs_gemm_desc> &products, int E, const cavs_colsum_desc *sums) {
+void Engine::gemm_group_embedding_backward(const std::vector<cavs_gemm_desc> &products, int E, unsigned lookups, const cavs_colsum_desc *sums) {
   Param &emb = param("Emb");
   const bool owned = emb.g == emb.own_g.get();
   if (emb_cleared_) {
@@ -1999,11 +1999,18 @@ void Engine::gemm_group_embedding_backward(const std::vector<cavs_gemm_desc> &pr
     c_launches_ += 1;
   }
   const int count = (int)products.size();
+  // (the inner vertices of parse trees look up one row: behind the leaves' the rows may well be equal)
+  if (words_ || nch_ != 2) lookups = 0;
+  const int from = sched_->leaf_prefix;
   float *ws = workspace(cavs_sgemm_group_workspace(count, products.data()));
   {
     ProfScope ps(this, K_GEMM);
     const float *ids = words_ ? reinterpret_cast<const float *>(d_words_index_ + 4 + 3 * (size_t)N_) : xs_.get();
-    check(cavs_sgemm_group_once(count, products.data(), 0, emb.g, ids, ws, ws_.capacity() * 4, group_counters(), kGroupCounters, sums, stream_));
+    if (lookups)
+      check(cavs_sgemm_group_lookups(count, products.data(), 0, emb.g, ids, lookups, from, ws, ws_.capacity() * 4, group_counters(),
+                                     kGroupCounters, sums, stream_));
+    else
+      check(cavs_sgemm_group_once(count, products.data(), 0, emb.g, ids, ws, ws_.capacity() * 4, group_counters(), kGroupCounters, sums, stream_));
   }
   for (const cavs_gemm_desc &q : products) {
     c_gemm_flops_ += desc_flops(q);
@@ -2195,7 +2202,7 @@ void Engine::lstm_backward() {
       {1, 0, E, 4 * H, N, 1.f, 0.f, e_.get(), E, dx, 4 * H, dW, 4 * H, 0, 0, 0, live, words_expected()},
       {1, 0, H, 4 * H, N - lp, 1.f, 0.f, G_.at((size_t)lp * 2 * H), 2 * H, dxW_.at((size_t)lp * 4 * H), 4 * H,
        dW + (size_t)4 * H * E, 4 * H},
-  }, E, &sums); });
+  }, E, 0, &sums); });
 }
 
 // ------------------------------------------------------------------ Tree-FC
@@ -2619,7 +2626,7 @@ void Engine::cell_backward() {
     size_t at = 0;
     if (wv == 0 && c0.NX > 0 && L == 1 && !w.empty()) {  // d e is complete after this launch
       const size_t take = std::min(w.size(), kGroup);
-      gemm_group_embedding_backward(std::vector<cavs_gemm_desc>(w.begin(), w.begin() + take), E_, rider());
+      gemm_group_embedding_backward(std::vector<cavs_gemm_desc>(w.begin(), w.begin() + take), E_, 3, rider());
       at = take;
       embedded = true;
     }

@@ -253,6 +253,14 @@ typedef struct {
 int cavs_sgemm_group_once(int count, const cavs_gemm_desc *products, int embed_product, float *dtable, const float *ids,
                           void *workspace, size_t workspace_bytes, int *counters, int n_counters, const cavs_colsum_desc *sums,
                           void *stream);
+/* cavs_sgemm_group_once where some products (bit p of lookup_products) are over the rows that `ids` looked up: A of M rows in the
+ * product that feeds the table, A^T over K rows in the others.  Where rows from same_from on have one id -- a parse tree's inner
+ * vertices carry no word -- their share is the sum of their gradients times that one row, and C of the product that feeds the table
+ * then holds the sum of such rows of a block of 64 in the first of them, zeros in the others.  Otherwise the results
+ * are those of cavs_sgemm_group_once up to the order of sums.  A product with `live` is taken as it is. */
+int cavs_sgemm_group_lookups(int count, const cavs_gemm_desc *products, int embed_product, float *dtable, const float *ids,
+                             unsigned lookup_products, int same_from, void *workspace, size_t workspace_bytes, int *counters, int n_counters,
+                             const cavs_colsum_desc *sums, void *stream);
 /* C[r,:] = op(A)*op(B) + D[r >> d_shift, :]: the GEMM and the Accumulate that
  * follows it in the backward of a Mirror'ed operand
  * (cavs/backend/op_decl_slice_join.cc:173-182) in one pass.  Workspace as above. */
