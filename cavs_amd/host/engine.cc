@@ -173,11 +173,29 @@ int Engine::tail_limit() const {
   return cfg_.tail_rows > 0 ? cfg_.tail_rows : 64;
 }
 
-// A group takes a round of up to this many rows (in slices of 32); larger rounds are launches of their own.
+// A group takes a round of up to this many rows (in slices of 32); larger rounds are launches of their own.  A share of 64 leaves
+// a forward pass of most sizes level with those launches (0.84 .. 1.15 of the time with 256, by the batch).  Where a group is all
+// of its chiplet's workgroups a larger share is the faster one: trees of 256 parses at H = 512 0.463 -> 0.442 ms a pass, chains
+// in batches of 1024 0.741 -> 0.714 ms, at H = 384 0.708 -> 0.618 (Tree-LSTM at H = 384: no difference; Tree-FC at 512, one product
+// of its row: 0.80 -> 0.80 .. 1.39 -> 1.42).  A training pass gains both ways: H = 512, 256 parses 1.289 -> 1.151 ms a step, Tree-FC
+// 0.422 -> 0.374, chains in batches of 1024 1.745 -> 1.538; H = 256 0.697 -> 0.655.
 int Engine::group_limit() const {
   if (!resident_ || fused_rows() <= 0 || (cell_ && cell_->rounds.empty()) || !cavs_group_rounds_ok(cfg_.H)) return 0;
   if (cfg_.tail_rows > 0) return tail_limit() > 0 ? 0 : cfg_.tail_rows;
-  return 64;
+  if (cell_) return 64;
+  if (!lists_forward_only()) return 512;
+  return (cfg_.model == CAVS_MODEL_TREELSTM && cfg_.H > 384) || (cfg_.model == CAVS_MODEL_LSTM && cfg_.H >= 384) ? 256 : 64;
+}
+
+// Rounds of at most this many rows keep a training pass's message flow a forest, whose backward rounds are one launch each and
+// can be resident.  A round above fused_rows() is slower as such a launch than as products, but with one of them in the batch
+// every round was: 128 trees of 30 .. 120 leaves (largest round 3086) gain 1.07 (Tree-FC, H = 64) .. 1.32 (H = 256) and 1.11 ..
+// 1.64 (Tree-LSTM), 256 of them (6181) 1.01 (Tree-LSTM, H = 384) .. 1.18, but Tree-FC 0.92 at H = 64 and 0.96 at 128; at 10400 rows it
+// is 0.85 .. 1.11, at 23700 0.6 .. 1.0.
+int Engine::forest_rows() const {
+  const int fused = fused_rows();
+  if (cell_ || cfg_.fused_round_rows != 0 || nch_ != 2 || group_limit() <= 0) return fused;
+  return std::max(fused, cfg_.model == CAVS_MODEL_TREELSTM || cfg_.H >= 192 ? 8192 : 4096);
 }
 
 // Lists of the group launches for the batch whose index lists are given, and the tiles they run in.
@@ -825,7 +843,7 @@ void Engine::build_late_lists(HostLists &h) {
   const int N = N_;
   int *t2j = h.host.get(), *pair = t2j + N, *child = pair + N, *kids = child + (size_t)nch_ * N + s.B, *orphans = kids + (size_t)nch_ * N;
   // (the resident launches of a forward pass read the lists whatever runs the larger rounds)
-  const bool forest = build_forest_lists(s, nch_, lists_forward_only() ? N : fused_rows(), pair, child, kids, orphans, &n_orphans_);
+  const bool forest = build_forest_lists(s, nch_, lists_forward_only() ? N : forest_rows(), pair, child, kids, orphans, &n_orphans_);
   forest_ = forest && !lists_forward_only();
   if (!forest) return;
   if (group_limit() > 0) build_group_plan(t2j, pair, child, kids, orphans, h.host.get() + group_at_);
@@ -1038,10 +1056,10 @@ void Engine::schedule_on_device(const int *graph, int B, int maxlen) {
   d_orphans_ = orph;
   // every sample has one root, so B slab rows send no message; the message flow of a well-formed
   // batch is a forest by construction, what remains to ask is whether every round with children
-  // runs as a fused launch
+  // may be a launch of its own
   n_orphans_ = B;
   forest_ = !cfg_.split_backward_rounds && fused_rows() > 0;
-  for (int r = 1; r < R && forest_; r++) forest_ = s.rounds[r].n <= fused_rows();
+  for (int r = 1; r < R && forest_; r++) forest_ = s.rounds[r].n <= forest_rows();
   tail_ = TailPlan();
   group_ = GroupLists();
   // The group launches' block is host work on all of the lists: they come back, the block goes up.

@@ -450,6 +450,8 @@ class Engine {
   bool wide_head() const;
   // rounds of at most this many rows run as fused launches (0: none)
   int fused_rows() const;
+  // rounds of at most this many rows keep the message flow a forest
+  int forest_rows() const;
 
   // (the tail launches, continued)
   TailPlan tail_;

@@ -434,6 +434,8 @@ static int group_tile_rows(const std::vector<int> &per, int rounds, int slice) {
   return wide < four ? 16 : 4;
 }
 
+static constexpr int kUnevenShare = 64;
+
 void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pair, const int *child, const int *kid_rows, const int *orphans,
                        int n_orphans, int lim, int groups, int slice, bool only_wide, GroupLists *out, int *block) {
   const bool back = orphans != nullptr;
@@ -467,6 +469,13 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
         const int i = group[comp[b]] * nr + (k - k0);
         cell[b - lo] = i;
         ok &= ++per[i] <= lim;
+      }
+    // A share of more rows than a workgroup takes in two slices wants the groups evenly loaded: where few trees hold a round's
+    // rows, most of the device would wait for one group.
+    for (int k = k0; k < R && ok && lim > kUnevenShare; k++)
+      for (int g = 0; g < G && ok; g++) {
+        const long share = per[(size_t)g * nr + (k - k0)];
+        ok = share <= kUnevenShare || share * groups <= 2L * s.rounds[k].n;
       }
     if (!ok) continue;
 

@@ -152,3 +152,25 @@ def test_a_forward_pass_plans_for_itself(model, H, B):
         close(got[k], v, k)
     for x in (ref, s, few):
         x.close()
+
+
+@pytest.mark.parametrize("model,H,schedule,plan_cache", [("treelstm", 64, "host", 0), ("treelstm", 512, "device", 0), ("treefc", 96, "host", 2),
+                                                         ("treefc", 512, "device", 2)])
+def test_training_with_a_round_above_the_fused_limit(model, H, schedule, plan_cache):
+    """A round of more rows than a fused launch is used for (2048) leaves a training pass's smaller rounds resident: what products
+    and launches of their own give (other orders of the same sums), in both passes and on a batch seen before."""
+    w = small_workload(model, 81, B=1700, H=H, E=12, V=31, C=5)
+    sizes = np.diff(session.schedule_trace(w["graph"])["round2offset"])
+    assert 2048 < sizes[1:].max() <= 4096
+    # (a limit that is given is what it was)
+    s, ref = _session(model, H, w, schedule=schedule, plan_cache=plan_cache), _session(model, H, w, fused_round_rows=2048)
+    for k in range(2):
+        for x in (s, ref):
+            x.step(w["graph"], w["x"], w["labels"], backward=True, lr=1e-6)
+        assert s.counter("tail_rounds") > 0 and ref.counter("tail_rounds") == 0
+        close(s.fetch("graph_out"), ref.fetch("graph_out"), "graph_out")
+        got, want = s.grads(), ref.grads()
+        for name, v in want.items():
+            close(got[name], v, name)
+    for x in (s, ref):
+        x.close()

@@ -248,3 +248,23 @@ def test_what_planning_a_new_batch_takes(nchild, B, lo, hi):
     fwd = session.group_lists(graph, nchild, forward_only=True)
     assert fwd["first"] == g["first"] and fwd["bwd"] is None
     np.testing.assert_array_equal(fwd["fwd"]["recs"], g["fwd"]["recs"])
+
+
+@pytest.mark.parametrize("large", [1, 3, 64])
+def test_a_large_share_wants_the_groups_evenly_loaded(large):
+    """Eight groups: a round is resident with more than 64 of its rows in one group only where that is at most twice an even share."""
+    rng = synth.SplitMix64(51)
+    trees = [synth.random_binary_tree(rng, 900 if i < large else 2) for i in range(64)]
+    graph = synth.pack_graph(trees, 1799)
+    sizes = np.diff(session.schedule_trace(graph)["round2offset"])
+    for limit in (64, 512, 1 << 20):
+        g = session.group_lists(graph, 2, rows_limit=limit, groups=8)
+        share = np.zeros((8, len(sizes)), int)
+        of = np.repeat(np.arange(len(sizes)), sizes)
+        for i, (first, n, _, _) in enumerate(g["fwd"]["groups"]):
+            for at, rows, _, _ in g["fwd"]["lists"][first:first + n]:
+                np.add.at(share[i], of[g["fwd"]["recs"][at:at + rows, 0]], 1)
+        most = share.max(0)
+        assert (most <= limit).all() and ((most <= 64) | (8 * most <= 2 * sizes)).all()
+        if large == 64 and limit == 1 << 20:
+            assert most.max() > 512
