@@ -165,6 +165,7 @@ struct GroupFwdArgs {
   float *G, *hlr, *gates, *msg, *go;  // whole-batch slabs (msg, go may be null where the function allows)
   int H, act;
   GroupPlan plan;
+  bool x_by_vertex;    // Tree-FC: xW in the order of graph_out
 };
 
 // record of a row: {slab row, slab rows of its two children, row of dret of child 0}, {that of child 1, ...}
@@ -257,7 +258,8 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
     const int e_out = a.go && eon ? rt[2 * eb + 1].x : -1;
     float xw[4] = {0.f, 0.f, 0.f, 0.f};
     {
-      const float *p = row_at(x_rows, max(rec.x, 0), x_ld) + ej;
+      const int row = MODEL == GROUP_TREEFC && a.x_by_vertex ? rt[eon ? 2 * eb + 1 : 1].x : rec.x;
+      const float *p = row_at(x_rows, max(row, 0), x_ld) + ej;
 #pragma unroll
       for (int k = 0; k < (MODEL == GROUP_TREEFC ? 1 : 4); k++) xw[k] = p[k * H];
     }

@@ -15,6 +15,15 @@ static int group_plan(const char *who, const cavs_group_plan *p, int H, bool who
   return CAVS_OK;
 }
 
+static int treefc_group_fwd(const char *who, float *pool, const float *x, bool by_vertex, const float *Wp, const float *bias, float *G, float *msg,
+                            float *graph_out, int H, int act, const cavs_group_plan *plan, void *stream) {
+  GroupFwdArgs a{pool, x, H, Wp, bias, G, nullptr, nullptr, msg, graph_out, H, act, {}, by_vertex};
+  if (int rc = group_plan(who, plan, H, line_rows(pool, H), &a.plan)) return rc;
+  CAVS_REQUIRE(pool && Wp && G && msg && (act == 0 || act == 1), "%s: null pointer or act=%d", who, act);
+  CAVS_REQUIRE(aligned16(pool) && aligned16(Wp), "%s: pool and Wp must be 16-byte aligned", who);
+  return a.plan.wide ? group_fwd<GROUP_TREEFC, true>(a, stream) : group_fwd<GROUP_TREEFC, false>(a, stream);
+}
+
 }  // namespace cavs
 
 using namespace cavs;
@@ -45,11 +54,12 @@ int cavs_lstm_group_fwd(float *pool, const float *xW, int ld_xw, const float *Wh
 
 int cavs_treefc_group_fwd(float *pool, const float *x, const float *Wp, const float *bias, float *G, float *msg, float *graph_out, int H,
                           int act, const cavs_group_plan *plan, void *stream) {
-  GroupFwdArgs a{pool, x, H, Wp, bias, G, nullptr, nullptr, msg, graph_out, H, act, {}};
-  if (int rc = group_plan("cavs_treefc_group_fwd", plan, H, line_rows(pool, H), &a.plan)) return rc;
-  CAVS_REQUIRE(pool && Wp && G && msg && (act == 0 || act == 1), "cavs_treefc_group_fwd: null pointer or act=%d", act);
-  CAVS_REQUIRE(aligned16(pool) && aligned16(Wp), "cavs_treefc_group_fwd: pool and Wp must be 16-byte aligned");
-  return a.plan.wide ? group_fwd<GROUP_TREEFC, true>(a, stream) : group_fwd<GROUP_TREEFC, false>(a, stream);
+  return treefc_group_fwd("cavs_treefc_group_fwd", pool, x, false, Wp, bias, G, msg, graph_out, H, act, plan, stream);
+}
+
+int cavs_treefc_group_pull_fwd(float *pool, const float *x, const float *Wp, const float *bias, float *G, float *msg, float *graph_out, int H,
+                               int act, const cavs_group_plan *plan, void *stream) {
+  return treefc_group_fwd("cavs_treefc_group_pull_fwd", pool, x, true, Wp, bias, G, msg, graph_out, H, act, plan, stream);
 }
 
 int cavs_treelstm_group_bwd(float *dxW, int ld_dxw, float *dF, float *dc, const float *UTp, const float *gates, const float *G,

@@ -604,6 +604,7 @@ struct TreeFcLeavesArgs {
   float *msg, *pool, *go;
   const int *out_rows;
   int n, H, act;
+  const int *x_rows;  // null: row r of x
 };
 
 template <int W>
@@ -613,12 +614,13 @@ __global__ void treefc_round_leaves_fwd_kernel(TreeFcLeavesArgs a) {
   if (idx >= (long)a.n * hw) return;
   const int r = (int)(idx / hw), j = (int)(idx % hw) * W;
   const int dst = a.pair[r], out = a.go ? a.out_rows[r] : -1;
+  const long xr = a.x_rows ? a.x_rows[r] : r;
   float h[W];
 #pragma unroll
   for (int k = 0; k < W; k++) {
     float t = 0.f;
     if (a.bias) t += a.bias[j + k];
-    if (a.x) t += a.x[(long)r * H + j + k];
+    if (a.x) t += a.x[xr * H + j + k];
     h[k] = a.act ? tanh_r(t) : (t > 0.f ? t : 0.f);
   }
   stw<W>(a.msg + (long)r * H + j, h);
@@ -860,11 +862,16 @@ int cavs_treefc_round_fwd(float *pool, const int *child, const int *pair, const 
 
 int cavs_treefc_round_leaves_fwd(float *pool, const int *pair, const float *bias, const float *x, float *msg,
                                  float *graph_out, const int *out_rows, int n, int H, int act, void *stream) {
+  return cavs_treefc_round_leaves_pull_fwd(pool, pair, bias, x, nullptr, msg, graph_out, out_rows, n, H, act, stream);
+}
+
+int cavs_treefc_round_leaves_pull_fwd(float *pool, const int *pair, const float *bias, const float *x, const int *x_rows, float *msg,
+                                      float *graph_out, const int *out_rows, int n, int H, int act, void *stream) {
   CAVS_REQUIRE(n >= 0 && H > 0 && (act == 0 || act == 1), "cavs_treefc_round_leaves_fwd: bad argument n=%d H=%d act=%d", n, H, act);
   if (n == 0) return CAVS_OK;
   CAVS_REQUIRE(pool && pair && msg, "cavs_treefc_round_leaves_fwd: null pointer");
   CAVS_REQUIRE(!graph_out || out_rows, "cavs_treefc_round_leaves_fwd: graph_out needs out_rows");
-  TreeFcLeavesArgs a{bias, x, pair, msg, pool, graph_out, out_rows, n, H, act};
+  TreeFcLeavesArgs a{bias, x, pair, msg, pool, graph_out, out_rows, n, H, act, x_rows};
   const bool vec = H % 4 == 0 && all16({pool, bias, x, msg, graph_out});
   launch_pointwise(a, n, H, vec, as_stream(stream), treefc_round_leaves_fwd_kernel<4>, treefc_round_leaves_fwd_kernel<1>);
   CAVS_LAUNCH_CHECK();

@@ -2229,20 +2229,42 @@ void Engine::treefc_forward() {
   const int N = N_, H = cfg_.H;
   const float *W = param("W").w;
   const float *Bv = cfg_.use_bias ? param("Bv").w : nullptr;
-  if (cfg_.use_x) gather(xs_.get(), H, d_x_, uH_, d_t2j_, N, uH_);
-  if (!sched_->batching) check(cavs_zero(G_.get(), (size_t)N * 2 * H * 4, stream_));
-  finish_lists();
   const int fused = fused_rows();
-  out_folded_ = fused > 0 && sched_->max_round <= fused && fwd_out_ != nullptr;
+  // The leaves' launch and the group launch read x by vertex, where it has their width; else, and for rounds that are launches
+  // of their own, its rows are brought into slab order first.  A leaf multiplies nothing: its round is one launch whatever its
+  // rows.  (64 trees of 2 .. 64 leaves, H = 256, 4200 vertices: four launches less where the leaves are more than 2048, one
+  // elsewhere, 4.6 to 5.0 us each of a step of 122)
+  const bool by_vertex = cfg_.use_x && uH_ == H && fused > 0;
+  if (cfg_.use_x && !by_vertex) gather(xs_.get(), H, d_x_, uH_, d_t2j_, N, uH_);
+  if (!sched_->batching) check(cavs_zero(G_.get(), (size_t)N * 2 * H * 4, stream_));
+  bool folds = fused > 0 && fwd_out_ != nullptr;
+  for (const Round &r : sched_->rounds) folds &= r.n <= fused || leaf_round(r);
+  out_folded_ = folds;
   float *go = out_folded_ ? fwd_out_ : nullptr;
+  size_t lead = 0;  // the leaves do not wait for the lists
+  for (; fused > 0 && lead < sched_->rounds.size() && leaf_round(sched_->rounds[lead]); lead++) {
+    const Round &r = sched_->rounds[lead];
+    const size_t off = r.offset;
+    CAVS_TIMED(K_GATES, cavs_treefc_round_leaves_pull_fwd(pool_.get(), d_pair_ + off, Bv, by_vertex ? d_x_ : cfg_.use_x ? xs_.at(off * H) : nullptr,
+                                                          by_vertex ? d_t2j_ + off : nullptr, msg_.at(off * H), go, d_t2j_ + off, r.n, H, cfg_.act,
+                                                          stream_));
+    c_scatter_rows_ += r.n;
+    c_launches_ += 1;
+  }
+  finish_lists();
+  if (by_vertex) {
+    const int from = lead < sched_->rounds.size() ? sched_->rounds[lead].offset : N, to = group_.first >= 0 ? sched_->rounds[group_.first].offset : N;
+    if (from < to) gather(xs_.at((size_t)from * H), H, d_x_, H, d_t2j_ + from, to - from, H);
+  }
   if (group_.first >= 0) ensure_packed();
-  for (size_t rk = 0; rk < sched_->rounds.size(); rk++) {
+  for (size_t rk = lead; rk < sched_->rounds.size(); rk++) {
     const Round &r = sched_->rounds[rk];
     if (group_.first >= 0 && (int)rk == group_.first) {
       const cavs_group_plan plan = group_plan(group_.fwd);
       last_launch(1, out_folded_, [&] {
-        CAVS_TIMED(K_ROUND, cavs_treefc_group_fwd(pool_.get(), cfg_.use_x ? xs_.get() : nullptr, Upk_.get(), Bv, G_.get(), msg_.get(), go, H, cfg_.act,
-                                                  &plan, stream_));
+        CAVS_TIMED(K_ROUND, (by_vertex ? cavs_treefc_group_pull_fwd : cavs_treefc_group_fwd)(
+                                pool_.get(), by_vertex ? d_x_ : cfg_.use_x ? xs_.get() : nullptr, Upk_.get(), Bv, G_.get(), msg_.get(), go, H, cfg_.act,
+                                &plan, stream_));
       });
       group_launched();
       break;
@@ -2250,16 +2272,11 @@ void Engine::treefc_forward() {
     const size_t off = r.offset;
     const float *xin = cfg_.use_x ? xs_.at(off * H) : nullptr;
     float *msg = msg_.at(off * H);
-    if (r.n <= fused) {  // one launch: Gather, [h_l;h_r]*W, activation, Scatter, Push/PopRet
-      if (leaf_round(r)) {
-        CAVS_TIMED(K_GATES, cavs_treefc_round_leaves_fwd(pool_.get(), d_pair_ + off, Bv, xin, msg, go, d_t2j_ + off, r.n, H, cfg_.act,
-                                                         stream_));
-      } else {
-        CAVS_TIMED(K_ROUND, cavs_treefc_round_fwd(pool_.get(), d_child_ + 2 * off, d_pair_ + off, W, Bv, xin, G_.at(2 * off * H), msg, go,
-                                                  d_t2j_ + off, r.n, H, cfg_.act, stream_));
-        c_round_flops_ += 2.0 * r.n * H * 2.0 * H;
-        c_gather_rows_ += 2.0 * r.n;
-      }
+    if (r.n <= fused && !leaf_round(r)) {  // one launch: Gather, [h_l;h_r]*W, activation, Scatter, Push/PopRet
+      CAVS_TIMED(K_ROUND, cavs_treefc_round_fwd(pool_.get(), d_child_ + 2 * off, d_pair_ + off, W, Bv, xin, G_.at(2 * off * H), msg, go,
+                                                d_t2j_ + off, r.n, H, cfg_.act, stream_));
+      c_round_flops_ += 2.0 * r.n * H * 2.0 * H;
+      c_gather_rows_ += 2.0 * r.n;
       c_scatter_rows_ += r.n;
       c_launches_ += 1;
       continue;

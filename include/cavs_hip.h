@@ -560,6 +560,9 @@ int cavs_lstm_group_bwd(float *da, int ld_da, float *dc, const float *WhTp, cons
                         int leaf_rows, int H, const cavs_group_plan *plan, void *stream);
 int cavs_treefc_group_fwd(float *pool, const float *x, const float *Wp, const float *bias, float *G, float *msg, float *graph_out,
                           int H, int act, const cavs_group_plan *plan, void *stream);
+/* x by vertex: row r of the plan reads x's row of graph_out's (the fifth int of its record) */
+int cavs_treefc_group_pull_fwd(float *pool, const float *x, const float *Wp, const float *bias, float *G, float *msg, float *graph_out,
+                               int H, int act, const cavs_group_plan *plan, void *stream);
 int cavs_treefc_group_bwd(float *dz, const float *WTp, const float *h, const float *dret, int H, int act, const cavs_group_plan *plan,
                           void *stream);
 int cavs_treelstm_tail_fwd(float *pool, const int *child, const int *pair, const float *xW, int ld_xw,
@@ -635,6 +638,10 @@ int cavs_treefc_round_fwd(float *pool, const int *child, const int *pair, const 
 int cavs_treefc_round_leaves_fwd(float *pool, const int *pair, const float *bias, const float *x,
                                  float *msg, float *graph_out, const int *out_rows, int n, int H,
                                  int act, void *stream);
+/* vertex b reads row x_rows[b] of x (x_rows null: row b) */
+int cavs_treefc_round_leaves_pull_fwd(float *pool, const int *pair, const float *bias, const float *x,
+                                      const int *x_rows, float *msg, float *graph_out,
+                                      const int *out_rows, int n, int H, int act, void *stream);
 /* dz = act'(h) * (d msg read from dpool row pair[b] + d return value) */
 int cavs_treefc_round_bwd(const float *dpool, const int *pair, const float *dret, const int *dret_rows,
                           const float *h, float *dz, int n, int H, int act, void *stream);

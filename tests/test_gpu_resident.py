@@ -174,3 +174,27 @@ def test_training_with_a_round_above_the_fused_limit(model, H, schedule, plan_ca
             close(got[name], v, name)
     for x in (s, ref):
         x.close()
+
+
+@pytest.mark.parametrize("H,B,kw", [(32, 5, {}), (96, 40, {}), (256, 600, {}), (64, 600, dict(tail_rows=-1)), (64, 600, dict(fused_round_rows=300)),
+                                    (40, 30, {})])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_vertex_inputs_read_by_vertex(H, B, kw, shift):
+    """Tree-FC: the leaves and the resident rounds read the caller's rows where they lie (also off a 16-byte boundary), rounds that are
+    launches of their own have them brought into order: what rows in order give.  600 trees: more leaves than a fused launch's limit."""
+    import torch
+
+    w = small_workload("treefc", 91, B=B, H=H, E=12, V=31, C=5)
+    s, ref = _session("treefc", H, w, **kw), _session("treefc", H, w, fused_round_rows=-1)
+    room = torch.zeros(w["x"].size + 4, device="cuda")
+    x = room[shift:shift + w["x"].size]
+    x.copy_(torch.from_numpy(w["x"].reshape(-1)))
+    for k in range(2):
+        s.step(w["graph"], x.view(-1, H), torch.from_numpy(w["labels"]).cuda(), backward=True, lr=1e-6)
+        ref.step(w["graph"], w["x"], w["labels"], backward=True, lr=1e-6)
+        close(s.fetch("graph_out"), ref.fetch("graph_out"), "graph_out")
+        got, want = s.grads(), ref.grads()
+        for name, v in want.items():
+            close(got[name], v, name)
+    for z in (s, ref):
+        z.close()
