@@ -605,6 +605,7 @@ struct TreeFcLeavesArgs {
   const int *out_rows;
   int n, H, act;
   const int *x_rows;  // null: row r of x
+  int whole_tanh;     // tanhf, which keeps its relative accuracy near zero
 };
 
 template <int W>
@@ -621,7 +622,7 @@ __global__ void treefc_round_leaves_fwd_kernel(TreeFcLeavesArgs a) {
     float t = 0.f;
     if (a.bias) t += a.bias[j + k];
     if (a.x) t += a.x[xr * H + j + k];
-    h[k] = a.act ? tanh_r(t) : (t > 0.f ? t : 0.f);
+    h[k] = !a.act ? (t > 0.f ? t : 0.f) : a.whole_tanh ? tanhf(t) : tanh_r(t);
   }
   stw<W>(a.msg + (long)r * H + j, h);
   if (dst >= 0) stw<W>(a.pool + (long)dst * H + j, h);
@@ -862,16 +863,16 @@ int cavs_treefc_round_fwd(float *pool, const int *child, const int *pair, const 
 
 int cavs_treefc_round_leaves_fwd(float *pool, const int *pair, const float *bias, const float *x, float *msg,
                                  float *graph_out, const int *out_rows, int n, int H, int act, void *stream) {
-  return cavs_treefc_round_leaves_pull_fwd(pool, pair, bias, x, nullptr, msg, graph_out, out_rows, n, H, act, stream);
+  return cavs_treefc_round_leaves_pull_fwd(pool, pair, bias, x, nullptr, msg, graph_out, out_rows, n, H, act, 0, stream);
 }
 
 int cavs_treefc_round_leaves_pull_fwd(float *pool, const int *pair, const float *bias, const float *x, const int *x_rows, float *msg,
-                                      float *graph_out, const int *out_rows, int n, int H, int act, void *stream) {
+                                      float *graph_out, const int *out_rows, int n, int H, int act, int whole_tanh, void *stream) {
   CAVS_REQUIRE(n >= 0 && H > 0 && (act == 0 || act == 1), "cavs_treefc_round_leaves_fwd: bad argument n=%d H=%d act=%d", n, H, act);
   if (n == 0) return CAVS_OK;
   CAVS_REQUIRE(pool && pair && msg, "cavs_treefc_round_leaves_fwd: null pointer");
   CAVS_REQUIRE(!graph_out || out_rows, "cavs_treefc_round_leaves_fwd: graph_out needs out_rows");
-  TreeFcLeavesArgs a{bias, x, pair, msg, pool, graph_out, out_rows, n, H, act, x_rows};
+  TreeFcLeavesArgs a{bias, x, pair, msg, pool, graph_out, out_rows, n, H, act, x_rows, whole_tanh};
   const bool vec = H % 4 == 0 && all16({pool, bias, x, msg, graph_out});
   launch_pointwise(a, n, H, vec, as_stream(stream), treefc_round_leaves_fwd_kernel<4>, treefc_round_leaves_fwd_kernel<1>);
   CAVS_LAUNCH_CHECK();

@@ -158,7 +158,7 @@ _SIGS = {
     "cavs_lstm_round_bwd_gates": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
     "cavs_treefc_round_fwd": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
     "cavs_treefc_round_leaves_fwd": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
-    "cavs_treefc_round_leaves_pull_fwd": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
+    "cavs_treefc_round_leaves_pull_fwd": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
     "cavs_treefc_round_bwd": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
     "cavs_round_bwd_children": [_P, _I, _I, _P, _I, _I, _P, _P, _I, _I, _I, _P],
     "cavs_lstm_round_bwd_children_gates": [_P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],

@@ -177,13 +177,15 @@ int Engine::tail_limit() const {
 // a forward pass of most sizes level with those launches (0.84 .. 1.15 of the time with 256, by the batch).  Where a group is all
 // of its chiplet's workgroups a larger share is the faster one: trees of 256 parses at H = 512 0.463 -> 0.442 ms a pass, chains
 // in batches of 1024 0.741 -> 0.714 ms, at H = 384 0.708 -> 0.618 (Tree-LSTM at H = 384: no difference; Tree-FC at 512, one product
-// of its row: 0.80 -> 0.80 .. 1.39 -> 1.42).  A training pass gains both ways: H = 512, 256 parses 1.289 -> 1.151 ms a step, Tree-FC
-// 0.422 -> 0.374, chains in batches of 1024 1.745 -> 1.538; H = 256 0.697 -> 0.655.
+// of its row: 0.80 -> 0.80 .. 1.39 -> 1.42).  A training pass gains both ways: H = 512, 256 parses 1.289 -> 1.151 ms a step,
+// chains in batches of 1024 1.745 -> 1.538; H = 256 0.697 -> 0.655.  Tree-FC keeps its rounds' order of sums above H = 256: its
+// training multiplies a difference in rounding by up to 1.4 a step there (1e-6 after one step at H = 512, 2e-4 after 16, whichever
+// two orders are compared), at 256 by 1.05.
 int Engine::group_limit() const {
   if (!resident_ || fused_rows() <= 0 || (cell_ && cell_->rounds.empty()) || !cavs_group_rounds_ok(cfg_.H)) return 0;
   if (cfg_.tail_rows > 0) return tail_limit() > 0 ? 0 : cfg_.tail_rows;
   if (cell_) return 64;
-  if (!lists_forward_only()) return 512;
+  if (!lists_forward_only()) return cfg_.model == CAVS_MODEL_TREEFC && cfg_.H > 256 ? 64 : 512;
   return (cfg_.model == CAVS_MODEL_TREELSTM && cfg_.H > 384) || (cfg_.model == CAVS_MODEL_LSTM && cfg_.H >= 384) ? 256 : 64;
 }
 
@@ -191,10 +193,11 @@ int Engine::group_limit() const {
 // can be resident.  A round above fused_rows() is slower as such a launch than as products, but with one of them in the batch
 // every round was: 128 trees of 30 .. 120 leaves (largest round 3086) gain 1.07 (Tree-FC, H = 64) .. 1.32 (H = 256) and 1.11 ..
 // 1.64 (Tree-LSTM), 256 of them (6181) 1.01 (Tree-LSTM, H = 384) .. 1.18, but Tree-FC 0.92 at H = 64 and 0.96 at 128; at 10400 rows it
-// is 0.85 .. 1.11, at 23700 0.6 .. 1.0.
+// is 0.85 .. 1.11, at 23700 0.6 .. 1.0.  (Tree-FC up to H = 256, as above)
 int Engine::forest_rows() const {
   const int fused = fused_rows();
   if (cell_ || cfg_.fused_round_rows != 0 || nch_ != 2 || group_limit() <= 0) return fused;
+  if (cfg_.model == CAVS_MODEL_TREEFC && cfg_.H > 256) return fused;
   return std::max(fused, cfg_.model == CAVS_MODEL_TREELSTM || cfg_.H >= 192 ? 8192 : 4096);
 }
 
@@ -2247,7 +2250,7 @@ void Engine::treefc_forward() {
     const size_t off = r.offset;
     CAVS_TIMED(K_GATES, cavs_treefc_round_leaves_pull_fwd(pool_.get(), d_pair_ + off, Bv, by_vertex ? d_x_ : cfg_.use_x ? xs_.at(off * H) : nullptr,
                                                           by_vertex ? d_t2j_ + off : nullptr, msg_.at(off * H), go, d_t2j_ + off, r.n, H, cfg_.act,
-                                                          stream_));
+                                                          r.n > fused, stream_));
     c_scatter_rows_ += r.n;
     c_launches_ += 1;
   }

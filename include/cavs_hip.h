@@ -638,10 +638,11 @@ int cavs_treefc_round_fwd(float *pool, const int *child, const int *pair, const 
 int cavs_treefc_round_leaves_fwd(float *pool, const int *pair, const float *bias, const float *x,
                                  float *msg, float *graph_out, const int *out_rows, int n, int H,
                                  int act, void *stream);
-/* vertex b reads row x_rows[b] of x (x_rows null: row b) */
+/* vertex b reads row x_rows[b] of x (x_rows null: row b); whole_tanh: tanh as the library's tanhf, not the 1e-7 absolute of the rounds */
 int cavs_treefc_round_leaves_pull_fwd(float *pool, const int *pair, const float *bias, const float *x,
                                       const int *x_rows, float *msg, float *graph_out,
-                                      const int *out_rows, int n, int H, int act, void *stream);
+                                      const int *out_rows, int n, int H, int act, int whole_tanh,
+                                      void *stream);
 /* dz = act'(h) * (d msg read from dpool row pair[b] + d return value) */
 int cavs_treefc_round_bwd(const float *dpool, const int *pair, const float *dret, const int *dret_rows,
                           const float *h, float *dz, int n, int H, int act, void *stream);

@@ -155,7 +155,7 @@ def test_a_forward_pass_plans_for_itself(model, H, B):
 
 
 @pytest.mark.parametrize("model,H,schedule,plan_cache", [("treelstm", 64, "host", 0), ("treelstm", 512, "device", 0), ("treefc", 96, "host", 2),
-                                                         ("treefc", 512, "device", 2)])
+                                                         ("treefc", 256, "device", 2)])
 def test_training_with_a_round_above_the_fused_limit(model, H, schedule, plan_cache):
     """A round of more rows than a fused launch is used for (2048) leaves a training pass's smaller rounds resident: what products
     and launches of their own give (other orders of the same sums), in both passes and on a batch seen before."""
