@@ -403,8 +403,8 @@ bool Engine::update_jobs(float *w, float *g, float lr, std::vector<cavs_task> *o
   }
   if (Upk_.capacity() == 0) return false;
   const long long H = cfg_.H;
-  // the transposed copy as well, where the resident backward launch reads one (a recorded step makes it each time)
-  float *tp = UTp_.capacity() > 0 && !cfg_.graph_replay ? UTp_.get() : nullptr;
+  // the transposed copy as well, where the resident backward launch reads one
+  float *tp = UTp_.capacity() > 0 ? UTp_.get() : nullptr;
   if (cfg_.model == CAVS_MODEL_TREELSTM && w == param("U").w) {
     out->push_back({CAVS_TASK_SGD_PACK, lr, H, 3 * H, 0, Upk_.get(), w, g, tp});
     out->push_back({CAVS_TASK_SGD_PACK, lr, H, H, 0, Upk_.at((size_t)3 * H * H), w + 3 * H * H, g + 3 * H * H, tp ? tp + 3 * H * H : nullptr});
@@ -1316,6 +1316,7 @@ Engine::StepSig Engine::step_signature(const void *x, const void *labels, bool b
   g.emb_sparse_valid = emb_sparse_valid_;
   g.emb_cleared = emb_cleared_;
   g.upk_valid = upk_valid_;
+  g.utp_valid = utp_valid_;
   g.wfct_valid = wfct_valid_;
   g.emb_dirty_n = emb_dirty_n_;
   g.pairing = cfg_.pairing;
@@ -1332,6 +1333,7 @@ Engine::StepState Engine::step_state() const {
   st.emb_sparse_valid = emb_sparse_valid_;
   st.emb_cleared = emb_cleared_;
   st.upk_valid = upk_valid_;
+  st.utp_valid = utp_valid_;
   st.wfct_valid = wfct_valid_;
   st.tail_pending = tail_pending_;
   st.fwd_out = fwd_out_;
@@ -1352,6 +1354,7 @@ void Engine::restore_step_state(const StepState &st) {
   emb_sparse_valid_ = st.emb_sparse_valid;
   emb_cleared_ = st.emb_cleared;
   upk_valid_ = st.upk_valid;
+  utp_valid_ = st.utp_valid;
   wfct_valid_ = st.wfct_valid;
   tail_pending_ = tail_pending_ || st.tail_pending;
   fwd_out_ = st.fwd_out;
@@ -1417,7 +1420,7 @@ void Engine::step(const int *graph, int B, int maxlen, const void *x, const void
   trains_ = may_backward_ = backward;
   whole_step_ = false;
   begin_step(graph, B, maxlen);
-  whole_step_ = backward && !cfg_.graph_replay && !profile_;
+  whole_step_ = backward && !profile_;
   const int N = N_;
   const bool needs_x = cfg_.model != CAVS_MODEL_TREEFC || cfg_.use_x;
   const size_t xw = cfg_.model == CAVS_MODEL_TREEFC ? uH_ : 1;
@@ -1731,7 +1734,7 @@ void Engine::treelstm_backward() {
   if (grouped_tp && !utp_valid_) {
     opening.push_back({CAVS_TASK_PACK_T, 0.f, H, 3 * H, 0, UTp_.get(), const_cast<float *>(U), nullptr, nullptr});
     opening.push_back({CAVS_TASK_PACK_T, 0.f, H, H, 0, UTp_.at((size_t)3 * H * H), const_cast<float *>(U) + (size_t)3 * H * H, nullptr, nullptr});
-    utp_valid_ = !cfg_.graph_replay && param("U").w == param("U").own_w.get();
+    utp_valid_ = param("U").w == param("U").own_w.get();
   }
   if (fused > 0 && rest) {  // U_iou^T and U_f^T: the B operand of the children products, k-major
     const int kind = packed ? CAVS_TASK_PACK_T : CAVS_TASK_TRANSPOSE;
@@ -1980,7 +1983,7 @@ void Engine::clear_embedding(std::vector<cavs_task> *tasks) {
 // weights written by the update, the roots in the resident launch and the head's sums in the launch of the updates, nothing opens a
 // backward pass any more: 64 trees, H = 512, 329 -> 324 us a step, 25 trees, H = 150, 189 -> 184.)
 bool Engine::leaves_with_company(cavs_task leaves) {
-  if (!whole_step_ || cfg_.H % 4) return false;
+  if (!whole_step_ || cfg_.graph_replay || cfg_.H % 4) return false;
   std::vector<cavs_task> tasks{leaves};
   clear_embedding(&tasks);
   if (tasks.size() == 1) return false;
@@ -2129,7 +2132,7 @@ void Engine::lstm_backward() {
     opening.push_back({packed ? CAVS_TASK_PACK_T : CAVS_TASK_TRANSPOSE, 0.f, H, 4 * H, 0, UT_.get(), const_cast<float *>(Wh), nullptr, nullptr});
   if (grouped_tp && !utp_valid_) {
     opening.push_back({CAVS_TASK_PACK_T, 0.f, H, 4 * H, 0, UTp_.get(), const_cast<float *>(Wh), nullptr, nullptr});
-    utp_valid_ = !cfg_.graph_replay && param("W").w == param("W").own_w.get();
+    utp_valid_ = param("W").w == param("W").own_w.get();
   }
   backward_prologue(opening, true);
   const bool folded = forest_;  // one launch per round, as in treelstm_backward
@@ -2235,7 +2238,7 @@ void Engine::treefc_forward() {
   const int fused = fused_rows();
   // The leaves' launch and the group launch read x by vertex, where it has their width; else, and for rounds that are launches
   // of their own, its rows are brought into slab order first.  A leaf multiplies nothing: its round is one launch whatever its
-  // rows.  (64 trees of 2 .. 64 leaves, H = 256, 4200 vertices: four launches less where the leaves are more than 2048, one
+  // rows (above the fused limit with the tanhf of the launches that ran it there).  (64 trees of 2 .. 64 leaves, H = 256, 4200 vertices: four launches less where the leaves are more than 2048, one
   // elsewhere, 4.6 to 5.0 us each of a step of 122)
   const bool by_vertex = cfg_.use_x && uH_ == H && fused > 0;
   if (cfg_.use_x && !by_vertex) gather(xs_.get(), H, d_x_, uH_, d_t2j_, N, uH_);
@@ -2316,7 +2319,7 @@ void Engine::treefc_backward() {
     if (rest) opening.push_back({CAVS_TASK_TRANSPOSE, 0.f, 2 * H, H, 0, UT_.get(), const_cast<float *>(W), nullptr, nullptr});
     if (group_.first >= 0 && !utp_valid_) {
       opening.push_back({CAVS_TASK_PACK_T, 0.f, 2 * H, H, 0, UTp_.get(), const_cast<float *>(W), nullptr, nullptr});
-      utp_valid_ = !cfg_.graph_replay && param("W").w == param("W").own_w.get();
+      utp_valid_ = param("W").w == param("W").own_w.get();
     }
     backward_prologue(opening, false);
   } else {

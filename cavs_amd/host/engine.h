@@ -291,13 +291,13 @@ class Engine {
   // state it left is then put in place as if the launches had been issued one by one.
   struct StepSig {
     const void *x = nullptr, *labels = nullptr, *xs = nullptr, *xs_prev = nullptr;
-    bool backward = false, resident = false, emb_sparse_valid = false, emb_cleared = false, upk_valid = false, wfct_valid = false;
+    bool backward = false, resident = false, emb_sparse_valid = false, emb_cleared = false, upk_valid = false, utp_valid = false, wfct_valid = false;
     int emb_dirty_n = 0, pairing = 0;
     size_t e_ones_rows = 0;
     uint64_t alloc_epoch = 0, state_epoch = 0;
     bool operator==(const StepSig &o) const {
       return x == o.x && labels == o.labels && xs == o.xs && xs_prev == o.xs_prev && backward == o.backward && resident == o.resident &&
-             emb_sparse_valid == o.emb_sparse_valid && emb_cleared == o.emb_cleared && upk_valid == o.upk_valid &&
+             emb_sparse_valid == o.emb_sparse_valid && emb_cleared == o.emb_cleared && upk_valid == o.upk_valid && utp_valid == o.utp_valid &&
              wfct_valid == o.wfct_valid && emb_dirty_n == o.emb_dirty_n && pairing == o.pairing && e_ones_rows == o.e_ones_rows &&
              alloc_epoch == o.alloc_epoch && state_epoch == o.state_epoch;
     }
@@ -310,7 +310,7 @@ class Engine {
   };
   struct StepState {
     bool did_backward = false, out_folded = false, emb_sparse_valid = false, emb_cleared = false, upk_valid = false,
-         wfct_valid = false, tail_pending = false;
+         utp_valid = false, wfct_valid = false, tail_pending = false;
     float *fwd_out = nullptr;
     const float *d_dgo = nullptr;
     const void *xs = nullptr;
