@@ -1094,12 +1094,13 @@ std::string write_rounds(const Chain &b) {
     for (int i = 0; i < L; i++)
       o << "  f4 w" << i << "[Cell" << i << "::NBK][GPW];\n  rounds_weights<Cell" << i << "::NBK>(A.a[" << i << "], " << back << ", wk.ct, w" << i << ");\n";
     o << "  if ((threadIdx.x >> 6) < 4) __builtin_amdgcn_s_setprio(2);\n  __syncthreads();\n  for (int r = 0; r < wk.nlists; r++) {\n"
-         "    const i4 *rt = s_rec[r & 1];\n    const int n = wk.cur[1] < ROWS ? wk.cur[1] : ROWS;\n    wk.fetch_next(r);\n"
+         "    const i4 *rt = s_rec[r & 1];\n    const int n = wk.cur[1] < ROWS ? wk.cur[1] : ROWS;\n    wk.ask();\n    wk.fetch_next(r);\n"
       << (back ? "    const bool alone = wk.cur[3] & 2;\n" : "");
     // (a list whose plan says it waits for nothing reads nothing an earlier list of this launch wrote that the one before it did not wait for)
     for (int s = 0; s < L; s++) {
       const int i = back ? L - 1 - s : s, f = (i + L - 1) % L;
       const std::string target = s == 0 ? "wk.cur[2] > 0 ? wk.arrived : 0u" : "wk.arrived";  // (every workgroup of the group has arrived as often)
+      if (s > 0) o << "    wk.ask();\n";
       o << "    if (" << (back && i > 0 ? "!alone && " : "") << "!" << (back ? "rounds_backward<Cell" : "rounds_forward<Cell") << i << ", "
         << (back ? "Cell" + std::to_string(f) + ", " + (i == 0 ? "true" : "false") : std::string(i == 0 ? "true" : "false") + ", " + (i == L - 1 ? "true" : "false"))
         << ">(A.a[" << i << "], w" << i << ", wk, rt, n, " << target << ", " << (s == L - 1 ? "true" : "false") << (back ? i == 0 ? ", alone" : ", false" : "")
