@@ -401,22 +401,25 @@ __global__ __launch_bounds__(256) void spread_rows_kernel(float4 *__restrict__ d
 // part that began in an earlier piece, row 2c + 1 the one that goes on in the next (a segment that
 // does both: row 2c).
 // Pieces of 16 rows (one batch of loads) while they are few, else of 64 (2368 x 2048: 13.3 us in pieces of 64).
+// TOTALS: the sum of all of a piece's rows to row c of `totals` as well: what is left to read for the sum of all rows is a
+// sixteenth or less of them (73000 rows of 4096: 321 -> 323 us here, the bias's own pass over them 239 -> 15).
 constexpr int kSumFew = 8192;
 static int sum_rows(int n) { return n <= kSumFew ? 16 : 64; }
-template <int kSumRows>
+template <int kSumRows, bool TOTALS>
 __global__ __launch_bounds__(256) void gather_sums_kernel(float *__restrict__ dst, long ld_dst, const float *__restrict__ src, long ld_src,
                                                           const int *__restrict__ order, const int *__restrict__ at, int n, int w,
-                                                          float *__restrict__ part) {
+                                                          float *__restrict__ part, float *__restrict__ totals) {
   const int lane = threadIdx.x & 63, c = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int p0 = c * kSumRows, count = min(kSumRows, n - p0), col = blockIdx.y * 256 + 4 * lane;
   if (count <= 0) return;
   const int row = lane < count ? order[p0 + lane] : 0, slot = lane < count ? at[p0 + lane] : -1;
   const int before = p0 > 0 ? at[p0 - 1] : -1, after = p0 + count < n ? at[p0 + count] : -1;
   const bool in = col < w;
-  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f), all = acc;
   int cur = __builtin_amdgcn_readlane(slot, 0);
   auto put = [&](float *to) {
     if (in) *reinterpret_cast<float4 *>(to + col) = acc;
+    if (TOTALS) all.x += acc.x, all.y += acc.y, all.z += acc.z, all.w += acc.w;
     acc = make_float4(0.f, 0.f, 0.f, 0.f);
   };
   constexpr int U = 16;
@@ -441,6 +444,7 @@ __global__ __launch_bounds__(256) void gather_sums_kernel(float *__restrict__ ds
   if (cur == before) put(part + (long)2 * c * w);
   else if (cur == after) put(part + (long)(2 * c + 1) * w);
   else put(dst + cur * ld_dst);
+  if (TOTALS && in) *reinterpret_cast<float4 *>(totals + (long)c * w + col) = all;
 }
 
 // The segments that cross borders: the workgroup of the piece where one begins adds up its parts, a
@@ -573,17 +577,25 @@ size_t cavs_gather_sums_workspace(int n, int w) {
 
 int cavs_gather_sums(float *dst, int ld_dst, const float *src, int ld_src, const int *index, int n, int w, void *workspace,
                      size_t workspace_bytes, void *stream) {
+  return cavs_gather_sums_totals(dst, ld_dst, src, ld_src, index, n, w, nullptr, workspace, workspace_bytes, stream);
+}
+
+int cavs_gather_sums_pieces(int n) { return n > 0 ? (n + sum_rows(n) - 1) / sum_rows(n) : 0; }
+
+int cavs_gather_sums_totals(float *dst, int ld_dst, const float *src, int ld_src, const int *index, int n, int w, float *totals, void *workspace,
+                            size_t workspace_bytes, void *stream) {
   CAVS_REQUIRE(n >= 0 && w >= 0 && w % 4 == 0 && ld_dst >= w && ld_src >= w && ld_dst % 4 == 0 && ld_src % 4 == 0,
                "cavs_gather_sums: bad shape n=%d w=%d ld=%d,%d", n, w, ld_dst, ld_src);
   if (n == 0 || w == 0) return CAVS_OK;
-  CAVS_REQUIRE(dst && src && index && aligned16(dst) && aligned16(src), "cavs_gather_sums: null or misaligned pointer");
+  CAVS_REQUIRE(dst && src && index && aligned16(dst) && aligned16(src) && (!totals || aligned16(totals)), "cavs_gather_sums: null or misaligned pointer");
   const size_t need = cavs_gather_sums_workspace(n, w);
   CAVS_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace), "cavs_gather_sums: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
   const int per = sum_rows(n), pieces = (n + per - 1) / per, cols = (w + 255) / 256;
   const int *order = index + 4 + n, *at = order + n;
   float *part = static_cast<float *>(workspace);
   hipStream_t st = as_stream(stream);
-  launch(per == 16 ? gather_sums_kernel<16> : gather_sums_kernel<64>, dim3((pieces + 3) / 4, cols), 256, 0, st, dst, ld_dst, src, ld_src, order, at, n, w, part);
+  launch(per == 16 ? totals ? gather_sums_kernel<16, true> : gather_sums_kernel<16, false> : totals ? gather_sums_kernel<64, true> : gather_sums_kernel<64, false>,
+         dim3((pieces + 3) / 4, cols), 256, 0, st, dst, ld_dst, src, ld_src, order, at, n, w, part, totals);
   CAVS_LAUNCH_CHECK();
   if (pieces > 1) {
     launch(per == 16 ? gather_sums_across_kernel<16> : gather_sums_across_kernel<64>, dim3(pieces - 1, cols), 256, 0, st, dst, ld_dst, at, n, w, part);

@@ -183,12 +183,85 @@ __global__ __launch_bounds__(256) void softmax_xent_rows_kernel(float *__restric
     const int j = tid + 256 * k;
     if (j >= C4) continue;
     float4 p = make_float4(v[k].x / sum, v[k].y / sum, v[k].z / sum, v[k].w / sum);
-    if (lab >> 2 == j) {
+    if (lab >> 2 == j) {  // (one by one: a reference to one of them would put them all into memory)
       const int c = lab & 3;
-      (c == 0 ? p.x : c == 1 ? p.y : c == 2 ? p.z : p.w) -= 1.f;
+      p.x -= c == 0 ? 1.f : 0.f, p.y -= c == 1 ? 1.f : 0.f, p.z -= c == 2 ? 1.f : 0.f, p.w -= c == 3 ? 1.f : 0.f;
     }
     d[j] = make_float4(p.x * inv_n, p.y * inv_n, p.z * inv_n, p.w * inv_n);
   }
+}
+
+// The same with the sums of d logits' columns, which are the gradient of the head's bias: a workgroup takes every gridDim.x-th row,
+// keeps the sums over its rows in registers and leaves them as a row of `sums`, a pass over a few hundred rows instead of one over all
+// of d logits.  Two workgroups of 512 to a CU; a row is on its way while the one before is worked on.  Bound as much by the exponentials
+// as by memory.  MEASURED
+constexpr int kSumsThreads = 512;
+template <int NV>
+__global__ __launch_bounds__(kSumsThreads) void softmax_xent_sums_kernel(float *__restrict__ loss, float *__restrict__ dlogits,
+                                                                         const float *__restrict__ logits, const float *__restrict__ labels, int n,
+                                                                         int C, float inv_n, float *__restrict__ sums) {
+  constexpr int WAVES = kSumsThreads / 64;
+  __shared__ float part[2][2][WAVES];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, C4 = C / 4;
+  float4 v[NV], next[NV], acc[NV];
+  auto fetch = [&](int row, float4 (&o)[NV]) {
+    const float4 *x = reinterpret_cast<const float4 *>(logits + (long)row * C);
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+      const int j = tid + kSumsThreads * k;
+      o[k] = j < C4 ? x[j] : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < NV; k++) acc[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+  fetch(blockIdx.x, v);
+  int turn = 0;
+  for (int row = blockIdx.x; row < n; row += gridDim.x, turn ^= 1) {
+    const int lab = (int)labels[row];
+    if (row + (int)gridDim.x < n) fetch(row + gridDim.x, next);
+    float mx = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < NV; k++) mx = fmaxf(fmaxf(mx, fmaxf(v[k].x, v[k].y)), fmaxf(v[k].z, v[k].w));
+    mx = wave_max(mx);
+    if (lane == 0) part[turn][0][wave] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < WAVES; q++) mx = fmaxf(mx, part[turn][0][q]);
+    float sum = 0.f;
+#pragma unroll
+    for (int k = 0; k < NV; k++) {  // exp(-inf) = 0 past the end of the row
+      v[k].x = expf(v[k].x - mx); v[k].y = expf(v[k].y - mx); v[k].z = expf(v[k].z - mx); v[k].w = expf(v[k].w - mx);
+      sum += (v[k].x + v[k].y) + (v[k].z + v[k].w);
+    }
+    sum = wave_sum(sum);
+    if (lane == 0) part[turn][1][wave] = sum;
+    __syncthreads();
+    sum = 0.f;
+#pragma unroll
+    for (int q = 0; q < WAVES; q += 2) sum += part[turn][1][q] + part[turn][1][q + 1];
+    if (tid == 0 && (unsigned)lab >= (unsigned)C) loss[row] = -logf(expf(logits[(long)row * C + lab] - mx) / sum);  // (no class: as ever)
+    float4 *d = reinterpret_cast<float4 *>(dlogits + (long)row * C);
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+      const int j = tid + kSumsThreads * k;
+      if (j < C4) {
+        float4 p = make_float4(v[k].x / sum, v[k].y / sum, v[k].z / sum, v[k].w / sum);
+        if (lab >> 2 == j) {
+          const int c = lab & 3;
+          loss[row] = -logf(c == 0 ? p.x : c == 1 ? p.y : c == 2 ? p.z : p.w);
+          p.x -= c == 0 ? 1.f : 0.f, p.y -= c == 1 ? 1.f : 0.f, p.z -= c == 2 ? 1.f : 0.f, p.w -= c == 3 ? 1.f : 0.f;
+        }
+        p = make_float4(p.x * inv_n, p.y * inv_n, p.z * inv_n, p.w * inv_n);
+        acc[k].x += p.x, acc[k].y += p.y, acc[k].z += p.z, acc[k].w += p.w;
+        d[j] = p;
+      }
+      v[k] = next[k];
+    }
+  }
+  float4 *s = reinterpret_cast<float4 *>(sums + (long)blockIdx.x * C);
+#pragma unroll
+  for (int k = 0; k < NV; k++)
+    if (tid + kSumsThreads * k < C4) s[tid + kSumsThreads * k] = acc[k];
 }
 
 // ------------------------------------------------------------------ elementwise
@@ -336,6 +409,21 @@ int cavs_bias_add_rows(float *out, const float *inp, const float *bias, int n, i
 int cavs_softmax_xent(float *loss, float *dlogits, const float *logits, const float *labels, int n,
                       int C, void *stream) {
   return cavs_softmax_xent_part(loss, dlogits, logits, labels, n, C, n, stream);
+}
+
+// (rows enough that the sums are few beside them)
+int cavs_softmax_xent_sum_rows(int n, int C) { return n >= 4096 && C >= 512 && C % 4 == 0 && C <= 16384 ? 512 : 0; }
+
+int cavs_softmax_xent_sums(float *loss, float *dlogits, const float *logits, const float *labels, float *sums, int n, int C, void *stream) {
+  const int rows = cavs_softmax_xent_sum_rows(n, C);
+  CAVS_REQUIRE(rows > 0, "cavs_softmax_xent_sums: unsupported shape n=%d C=%d (cavs_softmax_xent_sum_rows)", n, C);
+  CAVS_REQUIRE(loss && dlogits && logits && labels && sums, "cavs_softmax_xent_sums: null pointer");
+  CAVS_REQUIRE(aligned16(dlogits) && aligned16(logits) && aligned16(sums), "cavs_softmax_xent_sums: d logits, logits and sums must be 16-byte aligned");
+  const float inv_n = 1.f / (float)n;
+  launch(C <= 2048 ? softmax_xent_sums_kernel<1> : C <= 4096 ? softmax_xent_sums_kernel<2> : C <= 10240 ? softmax_xent_sums_kernel<5> : softmax_xent_sums_kernel<8>,
+         rows, kSumsThreads, 0, as_stream(stream), loss, dlogits, logits, labels, n, C, inv_n, sums);
+  CAVS_LAUNCH_CHECK();
+  return CAVS_OK;
 }
 
 int cavs_softmax_xent_part(float *loss, float *dlogits, const float *logits, const float *labels, int n,

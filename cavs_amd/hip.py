@@ -118,10 +118,12 @@ _SIGS = {
     "cavs_embed_words_bwd": [_P, _P, _P, _I, _I, _I, _P],
     "cavs_spread_rows": [_P, _I, _P, _I, _P, _I, _I, _I, _I, _P, _P, _P],
     "cavs_gather_sums": [_P, _I, _P, _I, _P, _I, _I, _P, _Z, _P],
+    "cavs_gather_sums_totals": [_P, _I, _P, _I, _P, _I, _I, _P, _P, _Z, _P],
     "cavs_embed_bwd": [_P, _P, _P, _I, _I, _I, _P],
     "cavs_bias_add_rows": [_P, _P, _P, _I, _I, _P],
     "cavs_softmax_xent": [_P, _P, _P, _P, _I, _I, _P],
     "cavs_softmax_xent_part": [_P, _P, _P, _P, _I, _I, _I, _P],
+    "cavs_softmax_xent_sums": [_P, _P, _P, _P, _P, _I, _I, _P],
     "cavs_sgd": [_P, _P, _F, _Z, _P],
     "cavs_ew_binary": [_I, _P, _P, _Z, _P, _Z, _Z, _I, _P],
     "cavs_ew_unary": [_I, _P, _P, _Z, _I, _P],
@@ -193,7 +195,7 @@ _BENCH_SIGS = {"cavs_mfma_probe": [_P, _Z, _I, C.POINTER(C.c_double), _P]}
 _RESTYPE = {"cavs_last_error": C.c_char_p, "cavs_abi_version": _I, "cavs_sgemm_splitk_workspace": _Z,
             "cavs_fc_softmax_xent_workspace": _Z, "cavs_colsum_blocks_workspace": _Z,
             "cavs_clip_grads_workspace": _Z, "cavs_sgemm_group_workspace": _Z, "cavs_fc_softmax_xent_parts": _I,
-            "cavs_colsum_parts": _I, "cavs_round_packed_ok": _I, "cavs_lstm_round_packed_ok": _I,
+            "cavs_colsum_parts": _I, "cavs_gather_sums_pieces": _I, "cavs_softmax_xent_sum_rows": _I, "cavs_round_packed_ok": _I, "cavs_lstm_round_packed_ok": _I,
             "cavs_group_rounds_ok": _I, "cavs_group_max_groups": _I, "cavs_group_rows": _I, "cavs_tail_rounds_ok": _I, "cavs_tail_max_rounds": _I, "cavs_tail_max_groups": _I, "cavs_tail_sync_bytes": _Z,
             "cavs_sgemm_splitk_static_max_bytes": _Z,
             "cavs_embed_index_ints": _Z, "cavs_embed_index_workspace": _Z, "cavs_gather_sums_workspace": _Z,
@@ -201,7 +203,7 @@ _RESTYPE = {"cavs_last_error": C.c_char_p, "cavs_abi_version": _I, "cavs_sgemm_s
 _NOCHECK = {"cavs_last_error": [], "cavs_abi_version": [], "cavs_sgemm_splitk_workspace": [_I, _I, _I],
             "cavs_fc_softmax_xent_workspace": [_I, _I, _I], "cavs_colsum_blocks_workspace": [_I, _I, _I],
             "cavs_clip_grads_workspace": [_I], "cavs_sgemm_group_workspace": [_I, C.POINTER(GemmDesc)],
-            "cavs_fc_softmax_xent_parts": [_I], "cavs_colsum_parts": [_I], "cavs_round_packed_ok": [_I, _I],
+            "cavs_fc_softmax_xent_parts": [_I], "cavs_colsum_parts": [_I], "cavs_gather_sums_pieces": [_I], "cavs_softmax_xent_sum_rows": [_I, _I], "cavs_round_packed_ok": [_I, _I],
             "cavs_lstm_round_packed_ok": [_I, _I], "cavs_sgemm_splitk_static_max_bytes": [],
             "cavs_group_rounds_ok": [_I], "cavs_group_max_groups": [_I], "cavs_group_rows": [], "cavs_tail_rounds_ok": [_I, _I], "cavs_tail_max_rounds": [], "cavs_tail_max_groups": [], "cavs_tail_sync_bytes": [],
             "cavs_embed_index_ints": [_I], "cavs_embed_index_workspace": [_I], "cavs_gather_sums_workspace": [_I, _I],

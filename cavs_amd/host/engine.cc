@@ -683,6 +683,7 @@ void Engine::reserve_edges() {
     R(xW_words_, cap * w);
     if (!cell_) R(d_words_, cap * w);
     R(word_parts_, cavs_gather_sums_workspace((int)cap, (int)most) / 4);
+    if (!cell_) R(word_totals_, cavs_gather_sums_workspace((int)cap, 4 * (int)H) / 8);
     const size_t ints = cavs_embed_index_ints((int)cap);
     if (word_index_.capacity() < ints) {
       check(cavs_stream_sync(stream_));
@@ -771,10 +772,10 @@ void Engine::words_forward(const float *W, int w, int leaf_w) {
   c_launches_ += 3;
 }
 
-// dst [L, w] = the rows of src [N, w] added up by word
-void Engine::words_sum(float *dst, const float *src, int ld_src, int w) {
+// dst [L, w] = the rows of src [N, w] added up by word; totals: rows that add up to the sum of all of src's, or null
+void Engine::words_sum(float *dst, const float *src, int ld_src, int w, float *totals) {
   ProfScope ps(this, K_OTHER);
-  check(cavs_gather_sums(dst, w, src, ld_src, d_words_index_, N_, w, word_parts_.get(), word_parts_.capacity() * 4, stream_));
+  check(cavs_gather_sums_totals(dst, w, src, ld_src, d_words_index_, N_, w, totals, word_parts_.get(), word_parts_.capacity() * 4, stream_));
   c_launches_ += 2;
 }
 
@@ -1870,7 +1871,7 @@ void Engine::treelstm_backward() {
   const float *dx = dxW_.get();  // the gradients of x * W, by vertex or by word
   const int *live = nullptr;
   if (words_) {
-    words_sum(d_words_.get(), dxW_.get(), 4 * H, 4 * H);
+    words_sum(d_words_.get(), dxW_.get(), 4 * H, 4 * H, bias_row ? nullptr : word_totals_.get());
     dx = d_words_.get();
     live = d_words_index_;
   }
@@ -1892,9 +1893,10 @@ void Engine::treelstm_backward() {
     return;
   }
   const int dst_block[4] = {0, 3, 2, 1};  // dxW block k ([i|o|u|f]) lands in bias block dst_block[k]
-  const size_t cs_bytes = cavs_colsum_blocks_workspace(N, H, 4);
+  const int rows = words_ ? cavs_gather_sums_pieces(N) : N;
+  const size_t cs_bytes = cavs_colsum_blocks_workspace(rows, H, 4);
   float *cs_ws = workspace(cs_bytes);
-  check(cavs_colsum_blocks(param("Bv").g, dxW_.get(), 4 * H, N, H, 4, dst_block, cs_ws, cs_bytes, stream_));
+  check(cavs_colsum_blocks(param("Bv").g, words_ ? word_totals_.get() : dxW_.get(), 4 * H, rows, H, 4, dst_block, cs_ws, cs_bytes, stream_));
   c_launches_ += 2;
 }
 
@@ -2216,11 +2218,12 @@ void Engine::lstm_backward() {
   const float *dx = dxW_.get();  // the gradients of x * W, by vertex or by word
   const int *live = nullptr;
   if (words_) {
-    words_sum(d_words_.get(), dxW_.get(), 4 * H, 4 * H);
+    words_sum(d_words_.get(), dxW_.get(), 4 * H, 4 * H, word_totals_.get());
     dx = d_words_.get();
     live = d_words_index_;
   }
-  const cavs_colsum_desc sums = bias_sums("Bv", dxW_.get(), N, 4 * H, bias_parts_);
+  const cavs_colsum_desc sums = words_ ? bias_sums("Bv", word_totals_.get(), cavs_gather_sums_pieces(N), 4 * H, bias_parts_)
+                                       : bias_sums("Bv", dxW_.get(), N, 4 * H, bias_parts_);
   last_launch(3, true, [&] { gemm_group_embedding_backward({
       {0, 1, N, E, 4 * H, 1.f, 0.f, dx, 4 * H, Wx, 4 * H, de_.get(), E, 0, 0, 0, live, words_expected()},
       {1, 0, E, 4 * H, N, 1.f, 0.f, e_.get(), E, dx, 4 * H, dW, 4 * H, 0, 0, 0, live, words_expected()},
@@ -2754,7 +2757,16 @@ void Engine::head_forward_backward(bool backward) {
       c_gemm_flops_ += 2.0 * N * C * H;
       c_launches_ += 1;
     }
-    check(cavs_softmax_xent(loss_.get(), backward ? dlogits_.get() : nullptr, logits_.get(), d_labels_, N, C, stream_));
+    // with its columns' sums, where the loss's launch can leave them behind: else the bias gradient reads all of d logits again
+    const int sum_rows = backward ? cavs_softmax_xent_sum_rows(N, C) : 0;
+    if (sum_rows > 0) {
+      ensure(head_sums_, (size_t)sum_rows * C);
+      check(cavs_softmax_xent_sums(loss_.get(), dlogits_.get(), logits_.get(), d_labels_, head_sums_.get(), N, C, stream_));
+    } else {
+      check(cavs_softmax_xent(loss_.get(), backward ? dlogits_.get() : nullptr, logits_.get(), d_labels_, N, C, stream_));
+    }
+    const float *biased = sum_rows > 0 ? head_sums_.get() : dlogits_.get();
+    const int biased_rows = sum_rows > 0 ? sum_rows : N;
     c_launches_ += 1;
     if (backward) {
       const cavs_gemm_desc dWd{1, 0, C, H, N, 1.f, 0.f, dlogits_.get(), C, GO_.get(), H, Wfc.g, H};
@@ -2780,12 +2792,12 @@ void Engine::head_forward_backward(bool backward) {
         check((group_.first >= 0 ? cavs_sgemm_group : cavs_sgemm_group_beside)(1, &dWd, ws_aux_.get(), ws_aux_.capacity() * 4, aux_stream_));
         c_gemm_flops_ += 2.0 * dWd.M * dWd.N * dWd.K;
         c_launches_ += 1;
-        bias_gradient("bfc", dlogits_.get(), N, C, head_bias_parts_, aux_stream_);
+        bias_gradient("bfc", biased, biased_rows, C, head_bias_parts_, aux_stream_);
         check(cavs_event_record(aux_join_ev_, aux_stream_));
         aux_pending_ = true;
       } else {
         // both read d logits and write different outputs: one launch when they are small
-        const cavs_colsum_desc sums = bias_sums("bfc", dlogits_.get(), N, C, head_bias_parts_);
+        const cavs_colsum_desc sums = bias_sums("bfc", biased, biased_rows, C, head_bias_parts_);
         last_launch(2, true, [&] { gemm_group({dWd, dGd}, &sums); });
       }
     }

@@ -416,13 +416,13 @@ class Engine {
   void clear_embedding(std::vector<cavs_task> *tasks);
   bool leaves_with_company(cavs_task leaves);
   const int *d_words_index_ = nullptr;
-  DeviceArray<float> xW_words_, d_words_, word_parts_;
+  DeviceArray<float> xW_words_, d_words_, word_parts_, word_totals_;
   int pad_block() const { return uH_ != cfg_.H ? cfg_.H : 0; }  // padding of x * W (cavs_gemm_desc::pad_block, uH_ used)
   bool words_wanted() const;
   int words_expected() const;
   void words_index(int leaf_rows);
   void words_forward(const float *W, int w, int leaf_w);
-  void words_sum(float *dst, const float *src, int ld_src, int w);
+  void words_sum(float *dst, const float *src, int ld_src, int w, float *totals = nullptr);
   size_t e_ones_rows_ = 0;       // rows of e_ whose ones column is initialised
   DeviceArray<float> ones_col_;  // [ld_e_]: 1 at column E
   bool bias_row_ok() const;
@@ -430,7 +430,7 @@ class Engine {
   // chunk sums of a column sum): delivered, and the parameter updated, by one job each of the
   // launch that ends the step.
   std::vector<BiasJob> bias_jobs_;
-  DeviceArray<float> bias_parts_, head_bias_parts_;
+  DeviceArray<float> bias_parts_, head_bias_parts_, head_sums_;
   // column sums of inp [n, w] as the gradient of `name`, in a fixed order
   cavs_colsum_desc bias_sums(const std::string &name, const float *inp, int n, int w, DeviceArray<float> &parts);
   void bias_gradient(const std::string &name, const float *inp, int n, int w, DeviceArray<float> &parts, void *stream);

@@ -309,6 +309,8 @@ int cavs_embed_pull_sgemm_padded(float *C, int ldc, float *e_out, int ld_e, floa
  * cavs_spread_rows: dst[b, 0:w] = src[word of b, 0:w]; rows below head_rows only columns below head_w; and
  *   ids_out[b] = ids[b] unless they are null.
  * cavs_gather_sums: dst[s, 0:w] = the sum of src[b, 0:w] over the rows b of word s, in a fixed order.
+ * cavs_gather_sums_totals: the same, and totals[p, 0:w], p < cavs_gather_sums_pieces(n) (null: none): rows that add up to
+ *   the sum of src[b, 0:w] over all b.
  * Widths and strides are multiples of 4, pointers 16-byte aligned. */
 size_t cavs_embed_index_ints(int n);
 size_t cavs_embed_index_workspace(int n);
@@ -321,6 +323,9 @@ int cavs_spread_rows(float *dst, int ld_dst, const float *src, int ld_src, const
 size_t cavs_gather_sums_workspace(int n, int w);
 int cavs_gather_sums(float *dst, int ld_dst, const float *src, int ld_src, const int *index, int n, int w, void *workspace,
                      size_t workspace_bytes, void *stream);
+int cavs_gather_sums_pieces(int n);
+int cavs_gather_sums_totals(float *dst, int ld_dst, const float *src, int ld_src, const int *index, int n, int w, float *totals,
+                            void *workspace, size_t workspace_bytes, void *stream);
 /* out[r, :] = inp[r, :] + bias[:]  (BinaryBroadcastingKernel,
  * cavs/backend/op_impl_elementwise.cuh:128-139; also the ones-vector bias GEMM of
  * cavs/backend/op_impl_fullyconnected_cublas.cc:74-76) */
@@ -337,6 +342,11 @@ int cavs_softmax_xent(float *loss, float *dlogits, const float *logits, const fl
  * values of the call over the whole batch. */
 int cavs_softmax_xent_part(float *loss, float *dlogits, const float *logits, const float *labels,
                            int n, int C, int n_total, void *stream);
+/* The whole batch, and sums [cavs_softmax_xent_sum_rows(n, C), C]: rows that add up to the sum of d logits' rows
+ * (no rows: not for this shape).  All pointers 16-byte aligned. */
+int cavs_softmax_xent_sum_rows(int n, int C);
+int cavs_softmax_xent_sums(float *loss, float *dlogits, const float *logits, const float *labels, float *sums, int n, int C,
+                           void *stream);
 /* SGD (cavs/backend/op_impl_sgd.cu): w -= lr * g */
 int cavs_sgd(float *w, const float *g, float lr, size_t n, void *stream);
 

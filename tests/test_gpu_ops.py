@@ -2102,3 +2102,51 @@ def test_products_over_the_words_alone(g, M, N, K, L, Z):
             close(got[:L], wantC, "rows of the words")
             np.testing.assert_array_equal(got[L:], 5.0)
             close(g.host(Gd), wantG, "sum over the words")
+
+
+@pytest.mark.parametrize("n,C_", [(4096, 512), (4097, 2052), (4609, 4100), (5000, 10004), (4096, 16384)])
+def test_softmax_leaves_its_columns_sums(g, n, C_):
+    """The loss's launch with the sums of d logits' columns (a workgroup has the rows it takes in turn: one more or less than the others,
+    and classes that fill no whole vector): the two launches' losses and gradients, and rows that add up to the sum in 64 bits."""
+    r = rng(n + C_)
+    logits = r.bulk_uniform(n * C_, -4, 4)
+    labels = np.floor(r.bulk_uniform(n) * C_).astype(np.float32)
+    labels[:2] = (0, C_ - 1)
+    x, lab = g.devf(logits), g.devf(labels)
+    rows = hip.lib().cavs_softmax_xent_sum_rows(n, C_)
+    loss, d, loss2, d2, sums = g.zeros(n), g.zeros(n, C_), g.zeros(n), g.zeros(n, C_), g.zeros(rows, C_)
+    g.call("cavs_softmax_xent", g.P(loss), g.P(d), g.P(x), g.P(lab), n, C_, g.stream())
+    g.call("cavs_softmax_xent_sums", g.P(loss2), g.P(d2), g.P(x), g.P(lab), g.P(sums), n, C_, g.stream())
+    want, got = g.host(d).reshape(n, C_), g.host(d2).reshape(n, C_)
+    # (the row's sum is added up in another order: some units in the last place)
+    np.testing.assert_allclose(g.host(loss2), g.host(loss), rtol=3e-6, atol=3e-6)
+    np.testing.assert_allclose(got, want, rtol=3e-6, atol=2e-7 / n)
+    total = got.astype(np.float64).sum(0)
+    # a column: n / rows additions of values up to 1 / n in a row, each half a unit of the sum so far off
+    np.testing.assert_allclose(g.host(sums).reshape(rows, C_).astype(np.float64).sum(0), total, rtol=2e-6, atol=1e-7 * np.abs(got).sum(0).max())
+    assert hip.lib().cavs_softmax_xent_sum_rows(4095, C_) == 0 and hip.lib().cavs_softmax_xent_sum_rows(n, 508) == 0
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 1000, 8192, 8193, 9000])
+def test_sums_by_word_leave_the_sum_of_all(g, n):
+    """Pieces of 16 and of 64 rows, the last one short: rows that add up to the sum of all rows, beside the words' own sums."""
+    w, V = 36, 50
+    r = rng(n)
+    src = r.bulk_normal(n * w)
+    ids = np.floor(r.bulk_uniform(n) * V).astype(np.float32)
+    L = hip.lib()
+    index = g.devi(np.zeros(L.cavs_embed_index_ints(n)))
+    ws, wb = g.zeros(L.cavs_embed_index_workspace(n) // 4 + 4), L.cavs_embed_index_workspace(n)
+    g.call("cavs_embed_index", g.P(index), g.P(g.zeros(n)), g.P(g.devf(ids)), g.P(g.devi(np.arange(n))), n, V, 0, g.P(ws), wb, g.stream())
+    room = L.cavs_gather_sums_workspace(n, w)
+    part, dst, dst2 = g.zeros(room // 4 + 4), g.zeros(n, w), g.zeros(n, w)
+    pieces = L.cavs_gather_sums_pieces(n)
+    totals = g.zeros(pieces, w)
+    x = g.devf(src)
+    g.call("cavs_gather_sums", g.P(dst), w, g.P(x), w, g.P(index), n, w, g.P(part), room, g.stream())
+    g.call("cavs_gather_sums_totals", g.P(dst2), w, g.P(x), w, g.P(index), n, w, g.P(totals), g.P(part), room, g.stream())
+    np.testing.assert_array_equal(g.host(dst2), g.host(dst))
+    want = src.reshape(n, w).astype(np.float64)
+    # up to 64 additions in a row: 64 half units of a partial sum of at most the magnitudes' sum
+    np.testing.assert_allclose(g.host(totals).reshape(pieces, w).astype(np.float64).sum(0), want.sum(0), rtol=0,
+                               atol=64 * 2.0 ** -24 * np.abs(want).sum(0).max())
