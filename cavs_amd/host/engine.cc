@@ -1709,7 +1709,10 @@ void Engine::treelstm_forward() {
 void Engine::treelstm_backward() {
   const int N = N_, H = cfg_.H, E = E_;
   const float *W = param("W").w, *U = param("U").w;
-  const int fused = fused_rows();
+  int fused = fused_rows();
+  // Where rounds are separate launches anyway, the crossover of a backward round lies lower from H = 1024 on: 912 rows 210 us as one
+  // launch of its children's products, 150 as products (256 trees of 32 .. 128 leaves 8.7 -> 8.3 ms a step; H = 768: 6.02 -> 6.03).
+  if (!forest_ && H >= 1024 && fused > 512 && cfg_.fused_round_rows == 0 && !cfg_.split_backward_rounds) fused = 512;
   // grad of Push is Pull: read through the list by the gate kernels of the fused path, or gathered up front
   const bool dret_folded = fused > 0;
   if (!dret_folded && !forest_) gather(dret_.get(), H, d_dgo_, H, d_t2j_, N, H);

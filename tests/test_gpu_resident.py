@@ -198,3 +198,20 @@ def test_vertex_inputs_read_by_vertex(H, B, kw, shift):
             close(got[name], v, name)
     for z in (s, ref):
         z.close()
+
+
+def test_a_wide_cell_leaves_middling_backward_rounds_to_products():
+    """H = 1024, a batch with a round above the fused limit (1024): its backward rounds of more than 512 rows are products, what
+    one launch of each gives (other orders of the same sums)."""
+    w = small_workload("treelstm", 83, B=700, H=1024, E=12, V=31, C=5)
+    sizes = np.diff(session.schedule_trace(w["graph"])["round2offset"])[1:]
+    assert sizes.max() > 1024 and ((sizes > 512) & (sizes <= 1024)).any() and (sizes <= 512).any()
+    s, ref = _session("treelstm", 1024, w), _session("treelstm", 1024, w, fused_round_rows=1024)
+    for x in (s, ref):
+        x.step(w["graph"], w["x"], w["labels"], backward=True, lr=1e-6)
+    close(s.fetch("loss"), ref.fetch("loss"), "loss")
+    got, want = s.grads(), ref.grads()
+    for name, v in want.items():
+        close(got[name], v, name)
+    for x in (s, ref):
+        x.close()
