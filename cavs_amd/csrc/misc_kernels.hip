@@ -194,7 +194,8 @@ __global__ __launch_bounds__(256) void softmax_xent_rows_kernel(float *__restric
 // The same with the sums of d logits' columns, which are the gradient of the head's bias: a workgroup takes every gridDim.x-th row,
 // keeps the sums over its rows in registers and leaves them as a row of `sums`, a pass over a few hundred rows instead of one over all
 // of d logits.  Two workgroups of 512 to a CU; a row is on its way while the one before is worked on.  Bound as much by the exponentials
-// as by memory.  MEASURED
+// as by memory (7000 rows of 10000: 106 us without the sums, 108 with them; the pass over d logits took 105 us beside the last products,
+// that over 512 rows 22).
 constexpr int kSumsThreads = 512;
 template <int NV>
 __global__ __launch_bounds__(kSumsThreads) void softmax_xent_sums_kernel(float *__restrict__ loss, float *__restrict__ dlogits,
