@@ -2244,8 +2244,8 @@ void Engine::treefc_forward() {
   const int fused = fused_rows();
   // The leaves' launch and the group launch read x by vertex, where it has their width; else, and for rounds that are launches
   // of their own, its rows are brought into slab order first.  A leaf multiplies nothing: its round is one launch whatever its
-  // rows (above the fused limit with the tanhf of the launches that ran it there).  (64 trees of 2 .. 64 leaves, H = 256, 4200 vertices: four launches less where the leaves are more than 2048, one
-  // elsewhere, 4.6 to 5.0 us each of a step of 122)
+  // rows (above the fused limit with the tanhf of the launches that ran it there).  64 trees of 2 .. 64 leaves, H = 256: three
+  // launches less where the leaves are more than 2048, one elsewhere, 4.6 to 5.0 us each of a step of 122.
   const bool by_vertex = cfg_.use_x && uH_ == H && fused > 0;
   if (cfg_.use_x && !by_vertex) gather(xs_.get(), H, d_x_, uH_, d_t2j_, N, uH_);
   if (!sched_->batching) check(cavs_zero(G_.get(), (size_t)N * 2 * H * 4, stream_));
