@@ -3,19 +3,9 @@
 // elementwise family.  All HBM-bound streaming kernels.
 #include "common.h"
 #include "embed_common.h"
+#include "wave_reduce.h"
 
 namespace cavs {
-
-__device__ inline float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-__device__ inline float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
-}
 
 // ------------------------------------------------------------------ column sums
 // Workgroup = 4 waves over a strip of 64 columns; lane = column (256-byte coalesced

@@ -9,14 +9,9 @@
 #include "colsum_common.h"
 #include "common.h"
 #include "round_common.h"
+#include "wave_reduce.h"
 
 namespace cavs {
-
-__device__ inline float wsum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
 
 // ------------------------------------------------------------------ classifier head
 // One wavefront per row, lane l owning columns l, l+64, ... (Q of them) of x and of every row
@@ -74,7 +69,7 @@ __global__ __launch_bounds__(256) void fc_xent_kernel(const float *__restrict__ 
       float s = 0.f;
 #pragma unroll
       for (int q = 0; q < Q; q++) s += xv[q] * w[c][q];
-      z[c] = wsum(s) + bias[c];
+      z[c] = wave_sum(s) + bias[c];
       mx = fmaxf(mx, z[c]);
     }
     // cavs/backend/op_impl_softmax_entropy_logits_loss.cu:94-140, :212-250
