@@ -1070,8 +1070,10 @@ void Engine::schedule_on_device(const int *graph, int B, int maxlen) {
   if (forest_ && group_limit() > 0 && N > 0) {
     const size_t all = need;
     const int ngroups = cavs_group_max_groups(cfg_.H);
-    d.kid_host.reserve(all);
-    d.tail_host.reserve(group_lists_bound(s, B, ngroups));
+    // (twice what the first batch takes, as for the host's lists: growing pins pages anew)
+    auto room = [](size_t n, size_t had) { return had == 0 ? 2 * n : grow(n, had); };
+    d.kid_host.reserve(room(all, d.kid_host.capacity()));
+    d.tail_host.reserve(room(group_lists_bound(s, B, ngroups), d.tail_host.capacity()));
     check(cavs_memcpy_d2h(d.kid_host.get(), t2j, all * sizeof(int), sched_stream_));
     check(cavs_stream_sync(sched_stream_));
     const int *h = d.kid_host.get();
