@@ -105,7 +105,7 @@ __global__ void bias_add_rows_kernel(float *__restrict__ out, const float *__res
 
 // ------------------------------------------------------------------ softmax cross-entropy
 // One wave per row: max, sum of exp and the gradient in three passes over the row
-// (the row stays in cache); reductions are wave-level shuffles, no LDS.
+// (the row stays in cache); reductions stay within the wavefront, no LDS.
 __global__ __launch_bounds__(256) void softmax_xent_kernel(float *__restrict__ loss,
                                                            float *__restrict__ dlogits,
                                                            const float *__restrict__ logits,
@@ -130,6 +130,14 @@ __global__ __launch_bounds__(256) void softmax_xent_kernel(float *__restrict__ l
       d[j] = (j == lab ? p - 1.f : p) * inv_n;
     }
   }
+}
+
+// a / b for one b and many a, r = 1 / b as the division rounds it: the product with r is off by an ulp at most, and its remainder, exact in
+// an fma, sets it right (Markstein's theorem: the division's own bits, while a is above 2^-100).  Three operations instead of the ten of a
+// division: 7000 rows of 10000 with their sums 108.8 -> 105.9 us, 5.3 TB/s.
+__device__ inline float quotient(float a, float b, float r) {
+  const float q = a * r;
+  return fmaf(fmaf(-q, b, a), r, q);
 }
 
 // One workgroup per row, the row held in registers between the passes (NV float4 per thread,
@@ -167,12 +175,13 @@ __global__ __launch_bounds__(256) void softmax_xent_rows_kernel(float *__restric
   const int lab = (int)labels[row];
   if (loss && tid == 0) loss[row] = -logf(expf(logits[(long)row * C + lab] - mx) / sum);
   if (!dlogits) return;
+  const float r = 1.f / sum;
   float4 *d = reinterpret_cast<float4 *>(dlogits + (long)row * C);
 #pragma unroll
   for (int k = 0; k < NV; k++) {
     const int j = tid + 256 * k;
     if (j >= C4) continue;
-    float4 p = make_float4(v[k].x / sum, v[k].y / sum, v[k].z / sum, v[k].w / sum);
+    float4 p = make_float4(quotient(v[k].x, sum, r), quotient(v[k].y, sum, r), quotient(v[k].z, sum, r), quotient(v[k].w, sum, r));
     if (lab >> 2 == j) {  // (one by one: a reference to one of them would put them all into memory)
       const int c = lab & 3;
       p.x -= c == 0 ? 1.f : 0.f, p.y -= c == 1 ? 1.f : 0.f, p.z -= c == 2 ? 1.f : 0.f, p.w -= c == 3 ? 1.f : 0.f;
@@ -184,7 +193,7 @@ __global__ __launch_bounds__(256) void softmax_xent_rows_kernel(float *__restric
 // The same with the sums of d logits' columns, which are the gradient of the head's bias: a workgroup takes every gridDim.x-th row,
 // keeps the sums over its rows in registers and leaves them as a row of `sums`, a pass over a few hundred rows instead of one over all
 // of d logits.  Two workgroups of 512 to a CU; a row is on its way while the one before is worked on.  Bound as much by the exponentials
-// as by memory (7000 rows of 10000: 106 us without the sums, 108 with them; the pass over d logits took 105 us beside the last products,
+// as by memory (7000 rows of 10000: the sums add 2 us to the 106 it takes; the pass over d logits took 105 us beside the last products,
 // that over 512 rows 22).
 constexpr int kSumsThreads = 512;
 template <int NV>
@@ -231,15 +240,16 @@ __global__ __launch_bounds__(kSumsThreads) void softmax_xent_sums_kernel(float *
 #pragma unroll
     for (int q = 0; q < WAVES; q += 2) sum += part[turn][1][q] + part[turn][1][q + 1];
     if (tid == 0 && (unsigned)lab >= (unsigned)C) loss[row] = -logf(expf(logits[(long)row * C + lab] - mx) / sum);  // (no class: as ever)
+    const float r = 1.f / sum;
     float4 *d = reinterpret_cast<float4 *>(dlogits + (long)row * C);
 #pragma unroll
     for (int k = 0; k < NV; k++) {
       const int j = tid + kSumsThreads * k;
       if (j < C4) {
-        float4 p = make_float4(v[k].x / sum, v[k].y / sum, v[k].z / sum, v[k].w / sum);
+        float4 p = make_float4(quotient(v[k].x, sum, r), quotient(v[k].y, sum, r), quotient(v[k].z, sum, r), quotient(v[k].w, sum, r));
         if (lab >> 2 == j) {
           const int c = lab & 3;
-          loss[row] = -logf(c == 0 ? p.x : c == 1 ? p.y : c == 2 ? p.z : p.w);
+          loss[row] = -logf((c == 0 ? v[k].x : c == 1 ? v[k].y : c == 2 ? v[k].z : v[k].w) / sum);  // (a probability may be tiny)
           p.x -= c == 0 ? 1.f : 0.f, p.y -= c == 1 ? 1.f : 0.f, p.z -= c == 2 ? 1.f : 0.f, p.w -= c == 3 ? 1.f : 0.f;
         }
         p = make_float4(p.x * inv_n, p.y * inv_n, p.z * inv_n, p.w * inv_n);
