@@ -131,7 +131,7 @@ struct SplitLoader {
       long off = -1;
       if (gx < g.M) {
         const float id = g.pull_x[g.pull_rows[gx]];
-        off = (long)(int)(id * (float)g.K);
+        off = max((long)(int)(id * (float)g.K), -1L);  // (any row without an id: -1, so that -2 says something else)
         if (ids_out && unit[i] == 0) ids_out[gx] = id;
       }
       if (i == 0) one = __builtin_amdgcn_readfirstlane(gx < g.M ? (int)off : -2);  // (rows ascend: beyond the last, all of them are)

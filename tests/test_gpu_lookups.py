@@ -58,6 +58,24 @@ def test_rows_times_weights(g, n, first, E, N, pad):
         within(g.host(Cd), want.astype(np.float64) @ B.astype(np.float64), np.abs(want).astype(np.float64) @ np.abs(B).astype(np.float64), E, "x W")
 
 
+@pytest.mark.parametrize("E,none", [(1, -1.0), (1, -2.0), (2, -1.0), (2, -3.0), (4, -1.0), (300, -1.0)])
+def test_rows_without_an_id(g, E, none):
+    """Rows with a negative id are zero rows, also where whole wavefronts of a tile (16 rows) have none and the others have one
+    and the same word: beside the first, beside the last, all of them, and in a tile that the rows do not fill."""
+    n, N, r = 64 * 5 + 40, 128, synth.SplitMix64(E)
+    table, B = r.bulk_normal(9 * E).reshape(9, E).astype(np.float32), r.bulk_uniform(E * N, -1, 1).reshape(E, N).astype(np.float32)
+    ids = np.full(n, 7.0, np.float32)
+    for a, b in ((16, 64), (64, 80), (144, 160), (192, 256), (272, 288), (320 + 16, n)):
+        ids[a:b] = none
+    Cd, e, xs = g.zeros(n, N, fill=float("nan")), g.zeros(n, E, fill=float("nan")), g.zeros(n, fill=float("nan"))
+    g.call("cavs_embed_pull_sgemm", g.P(Cd), N, g.P(e), E, g.P(xs), g.P(g.devf(ids)), g.P(g.devi(np.arange(n))), g.P(g.devf(table)), n, E,
+           g.P(g.devf(B)), N, N, 0, 0, g.stream())
+    want = np.where(ids[:, None] < 0, np.float32(0), table[7])
+    np.testing.assert_array_equal(g.host(e), want)
+    np.testing.assert_array_equal(g.host(xs), ids)
+    within(g.host(Cd), want.astype(np.float64) @ B.astype(np.float64), np.abs(want).astype(np.float64) @ np.abs(B).astype(np.float64), E, "x W")
+
+
 def test_an_infinite_row_times_weights(g):
     """An infinity in the row that many vertices share: infinities and NaN as the sum of products has them, padding zero."""
     n, E, N, r = 300, 20, 128, synth.SplitMix64(5)
