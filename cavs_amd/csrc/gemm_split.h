@@ -286,6 +286,8 @@ __device__ inline void unsplit_tile(const GemmArgs &g, int row, int col, int kbe
 //   x * W      one row times its columns of B, written to every row                    (same_rows_product)
 //   A^T * B    the sum of B's rows over its part of K, then one step of K = 1 as MFMA  (in split_tile)
 //   A * B^T    for the table: the sum of A's rows times its columns of B               (summed_rows_product)
+// Sums that leave a float's range are not used: A^T * B makes NaN of them, which unsplit_tile computes again row by row, A * B^T takes
+// the general way.
 // What bounds such a tile are trips to memory, so its loads are all in flight at once.  64 trees, H = 512 (1217 leaves, 1153 inner
 // vertices), us a launch: x * W 30.4 -> 20.5, the deferred products 75 -> 64; 256 trees x * W 73.5 -> 47; Tree-LSTM steps of 64
 // trees 10250 -> 9550 (32 of them, with the resident rounds' change before).
@@ -412,9 +414,10 @@ __device__ inline void sixteen_rows(const float *p, int ld, int last, int at, fl
 }
 
 // Rows m0 .. m0 + 64 of A (M x K) summed, times rows n0 .. n0 + 64 of B (N x K), over [kbeg, kend): the first row of the tile of C, and
-// zeros in the others.  kbeg, kend, lda, ldb are multiples of 4, A and B 16-byte aligned.
+// zeros in the others.  kbeg, kend, lda, ldb are multiples of 4, A and B 16-byte aligned.  False, with nothing stored, where a result is not
+// finite: the sum of the rows may pass a float's range where every row's product is inside it.
 template <bool THROUGH>
-__device__ __forceinline__ void summed_rows_product(const GemmArgs &g, int m0, int n0, int z, int kbeg, int kend, char *__restrict__ S) {
+__device__ __forceinline__ bool summed_rows_product(const GemmArgs &g, int m0, int n0, int z, int kbeg, int kend, char *__restrict__ S) {
   constexpr int KB = 1024, ROWS = 16;  // k at a time; rows of A and of B to a wavefront
   float *s = reinterpret_cast<float *>(S);  // [4][KB], the sums in the first
   float *out = s + 4 * KB;                  // [64]
@@ -469,13 +472,19 @@ __device__ __forceinline__ void summed_rows_product(const GemmArgs &g, int m0, i
   acc[0] += __shfl_xor(acc[0], 1, 64);
   if ((lane & 3) == 0) out[ROWS * q + (lane >> 2)] = acc[0];
   __syncthreads();
-  if (n0 + lane >= g.N) return;
-  const float sum = out[lane];
-#pragma unroll 4
-  for (int r = 0; r < ROWS; r++) {
-    const int row = m0 + ROWS * q + r;
-    if (row < g.M) put_result<THROUGH>(g, z, row, n0 + lane, row == m0 ? sum : 0.f);
+  const float sum = out[lane];  // (every wavefront looks at all of them)
+  if (!__all(n0 + lane >= g.N || fabsf(sum) < INFINITY)) {
+    __syncthreads();
+    return false;
   }
+  if (n0 + lane < g.N) {
+#pragma unroll 4
+    for (int r = 0; r < ROWS; r++) {
+      const int row = m0 + ROWS * q + r;
+      if (row < g.M) put_result<THROUGH>(g, z, row, n0 + lane, row == m0 ? sum : 0.f);
+    }
+  }
+  return true;
 }
 
 // Columns n0 .. n0 + 64 of B (K x N) summed over rows [kbeg, kend), to s[64] in LDS.  N, ldb are multiples of 4, B 16-byte aligned.
@@ -548,8 +557,9 @@ __device__ __forceinline__ void split_tile(const GemmArgs &g, int m0, int n0, in
         return same_rows_product<BM, BN, VEC>(g, g.A + (long)m0 * g.lda, m0, n0, S);
     }
     if constexpr (!TA && TB && VEC && THROUGH) {
-      if (g.row_ids && m0 >= g.ids_from && kend > kbeg && same_ids(g.row_ids, m0, min(m0 + BM, g.M)))
-        return summed_rows_product<THROUGH>(g, m0, n0, z, kbeg, kend, S);
+      if (g.row_ids && m0 >= g.ids_from && kend > kbeg && same_ids(g.row_ids, m0, min(m0 + BM, g.M)) &&
+          summed_rows_product<THROUGH>(g, m0, n0, z, kbeg, kend, S))
+        return;
     }
     la.prepare(g.lda, m0, g.M, tid);
   }

@@ -156,3 +156,29 @@ def test_an_infinite_gradient_of_lookups(g):
     got = g.host(dW)
     assert np.isposinf(got[3, 7]) and np.isnan(got[3, 11]) and np.isnan(got[3, np.arange(W) % 64 != 7][20:40]).all()
     assert np.isfinite(np.delete(got, 3, axis=0)).all()
+
+
+def test_gradients_whose_sum_passes_the_range_of_a_float(g):
+    """Gradients of 2e37 .. 3e37: the sum of a block of 64 rows is infinite, the products with weights of 1e-6 and their sums are not."""
+    import torch
+
+    n, first, E, W, r = 400, 100, 64, 128, synth.SplitMix64(11)
+    e = r.bulk_uniform(n * E, 1e-4, 1e-3).reshape(n, E).astype(np.float32)
+    e[first:] = e[first]
+    ids = np.where(np.arange(n) < first, np.arange(n) % 40, 50).astype(np.float32)
+    d = r.bulk_uniform(n * W, 2e37, 3e37).reshape(n, W).astype(np.float32)
+    Wt = r.bulk_uniform(E * W, 5e-7, 1e-6).reshape(E, W).astype(np.float32)
+    de, dW, grad = torch.zeros(n, E, device="cuda"), torch.zeros(E, W, device="cuda"), torch.zeros(60, E, device="cuda")
+    e_, d_, W_ = g.devf(e), g.devf(d), g.devf(Wt)
+    descs = (hip.GemmDesc * 2)()
+    descs[0] = hip.GemmDesc(0, 1, n, E, W, 1.0, 0.0, g.P(d_), W, g.P(W_), W, g.P(de), E)
+    descs[1] = hip.GemmDesc(1, 0, E, W, n, 1.0, 0.0, g.P(e_), E, g.P(d_), W, g.P(dW), W)
+    nbytes = hip.lib().cavs_sgemm_group_workspace(2, descs)
+    ws, counters = torch.empty(max(nbytes // 4, 1), device="cuda"), torch.zeros(4096, dtype=torch.int32, device="cuda")
+    g.call("cavs_sgemm_group_lookups", 2, descs, 0, g.P(grad), g.P(g.devf(ids)), 3, first, g.P(ws), nbytes, g.P(counters), 4096, None, g.stream())
+    f = lambda a: a.astype(np.float64)  # noqa: E731
+    want, rows = np.zeros((60, E)), f(d) @ f(Wt).T
+    np.add.at(want, ids.astype(int), rows)
+    within(g.host(grad), want, want, W + n, "table")  # (everything is positive)
+    dw = f(e).T @ f(d)
+    within(g.host(dW), dw, dw, n, "d W")
