@@ -64,7 +64,13 @@ __device__ inline float tanh_r(float x) {
 #pragma clang fp contract(off)
   return 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + exp_r(2.f * x));
 }
-
+// WHOLE: the library's functions, as the gate launches beside separate products have them (gate_kernels.hip), which keep their
+// relative accuracy.  A round of that many rows keeps it too where it runs inside a resident launch: of pre-activations of 1e-4 tanh
+// is 2^-23 off, not 1e-3.
+template <bool WHOLE>
+__device__ inline float sigm_of(float x) { return WHOLE ? 1.f / (1.f + expf(-x)) : sigm_r(x); }
+template <bool WHOLE>
+__device__ inline float tanh_of(float x) { return WHOLE ? tanhf(x) : tanh_r(x); }
 
 // The gates of one hidden unit of one vertex (apps/paper/tree-lstm-cavs.cc:132-171): xw = the unit's
 // four columns of x * W ([i|o|u|f]), v = its five recurrent pre-activations (i, o, u, f_l, f_r),
@@ -74,17 +80,18 @@ __device__ inline float tanh_r(float x) {
 struct TreeLstmCell {
   float i, o, u, f_l, f_r, tc, h, c;
 };
+template <bool WHOLE = false>
 __device__ inline TreeLstmCell treelstm_cell(const float (&xw)[4], const float (&v)[5], const float (&bias)[4], float c_left,
                                              float c_right) {
 #pragma clang fp contract(off)
   TreeLstmCell q;
-  q.i = sigm_r((xw[0] + v[0]) + bias[0]);
-  q.o = sigm_r((xw[1] + v[1]) + bias[3]);
-  q.u = tanh_r((xw[2] + v[2]) + bias[2]);
-  q.f_l = sigm_r((xw[3] + v[3]) + bias[1]);
-  q.f_r = sigm_r((xw[3] + v[4]) + bias[1]);
+  q.i = sigm_of<WHOLE>((xw[0] + v[0]) + bias[0]);
+  q.o = sigm_of<WHOLE>((xw[1] + v[1]) + bias[3]);
+  q.u = tanh_of<WHOLE>((xw[2] + v[2]) + bias[2]);
+  q.f_l = sigm_of<WHOLE>((xw[3] + v[3]) + bias[1]);
+  q.f_r = sigm_of<WHOLE>((xw[3] + v[4]) + bias[1]);
   q.c = (q.i * q.u + q.f_l * c_left) + q.f_r * c_right;
-  q.tc = tanh_r(q.c);
+  q.tc = tanh_of<WHOLE>(q.c);
   q.h = q.o * q.tc;
   return q;
 }
@@ -159,14 +166,15 @@ __device__ inline void treelstm_gates_rows_at(const BwdGatesRowsArgs &a, long id
 struct LstmCell {
   float i, f, u, o, tc, h, c;
 };
+template <bool WHOLE = false>
 __device__ inline LstmCell lstm_cell(const float (&xw)[4], const float (&v)[4], const float (&bias)[4], float c_prev) {
   LstmCell q;
-  q.i = sigm_r((xw[0] + v[0]) + bias[0]);
-  q.f = sigm_r((xw[1] + v[1]) + bias[1]);
-  q.u = tanh_r((xw[2] + v[2]) + bias[2]);
-  q.o = sigm_r((xw[3] + v[3]) + bias[3]);
+  q.i = sigm_of<WHOLE>((xw[0] + v[0]) + bias[0]);
+  q.f = sigm_of<WHOLE>((xw[1] + v[1]) + bias[1]);
+  q.u = tanh_of<WHOLE>((xw[2] + v[2]) + bias[2]);
+  q.o = sigm_of<WHOLE>((xw[3] + v[3]) + bias[3]);
   q.c = q.i * q.u + q.f * c_prev;
-  q.tc = tanh_r(q.c);
+  q.tc = tanh_of<WHOLE>(q.c);
   q.h = q.o * q.tc;
   return q;
 }

@@ -360,23 +360,24 @@ __global__ __launch_bounds__(512, 1) void group_fwd_kernel(GroupFwdArgs a) {
       e_c[k] = on ? e_c[k] : 0.f;
     }
     float st[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, h = 0.f, cc = 0.f;  // what the backward pass wants, and the state
+    const bool whole = w.cur.w & 4;
     if (eon) {
       float v[NP];
       if (WIDE && ks < 4 * TW) wide_sum<NP>(red, ks, lane, v);
       else group_sum<NP>(red, ks, slot, x, v);
       if constexpr (MODEL == GROUP_TREELSTM) {
-        const TreeLstmCell q = treelstm_cell(xw, v, bias, e_c[0], e_c[NC - 1]);
+        const TreeLstmCell q = whole ? treelstm_cell<true>(xw, v, bias, e_c[0], e_c[NC - 1]) : treelstm_cell(xw, v, bias, e_c[0], e_c[NC - 1]);
         st[0] = q.i; st[1] = q.o; st[2] = q.u; st[3] = q.f_l; st[4] = q.f_r; st[5] = q.tc;
         h = q.h; cc = q.c;
       } else if constexpr (MODEL == GROUP_LSTM) {
-        const LstmCell q = lstm_cell(xw, v, bias, e_c[0]);
+        const LstmCell q = whole ? lstm_cell<true>(xw, v, bias, e_c[0]) : lstm_cell(xw, v, bias, e_c[0]);
         st[0] = q.i; st[1] = q.f; st[2] = q.u; st[3] = q.o; st[4] = q.tc;
         h = q.h; cc = q.c;
       } else {
         float t = v[0] + v[1];
         if (a.bias) t += bias[0];
         if (a.xW) t += xw[0];
-        h = a.act ? tanh_r(t) : (t > 0.f ? t : 0.f);
+        h = !a.act ? (t > 0.f ? t : 0.f) : whole ? tanhf(t) : tanh_r(t);
       }
       // the message first: it is all a later round of this launch reads
       if (rec.w >= 0) {

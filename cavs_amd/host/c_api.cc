@@ -201,7 +201,7 @@ int cavs_schedule_group_lists(const int *graph, int B, int maxlen, int nchild, i
   std::vector<int> room(cavs::group_lists_bound(sch, N - sch.scatter_ids.size(), groups), mark);
   cavs::GroupLists t;
   cavs::build_group_lists(sch, nchild, t2j.data(), pair.data(), child.data(), kid.data(), forward_only ? nullptr : orphans.data(), n_orphans, rows_limit,
-                          groups, slice, only_wide != 0, &t, room.data());
+                          groups, slice, only_wide != 0, 1 << 30, &t, room.data());
   const int out[10] = {t.first, t.ngroups, t.tile_rows, (int)t.fwd.groups, (int)t.fwd.lists, (int)t.fwd.recs,
                        (int)t.bwd.groups, (int)t.bwd.lists, (int)t.bwd.recs, (int)room.size()};
   std::copy(out, out + 10, meta);

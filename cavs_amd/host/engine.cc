@@ -207,7 +207,7 @@ void Engine::build_group_plan(const int *t2j, const int *pair, const int *child,
   if (tail_limit() > 0 && std::all_of(sched_->rounds.begin(), sched_->rounds.end(), [&](const Round &r) { return r.n <= 8 || leaf_round(r); })) return;
   // (nor where tiles of four are the better ones: the tail launches are tuned for those)
   build_group_lists(*sched_, nch_, t2j, pair, child, kid_rows, lists_forward_only() ? nullptr : orphans, n_orphans_, group_limit(),
-                    cavs_group_max_groups(cfg_.H), cavs_group_rows(), tail_limit() > 0, &group_, block);
+                    cavs_group_max_groups(cfg_.H), cavs_group_rows(), tail_limit() > 0, fused_rows(), &group_, block);
 }
 
 cavs_group_plan Engine::group_plan(const GroupLists::Launch &l) const {

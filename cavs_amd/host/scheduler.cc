@@ -437,7 +437,7 @@ static int group_tile_rows(const std::vector<int> &per, int rounds, int slice) {
 static constexpr int kUnevenShare = 64;
 
 void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pair, const int *child, const int *kid_rows, const int *orphans,
-                       int n_orphans, int lim, int groups, int slice, bool only_wide, GroupLists *out, int *block) {
+                       int n_orphans, int lim, int groups, int slice, bool only_wide, int whole_from, GroupLists *out, int *block) {
   const bool back = orphans != nullptr;
   *out = GroupLists();
   const int R = (int)s.rounds.size(), N = s.N;
@@ -542,9 +542,9 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
         }
         done += alone > 0;
         for (int i = 0; i < nr; i++) {
-          const int k = dir ? nr - 1 - i : i, c = per[(size_t)g * nr + k];
+          const int k = dir ? nr - 1 - i : i, c = per[(size_t)g * nr + k], whole = !dir && s.rounds[k0 + k].n > whole_from ? 4 : 0;
           for (int c0 = 0; c0 < c; c0 += slice, nl++) {
-            const int row[4] = {at[(size_t)g * nr + k] + c0, std::min(slice, c - c0), c0 == 0 ? done : 0, c0 + slice >= c};
+            const int row[4] = {at[(size_t)g * nr + k] + c0, std::min(slice, c - c0), c0 == 0 ? done : 0, (c0 + slice >= c) | whole};
             std::copy(row, row + 4, lists + 4 * (size_t)nl);
           }
           done += c > 0;

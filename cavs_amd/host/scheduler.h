@@ -104,9 +104,10 @@ struct GroupLists {
 size_t group_lists_bound(const Schedule &s, size_t alone, int groups);
 // lists as build_index_lists / build_forest_lists leave them; orphans: null where no backward pass may follow
 // (its lists are left out); lim: most rows of a round a group may get; slice: most rows per list; only_wide: nothing
-// where the lists would run in tiles of four rows.  out->first stays -1 when no two rounds qualify.
+// where the lists would run in tiles of four rows; whole_from: forward lists of rounds of more rows are marked for whole gate
+// functions (cavs_group_plan).  out->first stays -1 when no two rounds qualify.
 void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pair, const int *child, const int *kid_rows, const int *orphans,
-                       int n_orphans, int lim, int groups, int slice, bool only_wide, GroupLists *out, int *block);
+                       int n_orphans, int lim, int groups, int slice, bool only_wide, int whole_from, GroupLists *out, int *block);
 // kid_rows as build_forest_lists leaves them (binary trees); rows_out: room for N ints.
 void build_tail_lists(const Schedule &s, const int *kid_rows, int lim, int groups, int max_lists, int slice, TailLists *out,
                       int *rows_out);

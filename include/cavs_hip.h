@@ -542,7 +542,8 @@ int cavs_tail_probe(unsigned *sync, int H, int spin_max, void *stream);
  *   groups  [ngroups][4]  first list, number of lists, arrivals of the launch, 0
  *   lists   [*][4]        first record, rows (at most cavs_group_rows()), arrivals that must be in, arrives (0 / 1); backward + 2: rows
  *                         that get no gradient from a parent, each named as its own child 0: what
- *                         cavs_*_bwd_rows does with them
+ *                         cavs_*_bwd_rows does with them; forward + 4: gate functions as the library's expf and
+ *                         tanhf, not the 1e-7 absolute of the rounds
  *   recs    [*][8]        forward:  slab row, pool rows of its children (-1: none), pool row its message goes
  *                                   to (-1: none), row of graph_out, 0, 0, 0
  *                         backward: slab row, slab rows of its children, row of dret of child 0, of child 1, 0, 0, 0

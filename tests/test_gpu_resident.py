@@ -176,6 +176,46 @@ def test_training_with_a_round_above_the_fused_limit(model, H, schedule, plan_ca
         x.close()
 
 
+@pytest.mark.parametrize("model,H,schedule,plan_cache", [("treelstm", 64, "host", 0), ("treelstm", 512, "device", 2), ("treefc", 64, "host", 2),
+                                                         ("treefc", 256, "host", 0)])
+def test_a_resident_round_above_the_fused_limit_keeps_relative_accuracy(model, H, schedule, plan_cache):
+    """Pre-activations of 1e-6 .. 1e-3, and gates near 0 and 1, in a round of more than 2048 rows: relative errors of a few
+    units, as the launches beside separate products give that ran such rounds.  Without weights, so that the pre-activations are what is declared."""
+    w = small_workload(model, 81, B=1700, H=H, E=12, V=31, C=5)
+    tr = session.schedule_trace(w["graph"])
+    r2o, t2j = np.array(tr["round2offset"]), np.array(tr["tids_to_jobids"])
+    big = int(np.argmax(np.diff(r2o)[1:])) + 1
+    at = t2j[r2o[big]:r2o[big + 1]]
+    assert 2048 < at.size <= 4096
+    r = synth.SplitMix64(H)
+    small = lambda n: (10.0 ** r.bulk_uniform(n, -6, -3) * np.where(r.bulk_uniform(n) < 0.5, -1, 1)).astype(np.float32)  # noqa: E731
+    w["params"]["W"] = np.zeros_like(w["params"]["W"])
+    if model == "treelstm":
+        w["params"].update(U=np.zeros_like(w["params"]["U"]), Bv=np.concatenate([r.bulk_uniform(2 * H, -12, 6), small(H), r.bulk_uniform(H, -12, 6)]))
+    else:
+        w["params"]["Bv"] = np.zeros_like(w["params"]["Bv"])
+        w["x"] = small(w["x"].size).reshape(-1, H)
+    s = _session(model, H, w, schedule=schedule, plan_cache=plan_cache)
+    for _ in range(2):
+        s.step(w["graph"], w["x"], w["labels"], backward=True, lr=0.0)
+        assert s.counter("tail_rounds") > 0
+        got = s.fetch("graph_out")[at].astype(np.float64)
+        if model == "treelstm":
+            sig = lambda v: 1 / (1 + np.exp(-v.astype(np.float64)))  # noqa: E731
+            bi, bf, bu, bo = np.asarray(w["params"]["Bv"], np.float32).reshape(4, H)
+            c = s.fetch("msg_pool")  # (the children's states, as they are: their round may have the rounds' functions)
+            child = np.array([[v for v in tr["fwd"][big]["gather"][k]] for k in (0, 1)])
+            cl, cr = (c[child[k]][:, H:].astype(np.float64) for k in (0, 1))
+            cc = sig(bi) * np.tanh(bu.astype(np.float64)) + sig(bf) * cl + sig(bf) * cr
+            want = sig(bo) * np.tanh(cc)
+        else:
+            want = np.tanh(w["x"][at].astype(np.float64))
+        # products of three gates, a sum of three terms of either sign: ten roundings of the terms' magnitudes
+        mag = np.abs(want) if model == "treefc" else sig(bo) * (sig(bi) * np.abs(np.tanh(bu.astype(np.float64))) + sig(bf) * (np.abs(cl) + np.abs(cr)))
+        assert (np.abs(got - want) <= 10 * 2.0 ** -23 * mag).all(), (np.abs(got - want) / mag).max()
+    s.close()
+
+
 @pytest.mark.parametrize("H,B,kw", [(32, 5, {}), (96, 40, {}), (256, 600, {}), (64, 600, dict(tail_rows=-1)), (64, 600, dict(fused_round_rows=300)),
                                     (40, 30, {})])
 @pytest.mark.parametrize("shift", [0, 1])
