@@ -913,6 +913,7 @@ void Engine::remember_plan(const int *graph, int B, int maxlen, uint64_t hash) {
     check(cavs_stream_sync(stream_));
     p = std::move(plans_[lru]);
     p->drop_graphs();
+    p->ran[0] = p->ran[1] = false;
     plans_.erase(plans_.begin() + lru);
   } else {
     p = std::make_unique<Plan>();
@@ -957,6 +958,7 @@ void Engine::remember_plan(const int *graph, int B, int maxlen, uint64_t hash) {
   d_orphans_ = kids ? base + 2 * N + 2 * nk + B : nullptr;
   d_tail_rows_ = base + 3 * N + 2 * nk + B;
   plans_.push_back(std::move(p));
+  step_plan_ = plans_.back().get();
 }
 
 // A schedule nobody holds any more (no cached plan), or a new one: a step's vectors keep their memory.
@@ -1170,7 +1172,7 @@ void Engine::begin_step(const int *graph, int B, int maxlen) {
     hash = hash_feed(graph, (size_t)B * maxlen, B, maxlen, cfg_.pairing);
     hit = find_plan(graph, B, maxlen, hash);
   }
-  hit_plan_ = hit;
+  hit_plan_ = step_plan_ = hit;
   if (probe_due_) tail_setup();
   resident_ = tail_ready_ && fused_rows() > 0 && claim_.take(cfg_.device);
   if (hit) {
@@ -1448,7 +1450,7 @@ void Engine::step(const int *graph, int B, int maxlen, const void *x, const void
     for (StepGraph &g : plan->graphs)
       if (g.sig == sig) recorded = &g;
     // (a plan whose signatures keep changing -- new feed buffers every step -- stops recording)
-    if (!recorded) record = plan->recordings++ < 6;
+    if (!recorded && plan->ran[backward]) record = plan->recordings++ < 6;
   }
   if (recorded) {
     check(cavs_graph_launch(recorded->exec, stream_));
@@ -1491,6 +1493,7 @@ void Engine::step(const int *graph, int B, int maxlen, const void *x, const void
     }
   } else {
     run_passes(backward);
+    if (step_plan_) step_plan_->ran[backward] = true;
   }
   if (backward) {
     aux_join();  // (the head's weight gradients)

@@ -348,6 +348,9 @@ class Engine {
     }
     std::vector<StepGraph> graphs;
     bool graph_off = false;  // recording failed once: ordinary steps from then on
+    // an ordinary pass of the kind has run (forward only; with its backward pass), so that a recorded one finds every buffer at its size:
+    // one that grows waits for the stream, which a stream that is being recorded cannot
+    bool ran[2] = {false, false};
     int recordings = 0;
     uint64_t hash = 0;
     int B = 0, maxlen = 0, pairing = 0;
@@ -367,7 +370,8 @@ class Engine {
   uint64_t plan_clock_ = 0;
   double c_plan_hits_ = 0, c_plan_misses_ = 0;
   int scheduler_used_ = 0;  // who produced the last step's lists: 0 host scheduler, 1 device scheduler, 2 plan cache
-  Plan *hit_plan_ = nullptr;  // the cached plan this step runs on (null: it was scheduled afresh)
+  Plan *hit_plan_ = nullptr;   // the cached plan this step runs on (null: it was scheduled afresh)
+  Plan *step_plan_ = nullptr;  // that, or the one its scheduling left in the cache
   Plan *find_plan(const int *graph, int B, int maxlen, uint64_t hash);
   void remember_plan(const int *graph, int B, int maxlen, uint64_t hash);
 

@@ -709,6 +709,38 @@ def test_sizes_that_are_no_multiple_of_a_tile(oracle, model, loss, kw, H, E):
     s.close()
 
 
+@pytest.mark.parametrize("model,H,C,B,replay", [("lstm", 64, 4096, 800, False), ("treelstm", 32, 600, 480, False), ("lstm", 64, 600, 800, True)])
+def test_a_head_over_thousands_of_rows_leaves_its_columns_sums(oracle, model, H, C, B, replay):
+    """4096 rows and more, 512 classes and more: the bias gradient from the sums that the loss's launch leaves, on the side stream
+    (C H >= 2^18), in the grouped launch, and in a session that records its steps and has seen the batch forward only; losses, gradients and
+    updated parameters against the oracle."""
+    import torch
+
+    w = small_workload(model, 97, B=B, H=H, E=12, V=31, C=C)
+    assert w["N"] >= 4096
+    s = session.Session(model, H=H, E=w["E"], V=31, C_=C, plan_cache=2 if replay else 0, graph_replay=replay)
+    p = {k: np.array(v, np.float32) for k, v in w["params"].items()}
+    s.set_params(p)
+    x, labels = w["x"], w["labels"]
+    if replay:
+        x, labels = (torch.from_numpy(np.ascontiguousarray(a, np.float32)).cuda() for a in (x, labels))
+        torch.cuda.synchronize()
+        for _ in range(2):
+            s.step(w["graph"], x, labels, backward=False)
+    lr = np.float32(0.05)
+    for step in range(4 if replay else 2):
+        s.step(w["graph"], x, labels, backward=True, lr=float(lr))
+        want = oracle.model_step(model, w["graph"], w["x"], w["labels"], dict(w["params"], **p), H=H, E=w["E"], V=31, Cc=C, precise=True, threads=16)
+        close(s.fetch("loss"), want["loss"], f"loss of step {step}", scaled=False)
+        got = s.grads()
+        for k, v in want["grads"].items():
+            close(got[k], v, f"{k} of step {step}", scaled=False)
+            p[k[1:]] = (p[k[1:]].ravel() - lr * np.asarray(v, np.float32).ravel()).reshape(p[k[1:]].shape)
+            close(s.param(k[1:], p[k[1:]].shape), p[k[1:]], f"{k[1:]} after step {step}")
+    assert s.counter("graph_replays") == (4 if replay else 0), s.counter("graph_replays")
+    s.close()
+
+
 @pytest.mark.parametrize("model,H,E,B", [("treelstm", 150, 60, 2), ("treelstm", 100, 64, 25), ("treelstm", 70, 300, 90), ("treelstm", 200, 2048, 90), ("lstm", 50, 50, 3), ("lstm", 200, 200, 40),
                                          ("lstm", 72, 72, 160)])
 def test_an_infinite_embedding_saturates_gates_and_nothing_else_at_sizes_stored_with_padding(model, H, E, B):
