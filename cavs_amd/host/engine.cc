@@ -293,6 +293,7 @@ std::string Engine::tail_settle() {
 
 Engine::~Engine() {
   cavs_stream_sync(stream_);
+  plans_.clear();  // (their recorded graphs in front of the stream they ran on)
   for (CellStage &st : cells_) cavs_cell_release(st.module);
   cavs_cell_release(cell_rounds_);
   for (auto &e : ev_) cavs_event_destroy(e);
@@ -1480,6 +1481,7 @@ void Engine::step(const int *graph, int B, int maxlen, const void *x, const void
     }
     if (ok) {
       if (plan->graphs.size() >= 4) {
+        check(cavs_stream_sync(stream_));  // (a launch of it may be under way)
         cavs_graph_destroy(plan->graphs.front().exec);
         plan->graphs.erase(plan->graphs.begin());
       }

@@ -51,6 +51,23 @@ def run(standin, script):
     return (*map(int, head.split()), faults)
 
 
+def test_recorded_graphs_go_before_the_streams_they_ran_on(standin):
+    """A session's graphs are given back before its streams, and none while a launch of it may be under way: not at the session's
+    end, not where a fifth recording of a batch takes the place of the first."""
+    recorded, replayed, faults = run(standin, """
+s = session.Session("treefc", H=32, E=0, V=0, C_=5, loss="root_sq", plan_cache=2, graph_replay=True, use_x=True)
+g = trees(4, 6)
+xs = [feeds(g, 5, 32) for _ in range(6)]
+s.step(g, *xs[0])
+for x in xs:
+    for _ in range(2):
+        s.step(g, *x)
+s.close()
+""")
+    assert recorded >= 5 and replayed > recorded
+    assert faults == []
+
+
 @pytest.mark.parametrize("model,loss,C,B,n", [("lstm", "softmax", 512, 300, 16), ("lstm", "softmax", 5, 20, 7), ("lstm", "softmax", 4096, 40, 9),
                                               ("treelstm", "softmax", 600, 300, 8), ("treelstm", "softmax", 5, 6, 9), ("treefc", "root_sq", 5, 6, 9),
                                               ("treefc", "sum_abs", 5, 20, 9), ("treelstm", "softmax", 5, 900, 7)])
