@@ -132,12 +132,17 @@ __global__ __launch_bounds__(256) void softmax_xent_kernel(float *__restrict__ l
   }
 }
 
-// a / b for one b and many a, r = 1 / b as the division rounds it: the product with r is off by an ulp at most, and its remainder, exact in
-// an fma, sets it right (Markstein's theorem: the division's own bits, while a is above 2^-100).  Three operations instead of the ten of a
-// division: 7000 rows of 10000 with their sums 108.8 -> 105.9 us, 5.3 TB/s.
+// a / b for one b and four a at a time, r = 1 / b as the division rounds it: the product with r is off by an ulp at most, and its remainder,
+// exact in an fma, sets it right (Markstein's theorem: the division's own bits, while a is above 2^-100 and the remainder a float).  Three
+// operations instead of the ten of a division: 7000 rows of 10000 with their sums 108.8 -> 105.9 us, 5.3 TB/s.  Below that (a logit 69 under
+// its row's largest) it is the division: by the remainder, quotients were up to 6e-4 of themselves off at 2^-126, and all of it at the least.
 __device__ inline float quotient(float a, float b, float r) {
   const float q = a * r;
   return fmaf(fmaf(-q, b, a), r, q);
+}
+__device__ inline float4 quotients(const float4 &a, float b, float r) {
+  if (fminf(fminf(a.x, a.y), fminf(a.z, a.w)) < 0x1p-100f) return make_float4(a.x / b, a.y / b, a.z / b, a.w / b);
+  return make_float4(quotient(a.x, b, r), quotient(a.y, b, r), quotient(a.z, b, r), quotient(a.w, b, r));
 }
 
 // One workgroup per row, the row held in registers between the passes (NV float4 per thread,
@@ -181,7 +186,7 @@ __global__ __launch_bounds__(256) void softmax_xent_rows_kernel(float *__restric
   for (int k = 0; k < NV; k++) {
     const int j = tid + 256 * k;
     if (j >= C4) continue;
-    float4 p = make_float4(quotient(v[k].x, sum, r), quotient(v[k].y, sum, r), quotient(v[k].z, sum, r), quotient(v[k].w, sum, r));
+    float4 p = quotients(v[k], sum, r);
     if (lab >> 2 == j) {  // (one by one: a reference to one of them would put them all into memory)
       const int c = lab & 3;
       p.x -= c == 0 ? 1.f : 0.f, p.y -= c == 1 ? 1.f : 0.f, p.z -= c == 2 ? 1.f : 0.f, p.w -= c == 3 ? 1.f : 0.f;
@@ -246,7 +251,7 @@ __global__ __launch_bounds__(kSumsThreads) void softmax_xent_sums_kernel(float *
     for (int k = 0; k < NV; k++) {
       const int j = tid + kSumsThreads * k;
       if (j < C4) {
-        float4 p = make_float4(quotient(v[k].x, sum, r), quotient(v[k].y, sum, r), quotient(v[k].z, sum, r), quotient(v[k].w, sum, r));
+        float4 p = quotients(v[k], sum, r);
         if (lab >> 2 == j) {
           const int c = lab & 3;
           loss[row] = -logf((c == 0 ? v[k].x : c == 1 ? v[k].y : c == 2 ? v[k].z : v[k].w) / sum);  // (a probability may be tiny)

@@ -2127,6 +2127,39 @@ def test_softmax_leaves_its_columns_sums(g, n, C_):
     assert hip.lib().cavs_softmax_xent_sum_rows(4095, C_) == 0 and hip.lib().cavs_softmax_xent_sum_rows(n, 508) == 0
 
 
+def _probabilities_of_any_size(n, C_):
+    """Logits with a sum of exponentials that no order of adding up changes: one entry at the row's largest, one up to 3 below it, the
+    others 30 .. 104 below, down to what exp makes a denormal or zero of."""
+    r = rng(n + C_)
+    x = -r.bulk_uniform(n * C_, 30, 104).reshape(n, C_)
+    at = np.floor(r.bulk_uniform(2 * n) * (C_ // 2)).astype(int).reshape(2, n)
+    x[np.arange(n), 2 * at[0]] = 0
+    x[np.arange(n), 2 * at[1] + 1] = -r.bulk_uniform(n, 0, 3)
+    labels = np.floor(r.bulk_uniform(n) * C_).astype(np.float32)
+    return x.astype(np.float32), labels
+
+
+@pytest.mark.parametrize("n,C_", [(1, 512), (1, 10004), (1, 16384), (4096, 512), (4096, 2052)])
+def test_softmax_of_wide_rows_divides_as_a_division(g, n, C_):
+    """Probabilities by the sum's reciprocal and a remainder, of every size down to zero: the bits of the kernel that divides (a
+    wavefront per row: what rows that are not 16-byte aligned run on)."""
+    import torch
+
+    logits, labels = _probabilities_of_any_size(n, C_)
+    x, lab = g.devf(logits), g.devf(labels)
+    off = torch.empty(n * C_ + 1, device="cuda")
+    off[1:] = x.reshape(-1)
+    loss, d, want_loss, want = g.zeros(n), g.zeros(n, C_), g.zeros(n), g.zeros(n, C_)
+    g.call("cavs_softmax_xent", g.P(want_loss), g.P(want), g.P(off) + 4, g.P(lab), n, C_, g.stream())
+    g.call("cavs_softmax_xent", g.P(loss), g.P(d), g.P(x), g.P(lab), n, C_, g.stream())
+    np.testing.assert_array_equal(g.host(d).view(np.uint32), g.host(want).view(np.uint32))
+    rows = hip.lib().cavs_softmax_xent_sum_rows(n, C_)
+    if rows:
+        d2, sums = g.zeros(n, C_), g.zeros(rows, C_)
+        g.call("cavs_softmax_xent_sums", g.P(loss), g.P(d2), g.P(x), g.P(lab), g.P(sums), n, C_, g.stream())
+        np.testing.assert_array_equal(g.host(d2).view(np.uint32), g.host(want).view(np.uint32))
+
+
 @pytest.mark.parametrize("n", [1, 16, 17, 1000, 8192, 8193, 9000])
 def test_sums_by_word_leave_the_sum_of_all(g, n):
     """Pieces of 16 and of 64 rows, the last one short: rows that add up to the sum of all rows, beside the words' own sums."""
