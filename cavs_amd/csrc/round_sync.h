@@ -103,8 +103,8 @@ __device__ inline float ld_row(const float *p) { return *p; }
 // lower half of the second; swapping two rows' accumulators and adding puts both partial sums into
 // one register, a butterfly of three swaps and three adds per product on the vector ALU (a shuffle
 // through the LDS crossbar costs eight cycles of a unit all eight wavefronts share).  Spelled out
-// as instructions because the compiler's builtins for the two swaps return the first result twice.
-// The compiler does not look inside such a statement, so the waits an instruction needs after the
+// as instructions, which change both operands where they are, in the order that is wanted between
+// other work.  The compiler does not look inside such a statement, so the waits an instruction needs after the
 // one that produced its operand are the caller's: all() carries its own (twelve cycles cover the
 // six a two-pass MFMA asks for before a vector-ALU read, two between an add and the swap that reads
 // it); the stages are for callers that put at least that many instructions between them.

@@ -2160,6 +2160,30 @@ def test_softmax_of_wide_rows_divides_as_a_division(g, n, C_):
         np.testing.assert_array_equal(g.host(d2).view(np.uint32), g.host(want).view(np.uint32))
 
 
+def test_sums_and_maxima_over_a_wavefront(g):
+    """Sums over a wavefront have the bits of six steps that each add lane l's value to that of lane l ^ 32, 16, 8, 4, 2, 1 (a head
+    whose logits are a row's 64 values added up), and every lane's value counts for the maximum (the one large logit in each of them)."""
+    n, H, C_, r = 200, 64, 3, rng(17)
+    X = (r.bulk_normal(n * H) * 10.0 ** r.bulk_uniform(n * H, -3, 3)).reshape(n, H).astype(np.float32)
+    W = np.stack([np.ones(H), -np.ones(H), 2.0 ** (np.arange(H) % 5)]).astype(np.float32)
+    loss, logits = g.zeros(n), g.zeros(n, C_)
+    g.call("cavs_fc_softmax_xent", g.P(g.devf(X)), g.P(g.devf(W)), g.P(g.devf(np.zeros(C_))), g.P(g.devf(np.zeros(n))), g.P(loss), g.P(logits),
+           None, None, None, None, 0, n, H, C_, g.stream())
+    want = np.empty((n, C_), np.float32)
+    for c in range(C_):
+        v = X * W[c]
+        for o in (32, 16, 8, 4, 2, 1):
+            v = v + v[:, np.arange(64) ^ o]
+        want[:, c] = v[:, 0]
+    np.testing.assert_array_equal(g.host(logits).view(np.uint32), want.view(np.uint32))
+    x = r.bulk_uniform(64 * 64, -300, -200).reshape(64, 64).astype(np.float32)
+    x[np.arange(64), np.arange(64)] = 200
+    loss, d = g.zeros(64), g.zeros(64, 64)
+    g.call("cavs_softmax_xent", g.P(loss), g.P(d), g.P(g.devf(x)), g.P(g.devf(np.arange(64))), 64, 64, g.stream())
+    np.testing.assert_array_equal(g.host(loss), 0)
+    np.testing.assert_array_equal(g.host(d), 0)
+
+
 @pytest.mark.parametrize("n", [1, 16, 17, 1000, 8192, 8193, 9000])
 def test_sums_by_word_leave_the_sum_of_all(g, n):
     """Pieces of 16 and of 64 rows, the last one short: rows that add up to the sum of all rows, beside the words' own sums."""
