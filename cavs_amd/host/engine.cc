@@ -181,11 +181,20 @@ int Engine::tail_limit() const {
 // chains in batches of 1024 1.745 -> 1.538; H = 256 0.697 -> 0.655.  Tree-FC keeps its rounds' order of sums above H = 256: its
 // training multiplies a difference in rounding by up to 1.4 a step there (1e-6 after one step at H = 512, 2e-4 after 16, whichever
 // two orders are compared), at 256 by 1.05.
+// A group that leaves more than a third of its chiplet idle (H = 288 and 320: 18 and 20 of 32 workgroups) takes 128 rows at most: larger
+// rounds fill the device better as launches of their own.  512 and 1024 trees of 5 .. 35 leaves, us a step with 512 / with 128: H = 288
+// 916 / 871 and 1578 / 1460, 320 938 / 911 and 1665 / 1601; H = 352 (22 workgroups) 1045 / 1047 and 1815 / 1794, with 256 trees 528 / 556.
+// (With 512 those at 288 were slower than no round of that size resident: 0.97 of the rate in training, evaluated by a kept plan
+// 0.94, 1600 chains of 10 .. 40 0.91; now 1.06, 1.04, 1.00.)
 int Engine::group_limit() const {
   if (!resident_ || fused_rows() <= 0 || (cell_ && cell_->rounds.empty()) || !cavs_group_rounds_ok(cfg_.H)) return 0;
   if (cfg_.tail_rows > 0) return tail_limit() > 0 ? 0 : cfg_.tail_rows;
   if (cell_) return 64;
-  if (!lists_forward_only()) return cfg_.model == CAVS_MODEL_TREEFC && cfg_.H > 256 ? 64 : 512;
+  if (!lists_forward_only()) {
+    if (cfg_.model == CAVS_MODEL_TREEFC && cfg_.H > 256) return 64;
+    const int used = cavs_group_max_groups(cfg_.H) / 8 * (cfg_.H / 16);  // of a chiplet's 32 workgroups
+    return 3 * used < 2 * 32 ? 128 : 512;
+  }
   return (cfg_.model == CAVS_MODEL_TREELSTM && cfg_.H > 384) || (cfg_.model == CAVS_MODEL_LSTM && cfg_.H >= 384) ? 256 : 64;
 }
 

@@ -154,6 +154,23 @@ def test_a_forward_pass_plans_for_itself(model, H, B):
         x.close()
 
 
+@pytest.mark.parametrize("H,B,resident", [(288, 1024, True), (288, 1040, False), (320, 1040, False), (352, 1040, True)])
+def test_a_group_that_leaves_much_of_its_chiplet_idle_takes_128_rows(H, B, resident):
+    """Chains of equal length in training: rounds of 128 rows a group (of eight) are resident at every size, rounds of 130 where a group
+    is at least two thirds of its chiplet's workgroups; both ways what launches of their own give."""
+    w = small_workload("lstm", 83, B=B, H=H, E=H, V=31, C=5, skew=False)
+    s, ref = (_session("lstm", H, w, tail_rows=k) for k in (0, -1))
+    for x in (s, ref):
+        x.step(w["graph"], w["x"], w["labels"], backward=True, lr=1e-3)
+    assert (s.counter("tail_rounds") > 0) == resident and ref.counter("tail_rounds") == 0
+    close(s.fetch("graph_out"), ref.fetch("graph_out"), "graph_out")
+    got, want = s.grads(), ref.grads()
+    for name, v in want.items():
+        close(got[name], v, name)
+    for x in (s, ref):
+        x.close()
+
+
 @pytest.mark.parametrize("model,H,schedule,plan_cache", [("treelstm", 64, "host", 0), ("treelstm", 512, "device", 0), ("treefc", 96, "host", 2),
                                                          ("treefc", 256, "device", 2)])
 def test_training_with_a_round_above_the_fused_limit(model, H, schedule, plan_cache):
