@@ -709,6 +709,26 @@ def test_sizes_that_are_no_multiple_of_a_tile(oracle, model, loss, kw, H, E):
     s.close()
 
 
+@pytest.mark.parametrize("model,H,E", [("treelstm", 150, 300), ("treelstm", 70, 33), ("lstm", 200, 200), ("lstm", 72, 72)])
+def test_sizes_stored_with_padding_against_the_oracle(oracle, model, H, E):
+    """One pass, then two SGD steps whose gradients and parameters must be those of w - lr * g, at sizes that small models are trained at."""
+    w = small_workload(model, 823, B=25, H=H, E=E)
+    got, want = run_both(oracle, w)
+    compare(got, want)
+    s = session.Session(model, H=H, E=w["E"], V=w["V"], C_=w["C"])
+    p = {k: np.array(v, np.float32) for k, v in w["params"].items()}
+    s.set_params(p)
+    lr = np.float32(0.05)
+    for step in range(2):
+        s.step(w["graph"], w["x"], w["labels"], backward=True, lr=float(lr))
+        want = oracle.model_step(model, w["graph"], w["x"], w["labels"], dict(w["params"], **p), H=H, E=w["E"], V=w["V"], Cc=w["C"], precise=True)
+        close(s.fetch("loss"), want["loss"], f"loss of step {step}")
+        for k, v in want["grads"].items():
+            p[k[1:]] = (p[k[1:]].ravel() - lr * np.asarray(v, np.float32).ravel()).reshape(p[k[1:]].shape)
+            close(s.param(k[1:], p[k[1:]].shape), p[k[1:]], k[1:])
+    s.close()
+
+
 @pytest.mark.parametrize("model,H,C,B,replay", [("lstm", 64, 4096, 800, False), ("treelstm", 32, 600, 480, False), ("lstm", 64, 600, 800, True)])
 def test_a_head_over_thousands_of_rows_leaves_its_columns_sums(oracle, model, H, C, B, replay):
     """4096 rows and more, 512 classes and more: the bias gradient from the sums that the loss's launch leaves, on the side stream
