@@ -181,6 +181,8 @@ int Engine::tail_limit() const {
 // chains in batches of 1024 1.745 -> 1.538; H = 256 0.697 -> 0.655.  Tree-FC keeps its rounds' order of sums above H = 256: its
 // training multiplies a difference in rounding by up to 1.4 a step there (1e-6 after one step at H = 512, 2e-4 after 16, whichever
 // two orders are compared), at 256 by 1.05.
+// (Forward, us with 64 / with 512: trees of 5 .. 35 leaves, 512 and 1024 of them, H = 288 320 / 352 and 541 / 624, 320 343 / 363 and 592 / 650, 352 361 /
+// 378 and 641 / 679; 1024 chains of 10 .. 40 H = 288 756 / 737, 320 816 / 756, 352 902 / 785, but 1600 of them at 288 1030 / 1110.)
 // A group that leaves more than a third of its chiplet idle (H = 288 and 320: 18 and 20 of 32 workgroups) takes 128 rows at most: larger
 // rounds fill the device better as launches of their own.  512 and 1024 trees of 5 .. 35 leaves, us a step with 512 / with 128: H = 288
 // 916 / 871 and 1578 / 1460, 320 938 / 911 and 1665 / 1601; H = 352 (22 workgroups) 1045 / 1047 and 1815 / 1794, with 256 trees 528 / 556.
@@ -202,7 +204,9 @@ int Engine::group_limit() const {
 // can be resident.  A round above fused_rows() is slower as such a launch than as products, but with one of them in the batch
 // every round was: 128 trees of 30 .. 120 leaves (largest round 3086) gain 1.07 (Tree-FC, H = 64) .. 1.32 (H = 256) and 1.11 ..
 // 1.64 (Tree-LSTM), 256 of them (6181) 1.01 (Tree-LSTM, H = 384) .. 1.18, but Tree-FC 0.92 at H = 64 and 0.96 at 128; at 10400 rows it
-// is 0.85 .. 1.11, at 23700 0.6 .. 1.0.  (Tree-FC up to H = 256, as above)
+// is 0.85 .. 1.11, at 23700 0.6 .. 1.0.  (Tree-FC up to H = 256, as above)  The rate of 90, 128, 165 and 250 such trees over that of rounds by
+// products, everything else of a step included: Tree-LSTM H = 64 1.39 .. 1.54, 128 .. 160 1.31 .. 1.61, 192 1.18 .. 1.46, 256 1.28 .. 1.50,
+// 384 1.08 .. 1.26, 512 1.07 .. 1.26; Tree-FC H = 192 and 256 1.41 .. 1.76, up to 4096 rows H = 64 .. 160 1.55 .. 1.85.
 int Engine::forest_rows() const {
   const int fused = fused_rows();
   if (cell_ || cfg_.fused_round_rows != 0 || nch_ != 2 || group_limit() <= 0) return fused;

@@ -471,7 +471,9 @@ void build_group_lists(const Schedule &s, int nch, const int *t2j, const int *pa
         ok &= ++per[i] <= lim;
       }
     // A share of more rows than a workgroup takes in two slices wants the groups evenly loaded: where few trees hold a round's
-    // rows, most of the device would wait for one group.
+    // rows, most of the device would wait for one group.  Training steps of eight batches of few large trees, or of some among many small ones,
+    // with shares of up to 512 however uneven / like this: Tree-LSTM H = 64 1.05 .. 1.65 times as long, 256 0.99 .. 1.41, 512 1.00 .. 1.24;
+    // Tree-FC 0.98 (a tree of 1500 leaves among 255 of 10 .. 28) .. 1.48.
     for (int k = k0; k < R && ok && lim > kUnevenShare; k++)
       for (int g = 0; g < G && ok; g++) {
         const long share = per[(size_t)g * nr + (k - k0)];
