@@ -31,9 +31,9 @@ FP32_MFMA_PEAK_TF = 157.3  # MI355X dense FP32 matrix
 SPLIT_MFMA_PEAK_TF = 2516.6 / 6
 MFMA_PEAK_TF = {"gemm": SPLIT_MFMA_PEAK_TF, "round": FP32_MFMA_PEAK_TF}
 # (workload, kernel class) -> HBM bytes per dispatch, from profiles/bench_<workload>_hbm_traffic_pmc.txt
-PMC_TRAFFIC_BYTES = {("C3", "gemm"): 115.1e6, ("C3", "round"): 99.55e6, ("C1", "gemm"): 6.68e6, ("C1", "round"): 4.99e6,
-                     ("C2", "gemm"): 25.0e6, ("C2", "round"): 19.16e6, ("C4", "gemm"): 361.3e6, ("C4", "round"): 290.9e6,
-                     ("C5", "gemm"): 342.6e6, ("C5", "round"): 118.9e6}
+PMC_TRAFFIC_BYTES = {("C3", "gemm"): 132.5e6, ("C3", "round"): 99.61e6, ("C1", "gemm"): 6.72e6, ("C1", "round"): 5.0e6,
+                     ("C2", "gemm"): 25.07e6, ("C2", "round"): 19.65e6, ("C4", "gemm"): 354.6e6, ("C4", "round"): 290.9e6,
+                     ("C5", "gemm"): 290.6e6, ("C5", "round"): 82.42e6}
 # a constant taken from the profile named, not a counter read during this run
 PMC_TRAFFIC_SOURCE = {k: f"profiles/bench_{k[0]}_hbm_traffic_pmc.txt (two rocprofv3 --pmc runs of this command, FETCH_SIZE and "
                          "WRITE_SIZE per dispatch of the class; a constant copied from there, not read in this run)"
